@@ -9,7 +9,8 @@ Two engines, as a program of a user drives them:
   A prompt is one `execute` over whole prompts whose last positions are scored; a decode case opens its sequences, runs their
   prompts and then one token per sequence and step, and closes them.
 
-The layers of a stack are alike, so four of them stand for a model of any depth.
+The layers of a stack are alike, so a few of them stand for a model of any depth: four where each step has to stream weights that no
+cache still holds, one for a prompt, whose products hide them.
 """
 import math
 
@@ -22,7 +23,7 @@ from qserve_amd.serving.registry import resolve_model
 
 F64 = torch.float64
 DEV = "cuda:0"
-LAYERS = 4
+LAYERS = {"llama_step": 4, "llama_prompt": 1, "serve_prompt": designs.LAYERS, "serve_decode": designs.LAYERS}
 SCORED = 64                       # positions at the end of a prompt whose logits are asked for
 SHAPES = {"llama3_8b": LLAMA3_8B, "llama2_7b": LLAMA2_7B}
 DESIGNS = ("Vekalorn", "Mumelix", "Rivolix")
@@ -90,7 +91,7 @@ def _lengths(n, top, spread):
 # ---- the W4A8KV4 stack -------------------------------------------------------------------------------------------------------
 
 def _shape(case):
-    return dict(SHAPES[case["shape"]], layers=LAYERS)
+    return dict(SHAPES[case["shape"]], layers=LAYERS[case["kind"]])
 
 
 def _llama_gen(seed):
@@ -119,7 +120,7 @@ def _llama_weights(case, seed, with_head):
     gain = lambda: (torch.rand((D,), device=DEV, generator=g) * 0.5 + 0.75).half()      # noqa: E731
     lin = lambda n, k, size=1.0: _llama_linear(g, n, k, case["group"], size)            # noqa: E731
     # (a layer adds less to the residual stream than the stream holds)
-    W = {"layers": [dict(ln1=gain(), ln2=gain(), qkv=lin((H + 2 * G) * 128, D), o=lin(D, H * 128, 0.4), gate_up=lin(2 * I, D), down=lin(D, I, 0.4))
+    W = {"layers": [dict(ln1=gain(), ln2=gain(), qkv=lin((H + 2 * G) * 128, D), o=lin(D, H * 128, 0.2), gate_up=lin(2 * I, D), down=lin(D, I, 0.2))
                     for _ in range(c["layers"])], "norm": gain()}
     if with_head:
         W["embed"] = torch.randn((c["vocab"], D), dtype=torch.float16, device=DEV, generator=g)
@@ -177,8 +178,7 @@ def _prepare_llama_prompt(case, seed):
 def _run_llama_prompt(st):
     eng = st["engine"]
     eng.prefill(st["case"]["tokens"], st["tokens"])
-    return {"logits": torch.matmul(eng.final, eng.lm_head.t()), "hidden": eng.hidden, "tokens": eng.tokens,
-            "cache": [p for pools in eng.pools for p in pools]}
+    return {"final": eng.final, "hidden": eng.hidden, "cache": [p for pools in eng.pools for p in pools]}
 
 
 # the same in 64 bits: the path's own integers (weights, per-token activations, cache) are part of what it computes
@@ -297,8 +297,7 @@ def _exact_llama_prompt(case, seed):
         return torch.cat(out)
 
     h = _llama64(case, W, W["embed"][tokens].double(), attend)[L - 1::L]
-    logits = _chunked(_rms64(h, W["norm"], c["eps"], False), W["lm_head"])
-    return {"logits": logits, "hidden": h, "tokens": None, "cache": [None] * (2 * c["layers"])}
+    return {"final": _rms64(h, W["norm"], c["eps"], False), "hidden": h, "cache": [None] * (2 * c["layers"])}
 
 
 def _llama_work(case):
@@ -325,7 +324,11 @@ def _design(case, seed):
     m = designs.MUMELIX[case["size"]]
     if d == "Vekalorn":
         cfg = designs.vekalorn_config(s)
-        return cfg, designs.random_weights(cfg, DEV, seed)
+        W = designs.random_weights(cfg, DEV, seed)
+        for n in W:
+            if n.endswith(".norm2"):
+                W[n] = W[n] * 0.15                                           # (gains as training leaves them: the experts add to the stream)
+        return cfg, W
     if d == "Mumelix":
         cfg = designs.mumelix_config(s, m)
         return cfg, designs.mumelix_weights(cfg, m, DEV, seed)
@@ -333,7 +336,7 @@ def _design(case, seed):
     W = designs.rivolix_weights(cfg, DEV, seed)
     for n in W:
         if n.endswith((".ls1", ".ls2")):
-            W[n] = W[n] * 0.4                                                # (layer scales as training leaves them: well below one)
+            W[n] = W[n] * (0.4 if n.endswith(".ls1") else 0.08)              # (layer scales as training leaves them: well below one)
     return cfg, W
 
 
@@ -614,14 +617,14 @@ def _serve_work(case):
         row, pair, state = kv / 2, aw * 2.0, m["g_heads"] * m["g_dim"] * m["g_vdim"]
     else:
         mixer, row, pair, state = D * (3 * aw + kv), kv * 0.75, 2.5 * m["a_heads"] * 2 * m["a_dim"], 0
-    shared = expert if d == "Rivolix" else 0
+    shared, layers = expert if d == "Rivolix" else 0, LAYERS[case["kind"]]
     per_token = mixer + top * expert + shared
 
     def step(T, keys_read, pairs, rows, seqs):
         experts = E * (1.0 - (1.0 - top / E) ** T)
-        return (LAYERS * (2.0 * (mixer + shared + experts * expert) + 2.0 * row * (keys_read + T) + 8.0 * state * seqs) + 2.0 * V * D
+        return (layers * (2.0 * (mixer + shared + experts * expert) + 2.0 * row * (keys_read + T) + 8.0 * state * seqs) + 2.0 * V * D
                 + 2.0 * T * D + 4.0 * rows * V,
-                LAYERS * (2.0 * T * per_token + pairs * pair + 7.0 * state * T) + 2.0 * rows * V * D)
+                layers * (2.0 * T * per_token + pairs * pair + 7.0 * state * T) + 2.0 * rows * V * D)
 
     lens = _lengths(case["seqs"], case["tokens"], case["spread"])
     n = len(lens)
@@ -649,15 +652,12 @@ def work(case):
 
 
 def tolerance(case):
-    """Measured against `exact` and against the same path with another order of the attention's sums or other expert products.
-    A stack of quantised layers: activations that round to the other int8 value, 0.05 of the result for per-channel weights (their
-    unsigned nibbles lift such a step above the centred ones of the group form: 0.02), and with them 0.2 of a 4-bit and 0.6 of an
-    8-bit prompt cache's bytes in the last layer; a step writes only one row per sequence.  A served model: bfloat16 between its
-    operations, 0.01, and tokens whose last chosen expert is a near tie, 0.06 where that expert weighs as much as the others."""
+    """Measured against `exact` and against the same path with another order of the attention's sums or other expert products.  A
+    quantised stack: activations and cache values that round to the other integer.  A served model: bfloat16 between its operations,
+    and tokens whose last chosen expert is a near tie ("max": one of those)."""
     if case["kind"].startswith("llama"):
-        return {"rel": 0.15 if case["group"] == -1 else 0.08,
-                "differ": 0.03 if case["kind"] == "llama_step" else 0.4 if case["kv_bits"] == 4 else 0.75}
-    return {"rel": 0.05 if case["design"] == "Mumelix" else 0.12}
+        return {"rel": 0.03, "max": 0.3, "differ": 0.01}
+    return {"rel": 0.03, "max": 0.95}
 
 
 @torch.no_grad()

@@ -230,6 +230,11 @@ int qsv_moe_down(void* y, const void* act, const void* down, const int32_t* idx,
  * rows / 2 wide).  Every weight is read once per launch.  K a multiple of 8, at most 4096. */
 int qsv_expert_rows(void* out, const void* X, const int64_t* x_index, int div, const void* W, const int64_t* offsets,
                     int n_experts, int rows, int K, int act, float limit, const float* in_weight, void* stream);
+/* The same without sorting: slot s = token t's k-th choice, s = t * div + k or any n slots whose input is X[s / div]; idx int32 [n] names each
+ * slot's expert (indices from n_experts on: no product, out's row stays unwritten); row s of out belongs to slot s.  float_out (act
+ * QSV_ACT_NONE only): out is float. */
+int qsv_expert_slots(void* out, int float_out, const void* X, int div, const void* W, const int32_t* idx, int n, int n_experts, int rows, int K,
+                     int act, float limit, const float* in_weight, void* stream);
 /* Grouped expert product on the bf16 matrix cores (prompt phase): the same out[s, n] for work tiles (expert, first sorted slot,
  * slots <= qsv_grouped_gemm_tile_slots()) listed in tiles int32 [n_tiles, 3]; K a multiple of qsv_grouped_gemm_k_step(), n_rows
  * a multiple of 4, n_tiles <= 65535.  act: QSV_ACT_* (QSV_ACT_GLU: out is n_rows / 2 wide). */
@@ -242,6 +247,9 @@ int qsv_relu_sq(void* a, int64_t n, int dtype, void* stream);
 /* (idx != NULL: slots with idx[t, k] >= n_experts take h[t] in place of a sorted row) */
 int qsv_moe_combine(void* y, const void* ys, const int64_t* inv, const float* weight, int n_tokens, int top_k, int width,
                     const int32_t* idx, const void* h, int n_experts, int dtype, void* stream);
+/* The same over float rows in slot order: y[t] = sum_k weight[t, k] * ys[t * top_k + k]. */
+int qsv_moe_combine_slots(void* y, const float* ys, const float* weight, int n_tokens, int top_k, int width, const int32_t* idx, const void* h,
+                          int n_experts, int dtype, void* stream);
 
 
 /* ---- several residual streams, statistics-free norm, token shift (serve_streams.hip) ---------------------------------------- */

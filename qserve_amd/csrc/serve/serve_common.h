@@ -40,15 +40,55 @@ __device__ __forceinline__ float ld(const bf16_t* p, size_t i) { return bf2f(p[i
 __device__ __forceinline__ void st(float* p, size_t i, float v) { p[i] = v; }
 __device__ __forceinline__ void st(bf16_t* p, size_t i, float v) { p[i] = f2bf(v); }
 
+// Reductions over a wave, all 64 lanes active: the xor butterfly (offsets 32, 16, 8, 4, 2, 1; the same pairs in the same order as a
+// __shfl_xor loop, so sums round alike) in register moves - permlane swaps for 32 and 16, DPP row rotations by 8 and by 4 (after the
+// step before, the row is 8-periodic) and quad permutations - instead of six round trips through the LDS crossbar, which were most of
+// a short row kernel's chain.
+#define QSV_DPP(v, ctrl) __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, 0xF, 0xF, true))
+template <class Op>
+__device__ __forceinline__ float wave_reduce(float v, Op op) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = op(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = op(__uint_as_float(b[0]), __uint_as_float(b[1]));
+    v = op(v, QSV_DPP(v, 0x128));   // row_ror:8
+    v = op(v, QSV_DPP(v, 0x124));   // row_ror:4
+    v = op(v, QSV_DPP(v, 0x4E));    // quad_perm [2, 3, 0, 1]
+    return op(v, QSV_DPP(v, 0xB1)); // quad_perm [1, 0, 3, 2]
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+    return wave_reduce(v, [](float a, float b) { return a + b; });
 }
 __device__ __forceinline__ float wave_max(float v) {
+    return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
+}
+// NV values per lane (a power of two, at most 64) summed over the wave and scattered: v[0] of lane l ends up with the sum of value
+// l / (64 / NV).  Half of the values left are exchanged with the lane across the next bit.
+template <int NV, int O = 32, int M = NV>
+__device__ __forceinline__ void wave_sum_scatter(float (&v)[NV], int lane) {
+    if constexpr (O >= 1) {
+        if constexpr (M > 1) {
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
+            for (int i = 0; i < M / 2; ++i) {
+                if constexpr (O == 32) {
+                    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[i]), __float_as_uint(v[i + M / 2]), false, false);
+                    v[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+                } else if constexpr (O == 16) {
+                    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[i]), __float_as_uint(v[i + M / 2]), false, false);
+                    v[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+                } else {
+                    const bool up = lane & O;
+                    const float give = up ? v[i] : v[i + M / 2], keep = up ? v[i + M / 2] : v[i];
+                    v[i] = keep + (O == 8 ? QSV_DPP(give, 0x128) : O == 4 ? QSV_DPP(give, 0x141) : O == 2 ? QSV_DPP(give, 0x4E) : QSV_DPP(give, 0xB1));
+                }
+            }
+            wave_sum_scatter<NV, O / 2, M / 2>(v, lane);
+        } else {
+            static_assert(O <= 4, "at least 8 values");
+            v[0] += O == 4 ? QSV_DPP(v[0], 0x141) : O == 2 ? QSV_DPP(v[0], 0x4E) : QSV_DPP(v[0], 0xB1);   // (half mirror, quad permutations)
+            wave_sum_scatter<NV, O / 2, 1>(v, lane);
+        }
+    }
 }
 // Sum over a workgroup of NT threads (a multiple of 64); every thread gets the result.  `red` holds NT / 64 + 1 floats.
 template <int NT>

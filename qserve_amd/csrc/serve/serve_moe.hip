@@ -22,6 +22,25 @@ __device__ __forceinline__ void load8(const float* p, float (&v)[8]) {
     const float4 a = *(const float4*)p, b = *(const float4*)(p + 4);
     v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
 }
+__device__ __forceinline__ void loadv(const bf16_t* p, float (&v)[4]) {
+    const uint2 u = *(const uint2*)p;
+    v[0] = __uint_as_float(u.x << 16);
+    v[1] = __uint_as_float(u.x & 0xffff0000u);
+    v[2] = __uint_as_float(u.y << 16);
+    v[3] = __uint_as_float(u.y & 0xffff0000u);
+}
+__device__ __forceinline__ void loadv(const float* p, float (&v)[4]) {
+    const float4 a = *(const float4*)p;
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+}
+template <typename T>
+__device__ __forceinline__ void loadv(const T* p, float (&v)[1]) { v[0] = ld(p, 0); }
+__device__ __forceinline__ void storev(bf16_t* p, const float (&v)[4]) {
+    *(uint2*)p = make_uint2((unsigned)f2bf(v[0]) | ((unsigned)f2bf(v[1]) << 16), (unsigned)f2bf(v[2]) | ((unsigned)f2bf(v[3]) << 16));
+}
+__device__ __forceinline__ void storev(float* p, const float (&v)[4]) { *(float4*)p = make_float4(v[0], v[1], v[2], v[3]); }
+template <typename T>
+__device__ __forceinline__ void storev(T* p, const float (&v)[1]) { st(p, 0, v[0]); }
 // (value, index) of the largest value over a wave; ties go to the lower index.  Lanes without a candidate pass index -1.
 __device__ __forceinline__ void wave_argmax(float& v, int& i) {
 #pragma unroll
@@ -156,6 +175,135 @@ __global__ __launch_bounds__(NT) void moe_route_kernel(int32_t* __restrict__ idx
             if (renorm) v /= chosen;
             weight[t * top_k + k] = v * scale;
         }
+}
+
+// The same for at most 64 experts and widths that are multiples of 8 (one expert per lane in the selection).  The wide form's time went
+// into serial steps: a wave took its experts one by one, six shuffles each, and the selection was (keep + top_k) wave-wide argmax searches
+// with a barrier each.  Here the four waves split the width and hold 16 experts' sums for TT tokens side by side, the sums are reduced and
+// scattered over the lanes in one butterfly, and a lane finds its expert's place by counting the better ones (broadcasts, no search).
+// TT = 4 tokens share the router's rows in prompts; in steps one token per workgroup keeps more workgroups busy.
+__device__ __forceinline__ unsigned order_key(float v) {         // larger key = larger value; -0 = +0, NaN below everything
+    const unsigned u = __float_as_uint(v + 0.0f);
+    return v != v ? 0u : u >> 31 ? ~u : u | 0x80000000u;
+}
+// number of lanes j < n in `mask` whose key is larger (or equal at a lower index): unique per lane of the mask
+__device__ __forceinline__ int place_of(unsigned key, unsigned long long mask, int n, int lane) {
+    int r = 0;
+    for (int j = 0; j < n; ++j) {
+        const unsigned kj = (unsigned)__builtin_amdgcn_readlane((int)key, j);
+        r += (mask >> j & 1) && (kj > key || (kj == key && j < lane));
+    }
+    return r;
+}
+template <typename T>
+struct Piece {
+    typedef uint4 type;
+};
+struct float8 {
+    float4 a, b;
+};
+template <>
+struct Piece<float> {
+    typedef float8 type;
+};
+template <typename T, int TT>
+__global__ __launch_bounds__(NT, 2) void moe_route_wave_kernel(int32_t* __restrict__ idx, float* __restrict__ weight, const T* __restrict__ h,
+                                                            const T* __restrict__ router, const T* __restrict__ bias, int renorm, int n, int D, int E,
+                                                            int top_k, int G, int keep, int score_fn, const float* __restrict__ correction,
+                                                            int group_top, float scale) {
+    constexpr int EC = 16, NV = TT * EC;
+    __shared__ float part[NW][TT][64];
+    __shared__ float cs[NW][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const size_t t0 = (size_t)blockIdx.x * TT;
+    const float lane_bias = bias && lane < E ? ld(bias, lane) : 0.f, lane_corr = correction && lane < E ? correction[lane] : 0.f;
+    for (int e0 = 0; e0 < E; e0 += EC) {
+        float v[NV];
+#pragma unroll
+        for (int i = 0; i < NV; ++i) v[i] = 0.f;
+        for (int c = threadIdx.x * 8; c < D; c += NT * 8) {
+            typename Piece<T>::type xr[TT], rr[EC];                // every load in flight before the first is used
+#pragma unroll
+            for (int tt = 0; tt < TT; ++tt) xr[tt] = *(const typename Piece<T>::type*)(h + min(t0 + tt, (size_t)n - 1) * D + c);
+#pragma unroll
+            for (int e = 0; e < EC; ++e) rr[e] = *(const typename Piece<T>::type*)(router + (size_t)min(e0 + e, E - 1) * D + c);
+            __builtin_amdgcn_sched_barrier(0);
+            float x[TT][8];
+#pragma unroll
+            for (int tt = 0; tt < TT; ++tt) load8((const T*)&xr[tt], x[tt]);
+#pragma unroll
+            for (int e = 0; e < EC; ++e) {
+                float r[8];
+                load8((const T*)&rr[e], r);
+#pragma unroll
+                for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) v[tt * EC + e] += r[q] * x[tt][q];
+            }
+        }
+        wave_sum_scatter<NV>(v, lane);
+        const int id = lane / (64 / NV);
+        if (lane % (64 / NV) == 0) part[w][id / EC][e0 + id % EC] = v[0];
+    }
+    __syncthreads();
+    if (w >= TT || t0 + w >= (size_t)n) return;                  // wave w selects for token w (no barrier follows)
+    const size_t t = t0 + w;
+    const bool mine = lane < E;
+    float s = -INFINITY;
+    if (mine) {
+        s = 0.f;
+#pragma unroll
+        for (int o = 0; o < NW; ++o) s += part[o][w][lane];
+        if (bias) s += lane_bias;
+    }
+    if (score_fn == 0) {
+        const float mx = wave_max(s);
+        s = mine ? expf(s - mx) : 0.f;
+        s *= 1.0f / wave_sum(s);
+    } else {
+        s = 1.0f / (1.0f + expf(-s));
+    }
+    const float c = mine ? (correction ? s + lane_corr : s) : 0.f;
+    unsigned long long ok = E == 64 ? ~0ull : (1ull << E) - 1;   // experts that may be chosen
+    if (keep < G) {
+        cs[w][lane] = c;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        const int per = E / G;
+        float gs = 0.f;
+        if (lane < G) {
+            float v1 = cs[w][lane * per], v2 = -INFINITY;        // the two largest
+            for (int e = 1; e < per; ++e) {
+                const float v = cs[w][lane * per + e];
+                if (v > v1) {
+                    v2 = v1;
+                    v1 = v;
+                } else if (v > v2) {
+                    v2 = v;
+                }
+            }
+            gs = (group_top == 2 && per > 1) ? v1 + v2 : v1;
+        }
+        const unsigned long long all = G == 64 ? ~0ull : (1ull << G) - 1;
+        const int place = place_of(order_key(gs), all, G, lane);
+        const unsigned long long kept = __ballot(lane < G && place < keep);
+        ok = __ballot(mine && (kept >> (min(lane, E - 1) / per) & 1));
+    }
+    const int place = place_of(order_key(c), ok, E, lane);
+    const bool chosen = mine && (ok >> lane & 1) && place < top_k;
+    float wt = s;
+    if (renorm) {                                                // over the chosen only, summed from the best down
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (chosen) cs[w][place] = s;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        float sum = 0.f;
+        for (int k = 0; k < top_k; ++k) sum += cs[w][k];
+        wt /= sum;
+    }
+    if (renorm || scale != 1.0f) wt *= scale;
+    if (chosen) {
+        idx[t * top_k + place] = lane;
+        weight[t * top_k + place] = wt;
+    }
 }
 
 // Activation of the first expert product.  ACT_GLU: the weight rows come in pairs (2f = gate, 2f + 1 = up) and output f is
@@ -336,80 +484,250 @@ __global__ __launch_bounds__(NT) void moe_down_vec_kernel(T* __restrict__ y, con
     }
 }
 
-// ---- expert-major form (decoding and short portions, bfloat16): slots sorted by expert ON THE DEVICE, workgroup = (16 output rows,
-// expert); a wave keeps its four weight rows in registers (packed bfloat16) and walks the tokens routed to the expert, so every
-// weight is read once per step however many tokens share the expert.  No host synchronisation. ----------------------------------
-typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
-template <int KI, int ACT>
-__global__ __launch_bounds__(NT) void expert_rows_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ X,
-                                                         const int64_t* __restrict__ x_index, int div, const bf16_t* __restrict__ W,
-                                                         const int64_t* __restrict__ offsets, int rows, int K, float limit,
-                                                         const float* __restrict__ in_weight) {
-    const int e = blockIdx.y;
-    const int64_t s0 = offsets[e], s1 = offsets[e + 1];
-    if (s0 == s1) return;                                                   // nobody chose this expert
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int r0 = (blockIdx.x * NW + w) * ROWS;
-    if (r0 >= rows) return;
-    uint4 wr[ROWS][KI];
+// ---- expert-major form (decoding and short portions, bfloat16): workgroup = (32 weight rows, expert), every weight read once per step
+// however many tokens share the expert.  Bound by HBM (the chosen experts' weights) and, below that, by launch latency.
+// * The slots (token t's k-th choice: slot t top_k + k) of an expert are found by the workgroup itself from the router's indices - no
+//   sort, no counts on the host - or given as sorted runs (`offsets`).
+// * The four waves split the reduction (stage i of 64 elements belongs to wave i % 4), so the expert's inputs are read once per workgroup.
+//   Each wave streams its stages - one 128-byte line of 32 weight rows and of 16 or 32 inputs - through a ring of its own in LDS
+//   (global_load_lds, whole lines; the wave waits for its own oldest stage only, no barrier in the loop) and multiplies them with
+//   v_mfma_f32_16x16x32_bf16, weights as the A operand.  Pieces of a row are permuted by its number: 16-byte reads without bank conflicts.
+// * The partial sums of the four waves meet in LDS; more than 32 slots per expert are walked in chunks (the weights then come from L2).
+// Two workgroups per CU keep up to 96 KiB of weights in flight.
+// Measured per launch in a step (MI355X): 64 tokens, 4 of 16 experts of 2048 x 1408 (92 MB a product) 55.6 / 62.4 us -> 23.8 / 21.1 us (up /
+// down) against the form it replaces, which kept weight rows in registers and paid a wave-wide sum per token and row; 16 tokens with
+// gated units (184 + 92 MB) 42.6 / 26.1 -> 36.5 / 19.3 us (5.0 TB/s); one token 1446 / 3117 us (the per-token kernels) -> 14.0 / 8.8 us.
+// The sort, search and permutation launches in front of it (60 us a layer) are gone.
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void* lds_ptr;
+constexpr int XR = 32;               // weight rows per workgroup
+constexpr int XK = 64;               // reduction elements per stage
+constexpr int XRING = 18 * 1024;     // ring of one wave
+constexpr int XLIST = 1024;          // router indices looked at in one go
+
+struct ExpertArgs {
+    void* out;                       // bf16, or float (no activation)
+    const bf16_t* X;
+    const bf16_t* W;
+    const int32_t* idx;              // the router's indices [n] (or NULL)
+    const int64_t* x_index;          // sorted runs: sorted slot -> slot (or NULL: itself)
+    const int64_t* offsets;
+    const float* in_weight;
+    int n, div, rows, K;
+    float limit;
+    bool wide;                       // out starts on 16 bytes
+};
+
+// SG: groups of 16 slots in the chunk
+template <int SG>
+struct ExpertRing {
+    static constexpr int STAGE = (XR + 16 * SG) * 128, INSTR = STAGE / 1024, DEPTH = XRING / STAGE;
+};
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ void lds_copy16(unsigned dst, const void* base, unsigned off) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(dst) : "memory");
+}
+__device__ __forceinline__ void lds_copy16(unsigned dst, const void* from) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(dst) : "memory");
+}
+
+// Products of the workgroup's rows with 16 SG inputs; row_of(i): input i's row of X.
+template <int SG, class Row>
+__device__ __forceinline__ void expert_chunk(const ExpertArgs& a, const bf16_t* W0, int rows_here, unsigned char* ring, int w, int lane, Row row_of,
+                                             v4f (&acc)[XR / 16][SG]) {
+    typedef ExpertRing<SG> R;
+    const int stages = (a.K + XK - 1) / XK, mine = stages > w ? (stages - w + NW - 1) / NW : 0;
+    const int piece = (lane & 7) ^ (lane >> 3);
+    unsigned woff[XR / 8];
+    const bf16_t* xrow[2 * SG];
 #pragma unroll
-    for (int r = 0; r < ROWS; ++r)
+    for (int j = 0; j < XR / 8; ++j) woff[j] = (unsigned)min(8 * j + (lane >> 3), rows_here - 1) * (unsigned)a.K * 2u;
 #pragma unroll
-        for (int i = 0; i < KI; ++i) {
-            const int c = (lane + 64 * i) * 8;
-            wr[r][i] = (r0 + r < rows && c < K) ? *(const uint4*)(W + ((size_t)e * rows + r0 + r) * K + c) : make_uint4(0u, 0u, 0u, 0u);
-        }
-    // TOK tokens at a time: their input pieces are all requested before the first is used (a token at a time, every token
-    // paid a full memory round trip with nothing else in flight)
-    constexpr int TOK = 4;
-    for (int64_t sb = s0; sb < s1; sb += TOK) {
-        uint4 xr[TOK][KI];
+    for (int j = 0; j < 2 * SG; ++j) xrow[j] = a.X + (size_t)row_of(8 * j + (lane >> 3)) * (size_t)a.K;
 #pragma unroll
-        for (int j = 0; j < TOK; ++j) {
-            const int64_t s = sb + j < s1 ? sb + j : s1 - 1;
-            const bf16_t* x = X + (size_t)(x_index ? x_index[s] / div : s) * K;
+    for (int r = 0; r < XR / 16; ++r)
 #pragma unroll
-            for (int i = 0; i < KI; ++i) {
-                const int c = (lane + 64 * i) * 8;
-                xr[j][i] = c < K ? *(const uint4*)(x + c) : make_uint4(0u, 0u, 0u, 0u);
+        for (int g = 0; g < SG; ++g) acc[r][g] = v4f{0.f, 0.f, 0.f, 0.f};
+    const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(lds_ptr)ring);
+    auto issue = [&](int i) {
+        const int k0 = (w + NW * i) * XK;
+        const unsigned po = k0 + piece * 8 < a.K ? (unsigned)piece * 16u : 0u;     // (beyond the row: any valid piece, masked below)
+        const unsigned dst = lds0 + (unsigned)(i % R::DEPTH) * R::STAGE;
+#pragma unroll
+        for (int j = 0; j < XR / 8; ++j) lds_copy16(dst + 1024 * j, W0 + k0, woff[j] + po);
+#pragma unroll
+        for (int j = 0; j < 2 * SG; ++j) lds_copy16(dst + 1024 * (XR / 8 + j), (const unsigned char*)(xrow[j] + k0) + po);
+    };
+    const int row = lane & 15, quad = lane >> 4;
+    wait_vm<0>();
+    for (int i = 0; i < min(R::DEPTH, mine); ++i) issue(i);
+    for (int i = 0; i < mine; ++i) {
+        const int ahead = min(R::DEPTH - 1, mine - 1 - i);                         // stages requested behind this one
+        if (ahead == 2) wait_vm<2 * R::INSTR>();
+        else if (ahead == 1) wait_vm<R::INSTR>();
+        else wait_vm<0>();
+        const unsigned char* st = ring + (i % R::DEPTH) * R::STAGE;
+        const int left = a.K - (w + NW * i) * XK;                                  // elements of this stage inside the row
+#pragma unroll
+        for (int ks = 0; ks < XK / 32; ++ks) {
+            const int p = 4 * ks + quad;
+            v4u A[XR / 16], B[SG];
+#pragma unroll
+            for (int r = 0; r < XR / 16; ++r) A[r] = *(const v4u*)(st + (16 * r + row) * 128 + ((p ^ (row & 7)) << 4));
+#pragma unroll
+            for (int g = 0; g < SG; ++g) B[g] = *(const v4u*)(st + (XR + 16 * g + row) * 128 + ((p ^ (row & 7)) << 4));
+            if (left < XK && p * 8 >= left) {
+#pragma unroll
+                for (int r = 0; r < XR / 16; ++r) A[r] = v4u{0u, 0u, 0u, 0u};
+#pragma unroll
+                for (int g = 0; g < SG; ++g) B[g] = v4u{0u, 0u, 0u, 0u};
             }
+#pragma unroll
+            for (int r = 0; r < XR / 16; ++r)
+#pragma unroll
+                for (int g = 0; g < SG; ++g)
+                    acc[r][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, A[r]), __builtin_bit_cast(bf8, B[g]), acc[r][g], 0, 0, 0);
         }
+        if (i + R::DEPTH < mine) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                     // the slot has been read
+            issue(i + R::DEPTH);
+        }
+    }
+}
+
+// The four waves' partial sums (through LDS), the weight on the input, the activation, the store: slot of column c by slot_of(c).
+template <int ACT, bool FOUT, int SG, class Slot>
+__device__ __forceinline__ void expert_finish(const ExpertArgs& a, int r0, int count, unsigned char* rings, int w, int lane, Slot slot_of,
+                                              const v4f (&acc)[XR / 16][SG]) {
+    constexpr int TILES = XR / 16 * SG;
+    v4f* red = (v4f*)rings;                                                        // [wave][tile][lane]
+    __syncthreads();                                                               // every wave is done with its ring
 #pragma unroll
-        for (int j = 0; j < TOK; ++j) {
-            float acc[ROWS] = {0.f, 0.f, 0.f, 0.f};
+    for (int r = 0; r < XR / 16; ++r)
 #pragma unroll
-            for (int i = 0; i < KI; ++i) {
-                const unsigned xu[4] = {xr[j][i].x, xr[j][i].y, xr[j][i].z, xr[j][i].w};
+        for (int g = 0; g < SG; ++g) red[(w * TILES + r * SG + g) * 64 + lane] = acc[r][g];
+    __syncthreads();
 #pragma unroll
-                for (int r = 0; r < ROWS; ++r) {
-                    const unsigned u[4] = {wr[r][i].x, wr[r][i].y, wr[r][i].z, wr[r][i].w};
+    for (int t0 = 0; t0 < TILES; t0 += NW) {
+        const int t = t0 + w, r = t / SG, c = 16 * (t % SG) + (lane & 15);
+        if (t < TILES && c < count) {
+            v4f v = red[t * 64 + lane];
 #pragma unroll
-                    for (int q = 0; q < 4; ++q)                           // v_dot2_f32_bf16: two products per instruction, no unpacking
-                        acc[r] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf2, u[q]), __builtin_bit_cast(bf2, xu[q]), acc[r], false);
+            for (int o = 1; o < NW; ++o) v += red[(o * TILES + t) * 64 + lane];
+            const int n0 = r0 + 16 * r + 4 * (lane >> 4);
+            int64_t slot;
+            float iw = 1.0f;                                                       // the expert works on weight * input
+            slot_of(c, slot, iw);
+            v *= iw;
+            float u[4] = {v[0], v[1], v[2], v[3]};
+            int m = 4, stride = a.rows, at = n0;
+            if (ACT == ACT_GLU) {
+                u[0] = glu(u[0], u[1], a.limit);
+                u[1] = glu(u[2], u[3], a.limit);
+                m = 2;
+                stride /= 2;
+                at /= 2;
+            } else if (ACT == ACT_RELU_SQ) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) u[q] = relu_sq(u[q]);
+            }
+            if (FOUT) {
+                float* o = (float*)a.out + (size_t)slot * stride + at;
+                if (a.wide && stride % 4 == 0 && at + 4 <= stride) *(v4f*)o = v4f{u[0], u[1], u[2], u[3]};
+                else
+                    for (int q = 0; q < m; ++q)
+                        if (at + q < stride) o[q] = u[q];
+            } else {
+                bf16_t* o = (bf16_t*)a.out + (size_t)slot * stride + at;
+                const unsigned lo = (unsigned)f2bf(u[0]) | ((unsigned)f2bf(u[1]) << 16);
+                if (a.wide && stride % m == 0 && at + m <= stride) {
+                    if (m == 2) *(unsigned*)o = lo;
+                    else *(uint2*)o = make_uint2(lo, (unsigned)f2bf(u[2]) | ((unsigned)f2bf(u[3]) << 16));
+                } else {
+                    for (int q = 0; q < m; ++q)
+                        if (at + q < stride) o[q] = f2bf(u[q]);
                 }
             }
-            if (sb + j < s1) {                                              // (wave-uniform)
-                float d[ROWS];
-#pragma unroll
-                for (int r = 0; r < ROWS; ++r) d[r] = wave_sum(acc[r]);
-                if (in_weight) {                                            // the expert works on weight * input
-                    const float iw = in_weight[x_index ? x_index[sb + j] : sb + j];
-#pragma unroll
-                    for (int r = 0; r < ROWS; ++r) d[r] *= iw;
-                }
-                if (lane == 0) {
-                    if (ACT == ACT_GLU) {
-#pragma unroll
-                        for (int r = 0; r < ROWS; r += 2)
-                            if (r0 + r < rows) out[(size_t)(sb + j) * (rows / 2) + (r0 + r) / 2] = f2bf(glu(d[r], d[r + 1], limit));
-                    } else {
-#pragma unroll
-                        for (int r = 0; r < ROWS; ++r)
-                            if (r0 + r < rows) out[(size_t)(sb + j) * rows + r0 + r] = f2bf(ACT == ACT_RELU_SQ ? relu_sq(d[r]) : d[r]);
-                    }
-                }
+        }
+    }
+    __syncthreads();                                                               // (the rings are free again)
+}
+
+template <int ACT, bool FOUT>
+__global__ __launch_bounds__(NT, 2) void expert_rows_kernel(ExpertArgs a) {
+    __shared__ __attribute__((aligned(128))) unsigned char rings[NW * XRING];
+    __shared__ unsigned short list[XLIST];
+    __shared__ int listed[NW];
+    const int e = blockIdx.y, lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r0 = blockIdx.x * XR, rows_here = min(XR, a.rows - r0);
+    const bf16_t* W0 = a.W + ((size_t)e * a.rows + r0) * (size_t)a.K;
+    unsigned char* ring = rings + w * XRING;
+    // `count` inputs: X row by row_of(i), output row (and weight) by slot_of(i)
+    auto walk = [&](int count, auto row_of, auto slot_of) {
+        for (int c0 = 0; c0 < count; c0 += 32) {
+            const int c = min(32, count - c0);
+            auto rows = [&](int i) { return row_of(c0 + min(i, c - 1)); };
+            auto slots = [&](int i, int64_t& slot, float& iw) { slot_of(c0 + i, slot, iw); };
+            if (c <= 16) {
+                v4f acc[XR / 16][1];
+                expert_chunk<1>(a, W0, rows_here, ring, w, lane, rows, acc);
+                expert_finish<ACT, FOUT, 1>(a, r0, c, rings, w, lane, slots, acc);
+            } else {
+                v4f acc[XR / 16][2];
+                expert_chunk<2>(a, W0, rows_here, ring, w, lane, rows, acc);
+                expert_finish<ACT, FOUT, 2>(a, r0, c, rings, w, lane, slots, acc);
             }
         }
+    };
+    if (a.offsets) {
+        const int64_t s0 = a.offsets[e];
+        walk((int)(a.offsets[e + 1] - s0),
+             [&](int i) {
+                 const int64_t s = s0 + i;
+                 return a.x_index ? a.x_index[s] / a.div : s;
+             },
+             [&](int i, int64_t& slot, float& iw) {
+                 slot = s0 + i;
+                 if (a.in_weight) iw = a.in_weight[a.x_index ? a.x_index[slot] : slot];
+             });
+        return;
+    }
+    for (int n0 = 0; n0 < a.n; n0 += XLIST) {
+        // this expert's slots among the next XLIST, in order: wave w looks at a quarter of them
+        const int len = min(XLIST, a.n - n0), span = (len + NT - 1) / NT * 64;
+        int found = 0;
+        unsigned long long hit[XLIST / NT];
+#pragma unroll
+        for (int q = 0; q < XLIST / NT; ++q) {
+            const int i = w * span + 64 * q + lane;
+            hit[q] = __ballot(64 * q < span && i < len && a.idx[n0 + i] == e);
+            found += __popcll(hit[q]);
+        }
+        if (lane == 0) listed[w] = found;
+        __syncthreads();
+        int at = 0, count = 0;
+#pragma unroll
+        for (int o = 0; o < NW; ++o) {
+            at += o < w ? listed[o] : 0;
+            count += listed[o];
+        }
+#pragma unroll
+        for (int q = 0; q < XLIST / NT; ++q) {
+            if (hit[q] >> lane & 1) list[at + __popcll(hit[q] & ((1ull << lane) - 1))] = (unsigned short)(w * span + 64 * q + lane);
+            at += __popcll(hit[q]);
+        }
+        __syncthreads();
+        walk(count, [&](int i) { return (int64_t)((n0 + list[i]) / a.div); },
+             [&](int i, int64_t& slot, float& iw) {
+                 slot = n0 + list[i];
+                 if (a.in_weight) iw = a.in_weight[slot];
+             });
+        __syncthreads();
     }
 }
 
@@ -430,19 +748,26 @@ __global__ __launch_bounds__(NT) void relu_sq_kernel(T* __restrict__ a, size_t n
         st(a, i, v * v);
     }
 }
-// y[t] = sum_k weight[t, k] * ys[inv[t top_k + k]]   (weight NULL: ones)
-template <typename T>
-__global__ __launch_bounds__(NT) void moe_combine_kernel(T* __restrict__ y, const T* __restrict__ ys, const int64_t* __restrict__ inv,
+// y[t] = sum_k weight[t, k] * ys[inv ? inv[t top_k + k] : t top_k + k]   (weight NULL: ones).  VEC coordinates per thread.
+template <typename T, typename Y, int VEC>
+__global__ __launch_bounds__(NT) void moe_combine_kernel(T* __restrict__ y, const Y* __restrict__ ys, const int64_t* __restrict__ inv,
                                                          const float* __restrict__ weight, int top_k, int D,
                                                          const int32_t* __restrict__ idx, const T* __restrict__ h, int n_experts) {
     const size_t t = blockIdx.x;
-    for (int c = threadIdx.x; c < D; c += NT) {
-        float a = 0.f;
+    for (int c = (blockIdx.y * NT + threadIdx.x) * VEC; c < D; c += gridDim.y * NT * VEC) {
+        float a[VEC] = {};
+#pragma unroll 4
         for (int k = 0; k < top_k; ++k) {
-            const bool same = idx && idx[t * top_k + k] >= n_experts;       // an identity expert's slot has no sorted row
-            a += (weight ? weight[t * top_k + k] : 1.0f) * (same ? ld(h, t * D + c) : ld(ys, (size_t)inv[t * top_k + k] * D + c));
+            const size_t slot = t * top_k + k;
+            const bool same = idx && idx[slot] >= n_experts;                // an identity expert's slot has no row of its own
+            const float wk = weight ? weight[slot] : 1.0f;
+            float v[VEC];
+            if (same) loadv(h + t * D + c, v);
+            else loadv(ys + (size_t)(inv ? inv[slot] : (int64_t)slot) * D + c, v);
+#pragma unroll
+            for (int q = 0; q < VEC; ++q) a[q] += wk * v[q];
         }
-        st(y, t * D + c, a);
+        storev(y + t * D + c, a);
     }
 }
 }  // namespace
@@ -456,37 +781,36 @@ extern "C" int qsv_gather_rows(void* out, const void* src, const int64_t* order,
                                     order, div, width));
     return qsv_launch_status("qsv_gather_rows");
 }
-// out[s, r] = act(W[e][r, :] . X[x_index ? x_index[s] / div : s, :]) for the sorted slots s in [offsets[e], offsets[e + 1]) of every
-// expert e; W [E, rows, K] bfloat16, act: 0 nothing, 1 relu^2, 2 gated unit (row pairs; out is rows / 2 wide).  K % 8 == 0, K <= 4096.
+static int launch_expert_rows(const char* what, ExpertArgs a, int n_experts, int act, bool float_out, void* stream) {
+    QSV_REQUIRE(a.out && a.X && a.W && n_experts > 0 && a.rows > 0 && a.div > 0, "%s: bad arguments", what);
+    QSV_REQUIRE(act == ACT_NONE || act == ACT_RELU_SQ || ((act == ACT_GLU || act == QSV_ACT_CLAMPED_GLU) && a.rows % 2 == 0), "%s: activation %d", what,
+                act);
+    QSV_REQUIRE(act != QSV_ACT_CLAMPED_GLU || a.limit > 0.f, "%s: clamped units need a positive limit", what);
+    if (act == QSV_ACT_CLAMPED_GLU) act = ACT_GLU;
+    else a.limit = 0.f;
+    QSV_REQUIRE(a.K > 0 && a.K % 8 == 0 && a.K <= 4096, "%s: inner width %d (a multiple of 8, at most 4096)", what, a.K);
+    QSV_REQUIRE(n_experts <= 65535, "%s: too many experts", what);
+    QSV_REQUIRE(((uintptr_t)a.X | (uintptr_t)a.W) % 16 == 0, "%s: inputs and weights start on 16 bytes", what);
+    a.wide = (uintptr_t)a.out % 16 == 0;
+    const dim3 grid((a.rows + XR - 1) / XR, n_experts), block(NT);
+    if (float_out) hipLaunchKernelGGL((expert_rows_kernel<ACT_NONE, true>), grid, block, 0, (hipStream_t)stream, a);
+    else if (act == ACT_RELU_SQ) hipLaunchKernelGGL((expert_rows_kernel<ACT_RELU_SQ, false>), grid, block, 0, (hipStream_t)stream, a);
+    else if (act == ACT_GLU) hipLaunchKernelGGL((expert_rows_kernel<ACT_GLU, false>), grid, block, 0, (hipStream_t)stream, a);
+    else hipLaunchKernelGGL((expert_rows_kernel<ACT_NONE, false>), grid, block, 0, (hipStream_t)stream, a);
+    return qsv_launch_status(what);
+}
 extern "C" int qsv_expert_rows(void* out, const void* X, const int64_t* x_index, int div, const void* W, const int64_t* offsets,
                                int n_experts, int rows, int K, int act, float limit, const float* in_weight, void* stream) {
-    QSV_REQUIRE(out && X && W && offsets && n_experts > 0 && rows > 0 && div > 0, "qsv_expert_rows: bad arguments");
-    QSV_REQUIRE(act == ACT_NONE || act == ACT_RELU_SQ || ((act == ACT_GLU || act == QSV_ACT_CLAMPED_GLU) && rows % 2 == 0),
-                "qsv_expert_rows: activation %d", act);
-    QSV_REQUIRE(act != QSV_ACT_CLAMPED_GLU || limit > 0.f, "qsv_expert_rows: clamped units need a positive limit");
-    if (act == QSV_ACT_CLAMPED_GLU) act = ACT_GLU;
-    else limit = 0.f;
-    QSV_REQUIRE(K > 0 && K % 8 == 0 && K <= 4096, "qsv_expert_rows: inner width %d (a multiple of 8, at most 4096)", K);
-    QSV_REQUIRE(n_experts <= 65535, "qsv_expert_rows: too many experts");
-    const dim3 grid((rows + NW * ROWS - 1) / (NW * ROWS), n_experts), block(NT);
-#define QSV_ER(KI)                                                                                                           \
-    do {                                                                                                                     \
-        if (act == ACT_RELU_SQ)                                                                                              \
-            hipLaunchKernelGGL((expert_rows_kernel<KI, ACT_RELU_SQ>), grid, block, 0, (hipStream_t)stream, (bf16_t*)out,         \
-                               (const bf16_t*)X, x_index, div, (const bf16_t*)W, offsets, rows, K, limit, in_weight);                          \
-        else if (act == ACT_GLU)                                                                                             \
-            hipLaunchKernelGGL((expert_rows_kernel<KI, ACT_GLU>), grid, block, 0, (hipStream_t)stream, (bf16_t*)out,             \
-                               (const bf16_t*)X, x_index, div, (const bf16_t*)W, offsets, rows, K, limit, in_weight);                          \
-        else                                                                                                                 \
-            hipLaunchKernelGGL((expert_rows_kernel<KI, ACT_NONE>), grid, block, 0, (hipStream_t)stream, (bf16_t*)out,            \
-                               (const bf16_t*)X, x_index, div, (const bf16_t*)W, offsets, rows, K, limit, in_weight);                          \
-    } while (0)
-    if (K <= 512) QSV_ER(1);
-    else if (K <= 1024) QSV_ER(2);
-    else if (K <= 2048) QSV_ER(4);
-    else QSV_ER(8);
-#undef QSV_ER
-    return qsv_launch_status("qsv_expert_rows");
+    QSV_REQUIRE(offsets, "qsv_expert_rows: bad arguments");
+    const ExpertArgs a = {out, (const bf16_t*)X, (const bf16_t*)W, nullptr, x_index, offsets, in_weight, 0, div, rows, K, limit, false};
+    return launch_expert_rows("qsv_expert_rows", a, n_experts, act, false, stream);
+}
+extern "C" int qsv_expert_slots(void* out, int float_out, const void* X, int div, const void* W, const int32_t* idx, int n, int n_experts, int rows,
+                                int K, int act, float limit, const float* in_weight, void* stream) {
+    QSV_REQUIRE(idx && n >= 0 && (!float_out || act == ACT_NONE), "qsv_expert_slots: bad arguments");
+    if (n == 0) return QSV_OK;
+    const ExpertArgs a = {out, (const bf16_t*)X, (const bf16_t*)W, idx, nullptr, nullptr, in_weight, n, div, rows, K, limit, false};
+    return launch_expert_rows("qsv_expert_slots", a, n_experts, act, float_out != 0, stream);
 }
 extern "C" int qsv_relu_sq(void* a, int64_t n, int dtype, void* stream) {
     QSV_REQUIRE(a && n >= 0 && n < (1ll << 31) * NT, "qsv_relu_sq: bad arguments");
@@ -496,14 +820,33 @@ extern "C" int qsv_relu_sq(void* a, int64_t n, int dtype, void* stream) {
                                     (size_t)n));
     return qsv_launch_status("qsv_relu_sq");
 }
+// (four coordinates per thread where the rows' starts allow it; few tokens: a token's row over several workgroups)
+template <typename T, typename Y>
+static void launch_combine(void* y, const void* ys, const int64_t* inv, const float* weight, int n, int top_k, int D, const int32_t* idx,
+                           const void* h, int n_experts, void* stream) {
+    const bool vec = D % 4 == 0 && ((uintptr_t)ys % (4 * sizeof(Y)) == 0) && ((uintptr_t)y % (4 * sizeof(T)) == 0) && (!h || (uintptr_t)h % (4 * sizeof(T)) == 0);
+    const int per = NT * (vec ? 4 : 1), need = (D + per - 1) / per;
+    const dim3 grid(n, n < 1024 ? need : 1);
+    if (vec)
+        hipLaunchKernelGGL((moe_combine_kernel<T, Y, 4>), grid, dim3(NT), 0, (hipStream_t)stream, (T*)y, (const Y*)ys, inv, weight, top_k, D, idx,
+                           (const T*)h, n_experts);
+    else
+        hipLaunchKernelGGL((moe_combine_kernel<T, Y, 1>), grid, dim3(NT), 0, (hipStream_t)stream, (T*)y, (const Y*)ys, inv, weight, top_k, D, idx,
+                           (const T*)h, n_experts);
+}
 extern "C" int qsv_moe_combine(void* y, const void* ys, const int64_t* inv, const float* weight, int n, int top_k, int D,
                                const int32_t* idx, const void* h, int n_experts, int dtype, void* stream) {
     QSV_REQUIRE(y && ys && inv && n >= 0 && top_k > 0 && D > 0 && (!idx || h), "qsv_moe_combine: bad arguments");
     if (n == 0) return QSV_OK;
-    QSV_DISPATCH(dtype, "qsv_moe_combine",
-                 hipLaunchKernelGGL(moe_combine_kernel<T>, dim3(n), dim3(NT), 0, (hipStream_t)stream, (T*)y, (const T*)ys, inv,
-                                    weight, top_k, D, idx, (const T*)h, n_experts));
+    QSV_DISPATCH(dtype, "qsv_moe_combine", (launch_combine<T, T>(y, ys, inv, weight, n, top_k, D, idx, h, n_experts, stream)));
     return qsv_launch_status("qsv_moe_combine");
+}
+extern "C" int qsv_moe_combine_slots(void* y, const float* ys, const float* weight, int n, int top_k, int D, const int32_t* idx, const void* h,
+                                     int n_experts, int dtype, void* stream) {
+    QSV_REQUIRE(y && ys && n >= 0 && top_k > 0 && D > 0 && (!idx || h), "qsv_moe_combine_slots: bad arguments");
+    if (n == 0) return QSV_OK;
+    QSV_DISPATCH(dtype, "qsv_moe_combine_slots", (launch_combine<T, float>(y, ys, nullptr, weight, n, top_k, D, idx, h, n_experts, stream)));
+    return qsv_launch_status("qsv_moe_combine_slots");
 }
 
 extern "C" int qsv_moe_route(int32_t* idx, float* weight, const void* h, const void* router, const void* bias, int renorm, int n,
@@ -516,6 +859,17 @@ extern "C" int qsv_moe_route(int32_t* idx, float* weight, const void* h, const v
                     top_k <= keep * (E / G),
                 "qsv_moe_route: %d experts in %d groups, %d groups kept, top %d", E, G, keep, top_k);
     if (n == 0) return QSV_OK;
+    if (E <= 64 && D % 8 == 0) {
+#define QSV_ROUTE(TT)                                                                                                            \
+    QSV_DISPATCH(dtype, "qsv_moe_route",                                                                                         \
+                 hipLaunchKernelGGL((moe_route_wave_kernel<T, TT>), dim3((n + TT - 1) / TT), dim3(NT), 0, (hipStream_t)stream, idx, weight, \
+                                    (const T*)h, (const T*)router, (const T*)bias, renorm, n, D, E, top_k, G, keep, score_fn, correction, \
+                                    group_top, scale))
+        if (n >= 1024) QSV_ROUTE(4);
+        else QSV_ROUTE(1);
+#undef QSV_ROUTE
+        return qsv_launch_status("qsv_moe_route");
+    }
     QSV_DISPATCH(dtype, "qsv_moe_route",
                  hipLaunchKernelGGL(moe_route_kernel<T>, dim3(n), dim3(NT), 0, (hipStream_t)stream, idx, weight, (const T*)h,
                                     (const T*)router, (const T*)bias, renorm, D, E, top_k, G, keep, score_fn, correction,

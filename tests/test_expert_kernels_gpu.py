@@ -1,0 +1,111 @@
+"""The expert-major products and the one-expert-per-lane router at the edges of their tiles, against float64."""
+import pytest
+import torch
+
+from qserve_amd.layers.ops import make_ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _silu(x):
+    return x * torch.sigmoid(x)
+
+
+@pytest.fixture(scope="module")
+def ops():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return make_ops("hip", torch.bfloat16, torch.device("cuda:0"))
+
+
+# tokens, top, experts, identity outputs, width, ff: tiles of 32 weight rows, stages of 64 elements in four waves, chunks of 16 and 32
+# slots, windows of 1024 slots
+@pytest.mark.parametrize("T, top, E, ident, D, ff", [
+    (1, 1, 1, 0, 8, 8), (1, 4, 16, 0, 2048, 1408), (2, 2, 3, 2, 72, 40), (3, 4, 5, 0, 64, 32), (16, 1, 1, 0, 200, 24), (17, 1, 1, 0, 264, 33 * 8),
+    (32, 1, 1, 0, 4096, 16), (33, 1, 2, 0, 16, 4096), (70, 2, 4, 1, 520, 136), (64, 4, 16, 0, 2048, 96), (300, 4, 6, 1, 56, 64)])
+@pytest.mark.parametrize("act, weigh", [("relu_sq", "output"), ("swiglu", "input"), ("clamped_glu", "output")])
+def test_expert_major_form(ops, T, top, E, ident, D, ff, act, weigh):
+    g = torch.Generator().manual_seed(T * 131 + D)
+    dev, gated = "cuda:0", act != "relu_sq"
+    h = torch.randn(T + 1, D, generator=g).bfloat16()
+    up = (torch.randn(E, 2 * ff if gated else ff, D, generator=g) / D ** 0.5).bfloat16()
+    down = (torch.randn(E, D, ff, generator=g) / ff ** 0.5).bfloat16()
+    idx = torch.rand(T, E + ident, generator=g).argsort(dim=1)[:, :top].int()
+    if T > 4:
+        idx[: T // 2, 0] = 0                                            # one crowded expert
+        idx[:, 1:][idx[:, 1:] == 0] = E + ident - 1
+    wt = torch.rand(T, top, generator=g)
+    limit = 1.0 if act == "clamped_glu" else 0.0
+    o = make_ops("hip", torch.bfloat16, torch.device(dev))
+    o.moe_expert_major_slots = 10 ** 9
+    hd = h.to(dev)[1:] if T % 2 else h[1:].to(dev)                      # (also a view that starts inside a row of 16 bytes for narrow widths)
+    y = o.moe_experts(hd, up.to(dev), down.to(dev), idx.to(dev), wt.to(dev), act=act, limit=limit, weigh=weigh).double().cpu()
+    x, ref, size = h[1:].double(), torch.zeros(T, D, dtype=torch.float64), torch.zeros(T, D, dtype=torch.float64)
+    for e in range(E + ident):
+        t, k = (idx == e).nonzero(as_tuple=True)
+        if not len(t):
+            continue
+        w = wt[t, k].double()[:, None]
+        if e >= E:
+            v = x[t] * (w if weigh == "output" else 1.0)
+        else:
+            a = (x[t] @ up[e].double().T) * (w if weigh == "input" else 1.0)
+            if act == "relu_sq":
+                a = torch.relu(a) ** 2
+            elif act == "swiglu":
+                a = _silu(a[:, 0::2]) * a[:, 1::2]
+            else:
+                p, q = a[:, 0::2].clamp(max=limit), a[:, 1::2].clamp(-limit, limit)
+                a = p * torch.sigmoid(1.702 * p) * (q + 1.0)
+            v = (a @ down[e].double().T) * (w if weigh == "output" else 1.0)
+            # the activations are stored in bfloat16 (relative 2^-9 each, independent): error of the second product
+            size.index_add_(0, t, (a.pow(2) @ down[e].double().pow(2).T) * (w * w if weigh == "output" else 1.0))
+        ref.index_add_(0, t, v)
+    bound = 2.0 ** -8 * ref.abs() + 6 * 2.0 ** -9 * size.sqrt() + 1e-5
+    assert ((y - ref).abs() <= bound).all(), ((y - ref).abs() / bound).max()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n", [1, 5, 1023, 1025])
+@pytest.mark.parametrize("E, G, keep, top, D, score, group_top, renorm", [
+    (1, 1, 1, 1, 8, "softmax", 1, False), (16, 4, 2, 4, 2048, "softmax", 1, False), (16, 1, 1, 4, 2040, "softmax", 1, True),
+    (17, 17, 5, 3, 64, "sigmoid", 1, False), (64, 8, 3, 24, 4096, "sigmoid", 2, True), (33, 1, 1, 33, 136, "sigmoid", 1, False),
+    (64, 64, 64, 6, 8, "softmax", 1, False)])
+def test_router(dtype, n, E, G, keep, top, D, score, group_top, renorm):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    dev = torch.device("cuda:0")
+    o = make_ops("hip", dtype, dev)
+    g = torch.Generator().manual_seed(n + E)
+    h, r = torch.randn(n, D, generator=g).to(dtype), (torch.randn(E, D, generator=g) / D ** 0.5 * 2).to(dtype)
+    corr = torch.randn(E, generator=g) * 0.1
+    idx, wt = o.moe_route(h.to(dev), r.to(dev), top, G, keep, score=score, correction=corr.to(dev), group_top=group_top, renorm=renorm, scale=1.5)
+    idx, wt = idx.cpu().long(), wt.cpu().double()
+    z = h.double() @ r.double().T
+    s = torch.softmax(z, -1) if score == "softmax" else torch.sigmoid(z)
+    c = s + corr.double()
+    best = c.view(n, G, E // G).sort(-1, descending=True).values[..., :group_top].sum(-1)
+    kept = torch.zeros(n, G, dtype=torch.bool).scatter_(1, best.topk(keep, -1).indices, True)
+    c = c.masked_fill(~kept.repeat_interleave(E // G, 1), -9.0)
+    tol = 4e-6                                                          # float sums of D products of order one
+    # every chosen expert is eligible and the k-th of them is as good as the k-th best, up to float rounding of the scores
+    got = c.gather(1, idx)
+    assert (idx.sort(1).values.diff(dim=1) > 0).all() and ((got - c.topk(top, -1).values).abs() <= tol).all()
+    w = s.gather(1, idx)
+    w = (w / w.sum(-1, keepdim=True) if renorm else w) * 1.5
+    assert ((wt - w).abs() <= 4 * tol).all()
+
+
+def test_router_takes_what_is_not_a_number_last_and_ties_by_index():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    dev = torch.device("cuda:0")
+    o = make_ops("hip", torch.float32, dev)
+    h = torch.zeros(1, 8)
+    h[0, 0] = 1.0
+    r = torch.zeros(6, 8)
+    r[:, 0] = torch.tensor([0.0, -0.0, 2.0, float("nan"), 2.0, float("-inf")])
+    idx, _ = o.moe_route(h.to(dev), r.to(dev), 6, 1, 1, score="sigmoid")
+    assert idx.cpu()[0].tolist() == [2, 4, 0, 1, 5, 3]
+    idx, _ = o.moe_route(torch.full_like(h, float("nan")).to(dev), r.to(dev), 3, 3, 2)
+    assert sorted(set(idx.cpu()[0].tolist())) == sorted(idx.cpu()[0].tolist()) and idx.min() >= 0 and idx.max() < 6

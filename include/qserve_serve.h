@@ -235,18 +235,22 @@ int qsv_expert_rows(void* out, const void* X, const int64_t* x_index, int div, c
  * QSV_ACT_NONE only): out is float. */
 int qsv_expert_slots(void* out, int float_out, const void* X, int div, const void* W, const int32_t* idx, int n, int n_experts, int rows, int K,
                      int act, float limit, const float* in_weight, void* stream);
-/* Grouped expert product on the bf16 matrix cores (prompt phase): the same out[s, n] for work tiles (expert, first sorted slot,
- * slots <= qsv_grouped_gemm_tile_slots()) listed in tiles int32 [n_tiles, 3]; K a multiple of qsv_grouped_gemm_k_step(), n_rows
- * a multiple of 4, n_tiles <= 65535.  act: QSV_ACT_* (QSV_ACT_GLU: out is n_rows / 2 wide). */
-int qsv_grouped_gemm_tile_slots(void);
-int qsv_grouped_gemm_k_step(void);
-int qsv_grouped_gemm(void* out, const void* X, const int64_t* x_index, int div, const void* W, const int32_t* tiles,
-                     int n_tiles, int n_rows, int K, int act, float limit, const float* in_weight, void* stream);
+/* Grouped expert product on the bf16 matrix cores (prompt phase): qsv_moe_sort orders the n slots by expert (order: sorted slot -> slot,
+ * place: slot -> sorted slot, offsets [n_experts + 1]: first sorted slot of every expert; indices from n_experts on are left out of all
+ * three), and the product takes those: out[s, r] = act(W[e][r, :] . X[order ? order[s] / div : s, :]) for the sorted slots of every expert
+ * e, the input times in_weight[order ? order[s] : s] if given.  act: QSV_ACT_* (QSV_ACT_GLU: out is n_rows / 2 wide).  n_rows a multiple of
+ * 4, K a multiple of 64, at most 1024 experts (_ok). */
+int qsv_moe_sort(int32_t* order, int32_t* place, int32_t* offsets, const int32_t* idx, int n, int n_experts, void* stream);
+int qsv_grouped_gemm_sorted_ok(int n_experts, int n_rows, int K);
+int qsv_grouped_gemm_sorted(void* out, const void* X, const int32_t* order, int div, const void* W, const int32_t* offsets, int n_experts,
+                            int n_rows, int K, int act, float limit, const float* in_weight, void* stream);
 int qsv_gather_rows(void* out, const void* src, const int64_t* order, int div, int n_rows, int width, int dtype, void* stream);
 int qsv_relu_sq(void* a, int64_t n, int dtype, void* stream);
 /* (idx != NULL: slots with idx[t, k] >= n_experts take h[t] in place of a sorted row) */
 int qsv_moe_combine(void* y, const void* ys, const int64_t* inv, const float* weight, int n_tokens, int top_k, int width,
                     const int32_t* idx, const void* h, int n_experts, int dtype, void* stream);
+int qsv_moe_combine_sorted(void* y, const void* ys, const int32_t* place, const float* weight, int n_tokens, int top_k, int width,
+                           const int32_t* idx, const void* h, int n_experts, int dtype, void* stream);
 /* The same over float rows in slot order: y[t] = sum_k weight[t, k] * ys[t * top_k + k]. */
 int qsv_moe_combine_slots(void* y, const float* ys, const float* weight, int n_tokens, int top_k, int width, const int32_t* idx, const void* h,
                           int n_experts, int dtype, void* stream);

@@ -749,8 +749,8 @@ __global__ __launch_bounds__(NT) void relu_sq_kernel(T* __restrict__ a, size_t n
     }
 }
 // y[t] = sum_k weight[t, k] * ys[inv ? inv[t top_k + k] : t top_k + k]   (weight NULL: ones).  VEC coordinates per thread.
-template <typename T, typename Y, int VEC>
-__global__ __launch_bounds__(NT) void moe_combine_kernel(T* __restrict__ y, const Y* __restrict__ ys, const int64_t* __restrict__ inv,
+template <typename T, typename Y, int VEC, typename I>
+__global__ __launch_bounds__(NT) void moe_combine_kernel(T* __restrict__ y, const Y* __restrict__ ys, const I* __restrict__ inv,
                                                          const float* __restrict__ weight, int top_k, int D,
                                                          const int32_t* __restrict__ idx, const T* __restrict__ h, int n_experts) {
     const size_t t = blockIdx.x;
@@ -763,7 +763,7 @@ __global__ __launch_bounds__(NT) void moe_combine_kernel(T* __restrict__ y, cons
             const float wk = weight ? weight[slot] : 1.0f;
             float v[VEC];
             if (same) loadv(h + t * D + c, v);
-            else loadv(ys + (size_t)(inv ? inv[slot] : (int64_t)slot) * D + c, v);
+            else loadv(ys + (inv ? (size_t)inv[slot] : slot) * D + c, v);
 #pragma unroll
             for (int q = 0; q < VEC; ++q) a[q] += wk * v[q];
         }
@@ -821,31 +821,38 @@ extern "C" int qsv_relu_sq(void* a, int64_t n, int dtype, void* stream) {
     return qsv_launch_status("qsv_relu_sq");
 }
 // (four coordinates per thread where the rows' starts allow it; few tokens: a token's row over several workgroups)
-template <typename T, typename Y>
-static void launch_combine(void* y, const void* ys, const int64_t* inv, const float* weight, int n, int top_k, int D, const int32_t* idx,
+template <typename T, typename Y, typename I>
+static void launch_combine(void* y, const void* ys, const I* inv, const float* weight, int n, int top_k, int D, const int32_t* idx,
                            const void* h, int n_experts, void* stream) {
     const bool vec = D % 4 == 0 && ((uintptr_t)ys % (4 * sizeof(Y)) == 0) && ((uintptr_t)y % (4 * sizeof(T)) == 0) && (!h || (uintptr_t)h % (4 * sizeof(T)) == 0);
     const int per = NT * (vec ? 4 : 1), need = (D + per - 1) / per;
     const dim3 grid(n, n < 1024 ? need : 1);
     if (vec)
-        hipLaunchKernelGGL((moe_combine_kernel<T, Y, 4>), grid, dim3(NT), 0, (hipStream_t)stream, (T*)y, (const Y*)ys, inv, weight, top_k, D, idx,
+        hipLaunchKernelGGL((moe_combine_kernel<T, Y, 4, I>), grid, dim3(NT), 0, (hipStream_t)stream, (T*)y, (const Y*)ys, inv, weight, top_k, D, idx,
                            (const T*)h, n_experts);
     else
-        hipLaunchKernelGGL((moe_combine_kernel<T, Y, 1>), grid, dim3(NT), 0, (hipStream_t)stream, (T*)y, (const Y*)ys, inv, weight, top_k, D, idx,
+        hipLaunchKernelGGL((moe_combine_kernel<T, Y, 1, I>), grid, dim3(NT), 0, (hipStream_t)stream, (T*)y, (const Y*)ys, inv, weight, top_k, D, idx,
                            (const T*)h, n_experts);
 }
 extern "C" int qsv_moe_combine(void* y, const void* ys, const int64_t* inv, const float* weight, int n, int top_k, int D,
                                const int32_t* idx, const void* h, int n_experts, int dtype, void* stream) {
     QSV_REQUIRE(y && ys && inv && n >= 0 && top_k > 0 && D > 0 && (!idx || h), "qsv_moe_combine: bad arguments");
     if (n == 0) return QSV_OK;
-    QSV_DISPATCH(dtype, "qsv_moe_combine", (launch_combine<T, T>(y, ys, inv, weight, n, top_k, D, idx, h, n_experts, stream)));
+    QSV_DISPATCH(dtype, "qsv_moe_combine", (launch_combine<T, T, int64_t>(y, ys, inv, weight, n, top_k, D, idx, h, n_experts, stream)));
     return qsv_launch_status("qsv_moe_combine");
+}
+extern "C" int qsv_moe_combine_sorted(void* y, const void* ys, const int32_t* place, const float* weight, int n, int top_k, int D, const int32_t* idx,
+                                      const void* h, int n_experts, int dtype, void* stream) {
+    QSV_REQUIRE(y && ys && place && n >= 0 && top_k > 0 && D > 0 && (!idx || h), "qsv_moe_combine_sorted: bad arguments");
+    if (n == 0) return QSV_OK;
+    QSV_DISPATCH(dtype, "qsv_moe_combine_sorted", (launch_combine<T, T, int32_t>(y, ys, place, weight, n, top_k, D, idx, h, n_experts, stream)));
+    return qsv_launch_status("qsv_moe_combine_sorted");
 }
 extern "C" int qsv_moe_combine_slots(void* y, const float* ys, const float* weight, int n, int top_k, int D, const int32_t* idx, const void* h,
                                      int n_experts, int dtype, void* stream) {
     QSV_REQUIRE(y && ys && n >= 0 && top_k > 0 && D > 0 && (!idx || h), "qsv_moe_combine_slots: bad arguments");
     if (n == 0) return QSV_OK;
-    QSV_DISPATCH(dtype, "qsv_moe_combine_slots", (launch_combine<T, float>(y, ys, nullptr, weight, n, top_k, D, idx, h, n_experts, stream)));
+    QSV_DISPATCH(dtype, "qsv_moe_combine_slots", (launch_combine<T, float, int32_t>(y, ys, nullptr, weight, n, top_k, D, idx, h, n_experts, stream)));
     return qsv_launch_status("qsv_moe_combine_slots");
 }
 

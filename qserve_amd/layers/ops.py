@@ -698,6 +698,7 @@ class HipOps:
         expert's input, y[t] = sum_k down[..] a(up[..] (wt[t, k] h[t])) (the products' results are scaled, in float)."""
         T, D = h.shape
         top_k, rows = idx.size(1), up.size(1)
+        idx = idx.to(torch.int32).contiguous()
         a = self.ACTS[act]
         ff = rows // 2 if a >= 2 else rows
         if (self.code == BF16 and self.moe_token_slots < T * top_k <= self.moe_expert_major_slots and D % 8 == 0 and ff % 8 == 0
@@ -727,7 +728,8 @@ class HipOps:
     # one workgroup per token walks a whole product (one token at 2048 x 1408, 4 of 16 experts: 4.6 ms against 0.04 ms) - serve
     # float storage and widths the others do not take.
     moe_token_slots = 0
-    moe_expert_major_slots = 1024
+    # (crossover measured: 16 experts of 2048 x 1408 at 1000 (relu^2) and 850 slots (gated), 32 of 4096 x 2752 at 850)
+    moe_expert_major_slots = 896
 
     @staticmethod
     def _weights_at(wt, weigh):
@@ -772,27 +774,32 @@ class HipOps:
         E, rows, K = up.size(0), up.size(1), idx.size(1)
         ff = rows // 2 if code >= 2 else rows
         n = T * K
+        L = self.L
+        if (self.moe_grouped_kernel and self.code == BF16 and L.qsv_grouped_gemm_sorted_ok(E, rows, D) and L.qsv_grouped_gemm_sorted_ok(E, D, ff)
+                and up.data_ptr() % 16 == 0 and down.data_ptr() % 16 == 0):
+            # own grouped matrix-core kernel: gather in its loads, the activation in the first product's epilogue, tiles found on the device
+            if h.data_ptr() % 16:                                      # (a row view: the kernel copies 16-byte pieces)
+                h = h.clone()
+            self._need(h, up, down, idx, wt)
+            order, place = (torch.empty((n,), dtype=torch.int32, device=h.device) for _ in range(2))
+            offsets = torch.empty((E + 1,), dtype=torch.int32, device=h.device)
+            act = torch.empty((n, ff), dtype=self.dtype, device=h.device)
+            ys = torch.empty((n, D), dtype=self.dtype, device=h.device)
+            y = torch.empty((T, D), dtype=self.dtype, device=h.device)
+            s = self._s()
+            self.check(L.qsv_moe_sort(order.data_ptr(), place.data_ptr(), offsets.data_ptr(), idx.data_ptr(), n, E, s), "moe_sort")
+            self.check(L.qsv_grouped_gemm_sorted(act.data_ptr(), h.data_ptr(), order.data_ptr(), K, up.data_ptr(), offsets.data_ptr(), E, rows, D, code,
+                                                 float(limit), w_in, s), "grouped_gemm(up)")
+            self.check(L.qsv_grouped_gemm_sorted(ys.data_ptr(), act.data_ptr(), 0, 1, down.data_ptr(), offsets.data_ptr(), E, D, ff, 0, 0.0, 0, s),
+                       "grouped_gemm(down)")
+            self.check(L.qsv_moe_combine_sorted(y.data_ptr(), ys.data_ptr(), place.data_ptr(), w_out, T, K, D, idx.data_ptr(), h.data_ptr(), E,
+                                                self.code, s), "moe_combine_sorted")
+            return y
         flat = idx.reshape(-1)
         order = torch.argsort(flat, stable=True)                       # sorted slot -> slot (t K + k)
         counts = torch.bincount(flat, minlength=E).tolist()[:E]        # (host synchronisation: the runs' lengths; identity experts sort last)
         inv = torch.empty_like(order)
         inv[order] = torch.arange(n, device=h.device)                  # slot -> sorted slot
-        ks, ts = self.L.qsv_grouped_gemm_k_step(), self.L.qsv_grouped_gemm_tile_slots()
-        if self.moe_grouped_kernel and self.code == BF16 and D % ks == 0 and ff % ks == 0:
-            # own grouped matrix-core kernel: gather in its loads, the activation in the first product's epilogue
-            tiles, a = [], 0
-            for e, c in enumerate(counts):
-                tiles += [(e, a + o, min(ts, c - o)) for o in range(0, c, ts)]
-                a += c
-            act = torch.empty((n, ff), dtype=self.dtype, device=h.device)
-            ys = torch.empty((n, D), dtype=self.dtype, device=h.device)
-            for lo in range(0, len(tiles), 65535):
-                tl = torch.tensor(tiles[lo:lo + 65535], dtype=torch.int32).to(h.device)
-                self.check(self.L.qsv_grouped_gemm(act.data_ptr(), h.data_ptr(), order.data_ptr(), K, up.data_ptr(), tl.data_ptr(),
-                                                   tl.size(0), rows, D, code, float(limit), w_in, self._s()), "grouped_gemm(up)")
-                self.check(self.L.qsv_grouped_gemm(ys.data_ptr(), act.data_ptr(), 0, 1, down.data_ptr(), tl.data_ptr(),
-                                                   tl.size(0), D, ff, 0, 0.0, 0, self._s()), "grouped_gemm(down)")
-            return self._combine(h, ys, inv, idx, w_out, E)
         xs = torch.empty((n, D), dtype=self.dtype, device=h.device)
         self.check(self.L.qsv_gather_rows(xs.data_ptr(), h.data_ptr(), order.data_ptr(), K, n, D, self.code, self._s()),
                    "gather_rows")

@@ -18,13 +18,8 @@ def ops():
     return make_ops("hip", torch.bfloat16, torch.device("cuda:0"))
 
 
-# tokens, top, experts, identity outputs, width, ff: tiles of 32 weight rows, stages of 64 elements in four waves, chunks of 16 and 32
-# slots, windows of 1024 slots
-@pytest.mark.parametrize("T, top, E, ident, D, ff", [
-    (1, 1, 1, 0, 8, 8), (1, 4, 16, 0, 2048, 1408), (2, 2, 3, 2, 72, 40), (3, 4, 5, 0, 64, 32), (16, 1, 1, 0, 200, 24), (17, 1, 1, 0, 264, 33 * 8),
-    (32, 1, 1, 0, 4096, 16), (33, 1, 2, 0, 16, 4096), (70, 2, 4, 1, 520, 136), (64, 4, 16, 0, 2048, 96), (300, 4, 6, 1, 56, 64)])
-@pytest.mark.parametrize("act, weigh", [("relu_sq", "output"), ("swiglu", "input"), ("clamped_glu", "output")])
-def test_expert_major_form(ops, T, top, E, ident, D, ff, act, weigh):
+def check(o, T, top, E, ident, D, ff, act, weigh, crowd):
+    """crowd: about that share of the tokens has expert 0 first."""
     g = torch.Generator().manual_seed(T * 131 + D)
     dev, gated = "cuda:0", act != "relu_sq"
     h = torch.randn(T + 1, D, generator=g).bfloat16()
@@ -32,12 +27,10 @@ def test_expert_major_form(ops, T, top, E, ident, D, ff, act, weigh):
     down = (torch.randn(E, D, ff, generator=g) / ff ** 0.5).bfloat16()
     idx = torch.rand(T, E + ident, generator=g).argsort(dim=1)[:, :top].int()
     if T > 4:
-        idx[: T // 2, 0] = 0                                            # one crowded expert
+        idx[: int(T * crowd), 0] = 0
         idx[:, 1:][idx[:, 1:] == 0] = E + ident - 1
     wt = torch.rand(T, top, generator=g)
     limit = 1.0 if act == "clamped_glu" else 0.0
-    o = make_ops("hip", torch.bfloat16, torch.device(dev))
-    o.moe_expert_major_slots = 10 ** 9
     hd = h.to(dev)[1:] if T % 2 else h[1:].to(dev)                      # (also a view that starts inside a row of 16 bytes for narrow widths)
     y = o.moe_experts(hd, up.to(dev), down.to(dev), idx.to(dev), wt.to(dev), act=act, limit=limit, weigh=weigh).double().cpu()
     x, ref, size = h[1:].double(), torch.zeros(T, D, dtype=torch.float64), torch.zeros(T, D, dtype=torch.float64)
@@ -58,11 +51,38 @@ def test_expert_major_form(ops, T, top, E, ident, D, ff, act, weigh):
                 p, q = a[:, 0::2].clamp(max=limit), a[:, 1::2].clamp(-limit, limit)
                 a = p * torch.sigmoid(1.702 * p) * (q + 1.0)
             v = (a @ down[e].double().T) * (w if weigh == "output" else 1.0)
-            # the activations are stored in bfloat16 (relative 2^-9 each, independent): error of the second product
-            size.index_add_(0, t, (a.pow(2) @ down[e].double().pow(2).T) * (w * w if weigh == "output" else 1.0))
+            # the activations are stored in bfloat16 (relative 2^-9 each, independent), in the grouped form the experts' rows too
+            size.index_add_(0, t, (a.pow(2) @ down[e].double().pow(2).T) * (w * w if weigh == "output" else 1.0) + v.pow(2))
         ref.index_add_(0, t, v)
     bound = 2.0 ** -8 * ref.abs() + 6 * 2.0 ** -9 * size.sqrt() + 1e-5
     assert ((y - ref).abs() <= bound).all(), ((y - ref).abs() / bound).max()
+
+
+ACTS = pytest.mark.parametrize("act, weigh", [("relu_sq", "output"), ("swiglu", "input"), ("clamped_glu", "output")])
+
+
+# tokens, top, experts, identity outputs, width, ff: tiles of 32 weight rows, stages of 64 elements in four waves, chunks of 16 and 32
+# slots, windows of 1024 slots
+@pytest.mark.parametrize("T, top, E, ident, D, ff", [
+    (1, 1, 1, 0, 8, 8), (1, 4, 16, 0, 2048, 1408), (2, 2, 3, 2, 72, 40), (3, 4, 5, 0, 64, 32), (16, 1, 1, 0, 200, 24), (17, 1, 1, 0, 264, 33 * 8),
+    (32, 1, 1, 0, 4096, 16), (33, 1, 2, 0, 16, 4096), (70, 2, 4, 1, 520, 136), (64, 4, 16, 0, 2048, 96), (300, 4, 6, 1, 56, 64)])
+@ACTS
+def test_expert_major_form(ops, T, top, E, ident, D, ff, act, weigh):
+    o = make_ops("hip", torch.bfloat16, torch.device("cuda:0"))
+    o.moe_expert_major_slots = 10 ** 9
+    check(o, T, top, E, ident, D, ff, act, weigh, 0.5)
+
+
+# tiles of 256 rows x 256, 128 or 64 slots, K steps of 64 in two halves of the buffer; more tiles than workgroups; more experts than lanes
+@pytest.mark.parametrize("T, top, E, ident, D, ff, crowd", [
+    (1, 1, 1, 0, 64, 64, 0.0), (64, 1, 1, 0, 128, 64, 1.0), (65, 1, 1, 0, 64, 192, 1.0), (128, 1, 1, 0, 320, 128, 1.0), (129, 2, 3, 0, 256, 64, 1.0),
+    (256, 1, 2, 0, 64, 320, 1.0), (257, 1, 1, 0, 1088, 64, 1.0), (700, 4, 6, 2, 512, 448, 0.5), (1500, 4, 100, 5, 64, 64, 0.2), (40, 3, 70, 0, 4096, 64, 0.0),
+    (2100, 2, 2, 0, 4096, 128, 0.3)])
+@ACTS
+def test_grouped_form(ops, T, top, E, ident, D, ff, crowd, act, weigh):
+    o = make_ops("hip", torch.bfloat16, torch.device("cuda:0"))
+    o.moe_expert_major_slots, o.moe_sorted_above = 0, 0
+    check(o, T, top, E, ident, D, ff, act, weigh, crowd)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])

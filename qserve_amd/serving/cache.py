@@ -13,7 +13,17 @@ a token shift) lives in per-slot tensors, one per `StateSpec`:
   (`step_rows`).  For state that the step's FIRST token reads and its LAST token writes from different workgroups.
 A sequence's state is never cleared: kernels take a run that starts at position 0 as starting from zeros.
 """
+import numpy as np
 import torch
+
+
+def upload(a, device):
+    """numpy array -> tensor on `device`.  To a GPU through a pinned buffer and without waiting for the copy (torch hands a pinned buffer
+    out again only after the copies from it have run); a copy from pageable memory would wait for everything on the stream."""
+    t = torch.from_numpy(a)
+    if torch.device(device).type != "cuda":
+        return t.to(device)
+    return torch.empty(t.shape, dtype=t.dtype, pin_memory=True).copy_(t).to(device, non_blocking=True)
 
 
 class CacheFull(RuntimeError):
@@ -64,8 +74,8 @@ class PagedCache:
         self.pages[s], self.length[s] = [], 0
         return s
 
-    def extend(self, slot, n):
-        """Make room for n more tokens of `slot`; returns their flat row indices (position order)."""
+    def _grow(self, slot, n):
+        """Pages for n more tokens of `slot`.  -> (its pages, tokens it held before)."""
         have, start = self.pages[slot], self.length[slot]
         need = self.pages_for(start + n) - len(have)
         if need > len(self.free_pages):
@@ -76,7 +86,18 @@ class PagedCache:
             have.append(p)
             self._dirty = True
         self.length[slot] = start + n
+        return have, start
+
+    def extend(self, slot, n):
+        """Make room for n more tokens of `slot`; returns their flat row indices (position order)."""
+        have, start = self._grow(slot, n)
         return [have[j // self.page] * self.page + j % self.page for j in range(start, start + n)]
+
+    def extend_array(self, slot, n):
+        """`extend` for many tokens: the row indices as an int64 array."""
+        have, start = self._grow(slot, n)
+        j = np.arange(start, start + n, dtype=np.int64)
+        return np.array(have, dtype=np.int64)[j // self.page] * self.page + j % self.page
 
     def step_rows(self, slot):
         """-> (row to read, row to write) of the two-copy states for this step of `slot`; the next step reads what this one
@@ -93,6 +114,9 @@ class PagedCache:
     def block_table(self):
         """The device copy of the block table, uploaded if pages were handed out since the last call."""
         if self._dirty:
-            self.table.copy_(self.table_host)
+            if self.table.is_cuda:                                     # (a pinned copy: the host's table may change before the device has read it)
+                self.table.copy_(torch.empty(self.table_host.shape, dtype=torch.int32, pin_memory=True).copy_(self.table_host), non_blocking=True)
+            else:
+                self.table.copy_(self.table_host)
             self._dirty = False
         return self.table

@@ -8,11 +8,12 @@ use `open_sequence` / `execute` / `close_sequence` directly and so drive the ver
 import itertools
 from dataclasses import dataclass, field
 
+import numpy as np
 import torch
 
 from ..layers.ops import make_ops
 from . import registry
-from .cache import PagedCache
+from .cache import PagedCache, upload
 from .sampler import SamplingParams, sample
 from .scheduler import Request, Scheduler
 
@@ -35,6 +36,7 @@ class StepBatch:
     state_wr: torch.Tensor = None   # int32 [T]  two-copy state row to write, on the LAST token of a run (-1 elsewhere)
     _tiles: dict = field(default_factory=dict)
     _runs: torch.Tensor = None
+    _single: torch.Tensor = None    # int32 [T, 3] = (slot, token, 1) where every run is one token: the tiles of any size
 
     def runs(self):
         """int32 [n_runs, 4] = (sequence slot, first flat token index, tokens, position of the first token), on the device.
@@ -48,23 +50,27 @@ class StepBatch:
     def tiles(self, tokens_per_tile):
         """Work tiles for kernels that serve a few consecutive tokens of one sequence per workgroup: int32 [n, 3] =
         (sequence slot, first flat token index, tokens <= tokens_per_tile), on the device; cached per size."""
+        if self._single is not None:
+            return self._single
         t = self._tiles.get(tokens_per_tile)
         if t is None:
             rows = [(slot, first + o, min(tokens_per_tile, n - o)) for slot, first, n in self.items
                     for o in range(0, n, tokens_per_tile)]
-            t = torch.tensor(rows, dtype=torch.int32).reshape(-1, 3).to(self.tokens.device if self.tokens is not None else self.pos.device)
+            t = upload(np.array(rows, dtype=np.int32).reshape(-1, 3), self.tokens.device if self.tokens is not None else self.pos.device)
             self._tiles[tokens_per_tile] = t
         return t
 
     def split_tiles(self, tokens_per_step_tile):
         """Work tiles for kernels with a form of their own for short runs: -> (prompt tiles, step tiles), int32 [n, 3] as `tiles`.  Runs of at
         most `tokens_per_step_tile` tokens become one step tile each, longer ones prompt tiles of up to four times as many tokens."""
+        if self._single is not None:
+            return self._single[:0], self._single
         n = int(tokens_per_step_tile)
         key = ("split", n)
         if key not in self._tiles:
             short = [run for run in self.items if run[2] <= n]
             long = [(slot, first + o, min(4 * n, cnt - o)) for slot, first, cnt in self.items if cnt > n for o in range(0, cnt, 4 * n)]
-            both = torch.tensor(short + long, dtype=torch.int32).reshape(-1, 3).to(self.pos.device)
+            both = upload(np.array(short + long, dtype=np.int32).reshape(-1, 3), self.pos.device)
             self._tiles[key] = both
         both, k = self._tiles[key], sum(1 for run in self.items if run[2] <= n)
         return both[k:], both[:k]
@@ -107,47 +113,67 @@ class Engine:
     def close_sequence(self, slot):
         self.cache.release(slot)
 
+    def _token_ids(self, t):
+        """The tokens of one run as an int64 array, checked against the vocabulary."""
+        a = np.array(t) if isinstance(t, (list, tuple)) else None
+        if a is None or a.dtype != np.int64 or a.ndim != 1:
+            ids = [int(v) for v in t]
+            if any(not 0 <= v < self.model.vocab for v in ids):
+                raise ValueError(f"token id outside the vocabulary of {self.model.vocab}")
+            return np.array(ids, dtype=np.int64)
+        if a.size and (a.min() < 0 or a.max() >= self.model.vocab):
+            raise ValueError(f"token id outside the vocabulary of {self.model.vocab}")
+        return a
+
     def _layout_host(self, items):
-        """Host side of a step's batch: extends the sequences' pages, swaps their two-copy states.  -> (meta int32 [6, T] =
-        token, slot, position, index in run, state row to read, state row to write; flat cache rows; runs) or None."""
-        toks, seq, pos, rows, runs, off, rd, wr = [], [], [], [], [], [], [], []
-        V = self.model.vocab
+        """Host side of a step's batch: extends the sequences' pages, swaps their two-copy states.  -> (everything the device needs as one
+        int32 array, see `_batch_of`; runs [(slot, first flat token, tokens)]; largest position) or None."""
         if len({slot for slot, t in items if len(t)}) != sum(1 for _, t in items if len(t)):
             raise ValueError("a sequence appears twice in one step")
+        cache, runs, cols, T, max_pos = self.cache, [], [], 0, 0
         for slot, t in items:
-            start, n = self.cache.length[slot], len(t)
-            if any(not 0 <= int(v) < V for v in t):
-                raise ValueError(f"token id outside the vocabulary of {V}")
+            start, n = cache.length[slot], len(t)
+            ids = self._token_ids(t)
             if not n:
                 continue
-            runs.append((slot, len(toks), n))
-            rows += self.cache.extend(slot, n)
-            toks += [int(v) for v in t]
-            seq += [slot] * n
-            pos += range(start, start + n)
-            r, w = self.cache.step_rows(slot)
-            off += range(n)
-            rd += [r if start else -1] * n
-            wr += [-1] * (n - 1) + [w]
-        if not toks:
+            rows = cache.extend(slot, 1) if n == 1 else cache.extend_array(slot, n)
+            runs.append((slot, T, n))
+            cols.append((ids, start, rows, *cache.step_rows(slot)))
+            T, max_pos = T + n, max(max_pos, start + n - 1)
+        if not runs:
             return None
-        return torch.tensor([toks, seq, pos, off, rd, wr], dtype=torch.int32), rows, runs
+        R, single = len(runs), T == len(runs)
+        flat = np.empty(8 * T + (7 if single else 4) * R, dtype=np.int32)
+        row_of, meta, runs4 = flat[:2 * T].view(np.int64), flat[2 * T:8 * T].reshape(6, T), flat[8 * T:8 * T + 4 * R].reshape(R, 4)
+        runs4[:] = [(slot, first, n, c[1]) for (slot, first, n), c in zip(runs, cols)]
+        if single:
+            row_of[:] = [c[2][0] for c in cols]
+            meta[:] = [[int(c[0][0]) for c in cols], [r[0] for r in runs], [c[1] for c in cols], [0] * T,
+                       [c[3] if c[1] else -1 for c in cols], [c[4] for c in cols]]
+            tiles = flat[8 * T + 4 * R:].reshape(R, 3)
+            tiles[:, :2], tiles[:, 2] = runs4[:, :2], 1
+        else:
+            for (slot, first, n), (ids, start, rows, rd, wr) in zip(runs, cols):
+                s = slice(first, first + n)
+                row_of[s], meta[0, s], meta[1, s] = rows, ids, slot
+                meta[2, s], meta[3, s] = np.arange(start, start + n), np.arange(n)
+                meta[4, s], meta[5, s], meta[5, first + n - 1] = rd if start else -1, -1, wr
+        return flat, runs, max_pos
 
     def layout(self, items):
         """items: [(slot, tokens)] -> the StepBatch of these tokens on the device (None if there are none).  Part of `execute`;
         callers that run single layers use it directly."""
         host = self._layout_host(items)
-        return None if host is None else self._to_device(*host)
+        return None if host is None else self._batch_of(upload(host[0], self.device), *host[1:])
 
-    def _to_device(self, meta, rows, runs):
-        dev = self.device
-        max_pos, T = int(meta[2].max()), meta.size(1)
-        runs4 = torch.tensor([(s, first, n, int(meta[2, first])) for s, first, n in runs], dtype=torch.int32)
-        flat = torch.cat([meta.reshape(-1), runs4.reshape(-1)]).to(dev)      # (one host tensor, one copy)
-        meta = flat[:6 * T].view(6, T)
-        return StepBatch(tokens=meta[0], seq=meta[1], pos=meta[2], slot=torch.tensor(rows, dtype=torch.int64).to(dev),
-                         block_table=self.cache.block_table(), max_pos=max_pos, n_tokens=T, items=runs,
-                         run_off=meta[3], state_rd=meta[4], state_wr=meta[5], _runs=flat[6 * T:].view(-1, 4))
+    def _batch_of(self, flat, runs, max_pos):
+        """The StepBatch over one int32 tensor: cache rows (int64 [T]) | token, slot, position, index in run, state row to read, state row to
+        write ([6, T]) | runs ([R, 4]) | the tiles of single tokens ([R, 3], where every run is one)."""
+        T, R = sum(n for _, _, n in runs), len(runs)
+        meta = flat[2 * T:8 * T].view(6, T)
+        return StepBatch(tokens=meta[0], seq=meta[1], pos=meta[2], slot=flat[:2 * T].view(torch.int64), block_table=self.cache.block_table(),
+                         max_pos=max_pos, n_tokens=T, items=list(runs), run_off=meta[3], state_rd=meta[4], state_wr=meta[5],
+                         _runs=flat[8 * T:8 * T + 4 * R].view(R, 4), _single=flat[8 * T + 4 * R:].view(R, 3) if T == R else None)
 
     @torch.no_grad()
     def execute(self, items, want):
@@ -156,15 +182,18 @@ class Engine:
         host = self._layout_host(items)
         if host is None:
             return None
-        if self.decode_graphs and all(n == 1 for _, _, n in host[2]):
+        if self.decode_graphs and all(n == 1 for _, _, n in host[1]):
             out = self._execute_graph(*host)
             if out is not None:
-                return out[torch.tensor(list(want), dtype=torch.int64, device=self.device)] if want else None
-        batch = self._to_device(*host)
+                if not want:
+                    return None
+                want = list(want)
+                return out.clone() if want == list(range(out.size(0))) else out[upload(np.array(want, dtype=np.int64), self.device)]
+        batch = self._batch_of(upload(host[0], self.device), *host[1:])
         x = self._forward(batch)
         if not want:
             return None
-        return self.model.logits(x, torch.tensor(list(want), dtype=torch.int32).to(self.device))
+        return self.model.logits(x, upload(np.array(list(want), dtype=np.int32), self.device))
 
     def _forward(self, batch):
         if self.cache.states:
@@ -174,27 +203,21 @@ class Engine:
     # ---- decode steps from a hipGraph ------------------------------------------------------------------------------------------
     GRAPH_BUCKET = 128                         # positions per context bucket (a graph freezes what is derived from max_pos)
 
-    def _execute_graph(self, meta, rows, runs):
-        """One token per sequence: fill the static inputs of the graph captured for (batch size, context bucket, model
-        signature) and replay it.  -> float logits for every row, or None if this shape runs eagerly."""
-        B, dev = meta.size(1), self.device
-        bucket = int(meta[2].max()) // self.GRAPH_BUCKET
+    def _execute_graph(self, flat, runs, max_pos):
+        """One token per sequence: fill the static input of the graph captured for (batch size, context bucket, model
+        signature) and replay it.  -> float logits for every row (the graph's own buffer), or None if this shape runs eagerly."""
+        B, dev = len(runs), self.device
+        bucket = max_pos // self.GRAPH_BUCKET
         sig = self.model.graph_signature() if hasattr(self.model, "graph_signature") else ()
         key = (B, bucket, sig)
         G = self._graphs.get(key)
         if G is False:
             return None
-        slot = torch.tensor(rows, dtype=torch.int64)
-        runs4 = torch.tensor([(s, first, n, int(meta[2, first])) for s, first, n in runs], dtype=torch.int32).reshape(-1, 4)
         if G is None:
             if len(self._graphs) >= 16:
                 self._graphs.clear()
-            batch = StepBatch(tokens=None, seq=None, pos=None, slot=slot.to(dev), block_table=self.cache.block_table(),
-                              max_pos=(bucket + 1) * self.GRAPH_BUCKET - 1, n_tokens=B, items=list(runs))
-            m = meta.to(dev)
-            batch.tokens, batch.seq, batch.pos, batch.run_off, batch.state_rd, batch.state_wr = m[0], m[1], m[2], m[3], m[4], m[5]
-            batch._runs = runs4.to(dev)
-            G = {"meta": m, "batch": batch, "rows": torch.arange(B, dtype=torch.int32, device=dev)}
+            G = {"flat": upload(flat, dev), "rows": torch.arange(B, dtype=torch.int32, device=dev)}
+            G["batch"] = batch = self._batch_of(G["flat"], runs, (bucket + 1) * self.GRAPH_BUCKET - 1)
             if hasattr(self.model, "reserve_positions"):
                 self.model.reserve_positions(batch.max_pos + 1)
                 key = (B, bucket, self.model.graph_signature() if hasattr(self.model, "graph_signature") else ())
@@ -217,12 +240,8 @@ class Engine:
                 self._graphs[key] = False
                 return None
             self._graphs[key] = G
-        batch = G["batch"]
-        G["meta"].copy_(meta)
-        batch.slot.copy_(slot)
-        batch._runs.copy_(runs4)
-        for tpb, t in batch._tiles.items():
-            t.copy_(torch.tensor([(s, first, 1) for s, first, _ in runs], dtype=torch.int32).reshape(-1, 3))
+        else:
+            G["flat"].copy_(torch.empty(flat.shape, dtype=torch.int32, pin_memory=True).copy_(torch.from_numpy(flat)), non_blocking=True)
         self.cache.block_table()
         G["graph"].replay()
         return G["logits"]

@@ -151,6 +151,13 @@ int qsv_latent_attention_mfma(void* out, const float* qf, const void* pool, cons
                               int q_first, int heads_per_pool, int64_t pool_stride, int chunk, const float* bias, int bias_len,
                               int keep_first, const float* sink, const void* pooled, int64_t pooled_stride, int pool_block,
                               int block_rows, const float* slopes, void* stream);
+/* The same for plain causal or windowed scores at exact sizes (_ok: row width / rank 576 / 512, 512 / 512, 256 / 128, bfloat16, pages of a
+ * multiple of 32): no options, tiles of at most qsv_latent_rows_tile_tokens(heads per pool) tokens. */
+int qsv_latent_rows_ok(int rank, int row_width, int page, int dtype);
+int qsv_latent_rows_tile_tokens(int heads);
+int qsv_latent_rows(void* out, const float* qf, const void* pool, const int32_t* block_table, int table_stride, const int32_t* pos,
+                    const int32_t* tiles, int n_tiles, int window, int heads, int rank, int row_width, int page, int key_splits, float* part_o,
+                    float* part_ml, int n_tokens, int q_first, int heads_per_pool, int64_t pool_stride, void* stream);
 
 /* ---- talking-heads attention (serve_talking.hip) ------------------------------------------------------------------------------
  * score(t, h, j) = qf[t, h] . k[kv(h), j], cap > 0: cap tanh(score / cap); w_h = softmax over max(0, pos - window + 1) <= j <= pos (window

@@ -311,6 +311,206 @@ __global__ __launch_bounds__(64 * NWV, (RT > 10 ? 1 : 2)) void latent_attention_
     }
 }
 
+// ---- plain rows (causal or windowed, nothing else on the scores) of exact sizes: R = 32 RT a multiple of 64, rank = 16 CT a multiple of 64 ----
+// The kernel above stages a key tile through registers and writes it twice, the second time transposed in 2-byte pieces; at 576-wide rows
+// that and 74 KB of code were its time (143 TFLOP/s in a prompt, 47 us for a step of 100 positions).  Here a tile is copied straight into
+// LDS as it lies in memory (32 rows of one page are contiguous), once, the 16-byte pieces of a row permuted by the row's number, two
+// tiles in turn with one barrier each; K is read from it row by row and V through the transposing read (ds_read_b64_tr_b16).  Eight waves
+// of 16 query rows (one token of 16 heads, or several of fewer).  Bound by the LDS reads: a wave reads the whole tile for its 16 rows.
+// Measured (MI355X): 8 prompts of 1024, 16 heads, 576 / 512: 1004 -> 335 us; 512 / 512: 973 -> 315 us; 256 / 128, 32 heads on 8 pools: 484 -> 242 us; steps
+// of 64 sequences at 100 / 1000 / 4000 positions, 576 / 512: 41 / 69 / 200 -> 15 / 31 / 71 us, 256 / 128, 16 heads on 4 pools: 15 / 45 / 135 -> 13 / 26 / 95 us.
+constexpr int RW = 8;
+typedef short s4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s4* lds_s4;
+typedef __attribute__((address_space(3))) void* lds_ptr;
+
+// (eight neighbouring rows: eight different pieces for the key reads; four: four different pairs for the transposing value reads)
+__device__ __forceinline__ int row_turn(int row) { return ((row & 3) << 1) | ((row >> 2) & 1); }
+
+// S0: every query is zero before element 32 S0
+template <int RT, int CT, int S0>
+__global__ __launch_bounds__(64 * RW, RT + CT > 24 ? 2 : 4) void latent_rows_kernel(
+    bf16_t* __restrict__ out, const float* __restrict__ qf, const bf16_t* __restrict__ pool_base, const int32_t* __restrict__ block_table,
+    int table_stride, const int32_t* __restrict__ pos, const int32_t* __restrict__ tiles, int n_tiles, int window, int H, int page, int HP, int TQ,
+    float* __restrict__ part_o, float* __restrict__ part_ml, int n_tokens, int per, int64_t pool_stride) {
+    constexpr int R = 32 * RT, RANK = 16 * CT, PPR = R / 8, TILE = BN * R * 2, NJ = (BN * PPR / 64 + RW - 1) / RW;
+    static_assert(R % 64 == 0 && RANK % 64 == 0, "");
+    __shared__ __attribute__((aligned(128))) unsigned char buf[2 * TILE];
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6) & (RW - 1);
+    const int col = lane & 15, g4 = lane >> 4;
+    const int32_t* tl = tiles + 3 * (n_tiles - 1 - (int)blockIdx.x);            // (a sequence's longest first)
+    const int slot = __builtin_amdgcn_readfirstlane(tl[0]), t0 = __builtin_amdgcn_readfirstlane(tl[1]), ntok = __builtin_amdgcn_readfirstlane(tl[2]);
+    const int gpp = (per + 15) / 16, pool_id = blockIdx.y / gpp;
+    const int h0 = pool_id * per + (blockIdx.y % gpp) * 16, h_end = pool_id * per + per;
+    const bf16_t* __restrict__ pool = pool_base + (size_t)pool_id * (size_t)pool_stride;
+    const int32_t* bt = block_table + (size_t)slot * table_stride;
+    const bool active = w * TQ < ntok;                                          // this wave has tokens
+    const int tok_in = w * TQ + col / HP, head = h0 + col % HP;
+    const bool row_ok = tok_in < ntok && head < h_end;
+    const int t = t0 + min(tok_in, ntok - 1);
+    // (tokens of a tile are consecutive positions)
+    const int p_first = __builtin_amdgcn_readfirstlane(pos[t0]), p_last = p_first + ntok - 1, p_row = p_first + (t - t0);
+    const int lo_row = window > 0 ? max(0, p_row - window + 1) : 0;
+    const int kstart = window > 0 ? max(0, p_first - window + 1) / BN * BN : 0;
+    const int nT = (p_last - kstart) / BN + 1;
+    const int wp_last = p_first + min(w * TQ + TQ - 1, ntok - 1), wlo = window > 0 ? max(0, p_first + w * TQ - window + 1) : 0;
+
+    // copies: piece i = 64 (w + RW j) + lane of the tile's BN x PPR, to where it lies; it carries piece (i % PPR) ^ row_turn(row) of its row
+    // (worked out anew for every tile: kept across the loop, the offsets would be spilled)
+    const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(lds_ptr)buf);
+    auto copy = [&](int k0, int page_id, int which) __attribute__((always_inline)) {
+        const bf16_t* base = pool + ((size_t)page_id * page + (size_t)(k0 % page)) * (size_t)R;
+        const int left = p_last - k0;                                           // rows past the last position repeat it
+        int me = lane;
+        asm volatile("" : "+v"(me));
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+            if (w + RW * j < BN * PPR / 64) {
+                const int i = 64 * (w + RW * j) + me, row = i / PPR;
+                const unsigned off = (unsigned)(min(row, left) * PPR + ((i - row * PPR) ^ row_turn(row))) * 16u;
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base),
+                             "s"(lds0 + which * TILE + (w + RW * j) * 1024)
+                             : "memory");
+            }
+    };
+    const int Z = gridDim.z, z = blockIdx.z;
+    auto page_of = [&](int tile) __attribute__((always_inline)) { return bt[(kstart + min(tile, nT - 1) * BN) / page]; };
+    int next_page = 0;
+    if (z < nT) {
+        copy(kstart + z * BN, __builtin_amdgcn_readfirstlane(page_of(z)), 0);
+        next_page = page_of(z + Z);
+    }
+    v4u qfrag[RT];
+    {
+        const float* qrow = qf + ((size_t)t * H + (row_ok ? head : h0)) * (size_t)R;
+#pragma unroll
+        for (int s = 0; s < RT; ++s) {
+            qfrag[s] = v4u{0u, 0u, 0u, 0u};
+            if (row_ok && s >= S0) {
+                const float4 a = *(const float4*)(qrow + 32 * s + 8 * g4), b = *(const float4*)(qrow + 32 * s + 8 * g4 + 4);
+                qfrag[s] = v4u{pack_bf2(a.x, a.y), pack_bf2(a.z, a.w), pack_bf2(b.x, b.y), pack_bf2(b.z, b.w)};
+            }
+        }
+    }
+    v4f oacc[CT];
+#pragma unroll
+    for (int c = 0; c < CT; ++c) oacc[c] = v4f{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.f;
+    // K: key 16 mt + col, pieces 4 s + g4;  V: keys 4 g4 + col / 4 (+ 16), pieces 2 c + (col & 3) / 2, half col & 1
+    const int k_at = col * (R * 2), k_odd[2] = {(g4 ^ row_turn(col)) << 4, ((4 + g4) ^ row_turn(col)) << 4};
+    const int vk = 4 * g4 + (col >> 2), v_at = vk * (R * 2) + (col & 1) * 8;
+    int v_turn[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) v_turn[c] = ((2 * c + ((col & 3) >> 1)) ^ row_turn(vk)) << 4;
+    int which = 0;
+    for (int tile = z; tile < nT; tile += Z) {
+        const int k0 = kstart + tile * BN;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();                                           // this tile has landed; the other half has been read by everyone
+        asm volatile("" ::: "memory");
+        const unsigned char* T = buf + which * TILE;
+        which ^= 1;
+        if (tile + Z < nT) {
+            copy(k0 + Z * BN, __builtin_amdgcn_readfirstlane(next_page), which);
+            next_page = page_of(tile + 2 * Z);
+        }
+        if (!active || k0 > wp_last || k0 + BN - 1 < wlo) continue;             // (wave-uniform)
+        // operands are requested a few products ahead (the order is the source's: left alone, the compiler reads each one just before use)
+        v4f sacc[2] = {v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}};
+        constexpr int KN = 2 * (RT - S0), RING = RT + CT >= 50 ? 4 : RT + CT > 24 ? 5 : 6;
+        v4u ring[RING];
+        auto read = [&](int u) __attribute__((always_inline)) {                 // operand u: the KN of the keys, then the CT of the values
+            if (u < KN) {
+                const int s = S0 + (u >> 1);
+                ring[u % RING] = *(const v4u*)(T + k_at + 16 * (u & 1) * (R * 2) + (s >> 1) * 128 + k_odd[s & 1]);
+            } else if (u < KN + CT) {
+                const int c = u - KN;
+                const unsigned char* v = T + v_at + (c >> 2) * 128 + v_turn[c & 3];
+                const v2u a0 = __builtin_bit_cast(v2u, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)v));
+                const v2u a1 = __builtin_bit_cast(v2u, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)(v + 16 * (R * 2))));
+                ring[u % RING] = v4u{a0[0], a0[1], a1[0], a1[1]};
+            }
+        };
+#pragma unroll
+        for (int u = 0; u < RING - 1; ++u) read(u);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < KN; ++u) {
+            read(u + RING - 1);
+            __builtin_amdgcn_sched_barrier(0);
+            sacc[u & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, ring[u % RING]), __builtin_bit_cast(bf8, qfrag[S0 + (u >> 1)]),
+                                                                  sacc[u & 1], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // this lane: keys k0 + 16 mt + 4 g4 + r of its query row (the other 24 sit in lanes ^16, ^32, ^48)
+        float tmax = -INFINITY;
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int key = k0 + 16 * mt + 4 * g4 + r;
+                sacc[mt][r] = key <= p_row && key >= lo_row ? sacc[mt][r] : -INFINITY;
+                tmax = fmaxf(tmax, sacc[mt][r]);
+            }
+        const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(tmax), __float_as_uint(tmax), false, false);
+        tmax = fmaxf(__uint_as_float(x[0]), __uint_as_float(x[1]));
+        const auto y = __builtin_amdgcn_permlane32_swap(__float_as_uint(tmax), __float_as_uint(tmax), false, false);
+        tmax = fmaxf(__uint_as_float(y[0]), __uint_as_float(y[1]));
+        const float mnew = fmaxf(m, tmax);
+        const float msafe = mnew == -INFINITY ? 0.f : mnew;
+        const float alpha = __expf(m - msafe);                                  // m = -inf: 0
+        float psum = 0.f;
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                sacc[mt][r] = __expf(sacc[mt][r] - msafe);
+                psum += sacc[mt][r];
+            }
+        l = l * alpha + psum;                                                   // (this lane's share; the four shares are added after the loop)
+        m = mnew;
+        if (__any(alpha != 1.0f)) {
+#pragma unroll
+            for (int c = 0; c < CT; ++c) oacc[c] *= alpha;
+        }
+        // probabilities as B operand: k-slot (g4, e) <-> key 16 (e / 4) + 4 g4 + e % 4, i.e. exactly this lane's eight scores
+        const v4u pb = {pack_bf2(sacc[0][0], sacc[0][1]), pack_bf2(sacc[0][2], sacc[0][3]), pack_bf2(sacc[1][0], sacc[1][1]),
+                        pack_bf2(sacc[1][2], sacc[1][3])};
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+            read(KN + c + RING - 1);
+            __builtin_amdgcn_sched_barrier(0);
+            oacc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, ring[(KN + c) % RING]), __builtin_bit_cast(bf8, pb), oacc[c], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    int me = lane;                                                              // (as above: the row's place is worked out again)
+    asm volatile("" : "+v"(me));
+    const int my_tok = w * TQ + (me & 15) / HP, my_head = h0 + (me & 15) % HP;
+    if (my_tok >= ntok || my_head >= h_end) return;
+    const size_t my_row = (size_t)(t0 + my_tok) * H + my_head;
+    const int c4 = 4 * (me >> 4);
+    if (Z > 1) {                                                                // partial result of this key split: [z][t][h][rank] and (m, l)
+        const size_t rowi = (size_t)z * n_tokens * H + my_row;
+        if (c4 == 0) {
+            part_ml[rowi * 2] = m;
+            part_ml[rowi * 2 + 1] = l;
+        }
+        float* po = part_o + rowi * RANK + c4;
+#pragma unroll
+        for (int c = 0; c < CT; ++c) *(v4f*)(po + 16 * c) = oacc[c];
+        return;
+    }
+    const float inv = 1.0f / l;
+    bf16_t* o = out + my_row * RANK + c4;
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+        *(v2u*)(o + 16 * c) = v2u{pack_bf2(oacc[c][0] * inv, oacc[c][1] * inv), pack_bf2(oacc[c][2] * inv, oacc[c][3] * inv)};
+}
+
 // out[t, h] = sum_z e^(m_z - M) o_z / sum_z e^(m_z - M) l_z   (one workgroup per (token, head))
 __global__ __launch_bounds__(256) void latent_attention_merge_kernel(bf16_t* __restrict__ out, const float* __restrict__ part_o,
                                                                      const float* __restrict__ part_ml, int Z, int rows, int rank) {
@@ -406,4 +606,41 @@ extern "C" int qsv_latent_attention_mfma(void* out, const float* qf, const void*
                            part_o, part_ml, key_splits, n_tokens * H, rank);
     }
     return qsv_launch_status("qsv_latent_attention_mfma");
+}
+
+// The plain-rows kernel: 1 if it takes these sizes, tokens per tile, and the launch (arguments as above; no option changes the scores).
+extern "C" int qsv_latent_rows_ok(int rank, int row_width, int page, int dtype) {
+    return dtype == QSV_BF16 && page > 0 && page % BN == 0 &&
+           ((row_width == 576 && rank == 512) || (row_width == 512 && rank == 512) || (row_width == 256 && rank == 128));
+}
+extern "C" int qsv_latent_rows_tile_tokens(int heads) { return heads <= 0 ? 0 : RW * geometry(heads).TQ; }
+extern "C" int qsv_latent_rows(void* out, const float* qf, const void* pool, const int32_t* block_table, int table_stride, const int32_t* pos,
+                               const int32_t* tiles, int n_tiles, int window, int H, int rank, int R, int page, int key_splits, float* part_o,
+                               float* part_ml, int n_tokens, int q_first, int heads_per_pool, int64_t pool_stride, void* stream) {
+    QSV_REQUIRE(out && qf && pool && block_table && pos && tiles && n_tiles >= 0 && H > 0 && window >= 0, "qsv_latent_rows: bad arguments");
+    QSV_REQUIRE(qsv_latent_rows_ok(rank, R, page, QSV_BF16), "qsv_latent_rows: sizes not supported (rank %d, row %d, page %d)", rank, R, page);
+    QSV_REQUIRE(((uintptr_t)pool | (uintptr_t)qf) % 16 == 0 && pool_stride % 8 == 0, "qsv_latent_rows: rows start on 16 bytes");
+    if (n_tiles == 0) return QSV_OK;
+    QSV_REQUIRE(heads_per_pool > 0 && H % heads_per_pool == 0 && pool_stride >= 0, "qsv_latent_rows: %d heads over pools of %d", H, heads_per_pool);
+    QSV_REQUIRE(key_splits >= 1 && key_splits <= 64 && (key_splits == 1 || (part_o && part_ml && n_tokens > 0)),
+                "qsv_latent_rows: key splits without workspace");
+    QSV_REQUIRE(q_first >= 0 && q_first < R, "qsv_latent_rows: first query element %d of %d", q_first, R);
+    const Geometry g = geometry(heads_per_pool);
+    const dim3 grid(n_tiles, (H / heads_per_pool) * ((heads_per_pool + 15) / 16), key_splits), block(64 * RW);
+#define QSV_ROWS(RT, CT, S0)                                                                                                                   \
+    hipLaunchKernelGGL((latent_rows_kernel<RT, CT, S0>), grid, block, 0, (hipStream_t)stream, (bf16_t*)out, qf, (const bf16_t*)pool,             \
+                       block_table, table_stride, pos, tiles, n_tiles, window, H, page, g.HP, g.TQ, part_o, part_ml, n_tokens, heads_per_pool,   \
+                       pool_stride)
+    if (R == 576) QSV_ROWS(18, 32, 0);
+    else if (R == 512) QSV_ROWS(16, 32, 0);
+    else if (q_first >= 128) QSV_ROWS(8, 8, 4);
+    else QSV_ROWS(8, 8, 0);
+#undef QSV_ROWS
+    if (key_splits > 1) {
+        const int rc = qsv_launch_status("qsv_latent_rows");
+        if (rc != QSV_OK) return rc;
+        hipLaunchKernelGGL(latent_attention_merge_kernel, dim3(n_tokens * H), dim3(256), 0, (hipStream_t)stream, (bf16_t*)out, part_o, part_ml,
+                           key_splits, n_tokens * H, rank);
+    }
+    return qsv_launch_status("qsv_latent_rows");
 }

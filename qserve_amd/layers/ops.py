@@ -91,6 +91,7 @@ class HipOps:
                    "latent_query")
         return qf
 
+    plain_rows_kernel = True            # exact row sizes without options: the kernel that copies whole rows into LDS
     attention_split_target = 512        # workgroups a launch of the matrix-core attention should at least have
 
     def latent_attention(self, qf, pool, batch, window, rank, page, variant=0, key_splits=None, q_first=0, chunk=None, bias=None,
@@ -123,6 +124,23 @@ class HipOps:
         assert pool.size(-1) == R and block_table.dtype == torch.int32 and seq.dtype == torch.int32
         per, pool_stride = (H, 0) if pool.dim() == 2 else (H // pool.size(0), pool.stride(0))
         assert pool.dim() == 2 or H % pool.size(0) == 0
+        plain = bias is None and not chunk and not keep_first and sink is None and pooled is None and slopes is None
+        if (variant == 0 and plain and self.plain_rows_kernel and self.L.qsv_latent_rows_ok(rank, R, page, self.code) and pool.data_ptr() % 16 == 0
+                and pool_stride % 8 == 0 and qf.data_ptr() % 16 == 0):
+            tiles = batch.tiles(self.L.qsv_latent_rows_tile_tokens(per))
+            groups = tiles.size(0) * (H // per) * ((per + 15) // 16)
+            span = min(batch.max_pos + 1, int(window)) if window else batch.max_pos + 1
+            # (one workgroup per CU at 512 columns and more, two below; measured best at 64 sequences of 1000 and 4000 positions)
+            splits = max(1, min((256 if R > 320 else 512) // max(groups, 1), span // 64, 32)) if key_splits is None else key_splits
+            po = pm = None
+            if splits > 1:
+                po = torch.empty((splits, T, H, rank), dtype=torch.float32, device=qf.device)
+                pm = torch.empty((splits, T, H, 2), dtype=torch.float32, device=qf.device)
+            self.check(self.L.qsv_latent_rows(out.data_ptr(), qf.data_ptr(), pool.data_ptr(), block_table.data_ptr(), block_table.stride(0),
+                                              pos.data_ptr(), tiles.data_ptr(), tiles.size(0), int(window or 0), H, rank, R, page, splits,
+                                              0 if po is None else po.data_ptr(), 0 if pm is None else pm.data_ptr(), T, int(q_first), per,
+                                              pool_stride, self._s()), "latent_rows")
+            return out
         if variant == 0 and page % 32 == 0 and self.L.qsv_latent_attention_mfma_ok(rank, R, self.code):
             tiles = batch.tiles(self.L.qsv_latent_attention_tile_tokens(per))
             # few workgroups and long contexts (decoding): cut the keys over several workgroups, merged by a second launch

@@ -24,6 +24,9 @@ SIGNATURES = {
     "qsv_latent_attention_mfma_ok": (_i, [_i, _i, _i]),
     "qsv_latent_attention_mfma": (_i, [_vp, _vp, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _vp, _i, _i, _i, _i64, _i, _vp,
                                        _i, _i, _vp, _vp, _i64, _i, _i, _vp, _vp]),
+    "qsv_latent_rows_ok": (_i, [_i, _i, _i, _i]),
+    "qsv_latent_rows_tile_tokens": (_i, [_i]),
+    "qsv_latent_rows": (_i, [_vp, _vp, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _vp, _i, _i, _i, _i64, _vp]),
     "qsv_talking_attention_key_pools": (_i, [_i, _i, _i, _i]),
     "qsv_talking_attention_tile_tokens": (_i, [_i, _i, _i]),
     "qsv_talking_attention_mfma_ok": (_i, [_i, _i, _i, _i]),

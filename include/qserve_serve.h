@@ -20,6 +20,10 @@ int qsv_version(void);
 const char* qsv_arch(void);
 const char* qsv_last_error(void);
 
+/* out [n_rows, N] = x [n_rows, K] @ w [N, K]^T, bfloat16 with float accumulation, for few rows (a decoding step); x_stride: elements from one
+ * row of x to the next.  K and x_stride multiples of 8, x and w on 16 bytes. */
+int qsv_skinny_linear(void* out, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K, void* stream);
+
 /* x[t] = table[tokens[t]] (float) and h[t] = the same row in the storage type. */
 int qsv_embed(float* x, void* h, const void* table, const int32_t* tokens, int n_tokens, int width, int dtype, void* stream);
 

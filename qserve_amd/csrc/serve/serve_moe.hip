@@ -3,6 +3,7 @@
 // Router scores are float from the first product to the chosen weights.  The expert kernels keep one token's input in LDS
 // and let every wave walk output rows with its lanes spread along the reduction (coalesced weight rows).
 #include "serve_common.h"
+#include "serve_stream.h"
 
 namespace {
 constexpr int NT = 256;
@@ -488,23 +489,14 @@ __global__ __launch_bounds__(NT) void moe_down_vec_kernel(T* __restrict__ y, con
 // however many tokens share the expert.  Bound by HBM (the chosen experts' weights) and, below that, by launch latency.
 // * The slots (token t's k-th choice: slot t top_k + k) of an expert are found by the workgroup itself from the router's indices - no
 //   sort, no counts on the host - or given as sorted runs (`offsets`).
-// * The four waves split the reduction (stage i of 64 elements belongs to wave i % 4), so the expert's inputs are read once per workgroup.
-//   Each wave streams its stages - one 128-byte line of 32 weight rows and of 16 or 32 inputs - through a ring of its own in LDS
-//   (global_load_lds, whole lines; the wave waits for its own oldest stage only, no barrier in the loop) and multiplies them with
-//   v_mfma_f32_16x16x32_bf16, weights as the A operand.  Pieces of a row are permuted by its number: 16-byte reads without bank conflicts.
+// * The weights stream through per-wave LDS rings (serve_stream.h); the expert's inputs are read once per workgroup.
 // * The partial sums of the four waves meet in LDS; more than 32 slots per expert are walked in chunks (the weights then come from L2).
 // Two workgroups per CU keep up to 96 KiB of weights in flight.
 // Measured per launch in a step (MI355X): 64 tokens, 4 of 16 experts of 2048 x 1408 (92 MB a product) 55.6 / 62.4 us -> 23.8 / 21.1 us (up /
 // down) against the form it replaces, which kept weight rows in registers and paid a wave-wide sum per token and row; 16 tokens with
 // gated units (184 + 92 MB) 42.6 / 26.1 -> 36.5 / 19.3 us (5.0 TB/s); one token 1446 / 3117 us (the per-token kernels) -> 14.0 / 8.8 us.
 // The sort, search and permutation launches in front of it (60 us a layer) are gone.
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
-typedef unsigned int v4u __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) void* lds_ptr;
 constexpr int XR = 32;               // weight rows per workgroup
-constexpr int XK = 64;               // reduction elements per stage
-constexpr int XRING = 18 * 1024;     // ring of one wave
 constexpr int XLIST = 1024;          // router indices looked at in one go
 
 struct ExpertArgs {
@@ -519,86 +511,6 @@ struct ExpertArgs {
     float limit;
     bool wide;                       // out starts on 16 bytes
 };
-
-// SG: groups of 16 slots in the chunk
-template <int SG>
-struct ExpertRing {
-    static constexpr int STAGE = (XR + 16 * SG) * 128, INSTR = STAGE / 1024, DEPTH = XRING / STAGE;
-};
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-__device__ __forceinline__ void lds_copy16(unsigned dst, const void* base, unsigned off) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(dst) : "memory");
-}
-__device__ __forceinline__ void lds_copy16(unsigned dst, const void* from) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(dst) : "memory");
-}
-
-// Products of the workgroup's rows with 16 SG inputs; row_of(i): input i's row of X.
-template <int SG, class Row>
-__device__ __forceinline__ void expert_chunk(const ExpertArgs& a, const bf16_t* W0, int rows_here, unsigned char* ring, int w, int lane, Row row_of,
-                                             v4f (&acc)[XR / 16][SG]) {
-    typedef ExpertRing<SG> R;
-    const int stages = (a.K + XK - 1) / XK, mine = stages > w ? (stages - w + NW - 1) / NW : 0;
-    const int piece = (lane & 7) ^ (lane >> 3);
-    unsigned woff[XR / 8];
-    const bf16_t* xrow[2 * SG];
-#pragma unroll
-    for (int j = 0; j < XR / 8; ++j) woff[j] = (unsigned)min(8 * j + (lane >> 3), rows_here - 1) * (unsigned)a.K * 2u;
-#pragma unroll
-    for (int j = 0; j < 2 * SG; ++j) xrow[j] = a.X + (size_t)row_of(8 * j + (lane >> 3)) * (size_t)a.K;
-#pragma unroll
-    for (int r = 0; r < XR / 16; ++r)
-#pragma unroll
-        for (int g = 0; g < SG; ++g) acc[r][g] = v4f{0.f, 0.f, 0.f, 0.f};
-    const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(lds_ptr)ring);
-    auto issue = [&](int i) {
-        const int k0 = (w + NW * i) * XK;
-        const unsigned po = k0 + piece * 8 < a.K ? (unsigned)piece * 16u : 0u;     // (beyond the row: any valid piece, masked below)
-        const unsigned dst = lds0 + (unsigned)(i % R::DEPTH) * R::STAGE;
-#pragma unroll
-        for (int j = 0; j < XR / 8; ++j) lds_copy16(dst + 1024 * j, W0 + k0, woff[j] + po);
-#pragma unroll
-        for (int j = 0; j < 2 * SG; ++j) lds_copy16(dst + 1024 * (XR / 8 + j), (const unsigned char*)(xrow[j] + k0) + po);
-    };
-    const int row = lane & 15, quad = lane >> 4;
-    wait_vm<0>();
-    for (int i = 0; i < min(R::DEPTH, mine); ++i) issue(i);
-    for (int i = 0; i < mine; ++i) {
-        const int ahead = min(R::DEPTH - 1, mine - 1 - i);                         // stages requested behind this one
-        if (ahead == 2) wait_vm<2 * R::INSTR>();
-        else if (ahead == 1) wait_vm<R::INSTR>();
-        else wait_vm<0>();
-        const unsigned char* st = ring + (i % R::DEPTH) * R::STAGE;
-        const int left = a.K - (w + NW * i) * XK;                                  // elements of this stage inside the row
-#pragma unroll
-        for (int ks = 0; ks < XK / 32; ++ks) {
-            const int p = 4 * ks + quad;
-            v4u A[XR / 16], B[SG];
-#pragma unroll
-            for (int r = 0; r < XR / 16; ++r) A[r] = *(const v4u*)(st + (16 * r + row) * 128 + ((p ^ (row & 7)) << 4));
-#pragma unroll
-            for (int g = 0; g < SG; ++g) B[g] = *(const v4u*)(st + (XR + 16 * g + row) * 128 + ((p ^ (row & 7)) << 4));
-            if (left < XK && p * 8 >= left) {
-#pragma unroll
-                for (int r = 0; r < XR / 16; ++r) A[r] = v4u{0u, 0u, 0u, 0u};
-#pragma unroll
-                for (int g = 0; g < SG; ++g) B[g] = v4u{0u, 0u, 0u, 0u};
-            }
-#pragma unroll
-            for (int r = 0; r < XR / 16; ++r)
-#pragma unroll
-                for (int g = 0; g < SG; ++g)
-                    acc[r][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, A[r]), __builtin_bit_cast(bf8, B[g]), acc[r][g], 0, 0, 0);
-        }
-        if (i + R::DEPTH < mine) {
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                     // the slot has been read
-            issue(i + R::DEPTH);
-        }
-    }
-}
 
 // The four waves' partial sums (through LDS), the weight on the input, the activation, the store: slot of column c by slot_of(c).
 template <int ACT, bool FOUT, int SG, class Slot>
@@ -671,15 +583,15 @@ __global__ __launch_bounds__(NT, 2) void expert_rows_kernel(ExpertArgs a) {
     auto walk = [&](int count, auto row_of, auto slot_of) {
         for (int c0 = 0; c0 < count; c0 += 32) {
             const int c = min(32, count - c0);
-            auto rows = [&](int i) { return row_of(c0 + min(i, c - 1)); };
+            auto rows = [&](int i) { return a.X + (size_t)row_of(c0 + min(i, c - 1)) * (size_t)a.K; };
             auto slots = [&](int i, int64_t& slot, float& iw) { slot_of(c0 + i, slot, iw); };
             if (c <= 16) {
                 v4f acc[XR / 16][1];
-                expert_chunk<1>(a, W0, rows_here, ring, w, lane, rows, acc);
+                stream_products<XR / 16, 1>(W0, a.K, rows_here, ring, w, lane, rows, acc);
                 expert_finish<ACT, FOUT, 1>(a, r0, c, rings, w, lane, slots, acc);
             } else {
                 v4f acc[XR / 16][2];
-                expert_chunk<2>(a, W0, rows_here, ring, w, lane, rows, acc);
+                stream_products<XR / 16, 2>(W0, a.K, rows_here, ring, w, lane, rows, acc);
                 expert_finish<ACT, FOUT, 2>(a, r0, c, rings, w, lane, slots, acc);
             }
         }

@@ -1,0 +1,100 @@
+// serve_stream.h -- products of many weight rows with few inputs (bfloat16): every weight read once, streamed through LDS.
+//
+// The four waves of a workgroup split the reduction (stage i of 64 elements belongs to wave i % 4).  Each streams its stages - one 128-byte
+// line of 16 RB weight rows and of 16 SG inputs - through a ring of its own in LDS (global_load_lds, whole lines; the wave waits for its
+// own oldest stage only, no barrier in the loop) and multiplies them with v_mfma_f32_16x16x32_bf16, weights as the A operand.  Pieces of
+// a row are permuted by its number: 16-byte reads without bank conflicts.
+#pragma once
+#include "serve_common.h"
+
+namespace {
+constexpr int STREAM_WAVES = 4;
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void* lds_ptr;
+constexpr int XK = 64;               // reduction elements per stage
+constexpr int XRING = 18 * 1024;     // ring of one wave: two workgroups fit a CU
+
+template <int RB, int SG>
+struct StreamRing {
+    static constexpr int STAGE = 16 * (RB + SG) * 128, INSTR = STAGE / 1024, DEPTH = XRING / STAGE;
+    static_assert(DEPTH >= 2 && DEPTH <= 4, "");
+};
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ void lds_copy16(unsigned dst, const void* base, unsigned off) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(dst) : "memory");
+}
+__device__ __forceinline__ void lds_copy16(unsigned dst, const void* from) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(dst) : "memory");
+}
+
+// acc[r][g]: this wave's share of the products of weight rows W0 + 16 r + .. (rows_here of them, K elements each) with inputs 16 g + ..;
+// input(i): where input i starts.  w (the wave) is wave-uniform; `ring`: its XRING bytes of LDS.
+template <int RB, int SG, class Input>
+__device__ __forceinline__ void stream_products(const bf16_t* W0, int K, int rows_here, unsigned char* ring, int w, int lane, Input input,
+                                                v4f (&acc)[RB][SG]) {
+    typedef StreamRing<RB, SG> R;
+    const int stages = (K + XK - 1) / XK, mine = stages > w ? (stages - w + STREAM_WAVES - 1) / STREAM_WAVES : 0;
+    const int piece = (lane & 7) ^ (lane >> 3);
+    unsigned woff[2 * RB];
+    const bf16_t* xrow[2 * SG];
+#pragma unroll
+    for (int j = 0; j < 2 * RB; ++j) woff[j] = (unsigned)min(8 * j + (lane >> 3), rows_here - 1) * (unsigned)K * 2u;
+#pragma unroll
+    for (int j = 0; j < 2 * SG; ++j) xrow[j] = input(8 * j + (lane >> 3));
+#pragma unroll
+    for (int r = 0; r < RB; ++r)
+#pragma unroll
+        for (int g = 0; g < SG; ++g) acc[r][g] = v4f{0.f, 0.f, 0.f, 0.f};
+    const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(lds_ptr)ring);
+    auto issue = [&](int i) {
+        const int k0 = (w + STREAM_WAVES * i) * XK;
+        const unsigned po = k0 + piece * 8 < K ? (unsigned)piece * 16u : 0u;       // (beyond the row: any valid piece, masked below)
+        const unsigned dst = lds0 + (unsigned)(i % R::DEPTH) * R::STAGE;
+#pragma unroll
+        for (int j = 0; j < 2 * RB; ++j) lds_copy16(dst + 1024 * j, W0 + k0, woff[j] + po);
+#pragma unroll
+        for (int j = 0; j < 2 * SG; ++j) lds_copy16(dst + 1024 * (2 * RB + j), (const unsigned char*)(xrow[j] + k0) + po);
+    };
+    const int row = lane & 15, quad = lane >> 4;
+    wait_vm<0>();
+    for (int i = 0; i < min(R::DEPTH, mine); ++i) issue(i);
+    for (int i = 0; i < mine; ++i) {
+        const int ahead = min(R::DEPTH - 1, mine - 1 - i);                         // stages requested behind this one
+        if (R::DEPTH > 3 && ahead == 3) wait_vm<3 * R::INSTR>();
+        else if (R::DEPTH > 2 && ahead == 2) wait_vm<2 * R::INSTR>();
+        else if (ahead == 1) wait_vm<R::INSTR>();
+        else wait_vm<0>();
+        const unsigned char* st = ring + (i % R::DEPTH) * R::STAGE;
+        const int left = K - (w + STREAM_WAVES * i) * XK;                          // elements of this stage inside the row
+#pragma unroll
+        for (int ks = 0; ks < XK / 32; ++ks) {
+            const int p = 4 * ks + quad;
+            v4u A[RB], B[SG];
+#pragma unroll
+            for (int r = 0; r < RB; ++r) A[r] = *(const v4u*)(st + (16 * r + row) * 128 + ((p ^ (row & 7)) << 4));
+#pragma unroll
+            for (int g = 0; g < SG; ++g) B[g] = *(const v4u*)(st + (16 * (RB + g) + row) * 128 + ((p ^ (row & 7)) << 4));
+            if (left < XK && p * 8 >= left) {
+#pragma unroll
+                for (int r = 0; r < RB; ++r) A[r] = v4u{0u, 0u, 0u, 0u};
+#pragma unroll
+                for (int g = 0; g < SG; ++g) B[g] = v4u{0u, 0u, 0u, 0u};
+            }
+#pragma unroll
+            for (int r = 0; r < RB; ++r)
+#pragma unroll
+                for (int g = 0; g < SG; ++g)
+                    acc[r][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, A[r]), __builtin_bit_cast(bf8, B[g]), acc[r][g], 0, 0, 0);
+        }
+        if (i + R::DEPTH < mine) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                     // the slot has been read
+            issue(i + R::DEPTH);
+        }
+    }
+}
+}  // namespace

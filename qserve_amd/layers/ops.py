@@ -21,8 +21,24 @@ def dtype_code(dtype):
     raise ValueError(f"the serving kernels store bfloat16 or float32, not {dtype}")
 
 
+def _skinny(T, N, K):
+    """Whether the kernel that streams the weight beats the vendor's product for T rows (measured from HBM, N 1024 - 32000, K 64 - 4096: always
+    up to 16 rows; up to 32 but for 11008 x 4096, 26 against 23 us; up to 64 while one round of workgroups holds the weight)."""
+    return T <= 16 or (T <= 32 and (K <= 2048 or N * K <= 36_000_000)) or (T <= 64 and N <= 6144 and N * K <= 13_000_000)
+
+
 def linear(x, w):
-    """x [T, in] @ w [out, in]^T in the storage type (hipBLASLt / rocBLAS through torch; float accumulation)."""
+    """x [T, in] @ w [out, in]^T in the storage type, float accumulation: the few rows of a decoding step (bfloat16 on a GPU) through
+    qsv_skinny_linear, everything else through hipBLASLt / rocBLAS."""
+    if (type(x) is torch.Tensor and x.is_cuda and x.dim() == 2 and w.dim() == 2 and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+            and w.is_contiguous() and 0 < x.size(0) and x.size(1) == w.size(1) and x.size(1) and w.size(0) and _skinny(x.size(0), w.size(0), w.size(1))
+            and x.stride(1) == 1 and x.size(1) % 8 == 0 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and x.device == w.device and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))):
+        from ..serving._lib import check, lib
+        out = torch.empty((x.size(0), w.size(0)), dtype=x.dtype, device=x.device)
+        check(lib().qsv_skinny_linear(out.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(), x.size(0), w.size(0), x.size(1),
+                                      torch.cuda.current_stream(x.device).cuda_stream), "skinny_linear")
+        return out
     return torch.matmul(x, w.t())
 
 

@@ -24,6 +24,15 @@ const char* qsv_last_error(void);
  * row of x to the next.  K and x_stride multiples of 8, x and w on 16 bytes. */
 int qsv_skinny_linear(void* out, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K, void* stream);
 
+/* out [T, H, N] = x[t, h] @ w[h], w [H, K, N], bfloat16 with float accumulation, for up to 64 rows; x_tok, x_head: elements from one token / head
+ * of x to the next.  K and N multiples of 32, x_tok and x_head of 8, x on 16 bytes. */
+int qsv_head_product(void* out, const void* x, int64_t x_tok, int64_t x_head, const void* w, int T, int H, int K, int N, void* stream);
+
+/* The product with w_uk [H, dim, rank] and qsv_latent_query in one (bfloat16, up to 64 rows; dim and rank multiples of 32, dim + rot_dim of 8,
+ * rot_dim even): the absorbed part is not rounded in between. */
+int qsv_latent_query_product(float* qf, const void* q, const void* w_uk, const float* rope, const int32_t* pos, float scale, int n_tokens, int heads,
+                             int dim, int rot_dim, int rot_n, int rank, void* stream);
+
 /* x[t] = table[tokens[t]] (float) and h[t] = the same row in the storage type. */
 int qsv_embed(float* x, void* h, const void* table, const int32_t* tokens, int n_tokens, int width, int dtype, void* stream);
 

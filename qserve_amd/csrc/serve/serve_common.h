@@ -103,6 +103,23 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
     return s;
 }
 
+// four neighbouring elements at a multiple of four from an address that holds them whole
+__device__ __forceinline__ void ld4t(const float* p, size_t i, float (&v)[4]) {
+    const float4 a = *(const float4*)(p + i);
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+}
+__device__ __forceinline__ void ld4t(const bf16_t* p, size_t i, float (&v)[4]) {
+    const uint2 u = *(const uint2*)(p + i);
+    v[0] = __uint_as_float(u.x << 16); v[1] = __uint_as_float(u.x & 0xffff0000u);
+    v[2] = __uint_as_float(u.y << 16); v[3] = __uint_as_float(u.y & 0xffff0000u);
+}
+__device__ __forceinline__ void st4t(float* p, size_t i, const float (&v)[4]) { *(float4*)(p + i) = make_float4(v[0], v[1], v[2], v[3]); }
+__device__ __forceinline__ void st4t(bf16_t* p, size_t i, const float (&v)[4]) {
+    *(uint2*)(p + i) = make_uint2((unsigned)f2bf(v[0]) | ((unsigned)f2bf(v[1]) << 16), (unsigned)f2bf(v[2]) | ((unsigned)f2bf(v[3]) << 16));
+}
+// an address that 4 elements of its type may be read from at once
+inline bool fits4(const void* p, int dtype) { return (uintptr_t)p % (dtype == QSV_BF16 ? 8 : 16) == 0; }
+
 // dtype dispatch of a templated launcher: F<bf16_t>() or F<float>()
 #define QSV_DISPATCH(dtype, what, CALL)                                  \
     do {                                                                 \

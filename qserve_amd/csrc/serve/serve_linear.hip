@@ -1,4 +1,4 @@
-// serve_linear.hip -- x [T, K] @ w [N, K]^T for the few rows of a decoding step (bfloat16, float accumulation).
+// serve_linear.hip -- products of the few rows of a decoding step (bfloat16, float accumulation): x [T, K] @ w [N, K]^T, and one product per head.
 //
 // Bound by HBM (the weight, read once) and below about 20 MB by the launch.  Workgroup = 16 or 32 weight rows and up to 32 inputs, the
 // weight streamed through LDS rings (serve_stream.h), the four waves' shares of the reduction added in LDS.
@@ -41,7 +41,134 @@ __global__ __launch_bounds__(64 * STREAM_WAVES, 2) void skinny_linear_kernel(bf1
         }
     }
 }
+
+// ---- one product per head: y[t, h] = x[t, h] @ W[h], W [H, K, N] with N contiguous -------------------------------------------------------
+// Up to 64 tokens.  Bound by latency (16 heads of 128 x 512: 2 MB), so everything a wave needs is requested at once: a workgroup owns 32
+// columns of one head, its four waves take the 32-deep steps of the reduction in turn (S of them at a time), and the B operands - eight
+// consecutive k of a column - are put together in registers from eight rows' pairs of columns, so the weight needs neither LDS nor a second
+// layout.  The waves' sums meet in LDS.
+// QUERY: the result is the absorbed part of the latent query, scaled, in float rows of N + rot_dim; workgroups behind the N / 32 of the
+// product turn and scale the rest of the row.
+struct HeadProductArgs {
+    void* out;
+    const bf16_t *x, *w;
+    int64_t x_tok, x_head;
+    int T, K, N, H;
+    const float* rope;
+    const int32_t* pos;
+    float scale;
+    int dim, rot_dim, rot_n;
+};
+template <int RT, int S, bool QUERY>
+__global__ __launch_bounds__(256) void head_product_kernel(HeadProductArgs a) {
+    __shared__ __attribute__((aligned(16))) float red[4][RT * 16][32];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = blockIdx.y;
+    if (QUERY && (int)blockIdx.x * 32 >= a.N) {
+        const int i = ((int)blockIdx.x - a.N / 32) * 256 + tid, t = i / a.rot_dim, c = i - t * a.rot_dim;
+        if (t >= a.T) return;
+        const bf16_t* qr = a.x + t * a.x_tok + h * a.x_head + a.dim;
+        float v = ld(qr, c);
+        if (c < a.rot_n) {
+            const int half = a.rot_n / 2, p = c >> 1;
+            const float* cs = a.rope + (size_t)a.pos[t] * (size_t)a.rot_n;
+            const float co = cs[p], sn = cs[half + p], u = ld(qr, 2 * p), w2 = ld(qr, 2 * p + 1);
+            v = (c & 1) ? (w2 * co + u * sn) : (u * co - w2 * sn);
+        }
+        ((float*)a.out)[((size_t)t * a.H + h) * (a.N + a.rot_dim) + a.N + c] = v * a.scale;
+        return;
+    }
+    const int n0 = blockIdx.x * 32, kq = (lane >> 4) * 8;
+    const bf16_t* W = a.w + (size_t)h * a.K * a.N + n0 + 2 * (lane & 15);
+    const bf16_t* X = a.x + h * a.x_head;
+    v4f acc[RT][2];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) acc[r][0] = acc[r][1] = (v4f){0.f, 0.f, 0.f, 0.f};
+    for (int k0 = wave * 32 * S; k0 < a.K; k0 += 4 * 32 * S) {                  // (K is a multiple of 32 S)
+        unsigned b[S][8];
+        v4u x[S][RT];
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const int k = k0 + 32 * s + kq;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) b[s][i] = *(const unsigned*)(W + (size_t)(k + i) * a.N);
+#pragma unroll
+            for (int r = 0; r < RT; ++r) x[s][r] = *(const v4u*)(X + min(16 * r + (lane & 15), a.T - 1) * a.x_tok + k);
+        }
+        __builtin_amdgcn_sched_barrier(0);                                     // every request before the first use
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            v4u lo, hi;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                lo[i] = __builtin_amdgcn_perm(b[s][2 * i + 1], b[s][2 * i], 0x05040100u);
+                hi[i] = __builtin_amdgcn_perm(b[s][2 * i + 1], b[s][2 * i], 0x07060302u);
+            }
+#pragma unroll
+            for (int r = 0; r < RT; ++r) {
+                acc[r][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, x[s][r]), __builtin_bit_cast(bf8, lo), acc[r][0], 0, 0, 0);
+                acc[r][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, x[s][r]), __builtin_bit_cast(bf8, hi), acc[r][1], 0, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) *(float2*)&red[wave][16 * r + 4 * (lane >> 4) + j][2 * (lane & 15)] = make_float2(acc[r][0][j], acc[r][1][j]);
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+        const int t = 16 * r + (tid >> 4), c = 2 * (tid & 15);
+        if (t >= a.T) continue;
+        float2 v = make_float2(0.f, 0.f);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const float2 p = *(const float2*)&red[w][t][c];
+            v.x += p.x;
+            v.y += p.y;
+        }
+        if (QUERY) *(float2*)((float*)a.out + ((size_t)t * a.H + h) * (a.N + a.rot_dim) + n0 + c) = make_float2(v.x * a.scale, v.y * a.scale);
+        else *(unsigned*)((bf16_t*)a.out + ((size_t)t * a.H + h) * a.N + n0 + c) = (unsigned)f2bf(v.x) | ((unsigned)f2bf(v.y) << 16);
+    }
+}
+template <int RT, bool QUERY>
+void launch_head_product(const HeadProductArgs& a, int steps, int tail, hipStream_t stream) {
+    const dim3 grid(a.N / 32 + tail, a.H), block(256);
+    if (steps == 4) hipLaunchKernelGGL((head_product_kernel<RT, 4, QUERY>), grid, block, 0, stream, a);
+    else if (steps == 2) hipLaunchKernelGGL((head_product_kernel<RT, 2, QUERY>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((head_product_kernel<RT, 1, QUERY>), grid, block, 0, stream, a);
+}
+bool head_product_ok(int T, int64_t x_tok, int64_t x_head, const void* x, const void* w, int K, int N, int H) {
+    return T > 0 && T <= 64 && H > 0 && H <= 65535 && K > 0 && N > 0 && K % 32 == 0 && N % 32 == 0 && (int64_t)K * N < (1ll << 31) && x_tok >= 0 &&
+           x_head >= 0 && x_tok % 8 == 0 && x_head % 8 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 4 == 0;
+}
+template <bool QUERY>
+int run_head_product(const HeadProductArgs& a, hipStream_t stream, const char* what) {
+    const int tail = QUERY ? (a.T * a.rot_dim + 255) / 256 : 0;
+    const int steps = a.K % 512 == 0 ? 4 : a.K % 256 == 0 ? 2 : 1;            // per wave at once: the four waves share K evenly
+    if (a.T <= 16) launch_head_product<1, QUERY>(a, steps, tail, stream);
+    else if (a.T <= 32) launch_head_product<2, QUERY>(a, steps, tail, stream);
+    else launch_head_product<4, QUERY>(a, steps, tail, stream);
+    return qsv_launch_status(what);
+}
 }  // namespace
+
+// out [T, H, N] = x[t, h] @ w[h], x rows x_tok / x_head elements apart, w [H, K, N]
+extern "C" int qsv_head_product(void* out, const void* x, int64_t x_tok, int64_t x_head, const void* w, int T, int H, int K, int N, void* stream) {
+    QSV_REQUIRE(out && x && w && head_product_ok(T, x_tok, x_head, x, w, K, N, H) && (uintptr_t)out % 4 == 0, "qsv_head_product: bad arguments");
+    return run_head_product<false>({out, (const bf16_t*)x, (const bf16_t*)w, x_tok, x_head, T, K, N, H, nullptr, nullptr, 1.0f, 0, 0, 0},
+                                   (hipStream_t)stream, "qsv_head_product");
+}
+
+// qf [T, H, rank + rot_dim] (float) = scale * [q[t, h, :dim] @ w_uk[h] | rotated q[t, h, dim:]], q [T, H, dim + rot_dim], w_uk [H, dim, rank]
+extern "C" int qsv_latent_query_product(float* qf, const void* q, const void* w_uk, const float* rope, const int32_t* pos, float scale, int T, int H,
+                                        int dim, int rot_dim, int rot_n, int rank, void* stream) {
+    QSV_REQUIRE(qf && q && w_uk && pos && dim > 0 && rot_dim >= 0 && rot_n >= 0 && rot_n <= rot_dim && rot_n % 2 == 0 && (rot_n == 0 || rope) &&
+                    rot_dim <= (1 << 20) && rot_dim % 2 == 0 && (uintptr_t)qf % 8 == 0, "qsv_latent_query_product: bad arguments");
+    const int64_t row = dim + rot_dim;
+    QSV_REQUIRE(head_product_ok(T, row * H, row, q, w_uk, dim, rank, H), "qsv_latent_query_product: sizes or addresses it does not take");
+    return run_head_product<true>({qf, (const bf16_t*)q, (const bf16_t*)w_uk, row * H, row, T, dim, rank, H, rope, pos, scale, dim, rot_dim, rot_n},
+                                  (hipStream_t)stream, "qsv_latent_query_product");
+}
 
 extern "C" int qsv_skinny_linear(void* out, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K, void* stream) {
     QSV_REQUIRE(out && x && w && n_rows >= 0 && N > 0 && K > 0 && K % 8 == 0 && x_stride % 8 == 0 && x_stride >= 0, "qsv_skinny_linear: bad arguments");

@@ -59,10 +59,68 @@ __global__ __launch_bounds__(NT) void add_layer_norm_kernel(float* __restrict__ 
         st(h, t * D + i, v);
     }
 }
+// The same, and the plain norm below, for rows of up to 1024 P elements, a multiple of four: one trip to memory - every operand is requested
+// before the first sum and stays in registers.  Bound by the row's latency in a step, by HBM in a prompt (64 / 8192 rows of 2048: 8.8 ->
+// 2.7 / 130 -> 33 us).
+template <typename T, int P, bool ADD>
+__global__ __launch_bounds__(NT) void layer_norm_vec_kernel(T* __restrict__ h, float* __restrict__ x, const T* __restrict__ y,
+                                                            const int32_t* __restrict__ rows, const T* __restrict__ w, float eps, int D) {
+    __shared__ float red[NT / 64 + 1];
+    const size_t t = blockIdx.x, from = ADD ? t : rows ? (size_t)rows[t] : t;
+    float v[P][4], g[P][4], old[P][4];
+#pragma unroll
+    for (int k = 0; k < P; ++k) {
+        const int i = (k * NT + threadIdx.x) * 4;
+        v[k][0] = v[k][1] = v[k][2] = v[k][3] = 0.f;
+        if (i >= D) continue;
+        if (ADD) ld4t(y, t * D + i, v[k]);
+        else ld4t(x, from * D + i, v[k]);
+        ld4t(w, i, g[k]);
+        if (ADD) ld4t(x, t * D + i, old[k]);
+    }
+    float s = 0.f;
+#pragma unroll
+    for (int k = 0; k < P; ++k) s += (v[k][0] + v[k][1]) + (v[k][2] + v[k][3]);
+    const float mean = block_sum<NT>(s, red) / (float)D;
+    float q = 0.f;
+#pragma unroll
+    for (int k = 0; k < P; ++k)
+        if ((k * NT + (int)threadIdx.x) * 4 < D) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                v[k][j] -= mean;
+                q += v[k][j] * v[k][j];
+            }
+        }
+    const float inv = 1.0f / sqrtf(block_sum<NT>(q, red) / (float)D + eps);
+#pragma unroll
+    for (int k = 0; k < P; ++k) {
+        const int i = (k * NT + threadIdx.x) * 4;
+        if (i >= D) continue;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[k][j] = (ADD ? old[k][j] : 0.f) + v[k][j] * inv * g[k][j];
+        if (ADD) st4t(x, t * D + i, v[k]);
+        st4t(h, t * D + i, v[k]);
+    }
+}
+template <typename T, bool ADD>
+static void launch_layer_norm_vec(T* h, float* x, const T* y, const int32_t* rows, const T* w, float eps, int n, int D, hipStream_t stream) {
+    if (D <= NT * 4) hipLaunchKernelGGL((layer_norm_vec_kernel<T, 1, ADD>), dim3(n), dim3(NT), 0, stream, h, x, y, rows, w, eps, D);
+    else if (D <= NT * 8) hipLaunchKernelGGL((layer_norm_vec_kernel<T, 2, ADD>), dim3(n), dim3(NT), 0, stream, h, x, y, rows, w, eps, D);
+    else hipLaunchKernelGGL((layer_norm_vec_kernel<T, 4, ADD>), dim3(n), dim3(NT), 0, stream, h, x, y, rows, w, eps, D);
+}
+static bool layer_norm_fits(const void* x, const void* h, const void* y, const void* w, int D, int dtype) {
+    return D % 4 == 0 && D <= NT * 16 && fits4(x, QSV_F32) && fits4(h, dtype) && fits4(y, dtype) && fits4(w, dtype);
+}
 extern "C" int qsv_add_layer_norm(float* x, void* h, const void* y, const void* w, float eps, int n, int D, int dtype,
                                   void* stream) {
     QSV_REQUIRE(x && h && y && w && n >= 0 && D > 0, "qsv_add_layer_norm: bad arguments");
     if (n == 0) return QSV_OK;
+    if (layer_norm_fits(x, h, y, w, D, dtype)) {
+        QSV_DISPATCH(dtype, "qsv_add_layer_norm",
+                     (launch_layer_norm_vec<T, true>((T*)h, x, (const T*)y, nullptr, (const T*)w, eps, n, D, (hipStream_t)stream)));
+        return qsv_launch_status("qsv_add_layer_norm");
+    }
     QSV_DISPATCH(dtype, "qsv_add_layer_norm",
                  hipLaunchKernelGGL(add_layer_norm_kernel<T>, dim3(n), dim3(NT), 0, (hipStream_t)stream, x, (T*)h, (const T*)y,
                                     (const T*)w, eps, D));
@@ -91,6 +149,11 @@ extern "C" int qsv_layer_norm_rows(void* out, const float* x, const int32_t* row
                                    int dtype, void* stream) {
     QSV_REQUIRE(out && x && w && n >= 0 && D > 0, "qsv_layer_norm_rows: bad arguments");
     if (n == 0) return QSV_OK;
+    if (layer_norm_fits(x, out, out, w, D, dtype)) {
+        QSV_DISPATCH(dtype, "qsv_layer_norm_rows",
+                     (launch_layer_norm_vec<T, false>((T*)out, (float*)x, nullptr, rows, (const T*)w, eps, n, D, (hipStream_t)stream)));
+        return qsv_launch_status("qsv_layer_norm_rows");
+    }
     QSV_DISPATCH(dtype, "qsv_layer_norm_rows",
                  hipLaunchKernelGGL(layer_norm_rows_kernel<T>, dim3(n), dim3(NT), 0, (hipStream_t)stream, (T*)out, x, rows,
                                     (const T*)w, eps, D));
@@ -184,6 +247,35 @@ __global__ __launch_bounds__(NT) void latent_query_kernel(float* __restrict__ qf
         dst[(size_t)h * R + rank + c] = v * scale;
     }
 }
+// The same, four columns per thread, `chunks` workgroups per token (sizes that are multiples of four; the same values).
+// Bound by HBM in a prompt, by the launch in a step (16 heads of 576: 8192 tokens 143 -> 130 us, 64 tokens 17.7 -> 2.7 us).
+template <typename T>
+__global__ __launch_bounds__(NT) void latent_query_vec_kernel(float* __restrict__ qf, const T* __restrict__ q, const T* __restrict__ q_abs,
+                                                              const float* __restrict__ rope, const int32_t* __restrict__ pos, float scale,
+                                                              int n_tokens, int H, int dim, int rot_dim, int rot_n, int rank, int chunks) {
+    const unsigned t = blockIdx.x / (unsigned)chunks, i = (blockIdx.x - t * chunks) * NT + threadIdx.x;
+    const unsigned R = rank + rot_dim, h = i / (R / 4), c = (i - h * (R / 4)) * 4;
+    if (h >= (unsigned)H) return;
+    float v[4];
+    if (c < (unsigned)rank) {
+        ld4t(q_abs, ((size_t)h * n_tokens + t) * (size_t)rank + c, v);
+    } else {
+        const int d = c - rank, half = rot_n / 2;
+        ld4t(q, ((size_t)t * H + h) * (size_t)(dim + rot_dim) + dim + d, v);
+        if (d < rot_n) {
+            const float* cs = rope + (size_t)pos[t] * (size_t)rot_n + (d >> 1);
+#pragma unroll
+            for (int p = 0; p < 2; ++p) {
+                const float co = cs[p], sn = cs[half + p], u = v[2 * p], w2 = v[2 * p + 1];
+                v[2 * p] = u * co - w2 * sn;
+                v[2 * p + 1] = w2 * co + u * sn;
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] *= scale;
+    st4t(qf, ((size_t)t * H + h) * R + c, v);
+}
 extern "C" int qsv_latent_query(float* qf, const void* q, const void* q_abs, const float* rope, const int32_t* pos, float scale,
                                 int n, int H, int dim, int rot_dim, int rot_n, int rank, int dtype, void* stream) {
     QSV_REQUIRE(qf && q && q_abs && pos && n >= 0 && H > 0 && dim > 0 && rank > 0, "qsv_latent_query: bad arguments");
@@ -191,6 +283,14 @@ extern "C" int qsv_latent_query(float* qf, const void* q, const void* q_abs, con
                 "qsv_latent_query: bad rotary sizes (%d of %d)", rot_n, rot_dim);
     if (n == 0) return QSV_OK;
     QSV_REQUIRE((int64_t)n * H < (1ll << 31), "qsv_latent_query: too many (token, head) pairs");
+    const int64_t chunks = ((int64_t)H * ((rank + rot_dim) / 4) + NT - 1) / NT;
+    if (dim % 4 == 0 && rot_dim % 4 == 0 && rot_n % 4 == 0 && rank % 4 == 0 && fits4(qf, QSV_F32) && fits4(q, dtype) && fits4(q_abs, dtype) &&
+        chunks * n < (1ll << 31)) {
+        QSV_DISPATCH(dtype, "qsv_latent_query",
+                     hipLaunchKernelGGL(latent_query_vec_kernel<T>, dim3((unsigned)(chunks * n)), dim3(NT), 0, (hipStream_t)stream, qf,
+                                        (const T*)q, (const T*)q_abs, rope, pos, scale, n, H, dim, rot_dim, rot_n, rank, (int)chunks));
+        return qsv_launch_status("qsv_latent_query");
+    }
     QSV_DISPATCH(dtype, "qsv_latent_query",
                  hipLaunchKernelGGL(latent_query_kernel<T>, dim3(n), dim3(NT), 0, (hipStream_t)stream, qf, (const T*)q,
                                     (const T*)q_abs, rope, pos, scale, n, H, dim, rot_dim, rot_n, rank));

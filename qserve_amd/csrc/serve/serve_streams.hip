@@ -80,19 +80,6 @@ __global__ __launch_bounds__(NT) void hc_write_kernel(float* __restrict__ x, con
 }
 
 // ---- the same two kernels for widths that are multiples of four: 16-byte stream accesses, four elements per thread and pass ----
-__device__ __forceinline__ void ld4t(const float* p, size_t i, float (&v)[4]) {
-    const float4 a = *(const float4*)(p + i);
-    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-}
-__device__ __forceinline__ void ld4t(const bf16_t* p, size_t i, float (&v)[4]) {
-    const uint2 u = *(const uint2*)(p + i);
-    v[0] = __uint_as_float(u.x << 16); v[1] = __uint_as_float(u.x & 0xffff0000u);
-    v[2] = __uint_as_float(u.y << 16); v[3] = __uint_as_float(u.y & 0xffff0000u);
-}
-__device__ __forceinline__ void st4t(float* p, size_t i, const float (&v)[4]) { *(float4*)(p + i) = make_float4(v[0], v[1], v[2], v[3]); }
-__device__ __forceinline__ void st4t(bf16_t* p, size_t i, const float (&v)[4]) {
-    *(uint2*)(p + i) = make_uint2((unsigned)f2bf(v[0]) | ((unsigned)f2bf(v[1]) << 16), (unsigned)f2bf(v[2]) | ((unsigned)f2bf(v[3]) << 16));
-}
 __device__ __forceinline__ void stream_sum4(const float* __restrict__ x, const float* __restrict__ w_in, size_t t, int S, int D, int i,
                                             float (&u)[4]) {
     u[0] = u[1] = u[2] = u[3] = 0.f;

@@ -51,11 +51,9 @@ class LatentAttention:
         cq = ops.latent_prep(down, self.q_off, self.q_rank, self.dq_norm, self.kv_off, self.rank, self.dkv_norm, self.rot_dim,
                              self.rot_n, rope, pool, batch.slot, batch.pos, self.eps)
         q = linear(cq, self.w_uq)                                                   # [T, H (dim + rot_dim)]
-        qn = q.view(T, H, self.dim + self.rot_dim)[..., :self.dim].transpose(0, 1)  # [H, T, dim] (strided view)
-        q_abs = torch.bmm(qn, self.w_uk)                                            # [H, T, rank]
-        qf = ops.latent_query(q, q_abs, rope, batch.pos, self.scale, H, self.dim, self.rot_dim, self.rot_n, self.rank)
+        qf = ops.latent_queries(q, self.w_uk, rope, batch.pos, self.scale, H, self.dim, self.rot_dim, self.rot_n, self.rank)
         o_lat = ops.latent_attention(qf, pool, batch, self.window, self.rank, self.page)
-        o = torch.bmm(o_lat.transpose(0, 1), self.w_uv_t).transpose(0, 1).reshape(T, H * self.vdim)
+        o = ops.head_products(o_lat, self.w_uv_t)                                   # [T, H vdim]
         if self.gated:
             ops.sigmoid_gate(o, down[:, self.g_off:self.g_off + H * self.vdim])
         return linear(o, self.w_o)

@@ -42,6 +42,16 @@ def linear(x, w):
     return torch.matmul(x, w.t())
 
 
+def _absorbed(q, w_uk):
+    """q [T, H (dim + rot)] -> [H, T, rank]: the first dim dimensions of every head times w_uk [H, dim, rank] (a strided view, no copy)."""
+    H, dim = w_uk.size(0), w_uk.size(1)
+    return torch.bmm(q.view(q.size(0), H, -1)[..., :dim].transpose(0, 1), w_uk)
+
+
+def _head_products(x, w):
+    return torch.bmm(x.transpose(0, 1), w).transpose(0, 1).reshape(x.size(0), w.size(0) * w.size(2))
+
+
 class HipOps:
     name = "hip"
 
@@ -106,6 +116,37 @@ class HipOps:
                                            pos.data_ptr(), scale, T, heads, dim, rot_dim, rot_n, rank, self.code, self._s()),
                    "latent_query")
         return qf
+
+    def latent_queries(self, q, w_uk, rope, pos, scale, heads, dim, rot_dim, rot_n, rank):
+        """qf [T, heads, rank + rot_dim] (float) from q [T, heads (dim + rot_dim)] and w_uk [heads, dim, rank].  A step's few rows: one launch
+        (16 heads of 128 to 512 + 64, 1 / 16 / 64 tokens: 3.0 / 3.3 / 4.6 us against 6.6 / 7.0 / 7.9); beyond 64 rows
+        the vendor's batched product and latent_query."""
+        T = q.size(0)
+        if self._head_products_fit(T, q, w_uk, dim + rot_dim) and rot_dim % 2 == 0:
+            self._need(q, w_uk, rope, pos)
+            assert q.numel() == T * heads * (dim + rot_dim) and w_uk.shape == (heads, dim, rank)
+            qf = torch.empty((T, heads, rank + rot_dim), dtype=torch.float32, device=q.device)
+            self.check(self.L.qsv_latent_query_product(qf.data_ptr(), q.data_ptr(), w_uk.data_ptr(), 0 if rope is None else rope.data_ptr(),
+                                                       pos.data_ptr(), scale, T, heads, dim, rot_dim, rot_n, rank, self._s()), "latent_queries")
+            return qf
+        q_abs = _absorbed(q, w_uk)
+        return self.latent_query(q, q_abs, rope, pos, scale, heads, dim, rot_dim, rot_n, rank)
+
+    def _head_products_fit(self, T, x, w, row):
+        return (0 < T <= 64 and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous()
+                and w.size(1) % 32 == 0 and w.size(2) % 32 == 0 and row % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 4 == 0)
+
+    def head_products(self, x, w):
+        """x [T, H, K], w [H, K, N] -> [T, H N], head by head: a step's few rows (up to 64) in one launch (16 heads of 512 to 128, 1 / 16 / 64 tokens:
+        3.1 / 3.5 / 5.3 us, the vendor's with its copy back to rows 9.8 / 12.9 / 13.3), more through the vendor's batched product."""
+        T, H, K = x.shape
+        if self._head_products_fit(T, x, w, K):
+            self._need(x, w)
+            assert w.size(0) == H and w.size(1) == K
+            out = torch.empty((T, H * w.size(2)), dtype=x.dtype, device=x.device)
+            self.check(self.L.qsv_head_product(out.data_ptr(), x.data_ptr(), H * K, K, w.data_ptr(), T, H, K, w.size(2), self._s()), "head_products")
+            return out
+        return _head_products(x, w)
 
     plain_rows_kernel = True            # exact row sizes without options: the kernel that copies whole rows into LDS
     attention_split_target = 512        # workgroups a launch of the matrix-core attention should at least have
@@ -915,6 +956,12 @@ class TorchOps:
         T = q.size(0)
         qr = _rotate(q.view(T, heads, dim + rot_dim)[..., dim:].float(), rope, pos, rot_n)
         return (torch.cat([q_abs.transpose(0, 1).float(), qr], dim=-1) * scale).contiguous()
+
+    def latent_queries(self, q, w_uk, rope, pos, scale, heads, dim, rot_dim, rot_n, rank):
+        return self.latent_query(q, _absorbed(q, w_uk), rope, pos, scale, heads, dim, rot_dim, rot_n, rank)
+
+    def head_products(self, x, w):
+        return _head_products(x, w)
 
     def latent_attention(self, qf, pool, batch, window, rank, page, variant=0, key_splits=None, q_first=0, chunk=None, bias=None,
                          keep_first=0, sink=None, pooled=None, pool_block=0, slopes=None):

@@ -68,19 +68,6 @@ __global__ __launch_bounds__(NT) void conv_silu_unit_kernel(float* __restrict__ 
     for (int c = n_unit * unit_dim + threadIdx.x; c < C; c += NT) out[t * C + c] = ys[c];
 }
 
-// ---- the recurrence ---------------------------------------------------------------------------------------------------------
-// Columns of S (value channels) never meet: column j of head h needs k, q and the decay of the token and its own v_j.  A
-// workgroup owns a block of columns of one (run, head): a wave 64 / LPC groups of NC of them, a lane R rows of its NC columns;
-// the LPC lanes of a column are neighbours and add their partial dot products through DPP moves.  The run's tokens are walked in order, CT at
-// a time: the workgroup stages k, q, the decay (float, zero-padded to LPC * R rows), its v columns and sigmoid(beta) of CT
-// tokens in LDS - the next CT tokens' values are already in registers while these are computed - so a token's step reads
-// LDS only, and the only exchange on the state's dependency chain is the delta rule's S^T k; the read-outs' partial sums wait
-// in registers until the chunk's end and are exchanged together.  The state is read once before and written once after (a run
-// that starts its sequence starts from zeros).
-constexpr int SCAN_CT = 16;       // tokens per staged chunk, at most
-constexpr int SCAN_PFK = 24;      // staged k / q / decay values per thread and chunk, at most
-constexpr int SCAN_PFV = 16;      // staged v values per thread and chunk, at most
-
 template <int CTRL>
 __device__ __forceinline__ float dpp_add(float v) {
     return v + __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
@@ -95,6 +82,67 @@ __device__ __forceinline__ float column_sum(float v, int lpc) {
     if (lpc >= 64) v += __shfl_xor(v, 32, 64);
     return v;
 }
+
+// The same for channels in fours (TAPS taps; whole groups of 4 to 256 channels, a power of two): a thread owns four channels of a token, so every
+// tap of theirs is requested before the first is used, a group is 1 - 64 neighbouring lanes, and a token is `chunks` workgroups.  The entries of
+// the new history are the taps behind the first, already in registers.  Bound by latency in a step, by HBM in a prompt (2560 channels: 16 tokens
+// 15.7 -> 2.7 us, 8192 tokens 137 -> 55 us).
+template <typename T, int TAPS>
+__global__ __launch_bounds__(NT) void conv_silu_unit_vec_kernel(float* __restrict__ out, const T* __restrict__ proj, int64_t stride, int off, int C,
+                                                                const float* __restrict__ w, float* __restrict__ hist,
+                                                                const int32_t* __restrict__ run_off, const int32_t* __restrict__ state_rd,
+                                                                const int32_t* __restrict__ state_wr, int unit_channels, int group_lanes, int act,
+                                                                int chunks) {
+    constexpr int PAST = TAPS - 1;
+    const unsigned t = blockIdx.x / (unsigned)chunks;
+    const int c = ((blockIdx.x - t * chunks) * NT + threadIdx.x) * 4;
+    const bool in = c < C;
+    const int from = in ? c : 0;                                   // (lanes behind the end stay for the sums below)
+    const int i = run_off[t], rd = state_rd[t], wr = state_wr[t];
+    float x[TAPS][4], wt[TAPS][4];
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) ld4t(w, (size_t)from * TAPS + 4 * j, wt[j]);
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) {
+        const int d = PAST - j;
+        x[j][0] = x[j][1] = x[j][2] = x[j][3] = 0.f;
+        if (d <= i) ld4t(proj, (size_t)(t - d) * stride + off + from, x[j]);
+        else if (rd >= 0) ld4t(hist, ((size_t)rd * PAST + (PAST + i - d)) * C + from, x[j]);
+    }
+    float y[4], s = 0.f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        float acc = 0.f;
+#pragma unroll
+        for (int j = 0; j < TAPS; ++j) acc += wt[(q * TAPS + j) / 4][(q * TAPS + j) % 4] * x[j][q];
+        y[q] = act ? acc / (1.0f + expf(-acc)) : acc;
+        s += y[q] * y[q];
+    }
+    const float inv = 1.0f / sqrtf(column_sum(s, group_lanes) + 1e-6f);
+    if (!in) return;
+    if (wr >= 0) {
+#pragma unroll
+        for (int jj = 0; jj < PAST; ++jj) st4t(hist, ((size_t)wr * PAST + jj) * C + c, x[jj + 1]);
+    }
+    if (c < unit_channels) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) y[q] *= inv;
+    }
+    st4t(out, (size_t)t * C + c, y);
+}
+
+// ---- the recurrence ---------------------------------------------------------------------------------------------------------
+// Columns of S (value channels) never meet: column j of head h needs k, q and the decay of the token and its own v_j.  A
+// workgroup owns a block of columns of one (run, head): a wave 64 / LPC groups of NC of them, a lane R rows of its NC columns;
+// the LPC lanes of a column are neighbours and add their partial dot products through DPP moves.  The run's tokens are walked in order, CT at
+// a time: the workgroup stages k, q, the decay (float, zero-padded to LPC * R rows), its v columns and sigmoid(beta) of CT
+// tokens in LDS - the next CT tokens' values are already in registers while these are computed - so a token's step reads
+// LDS only, and the only exchange on the state's dependency chain is the delta rule's S^T k; the read-outs' partial sums wait
+// in registers until the chunk's end and are exchanged together.  The state is read once before and written once after (a run
+// that starts its sequence starts from zeros).
+constexpr int SCAN_CT = 16;       // tokens per staged chunk, at most
+constexpr int SCAN_PFK = 24;      // staged k / q / decay values per thread and chunk, at most
+constexpr int SCAN_PFV = 16;      // staged v values per thread and chunk, at most
 
 __device__ __forceinline__ float4 ld4(const float* p, size_t i) { return *(const float4*)(p + i); }
 __device__ __forceinline__ float4 ld4(const bf16_t* p, size_t i) {
@@ -382,6 +430,109 @@ __global__ __launch_bounds__(256) void recurrent_step_kernel(float* __restrict__
         if (r0 + i < dim) Sg[(size_t)(r0 + i) * vdim] = S[i];
 }
 
+// The same for states whose columns come in fours: a workgroup owns 128 columns of one (run, head), a thread four of them (16-byte accesses, a
+// row's 512 bytes together) and 8 rows of every 64.  Row sums meet across two half waves and, through LDS, four waves.  Bound by the state's two
+// trips to memory (16 sequences of 16 heads, 64 x 128: 17 MB; 11.9 -> 4.9 us
+// with the delta rule; 64 sequences of 128 x 128 132 -> 25 us: the form above reads 32 bytes of a row at a time).
+template <typename TQ, typename TB, bool DELTA, int P>
+__global__ __launch_bounds__(256) void recurrent_step_wide_kernel(float* __restrict__ o, const TQ* __restrict__ q, int64_t q_stride,
+                                                                  const TQ* __restrict__ k, int64_t k_stride, const TQ* __restrict__ v,
+                                                                  int64_t v_stride, const float* __restrict__ decay, const TB* __restrict__ beta,
+                                                                  int64_t beta_stride, float* __restrict__ state,
+                                                                  const int32_t* __restrict__ runs, int H, int QH, int dim, int vdim, float q_scale,
+                                                                  const float* __restrict__ kscale, int head_decay, int v_cols) {
+    __shared__ float4 sums[2][4][32];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, cg = tid & 31, rg = tid >> 5;
+    const int j = blockIdx.z * 128 + cg * 4;
+    const bool col_ok = j < vdim;
+    const int slot = runs[4 * blockIdx.x];
+    const size_t t = (size_t)runs[4 * blockIdx.x + 1];
+    const bool fresh = runs[4 * blockIdx.x + 3] == 0;
+    const int h = blockIdx.y, qh = h / (H / QH);
+    float* Sg = state + (((size_t)slot * H + h) * dim) * (size_t)vdim + (col_ok ? j : 0);
+    float S[P][8][4], kc[P][8], qc[P][8], gc[P][8], vc[4];
+    const float kb = kscale ? kscale[t * H + h] : 1.0f;
+    const float hd = head_decay == 2 ? decay[h] : head_decay ? decay[t * H + h] : 0.f;
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const int r0 = p * 64 + rg * 8;
+        const bool ok = r0 < dim;                                   // (dim is a multiple of 8)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            S[p][i][0] = S[p][i][1] = S[p][i][2] = S[p][i][3] = 0.f;
+            if (ok && col_ok && !fresh) ld4t(Sg, (size_t)(r0 + i) * vdim, S[p][i]);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; i += 4) {
+            float a[4] = {0.f, 0.f, 0.f, 0.f}, b[4] = {0.f, 0.f, 0.f, 0.f}, g[4] = {hd, hd, hd, hd};
+            if (ok) {
+                ld4t(k, t * k_stride + (size_t)qh * dim + r0 + i, a);
+                ld4t(q, t * q_stride + (size_t)qh * dim + r0 + i, b);
+                if (!head_decay) ld4t(decay, (t * H + h) * (size_t)dim + r0 + i, g);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) kc[p][i + e] = a[e], qc[p][i + e] = b[e], gc[p][i + e] = g[e];
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) vc[c] = j + c < v_cols ? ld(v, t * v_stride + (size_t)h * v_cols + j + c) : j + c == v_cols ? 1.0f : 0.f;
+    const float rate = DELTA ? 1.0f / (1.0f + expf(-ld(beta, t * beta_stride + h))) : 0.f;
+    // sum over the workgroup's rows; every thread gets its columns'
+    auto row_sum = [&](float (&a)[4], int buffer) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) a[c] += __shfl_xor(a[c], 32, 64);
+        if (lane < 32) sums[buffer][wave][cg] = make_float4(a[0], a[1], a[2], a[3]);
+        __syncthreads();
+        const float4 s0 = sums[buffer][0][cg], s1 = sums[buffer][1][cg], s2 = sums[buffer][2][cg], s3 = sums[buffer][3][cg];
+        a[0] = (s0.x + s1.x) + (s2.x + s3.x);
+        a[1] = (s0.y + s1.y) + (s2.y + s3.y);
+        a[2] = (s0.z + s1.z) + (s2.z + s3.z);
+        a[3] = (s0.w + s1.w) + (s2.w + s3.w);
+    };
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    if (DELTA) {
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float kk = kc[p][i] * kb;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    S[p][i][c] *= gc[p][i];
+                    acc[c] += S[p][i][c] * kk;
+                }
+            }
+        row_sum(acc, 0);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            vc[c] = (vc[c] - acc[c]) * rate;
+            acc[c] = 0.f;
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float kk = kc[p][i] * kb;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                S[p][i][c] = (DELTA ? S[p][i][c] : gc[p][i] * S[p][i][c]) + kk * vc[c];
+                acc[c] += S[p][i][c] * qc[p][i];
+            }
+        }
+#pragma unroll
+    for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (col_ok && p * 64 + rg * 8 < dim) st4t(Sg, (size_t)(p * 64 + rg * 8 + i) * vdim, S[p][i]);
+    row_sum(acc, 1);
+    if (tid < 32 && col_ok) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[c] *= q_scale;
+        st4t(o, (t * H + h) * (size_t)vdim + j, acc);
+    }
+}
+
 // ---- per-head RMS norm of the read-out, times a weight, times a gate ------------------------------------------------------------
 // gate_kind 0: silu(g), 1: sigmoid(g).  o rows are o_stride floats apart per head (>= vdim); w_stride 0: one weight row shared by
 // the heads, vdim: a row per head.  den_m != NULL: before the norm the read-out is divided by max(|o[vdim]|, exp(-den_m[t, h])) +
@@ -405,6 +556,38 @@ __global__ __launch_bounds__(NT) void head_rms_gate_kernel(T* __restrict__ out, 
             st(out, (t * H + h) * (size_t)vdim + e, oh[e] * sc * inv * ld(w, (size_t)h * w_stride + e) * (gate_kind == 0 ? g * sg : sg));
         }
     }
+}
+
+// The same for heads of 4 to 256 values, a power of two: a thread owns four values of a head, a head is 1 - 64 neighbouring lanes, a token `chunks`
+// workgroups; everything is read once, before the sum.  (16 heads of 128: 16 tokens 5.6 -> 2.3 us, 8192 tokens 44 -> 31 us.)
+template <typename T>
+__global__ __launch_bounds__(NT) void head_rms_gate_vec_kernel(T* __restrict__ out, const float* __restrict__ o, const T* __restrict__ w,
+                                                               const T* __restrict__ gate, int64_t gate_stride, int gate_kind, float eps, int H,
+                                                               int vdim, int lanes_log, int o_stride, int w_stride,
+                                                               const float* __restrict__ den_m, int chunks) {
+    const unsigned t = blockIdx.x / (unsigned)chunks, idx = (blockIdx.x - t * chunks) * NT + threadIdx.x;
+    const bool in = (int)(idx >> lanes_log) < H;
+    const int h = in ? idx >> lanes_log : 0, e = (idx & ((1 << lanes_log) - 1)) * 4;
+    const size_t th = (size_t)t * H + h;
+    float x[4], g[4], ww[4];
+    ld4t(o, th * (size_t)o_stride + e, x);
+    ld4t(gate, t * gate_stride + (size_t)h * vdim + e, g);
+    ld4t(w, (size_t)h * w_stride + e, ww);
+    const float sc = den_m ? 1.0f / (fmaxf(fabsf(o[th * (size_t)o_stride + vdim]), expf(-den_m[th])) + 1e-6f) : 1.0f;
+    float s = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        x[j] *= sc;
+        s += x[j] * x[j];
+    }
+    const float inv = 1.0f / sqrtf(column_sum(s, 1 << lanes_log) / (float)vdim + eps);
+    if (!in) return;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const float sg = 1.0f / (1.0f + expf(-g[j]));
+        x[j] = x[j] * inv * ww[j] * (gate_kind == 0 ? g[j] * sg : sg);
+    }
+    st4t(out, th * (size_t)vdim + e, x);
 }
 
 // ---- exponential gates kept in range by a running maximum (mLSTM) ----------------------------------------------------------------
@@ -485,6 +668,48 @@ __global__ __launch_bounds__(NT) void attention_prep_kernel(float* __restrict__ 
     }
 }
 
+// The same, four columns per thread (sizes, halves and offsets that are multiples of four), `chunks` workgroups per token.  Bound by latency in a
+// step, by HBM in a prompt (16 + 4 heads of 128 + 128: 16 tokens 7.3 -> 2.6 us, 8192 tokens 53 -> 47 us).
+template <typename T>
+__device__ __forceinline__ void rotated4(const T* vec, int d, int n, const float* cs, float (&out)[4]) {
+    if (d >= n) return ld4t(vec, d, out);
+    const int half = n >> 1, p = d < half ? d : d - half;
+    float lo[4], hi[4], c[4], s[4];
+    ld4t(vec, p, lo);
+    ld4t(vec, p + half, hi);
+    ld4t(cs, p, c);
+    ld4t(cs, half + p, s);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) out[j] = rot_halves(lo[j], hi[j], d >= half, c[j], s[j]);
+}
+template <typename T>
+__global__ __launch_bounds__(NT) void attention_prep_vec_kernel(float* __restrict__ qf, T* __restrict__ pool, int64_t pool_rows,
+                                                                const T* __restrict__ proj, int64_t stride, int q_off, int k_off, int v_off, int H,
+                                                                int G, int dim, int vdim, int rot_n, const float* __restrict__ rope_k,
+                                                                const float* __restrict__ rope_v, float scale, const int64_t* __restrict__ slot,
+                                                                const int32_t* __restrict__ pos, int chunks) {
+    const unsigned t = blockIdx.x / (unsigned)chunks, idx = (blockIdx.x - t * chunks) * NT + threadIdx.x;
+    const unsigned R = vdim + dim;
+    const int u = idx / (R / 4), c = (idx - u * (R / 4)) * 4, p = pos[t];
+    if (u >= H + G) return;
+    const T* row = proj + (size_t)t * stride;
+    const float* ck = rope_k + (size_t)p * rot_n;
+    float v[4] = {0.f, 0.f, 0.f, 0.f};
+    if (u < H) {
+        if (c >= vdim) {
+            rotated4(row + q_off + u * dim, c - vdim, rot_n, ck, v);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] *= scale;
+        }
+        st4t(qf, ((size_t)t * H + u) * R + c, v);
+    } else {
+        const int g = u - H;
+        if (c < vdim) rotated4(row + v_off + g * vdim, c, vdim, rope_v + (size_t)p * vdim, v);
+        else rotated4(row + k_off + g * dim, c - vdim, rot_n, ck, v);
+        st4t(pool, ((size_t)g * pool_rows + (size_t)slot[t]) * R + c, v);
+    }
+}
+
 // o[t, h, :n] turned by sign * pos[t] in place
 template <typename T>
 __global__ __launch_bounds__(NT) void rotate_heads_kernel(T* __restrict__ o, const float* __restrict__ rope,
@@ -523,6 +748,22 @@ extern "C" int qsv_conv_silu_unit(float* out, const void* proj, int64_t stride, 
                 "qsv_conv_silu_unit: bad sizes");
     QSV_REQUIRE((size_t)channels * 4 <= 64 * 1024, "qsv_conv_silu_unit: %d channels do not fit the workgroup's LDS", channels);
     if (n_tokens == 0) return QSV_OK;
+    const int64_t chunks = ((int64_t)channels / 4 + NT - 1) / NT;
+    if (taps >= 2 && taps <= 4 && channels % 4 == 0 && off % 4 == 0 && stride % 4 == 0 && fits4(proj, dtype) && fits4(out, QSV_F32) &&
+        fits4(w, QSV_F32) && fits4(hist, QSV_F32) && chunks * n_tokens < (1ll << 31) &&
+        (n_unit == 0 || (unit_dim >= 4 && unit_dim <= 256 && (unit_dim & (unit_dim - 1)) == 0))) {
+        const dim3 grid((unsigned)(chunks * n_tokens));
+        const int lanes = n_unit ? unit_dim / 4 : 1;
+#define QSV_CONV(TAPS)                                                                                                                        \
+    QSV_DISPATCH(dtype, "qsv_conv_silu_unit",                                                                                                 \
+                 hipLaunchKernelGGL((conv_silu_unit_vec_kernel<T, TAPS>), grid, dim3(NT), 0, (hipStream_t)stream, out, (const T*)proj, stride, \
+                                    off, channels, w, hist, run_off, state_rd, state_wr, n_unit* unit_dim, lanes, act, (int)chunks))
+        if (taps == 4) QSV_CONV(4);
+        else if (taps == 3) QSV_CONV(3);
+        else QSV_CONV(2);
+#undef QSV_CONV
+        return qsv_launch_status("qsv_conv_silu_unit");
+    }
     QSV_DISPATCH(dtype, "qsv_conv_silu_unit",
                  hipLaunchKernelGGL(conv_silu_unit_kernel<T>, dim3(n_tokens), dim3(NT), (size_t)channels * 4, (hipStream_t)stream, out,
                                     (const T*)proj, stride, off, channels, taps, w, hist, run_off, state_rd, state_wr, n_unit,
@@ -530,6 +771,18 @@ extern "C" int qsv_conv_silu_unit(float* out, const void* proj, int64_t stride, 
     return qsv_launch_status("qsv_conv_silu_unit");
 }
 
+// the operand types a step's launch is made for
+#define QSV_STEP_TYPES                                                                                     \
+    if (beta) {                                                                                            \
+        if (qkv_dtype == QSV_F32 && beta_dtype == QSV_F32) QSV_STEP(float, float, true);                   \
+        else if (qkv_dtype == QSV_F32 && beta_dtype == QSV_BF16) QSV_STEP(float, bf16_t, true);            \
+        else if (qkv_dtype == QSV_BF16 && beta_dtype == QSV_BF16) QSV_STEP(bf16_t, bf16_t, true);          \
+        else QSV_REQUIRE(false, "qsv_recurrent_scan: operand types %d / %d", qkv_dtype, beta_dtype);       \
+    } else {                                                                                               \
+        if (qkv_dtype == QSV_F32) QSV_STEP(float, float, false);                                           \
+        else if (qkv_dtype == QSV_BF16) QSV_STEP(bf16_t, bf16_t, false);                                   \
+        else QSV_REQUIRE(false, "qsv_recurrent_scan: operand type %d", qkv_dtype);                         \
+    }
 extern "C" int qsv_recurrent_scan(float* o, const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v,
                                   int64_t v_stride, int qkv_dtype, const float* decay, const void* beta, int64_t beta_stride,
                                   int beta_dtype, float* state, const int32_t* runs, int n_runs, int max_run, int heads, int qk_heads,
@@ -538,6 +791,25 @@ extern "C" int qsv_recurrent_scan(float* o, const void* q, int64_t q_stride, con
     if (v_cols <= 0) v_cols = vdim;
     QSV_REQUIRE(v_cols <= vdim, "qsv_recurrent_scan: %d value columns for a state of %d", v_cols, vdim);
     if (max_run == 1 && n_runs > 0 && dim <= 64 * 8 && heads > 0 && qk_heads > 0 && heads % qk_heads == 0 && vdim > 0 && heads <= 65535) {
+        const int qkv = qkv_dtype == QSV_F32 ? QSV_F32 : QSV_BF16;
+        if (dim % 8 == 0 && dim <= 256 && vdim % 4 == 0 && q_stride % 4 == 0 && k_stride % 4 == 0 && fits4(q, qkv) && fits4(k, qkv) &&
+            fits4(decay, QSV_F32) && fits4(state, QSV_F32) && fits4(o, QSV_F32) && (vdim + 127) / 128 <= 65535) {
+            const dim3 grid(n_runs, heads, (vdim + 127) / 128), block(256);   // (heads and vdim are checked above)
+#define QSV_STEP_P(TQ, TB, DELTA, P)                                                                                            \
+    hipLaunchKernelGGL((recurrent_step_wide_kernel<TQ, TB, DELTA, P>), grid, block, 0, (hipStream_t)stream, o, (const TQ*)q, q_stride, \
+                       (const TQ*)k, k_stride, (const TQ*)v, v_stride, decay, (const TB*)beta, beta_stride, state, runs, heads,  \
+                       qk_heads, dim, vdim, q_scale, kscale, head_decay, v_cols)
+#define QSV_STEP(TQ, TB, DELTA)                            \
+    do {                                                   \
+        if (dim <= 64) QSV_STEP_P(TQ, TB, DELTA, 1);       \
+        else if (dim <= 128) QSV_STEP_P(TQ, TB, DELTA, 2); \
+        else QSV_STEP_P(TQ, TB, DELTA, 4);                 \
+    } while (0)
+            QSV_STEP_TYPES
+#undef QSV_STEP
+#undef QSV_STEP_P
+            return qsv_launch_status("qsv_recurrent_scan");
+        }
         int lpc = 1, lpc_log = 0;
         while (lpc * 8 < dim) lpc <<= 1, ++lpc_log;
         const int per_block = 4 * (64 / lpc);
@@ -547,16 +819,7 @@ extern "C" int qsv_recurrent_scan(float* o, const void* q, int64_t q_stride, con
     hipLaunchKernelGGL((recurrent_step_kernel<TQ, TB, DELTA>), grid, block, 0, (hipStream_t)stream, o, (const TQ*)q, q_stride,    \
                        (const TQ*)k, k_stride, (const TQ*)v, v_stride, decay, (const TB*)beta, beta_stride, state, runs, heads,  \
                        qk_heads, dim, vdim, lpc_log, q_scale, kscale, head_decay, v_cols)
-        if (beta) {
-            if (qkv_dtype == QSV_F32 && beta_dtype == QSV_F32) QSV_STEP(float, float, true);
-            else if (qkv_dtype == QSV_F32 && beta_dtype == QSV_BF16) QSV_STEP(float, bf16_t, true);
-            else if (qkv_dtype == QSV_BF16 && beta_dtype == QSV_BF16) QSV_STEP(bf16_t, bf16_t, true);
-            else QSV_REQUIRE(false, "qsv_recurrent_scan: operand types %d / %d", qkv_dtype, beta_dtype);
-        } else {
-            if (qkv_dtype == QSV_F32) QSV_STEP(float, float, false);
-            else if (qkv_dtype == QSV_BF16) QSV_STEP(bf16_t, bf16_t, false);
-            else QSV_REQUIRE(false, "qsv_recurrent_scan: operand type %d", qkv_dtype);
-        }
+        QSV_STEP_TYPES
 #undef QSV_STEP
         return qsv_launch_status("qsv_recurrent_scan");
     }
@@ -657,6 +920,19 @@ extern "C" int qsv_head_rms_gate(void* out, const float* o, const void* w, const
     QSV_REQUIRE(o_stride >= vdim && (!den_m || o_stride > vdim), "qsv_head_rms_gate: read-out rows of %d floats for %d values%s",
                 o_stride, vdim, den_m ? " and the normaliser's column" : "");
     if (n_tokens == 0) return QSV_OK;
+    if (vdim >= 4 && vdim <= 256 && (vdim & (vdim - 1)) == 0 && o_stride % 4 == 0 && gate_stride % 4 == 0 && fits4(out, dtype) &&
+        fits4(o, QSV_F32) && fits4(w, dtype) && fits4(gate, dtype) && heads <= (1 << 20)) {
+        int lanes_log = 0;
+        while ((4 << lanes_log) < vdim) ++lanes_log;
+        const int64_t chunks = (((int64_t)heads << lanes_log) + NT - 1) / NT;
+        if (chunks * n_tokens < (1ll << 31)) {
+            QSV_DISPATCH(dtype, "qsv_head_rms_gate",
+                         hipLaunchKernelGGL(head_rms_gate_vec_kernel<T>, dim3((unsigned)(chunks * n_tokens)), dim3(NT), 0, (hipStream_t)stream,
+                                            (T*)out, o, (const T*)w, (const T*)gate, gate_stride, gate_kind, eps, heads, vdim, lanes_log, o_stride,
+                                            w_per_head ? vdim : 0, den_m, (int)chunks));
+            return qsv_launch_status("qsv_head_rms_gate");
+        }
+    }
     QSV_DISPATCH(dtype, "qsv_head_rms_gate",
                  hipLaunchKernelGGL(head_rms_gate_kernel<T>, dim3(n_tokens), dim3(NT), 0, (hipStream_t)stream, (T*)out, o, (const T*)w,
                                     (const T*)gate, gate_stride, gate_kind, eps, heads, vdim, o_stride, w_per_head ? vdim : 0, den_m));
@@ -685,6 +961,16 @@ extern "C" int qsv_attention_prep(float* qf, void* pool, int64_t pool_rows, cons
                     k_off + (int64_t)kv_heads * dim <= stride && v_off + (int64_t)kv_heads * vdim <= stride && n_tokens >= 0,
                 "qsv_attention_prep: bad sizes");
     if (n_tokens == 0) return QSV_OK;
+    const int64_t chunks = (((int64_t)heads + kv_heads) * ((vdim + dim) / 4) + NT - 1) / NT;
+    if (dim % 4 == 0 && vdim % 8 == 0 && rot_n % 8 == 0 && stride % 4 == 0 && q_off % 4 == 0 && k_off % 4 == 0 && v_off % 4 == 0 &&
+        fits4(qf, QSV_F32) && fits4(pool, dtype) && fits4(proj, dtype) && fits4(rope_k, QSV_F32) && fits4(rope_v, QSV_F32) &&
+        chunks * n_tokens < (1ll << 31) && chunks < (1 << 22)) {
+        QSV_DISPATCH(dtype, "qsv_attention_prep",
+                     hipLaunchKernelGGL(attention_prep_vec_kernel<T>, dim3((unsigned)(chunks * n_tokens)), dim3(NT), 0, (hipStream_t)stream, qf,
+                                        (T*)pool, pool_rows, (const T*)proj, stride, q_off, k_off, v_off, heads, kv_heads, dim, vdim, rot_n, rope_k,
+                                        rope_v, scale, slot, pos, (int)chunks));
+        return qsv_launch_status("qsv_attention_prep");
+    }
     QSV_DISPATCH(dtype, "qsv_attention_prep",
                  hipLaunchKernelGGL(attention_prep_kernel<T>, dim3(n_tokens), dim3(NT), 0, (hipStream_t)stream, qf, (T*)pool, pool_rows,
                                     (const T*)proj, stride, q_off, k_off, v_off, heads, kv_heads, dim, vdim, rot_n, rope_k, rope_v,

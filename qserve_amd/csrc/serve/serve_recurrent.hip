@@ -369,6 +369,207 @@ __global__ __launch_bounds__(256, OCC) void recurrent_scan_kernel(float* __restr
             if (j + c < vdim && r0 + i < dim) Sg[(size_t)(r0 + i) * vdim + j + c] = S[c][i];
 }
 
+// ---- the same recurrence for 33 - 128 rows, operands in fours -------------------------------------------------------------------------------
+// A token's step is three or four multiply-adds per element of the state and lane, behind twelve 16-byte LDS reads of its k, q and decay: what
+// bounds it is the wait for those reads and the issue of both.  So a lane holds 16 rows of NC columns (two: every read serves twice as many
+// multiply-adds; one where two would leave CUs without a workgroup), LPC lanes a column; a chunk of 16 tokens is straight-line code in which the
+// next token's operands are requested before the current one is computed; the chunks alternate between two LDS buffers (one barrier each), the
+// chunk after in registers meanwhile.  A run's last tokens, fewer than a chunk, go one by one.  Rows of the parts 4 .. 7 are taken in another
+// order, so that their reads fall on other banks than those of 0 .. 3.
+// Measured (8 runs of 1024 tokens, delta rule / plain; before: the form above): 32 heads of 64 x 128 1102 -> 428 / 1000 -> 365 us, 16 heads 477 -> 253 /
+// 431 -> 220, 32 heads of 128 x 128 2424 -> 617 / 1971 -> 456; 64 runs of 4 tokens 63 -> 21 / 31 -> 18, one of 2 6.8 -> 5.3 / 6.5 -> 4.1.
+// (Reads laid between the rows of the token before, instead of ahead of them: the same time, and spills.)
+constexpr int ROWS_CT = 16;
+template <int NC>
+struct TokenRows {
+    float k[16], q[16], g[16], v[NC], b;
+};
+template <typename TQ, typename TB, bool DELTA, int LPC, int NC>
+__global__ __launch_bounds__(256, 2) void recurrent_rows_kernel(float* __restrict__ o, const TQ* __restrict__ q, int64_t q_stride,
+                                                                const TQ* __restrict__ k, int64_t k_stride, const TQ* __restrict__ v,
+                                                                int64_t v_stride, const float* __restrict__ decay, const TB* __restrict__ beta,
+                                                                int64_t beta_stride, float* __restrict__ state, const int32_t* __restrict__ runs,
+                                                                int H, int QH, int dim, int vdim, float q_scale, const float* __restrict__ kscale,
+                                                                int head_decay, int v_cols) {
+    constexpr int CT = ROWS_CT, D = 16 * LPC, COLS = 64 / LPC, VB = 4 * COLS * NC;
+    constexpr int KP = CT * D / 4 / 256, VPIECES = CT * VB / 4, VP = (VPIECES + 255) / 256;
+    static_assert(CT * D % 1024 == 0, "");
+    __shared__ __attribute__((aligned(16))) float rows[2][3][CT][D];     // k, q, decay
+    __shared__ __attribute__((aligned(16))) float vs[2][CT][VB];
+    __shared__ float rates[2][CT];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, part = lane & (LPC - 1), turn = part >> 2;
+    const int cb = (wave * COLS + lane / LPC) * NC, j = blockIdx.z * VB + cb;
+    const int slot = runs[4 * blockIdx.x], first = runs[4 * blockIdx.x + 1], n = runs[4 * blockIdx.x + 2];
+    const bool fresh = runs[4 * blockIdx.x + 3] == 0;
+    const int h = blockIdx.y, qh = h / (H / QH);
+    const bool col_ok = j < vdim;                                  // (vdim is a multiple of 4: both columns or none)
+    float* Sg = state + (((size_t)slot * H + h) * dim) * (size_t)vdim + (col_ok ? j : 0);
+    float S[NC][16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int r = part * 16 + 4 * ((i >> 2) ^ turn) + (i & 3);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) S[c][i] = (!fresh && col_ok && r < dim) ? Sg[(size_t)r * vdim + c] : 0.f;
+    }
+    float4 pk[KP], pq[KP], pg[KP], pv[VP];
+    float pb = 0.f;
+    auto fetch = [&](int c0, int ct) __attribute__((always_inline)) {                 // requests the operands of tokens c0 .. c0 + ct of the run
+#pragma unroll
+        for (int i = 0; i < KP; ++i) {
+            const int piece = tid + 256 * i, tt = piece / (D / 4), r = (piece % (D / 4)) * 4;
+            pk[i] = pq[i] = pg[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (tt < ct && r < dim) {
+                const size_t t = (size_t)(first + c0 + tt);
+                pk[i] = ld4(k, t * k_stride + (size_t)qh * dim + r);
+                pq[i] = ld4(q, t * q_stride + (size_t)qh * dim + r);
+                if (head_decay) {
+                    const float g = head_decay == 2 ? decay[h] : decay[t * H + h];
+                    pg[i] = make_float4(g, g, g, g);
+                } else {
+                    pg[i] = ld4(decay, (t * H + h) * (size_t)dim + r);
+                }
+                if (kscale) {
+                    const float b = kscale[t * H + h];
+                    pk[i].x *= b; pk[i].y *= b; pk[i].z *= b; pk[i].w *= b;
+                }
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < VP; ++i) {
+            const int piece = tid + 256 * i, tt = piece / (VB / 4), jj = blockIdx.z * VB + (piece % (VB / 4)) * 4;
+            pv[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (tt < ct) {
+                if (jj < v_cols) pv[i] = ld4(v, (size_t)(first + c0 + tt) * v_stride + (size_t)h * v_cols + jj);
+                else if (jj == v_cols && jj < vdim) pv[i].x = 1.0f;       // the state's column of ones (a state wider than v)
+            }
+        }
+        if (DELTA && tid < ct) pb = ld(beta, (size_t)(first + c0 + tid) * beta_stride + h);
+    };
+    auto stage = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < KP; ++i) {
+            const int piece = tid + 256 * i, tt = piece / (D / 4), r = (piece % (D / 4)) * 4;
+            *(float4*)&rows[buf][0][tt][r] = pk[i];
+            *(float4*)&rows[buf][1][tt][r] = pq[i];
+            *(float4*)&rows[buf][2][tt][r] = pg[i];
+        }
+#pragma unroll
+        for (int i = 0; i < VP; ++i) {
+            const int piece = tid + 256 * i;
+            if (VPIECES % 256 == 0 || piece < VPIECES) *(float4*)&vs[buf][piece / (VB / 4)][(piece % (VB / 4)) * 4] = pv[i];
+        }
+        if (DELTA && tid < CT) rates[buf][tid] = 1.0f / (1.0f + expf(-pb));
+    };
+    auto request = [&](TokenRows<NC>& x, int buf, int tt) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = part * 16 + 4 * (i ^ turn);
+            const float4 a = *(const float4*)&rows[buf][0][tt][r], b = *(const float4*)&rows[buf][1][tt][r], c = *(const float4*)&rows[buf][2][tt][r];
+            x.k[4 * i] = a.x, x.k[4 * i + 1] = a.y, x.k[4 * i + 2] = a.z, x.k[4 * i + 3] = a.w;
+            x.q[4 * i] = b.x, x.q[4 * i + 1] = b.y, x.q[4 * i + 2] = b.z, x.q[4 * i + 3] = b.w;
+            x.g[4 * i] = c.x, x.g[4 * i + 1] = c.y, x.g[4 * i + 2] = c.z, x.g[4 * i + 3] = c.w;
+        }
+#pragma unroll
+        for (int c = 0; c < NC; ++c) x.v[c] = vs[buf][tt][cb + c];
+        x.b = DELTA ? rates[buf][tt] : 0.f;
+    };
+    auto step = [&](const TokenRows<NC>& x, float (&out)[NC]) __attribute__((always_inline)) {   // out: this lane's share of the read-out
+        float u[NC];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            u[c] = x.v[c];
+            if (DELTA) {
+                float a = 0.f, b = 0.f;
+#pragma unroll
+                for (int i = 0; i < 16; i += 2) {
+                    S[c][i] *= x.g[i];
+                    S[c][i + 1] *= x.g[i + 1];
+                    a += S[c][i] * x.k[i];
+                    b += S[c][i + 1] * x.k[i + 1];
+                }
+                u[c] = a + b;
+            }
+        }
+        if (DELTA) {
+#pragma unroll
+            for (int c = 0; c < NC; ++c) u[c] = (x.v[c] - column_sum(u[c], LPC)) * x.b;
+        }
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            float a = 0.f, b = 0.f;
+#pragma unroll
+            for (int i = 0; i < 16; i += 2) {
+                S[c][i] = (DELTA ? S[c][i] : x.g[i] * S[c][i]) + x.k[i] * u[c];
+                S[c][i + 1] = (DELTA ? S[c][i + 1] : x.g[i + 1] * S[c][i + 1]) + x.k[i + 1] * u[c];
+                a += S[c][i] * x.q[i];
+                b += S[c][i + 1] * x.q[i + 1];
+            }
+            out[c] = a + b;
+        }
+    };
+    fetch(0, min(CT, n));
+    int buf = 0;
+    for (int c0 = 0; c0 < n; c0 += CT, buf ^= 1) {
+        const int ct = min(CT, n - c0);
+        stage(buf);
+        __syncthreads();                                           // (the other buffer: every wave is behind the chunk that read it)
+        if (c0 + CT < n) fetch(c0 + CT, min(CT, n - c0 - CT));     // in flight while this chunk is computed
+        float* og = o + ((size_t)(first + c0) * H + h) * (size_t)vdim + j;
+        if (ct == CT) {
+            float out[8][NC];
+            TokenRows<NC> x[2];
+            request(x[0], buf, 0);
+#pragma unroll
+            for (int tt = 0; tt < CT; ++tt) {
+                if (tt + 1 < CT) request(x[(tt + 1) & 1], buf, tt + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                step(x[tt & 1], out[tt & 7]);
+                __builtin_amdgcn_sched_barrier(0);
+                if ((tt & 7) != 7) continue;
+#pragma unroll
+                for (int s = 0; s < 8; ++s)
+#pragma unroll
+                    for (int c = 0; c < NC; ++c) out[s][c] = column_sum(out[s][c], LPC);
+#pragma unroll
+                for (int t0 = 0; t0 < 8; t0 += LPC) {              // lane `part` of a column writes token t0 + part of the eight
+                    float w[NC];
+#pragma unroll
+                    for (int c = 0; c < NC; ++c) {
+                        w[c] = out[t0][c];
+#pragma unroll
+                        for (int p = 1; p < LPC; ++p) w[c] = part == p ? out[t0 + p][c] : w[c];
+                        w[c] *= q_scale;
+                    }
+                    if (col_ok) {
+                        float* d = og + (size_t)(tt - 7 + t0 + part) * H * vdim;
+                        if (NC == 2) *(float2*)d = make_float2(w[0], w[NC - 1]);
+                        else *d = w[0];
+                    }
+                }
+            }
+        } else {
+            for (int tt = 0; tt < ct; ++tt) {
+                TokenRows<NC> x;
+                float out[NC];
+                request(x, buf, tt);
+                step(x, out);
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    const float w = column_sum(out[c], LPC) * q_scale;
+                    if (col_ok && part == 0) og[(size_t)tt * H * vdim + c] = w;
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int r = part * 16 + 4 * ((i >> 2) ^ turn) + (i & 3);
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+            if (col_ok && r < dim) Sg[(size_t)r * vdim + c] = S[c][i];
+    }
+}
+
 // ---- one token per run (decoding): no staging, no barriers - every lane fetches its 8 rows of k, q and the decay itself, the
 // state makes one round trip -----------------------------------------------------------------------------------------------------
 template <typename TQ, typename TB, bool DELTA>
@@ -823,6 +1024,34 @@ extern "C" int qsv_recurrent_scan(float* o, const void* q, int64_t q_stride, con
 #undef QSV_STEP
         return qsv_launch_status("qsv_recurrent_scan");
     }
+    QSV_REQUIRE(heads > 0 && qk_heads > 0 && heads % qk_heads == 0 && dim > 0 && dim <= 64 * 16 && vdim > 0 && n_runs >= 0 &&
+                    heads <= 65535,
+                "qsv_recurrent_scan: bad sizes (%d heads over %d, state %d x %d)", heads, qk_heads, dim, vdim);
+    if (n_runs == 0) return QSV_OK;
+    const int qkv = qkv_dtype == QSV_F32 ? QSV_F32 : QSV_BF16;
+    if (dim > 32 && dim <= 128 && dim % 4 == 0 && vdim % 4 == 0 && v_cols % 4 == 0 && q_stride % 4 == 0 && k_stride % 4 == 0 && v_stride % 4 == 0 &&
+        fits4(q, qkv) && fits4(k, qkv) && fits4(v, qkv) && fits4(decay, QSV_F32) && fits4(o, QSV_F32) && vdim <= 65535 * 32) {
+        const int lpc = dim <= 64 ? 4 : 8, cols = 4 * 64 / lpc;
+        // two columns per lane while that gives every CU a workgroup (half as many CUs: a token costs them as much as it would cost all)
+        const bool two = (int64_t)n_runs * heads * ((vdim + 2 * cols - 1) / (2 * cols)) >= 256;
+        const dim3 grid(n_runs, heads, two ? (vdim + 2 * cols - 1) / (2 * cols) : (vdim + cols - 1) / cols), block(256);
+#define QSV_STEP_P(TQ, TB, DELTA, LPC, NC)                                                                                      \
+    hipLaunchKernelGGL((recurrent_rows_kernel<TQ, TB, DELTA, LPC, NC>), grid, block, 0, (hipStream_t)stream, o, (const TQ*)q, q_stride, \
+                       (const TQ*)k, k_stride, (const TQ*)v, v_stride, decay, (const TB*)beta, beta_stride, state, runs, heads,  \
+                       qk_heads, dim, vdim, q_scale, kscale, head_decay, v_cols)
+#define QSV_STEP(TQ, TB, DELTA)                                      \
+    do {                                                             \
+        if (lpc == 4 && two) QSV_STEP_P(TQ, TB, DELTA, 4, 2);        \
+        else if (lpc == 4) QSV_STEP_P(TQ, TB, DELTA, 4, 1);          \
+        else if (two) QSV_STEP_P(TQ, TB, DELTA, 8, 2);               \
+        else QSV_STEP_P(TQ, TB, DELTA, 8, 1);                        \
+    } while (0)
+        QSV_STEP_TYPES
+#undef QSV_STEP
+#undef QSV_STEP_P
+        return qsv_launch_status("qsv_recurrent_scan");
+    }
+    // States of other heights, and operands that are not in fours.
     // Rows of one column per lane: 8 while that leaves the launch at no more than ~2.5 waves per SIMD, else 16 (and for the tallest
     // states).  Measured at 16 heads, 64 x 128 states: 8 x 1024 tokens (2048 / 1024 waves) 0.46 / 0.51 ms plain, 0.50 / 0.55 ms
     // delta rule; 64 single tokens (16384 / 8192 waves) 56 / 43 us; two columns per lane 0.60 / 0.75 ms.  A token's step is a
@@ -854,10 +1083,6 @@ extern "C" int qsv_recurrent_scan(float* o, const void* q, int64_t q_stride, con
             R = 8;
         }
     }
-    QSV_REQUIRE(heads > 0 && qk_heads > 0 && heads % qk_heads == 0 && dim > 0 && dim <= 64 * 16 && vdim > 0 && n_runs >= 0 &&
-                    heads <= 65535,
-                "qsv_recurrent_scan: bad sizes (%d heads over %d, state %d x %d)", heads, qk_heads, dim, vdim);
-    if (n_runs == 0) return QSV_OK;
     int lpc = 1, lpc_log = 0;
     while (lpc * R < dim) lpc <<= 1, ++lpc_log;
     QSV_REQUIRE(lpc <= 64, "qsv_recurrent_scan: %d rows per lane for a state of %d rows", R, dim);

@@ -121,6 +121,33 @@ def test_one_token_of_the_recurrence(H, G, dim, vdim, v_cols, dtype, delta):
             assert ((o - ref).abs() <= bound).all() and ((s1 - s2).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("delta", [True, False])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("counts, H, G, dim, vdim, v_cols", [((1, 15, 16, 17, 33), 2, 1, 64, 128, 128), ((31, 32), 130, 65, 64, 132, 128), ((5, 48), 3, 3, 36, 4, 4),
+                                                             ((16, 49), 2, 1, 68, 36, 32), ((2, 40), 128, 64, 128, 64, 64), ((20, 3), 2, 2, 128, 68, 68),
+                                                             ((18, 2), 2, 2, 32, 64, 64), ((17, 2), 2, 2, 132, 12, 12), ((17, 2), 2, 2, 34, 10, 9)])
+def test_runs_of_the_recurrence(counts, H, G, dim, vdim, v_cols, dtype, delta):
+    """Full chunks of 16 tokens and what is left of them, one and two columns per lane, rows and columns that do not fill a workgroup."""
+    g = _gen(dim + vdim)
+    b = _batch(list(counts), [5, 0, 2, 0, 1][:len(counts)])
+    T = sum(counts)
+    unit = lambda *s: torch.nn.functional.normalize(torch.randn(*s, device=DEV, generator=g), dim=-1)       # noqa: E731
+    q, k = unit(T, G, dim).view(T, -1).to(dtype), unit(T, G, dim).view(T, -1).to(dtype)
+    v = torch.randn(T, H * v_cols, device=DEV, generator=g).to(dtype)
+    beta = torch.randn(T, H, device=DEV, generator=g).to(dtype) if delta else None
+    state = torch.randn(6, H, dim, vdim, device=DEV, generator=g).clamp(-4, 4)
+    for i, shape in enumerate(((T, H * dim), (T, H), (H,))):
+        decay, ks = torch.rand(*shape, device=DEV, generator=g) * 0.9, torch.rand(T, H, device=DEV, generator=g) if i == 1 else None
+        s1, s2 = state.clone(), state.clone()
+        o = HipOps(dtype).recurrent_scan(q, k, v, decay, beta, s1, b, H, G, dim, vdim, 0.5, ks, v_cols)
+        ref = TorchOps(dtype).recurrent_scan(q, k, v, decay, beta, s2, b, H, G, dim, vdim, 0.5, ks, v_cols)
+        # a token's own error as above (|S| <= 64: inputs below 8, decays below 0.9), carried on by decays of 0.9 at most: ten times it
+        bound = 10 * 4 * 2.0 ** -24 * (dim + 8) * 64 * (dim ** 0.5 + 4)
+        assert ((o - ref).abs() <= bound).all() and ((s1 - s2).abs() <= bound).all()
+        # and element by element against what rounding of that kind does on average (its square root): a wrong row or column stands out by far
+        assert ((o - ref).norm() / ref.norm()).item() < 2.0 ** -24 * dim * 16 and ((s1 - s2).norm() / s2.norm()).item() < 2.0 ** -24 * dim * 16
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("S, D", [(2, 4), (2, 1020), (3, 1028), (2, 2048), (4, 2052), (2, 6)])
 def test_streams_read_and_written(S, D, dtype):

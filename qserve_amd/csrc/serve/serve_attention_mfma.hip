@@ -511,20 +511,203 @@ __global__ __launch_bounds__(64 * RW, RT + CT > 24 ? 2 : 4) void latent_rows_ker
         *(v2u*)(o + 16 * c) = v2u{pack_bf2(oacc[c][0] * inv, oacc[c][1] * inv), pack_bf2(oacc[c][2] * inv, oacc[c][3] * inv)};
 }
 
-// out[t, h] = sum_z e^(m_z - M) o_z / sum_z e^(m_z - M) l_z   (one workgroup per (token, head))
-__global__ __launch_bounds__(256) void latent_attention_merge_kernel(bf16_t* __restrict__ out, const float* __restrict__ part_o,
+// ---- the same rows for steps: one token per tile ----------------------------------------------------------------------------------------------
+// With one token a single wave of the kernel above has queries, and a step waits for it: 64 keys took 4 us.  Here four waves share the token:
+// rounds of 64 keys, copied as above (two rounds in turn); a wave scores 16 of the keys (its rows of K only), the maximum and the
+// probabilities of a round meet in LDS, and a wave multiplies them with its quarter of the value columns.  Bound by latency at short contexts, by
+// HBM at long ones.
+// Measured (16 heads, 576 / 512, best split each, kernel above -> this one and the merge below): 64 sequences at 128 / 1000 / 2000 positions 15 -> 12 / 31 ->
+// 28 / 44 -> 37 us, 16 at 1000 25 -> 18, one at 300 / 2000 17 -> 13 / 28 -> 16; 256 / 128, 16 heads on 4 pools, 16 sequences at 1000: 15 -> 11.5 us.
+constexpr int SW = 4, SN = 64;       // waves, keys of a round
+template <int RT, int CT, int S0>
+__global__ __launch_bounds__(64 * SW, 1) void latent_step_kernel(
+    bf16_t* __restrict__ out, const float* __restrict__ qf, const bf16_t* __restrict__ pool_base, const int32_t* __restrict__ block_table,
+    int table_stride, const int32_t* __restrict__ pos, const int32_t* __restrict__ tiles, int window, int H, int page, int HP,
+    float* __restrict__ part_o, float* __restrict__ part_ml, int n_tokens, int per, int64_t pool_stride) {
+    constexpr int R = 32 * RT, RANK = 16 * CT, PPR = R / 8, TILE = SN * R * 2, NJ = 32 * PPR / 64 / SW, WC = CT / SW;
+    static_assert(32 * PPR % (64 * SW) == 0 && CT % SW == 0 && 2 * TILE + 4096 <= 160 * 1024, "");
+    __shared__ __attribute__((aligned(128))) unsigned char buf[2 * TILE];
+    __shared__ float tops[SW][16], sums[SW][16];
+    __shared__ uint2 probs[SW][64];
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6) & (SW - 1);
+    const int col = lane & 15, g4 = lane >> 4;
+    const int32_t* tl = tiles + 3 * (int)blockIdx.x;
+    const int slot = __builtin_amdgcn_readfirstlane(tl[0]), t = __builtin_amdgcn_readfirstlane(tl[1]);
+    const int gpp = (per + 15) / 16, pool_id = blockIdx.y / gpp;
+    const int h0 = pool_id * per + (blockIdx.y % gpp) * 16, h_end = pool_id * per + per;
+    const bf16_t* __restrict__ pool = pool_base + (size_t)pool_id * (size_t)pool_stride;
+    const int32_t* bt = block_table + (size_t)slot * table_stride;
+    const int head = h0 + col;
+    const bool row_ok = col < HP && head < h_end;
+    const int p_row = __builtin_amdgcn_readfirstlane(pos[t]), lo_row = window > 0 ? max(0, p_row - window + 1) : 0;
+    const int kstart = lo_row / BN * BN, nT = (p_row - kstart) / SN + 1, last_half = (p_row - kstart) / BN;
+    const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(lds_ptr)buf);
+    // piece i = 64 (w + SW j) + lane of a half round's BN x PPR, permuted by the row's number; halves behind the last position repeat its half,
+    // rows behind it its row
+    auto copy_half = [&](int half, int page_id, int at) __attribute__((always_inline)) {
+        const int k0 = kstart + min(half, last_half) * BN;
+        const bf16_t* base = pool + ((size_t)page_id * page + (size_t)(k0 % page)) * (size_t)R;
+        const int left = p_row - k0;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const int i = 64 * (w + SW * j) + lane, row = i / PPR;
+            const unsigned off = (unsigned)(min(row, left) * PPR + ((i - row * PPR) ^ row_turn(row))) * 16u;
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base),
+                         "s"(lds0 + at + (w + SW * j) * 1024)
+                         : "memory");
+        }
+    };
+    const int Z = gridDim.z, z = blockIdx.z;
+    auto page_of = [&](int half) __attribute__((always_inline)) { return bt[(kstart + min(half, last_half) * BN) / page]; };
+    auto copy = [&](int round, int which) __attribute__((always_inline)) {
+        const int a = __builtin_amdgcn_readfirstlane(page_of(2 * round)), b = __builtin_amdgcn_readfirstlane(page_of(2 * round + 1));
+        copy_half(2 * round, a, which * TILE);
+        copy_half(2 * round + 1, b, which * TILE + TILE / 2);
+    };
+    if (z < nT) copy(z, 0);
+    v4u qfrag[RT];
+    {
+        const float* qrow = qf + ((size_t)t * H + (row_ok ? head : h0)) * (size_t)R;
+#pragma unroll
+        for (int s = 0; s < RT; ++s) {
+            qfrag[s] = v4u{0u, 0u, 0u, 0u};
+            if (row_ok && s >= S0) {
+                const float4 a = *(const float4*)(qrow + 32 * s + 8 * g4), b = *(const float4*)(qrow + 32 * s + 8 * g4 + 4);
+                qfrag[s] = v4u{pack_bf2(a.x, a.y), pack_bf2(a.z, a.w), pack_bf2(b.x, b.y), pack_bf2(b.z, b.w)};
+            }
+        }
+    }
+    v4f oacc[WC];
+#pragma unroll
+    for (int c = 0; c < WC; ++c) oacc[c] = v4f{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.f;
+    // K: key 16 w + col of the round, pieces 4 s + g4;  V: keys 4 g4 + col / 4 (+ 16, + 32, + 48), column tile WC w + c
+    const int k_at = (16 * w + col) * (R * 2), k_odd[2] = {(g4 ^ row_turn(col)) << 4, ((4 + g4) ^ row_turn(col)) << 4};
+    const int vk = 4 * g4 + (col >> 2);
+    int v_at[WC];
+#pragma unroll
+    for (int c = 0; c < WC; ++c) {
+        const int ct = WC * w + c;
+        v_at[c] = vk * (R * 2) + (col & 1) * 8 + (ct >> 2) * 128 + (((2 * (ct & 3) + ((col & 3) >> 1)) ^ row_turn(vk)) << 4);
+    }
+    int which = 0;
+    for (int round = z; round < nT; round += Z) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();                                           // this round has landed; the other half has been read by everyone
+        asm volatile("" ::: "memory");
+        const unsigned char* T = buf + which * TILE;
+        which ^= 1;
+        if (round + Z < nT) copy(round + Z, which);
+        v4f sacc[2] = {v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}};
+        v4u kf[RT];
+#pragma unroll
+        for (int s = S0; s < RT; ++s) kf[s] = *(const v4u*)(T + k_at + (s >> 1) * 128 + k_odd[s & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = S0; s < RT; ++s)
+            sacc[s & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, kf[s]), __builtin_bit_cast(bf8, qfrag[s]), sacc[s & 1], 0, 0, 0);
+        float p[4], tmax = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {                                           // this lane: keys 16 w + 4 g4 + r of the round
+            const int key = kstart + round * SN + 16 * w + 4 * g4 + r;
+            p[r] = key <= p_row && key >= lo_row ? sacc[0][r] + sacc[1][r] : -INFINITY;
+            tmax = fmaxf(tmax, p[r]);
+        }
+        tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
+        tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+        if (g4 == 0) tops[w][col] = tmax;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        // the value operands do not wait for the probabilities
+        v4u vf[WC][2];
+#pragma unroll
+        for (int c = 0; c < WC; ++c)
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                const unsigned char* v = T + v_at[c] + b * 32 * (R * 2);
+                const v2u a0 = __builtin_bit_cast(v2u, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)v));
+                const v2u a1 = __builtin_bit_cast(v2u, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)(v + 16 * (R * 2))));
+                vf[c][b] = v4u{a0[0], a0[1], a1[0], a1[1]};
+            }
+        float mnew = m;
+#pragma unroll
+        for (int o = 0; o < SW; ++o) mnew = fmaxf(mnew, tops[o][col]);
+        const float msafe = mnew == -INFINITY ? 0.f : mnew;
+        const float alpha = __expf(m - msafe);                                  // m = -inf: 0
+        float psum = 0.f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            p[r] = __expf(p[r] - msafe);
+            psum += p[r];
+        }
+        l = l * alpha + psum;                                                   // (this lane's share)
+        m = mnew;
+        probs[w][lane] = make_uint2(pack_bf2(p[0], p[1]), pack_bf2(p[2], p[3]));
+        if (__any(alpha != 1.0f)) {
+#pragma unroll
+            for (int c = 0; c < WC; ++c) oacc[c] *= alpha;
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {                                           // 32 keys: k-slot (g4, e) <-> key 16 (e / 4) + 4 g4 + e % 4
+            const uint2 p0 = probs[2 * b][lane], p1 = probs[2 * b + 1][lane];
+            const v4u pb = {p0.x, p0.y, p1.x, p1.y};
+#pragma unroll
+            for (int c = 0; c < WC; ++c)
+                oacc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, vf[c][b]), __builtin_bit_cast(bf8, pb), oacc[c], 0, 0, 0);
+        }
+    }
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    if (g4 == 0) sums[w][col] = l;
+    __syncthreads();
+    l = (sums[0][col] + sums[1][col]) + (sums[2][col] + sums[3][col]);
+    if (!row_ok) return;
+    const size_t my_row = (size_t)t * H + head;
+    const int c0 = 16 * WC * w + 4 * g4;
+    if (Z > 1) {
+        const size_t rowi = (size_t)z * n_tokens * H + my_row;
+        if (w == 0 && g4 == 0) {
+            part_ml[rowi * 2] = m;
+            part_ml[rowi * 2 + 1] = l;
+        }
+        float* po = part_o + rowi * RANK + c0;
+#pragma unroll
+        for (int c = 0; c < WC; ++c) *(v4f*)(po + 16 * c) = oacc[c];
+        return;
+    }
+    const float inv = 1.0f / l;
+    bf16_t* o = out + my_row * RANK + c0;
+#pragma unroll
+    for (int c = 0; c < WC; ++c)
+        *(v2u*)(o + 16 * c) = v2u{pack_bf2(oacc[c][0] * inv, oacc[c][1] * inv), pack_bf2(oacc[c][2] * inv, oacc[c][3] * inv)};
+}
+
+// out[t, h] = sum_z e^(m_z - M) o_z / sum_z e^(m_z - M) l_z   (one workgroup per (token, head); rank a multiple of 4, at most 64 splits: lane z of
+// every wave weighs split z, a thread adds four columns, four splits requested at a time)
+__global__ __launch_bounds__(128) void latent_attention_merge_kernel(bf16_t* __restrict__ out, const float* __restrict__ part_o,
                                                                      const float* __restrict__ part_ml, int Z, int rows, int rank) {
     const size_t r = blockIdx.x;
-    float M = -INFINITY;
-    for (int z = 0; z < Z; ++z) M = fmaxf(M, part_ml[((size_t)z * rows + r) * 2]);
-    float L = 0.f;
-    for (int z = 0; z < Z; ++z) L += __expf(part_ml[((size_t)z * rows + r) * 2] - M) * part_ml[((size_t)z * rows + r) * 2 + 1];
-    const float inv = 1.0f / L;
-    for (int c = threadIdx.x; c < rank; c += 256) {
-        float a = 0.f;
-        for (int z = 0; z < Z; ++z)
-            a += __expf(part_ml[((size_t)z * rows + r) * 2] - M) * part_o[((size_t)z * rows + r) * (size_t)rank + c];
-        out[r * (size_t)rank + c] = f2bf(a * inv);
+    const int lane = threadIdx.x & 63;
+    const float2 ml = lane < Z ? *(const float2*)(part_ml + ((size_t)lane * rows + r) * 2) : make_float2(-INFINITY, 0.f);
+    const float M = wave_max(ml.x), e = lane < Z ? __expf(ml.x - M) : 0.f;
+    const float inv = 1.0f / wave_sum(e * ml.y);
+    for (int c = threadIdx.x * 4; c < rank; c += 128 * 4) {
+        const float* po = part_o + r * (size_t)rank + c;
+        const size_t step = (size_t)rows * rank;
+        v4f a = v4f{0.f, 0.f, 0.f, 0.f};
+        for (int z = 0; z < Z; z += 4) {
+            v4f v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = *(const v4f*)(po + (size_t)min(z + i, Z - 1) * step);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (z + i < Z) a += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(e), z + i)) * v[i];
+        }
+        *(v2u*)(out + r * (size_t)rank + c) = v2u{pack_bf2(a[0] * inv, a[1] * inv), pack_bf2(a[2] * inv, a[3] * inv)};
     }
 }
 
@@ -602,7 +785,7 @@ extern "C" int qsv_latent_attention_mfma(void* out, const float* qf, const void*
     if (key_splits > 1) {
         const int rc = qsv_launch_status("qsv_latent_attention_mfma");
         if (rc != QSV_OK) return rc;
-        hipLaunchKernelGGL(latent_attention_merge_kernel, dim3(n_tokens * H), dim3(256), 0, (hipStream_t)stream, (bf16_t*)out,
+        hipLaunchKernelGGL(latent_attention_merge_kernel, dim3(n_tokens * H), dim3(128), 0, (hipStream_t)stream, (bf16_t*)out,
                            part_o, part_ml, key_splits, n_tokens * H, rank);
     }
     return qsv_launch_status("qsv_latent_attention_mfma");
@@ -631,15 +814,24 @@ extern "C" int qsv_latent_rows(void* out, const float* qf, const void* pool, con
     hipLaunchKernelGGL((latent_rows_kernel<RT, CT, S0>), grid, block, 0, (hipStream_t)stream, (bf16_t*)out, qf, (const bf16_t*)pool,             \
                        block_table, table_stride, pos, tiles, n_tiles, window, H, page, g.HP, g.TQ, part_o, part_ml, n_tokens, heads_per_pool,   \
                        pool_stride)
-    if (R == 576) QSV_ROWS(18, 32, 0);
+#define QSV_STEP_ROWS(RT, CT, S0)                                                                                                              \
+    hipLaunchKernelGGL((latent_step_kernel<RT, CT, S0>), grid, dim3(64 * SW), 0, (hipStream_t)stream, (bf16_t*)out, qf, (const bf16_t*)pool,   \
+                       block_table, table_stride, pos, tiles, window, H, page, g.HP, part_o, part_ml, n_tokens, heads_per_pool, pool_stride)
+    if (n_tiles == n_tokens) {                                                 // (every tile holds a token, so each holds one)
+        if (R == 576) QSV_STEP_ROWS(18, 32, 0);
+        else if (R == 512) QSV_STEP_ROWS(16, 32, 0);
+        else if (q_first >= 128) QSV_STEP_ROWS(8, 8, 4);
+        else QSV_STEP_ROWS(8, 8, 0);
+    } else if (R == 576) QSV_ROWS(18, 32, 0);
     else if (R == 512) QSV_ROWS(16, 32, 0);
     else if (q_first >= 128) QSV_ROWS(8, 8, 4);
     else QSV_ROWS(8, 8, 0);
 #undef QSV_ROWS
+#undef QSV_STEP_ROWS
     if (key_splits > 1) {
         const int rc = qsv_launch_status("qsv_latent_rows");
         if (rc != QSV_OK) return rc;
-        hipLaunchKernelGGL(latent_attention_merge_kernel, dim3(n_tokens * H), dim3(256), 0, (hipStream_t)stream, (bf16_t*)out, part_o, part_ml,
+        hipLaunchKernelGGL(latent_attention_merge_kernel, dim3(n_tokens * H), dim3(128), 0, (hipStream_t)stream, (bf16_t*)out, part_o, part_ml,
                            key_splits, n_tokens * H, rank);
     }
     return qsv_launch_status("qsv_latent_rows");

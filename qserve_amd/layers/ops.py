@@ -187,8 +187,17 @@ class HipOps:
             tiles = batch.tiles(self.L.qsv_latent_rows_tile_tokens(per))
             groups = tiles.size(0) * (H // per) * ((per + 15) // 16)
             span = min(batch.max_pos + 1, int(window)) if window else batch.max_pos + 1
-            # (one workgroup per CU at 512 columns and more, two below; measured best at 64 sequences of 1000 and 4000 positions)
-            splits = max(1, min((256 if R > 320 else 512) // max(groups, 1), span // 64, 32)) if key_splits is None else key_splits
+            # (one workgroup per CU at 512 columns and more, two below)
+            wide = R > 320
+            if tiles.size(0) == T:              # one token per tile: the kernel for steps
+                # A split costs a trip of its partial result through memory and the merge, 2 - 3 us at two splits, 64 keys about 2 us: none up to 256
+                # keys (16 heads, 576 wide, 64 sequences of 128 / 200 / 500 / 1000 positions, one / two / four splits: 12 / 14 / 16, 15 / 18 / 18, 28 /
+                # 24 / 23, 43 / 32 / 28 us), then 96 keys or more each while the workgroups fit the chip at once (one sequence of 2000: 64 us with
+                # one, 18 with 8, 16 with 16; 256 wide on 4 pools, 64 sequences of 1000, one / two: 23 / 26 us)
+                splits = max(1, min((256 if wide else 384) // max(groups, 1), span // 96, 32)) if span > 256 else 1
+            else:
+                splits = max(1, min((256 if wide else 512) // max(groups, 1), span // 64, 32))
+            splits = splits if key_splits is None else key_splits
             po = pm = None
             if splits > 1:
                 po = torch.empty((splits, T, H, rank), dtype=torch.float32, device=qf.device)

@@ -13,7 +13,11 @@ pytestmark = pytest.mark.gpu
 # row, rank, heads, pools, first query element; runs: (context, new tokens)
 @pytest.mark.parametrize("R, rank, H, G, q_first", [(576, 512, 16, 1, 0), (512, 512, 20, 1, 0), (576, 512, 3, 1, 0), (256, 128, 12, 3, 128), (256, 128, 34, 2, 0)])
 @pytest.mark.parametrize("runs, window, splits", [(((1, 1), (33, 33)), None, None), (((64, 7), (65, 1), (200, 130)), None, 1), (((300, 1), (31, 1), (96, 1)), None, 5),
-                                                  (((150, 150), (129, 40)), 37, None), (((700, 9),), 64, 3)])
+                                                  (((150, 150), (129, 40)), 37, None), (((700, 9),), 64, 3),
+                                                  # one token each: rounds of 64 keys, halves of 32
+                                                  (tuple((c, 1) for c in (1, 31, 32, 33, 64, 65, 96, 97, 128, 129, 200)), None, 1),
+                                                  (tuple((c, 1) for c in (2, 64, 100, 193)), None, 2), (((700, 1), (65, 1), (3, 1)), 64, 3),
+                                                  (((300, 1), (40, 1)), 37, 1), (((1000, 1),), None, 16), (((1200, 1), (63, 1)), None, None)])
 def test_plain_rows(R, rank, H, G, q_first, runs, window, splits):
     if not torch.cuda.is_available():
         pytest.skip("no GPU")

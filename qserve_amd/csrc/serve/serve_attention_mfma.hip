@@ -593,7 +593,7 @@ __global__ __launch_bounds__(64 * SW, 1) void latent_step_kernel(
     int which = 0;
     for (int round = z; round < nT; round += Z) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();                                           // this round has landed; the other half has been read by everyone
+        __builtin_amdgcn_s_barrier();                                           // these keys have landed; the other half has been read by everyone
         asm volatile("" ::: "memory");
         const unsigned char* T = buf + which * TILE;
         which ^= 1;

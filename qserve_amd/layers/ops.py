@@ -6,7 +6,7 @@
   a GPU never falls back to it.
 
 Conventions: `x` is the float residual stream [T, D]; `h` and every other activation is in the storage type (bfloat16 or
-float32); matrix products are the vendor's (`linear`), with float accumulation.
+float32); matrix products (`linear`, the products per head) are own kernels for a step's few rows and the vendor's beyond, with float accumulation.
 """
 import torch
 

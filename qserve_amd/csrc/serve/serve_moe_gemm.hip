@@ -25,9 +25,11 @@ __device__ __forceinline__ unsigned pack_bf2(float a, float b) { return (unsigne
 // per step.  Workgroups are persistent (one per CU): each finds its tiles from the experts' offsets - no tile list, no count reaches
 // the host -, an XCD's workgroups walk neighbouring tiles (shared weight and input panels in its L2), and the last step of a tile copies the
 // first one of the next, so the epilogue's stores have something to hide behind.  A tile with few slots gives each wave fewer columns
-// instead of multiplying padding.
-// Measured (MI355X, both products with sort and combine): 8192 tokens, 4 of 16 experts of 2048 x 1408: 1010 us -> 490 us (762 TFLOP/s; the form
-// before: 256 x 128 tiles staged through registers, tile list from the host, torch's sort); 32 gated experts of 4096 x 2752: 3.5 -> 2.5 ms (880).
+// instead of multiplying padding, and no copies of inputs it does not have; the tiles of the last, part-empty round are cut into halves or
+// quarters by slots, so that every workgroup has a part.
+// Measured (MI355X, both products with sort and combine): 8192 tokens, 4 of 16 experts of 2048 x 1408: 1010 -> 448 us (844 TFLOP/s; the form before:
+// 256 x 128 tiles staged through registers, tile list from the host, torch's sort; without the cut of the last round 481); 32 gated experts of
+// 4096 x 2752: 3.5 -> 2.46 ms (899; 2.53); 600 tokens of the former 100 us (122).
 constexpr int PR = 256, PS = 256, PWAVES = 8, PT = 64 * PWAVES;
 constexpr int PBUF = (PR + PS) * 128;               // bytes of one K step
 constexpr int MAX_GROUPS = 1024;
@@ -116,25 +118,30 @@ __global__ __launch_bounds__(PT, 2) void grouped_gemm_persistent_kernel(GroupedA
     }
     __syncthreads();
     const int row_tiles = (a.N + PR - 1) / PR, total = __builtin_amdgcn_readfirstlane(tiles_before[a.E]) * row_tiles;
+    // An XCD's share of the tiles: whole rounds of its workgroups, then what is left - fewer tiles than workgroups - cut by slots into as many
+    // parts (two or four) as there are workgroups for.  Place p: tile (p) of the share, or a part of one.
     const int xcd = blockIdx.x & 7, per_xcd = gridDim.x >> 3, chunk = (total + 7) >> 3;
-    const int last = min((xcd + 1) * chunk, total);
-    int at = xcd * chunk + (blockIdx.x >> 3);
+    const int begin = xcd * chunk, here = max(0, min(chunk, total - begin));
+    const int whole = here / per_xcd * per_xcd, rest = here - whole, cut = rest * 4 <= per_xcd ? 2 : rest * 2 <= per_xcd ? 1 : 0;   // log2 of the parts
+    const int last = whole + (rest << cut);
+    int at = blockIdx.x >> 3;
     if (at >= last) return;
 
-    auto tile_at = [&](int L) __attribute__((always_inline)) {
-        const int s = L / row_tiles;                                // which slot tile
+    auto tile_at = [&](int place) __attribute__((always_inline)) {
+        const int over = place - whole, part = over >= 0 ? over & ((1 << cut) - 1) : 0, size = over >= 0 ? PS >> cut : PS;
+        const int L = begin + (over >= 0 ? whole + (over >> cut) : place), s = L / row_tiles;   // which slot tile
         int lo = 0, hi = a.E;                                       // tiles_before[lo] <= s < tiles_before[hi]
         while (hi - lo > 1) {
             const int m = (lo + hi) >> 1;
             if (__builtin_amdgcn_readfirstlane(tiles_before[m]) <= s) lo = m;
             else hi = m;
         }
-        const int skip = __builtin_amdgcn_readfirstlane(tiles_before[lo]), first = a.offsets[lo] + (s - skip) * PS;
+        const int skip = __builtin_amdgcn_readfirstlane(tiles_before[lo]), first = a.offsets[lo] + (s - skip) * PS + part * size;
         GroupedTile t;
         t.e = lo;
         t.n0 = (L % row_tiles) * PR;
         t.first = __builtin_amdgcn_readfirstlane(first);
-        t.ns = __builtin_amdgcn_readfirstlane(min(PS, a.offsets[lo + 1] - first));
+        t.ns = __builtin_amdgcn_readfirstlane(min(size, a.offsets[lo + 1] - first));   // (none or less: a part behind the expert's last slot)
         return t;
     };
     // copies: wave w brings rows 32 w .. 32 w + 31 of the weights and of the inputs, eight rows (of 128 bytes) per instruction
@@ -145,11 +152,14 @@ __global__ __launch_bounds__(PT, 2) void grouped_gemm_persistent_kernel(GroupedA
     };
     const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(lds_ptr)buf) + (unsigned)w * 4096u;
     GroupedTile t = tile_at(at);
+    if (t.ns <= 0) return;                                          // (parts are the last places: nothing follows)
     const bf16_t* W0 = a.W + ((size_t)t.e * a.N + t.n0) * (size_t)a.K;
     unsigned woff[4];
     const unsigned char* xrow[4];
+    int rows_here = 0;                                              // inputs of the tile that is being copied, from this wave's first on
     auto point = [&](const GroupedTile& g, const int (&slot)[4]) __attribute__((always_inline)) {
         W0 = a.W + ((size_t)g.e * a.N + g.n0) * (size_t)a.K;
+        rows_here = g.ns - 32 * w;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             woff[j] = (unsigned)min(32 * w + 8 * j + (lane >> 3), a.N - 1 - g.n0) * (unsigned)a.K * 2u + piece;
@@ -158,7 +168,7 @@ __global__ __launch_bounds__(PT, 2) void grouped_gemm_persistent_kernel(GroupedA
     };
     auto copy = [&](int j, int which, int k0) __attribute__((always_inline)) {   // one of the wave's eight copies of a step
         if (j < 4) lds_copy16(lds0 + which * PBUF + 1024 * j, W0 + k0, woff[j]);
-        else lds_copy16(lds0 + which * PBUF + PR * 128 + 1024 * (j - 4), xrow[j - 4] + (size_t)k0 * 2);
+        else if (8 * (j - 4) < rows_here) lds_copy16(lds0 + which * PBUF + PR * 128 + 1024 * (j - 4), xrow[j - 4] + (size_t)k0 * 2);
     };
     {
         int slot[4];
@@ -175,11 +185,11 @@ __global__ __launch_bounds__(PT, 2) void grouped_gemm_persistent_kernel(GroupedA
     auto run_tile = [&](auto nts) __attribute__((always_inline)) {
         constexpr int NTS = decltype(nts)::value;
         const int next = at + per_xcd;
-        const bool more = next < last;
-        const GroupedTile u = more ? tile_at(next) : t;
+        const GroupedTile u = next < last ? tile_at(next) : t;
+        const bool more = next < last && u.ns > 0;
         int slot[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) slot[j] = x_slot(u, j);
+        for (int j = 0; j < 4; ++j) slot[j] = x_slot(more ? u : t, j);
         v4f acc[4][NTS];
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt)
@@ -230,7 +240,7 @@ __global__ __launch_bounds__(PT, 2) void grouped_gemm_persistent_kernel(GroupedA
         }
         grouped_store<ACT, NTS>(a, t, 64 * wr, s_wave, lane, acc);
         asm volatile("" ::: "memory");                              // (the stores' branches join here: what follows stays uniform)
-        t = u;
+        if (more) t = u;
         at = next;
         return more;
     };

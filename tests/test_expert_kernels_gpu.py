@@ -77,7 +77,9 @@ def test_expert_major_form(ops, T, top, E, ident, D, ff, act, weigh):
 @pytest.mark.parametrize("T, top, E, ident, D, ff, crowd", [
     (1, 1, 1, 0, 64, 64, 0.0), (64, 1, 1, 0, 128, 64, 1.0), (65, 1, 1, 0, 64, 192, 1.0), (128, 1, 1, 0, 320, 128, 1.0), (129, 2, 3, 0, 256, 64, 1.0),
     (256, 1, 2, 0, 64, 320, 1.0), (257, 1, 1, 0, 1088, 64, 1.0), (700, 4, 6, 2, 512, 448, 0.5), (1500, 4, 100, 5, 64, 64, 0.2), (40, 3, 70, 0, 4096, 64, 0.0),
-    (2100, 2, 2, 0, 4096, 128, 0.3)])
+    (2100, 2, 2, 0, 4096, 128, 0.3),
+    # whole rounds of workgroups, and tiles left over in halves and quarters
+    (3000, 2, 8, 0, 64, 2816, 0.0), (2600, 1, 3, 0, 64, 7168, 0.4), (1024, 1, 1, 0, 128, 18432, 1.0)])
 @ACTS
 def test_grouped_form(ops, T, top, E, ident, D, ff, crowd, act, weigh):
     o = make_ops("hip", torch.bfloat16, torch.device("cuda:0"))

@@ -27,9 +27,9 @@ __device__ __forceinline__ unsigned pack_bf2(float a, float b) { return (unsigne
 // first one of the next, so the epilogue's stores have something to hide behind.  A tile with few slots gives each wave fewer columns
 // instead of multiplying padding, and no copies of inputs it does not have; the tiles of the last, part-empty round are cut into halves or
 // quarters by slots, so that every workgroup has a part.
-// Measured (MI355X, both products with sort and combine): 8192 tokens, 4 of 16 experts of 2048 x 1408: 1010 -> 448 us (844 TFLOP/s; the form before:
-// 256 x 128 tiles staged through registers, tile list from the host, torch's sort; without the cut of the last round 481); 32 gated experts of
-// 4096 x 2752: 3.5 -> 2.46 ms (899; 2.53); 600 tokens of the former 100 us (122).
+// Measured (MI355X, both products with sort and combine): 8192 tokens, 4 of 16 experts of 2048 x 1408: 1010 us (the form before: 256 x 128 tiles staged
+// through registers, tile list from the host, torch's sort) -> 485 -> 463 (with the cut of the last round, in turn; 815 TFLOP/s), gated
+// 647 -> 620 us (915), 600 tokens 121 -> 106 us; 32 gated experts of 4096 x 2752: 3.5 ms -> 2547 -> 2494 us (888).
 constexpr int PR = 256, PS = 256, PWAVES = 8, PT = 64 * PWAVES;
 constexpr int PBUF = (PR + PS) * 128;               // bytes of one K step
 constexpr int MAX_GROUPS = 1024;

@@ -114,8 +114,14 @@ class Engine:
         self.cache.release(slot)
 
     def _token_ids(self, t):
-        """The tokens of one run as an int64 array, checked against the vocabulary."""
-        a = np.array(t) if isinstance(t, (list, tuple)) else None
+        """The tokens of one run as an int64 array, checked against the vocabulary.  Anything whose elements int() takes: whole numbers go
+        through numpy at once, the rest (tensors on a GPU, other arrays) one by one."""
+        a = None
+        if isinstance(t, (list, tuple)) and t and type(t[0]) is int:
+            try:
+                a = np.array(t)
+            except Exception:                                          # (an element further on that numpy cannot convert)
+                pass
         if a is None or a.dtype != np.int64 or a.ndim != 1:
             ids = [int(v) for v in t]
             if any(not 0 <= v < self.model.vocab for v in ids):

@@ -9,6 +9,7 @@ Conventions: `x` is the float residual stream [T, D]; `h` and every other activa
 float32); matrix products (`linear`, the products per head) are own kernels for a step's few rows and the vendor's beyond, with float accumulation.
 """
 import torch
+from torch.autograd import forward_ad
 
 BF16, F32 = 0, 1
 
@@ -27,13 +28,22 @@ def _skinny(T, N, K):
     return T <= 16 or (T <= 32 and (K <= 2048 or N * K <= 36_000_000)) or (T <= 64 and N <= 6144 and N * K <= 13_000_000)
 
 
+def _called_plainly():
+    """Whether nobody looks at torch's calls from outside: no function transform (vmap, jvp), no forward-mode level, no dispatch mode, no trace.
+    A kernel launched past torch would be invisible to those.  (0.5 us.)"""
+    return (torch._C._functorch.peek_interpreter_stack() is None and forward_ad._current_level < 0 and torch._C._len_torch_dispatch_stack() == 0
+            and torch._C._get_tracing_state() is None and not torch.compiler.is_compiling())
+
+
 def linear(x, w):
     """x [T, in] @ w [out, in]^T in the storage type, float accumulation: the few rows of a decoding step (bfloat16 on a GPU) through
     qsv_skinny_linear, everything else through hipBLASLt / rocBLAS."""
-    if (type(x) is torch.Tensor and x.is_cuda and x.dim() == 2 and w.dim() == 2 and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
-            and w.is_contiguous() and 0 < x.size(0) and x.size(1) == w.size(1) and x.size(1) and w.size(0) and _skinny(x.size(0), w.size(0), w.size(1))
+    if (type(x) is torch.Tensor and type(w) in (torch.Tensor, torch.nn.Parameter) and x.is_cuda and x.dim() == 2 and w.dim() == 2
+            and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and w.is_contiguous() and 0 < x.size(0) and x.size(1) == w.size(1)
+            and x.size(1) and w.size(0) and _skinny(x.size(0), w.size(0), w.size(1)) and _called_plainly()
             and x.stride(1) == 1 and x.size(1) % 8 == 0 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-            and x.device == w.device and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))):
+            and x.device == w.device and x.device.index == torch.cuda.current_device()
+            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))):
         from ..serving._lib import check, lib
         out = torch.empty((x.size(0), w.size(0)), dtype=x.dtype, device=x.device)
         check(lib().qsv_skinny_linear(out.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(), x.size(0), w.size(0), x.size(1),

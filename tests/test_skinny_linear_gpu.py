@@ -29,3 +29,41 @@ def test_shapes_that_do_not_fit_still_raise():
     x, w = torch.zeros(2, 16, device="cuda:0").bfloat16(), torch.zeros(4, 24, device="cuda:0").bfloat16()
     with pytest.raises(RuntimeError):
         linear(x, w)
+
+
+def test_transforms_modes_and_traces_see_the_product():
+    """Few rows, and something around the call that follows torch's own operations."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from torch.autograd import forward_ad
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    g = torch.Generator(device="cuda:0").manual_seed(0)
+    xs, w, dx = (torch.randn(*s, device="cuda:0", generator=g).bfloat16() for s in ((3, 4, 64), (40, 64), (4, 64)))
+    plain = torch.stack([torch.matmul(x, w.t()) for x in xs]).float()
+    tol = 2.0 ** -7 * plain.abs().max()                                    # two roundings to bfloat16
+    assert ((torch.vmap(linear, in_dims=(0, None))(xs, w).float() - plain).abs() <= tol).all()
+    assert ((torch.vmap(linear, in_dims=(None, 0))(xs[0], torch.stack([w, w]))[1].float() - plain[0]).abs() <= tol).all()
+    want = torch.matmul(dx, w.t()).float()
+    y, dy = torch.func.jvp(lambda x: linear(x, w), (xs[0],), (dx,))
+    assert ((y.float() - plain[0]).abs() <= tol).all() and ((dy.float() - want).abs() <= 2.0 ** -7 * want.abs().max()).all()
+    with forward_ad.dual_level():
+        dy = forward_ad.unpack_dual(linear(forward_ad.make_dual(xs[0], dx), w)).tangent
+    assert dy is not None and ((dy.float() - want).abs() <= 2.0 ** -7 * want.abs().max()).all()
+
+    seen = []
+
+    class Listen(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    with Listen():
+        linear(xs[0], w)
+    assert any("mm" in f for f in seen), seen
+    traced = torch.jit.trace(lambda x: linear(x, w), (xs[0],), check_trace=False)
+    assert ((traced(xs[1]).float() - plain[1]).abs() <= tol).all()
+    wp = torch.nn.Parameter(w)
+    x = xs[0].clone().requires_grad_()
+    linear(x, wp).float().sum().backward()
+    assert x.grad is not None and wp.grad is not None

@@ -23,9 +23,22 @@ def dtype_code(dtype):
 
 
 def _skinny(T, N, K):
-    """Whether the kernel that streams the weight beats the vendor's product for T rows (measured from HBM, N 1024 - 32000, K 64 - 4096: always
-    up to 16 rows; up to 32 but for 11008 x 4096, 26 against 23 us; up to 64 while one round of workgroups holds the weight)."""
-    return T <= 16 or (T <= 32 and (K <= 2048 or N * K <= 36_000_000)) or (T <= 64 and N <= 6144 and N * K <= 13_000_000)
+    """Whether the kernel that streams the weight beats the vendor's product for T rows; measured from HBM for T 1 - 64, N 8 - 152064, K 64 -
+    28672 (vendor / own, us).  Beyond 64 rows never.
+    Rows up to 4096: up to 16 tokens while the weight is below 132 M elements or its rows are short (64 x 4096 10 / 6, 32000 x 4096 60 / 54; but
+    50304 x 4096 82 / 83, 128256 x 4096 188 / 195); up to 32 below 25.2 M (6144 x 4096 15.3 / 14.6, 12288 x 2048 15.0 / 15.3; but 14336 x 2048 15.7 / 18.0)
+    and for a vocabulary over rows of 2048 (32000: 32 / 31); up to 64 while one round of workgroups holds it (6144 x 2048 13.0 / 10.9, 2048 x 4096 13.9 / 9.1;
+    but 8192 x 2048 33 tokens 14.9 / 12.7 and 4096 x 3072 11.2 / 12.3).
+    Longer rows: the vendor's product splits the reduction where there are few of them (64 x 8192 8.4 / 10.6), and rows a multiple of 16 KB
+    apart slow the stream (8192 x 8192 31 / 36, 152064 x 8192 449 / 531); between, from 256 workgroups to 256 of the larger, it wins (4096 x 11008 38 / 22,
+    8192 x 14336 48 / 45) - but for the few workgroups more than CUs of 4097 - 5119 rows (4608 x 5120, 16 tokens 15.3 / 16.6)."""
+    if K > 4096:
+        return (N == 4096 or 5120 <= N <= 8192) and K % 8192 != 0 and ((T <= 16 and K <= 14336) or (T <= 32 and N * K <= 36_000_000))
+    if T <= 16:
+        return K <= 2048 or N * K <= 132_000_000
+    if T <= 32:
+        return N * K <= 25_200_000 or (1536 < K <= 2048 and N >= 24576)
+    return T <= 64 and N <= (6144 if K <= 2048 else 2048)
 
 
 def _called_plainly():

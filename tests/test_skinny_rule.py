@@ -1,0 +1,20 @@
+"""Which products of few rows go to the kernel that streams the weight: pairs of measured times on either side of the rule's lines."""
+import pytest
+
+from qserve_amd.layers.ops import _skinny
+
+
+# rows, N, K where the vendor's product is the faster one by more than the runs differ
+@pytest.mark.parametrize("T, N, K", [(1, 64, 8192), (16, 64, 6144), (33, 64, 7168), (17, 1024, 8192), (64, 1024, 6144), (1, 8192, 8192), (16, 8192, 8192),
+                                     (1, 128256, 4096), (16, 128256, 4096), (1, 152064, 8192), (16, 152064, 8192), (1, 32000, 8192), (1, 16384, 16384), (16, 4096, 16384),
+                                     (16, 16384, 5120), (16, 4608, 5120), (32, 4608, 5120), (32, 16384, 2048), (32, 14336, 2048), (17, 9216, 3072), (33, 4096, 3072),
+                                     (33, 8192, 4096), (64, 32000, 2048), (32, 64, 28672), (65, 2048, 2048)])
+def test_left_to_the_vendor(T, N, K):
+    assert not _skinny(T, N, K)
+
+
+@pytest.mark.parametrize("T, N, K", [(1, 16, 2048), (64, 64, 2048), (16, 64, 4096), (64, 1024, 4096), (1, 512, 64), (16, 32000, 4096), (32, 32000, 2048), (16, 128256, 2048),
+                                     (32, 8192, 2048), (32, 6144, 4096), (64, 6144, 2048), (64, 2048, 4096), (16, 11008, 4096), (16, 4096, 11008), (32, 4096, 5120),
+                                     (16, 8192, 14336), (16, 5120, 13824)])
+def test_streamed(T, N, K):
+    assert _skinny(T, N, K)

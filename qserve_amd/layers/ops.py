@@ -808,8 +808,11 @@ class HipOps:
         idx = idx.to(torch.int32).contiguous()
         a = self.ACTS[act]
         ff = rows // 2 if a >= 2 else rows
-        if (self.code == BF16 and self.moe_token_slots < T * top_k <= self.moe_expert_major_slots and D % 8 == 0 and ff % 8 == 0
-                and D <= 4096 and ff <= 4096 and up.data_ptr() % 16 == 0 and down.data_ptr() % 16 == 0):
+        major = self.moe_expert_major_slots
+        if major is None:
+            major = 896 if self._grouped_takes(up.size(0), rows, D, ff) else 1024
+        if (self.code == BF16 and self.moe_token_slots < T * top_k <= major and D % 8 == 0 and ff % 8 == 0
+                and D <= 4096 and ff <= 4096):
             return self._moe_experts_expert_major(h, up, down, idx, wt, a, limit, weigh)
         if T * top_k > self.moe_sorted_above:
             return self._moe_experts_sorted(h, up, down, idx, wt, a, limit, weigh)
@@ -831,12 +834,22 @@ class HipOps:
     moe_grouped_kernel = True
 
     # (token, expert) slots: up to moe_expert_major_slots the expert-major kernels (bfloat16; every expert weight read once, slots
-    # found on the device), above it the expert-sorted products (compute-bound sizes).  The per-token kernels - two launches, but
+    # found on the device, captured like any launch), above it the expert-sorted products (compute-bound sizes).  The per-token kernels - two launches, but
     # one workgroup per token walks a whole product (one token at 2048 x 1408, 4 of 16 experts: 4.6 ms against 0.04 ms) - serve
     # float storage and widths the others do not take.
     moe_token_slots = 0
-    # (crossover measured: 16 experts of 2048 x 1408 at 1000 (relu^2) and 850 slots (gated), 32 of 4096 x 2752 at 850)
-    moe_expert_major_slots = 896
+    # None: 896 (crossover measured: 16 experts of 2048 x 1408 at 1000 (relu^2) and 850 slots (gated), 32 of 4096 x 2752 at 850); 1024 where the
+    # grouped kernel does not take the sizes - the vendor products wait for the runs' lengths and cannot be captured
+    moe_expert_major_slots = None
+
+    def _grouped_takes(self, E, rows, D, ff):
+        L = self.L
+        return bool(self.moe_grouped_kernel and self.code == BF16 and L.qsv_grouped_gemm_sorted_ok(E, rows, D) and L.qsv_grouped_gemm_sorted_ok(E, D, ff))
+
+    @staticmethod
+    def _on_16_bytes(*ts):
+        """The tensors, copied if they start inside 16 bytes (a view into something else: the kernels copy pieces of 16)."""
+        return [t.clone() if t.data_ptr() % 16 else t for t in ts]
 
     @staticmethod
     def _weights_at(wt, weigh):
@@ -858,9 +871,8 @@ class HipOps:
         E, rows, K = up.size(0), up.size(1), idx.size(1)
         ff = rows // 2 if a >= 2 else rows
         n = T * K
-        if h.data_ptr() % 16:                                          # (a row view: the kernel copies 16-byte pieces)
-            h = h.clone()
         self._need(h, up, down, idx, wt)
+        h, up, down = self._on_16_bytes(h, up, down)
         act = torch.empty((n, ff), dtype=self.dtype, device=h.device)
         ys = torch.empty((n, D), dtype=torch.float32, device=h.device)
         y = torch.empty((T, D), dtype=self.dtype, device=h.device)
@@ -882,12 +894,10 @@ class HipOps:
         ff = rows // 2 if code >= 2 else rows
         n = T * K
         L = self.L
-        if (self.moe_grouped_kernel and self.code == BF16 and L.qsv_grouped_gemm_sorted_ok(E, rows, D) and L.qsv_grouped_gemm_sorted_ok(E, D, ff)
-                and up.data_ptr() % 16 == 0 and down.data_ptr() % 16 == 0):
+        if self._grouped_takes(E, rows, D, ff):
             # own grouped matrix-core kernel: gather in its loads, the activation in the first product's epilogue, tiles found on the device
-            if h.data_ptr() % 16:                                      # (a row view: the kernel copies 16-byte pieces)
-                h = h.clone()
             self._need(h, up, down, idx, wt)
+            h, up, down = self._on_16_bytes(h, up, down)
             order, place = (torch.empty((n,), dtype=torch.int32, device=h.device) for _ in range(2))
             offsets = torch.empty((E + 1,), dtype=torch.int32, device=h.device)
             act = torch.empty((n, ff), dtype=self.dtype, device=h.device)

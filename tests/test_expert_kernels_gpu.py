@@ -18,8 +18,9 @@ def ops():
     return make_ops("hip", torch.bfloat16, torch.device("cuda:0"))
 
 
-def check(o, T, top, E, ident, D, ff, act, weigh, crowd):
-    """crowd: about that share of the tokens has expert 0 first."""
+def check(o, T, top, E, ident, D, ff, act, weigh, crowd, shift=0, graph=False):
+    """crowd: about that share of the tokens has expert 0 first; shift: the weights start that many elements into their storage; graph: the
+    result of a captured call, replayed."""
     g = torch.Generator().manual_seed(T * 131 + D)
     dev, gated = "cuda:0", act != "relu_sq"
     h = torch.randn(T + 1, D, generator=g).bfloat16()
@@ -32,7 +33,21 @@ def check(o, T, top, E, ident, D, ff, act, weigh, crowd):
     wt = torch.rand(T, top, generator=g)
     limit = 1.0 if act == "clamped_glu" else 0.0
     hd = h.to(dev)[1:] if T % 2 else h[1:].to(dev)                      # (also a view that starts inside a row of 16 bytes for narrow widths)
-    y = o.moe_experts(hd, up.to(dev), down.to(dev), idx.to(dev), wt.to(dev), act=act, limit=limit, weigh=weigh).double().cpu()
+    upd, downd = (torch.cat([w.new_zeros(shift), w.flatten()]).to(dev)[shift:].view(w.shape) for w in (up, down))
+    args = (hd, upd, downd, idx.to(dev), wt.to(dev))
+    call = lambda: o.moe_experts(*args, act=act, limit=limit, weigh=weigh)                                # noqa: E731
+    if graph:
+        call()
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            y = call()
+        for _ in range(3):
+            y.zero_()
+            g.replay()
+    else:
+        y = call()
+    y = y.double().cpu()
     x, ref, size = h[1:].double(), torch.zeros(T, D, dtype=torch.float64), torch.zeros(T, D, dtype=torch.float64)
     for e in range(E + ident):
         t, k = (idx == e).nonzero(as_tuple=True)
@@ -85,6 +100,14 @@ def test_grouped_form(ops, T, top, E, ident, D, ff, crowd, act, weigh):
     o = make_ops("hip", torch.bfloat16, torch.device("cuda:0"))
     o.moe_expert_major_slots, o.moe_sorted_above = 0, 0
     check(o, T, top, E, ident, D, ff, act, weigh, crowd)
+
+
+# sizes the grouped kernel does not take, weights inside 16 bytes: what was computed (any weighting) and captured stays so
+@pytest.mark.parametrize("T, top, E, D, ff, shift, graph", [(500, 2, 4, 72, 40, 0, False), (256, 4, 6, 200, 64, 0, True), (450, 2, 4, 64, 128, 3, False),
+                                                            (20, 3, 5, 64, 64, 1, False), (600, 2, 4, 64, 128, 5, False)])
+@pytest.mark.parametrize("act, weigh", [("relu_sq", "input"), ("relu_sq", "output"), ("swiglu", "input")])
+def test_sizes_and_addresses_between_the_forms(ops, T, top, E, D, ff, shift, graph, act, weigh):
+    check(ops, T, top, E, 0, D, ff, act, weigh, 0.3, shift, graph)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])

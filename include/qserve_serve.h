@@ -247,7 +247,8 @@ int qsv_moe_down(void* y, const void* act, const void* down, const int32_t* idx,
  *   y[t]   = sum_k weight[t, k] * ys[inv[t * top_k + k]]            (sorted rows back, weighted; float accumulation) */
 /* Expert-major form (bfloat16): out[s, r] = act(W[e][r, :] . X[x_index ? x_index[s] / div : s, :]) for the sorted slots
  * s in [offsets[e], offsets[e + 1]) of every expert e; W [n_experts, rows, K]; act = one of QSV_ACT_* (QSV_ACT_GLU: out is
- * rows / 2 wide).  Every weight is read once per launch.  K a multiple of 8, at most 4096. */
+ * rows / 2 wide).  Every weight is read once per launch.  K a multiple of 8, at most 2^25; X and W on
+ * 16 bytes. */
 int qsv_expert_rows(void* out, const void* X, const int64_t* x_index, int div, const void* W, const int64_t* offsets,
                     int n_experts, int rows, int K, int act, float limit, const float* in_weight, void* stream);
 /* The same without sorting: slot s = token t's k-th choice, s = t * div + k or any n slots whose input is X[s / div]; idx int32 [n] names each

@@ -700,7 +700,8 @@ static int launch_expert_rows(const char* what, ExpertArgs a, int n_experts, int
     QSV_REQUIRE(act != QSV_ACT_CLAMPED_GLU || a.limit > 0.f, "%s: clamped units need a positive limit", what);
     if (act == QSV_ACT_CLAMPED_GLU) act = ACT_GLU;
     else a.limit = 0.f;
-    QSV_REQUIRE(a.K > 0 && a.K % 8 == 0 && a.K <= 4096, "%s: inner width %d (a multiple of 8, at most 4096)", what, a.K);
+    // (a workgroup's rows within 32-bit byte offsets)
+    QSV_REQUIRE(a.K > 0 && a.K % 8 == 0 && a.K <= 1 << 25, "%s: inner width %d (a multiple of 8, at most 2^25)", what, a.K);
     QSV_REQUIRE(n_experts <= 65535, "%s: too many experts", what);
     QSV_REQUIRE(((uintptr_t)a.X | (uintptr_t)a.W) % 16 == 0, "%s: inputs and weights start on 16 bytes", what);
     a.wide = (uintptr_t)a.out % 16 == 0;

@@ -810,11 +810,10 @@ class HipOps:
         ff = rows // 2 if a >= 2 else rows
         major = self.moe_expert_major_slots
         if major is None:
-            major = 896 if self._grouped_takes(up.size(0), rows, D, ff) else 1024
-        if (self.code == BF16 and self.moe_token_slots < T * top_k <= major and D % 8 == 0 and ff % 8 == 0
-                and D <= 4096 and ff <= 4096):
+            major = self.moe_sorted_above if max(D, ff) > 4096 else 896 if self._grouped_takes(up.size(0), rows, D, ff) else 1024
+        if self.code == BF16 and self.moe_token_slots < T * top_k <= major and D % 8 == 0 and ff % 8 == 0 and max(D, ff) <= 1 << 25:
             return self._moe_experts_expert_major(h, up, down, idx, wt, a, limit, weigh)
-        if T * top_k > self.moe_sorted_above:
+        if T * top_k > self.moe_sorted_above or (T and max(D, top_k * ff) * 4 > 64 * 1024):     # (the per-token kernels keep a token's rows in 64 KiB of LDS)
             return self._moe_experts_sorted(h, up, down, idx, wt, a, limit, weigh)
         act = torch.empty((T, top_k, ff), dtype=self.dtype, device=h.device)
         y = torch.empty((T, D), dtype=self.dtype, device=h.device)
@@ -838,8 +837,10 @@ class HipOps:
     # one workgroup per token walks a whole product (one token at 2048 x 1408, 4 of 16 experts: 4.6 ms against 0.04 ms) - serve
     # float storage and widths the others do not take.
     moe_token_slots = 0
-    # None: 896 (crossover measured: 16 experts of 2048 x 1408 at 1000 (relu^2) and 850 slots (gated), 32 of 4096 x 2752 at 850); 1024 where the
-    # grouped kernel does not take the sizes - the vendor products wait for the runs' lengths and cannot be captured
+    # None: 896 (crossover measured: 16 experts of 2048 x 1408 at 1000 (relu^2) and 850 slots (gated), 32 of 4096 x 2752 at 850; it moves with the
+    # slots per expert: 2 of 2048 x 1408 at 450, 8 of 4096 x 2752 at 320, 128 and 256 of 2048 x 768 / 512 at 1000); 1024 where the grouped kernel does
+    # not take the sizes - the vendor products wait for the runs' lengths and cannot be captured; 64 (moe_sorted_above) for rows longer than 4096 (8 of
+    # 5120 x 5632, gated, 64 / 256 / 512 slots: 235 / 338 / 523 us, grouped 371 / 381 / 402; 16 of 8192 x 4096 64 / 256: 429 / 440, grouped 388 / 396)
     moe_expert_major_slots = None
 
     def _grouped_takes(self, E, rows, D, ff):

@@ -102,6 +102,27 @@ def test_grouped_form(ops, T, top, E, ident, D, ff, crowd, act, weigh):
     check(o, T, top, E, ident, D, ff, act, weigh, crowd)
 
 
+# rows longer than 4096, up to a layer of 5120 x 5632
+@pytest.mark.parametrize("T, top, E, D, ff", [(1, 4, 6, 5120, 5632), (16, 4, 6, 4104, 16), (17, 2, 3, 64, 8200), (3, 4, 4, 20000, 24), (20, 3, 4, 24, 12288)])
+@ACTS
+def test_expert_major_form_of_wide_layers(ops, T, top, E, D, ff, act, weigh):
+    check(ops, T, top, E, 0, D, ff, act, weigh, 0.5)
+
+
+@pytest.mark.parametrize("T, D, ff", [(2, 64, 4104), (3, 16400, 24)])
+def test_float_storage_beyond_a_workgroups_lds(T, D, ff):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    dev, E, top = torch.device("cuda:0"), 5, 4
+    g = torch.Generator().manual_seed(ff)
+    h, up, down = torch.randn(T, D, generator=g), torch.randn(E, ff, D, generator=g) / D ** 0.5, torch.randn(E, D, ff, generator=g) / ff ** 0.5
+    idx, wt = torch.rand(T, E, generator=g).argsort(1)[:, :top].int(), torch.rand(T, top, generator=g)
+    y = make_ops("hip", torch.float32, dev).moe_experts(*(t.to(dev) for t in (h, up, down, idx, wt))).double().cpu()
+    ref = torch.stack([sum(w.double() * (down[e].double() @ torch.relu(up[e].double() @ h[t].double()) ** 2) for e, w in zip(idx[t], wt[t])) for t in range(T)])
+    # float sums of D and of ff products of order one on average, squared in between
+    assert ((y - ref).abs() <= 2.0 ** -23 * (2 * D + ff) * 4).all()
+
+
 # sizes the grouped kernel does not take, weights inside 16 bytes: what was computed (any weighting) and captured stays so
 @pytest.mark.parametrize("T, top, E, D, ff, shift, graph", [(500, 2, 4, 72, 40, 0, False), (256, 4, 6, 200, 64, 0, True), (450, 2, 4, 64, 128, 3, False),
                                                             (20, 3, 5, 64, 64, 1, False), (600, 2, 4, 64, 128, 5, False)])

@@ -260,7 +260,7 @@ int qsv_expert_slots(void* out, int float_out, const void* X, int div, const voi
  * place: slot -> sorted slot, offsets [n_experts + 1]: first sorted slot of every expert; indices from n_experts on are left out of all
  * three), and the product takes those: out[s, r] = act(W[e][r, :] . X[order ? order[s] / div : s, :]) for the sorted slots of every expert
  * e, the input times in_weight[order ? order[s] : s] if given.  act: QSV_ACT_* (QSV_ACT_GLU: out is n_rows / 2 wide).  n_rows a multiple of
- * 4, K a multiple of 64, at most 1024 experts (_ok). */
+ * 4, K a multiple of 64, at most 8064 experts (_ok). */
 int qsv_moe_sort(int32_t* order, int32_t* place, int32_t* offsets, const int32_t* idx, int n, int n_experts, void* stream);
 int qsv_grouped_gemm_sorted_ok(int n_experts, int n_rows, int K);
 int qsv_grouped_gemm_sorted(void* out, const void* X, const int32_t* order, int div, const void* W, const int32_t* offsets, int n_experts,

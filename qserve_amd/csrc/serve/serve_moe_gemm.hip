@@ -32,7 +32,7 @@ __device__ __forceinline__ unsigned pack_bf2(float a, float b) { return (unsigne
 // 647 -> 620 us (915), 600 tokens 121 -> 106 us; 32 gated experts of 4096 x 2752: 3.5 ms -> 2547 -> 2494 us (888).
 constexpr int PR = 256, PS = 256, PWAVES = 8, PT = 64 * PWAVES;
 constexpr int PBUF = (PR + PS) * 128;               // bytes of one K step
-constexpr int MAX_GROUPS = 1024;
+constexpr int MAX_GROUPS = 8064;                   // (what is left of 160 KiB of LDS holds a count for each)
 
 typedef __attribute__((address_space(3))) void* lds_ptr;
 __device__ __forceinline__ void lds_copy16(unsigned dst, const void* base, unsigned off) {

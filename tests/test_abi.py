@@ -90,6 +90,12 @@ def test_serve_library_builds_and_matches_its_header():
     assert _lib.lib().qsv_arch() == b"gfx950"
 
 
+def test_grouped_products_of_many_experts_are_taken():
+    from qserve_amd.serving._lib import lib
+    ok = lib().qsv_grouped_gemm_sorted_ok
+    assert [ok(e, 128, 64) for e in (1, 1024, 1025, 8064, 8065)] == [1, 1, 1, 1, 0]
+
+
 def test_serve_argument_validation_without_gpu():
     from qserve_amd.serving._lib import check, lib
     L = lib()

@@ -102,6 +102,11 @@ def test_grouped_form(ops, T, top, E, ident, D, ff, crowd, act, weigh):
     check(o, T, top, E, ident, D, ff, act, weigh, crowd)
 
 
+@pytest.mark.parametrize("E", [1025, 1600, 8064])
+def test_grouped_form_of_many_experts(ops, E):
+    check(ops, 600, 2, E, 3, 64, 64, "relu_sq", "input", 0.1)
+
+
 # rows longer than 4096, up to a layer of 5120 x 5632
 @pytest.mark.parametrize("T, top, E, D, ff", [(1, 4, 6, 5120, 5632), (16, 4, 6, 4104, 16), (17, 2, 3, 64, 8200), (3, 4, 4, 20000, 24), (20, 3, 4, 24, 12288)])
 @ACTS

@@ -265,6 +265,13 @@ int qsv_moe_sort(int32_t* order, int32_t* place, int32_t* offsets, const int32_t
 int qsv_grouped_gemm_sorted_ok(int n_experts, int n_rows, int K);
 int qsv_grouped_gemm_sorted(void* out, const void* X, const int32_t* order, int div, const void* W, const int32_t* offsets, int n_experts,
                             int n_rows, int K, int act, float limit, const float* in_weight, void* stream);
+/* The same product over work tiles that the caller lists: tiles int32 [n_tiles, 3] = (expert, first sorted slot, slots <=
+ * qsv_grouped_gemm_tile_slots()), out[s, n] = act(W[e][n, :] . X[x_index ? x_index[s] / div : s, :]); K a multiple of
+ * qsv_grouped_gemm_k_step(), n_rows a multiple of 4, n_tiles <= 65535.  X and W on 16 bytes. */
+int qsv_grouped_gemm_tile_slots(void);
+int qsv_grouped_gemm_k_step(void);
+int qsv_grouped_gemm(void* out, const void* X, const int64_t* x_index, int div, const void* W, const int32_t* tiles,
+                     int n_tiles, int n_rows, int K, int act, float limit, const float* in_weight, void* stream);
 int qsv_gather_rows(void* out, const void* src, const int64_t* order, int div, int n_rows, int width, int dtype, void* stream);
 int qsv_relu_sq(void* a, int64_t n, int dtype, void* stream);
 /* (idx != NULL: slots with idx[t, k] >= n_experts take h[t] in place of a sorted row) */

@@ -32,6 +32,7 @@ __device__ __forceinline__ unsigned pack_bf2(float a, float b) { return (unsigne
 // 647 -> 620 us (915), 600 tokens 121 -> 106 us; 32 gated experts of 4096 x 2752: 3.5 ms -> 2547 -> 2494 us (888).
 constexpr int PR = 256, PS = 256, PWAVES = 8, PT = 64 * PWAVES;
 constexpr int PBUF = (PR + PS) * 128;               // bytes of one K step
+constexpr int LISTED_SLOTS = 128;                   // slots of a tile in a caller's list, at most
 constexpr int MAX_GROUPS = 8064;                   // (what is left of 160 KiB of LDS holds a count for each)
 
 typedef __attribute__((address_space(3))) void* lds_ptr;
@@ -51,12 +52,16 @@ struct GroupedArgs {
     const float* in_weight;
     int div, E, N, K;
     float limit;
+    // the caller's own tiles in place of offsets (LISTED): [n_tiles][3] expert, first sorted slot, slots; x_index for order
+    const int32_t* tiles;
+    const int64_t* x_index;
+    int n_tiles;
 };
 struct GroupedTile {
     int e, n0, first, ns;            // expert, first weight row, first sorted slot, slots
 };
 
-template <int ACT, int NTS>
+template <int ACT, bool LISTED, int NTS>
 __device__ __forceinline__ void grouped_store(const GroupedArgs& a, const GroupedTile& t, int n_wave, int s_wave, int lane, const v4f (&acc)[4][NTS]) {
     const int col = lane & 15, g4 = lane >> 4;
 #pragma unroll
@@ -64,7 +69,7 @@ __device__ __forceinline__ void grouped_store(const GroupedArgs& a, const Groupe
         const int sl = s_wave + 16 * nt + col;
         if (sl >= t.ns) continue;
         float iw = 1.0f;                                            // the expert works on iw * input
-        if (a.in_weight) iw = a.in_weight[a.order ? a.order[t.first + sl] : t.first + sl];
+        if (a.in_weight) iw = a.in_weight[LISTED ? (a.x_index ? a.x_index[t.first + sl] : t.first + sl) : (a.order ? a.order[t.first + sl] : t.first + sl)];
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt) {
             const int n = t.n0 + n_wave + 16 * mt + 4 * g4;
@@ -96,12 +101,12 @@ __device__ __forceinline__ void grouped_store(const GroupedArgs& a, const Groupe
     }
 }
 
-template <int ACT>
+template <int ACT, bool LISTED>
 __global__ __launch_bounds__(PT, 2) void grouped_gemm_persistent_kernel(GroupedArgs a) {
     __shared__ __attribute__((aligned(128))) unsigned char buf[2 * PBUF];
     __shared__ int tiles_before[MAX_GROUPS + 1];                    // slot tiles of the experts before e
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    if (w == 0) {
+    if (!LISTED && w == 0) {
         int carry = 0;
         for (int e0 = 0; e0 < a.E; e0 += 64) {
             const int e = e0 + lane;
@@ -117,12 +122,12 @@ __global__ __launch_bounds__(PT, 2) void grouped_gemm_persistent_kernel(GroupedA
         if (lane == 0) tiles_before[0] = 0;
     }
     __syncthreads();
-    const int row_tiles = (a.N + PR - 1) / PR, total = __builtin_amdgcn_readfirstlane(tiles_before[a.E]) * row_tiles;
+    const int row_tiles = (a.N + PR - 1) / PR, total = (LISTED ? a.n_tiles : __builtin_amdgcn_readfirstlane(tiles_before[a.E])) * row_tiles;
     // An XCD's share of the tiles: whole rounds of its workgroups, then what is left - fewer tiles than workgroups - cut by slots into as many
     // parts (two or four) as there are workgroups for.  Place p: tile (p) of the share, or a part of one.
     const int xcd = blockIdx.x & 7, per_xcd = gridDim.x >> 3, chunk = (total + 7) >> 3;
     const int begin = xcd * chunk, here = max(0, min(chunk, total - begin));
-    const int whole = here / per_xcd * per_xcd, rest = here - whole, cut = rest * 4 <= per_xcd ? 2 : rest * 2 <= per_xcd ? 1 : 0;   // log2 of the parts
+    const int whole = here / per_xcd * per_xcd, rest = here - whole, cut = LISTED ? 0 : rest * 4 <= per_xcd ? 2 : rest * 2 <= per_xcd ? 1 : 0;   // log2 of the parts
     const int last = whole + (rest << cut);
     int at = blockIdx.x >> 3;
     if (at >= last) return;
@@ -130,6 +135,14 @@ __global__ __launch_bounds__(PT, 2) void grouped_gemm_persistent_kernel(GroupedA
     auto tile_at = [&](int place) __attribute__((always_inline)) {
         const int over = place - whole, part = over >= 0 ? over & ((1 << cut) - 1) : 0, size = over >= 0 ? PS >> cut : PS;
         const int L = begin + (over >= 0 ? whole + (over >> cut) : place), s = L / row_tiles;   // which slot tile
+        GroupedTile t;
+        t.n0 = (L % row_tiles) * PR;
+        if (LISTED) {
+            t.e = __builtin_amdgcn_readfirstlane(a.tiles[3 * s]);
+            t.first = __builtin_amdgcn_readfirstlane(a.tiles[3 * s + 1]);
+            t.ns = __builtin_amdgcn_readfirstlane(min(max(a.tiles[3 * s + 2], 0), LISTED_SLOTS));
+            return t;
+        }
         int lo = 0, hi = a.E;                                       // tiles_before[lo] <= s < tiles_before[hi]
         while (hi - lo > 1) {
             const int m = (lo + hi) >> 1;
@@ -137,9 +150,7 @@ __global__ __launch_bounds__(PT, 2) void grouped_gemm_persistent_kernel(GroupedA
             else hi = m;
         }
         const int skip = __builtin_amdgcn_readfirstlane(tiles_before[lo]), first = a.offsets[lo] + (s - skip) * PS + part * size;
-        GroupedTile t;
         t.e = lo;
-        t.n0 = (L % row_tiles) * PR;
         t.first = __builtin_amdgcn_readfirstlane(first);
         t.ns = __builtin_amdgcn_readfirstlane(min(size, a.offsets[lo + 1] - first));   // (none or less: a part behind the expert's last slot)
         return t;
@@ -147,12 +158,14 @@ __global__ __launch_bounds__(PT, 2) void grouped_gemm_persistent_kernel(GroupedA
     // copies: wave w brings rows 32 w .. 32 w + 31 of the weights and of the inputs, eight rows (of 128 bytes) per instruction
     const int piece = ((lane & 7) ^ (lane >> 3)) * 16;
     auto x_slot = [&](const GroupedTile& t, int j) __attribute__((always_inline)) {
+        if (LISTED && t.ns <= 0) return 0;                          // (an empty tile of the list: nothing is read or stored)
         const int s = t.first + min(32 * w + 8 * j + (lane >> 3), t.ns - 1);
+        if (LISTED) return a.x_index ? (int)a.x_index[s] : s;
         return a.order ? a.order[s] : s;
     };
     const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(lds_ptr)buf) + (unsigned)w * 4096u;
     GroupedTile t = tile_at(at);
-    if (t.ns <= 0) return;                                          // (parts are the last places: nothing follows)
+    if (!LISTED && t.ns <= 0) return;                                        // (parts are the last places: nothing follows)
     const bf16_t* W0 = a.W + ((size_t)t.e * a.N + t.n0) * (size_t)a.K;
     unsigned woff[4];
     const unsigned char* xrow[4];
@@ -186,7 +199,7 @@ __global__ __launch_bounds__(PT, 2) void grouped_gemm_persistent_kernel(GroupedA
         constexpr int NTS = decltype(nts)::value;
         const int next = at + per_xcd;
         const GroupedTile u = next < last ? tile_at(next) : t;
-        const bool more = next < last && u.ns > 0;
+        const bool more = next < last && (LISTED || u.ns > 0);
         int slot[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) slot[j] = x_slot(more ? u : t, j);
@@ -238,7 +251,7 @@ __global__ __launch_bounds__(PT, 2) void grouped_gemm_persistent_kernel(GroupedA
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        grouped_store<ACT, NTS>(a, t, 64 * wr, s_wave, lane, acc);
+        grouped_store<ACT, LISTED, NTS>(a, t, 64 * wr, s_wave, lane, acc);
         asm volatile("" ::: "memory");                              // (the stores' branches join here: what follows stays uniform)
         if (more) t = u;
         at = next;
@@ -312,21 +325,38 @@ extern "C" int qsv_moe_sort(int32_t* order, int32_t* place, int32_t* offsets, co
     hipLaunchKernelGGL(sort_slots_kernel, dim3(n_experts), dim3(ST), 0, (hipStream_t)stream, order, place, offsets, idx, n, n_experts);
     return qsv_launch_status("qsv_moe_sort");
 }
+template <bool LISTED>
+static int launch_grouped(const char* what, GroupedArgs a, int act, void* stream) {
+    QSV_REQUIRE(act == QSV_ACT_NONE || act == QSV_ACT_RELU_SQ || act == QSV_ACT_GLU || (act == QSV_ACT_CLAMPED_GLU && a.limit > 0.f),
+                "%s: activation %d (limit %g)", what, act, (double)a.limit);
+    QSV_REQUIRE(((uintptr_t)a.X | (uintptr_t)a.W) % 16 == 0 && (uintptr_t)a.out % 8 == 0, "%s: inputs and weights start on 16 bytes", what);
+    if (act == QSV_ACT_CLAMPED_GLU) act = QSV_ACT_GLU;
+    else a.limit = 0.f;
+    const dim3 grid(256), block(PT);                                // one workgroup per CU, 32 per XCD
+    if (act == QSV_ACT_RELU_SQ) hipLaunchKernelGGL((grouped_gemm_persistent_kernel<1, LISTED>), grid, block, 0, (hipStream_t)stream, a);
+    else if (act == QSV_ACT_GLU) hipLaunchKernelGGL((grouped_gemm_persistent_kernel<2, LISTED>), grid, block, 0, (hipStream_t)stream, a);
+    else hipLaunchKernelGGL((grouped_gemm_persistent_kernel<0, LISTED>), grid, block, 0, (hipStream_t)stream, a);
+    return qsv_launch_status(what);
+}
 extern "C" int qsv_grouped_gemm_sorted_ok(int n_experts, int N, int K) { return n_experts > 0 && n_experts <= MAX_GROUPS && N > 0 && N % 4 == 0 && K > 0 && K % KS == 0; }
 extern "C" int qsv_grouped_gemm_sorted(void* out, const void* X, const int32_t* order, int div, const void* W, const int32_t* offsets, int n_experts,
                                        int N, int K, int act, float limit, const float* in_weight, void* stream) {
     QSV_REQUIRE(out && X && W && offsets && div > 0, "qsv_grouped_gemm_sorted: bad arguments");
     QSV_REQUIRE(qsv_grouped_gemm_sorted_ok(n_experts, N, K), "qsv_grouped_gemm_sorted: %d experts (at most %d), N %d (a multiple of 4), K %d (a multiple of %d)",
                 n_experts, MAX_GROUPS, N, K, KS);
-    QSV_REQUIRE(act == QSV_ACT_NONE || act == QSV_ACT_RELU_SQ || act == QSV_ACT_GLU || (act == QSV_ACT_CLAMPED_GLU && limit > 0.f),
-                "qsv_grouped_gemm_sorted: activation %d (limit %g)", act, (double)limit);
-    QSV_REQUIRE(((uintptr_t)X | (uintptr_t)W) % 16 == 0 && (uintptr_t)out % 8 == 0, "qsv_grouped_gemm_sorted: inputs and weights start on 16 bytes");
-    if (act == QSV_ACT_CLAMPED_GLU) act = QSV_ACT_GLU;
-    else limit = 0.f;
-    const GroupedArgs a = {(bf16_t*)out, (const bf16_t*)X, (const bf16_t*)W, order, offsets, in_weight, div, n_experts, N, K, limit};
-    const dim3 grid(256), block(PT);                                // one workgroup per CU, 32 per XCD
-    if (act == QSV_ACT_RELU_SQ) hipLaunchKernelGGL(grouped_gemm_persistent_kernel<1>, grid, block, 0, (hipStream_t)stream, a);
-    else if (act == QSV_ACT_GLU) hipLaunchKernelGGL(grouped_gemm_persistent_kernel<2>, grid, block, 0, (hipStream_t)stream, a);
-    else hipLaunchKernelGGL(grouped_gemm_persistent_kernel<0>, grid, block, 0, (hipStream_t)stream, a);
-    return qsv_launch_status("qsv_grouped_gemm_sorted");
+    return launch_grouped<false>("qsv_grouped_gemm_sorted", {(bf16_t*)out, (const bf16_t*)X, (const bf16_t*)W, order, offsets, in_weight, div, n_experts, N, K,
+                                                             limit, nullptr, nullptr, 0}, act, stream);
+}
+// The same over the caller's own tiles.
+extern "C" int qsv_grouped_gemm_tile_slots(void) { return LISTED_SLOTS; }
+extern "C" int qsv_grouped_gemm_k_step(void) { return KS; }
+extern "C" int qsv_grouped_gemm(void* out, const void* X, const int64_t* x_index, int div, const void* W, const int32_t* tiles, int n_tiles, int N, int K,
+                                int act, float limit, const float* in_weight, void* stream) {
+    QSV_REQUIRE(out && X && W && tiles && div > 0 && n_tiles >= 0, "qsv_grouped_gemm: bad arguments");
+    QSV_REQUIRE(N > 0 && N % 4 == 0 && K > 0 && K % KS == 0, "qsv_grouped_gemm: N %d (a multiple of 4), K %d (a multiple of %d)", N, K, KS);
+    QSV_REQUIRE(n_tiles <= 65535, "qsv_grouped_gemm: %d tiles (at most 65535 per launch)", n_tiles);
+    QSV_REQUIRE((int64_t)n_tiles * ((N + PR - 1) / PR) < (1ll << 30), "qsv_grouped_gemm: %d tiles of %d rows", n_tiles, N);
+    if (n_tiles == 0) return QSV_OK;
+    return launch_grouped<true>("qsv_grouped_gemm", {(bf16_t*)out, (const bf16_t*)X, (const bf16_t*)W, nullptr, nullptr, in_weight, x_index ? div : 1, 0, N, K,
+                                                     limit, tiles, x_index, n_tiles}, act, stream);
 }

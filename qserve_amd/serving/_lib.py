@@ -52,6 +52,9 @@ SIGNATURES = {
     "qsv_moe_sort": (_i, [_vp, _vp, _vp, _vp, _i, _i, _vp]),
     "qsv_grouped_gemm_sorted_ok": (_i, [_i, _i, _i]),
     "qsv_grouped_gemm_sorted": (_i, [_vp, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _i, _f, _vp, _vp]),
+    "qsv_grouped_gemm_tile_slots": (_i, []),
+    "qsv_grouped_gemm_k_step": (_i, []),
+    "qsv_grouped_gemm": (_i, [_vp, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _i, _f, _vp, _vp]),
     "qsv_gather_rows": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _vp]),
     "qsv_relu_sq": (_i, [_vp, _i64, _i, _vp]),
     "qsv_moe_combine": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _vp, _vp, _i, _i, _vp]),

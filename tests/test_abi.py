@@ -90,6 +90,17 @@ def test_serve_library_builds_and_matches_its_header():
     assert _lib.lib().qsv_arch() == b"gfx950"
 
 
+def test_serve_header_keeps_the_entries_of_its_version():
+    """qsv_version 1 had these grouped products before the sorted ones joined them."""
+    from qserve_amd.serving._lib import lib
+    assert lib().qsv_version() == 1
+    assert {"qsv_grouped_gemm", "qsv_grouped_gemm_tile_slots", "qsv_grouped_gemm_k_step", "qsv_expert_rows"} <= set(serve_header_symbols())
+    assert (lib().qsv_grouped_gemm_tile_slots(), lib().qsv_grouped_gemm_k_step()) == (128, 64)
+    assert lib().qsv_grouped_gemm(16, 16, None, 1, 16, 16, 1, 130, 64, 0, 0.0, None, None) == 1 and b"multiple of 4" in lib().qsv_last_error()
+    assert lib().qsv_grouped_gemm(16, 16, None, 1, 16, 16, 65536, 128, 64, 0, 0.0, None, None) == 1 and b"tiles" in lib().qsv_last_error()
+    assert lib().qsv_grouped_gemm(16, 16, None, 1, 16, 16, 0, 128, 64, 0, 0.0, None, None) == 0
+
+
 def test_grouped_products_of_many_experts_are_taken():
     from qserve_amd.serving._lib import lib
     ok = lib().qsv_grouped_gemm_sorted_ok

@@ -1,0 +1,55 @@
+"""Entries of the C ABI that take slots sorted by the caller, against float64 (the engine sorts on the device and uses others)."""
+import pytest
+import torch
+
+from qserve_amd.serving._lib import check, lib
+
+pytestmark = pytest.mark.gpu
+ACTS = pytest.mark.parametrize("act, limit", [(0, 0.0), (1, 0.0), (2, 0.0), (3, 1.0)], ids=["none", "relu_sq", "glu", "clamped_glu"])
+
+
+def _inputs(counts, top, N, K, act, indexed, weighted):
+    """Slots sorted by expert (counts of them each), slot s of the list being slot order[s] of the tokens'."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    g = torch.Generator().manual_seed(N + K + len(counts))
+    n = sum(counts)
+    order = torch.randperm(n, generator=g) if indexed else None
+    X = torch.randn((n + top - 1) // top if indexed else n, K, generator=g).bfloat16()
+    W = (torch.randn(len(counts), N, K, generator=g) / K ** 0.5).bfloat16()
+    wt = torch.rand(n, generator=g) if weighted else None
+    rows = X[order // top] if indexed else X
+    iw = torch.ones(n) if wt is None else wt[order] if indexed else wt
+    z = torch.cat([rows[a:a + c].double() @ W[e].double().T for e, (a, c) in enumerate(zip(torch.tensor([0] + list(counts)).cumsum(0).tolist(), counts))])
+    z = z * iw.double()[:, None]
+    if act == 1:
+        z = torch.relu(z) ** 2
+    elif act == 2:
+        z = z[:, 0::2] * torch.sigmoid(z[:, 0::2]) * z[:, 1::2]
+    elif act == 3:
+        p = z[:, 0::2].clamp(max=1.0)
+        z = p * torch.sigmoid(1.702 * p) * (z[:, 1::2].clamp(-1.0, 1.0) + 1.0)
+    d = lambda t: None if t is None else t.cuda()                                                # noqa: E731
+    return d(order), d(X), d(W), d(wt), z, torch.full(z.shape, float("nan"), dtype=torch.bfloat16, device="cuda")
+
+
+def _close(out, ref, K):
+    # one rounding to bfloat16 and a float sum of K products with unit spread, squared or multiplied by a value below 8 at most
+    assert ((out.double().cpu() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2.0 ** -22 * K ** 0.5 * 64).all()
+
+
+# tiles of up to 128 slots (an empty one among them), rows that do not fill a tile of 256, more tiles than workgroups
+@pytest.mark.parametrize("counts, top, N, K", [((1,), 1, 4, 64), ((64, 0, 65, 128), 2, 132, 192), ((129, 7, 300), 3, 260, 128), ((40,) * 90, 4, 1024, 64)])
+@pytest.mark.parametrize("indexed, weighted", [(True, False), (True, True), (False, True)])
+@ACTS
+def test_tiles_that_the_caller_lists(counts, top, N, K, indexed, weighted, act, limit):
+    order, X, W, wt, ref, out = _inputs(counts, top, N, K, act, indexed, weighted)
+    L, s, tiles, a = lib(), torch.cuda.current_stream().cuda_stream, [], 0
+    for e, c in enumerate(counts):
+        tiles += [(e, a + o, min(L.qsv_grouped_gemm_tile_slots(), c - o)) for o in range(0, c, L.qsv_grouped_gemm_tile_slots())] or [(e, a, 0)]
+        a += c
+    tiles = torch.tensor(tiles, dtype=torch.int32, device="cuda")
+    check(L.qsv_grouped_gemm(out.data_ptr(), X.data_ptr(), None if order is None else order.data_ptr(), top, W.data_ptr(), tiles.data_ptr(), tiles.size(0),
+                             N, K, act, limit, None if wt is None else wt.data_ptr(), s), "grouped_gemm")
+    _close(out, ref, K)
+    assert K % L.qsv_grouped_gemm_k_step() == 0

@@ -53,3 +53,15 @@ def test_tiles_that_the_caller_lists(counts, top, N, K, indexed, weighted, act, 
                              N, K, act, limit, None if wt is None else wt.data_ptr(), s), "grouped_gemm")
     _close(out, ref, K)
     assert K % L.qsv_grouped_gemm_k_step() == 0
+
+
+# runs of 16, 32 and more slots, empty ones, rows that do not fill 32, the last stage of the reduction part-empty
+@pytest.mark.parametrize("counts, top, N, K", [((1,), 1, 2, 8), ((16, 0, 17), 3, 34, 72), ((33, 2, 70, 0), 4, 66, 4104), ((5,) * 40, 2, 128, 200)])
+@pytest.mark.parametrize("indexed, weighted", [(True, False), (True, True), (False, True)])
+@ACTS
+def test_runs_that_the_caller_sorted(counts, top, N, K, indexed, weighted, act, limit):
+    order, X, W, wt, ref, out = _inputs(counts, top, N, K, act, indexed, weighted)
+    offsets = torch.tensor([0] + list(counts)).cumsum(0).cuda()
+    check(lib().qsv_expert_rows(out.data_ptr(), X.data_ptr(), None if order is None else order.data_ptr(), top, W.data_ptr(), offsets.data_ptr(), len(counts), N, K,
+                                act, limit, None if wt is None else wt.data_ptr(), torch.cuda.current_stream().cuda_stream), "expert_rows")
+    _close(out, ref, K)

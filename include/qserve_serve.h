@@ -389,7 +389,7 @@ int qsv_max_gates(float* a, float* b, float* m, const void* zi, const void* zf, 
 /* Rotations in the halves layout (pair p of n rotated dimensions = p and p + n / 2; rope: float [positions, 2, n / 2]):
  *   qf[t, h]           = [ 0 (vdim) | rot_k(q[t, h]) * scale ]            float [T, heads, vdim + dim]
  *   pool[g, slot[t]]   = [ rot_v(v[t, g]) | rot_k(k[t, g]) ]              [kv_heads, pool_rows, vdim + dim]
- * rot_k turns the first rot_n of dim dimensions, rot_v all vdim; q, k, v are column ranges of proj. */
+ * rot_k turns the first rot_n of dim dimensions (rope_k may be NULL if rot_n is 0), rot_v all vdim; q, k, v are column ranges of proj. */
 int qsv_attention_prep(float* qf, void* pool, int64_t pool_rows, const void* proj, int64_t stride, int q_off, int k_off, int v_off,
                        int heads, int kv_heads, int dim, int vdim, int rot_n, const float* rope_k, const float* rope_v,
                        float scale, const int64_t* slot, const int32_t* pos, int n_tokens, int dtype, void* stream);

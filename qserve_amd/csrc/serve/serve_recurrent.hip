@@ -1180,7 +1180,7 @@ extern "C" int qsv_attention_prep(float* qf, void* pool, int64_t pool_rows, cons
                                   int v_off, int heads, int kv_heads, int dim, int vdim, int rot_n, const float* rope_k,
                                   const float* rope_v, float scale, const int64_t* slot, const int32_t* pos, int n_tokens,
                                   int dtype, void* stream) {
-    QSV_REQUIRE(qf && pool && proj && rope_k && rope_v && slot && pos, "qsv_attention_prep: null argument");
+    QSV_REQUIRE(qf && pool && proj && (rope_k || rot_n == 0) && rope_v && slot && pos, "qsv_attention_prep: null argument");
     QSV_REQUIRE(heads > 0 && kv_heads > 0 && dim > 0 && vdim > 0 && vdim % 2 == 0 && rot_n >= 0 && rot_n % 2 == 0 && rot_n <= dim &&
                     q_off >= 0 && k_off >= 0 && v_off >= 0 && q_off + (int64_t)heads * dim <= stride &&
                     k_off + (int64_t)kv_heads * dim <= stride && v_off + (int64_t)kv_heads * vdim <= stride && n_tokens >= 0,

@@ -83,13 +83,7 @@ def test_attention_rows(H, G, dim, vdim, rot, dtype):
     rk, rv = table(rot), table(vdim)
     p1 = torch.zeros(G, T + 2, vdim + dim, device=DEV, dtype=dtype)
     p2 = p1.clone()
-    if not rot:
-        rk = torch.zeros(16, 2, 0, device=DEV)
-        rk_hip = torch.zeros(16, 2, 1, device=DEV)[..., :0]
-        rk = rk_hip
     args = (proj, off, off + H * dim, off + (H + G) * dim, H, G, dim, vdim, rot, rk, rv, 0.25)
-    if not rot and rk.data_ptr() == 0:
-        pytest.skip("an empty table has no address")
     qf, ref = HipOps(dtype).attention_prep(*args, p1, b), TorchOps(torch.float32).attention_prep(*args, p2.float(), b)
     p3 = p2.float()
     TorchOps(torch.float32).attention_prep(*args, p3, b)

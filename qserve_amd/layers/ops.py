@@ -145,7 +145,7 @@ class HipOps:
         (16 heads of 128 to 512 + 64, 1 / 16 / 64 tokens: 3.0 / 3.3 / 4.6 us against 6.6 / 7.0 / 7.9); beyond 64 rows
         the vendor's batched product and latent_query."""
         T = q.size(0)
-        if self._head_products_fit(T, q, w_uk, dim + rot_dim) and rot_dim % 2 == 0:
+        if self._head_products_fit(T, q, w_uk, dim + rot_dim) and rot_dim % 2 == 0 and rot_dim <= 1 << 20:
             self._need(q, w_uk, rope, pos)
             assert q.numel() == T * heads * (dim + rot_dim) and w_uk.shape == (heads, dim, rank)
             qf = torch.empty((T, heads, rank + rot_dim), dtype=torch.float32, device=q.device)
@@ -157,7 +157,8 @@ class HipOps:
 
     def _head_products_fit(self, T, x, w, row):
         return (0 < T <= 64 and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous()
-                and w.size(1) % 32 == 0 and w.size(2) % 32 == 0 and row % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 4 == 0)
+                and w.size(1) % 32 == 0 and w.size(2) % 32 == 0 and row % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 4 == 0
+                and w.size(0) <= 65535 and w.size(1) * w.size(2) < 2 ** 31)
 
     def head_products(self, x, w):
         """x [T, H, K], w [H, K, N] -> [T, H N], head by head: a step's few rows (up to 64) in one launch (16 heads of 512 to 128, 1 / 16 / 64 tokens:

@@ -18,3 +18,12 @@ def test_left_to_the_vendor(T, N, K):
                                      (16, 8192, 14336), (16, 5120, 13824)])
 def test_streamed(T, N, K):
     assert _skinny(T, N, K)
+
+
+@pytest.mark.parametrize("heads, K, N, takes", [(16, 128, 512, True), (65535, 32, 32, True), (65536, 32, 32, False), (1, 65536, 32768, False), (1, 32, 2 ** 26 - 32, True),
+                                                (4, 48, 64, False), (4, 64, 40, False)])
+def test_products_per_head_that_the_kernel_takes(heads, K, N, takes):
+    import torch
+    from qserve_amd.layers.ops import HipOps
+    x, w = torch.empty(2, heads, K, dtype=torch.bfloat16, device="meta"), torch.empty(heads, K, N, dtype=torch.bfloat16, device="meta")
+    assert HipOps._head_products_fit(None, 2, x, w, K) is takes

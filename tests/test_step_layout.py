@@ -3,6 +3,7 @@ import numpy as np
 import pytest
 import torch
 
+from qserve_amd.serving.cache import CacheFull, PagedCache, StateSpec
 from qserve_amd.serving.engine import Engine
 
 
@@ -41,3 +42,80 @@ def test_tokens_are_whatever_int_takes(tokens):
 def test_tokens_outside_the_vocabulary_are_refused(tokens):
     with pytest.raises(ValueError, match="vocabulary"):
         _engine()._token_ids(tokens)
+
+
+def _pair(seqs=5, pages=40, page=8):
+    """An engine over a cache with a two-copy state, and a cache of the same sizes for the plain statement."""
+    e = _engine()
+    e.device = "cpu"
+    make = lambda: PagedCache([4], num_pages=pages, max_seqs=seqs, dtype=torch.float32, device="cpu", page=page, states=[StateSpec((3,), copies=2)])      # noqa: E731
+    e.cache, plain = make(), make()
+    return e, plain, [(e.open_sequence(), plain.admit()) for _ in range(seqs)]
+
+
+def _plain_layout(cache, items):
+    """A step's arrays, token by token."""
+    tokens, seq, pos, off, rd, wr, rows, runs = [], [], [], [], [], [], [], []
+    for slot, t in items:
+        start = cache.length[slot]
+        if not len(t):
+            continue
+        runs.append((slot, len(tokens), len(t)))
+        new = cache.extend(slot, len(t))
+        r, w = cache.step_rows(slot)
+        for i, v in enumerate(t):
+            tokens.append(int(v))
+            seq.append(slot)
+            pos.append(start + i)
+            off.append(i)
+            rd.append(r if start else -1)
+            wr.append(w if i == len(t) - 1 else -1)
+            rows.append(new[i])
+    return tokens, seq, pos, off, rd, wr, rows, runs
+
+
+def _tiles(runs, n):
+    return [[s, f + o, min(n, c - o)] for s, f, c in runs for o in range(0, c, n)]
+
+
+# lengths of the five sequences' portions, step after step (pages of 8): prompts of odd sizes, steps of one token each, both mixed, idle sequences
+@pytest.mark.parametrize("steps", [[(1, 1, 1, 1, 1)] * 11, [(17, 8, 9, 1, 23), (1, 1, 1, 1, 1), (1, 1, 1, 1, 1), (0, 5, 1, 0, 1), (1, 0, 0, 1, 0)],
+                                   [(0, 0, 3, 0, 0), (0, 0, 1, 0, 0), (8, 0, 16, 1, 0), (1, 1, 1, 1, 1), (7, 1, 1, 1, 24)]])
+def test_a_steps_arrays_are_the_plain_ones(steps):
+    g = torch.Generator().manual_seed(len(steps))
+    e, plain, slots = _pair()
+    for n, counts in enumerate(steps):
+        if n == 3:                                                             # a sequence ends and its pages are used again
+            a, b = slots[1]
+            e.close_sequence(a)
+            plain.release(b)
+            slots[1] = (e.open_sequence(), plain.admit())
+        tokens = [torch.randint(0, 100, (c,), generator=g).tolist() for c in counts]
+        order = torch.randperm(len(slots), generator=g).tolist()
+        batch = e.layout([(slots[i][0], tokens[i]) for i in order])
+        ids, seq, pos, off, rd, wr, rows, runs = _plain_layout(plain, [(slots[i][1], tokens[i]) for i in order])
+        for got, want in ((batch.tokens, ids), (batch.seq, seq), (batch.pos, pos), (batch.run_off, off), (batch.state_rd, rd), (batch.state_wr, wr)):
+            assert got.dtype == torch.int32 and got.tolist() == want
+        assert batch.slot.dtype == torch.int64 and batch.slot.tolist() == rows
+        assert (batch.items, batch.n_tokens, batch.max_pos) == (runs, len(ids), max(pos))
+        assert batch.runs().tolist() == [[s, f, c, pos[f]] for s, f, c in runs]
+        assert torch.equal(batch.block_table, plain.block_table())
+        for n_tile in (1, 4, 64):
+            assert batch.tiles(n_tile).tolist() == _tiles(runs, n_tile) and batch.tiles(n_tile).is_contiguous()
+        for n_tile in (1, 2, 8):
+            long, short = batch.split_tiles(n_tile)
+            assert short.tolist() == [list(r) for r in runs if r[2] <= n_tile]
+            assert long.tolist() == _tiles([r for r in runs if r[2] > n_tile], 4 * n_tile)
+    assert e.layout([(slots[0][0], [])]) is None
+
+
+def test_rows_of_many_tokens_are_the_rows_one_by_one():
+    _, plain, _ = _pair()
+    e, other, slots = _pair()
+    for n in (1, 7, 8, 1, 24, 15, 16):
+        a, b = slots[n % 2]
+        assert e.cache.extend_array(a, n).tolist() == other.extend(b, n)
+    with pytest.raises(CacheFull):
+        e.cache.extend_array(slots[0][0], 10 ** 4)
+    with pytest.raises(ValueError, match="twice"):
+        e.layout([(slots[0][0], [1]), (slots[0][0], [2])])

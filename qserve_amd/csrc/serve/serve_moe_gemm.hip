@@ -25,8 +25,9 @@ __device__ __forceinline__ unsigned pack_bf2(float a, float b) { return (unsigne
 // per step.  Workgroups are persistent (one per CU): each finds its tiles from the experts' offsets - no tile list, no count reaches
 // the host -, an XCD's workgroups walk neighbouring tiles (shared weight and input panels in its L2), and the last step of a tile copies the
 // first one of the next, so the epilogue's stores have something to hide behind.  A tile with few slots gives each wave fewer columns
-// instead of multiplying padding, and no copies of inputs it does not have; the tiles of the last, part-empty round are cut into halves or
-// quarters by slots, so that every workgroup has a part.
+// instead of multiplying padding, and no copies of inputs it does not have; an XCD cuts the tiles of its last, part-empty round by slots into
+// halves where at most half of its 32 workgroups have one, into quarters where at most a quarter have: with more than half nothing is cut, and
+// fewer than eight tiles leave workgroups idle.  The XCDs' shares are ceil(tiles / 8) each, so the last of them can be short or empty.
 // Measured (MI355X, both products with sort and combine): 8192 tokens, 4 of 16 experts of 2048 x 1408: 1010 us (the form before: 256 x 128 tiles staged
 // through registers, tile list from the host, torch's sort) -> 485 -> 463 (with the cut of the last round, in turn; 815 TFLOP/s), gated
 // 647 -> 620 us (915), 600 tokens 121 -> 106 us; 32 gated experts of 4096 x 2752: 3.5 ms -> 2547 -> 2494 us (888).

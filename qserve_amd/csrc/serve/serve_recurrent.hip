@@ -1051,11 +1051,12 @@ extern "C" int qsv_recurrent_scan(float* o, const void* q, int64_t q_stride, con
 #undef QSV_STEP_P
         return qsv_launch_status("qsv_recurrent_scan");
     }
-    // States of other heights, and operands that are not in fours.
+    // States of other heights (up to 32 rows, 129 and more), and operands that are not in fours.
     // Rows of one column per lane: 8 while that leaves the launch at no more than ~2.5 waves per SIMD, else 16 (and for the tallest
-    // states).  Measured at 16 heads, 64 x 128 states: 8 x 1024 tokens (2048 / 1024 waves) 0.46 / 0.51 ms plain, 0.50 / 0.55 ms
-    // delta rule; 64 single tokens (16384 / 8192 waves) 56 / 43 us; two columns per lane 0.60 / 0.75 ms.  A token's step is a
-    // short chain of dependent instructions: up to the chip's fill, more and lighter waves win; beyond it, fewer and heavier ones.
+    // states).  The figures here are of 16 heads of 64 x 128, which come here only where their operands are not in fours: 8 x 1024 tokens
+    // (2048 / 1024 waves) 0.46 / 0.51 ms plain, 0.50 / 0.55 ms delta rule; 64 runs of a token (16384 / 8192 waves) 56 / 43 us; two columns per lane
+    // 0.60 / 0.75 ms.  A token's step is a short chain of dependent instructions: up to the chip's fill, more and lighter waves win; beyond
+    // it, fewer and heavier ones.
     int lpc8 = 1;
     while (lpc8 * 8 < dim) lpc8 <<= 1;
     const int64_t waves8 = (int64_t)n_runs * heads * (((int64_t)vdim * lpc8 + 63) / 64);

@@ -23,22 +23,34 @@ def dtype_code(dtype):
 
 
 def _skinny(T, N, K):
-    """Whether the kernel that streams the weight beats the vendor's product for T rows; measured from HBM for T 1 - 64, N 8 - 152064, K 64 -
-    28672 (vendor / own, us).  Beyond 64 rows never.
-    Rows up to 4096: up to 16 tokens while the weight is below 132 M elements or its rows are short (64 x 4096 10 / 6, 32000 x 4096 60 / 54; but
-    50304 x 4096 82 / 83, 128256 x 4096 188 / 195); up to 32 below 25.2 M (6144 x 4096 15.3 / 14.6, 12288 x 2048 15.0 / 15.3; but 14336 x 2048 15.7 / 18.0)
-    and for a vocabulary over rows of 2048 (32000: 32 / 31); up to 64 while one round of workgroups holds it (6144 x 2048 13.0 / 10.9, 2048 x 4096 13.9 / 9.1;
-    but 8192 x 2048 33 tokens 14.9 / 12.7 and 4096 x 3072 11.2 / 12.3).
-    Longer rows: the vendor's product splits the reduction where there are few of them (64 x 8192 8.4 / 10.6), and rows a multiple of 16 KB
-    apart slow the stream (8192 x 8192 31 / 36, 152064 x 8192 449 / 531); between, from 256 workgroups to 256 of the larger, it wins (4096 x 11008 38 / 22,
-    8192 x 14336 48 / 45) - but for the few workgroups more than CUs of 4097 - 5119 rows (4608 x 5120, 16 tokens 15.3 / 16.6)."""
-    if K > 4096:
-        return (N == 4096 or 5120 <= N <= 8192) and K % 8192 != 0 and ((T <= 16 and K <= 14336) or (T <= 32 and N * K <= 36_000_000))
+    """Whether the kernel that streams the weight beats the vendor's product for T rows.  Every line is from both sides' times, measured from HBM
+    for T 1 - 64, N 8 - 152064, K 64 - 29568 (vendor / own below, us); beyond 64 rows never.
+    * It has one workgroup per 16 or 32 weight rows, each reading the inputs again, so it loses where a second round of workgroups is nearly
+      empty (4608 x 5120, 16 tokens 15.3 / 16.6) or the inputs outweigh its lead (4096 x 3072, 33 tokens 11.2 / 12.3, 64: 16.1 / 12.9).
+    * It does not split the reduction; the vendor's product does for few outputs and long rows of a multiple of 512 (64 x 8192 8.4 / 10.6, 1024 x 6144
+      33 tokens 10.6 / 11.5; but 512 x 11008 33 / 14, 2048 x 18944 56 / 27).
+    * Rows a multiple of 16 KB apart slow the stream (8192 x 8192 31 / 36, 152064 x 8192 449 / 531).
+    Otherwise its lead is the start of the stream: 2048 x 2048 8.2 / 4.7, 4096 x 4096 15.5 / 9.2, 4096 x 11008 39 / 22, 27648 x 5120 81 / 58."""
     if T <= 16:
-        return K <= 2048 or N * K <= 132_000_000
+        if K <= 4864:
+            return K <= 2048 or N * K <= 135_000_000
+        if N > 8192:
+            return (T <= 8 or N >= 20480) and K % 8192 != 0 and K <= 14336
+        if K <= 5120:
+            return (T <= 8 or N >= 1024) and not 4096 < N < 5120
+        if K % 8192 == 0:
+            return 1536 <= N <= 3072 or (K > 16384 and (N <= 4096 or N == 5120))
+        return (N >= 1024 or K > 16384 or K % 512 != 0) and not 4096 < N < 5120
     if T <= 32:
-        return N * K <= 25_200_000 or (1536 < K <= 2048 and N >= 24576)
-    return T <= 64 and N <= (6144 if K <= 2048 else 2048)
+        if K <= 4864:
+            return K <= 512 or N * K <= 25_200_000 or (1536 < K <= 2048 and N >= 24576)
+        if N * K > 36_000_000 or 4096 < N < 5120:
+            return False
+        return K <= 5120 or N > 2048 or (N >= 512 and K > 16384) or (N >= 1024 and (K % 512 != 0 or (T == 32 and K <= 7168)))
+    if T > 64 or N > 6144 or N * K > 13_000_000:
+        return False
+    return (K < 2816 or (N <= 2560 and K <= 5120) or (1536 <= N <= 2048 and K <= 7168) or (T == 64 and K <= 3072) or K > 16384
+            or (N >= 512 and K > 5120 and K % 512 != 0))
 
 
 def _called_plainly():

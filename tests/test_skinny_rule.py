@@ -15,7 +15,8 @@ def test_left_to_the_vendor(T, N, K):
 
 @pytest.mark.parametrize("T, N, K", [(1, 16, 2048), (64, 64, 2048), (16, 64, 4096), (64, 1024, 4096), (1, 512, 64), (16, 32000, 4096), (32, 32000, 2048), (16, 128256, 2048),
                                      (32, 8192, 2048), (32, 6144, 4096), (64, 6144, 2048), (64, 2048, 4096), (16, 11008, 4096), (16, 4096, 11008), (32, 4096, 5120),
-                                     (16, 8192, 14336), (16, 5120, 13824)])
+                                     (16, 8192, 14336), (16, 5120, 13824), (64, 2048, 5632), (64, 4096, 2752), (16, 2048, 5632),
+                                     (17, 3072, 5632), (16, 27648, 5120), (16, 512, 11008), (17, 1024, 11008), (33, 1024, 11008), (16, 2048, 18944)])
 def test_streamed(T, N, K):
     assert _skinny(T, N, K)
 

@@ -193,13 +193,13 @@ class Engine:
             if out is not None:
                 if not want:
                     return None
-                want = list(want)
+                want = [int(v) for v in want]
                 return out.clone() if want == list(range(out.size(0))) else out[upload(np.array(want, dtype=np.int64), self.device)]
         batch = self._batch_of(upload(host[0], self.device), *host[1:])
         x = self._forward(batch)
         if not want:
             return None
-        return self.model.logits(x, upload(np.array(list(want), dtype=np.int32), self.device))
+        return self.model.logits(x, upload(np.array([int(v) for v in want], dtype=np.int32), self.device))
 
     def _forward(self, batch):
         if self.cache.states:

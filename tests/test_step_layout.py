@@ -119,3 +119,13 @@ def test_rows_of_many_tokens_are_the_rows_one_by_one():
         e.cache.extend_array(slots[0][0], 10 ** 4)
     with pytest.raises(ValueError, match="twice"):
         e.layout([(slots[0][0], [1]), (slots[0][0], [2])])
+
+
+@pytest.mark.parametrize("want", [[2, 0], (2, 0), [_OnAnotherDevice(2), _OnAnotherDevice(0)], [torch.tensor(2), 0], [np.int64(2), False]])
+def test_wanted_rows_are_whatever_int_takes(want):
+    e, _, slots = _pair()
+    e.decode_graphs, e._forward, seen = False, lambda batch: None, []
+    e.model = type("M", (), {"vocab": 100, "logits": lambda self, x, rows: seen.append(rows)})()
+    e.execute([(slots[0][0], [1, 2, 3])], want)
+    assert seen[0].dtype == torch.int32 and seen[0].tolist() == [2, 0]
+    assert e.execute([(slots[0][0], [4])], []) is None and len(seen) == 1

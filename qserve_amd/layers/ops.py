@@ -54,10 +54,10 @@ def _skinny(T, N, K):
 
 
 def _called_plainly():
-    """Whether nobody looks at torch's calls from outside: no function transform (vmap, jvp), no forward-mode level, no dispatch mode, no trace.
-    A kernel launched past torch would be invisible to those.  (0.5 us.)"""
+    """Whether nobody looks at torch's calls from outside: no function transform (vmap, jvp), no forward-mode level, no dispatch mode, no trace, no
+    autocast.  A kernel launched past torch would be invisible to those.  (About 1 us.)"""
     return (torch._C._functorch.peek_interpreter_stack() is None and forward_ad._current_level < 0 and torch._C._len_torch_dispatch_stack() == 0
-            and torch._C._get_tracing_state() is None and not torch.compiler.is_compiling())
+            and torch._C._get_tracing_state() is None and not torch.is_autocast_enabled("cuda") and not torch.compiler.is_compiling())
 
 
 def linear(x, w):

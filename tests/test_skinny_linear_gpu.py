@@ -67,3 +67,7 @@ def test_transforms_modes_and_traces_see_the_product():
     x = xs[0].clone().requires_grad_()
     linear(x, wp).float().sum().backward()
     assert x.grad is not None and wp.grad is not None
+    for dtype in (torch.float16, torch.float32, torch.bfloat16):
+        with torch.autocast("cuda", dtype=dtype, enabled=dtype != torch.float32):
+            y, want = linear(xs[0], w), torch.matmul(xs[0], w.t())
+        assert y.dtype == want.dtype and ((y.float() - want.float()).abs() <= tol).all()

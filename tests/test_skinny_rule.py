@@ -28,3 +28,21 @@ def test_products_per_head_that_the_kernel_takes(heads, K, N, takes):
     from qserve_amd.layers.ops import HipOps
     x, w = torch.empty(2, heads, K, dtype=torch.bfloat16, device="meta"), torch.empty(heads, K, N, dtype=torch.bfloat16, device="meta")
     assert HipOps._head_products_fit(None, 2, x, w, K) is takes
+
+
+def test_the_kernel_is_left_out_where_torch_itself_has_to_be_called():
+    import torch
+    from torch.autograd import forward_ad
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from qserve_amd.layers.ops import _called_plainly
+    x, seen = torch.ones(2, 3), []
+    note = lambda t: (seen.append(_called_plainly()), t * 2)[1]                                  # noqa: E731
+    assert _called_plainly()
+    torch.vmap(note)(x)
+    torch.func.jvp(note, (x,), (x,))
+    torch.jit.trace(note, (x,), check_trace=False)
+    with forward_ad.dual_level():
+        note(x)
+    with TorchDispatchMode():
+        seen.append(_called_plainly())
+    assert len(seen) == 5 and not any(seen) and _called_plainly()

@@ -228,7 +228,7 @@ int qsv_moe_route(int32_t* idx, float* weight, const void* h, const void* router
 #define QSV_ACT_GLU 2
 /* QSV_ACT_CLAMPED_GLU: the same pairs with g = min(gate, limit), u = clamp(up, -limit, limit), output f = g sigmoid(1.702 g) (u + 1);
  * `limit` is read by this activation only.  Expert indices >= n_experts name identity experts (output = input): the up kernels
- * skip their slots and the down / combine kernels add weight * h[t] for them. */
+ * skip their slots and the down / combine kernels add weight * h[t] for them.  Indices below 0 name no expert: nothing is added. */
 #define QSV_ACT_CLAMPED_GLU 3
 /* Weights on the expert's input: with in_weight != NULL (float, per slot t * top_k + k) an up product works on in_weight * input, and the
  * down / combine kernels take weight == NULL (ones). */
@@ -257,7 +257,7 @@ int qsv_expert_rows(void* out, const void* X, const int64_t* x_index, int div, c
 int qsv_expert_slots(void* out, int float_out, const void* X, int div, const void* W, const int32_t* idx, int n, int n_experts, int rows, int K,
                      int act, float limit, const float* in_weight, void* stream);
 /* Grouped expert product on the bf16 matrix cores (prompt phase): qsv_moe_sort orders the n slots by expert (order: sorted slot -> slot,
- * place: slot -> sorted slot, offsets [n_experts + 1]: first sorted slot of every expert; indices from n_experts on are left out of all
+ * place: slot -> sorted slot, offsets [n_experts + 1]: first sorted slot of every expert; indices below 0 and from n_experts on are left out of all
  * three), and the product takes those: out[s, r] = act(W[e][r, :] . X[order ? order[s] / div : s, :]) for the sorted slots of every expert
  * e, the input times in_weight[order ? order[s] : s] if given.  act: QSV_ACT_* (QSV_ACT_GLU: out is n_rows / 2 wide).  n_rows a multiple of
  * 4, K a multiple of 64, at most 8064 experts (_ok). */

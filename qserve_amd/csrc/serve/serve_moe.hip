@@ -331,7 +331,7 @@ __global__ __launch_bounds__(NT) void moe_up_kernel(T* __restrict__ act, const T
                                                         const float* __restrict__ in_weight) {
     extern __shared__ float xs[];
     const size_t slot = blockIdx.x;
-    if (idx[slot] >= n_experts) return;                      // an identity expert: the down kernel adds the input itself
+    if ((unsigned)idx[slot] >= (unsigned)n_experts) return;  // an identity expert: the down kernel adds the input itself (below 0: none)
     const size_t t = slot / top_k;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     for (int i = threadIdx.x; i < D; i += NT) xs[i] = ld(h, t * D + i);
@@ -374,6 +374,7 @@ __global__ __launch_bounds__(NT) void moe_down_kernel(T* __restrict__ y, const T
     for (int d = w; d < D; d += NW) {
         float total = 0.f;
         for (int k = 0; k < top_k; ++k) {
+            if (idx[t * top_k + k] < 0) continue;            // no expert
             if (idx[t * top_k + k] >= n_experts) {           // identity expert
                 total += (weight ? weight[t * top_k + k] : 1.0f) * ld(h, t * D + d);
                 continue;
@@ -397,7 +398,7 @@ __global__ __launch_bounds__(NT) void moe_up_vec_kernel(T* __restrict__ act, con
                                                         const float* __restrict__ in_weight) {
     extern __shared__ float xs[];
     const size_t slot = blockIdx.x;
-    if (idx[slot] >= n_experts) return;                      // an identity expert: the down kernel adds the input itself
+    if ((unsigned)idx[slot] >= (unsigned)n_experts) return;  // an identity expert: the down kernel adds the input itself (below 0: none)
     const size_t t = slot / top_k;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     for (int i = threadIdx.x; i < D; i += NT) xs[i] = ld(h, t * D + i);
@@ -450,6 +451,7 @@ __global__ __launch_bounds__(NT) void moe_down_vec_kernel(T* __restrict__ y, con
         float acc[ROWS] = {0.f, 0.f, 0.f, 0.f};
         for (int k = 0; k < top_k; ++k) {
             const float wk = weight ? weight[t * top_k + k] : 1.0f;
+            if (idx[t * top_k + k] < 0) continue;            // no expert
             if (idx[t * top_k + k] >= n_experts) {           // identity expert: lane 0's share carries the input (the rest add zero)
                 if (lane == 0) {
 #pragma unroll
@@ -671,7 +673,9 @@ __global__ __launch_bounds__(NT) void moe_combine_kernel(T* __restrict__ y, cons
 #pragma unroll 4
         for (int k = 0; k < top_k; ++k) {
             const size_t slot = t * top_k + k;
-            const bool same = idx && idx[slot] >= n_experts;                // an identity expert's slot has no row of its own
+            const int e = idx ? idx[slot] : 0;
+            if (e < 0) continue;                                            // no expert: the slot has neither a row nor a place
+            const bool same = idx && e >= n_experts;                        // an identity expert's slot has no row of its own
             const float wk = weight ? weight[slot] : 1.0f;
             float v[VEC];
             if (same) loadv(h + t * D + c, v);

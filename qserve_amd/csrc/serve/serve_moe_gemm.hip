@@ -268,7 +268,7 @@ __global__ __launch_bounds__(PT, 2) void grouped_gemm_persistent_kernel(GroupedA
 
 // ---- slots sorted by expert, in order --------------------------------------------------------------------------------------------------
 // Workgroup e gathers the slots of expert e: every wave counts its share of the indices (those of smaller experts give the first place, its
-// own the place within), then writes them.  Indices from E on are left out.
+// own the place within), then writes them.  Indices from E on and below 0 are left out.
 constexpr int ST = 1024;
 __global__ __launch_bounds__(ST) void sort_slots_kernel(int32_t* __restrict__ order, int32_t* __restrict__ place, int32_t* __restrict__ offsets,
                                                         const int32_t* __restrict__ idx, int n, int E) {
@@ -284,7 +284,7 @@ __global__ __launch_bounds__(ST) void sort_slots_kernel(int32_t* __restrict__ or
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
             same += __popcll(__ballot(v[q] == e));
-            less += __popcll(__ballot(v[q] < e));
+            less += __popcll(__ballot((unsigned)v[q] < (unsigned)e));   // (below 0: no expert, left out)
         }
     }
     if (lane == 0) {

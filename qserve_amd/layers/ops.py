@@ -814,7 +814,7 @@ class HipOps:
         """up [E, rows, D], down [E, D, ff]; y[t] = sum_k wt[t, k] * down[idx[t, k]] a(up[idx[t, k]] h[t]).  act "relu_sq":
         a = relu(.)^2, rows = ff; "swiglu": up's rows come in pairs (2f = gate, 2f + 1 = up), a_f = silu(gate_f) up_f, rows = 2 ff;
         "clamped_glu": the same pairs with g = min(gate_f, limit), u = clamp(up_f, -limit, limit), a_f = g sigmoid(1.702 g) (u + 1).
-        Indices at or above E (up.size(0)) name identity experts: their output is h[t] itself.  weigh "input": the weight multiplies the
+        Indices at or above E (up.size(0)) name identity experts: their output is h[t] itself; below 0: no expert.  weigh "input": the weight multiplies the
         expert's input, y[t] = sum_k down[..] a(up[..] (wt[t, k] h[t])) (the products' results are scaled, in float)."""
         T, D = h.shape
         top_k, rows = idx.size(1), up.size(1)

@@ -18,9 +18,9 @@ def ops():
     return make_ops("hip", torch.bfloat16, torch.device("cuda:0"))
 
 
-def check(o, T, top, E, ident, D, ff, act, weigh, crowd, shift=0, graph=False):
+def check(o, T, top, E, ident, D, ff, act, weigh, crowd, shift=0, graph=False, none=False):
     """crowd: about that share of the tokens has expert 0 first; shift: the weights start that many elements into their storage; graph: the
-    result of a captured call, replayed."""
+    result of a captured call, replayed; none: some slots name no expert."""
     g = torch.Generator().manual_seed(T * 131 + D)
     dev, gated = "cuda:0", act != "relu_sq"
     h = torch.randn(T + 1, D, generator=g).bfloat16()
@@ -30,6 +30,8 @@ def check(o, T, top, E, ident, D, ff, act, weigh, crowd, shift=0, graph=False):
     if T > 4:
         idx[: int(T * crowd), 0] = 0
         idx[:, 1:][idx[:, 1:] == 0] = E + ident - 1
+    if none:
+        idx[torch.rand(T, top, generator=g) < 0.3] = -1
     wt = torch.rand(T, top, generator=g)
     limit = 1.0 if act == "clamped_glu" else 0.0
     hd = h.to(dev)[1:] if T % 2 else h[1:].to(dev)                      # (also a view that starts inside a row of 16 bytes for narrow widths)
@@ -105,6 +107,15 @@ def test_grouped_form(ops, T, top, E, ident, D, ff, crowd, act, weigh):
 @pytest.mark.parametrize("E", [1025, 1600, 8064])
 def test_grouped_form_of_many_experts(ops, E):
     check(ops, 600, 2, E, 3, 64, 64, "relu_sq", "input", 0.1)
+
+
+@pytest.mark.parametrize("T, top, D, ff", [(3, 2, 64, 64), (40, 4, 72, 40), (1200, 2, 64, 128)])
+@pytest.mark.parametrize("knobs", [{}, dict(moe_token_slots=10 ** 9, moe_sorted_above=10 ** 9)], ids=["rule", "per token"])
+def test_slots_without_an_expert_add_nothing(T, top, D, ff, knobs):
+    o = make_ops("hip", torch.bfloat16, torch.device("cuda:0"))
+    for k, v in knobs.items():
+        setattr(o, k, v)
+    check(o, T, top, 6, 1, D, ff, "swiglu", "output", 0.2, none=True)
 
 
 # rows longer than 4096, up to a layer of 5120 x 5632

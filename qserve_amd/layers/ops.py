@@ -53,11 +53,12 @@ def _skinny(T, N, K):
             or (N >= 512 and K > 5120 and K % 512 != 0))
 
 
-def _called_plainly():
+def _called_plainly(*ts):
     """Whether nobody looks at torch's calls from outside: no function transform (vmap, jvp), no forward-mode level, no dispatch mode, no trace, no
-    autocast.  A kernel launched past torch would be invisible to those.  (About 1 us.)"""
+    autocast, no gradient for one of ts.  A kernel launched past torch would be invisible to those.  (About 1 us.)"""
     return (torch._C._functorch.peek_interpreter_stack() is None and forward_ad._current_level < 0 and torch._C._len_torch_dispatch_stack() == 0
-            and torch._C._get_tracing_state() is None and not torch.is_autocast_enabled("cuda") and not torch.compiler.is_compiling())
+            and torch._C._get_tracing_state() is None and not torch.is_autocast_enabled("cuda") and not torch.compiler.is_compiling()
+            and not (torch.is_grad_enabled() and any(t.requires_grad for t in ts)))
 
 
 def linear(x, w):
@@ -65,10 +66,9 @@ def linear(x, w):
     qsv_skinny_linear, everything else through hipBLASLt / rocBLAS."""
     if (type(x) is torch.Tensor and type(w) in (torch.Tensor, torch.nn.Parameter) and x.is_cuda and x.dim() == 2 and w.dim() == 2
             and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and w.is_contiguous() and 0 < x.size(0) and x.size(1) == w.size(1)
-            and x.size(1) and w.size(0) and _skinny(x.size(0), w.size(0), w.size(1)) and _called_plainly()
+            and x.size(1) and w.size(0) and _skinny(x.size(0), w.size(0), w.size(1)) and _called_plainly(x, w)
             and x.stride(1) == 1 and x.size(1) % 8 == 0 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-            and x.device == w.device and x.device.index == torch.cuda.current_device()
-            and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))):
+            and x.device == w.device and x.device.index == torch.cuda.current_device()):
         from ..serving._lib import check, lib
         out = torch.empty((x.size(0), w.size(0)), dtype=x.dtype, device=x.device)
         check(lib().qsv_skinny_linear(out.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(), x.size(0), w.size(0), x.size(1),
@@ -168,7 +168,7 @@ class HipOps:
         return self.latent_query(q, q_abs, rope, pos, scale, heads, dim, rot_dim, rot_n, rank)
 
     def _head_products_fit(self, T, x, w, row):
-        return (0 < T <= 64 and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous()
+        return (0 < T <= 64 and _called_plainly(x, w) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous()
                 and w.size(1) % 32 == 0 and w.size(2) % 32 == 0 and row % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 4 == 0
                 and w.size(0) <= 65535 and w.size(1) * w.size(2) < 2 ** 31)
 

@@ -46,3 +46,17 @@ def test_the_kernel_is_left_out_where_torch_itself_has_to_be_called():
     with TorchDispatchMode():
         seen.append(_called_plainly())
     assert len(seen) == 5 and not any(seen) and _called_plainly()
+
+
+def test_products_per_head_are_left_to_torch_where_it_has_to_be_called():
+    import torch
+    from qserve_amd.layers.ops import HipOps
+    x, w, seen = torch.ones(2, 3, 32).bfloat16(), torch.ones(3, 32, 64).bfloat16(), []
+    fits = lambda x, w: HipOps._head_products_fit(None, 2, x, w, 32)                             # noqa: E731
+    assert fits(x, w)
+    assert not fits(x, w.clone().requires_grad_()) and not fits(x.clone().requires_grad_(), w)
+    with torch.no_grad():
+        assert fits(x, w.clone().requires_grad_())
+    torch.vmap(lambda v: (seen.append(fits(x, v)), v)[1])(torch.stack([w, w]))
+    torch.func.jvp(lambda v: (seen.append(fits(x, v)), v)[1], (w,), (w,))
+    assert seen == [False, False]

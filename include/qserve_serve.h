@@ -260,14 +260,14 @@ int qsv_expert_slots(void* out, int float_out, const void* X, int div, const voi
  * place: slot -> sorted slot, offsets [n_experts + 1]: first sorted slot of every expert; indices below 0 and from n_experts on are left out of all
  * three), and the product takes those: out[s, r] = act(W[e][r, :] . X[order ? order[s] / div : s, :]) for the sorted slots of every expert
  * e, the input times in_weight[order ? order[s] : s] if given.  act: QSV_ACT_* (QSV_ACT_GLU: out is n_rows / 2 wide).  n_rows a multiple of
- * 4, K a multiple of 64, at most 8064 experts (_ok). */
+ * 4, K a multiple of 64 up to 2^23, at most 8064 experts (_ok). */
 int qsv_moe_sort(int32_t* order, int32_t* place, int32_t* offsets, const int32_t* idx, int n, int n_experts, void* stream);
 int qsv_grouped_gemm_sorted_ok(int n_experts, int n_rows, int K);
 int qsv_grouped_gemm_sorted(void* out, const void* X, const int32_t* order, int div, const void* W, const int32_t* offsets, int n_experts,
                             int n_rows, int K, int act, float limit, const float* in_weight, void* stream);
 /* The same product over work tiles that the caller lists: tiles int32 [n_tiles, 3] = (expert, first sorted slot, slots <=
  * qsv_grouped_gemm_tile_slots()), out[s, n] = act(W[e][n, :] . X[x_index ? x_index[s] / div : s, :]); K a multiple of
- * qsv_grouped_gemm_k_step(), n_rows a multiple of 4, n_tiles <= 65535.  X and W on 16 bytes. */
+ * qsv_grouped_gemm_k_step() up to 2^23, n_rows a multiple of 4, n_tiles <= 65535.  X and W on 16 bytes. */
 int qsv_grouped_gemm_tile_slots(void);
 int qsv_grouped_gemm_k_step(void);
 int qsv_grouped_gemm(void* out, const void* X, const int64_t* x_index, int div, const void* W, const int32_t* tiles,

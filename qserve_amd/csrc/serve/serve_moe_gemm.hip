@@ -33,6 +33,7 @@ __device__ __forceinline__ unsigned pack_bf2(float a, float b) { return (unsigne
 // 647 -> 620 us (915), 600 tokens 121 -> 106 us; 32 gated experts of 4096 x 2752: 3.5 ms -> 2547 -> 2494 us (888).
 constexpr int PR = 256, PS = 256, PWAVES = 8, PT = 64 * PWAVES;
 constexpr int PBUF = (PR + PS) * 128;               // bytes of one K step
+constexpr int MAX_K = 1 << 23;                      // (a tile's weight rows within 32-bit byte offsets)
 constexpr int LISTED_SLOTS = 128;                   // slots of a tile in a caller's list, at most
 constexpr int MAX_GROUPS = 8064;                   // (what is left of 160 KiB of LDS holds a count for each)
 
@@ -339,12 +340,12 @@ static int launch_grouped(const char* what, GroupedArgs a, int act, void* stream
     else hipLaunchKernelGGL((grouped_gemm_persistent_kernel<0, LISTED>), grid, block, 0, (hipStream_t)stream, a);
     return qsv_launch_status(what);
 }
-extern "C" int qsv_grouped_gemm_sorted_ok(int n_experts, int N, int K) { return n_experts > 0 && n_experts <= MAX_GROUPS && N > 0 && N % 4 == 0 && K > 0 && K % KS == 0; }
+extern "C" int qsv_grouped_gemm_sorted_ok(int n_experts, int N, int K) { return n_experts > 0 && n_experts <= MAX_GROUPS && N > 0 && N % 4 == 0 && K > 0 && K % KS == 0 && K <= MAX_K; }
 extern "C" int qsv_grouped_gemm_sorted(void* out, const void* X, const int32_t* order, int div, const void* W, const int32_t* offsets, int n_experts,
                                        int N, int K, int act, float limit, const float* in_weight, void* stream) {
     QSV_REQUIRE(out && X && W && offsets && div > 0, "qsv_grouped_gemm_sorted: bad arguments");
-    QSV_REQUIRE(qsv_grouped_gemm_sorted_ok(n_experts, N, K), "qsv_grouped_gemm_sorted: %d experts (at most %d), N %d (a multiple of 4), K %d (a multiple of %d)",
-                n_experts, MAX_GROUPS, N, K, KS);
+    QSV_REQUIRE(qsv_grouped_gemm_sorted_ok(n_experts, N, K), "qsv_grouped_gemm_sorted: %d experts (at most %d), N %d (a multiple of 4), K %d (a multiple of %d, at most %d)",
+                n_experts, MAX_GROUPS, N, K, KS, MAX_K);
     return launch_grouped<false>("qsv_grouped_gemm_sorted", {(bf16_t*)out, (const bf16_t*)X, (const bf16_t*)W, order, offsets, in_weight, div, n_experts, N, K,
                                                              limit, nullptr, nullptr, 0}, act, stream);
 }
@@ -354,7 +355,8 @@ extern "C" int qsv_grouped_gemm_k_step(void) { return KS; }
 extern "C" int qsv_grouped_gemm(void* out, const void* X, const int64_t* x_index, int div, const void* W, const int32_t* tiles, int n_tiles, int N, int K,
                                 int act, float limit, const float* in_weight, void* stream) {
     QSV_REQUIRE(out && X && W && tiles && div > 0 && n_tiles >= 0, "qsv_grouped_gemm: bad arguments");
-    QSV_REQUIRE(N > 0 && N % 4 == 0 && K > 0 && K % KS == 0, "qsv_grouped_gemm: N %d (a multiple of 4), K %d (a multiple of %d)", N, K, KS);
+    QSV_REQUIRE(N > 0 && N % 4 == 0 && K > 0 && K % KS == 0 && K <= MAX_K, "qsv_grouped_gemm: N %d (a multiple of 4), K %d (a multiple of %d, at most %d)", N,
+                K, KS, MAX_K);
     QSV_REQUIRE(n_tiles <= 65535, "qsv_grouped_gemm: %d tiles (at most 65535 per launch)", n_tiles);
     QSV_REQUIRE((int64_t)n_tiles * ((N + PR - 1) / PR) < (1ll << 30), "qsv_grouped_gemm: %d tiles of %d rows", n_tiles, N);
     if (n_tiles == 0) return QSV_OK;

@@ -107,6 +107,14 @@ def test_grouped_products_of_many_experts_are_taken():
     assert [ok(e, 128, 64) for e in (1, 1024, 1025, 8064, 8065)] == [1, 1, 1, 1, 0]
 
 
+def test_grouped_products_keep_a_tiles_weight_rows_within_32_bit_offsets():
+    from qserve_amd.serving._lib import lib
+    ok = lib().qsv_grouped_gemm_sorted_ok
+    K = [64 * k for k in (2 ** 17, 2 ** 17 + 1, 2 ** 18)]                    # 256 rows of 2^23 bfloat16 are 2^32 bytes
+    assert [ok(1, 256, k) for k in K] == [1, 0, 0]
+    assert lib().qsv_grouped_gemm(16, 16, None, 1, 16, 16, 1, 128, K[1], 0, 0.0, None, None) == 1 and b"at most" in lib().qsv_last_error()
+
+
 def test_serve_argument_validation_without_gpu():
     from qserve_amd.serving._lib import check, lib
     L = lib()

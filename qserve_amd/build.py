@@ -2,8 +2,8 @@
 
     python -m qserve_amd.build [--force]
 
-hipcc cross-compiles without a GPU, so this runs in the authoring container as well as on the MI355X box.
-The .so lands in qserve_amd/ (git-ignored, but shipped to the GPU box by gpurun).
+hipcc cross-compiles without a GPU, so this runs on any machine with ROCm's compiler.
+The .so lands in qserve_amd/ (git-ignored).
 """
 import argparse
 import concurrent.futures as cf

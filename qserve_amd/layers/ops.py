@@ -64,9 +64,9 @@ def _called_plainly(*ts):
 def linear(x, w):
     """x [T, in] @ w [out, in]^T in the storage type, float accumulation: the few rows of a decoding step (bfloat16 on a GPU) through
     qsv_skinny_linear, everything else through hipBLASLt / rocBLAS."""
-    if (type(x) is torch.Tensor and type(w) in (torch.Tensor, torch.nn.Parameter) and x.is_cuda and x.dim() == 2 and w.dim() == 2
+    if (type(x) is torch.Tensor and type(w) in (torch.Tensor, torch.nn.Parameter) and x.is_cuda and _called_plainly(x, w) and x.dim() == 2 and w.dim() == 2
             and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and w.is_contiguous() and 0 < x.size(0) and x.size(1) == w.size(1)
-            and x.size(1) and w.size(0) and _skinny(x.size(0), w.size(0), w.size(1)) and _called_plainly(x, w)
+            and x.size(1) and w.size(0) and _skinny(x.size(0), w.size(0), w.size(1))
             and x.stride(1) == 1 and x.size(1) % 8 == 0 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
             and x.device == w.device and x.device.index == torch.cuda.current_device()):
         from ..serving._lib import check, lib
@@ -168,7 +168,7 @@ class HipOps:
         return self.latent_query(q, q_abs, rope, pos, scale, heads, dim, rot_dim, rot_n, rank)
 
     def _head_products_fit(self, T, x, w, row):
-        return (0 < T <= 64 and _called_plainly(x, w) and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous()
+        return (_called_plainly(x, w) and 0 < T <= 64 and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous()
                 and w.size(1) % 32 == 0 and w.size(2) % 32 == 0 and row % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 4 == 0
                 and w.size(0) <= 65535 and w.size(1) * w.size(2) < 2 ** 31)
 

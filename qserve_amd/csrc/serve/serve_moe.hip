@@ -674,14 +674,18 @@ __global__ __launch_bounds__(NT) void moe_combine_kernel(T* __restrict__ y, cons
         for (int k = 0; k < top_k; ++k) {
             const size_t slot = t * top_k + k;
             const int e = idx ? idx[slot] : 0;
-            if (e < 0) continue;                                            // no expert: the slot has neither a row nor a place
-            const bool same = idx && e >= n_experts;                        // an identity expert's slot has no row of its own
+            const bool none = e < 0;                                        // no expert: the slot has neither a row nor a place
+            const bool same = idx && (unsigned)e >= (unsigned)n_experts;    // an identity expert's slot has no row of its own
             const float wk = weight ? weight[slot] : 1.0f;
             float v[VEC];
             if (same) loadv(h + t * D + c, v);
             else loadv(ys + (inv ? (size_t)inv[slot] : slot) * D + c, v);
+            // (taken out by value: behind a jump the slots' rows are requested one after another: 8192 tokens of 2048, top 4, 29 us against 40)
 #pragma unroll
-            for (int q = 0; q < VEC; ++q) a[q] += wk * v[q];
+            for (int q = 0; q < VEC; ++q) {
+                const float sum = a[q] + wk * v[q];
+                a[q] = none ? a[q] : sum;
+            }
         }
         storev(y + t * D + c, a);
     }

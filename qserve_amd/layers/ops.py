@@ -53,6 +53,18 @@ def _skinny(T, N, K):
             or (N >= 512 and K > 5120 and K % 512 != 0))
 
 
+def _prompt_splits(groups, span, partial_bytes, wide):
+    """Over how many workgroups the attention over plain rows cuts the keys of a prompt's tiles: `groups` workgroups without a cut, `span` keys at most,
+    partial_bytes of results one cut writes and the merge reads.  32 keys take a workgroup 1 us (3 us at rows of 512 and more), the merge 3.5 us and the partial
+    results move at 6.5 TB/s; no more workgroups than the chip holds at once.  Against every count over some 250 prompts of 3 - 4096 tokens, windows of 128 -
+    1024 among them: 1 % behind the best in the mean (2048 tokens, 16 heads on 4 pools, window 256: 26 us whole, 45 cut in two; 512 tokens behind 3584: 184
+    whole, 62 cut in eight)."""
+    most = max(1, min((256 if wide else 512) // max(groups, 1), span // 64, 32))
+    keys, moved = (span + 16) / 32 * (3.0 if wide else 1.0), partial_bytes / 6.5e6          # (us)
+    n = max(1, min(most, round((keys / moved) ** 0.5)))
+    return n if keys > 3.5 + keys / n + moved * n else 1
+
+
 def _called_plainly(*ts):
     """Whether nobody looks at torch's calls from outside: no function transform (vmap, jvp), no forward-mode level, no dispatch mode, no trace, no
     autocast, no gradient for one of ts.  A kernel launched past torch would be invisible to those.  (About 1 us.)"""
@@ -232,7 +244,7 @@ class HipOps:
                 # one, 18 with 8, 16 with 16; 256 wide on 4 pools, 64 sequences of 1000, one / two: 23 / 26 us)
                 splits = max(1, min((256 if wide else 384) // max(groups, 1), span // 96, 32)) if span > 256 else 1
             else:
-                splits = max(1, min((256 if wide else 512) // max(groups, 1), span // 64, 32))
+                splits = _prompt_splits(groups, span, 8 * T * H * rank, wide)
             splits = splits if key_splits is None else key_splits
             po = pm = None
             if splits > 1:

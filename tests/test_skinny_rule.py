@@ -1,7 +1,7 @@
 """Which products of few rows go to the kernel that streams the weight: pairs of measured times on either side of the rule's lines."""
 import pytest
 
-from qserve_amd.layers.ops import _skinny
+from qserve_amd.layers.ops import _prompt_splits, _skinny
 
 
 # rows, N, K where the vendor's product is the faster one by more than the runs differ
@@ -60,3 +60,12 @@ def test_products_per_head_are_left_to_torch_where_it_has_to_be_called():
     torch.vmap(lambda v: (seen.append(fits(x, v)), v)[1])(torch.stack([w, w]))
     torch.func.jvp(lambda v: (seen.append(fits(x, v)), v)[1], (w,), (w,))
     assert seen == [False, False]
+
+
+# workgroups without a cut, keys, tokens, heads, rank, wide rows: splits whose time is within a few per cent of the best
+@pytest.mark.parametrize("groups, span, T, H, rank, wide, good", [(256, 256, 2048, 16, 128, False, {1}), (256, 128, 2048, 16, 128, False, {1}), (128, 128, 512, 32, 128, False, {1}),
+                                                                  (192, 256, 2048, 12, 128, False, {1}), (256, 512, 4096, 8, 128, False, {1}), (64, 4096, 512, 16, 128, False, {6, 7, 8}),
+                                                                  (1, 4000, 8, 16, 512, True, {24, 32}), (128, 1024, 1024, 16, 512, True, {2}), (512, 4096, 4096, 16, 512, True, {1}),
+                                                                  (8, 64, 64, 16, 512, True, {1}), (64, 1000, 256, 16, 512, True, {4}), (1, 2, 2, 1, 128, False, {1})])
+def test_cuts_of_a_prompts_keys(groups, span, T, H, rank, wide, good):
+    assert _prompt_splits(groups, span, 8 * T * H * rank, wide) in good

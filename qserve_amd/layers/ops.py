@@ -53,6 +53,15 @@ def _skinny(T, N, K):
             or (N >= 512 and K > 5120 and K % 512 != 0))
 
 
+def _heads_stream(T, H, K, N):
+    """Whether the kernel for products per head beats the vendor's batched product and its copy back to rows for T <= 64 (both sides measured over H 1 - 128,
+    K 64 - 2048, N 64 - 2048; vendor / own, us).  It is made for weights that a step's latency outweighs and reads them again for every 32 columns, so it loses
+    with large ones (64 heads of 512 to 512, 1 / 64 rows 10.3 / 12.4, 16.7 / 18.3; 128 of 1536 to 192, 64 rows 24.7 / 46.4), sooner for one row of long
+    products, the vendor's best case (64 of 1024 to 128: 6.2 / 7.0), and for many rows (128 of 768 to 128, 64: 15.4 / 17.5; one of 2048 to 128, 33: 6.8 / 8.4)."""
+    size = H * K * N
+    return size <= (8_500_000 if T > 32 else 6_500_000 if T == 1 and K >= 1024 else 12_600_000) and (K <= 1024 or T <= 32)
+
+
 def _prompt_splits(groups, span, partial_bytes, wide):
     """Over how many workgroups the attention over plain rows cuts the keys of a prompt's tiles: `groups` workgroups without a cut, `span` keys at most,
     partial_bytes of results one cut writes and the merge reads.  32 keys take a workgroup 1 us (3 us at rows of 512 and more), the merge 3.5 us and the partial
@@ -188,7 +197,7 @@ class HipOps:
         """x [T, H, K], w [H, K, N] -> [T, H N], head by head: a step's few rows (up to 64) in one launch (16 heads of 512 to 128, 1 / 16 / 64 tokens:
         3.1 / 3.5 / 5.3 us, the vendor's with its copy back to rows 9.8 / 12.9 / 13.3), more through the vendor's batched product."""
         T, H, K = x.shape
-        if self._head_products_fit(T, x, w, K):
+        if _heads_stream(T, H, K, w.size(2)) and self._head_products_fit(T, x, w, K):
             self._need(x, w)
             assert w.size(0) == H and w.size(1) == K
             out = torch.empty((T, H * w.size(2)), dtype=x.dtype, device=x.device)

@@ -1,7 +1,7 @@
 """Which products of few rows go to the kernel that streams the weight: pairs of measured times on either side of the rule's lines."""
 import pytest
 
-from qserve_amd.layers.ops import _prompt_splits, _skinny
+from qserve_amd.layers.ops import _heads_stream, _prompt_splits, _skinny
 
 
 # rows, N, K where the vendor's product is the faster one by more than the runs differ
@@ -60,6 +60,14 @@ def test_products_per_head_are_left_to_torch_where_it_has_to_be_called():
     torch.vmap(lambda v: (seen.append(fits(x, v)), v)[1])(torch.stack([w, w]))
     torch.func.jvp(lambda v: (seen.append(fits(x, v)), v)[1], (w,), (w,))
     assert seen == [False, False]
+
+
+# rows, heads, K, N
+@pytest.mark.parametrize("T, H, K, N, takes", [(1, 16, 512, 128, True), (64, 16, 512, 128, True), (64, 128, 512, 128, True), (1, 32, 192, 1536, True), (16, 16, 1536, 192, True),
+                                               (1, 64, 1024, 128, False), (1, 64, 512, 512, False), (64, 128, 1536, 192, False), (64, 128, 768, 128, False),
+                                               (33, 1, 2048, 128, False), (16, 32, 2048, 512, False)])
+def test_products_per_head_that_the_kernel_is_faster_at(T, H, K, N, takes):
+    assert _heads_stream(T, H, K, N) is takes
 
 
 # workgroups without a cut, keys, tokens, heads, rank, wide rows: splits whose time is within a few per cent of the best

@@ -1029,11 +1029,15 @@ extern "C" int qsv_recurrent_scan(float* o, const void* q, int64_t q_stride, con
                 "qsv_recurrent_scan: bad sizes (%d heads over %d, state %d x %d)", heads, qk_heads, dim, vdim);
     if (n_runs == 0) return QSV_OK;
     const int qkv = qkv_dtype == QSV_F32 ? QSV_F32 : QSV_BF16;
-    if (dim > 32 && dim <= 128 && dim % 4 == 0 && vdim % 4 == 0 && v_cols % 4 == 0 && q_stride % 4 == 0 && k_stride % 4 == 0 && v_stride % 4 == 0 &&
+    // Short runs of narrow states leave its lanes without columns and its chunks without tokens, which counts once the CUs have no workgroup left over (64 runs
+    // of 2 tokens, 64 heads of 64 x 4: 13.6 us with the general kernel, 28 here; 64 heads of 64 x 24: 32 and 30; 64 runs of 64 tokens 0.9 of its time).
+    const bool narrow = vdim <= (dim <= 64 ? 16 : 8) && max_run <= 8 && (int64_t)n_runs * heads >= 1024;
+    if (!narrow && dim > 32 && dim <= 128 && dim % 4 == 0 && vdim % 4 == 0 && v_cols % 4 == 0 && q_stride % 4 == 0 && k_stride % 4 == 0 && v_stride % 4 == 0 &&
         fits4(q, qkv) && fits4(k, qkv) && fits4(v, qkv) && fits4(decay, QSV_F32) && fits4(o, QSV_F32) && vdim <= 65535 * 32) {
         const int lpc = dim <= 64 ? 4 : 8, cols = 4 * 64 / lpc;
-        // two columns per lane while that gives every CU a workgroup (half as many CUs: a token costs them as much as it would cost all)
-        const bool two = (int64_t)n_runs * heads * ((vdim + 2 * cols - 1) / (2 * cols)) >= 256;
+        // two columns per lane while that gives every CU a workgroup (half as many CUs: a token costs them as much as it would cost all) and the
+        // state has more columns than one per lane serves (16 runs of 64 tokens, 32 heads of 64 x 32, delta rule: 46 -> 29 us)
+        const bool two = vdim > cols && (int64_t)n_runs * heads * ((vdim + 2 * cols - 1) / (2 * cols)) >= 256;
         const dim3 grid(n_runs, heads, two ? (vdim + 2 * cols - 1) / (2 * cols) : (vdim + cols - 1) / cols), block(256);
 #define QSV_STEP_P(TQ, TB, DELTA, LPC, NC)                                                                                      \
     hipLaunchKernelGGL((recurrent_rows_kernel<TQ, TB, DELTA, LPC, NC>), grid, block, 0, (hipStream_t)stream, o, (const TQ*)q, q_stride, \

@@ -119,7 +119,10 @@ def test_one_token_of_the_recurrence(H, G, dim, vdim, v_cols, dtype, delta):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("counts, H, G, dim, vdim, v_cols", [((1, 15, 16, 17, 33), 2, 1, 64, 128, 128), ((31, 32), 130, 65, 64, 132, 128), ((5, 48), 3, 3, 36, 4, 4),
                                                              ((16, 49), 2, 1, 68, 36, 32), ((2, 40), 128, 64, 128, 64, 64), ((20, 3), 2, 2, 128, 68, 68),
-                                                             ((18, 2), 2, 2, 32, 64, 64), ((17, 2), 2, 2, 132, 12, 12), ((17, 2), 2, 2, 34, 10, 9)])
+                                                             ((18, 2), 2, 2, 32, 64, 64), ((17, 2), 2, 2, 132, 12, 12), ((17, 2), 2, 2, 34, 10, 9),
+                                                             # many workgroups: no more columns than one per lane, narrow states in short and in longer runs
+                                                             ((17, 2), 160, 80, 64, 24, 24), ((3, 2), 512, 256, 64, 16, 16), ((9, 2), 512, 256, 40, 16, 16),
+                                                             ((8, 1), 512, 512, 68, 8, 8), ((2, 3), 512, 512, 72, 12, 12)])
 def test_runs_of_the_recurrence(counts, H, G, dim, vdim, v_cols, dtype, delta):
     """Full chunks of 16 tokens and what is left of them, one and two columns per lane, rows and columns that do not fill a workgroup."""
     g = _gen(dim + vdim)

@@ -759,17 +759,19 @@ __global__ __launch_bounds__(NT) void head_rms_gate_kernel(T* __restrict__ out, 
     }
 }
 
-// The same for heads of 4 to 256 values, a power of two: a thread owns four values of a head, a head is 1 - 64 neighbouring lanes, a token `chunks`
-// workgroups; everything is read once, before the sum.  (16 heads of 128: 16 tokens 5.6 -> 2.3 us, 8192 tokens 44 -> 31 us.)
+// The same for heads of 4 to 256 values, a power of two: a thread owns four values of a head, a head is 1 - 64 neighbouring lanes, and the
+// heads of all tokens follow one another; everything is read once, before the sum.  (16 heads of 128: 16 tokens 5.6 -> 2.3 us, 8192 tokens 44 -> 31 us;
+// one head of 64, 8192 tokens: 3.4 us, with a workgroup per token 8.1.)
 template <typename T>
 __global__ __launch_bounds__(NT) void head_rms_gate_vec_kernel(T* __restrict__ out, const float* __restrict__ o, const T* __restrict__ w,
                                                                const T* __restrict__ gate, int64_t gate_stride, int gate_kind, float eps, int H,
                                                                int vdim, int lanes_log, int o_stride, int w_stride,
-                                                               const float* __restrict__ den_m, int chunks) {
-    const unsigned t = blockIdx.x / (unsigned)chunks, idx = (blockIdx.x - t * chunks) * NT + threadIdx.x;
-    const bool in = (int)(idx >> lanes_log) < H;
-    const int h = in ? idx >> lanes_log : 0, e = (idx & ((1 << lanes_log) - 1)) * 4;
-    const size_t th = (size_t)t * H + h;
+                                                               const float* __restrict__ den_m, unsigned n_heads) {
+    const unsigned idx = blockIdx.x * NT + threadIdx.x;
+    const bool in = idx >> lanes_log < n_heads;
+    const unsigned row = in ? idx >> lanes_log : 0, t = row / (unsigned)H;
+    const int h = row - t * H, e = (idx & ((1 << lanes_log) - 1)) * 4;
+    const size_t th = row;
     float x[4], g[4], ww[4];
     ld4t(o, th * (size_t)o_stride + e, x);
     ld4t(gate, t * gate_stride + (size_t)h * vdim + e, g);
@@ -1154,12 +1156,12 @@ extern "C" int qsv_head_rms_gate(void* out, const float* o, const void* w, const
         fits4(o, QSV_F32) && fits4(w, dtype) && fits4(gate, dtype) && heads <= (1 << 20)) {
         int lanes_log = 0;
         while ((4 << lanes_log) < vdim) ++lanes_log;
-        const int64_t chunks = (((int64_t)heads << lanes_log) + NT - 1) / NT;
-        if (chunks * n_tokens < (1ll << 31)) {
+        const int64_t n_heads = (int64_t)n_tokens * heads, lanes = n_heads << lanes_log;
+        if (lanes < (1ll << 32) - NT) {
             QSV_DISPATCH(dtype, "qsv_head_rms_gate",
                          hipLaunchKernelGGL(head_rms_gate_vec_kernel<T>, dim3((unsigned)(chunks * n_tokens)), dim3(NT), 0, (hipStream_t)stream,
                                             (T*)out, o, (const T*)w, (const T*)gate, gate_stride, gate_kind, eps, heads, vdim, lanes_log, o_stride,
-                                            w_per_head ? vdim : 0, den_m, (int)chunks));
+                                            w_per_head ? vdim : 0, den_m, (unsigned)n_heads));
             return qsv_launch_status("qsv_head_rms_gate");
         }
     }

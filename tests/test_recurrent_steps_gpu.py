@@ -56,7 +56,9 @@ def test_convolution_and_unit_vectors(C, taps, n_unit, dim, dtype):
 @pytest.mark.parametrize("kind", ["silu", "sigmoid"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("T, H, dv, extra, per_head", [(1, 16, 128, 0, False), (17, 5, 4, 0, True), (3, 3, 256, 4, True), (5, 7, 64, 0, True), (2, 2, 96, 0, False),
-                                                       (4, 3, 16, 1, False), (3, 2, 512, 0, True)])
+                                                       (4, 3, 16, 1, False), (3, 2, 512, 0, True),
+                                                       # heads of several tokens in a workgroup, the last one part empty
+                                                       (37, 1, 64, 0, True), (300, 1, 4, 4, False), (9, 3, 256, 0, True)])
 def test_read_out_norm_and_gate(T, H, dv, extra, per_head, dtype, kind):
     g = _gen(T + dv)
     o, gate = torch.randn(T, H, dv + extra, device=DEV, generator=g), torch.randn(T, H * dv + 8, device=DEV, generator=g).to(dtype)[:, 4:4 + H * dv]

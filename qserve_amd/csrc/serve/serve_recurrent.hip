@@ -1159,7 +1159,7 @@ extern "C" int qsv_head_rms_gate(void* out, const float* o, const void* w, const
         const int64_t n_heads = (int64_t)n_tokens * heads, lanes = n_heads << lanes_log;
         if (lanes < (1ll << 32) - NT) {
             QSV_DISPATCH(dtype, "qsv_head_rms_gate",
-                         hipLaunchKernelGGL(head_rms_gate_vec_kernel<T>, dim3((unsigned)(chunks * n_tokens)), dim3(NT), 0, (hipStream_t)stream,
+                         hipLaunchKernelGGL(head_rms_gate_vec_kernel<T>, dim3((unsigned)((lanes + NT - 1) / NT)), dim3(NT), 0, (hipStream_t)stream,
                                             (T*)out, o, (const T*)w, (const T*)gate, gate_stride, gate_kind, eps, heads, vdim, lanes_log, o_stride,
                                             w_per_head ? vdim : 0, den_m, (unsigned)n_heads));
             return qsv_launch_status("qsv_head_rms_gate");

@@ -180,7 +180,7 @@ __global__ __launch_bounds__(NT) void moe_route_kernel(int32_t* __restrict__ idx
 
 // The same for at most 64 experts and widths that are multiples of 8 (one expert per lane in the selection).  The wide form's time went
 // into serial steps: a wave took its experts one by one, six shuffles each, and the selection was (keep + top_k) wave-wide argmax searches
-// with a barrier each.  Here the four waves split the width and hold 16 experts' sums for TT tokens side by side, the sums are reduced and
+// with a barrier each.  Here the four waves split the width and hold EC experts' sums for TT tokens side by side, the sums are reduced and
 // scattered over the lanes in one butterfly, and a lane finds its expert's place by counting the better ones (broadcasts, no search).
 // TT = 4 tokens share the router's rows in prompts; in steps one token per workgroup keeps more workgroups busy.
 __device__ __forceinline__ unsigned order_key(float v) {         // larger key = larger value; -0 = +0, NaN below everything
@@ -207,12 +207,12 @@ template <>
 struct Piece<float> {
     typedef float8 type;
 };
-template <typename T, int TT>
+template <typename T, int TT, int EC>
 __global__ __launch_bounds__(NT, 2) void moe_route_wave_kernel(int32_t* __restrict__ idx, float* __restrict__ weight, const T* __restrict__ h,
                                                             const T* __restrict__ router, const T* __restrict__ bias, int renorm, int n, int D, int E,
                                                             int top_k, int G, int keep, int score_fn, const float* __restrict__ correction,
                                                             int group_top, float scale) {
-    constexpr int EC = 16, NV = TT * EC;
+    constexpr int NV = TT * EC;
     __shared__ float part[NW][TT][64];
     __shared__ float cs[NW][64];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -788,13 +788,18 @@ extern "C" int qsv_moe_route(int32_t* idx, float* weight, const void* h, const v
                 "qsv_moe_route: %d experts in %d groups, %d groups kept, top %d", E, G, keep, top_k);
     if (n == 0) return QSV_OK;
     if (E <= 64 && D % 8 == 0) {
-#define QSV_ROUTE(TT)                                                                                                            \
+#define QSV_ROUTE(TT, EC)                                                                                                         \
     QSV_DISPATCH(dtype, "qsv_moe_route",                                                                                         \
-                 hipLaunchKernelGGL((moe_route_wave_kernel<T, TT>), dim3((n + TT - 1) / TT), dim3(NT), 0, (hipStream_t)stream, idx, weight, \
+                 hipLaunchKernelGGL((moe_route_wave_kernel<T, TT, EC>), dim3((n + TT - 1) / TT), dim3(NT), 0, (hipStream_t)stream, idx, weight, \
                                     (const T*)h, (const T*)router, (const T*)bias, renorm, n, D, E, top_k, G, keep, score_fn, correction, \
                                     group_top, scale))
-        if (n >= 1024) QSV_ROUTE(4);
-        else QSV_ROUTE(1);
+        // four tokens a workgroup where the router's rows are long or the tokens fill the chip all the same (1024 tokens, 64 experts of 64, one token /
+        // four: 14.9 / 19.1 us; 8 of 8192 13.8 / 11.9); eight sums side by side for at most eight experts (1000 tokens, 2 of 8192: 13.6 -> 8.5 us)
+        const bool four = n >= 1024 && (D >= 1024 || n >= 2048);
+        if (E <= 8 && four) QSV_ROUTE(4, 8);
+        else if (E <= 8) QSV_ROUTE(1, 8);
+        else if (four) QSV_ROUTE(4, 16);
+        else QSV_ROUTE(1, 16);
 #undef QSV_ROUTE
         return qsv_launch_status("qsv_moe_route");
     }

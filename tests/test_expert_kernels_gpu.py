@@ -148,11 +148,11 @@ def test_sizes_and_addresses_between_the_forms(ops, T, top, E, D, ff, shift, gra
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("n", [1, 5, 1023, 1025])
+@pytest.mark.parametrize("n", [1, 5, 1023, 1025, 2050])
 @pytest.mark.parametrize("E, G, keep, top, D, score, group_top, renorm", [
     (1, 1, 1, 1, 8, "softmax", 1, False), (16, 4, 2, 4, 2048, "softmax", 1, False), (16, 1, 1, 4, 2040, "softmax", 1, True),
     (17, 17, 5, 3, 64, "sigmoid", 1, False), (64, 8, 3, 24, 4096, "sigmoid", 2, True), (33, 1, 1, 33, 136, "sigmoid", 1, False),
-    (64, 64, 64, 6, 8, "softmax", 1, False)])
+    (64, 64, 64, 6, 8, "softmax", 1, False), (8, 2, 1, 3, 1032, "softmax", 1, True), (9, 1, 1, 2, 1024, "sigmoid", 1, False)])
 def test_router(dtype, n, E, G, keep, top, D, score, group_top, renorm):
     if not torch.cuda.is_available():
         pytest.skip("no GPU")

@@ -117,6 +117,8 @@ __device__ __forceinline__ void st4t(float* p, size_t i, const float (&v)[4]) { 
 __device__ __forceinline__ void st4t(bf16_t* p, size_t i, const float (&v)[4]) {
     *(uint2*)(p + i) = make_uint2((unsigned)f2bf(v[0]) | ((unsigned)f2bf(v[1]) << 16), (unsigned)f2bf(v[2]) | ((unsigned)f2bf(v[3]) << 16));
 }
+// token of a workgroup where each has `chunks` of them, neighbours (one: no division, which a kernel of 3 us would notice)
+__device__ __forceinline__ unsigned token_of(unsigned block, int chunks) { return chunks == 1 ? block : block / (unsigned)chunks; }
 // an address that 4 elements of its type may be read from at once
 inline bool fits4(const void* p, int dtype) { return (uintptr_t)p % (dtype == QSV_BF16 ? 8 : 16) == 0; }
 

@@ -94,7 +94,7 @@ __global__ __launch_bounds__(NT) void conv_silu_unit_vec_kernel(float* __restric
                                                                 const int32_t* __restrict__ state_wr, int unit_channels, int group_lanes, int act,
                                                                 int chunks) {
     constexpr int PAST = TAPS - 1;
-    const unsigned t = blockIdx.x / (unsigned)chunks;
+    const unsigned t = token_of(blockIdx.x, chunks);
     const int c = ((blockIdx.x - t * chunks) * NT + threadIdx.x) * 4;
     const bool in = c < C;
     const int from = in ? c : 0;                                   // (lanes behind the end stay for the sums below)
@@ -891,7 +891,7 @@ __global__ __launch_bounds__(NT) void attention_prep_vec_kernel(float* __restric
                                                                 int G, int dim, int vdim, int rot_n, const float* __restrict__ rope_k,
                                                                 const float* __restrict__ rope_v, float scale, const int64_t* __restrict__ slot,
                                                                 const int32_t* __restrict__ pos, int chunks) {
-    const unsigned t = blockIdx.x / (unsigned)chunks, idx = (blockIdx.x - t * chunks) * NT + threadIdx.x;
+    const unsigned t = token_of(blockIdx.x, chunks), idx = (blockIdx.x - t * chunks) * NT + threadIdx.x;
     const unsigned R = vdim + dim;
     const int u = idx / (R / 4), c = (idx - u * (R / 4)) * 4, p = pos[t];
     if (u >= H + G) return;
@@ -952,7 +952,8 @@ extern "C" int qsv_conv_silu_unit(float* out, const void* proj, int64_t stride, 
     QSV_REQUIRE((size_t)channels * 4 <= 64 * 1024, "qsv_conv_silu_unit: %d channels do not fit the workgroup's LDS", channels);
     if (n_tokens == 0) return QSV_OK;
     const int64_t chunks = ((int64_t)channels / 4 + NT - 1) / NT;
-    if (taps >= 2 && taps <= 4 && channels % 4 == 0 && off % 4 == 0 && stride % 4 == 0 && fits4(proj, dtype) && fits4(out, QSV_F32) &&
+    // (a prompt of few channels: one lane in eight has any, 8192 tokens of 96: 11.3 -> 13.1 us)
+    if ((channels >= 256 || n_tokens < 1024) && taps >= 2 && taps <= 4 && channels % 4 == 0 && off % 4 == 0 && stride % 4 == 0 && fits4(proj, dtype) && fits4(out, QSV_F32) &&
         fits4(w, QSV_F32) && fits4(hist, QSV_F32) && chunks * n_tokens < (1ll << 31) &&
         (n_unit == 0 || (unit_dim >= 4 && unit_dim <= 256 && (unit_dim & (unit_dim - 1)) == 0))) {
         const dim3 grid((unsigned)(chunks * n_tokens));

@@ -253,7 +253,7 @@ template <typename T>
 __global__ __launch_bounds__(NT) void latent_query_vec_kernel(float* __restrict__ qf, const T* __restrict__ q, const T* __restrict__ q_abs,
                                                               const float* __restrict__ rope, const int32_t* __restrict__ pos, float scale,
                                                               int n_tokens, int H, int dim, int rot_dim, int rot_n, int rank, int chunks) {
-    const unsigned t = blockIdx.x / (unsigned)chunks, i = (blockIdx.x - t * chunks) * NT + threadIdx.x;
+    const unsigned t = token_of(blockIdx.x, chunks), i = (blockIdx.x - t * chunks) * NT + threadIdx.x;
     const unsigned R = rank + rot_dim, h = i / (R / 4), c = (i - h * (R / 4)) * 4;
     if (h >= (unsigned)H) return;
     float v[4];

@@ -82,9 +82,10 @@ __global__ __launch_bounds__(NT) void hc_write_kernel(float* __restrict__ x, con
 // ---- the same two kernels for widths that are multiples of four: 16-byte stream accesses, four elements per thread and pass, `chunks` workgroups
 // per token ----
 // A step's few tokens are spread over as many workgroups as their width fills: one pass each (read / written, 16 tokens of 2 x 2048: 3.2 -> 2.5 /
-// 5.4 -> 3.4 us, 64 of 2 x 4096: 4.6 -> 2.6 / 9.1 -> 3.6).  Enough tokens to fill the chip keep one, with fewer workgroups to start (8192 of 2 x
-// 2048, shifted: 47 us against 51).
-inline int stream_chunks(int n, int D) { return n >= 1024 ? 1 : (int)(((int64_t)D + 4 * NT - 1) / (4 * NT)); }
+// 5.4 -> 3.4 us, 64 of 2 x 4096: 4.6 -> 2.6 / 9.1 -> 3.6).  Enough tokens to fill the chip keep one, with fewer workgroups to start: from 1024 for the
+// reading kernel (8192 of 2 x 2048, shifted: 47 us against 51; 1023 of 4 x 2048 spread: 6.9 against 7.9), above 512 for the writing one, which keeps more
+// in registers (1023 of 2 x 4096: 17.6 us against 19.4).
+inline int stream_chunks(int n, int most, int D) { return n > most ? 1 : (int)(((int64_t)D + 4 * NT - 1) / (4 * NT)); }
 __device__ __forceinline__ void stream_sum4(const float* __restrict__ x, const float* __restrict__ w_in, size_t t, int S, int D, int i,
                                             float (&u)[4]) {
     u[0] = u[1] = u[2] = u[3] = 0.f;
@@ -103,7 +104,7 @@ __global__ __launch_bounds__(NT) void hc_read_vec_kernel(T* __restrict__ h, cons
                                                          const T* __restrict__ shift, float* __restrict__ prev,
                                                          const int32_t* __restrict__ run_off, const int32_t* __restrict__ state_rd,
                                                          const int32_t* __restrict__ state_wr, int S, int D, int chunks) {
-    const size_t t = blockIdx.x / (unsigned)chunks;
+    const size_t t = token_of(blockIdx.x, chunks);
     const bool shifted = shift != nullptr;
     const int off = shifted ? run_off[t] : 0, rd = shifted ? state_rd[t] : -1, wr = shifted ? state_wr[t] : -1;
     for (int i = ((blockIdx.x - (unsigned)t * chunks) * NT + threadIdx.x) * 4; i < D; i += chunks * NT * 4) {
@@ -136,7 +137,7 @@ __global__ __launch_bounds__(NT) void hc_write_vec_kernel(float* __restrict__ x,
                                                           const float* __restrict__ w_out, int S, int D, T* __restrict__ h_next,
                                                           const float* __restrict__ w_in_next, const T* __restrict__ nw,
                                                           const T* __restrict__ nb, float alpha, int chunks) {
-    const size_t t = blockIdx.x / (unsigned)chunks;
+    const size_t t = token_of(blockIdx.x, chunks);
     for (int i = ((blockIdx.x - (unsigned)t * chunks) * NT + threadIdx.x) * 4; i < D; i += chunks * NT * 4) {
         float old[MAX_STREAMS][4], yv[4], u[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -278,7 +279,7 @@ extern "C" int qsv_hc_read(void* h, const float* x, const float* w_in, const voi
     QSV_REQUIRE(h && x && w_in && norm_w && norm_b && n >= 0 && D > 0 && streams > 0, "qsv_hc_read: bad arguments");
     QSV_REQUIRE(!shift || (prev && run_off && state_rd && state_wr), "qsv_hc_read: token shift without its state");
     if (n == 0) return QSV_OK;
-    const int chunks = stream_chunks(n, D);
+    const int chunks = stream_chunks(n, 1023, D);
     if (D % 4 == 0)
         QSV_DISPATCH(dtype, "qsv_hc_read",
                      hipLaunchKernelGGL(hc_read_vec_kernel<T>, dim3((unsigned)(chunks * n)), dim3(NT), 0, (hipStream_t)stream, (T*)h, x, w_in,
@@ -297,7 +298,7 @@ extern "C" int qsv_hc_write(float* x, const void* y, const float* mix, const flo
     QSV_REQUIRE(!h_next || (w_in_next && norm_w && norm_b), "qsv_hc_write: the next sublayer's input without its weights");
     QSV_REQUIRE(streams > 0 && streams <= MAX_STREAMS, "qsv_hc_write: %d streams (at most %d)", streams, MAX_STREAMS);
     if (n == 0) return QSV_OK;
-    const int chunks = stream_chunks(n, D);
+    const int chunks = stream_chunks(n, 512, D);
     if (D % 4 == 0)
         QSV_DISPATCH(dtype, "qsv_hc_write",
                      hipLaunchKernelGGL(hc_write_vec_kernel<T>, dim3((unsigned)(chunks * n)), dim3(NT), 0, (hipStream_t)stream, x, (const T*)y, mix, w_out,

@@ -166,3 +166,30 @@ def test_streams_read_and_written(S, D, dtype):
     x1, x2 = x.clone(), x.clone()
     got, want = hip.hc_write(x1, y, mix, w_out, (w_in, norm)), ref.hc_write(x2, y, mix, w_out, (w_in, norm))
     assert ((x1 - x2).abs() <= tol).all() and ((got.float() - want).abs() <= tol + _rounded(dtype, want)).all()
+
+
+@pytest.mark.parametrize("T", [512, 513, 1023, 1024])
+def test_streams_at_the_lines_of_the_split(T):
+    """A token's row over several workgroups and in one, at both kernels' lines."""
+    g = _gen(T)
+    S, D = 2, 2052
+    x, y, w_in, mix, w_out = (torch.randn(*s, device=DEV, generator=g) for s in ((T, S, D), (T, D), (S,), (S, S), (S,)))
+    norm = (torch.randn(D, device=DEV, generator=g), torch.randn(D, device=DEV, generator=g), 0.7)
+    hip, ref = HipOps(torch.float32), TorchOps(torch.float32)
+    tol = 2.0 ** -24 * 64 * 16                                                # (values below 2^6, some ten float roundings on either side)
+    assert ((hip.hc_read(x, w_in, norm) - ref.hc_read(x, w_in, norm)).abs() <= tol).all()
+    x1, x2 = x.clone(), x.clone()
+    got, want = hip.hc_write(x1, y, mix, w_out, (w_in, norm)), ref.hc_write(x2, y, mix, w_out, (w_in, norm))
+    assert ((x1 - x2).abs() <= tol).all() and ((got - want).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("C", [96, 252, 256])
+@pytest.mark.parametrize("T", [1023, 1024])
+def test_convolution_of_few_channels(T, C):
+    g = _gen(T + C)
+    b = _batch([5, T - 5], [9, 0])
+    proj, w, hist = torch.randn(T, C, device=DEV, generator=g), torch.randn(C, 4, device=DEV, generator=g), torch.randn(4, 3, C, device=DEV, generator=g)
+    h1, h2 = hist.clone(), hist.clone()
+    y, ref = HipOps(torch.float32).conv_silu_unit(proj, 0, w, h1, b, 3, 4), TorchOps(torch.float32).conv_silu_unit(proj, 0, w, h2, b, 3, 4)
+    # values below 2^5, some ten float roundings on either side; a unit vector divides by a length above 2^-2
+    assert ((y - ref).abs() <= 2.0 ** -24 * 2.0 ** 5 * 20 * 4).all() and torch.equal(h1, h2)

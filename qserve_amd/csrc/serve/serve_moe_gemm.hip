@@ -19,30 +19,69 @@ constexpr int KS = 64;       // reduction elements per step
 
 __device__ __forceinline__ unsigned pack_bf2(float a, float b) { return (unsigned)f2bf(a) | ((unsigned)f2bf(b) << 16); }
 
-// Tiles of 256 weight rows x 256 slots (128 or 64 where an expert has no more left).  Bound by the matrix cores.  Eight waves (64 rows x 128
-// slots each, two per SIMD) multiply while the next K step of 64 is copied straight into the other half of a 128 KiB LDS buffer
-// (global_load_lds, one 128-byte line per row; pieces permuted by the row's number: 16-byte reads without bank conflicts); one barrier
-// per step.  Workgroups are persistent (one per CU): each finds its tiles from the experts' offsets - no tile list, no count reaches
-// the host -, an XCD's workgroups walk neighbouring tiles (shared weight and input panels in its L2), and the last step of a tile copies the
-// first one of the next, so the epilogue's stores have something to hide behind.  A tile with few slots gives each wave fewer columns
-// instead of multiplying padding, and no copies of inputs it does not have; an XCD cuts the tiles of its last, part-empty round by slots into
+// Tiles of 256 weight rows x 256 slots (128 or 64 where an expert has no more left).  Bound by the matrix cores.
+//
+// Eight waves, two per SIMD: waves 0 - 3 and 4 - 7 are half a phase apart, so that one of a SIMD's two always multiplies while the other reads
+// its next operands.  A K step of 64 has four phases, one per quarter of the tile (halves of 128 rows x halves of 128 slots; in each a wave has 64
+// rows x 32 slots: 16 instructions); a phase reads ONE operand half (8 or 4 reads of 16 bytes a lane), requests the same half of the step after the
+// next one into the place that the half read a phase earlier left (global_load_lds, whole 128-byte lines of a row; pieces permuted by the row's number:
+// 16-byte reads without bank conflicts), and waits for what the next phase reads, which was requested seven phases before: 96 - 112 KiB in flight
+// a CU, no wait for the youngest requests.  Every wave issues the same requests in every phase - of rows that a tile does not have with no
+// lane active - so that the counted waits hold whatever the tile's size.
+//
+// Workgroups are persistent (one per CU): each finds its tiles from the experts' offsets - no tile list, no count reaches the host -, the last
+// two steps of a tile request the first two of the next one, so the epilogue's stores have something to hide behind.  An XCD's workgroups walk
+// bands of 8 row tiles and through an expert's slots inside a band: 8 weight and 4 input panels are in its L2 at a time, where rows first meant 22
+// and 2.  A tile with few slots multiplies and requests those only; an XCD cuts the tiles of its last, part-empty round by slots into
 // halves where at most half of its 32 workgroups have one, into quarters where at most a quarter have: with more than half nothing is cut, and
 // fewer than eight tiles leave workgroups idle.  The XCDs' shares are ceil(tiles / 8) each, so the last of them can be short or empty.
-// Measured (MI355X, both products with sort and combine): 8192 tokens, 4 of 16 experts of 2048 x 1408: 1010 us (the form before: 256 x 128 tiles staged
-// through registers, tile list from the host, torch's sort) -> 485 -> 463 (with the cut of the last round, in turn; 815 TFLOP/s), gated
-// 647 -> 620 us (915), 600 tokens 121 -> 106 us; 32 gated experts of 4096 x 2752: 3.5 ms -> 2547 -> 2494 us (888).
+//
+// Measured (MI355X, one product, the form before -> now in one call; before: eight waves in step, one barrier and a wait for every request per K step, rows
+// first): 32768 slots x 4096 x 4096 1014 -> 866 us (1270 TFLOP/s; hipBLASLt's dense product of that size 740), 28480 slots over 32 experts gated
+// 5504 x 4096 1380 -> 1230 (1045), 4096 x 2752 686 -> 587 (1095), 32768 over 16 of 1408 x 2048 204 -> 203, 2048 x 1408 201 -> 185, 8188 over 16 gated 2816 x 2048
+// 118 -> 115, 2048 x 1408 63.6 -> 64.5, 1300 over 16 of these 44.4 -> 42.4, 28.9 -> 29.8.  A K step takes 1.5 us, which is the card's power: the same
+// instructions on constant data take 1.1.  How far ahead the requests run (3 - 7 phases) and bands of 4 - 12 make no difference.
 constexpr int PR = 256, PS = 256, PWAVES = 8, PT = 64 * PWAVES;
 constexpr int PBUF = (PR + PS) * 128;               // bytes of one K step
+constexpr int HALF = 128 * 128;                     // of an operand half of it
+constexpr int BAND = 8;                             // row tiles of a band
 constexpr int MAX_K = 1 << 23;                      // (a tile's weight rows within 32-bit byte offsets)
 constexpr int LISTED_SLOTS = 128;                   // slots of a tile in a caller's list, at most
-constexpr int MAX_GROUPS = 8064;                   // (what is left of 160 KiB of LDS holds a count for each)
+constexpr int SIDE = (160 * 1024 - 2 * PBUF) / 4;   // what is left of LDS, in words: a count for each expert,
+constexpr int AHEAD = SIDE - PWAVES * 64;           // and where they leave room the next tile's input rows
+constexpr int MAX_GROUPS = 8064;
 
 typedef __attribute__((address_space(3))) void* lds_ptr;
-__device__ __forceinline__ void lds_copy16(unsigned dst, const void* base, unsigned off) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(dst) : "memory");
+// A request into LDS by all lanes (left < 0: 1 KiB) or by the first one alone, for the counted waits' sake: an instruction without a lane need not count.
+__device__ __forceinline__ void lds_copy16(unsigned dst, const void* base, unsigned off, int left) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_ashr_i32 exec_hi, %3, 31\n\ts_or_b32 exec_lo, exec_hi, 1\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(off), "s"(base), "s"(dst), "s"(left) : "memory", "scc");
 }
-__device__ __forceinline__ void lds_copy16(unsigned dst, const void* from) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(dst) : "memory");
+__device__ __forceinline__ void lds_copy16(unsigned dst, const void* from, int left) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_ashr_i32 exec_hi, %2, 31\n\ts_or_b32 exec_lo, exec_hi, 1\n\tglobal_load_lds_dwordx4 %0, off\n\ts_mov_b64 exec, -1" ::"v"(from), "s"(dst), "s"(left) : "memory", "scc");
+}
+__device__ __forceinline__ void lds_copy4(unsigned dst, const void* from) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(from), "s"(dst) : "memory");
+}
+// two neighbouring words through the scalar path: the wave's requests in flight are not waited for
+__device__ __forceinline__ int2 scalar_pair(const int32_t* p) {
+    unsigned long long v;
+    asm volatile("s_load_dwordx2 %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(v) : "s"(p) : "memory");
+    return make_int2((int)v, (int)(v >> 32));
+}
+__device__ __forceinline__ int scalar_word(const int32_t* p) {
+    int v;
+    asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)" : "=s"(v) : "s"(p) : "memory");
+    return v;
+}
+template <int N>
+__device__ __forceinline__ void wait_copies() {     // all but the wave's N youngest, and every read of LDS
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ void step_barrier() {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
 }
 
 struct GroupedArgs {
@@ -63,42 +102,90 @@ struct GroupedTile {
     int e, n0, first, ns;            // expert, first weight row, first sorted slot, slots
 };
 
-template <int ACT, bool LISTED, int NTS>
-__device__ __forceinline__ void grouped_store(const GroupedArgs& a, const GroupedTile& t, int n_wave, int s_wave, int lane, const v4f (&acc)[4][NTS]) {
-    const int col = lane & 15, g4 = lane >> 4;
+// v[0 .. 3] of one slot's neighbouring rows -> what is stored of them: two words, for gated units the lower one
+template <int ACT>
+__device__ __forceinline__ v2u grouped_result(v4f v, float limit) {
+    if (ACT == 2) {
+        float u0, u1;
+        if (limit > 0.f) {                                          // clamped units: g sigmoid(1.702 g) (u + 1) (uniform over the launch)
+            const float ga = fminf(v[0], limit), gb = fminf(v[2], limit);
+            u0 = ga / (1.0f + expf(-1.702f * ga)) * (fminf(fmaxf(v[1], -limit), limit) + 1.0f);
+            u1 = gb / (1.0f + expf(-1.702f * gb)) * (fminf(fmaxf(v[3], -limit), limit) + 1.0f);
+        } else {
+            u0 = v[0] / (1.0f + expf(-v[0])) * v[1];
+            u1 = v[2] / (1.0f + expf(-v[2])) * v[3];
+        }
+        return v2u{pack_bf2(u0, u1), 0u};
+    }
+    if (ACT == 1) {
 #pragma unroll
-    for (int nt = 0; nt < NTS; ++nt) {
-        const int sl = s_wave + 16 * nt + col;
-        if (sl >= t.ns) continue;
-        float iw = 1.0f;                                            // the expert works on iw * input
-        if (a.in_weight) iw = a.in_weight[LISTED ? (a.x_index ? a.x_index[t.first + sl] : t.first + sl) : (a.order ? a.order[t.first + sl] : t.first + sl)];
+        for (int r = 0; r < 4; ++r) {
+            const float x = fmaxf(v[r], 0.f);
+            v[r] = x * x;
+        }
+    }
+    return v2u{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+}
+// A quarter of a tile: 16 mt + .. of the 64 rows from n0 on, 16 nt + .. of the slots from sl0 on.  The wide form (N a multiple of 16): the four lanes of
+// a slot exchange what they have, so that each ends up with 16 neighbouring rows; returns how many stores the wave has issued.
+__device__ __forceinline__ void swap_rows32(unsigned& a, unsigned& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0], b = r[1];
+}
+__device__ __forceinline__ void swap_rows16(unsigned& a, unsigned& b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0], b = r[1];
+}
+__device__ __forceinline__ void store16(void* to, v4u v, unsigned long long lanes) {
+    asm volatile("s_mov_b64 exec, %2\n\tglobal_store_dwordx4 %0, %1, off\n\ts_mov_b64 exec, -1\n\ts_nop 0" ::"v"(to), "v"(v), "s"(lanes) : "memory");
+}
+template <int ACT, int NT>
+__device__ __forceinline__ int grouped_store_wide(const GroupedArgs& a, const GroupedTile& t, int n0, int sl0, int lane, const float (&iw)[NT], const v4f (&acc)[4][NT]) {
+    constexpr int W = ACT == 2 ? 1 : 2;
+    const int n = n0 + 16 * (lane >> 4);
+    int issued = 0;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        const int sl = sl0 + 16 * nt + (lane & 15);
+        unsigned d[4][2];
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt) {
-            const int n = t.n0 + n_wave + 16 * mt + 4 * g4;
-            if (n >= a.N) continue;                                 // N % 4 == 0: the four rows are inside together
-            v4f v = acc[mt][nt] * iw;
-            if (ACT == 2) {
-                float u0, u1;
-                if (a.limit > 0.f) {                                // clamped units: g sigmoid(1.702 g) (u + 1) (uniform over the launch)
-                    const float ga = fminf(v[0], a.limit), gb = fminf(v[2], a.limit);
-                    u0 = ga / (1.0f + expf(-1.702f * ga)) * (fminf(fmaxf(v[1], -a.limit), a.limit) + 1.0f);
-                    u1 = gb / (1.0f + expf(-1.702f * gb)) * (fminf(fmaxf(v[3], -a.limit), a.limit) + 1.0f);
-                } else {
-                    u0 = v[0] / (1.0f + expf(-v[0])) * v[1];
-                    u1 = v[2] / (1.0f + expf(-v[2])) * v[3];
-                }
-                *(unsigned*)(a.out + (size_t)(t.first + sl) * (a.N / 2) + n / 2) = pack_bf2(u0, u1);
-                continue;
-            }
-            if (ACT == 1) {
+            const v2u r = grouped_result<ACT>(acc[mt][nt] * iw[nt], a.limit);
+            d[mt][0] = r[0], d[mt][1] = r[1];
+        }
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float x = fmaxf(v[r], 0.f);
-                    v[r] = x * x;
-                }
+        for (int x = 0; x < W; ++x) {                               // d[mt] of lanes 16 g + .. <-> d[g] of lanes 16 mt + ..
+            swap_rows32(d[0][x], d[2][x]), swap_rows32(d[1][x], d[3][x]);
+            swap_rows16(d[0][x], d[1][x]), swap_rows16(d[2][x], d[3][x]);
+        }
+        const unsigned long long lanes = __ballot(sl < t.ns && n < a.N);
+        bf16_t* to = a.out + (ACT == 2 ? ((size_t)(t.first + sl) * a.N + n) / 2 : (size_t)(t.first + sl) * a.N + n);
+        if (lanes) {
+            if (ACT == 2) {
+                store16(to, v4u{d[0][0], d[1][0], d[2][0], d[3][0]}, lanes);
+            } else {
+                store16(to, v4u{d[0][0], d[0][1], d[1][0], d[1][1]}, lanes);
+                store16(to + 8, v4u{d[2][0], d[2][1], d[3][0], d[3][1]}, lanes);
             }
-            const v2u pk = {pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
-            *(v2u*)(a.out + (size_t)(t.first + sl) * a.N + n) = pk;
+            issued += W;
+        }
+    }
+    return issued;
+}
+template <int ACT, int NT>
+__device__ __forceinline__ void grouped_store(const GroupedArgs& a, const GroupedTile& t, int n0, int sl0, int lane, const float (&iw)[NT], const v4f (&acc)[4][NT]) {
+    const int col = lane & 15, g4 = lane >> 4;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        const int sl = sl0 + 16 * nt + col;
+        if (sl >= t.ns) continue;
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) {
+            const int n = n0 + 16 * mt + 4 * g4;
+            if (n >= a.N) continue;                                 // N % 4 == 0: the four rows are inside together
+            const v2u r = grouped_result<ACT>(acc[mt][nt] * iw[nt], a.limit);
+            if (ACT == 2) *(unsigned*)(a.out + ((size_t)(t.first + sl) * a.N + n) / 2) = r[0];
+            else *(v2u*)(a.out + (size_t)(t.first + sl) * a.N + n) = r;
         }
     }
 }
@@ -106,7 +193,8 @@ __device__ __forceinline__ void grouped_store(const GroupedArgs& a, const Groupe
 template <int ACT, bool LISTED>
 __global__ __launch_bounds__(PT, 2) void grouped_gemm_persistent_kernel(GroupedArgs a) {
     __shared__ __attribute__((aligned(128))) unsigned char buf[2 * PBUF];
-    __shared__ int tiles_before[MAX_GROUPS + 1];                    // slot tiles of the experts before e
+    __shared__ int side[SIDE];                                      // slot tiles of the experts before e | from AHEAD on the next tile's input rows
+    static_assert(MAX_GROUPS < SIDE, "");
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     if (!LISTED && w == 0) {
         int carry = 0;
@@ -118,13 +206,13 @@ __global__ __launch_bounds__(PT, 2) void grouped_gemm_persistent_kernel(GroupedA
                 const int y = __shfl_up(x, o, 64);
                 if (lane >= o) x += y;
             }
-            if (e < a.E) tiles_before[e + 1] = carry + x;
+            if (e < a.E) side[e + 1] = carry + x;
             carry += __shfl(x, 63, 64);
         }
-        if (lane == 0) tiles_before[0] = 0;
+        if (lane == 0) side[0] = 0;
     }
     __syncthreads();
-    const int row_tiles = (a.N + PR - 1) / PR, total = (LISTED ? a.n_tiles : __builtin_amdgcn_readfirstlane(tiles_before[a.E])) * row_tiles;
+    const int row_tiles = (a.N + PR - 1) / PR, total = (LISTED ? a.n_tiles : __builtin_amdgcn_readfirstlane(side[a.E])) * row_tiles;
     // An XCD's share of the tiles: whole rounds of its workgroups, then what is left - fewer tiles than workgroups - cut by slots into as many
     // parts (two or four) as there are workgroups for.  Place p: tile (p) of the share, or a part of one.
     const int xcd = blockIdx.x & 7, per_xcd = gridDim.x >> 3, chunk = (total + 7) >> 3;
@@ -134,135 +222,249 @@ __global__ __launch_bounds__(PT, 2) void grouped_gemm_persistent_kernel(GroupedA
     int at = blockIdx.x >> 3;
     if (at >= last) return;
 
-    auto tile_at = [&](int place) __attribute__((always_inline)) {
+    auto tile_at = [&](int place, int from) __attribute__((always_inline)) {   // from: the expert of an earlier place
         const int over = place - whole, part = over >= 0 ? over & ((1 << cut) - 1) : 0, size = over >= 0 ? PS >> cut : PS;
-        const int L = begin + (over >= 0 ? whole + (over >> cut) : place), s = L / row_tiles;   // which slot tile
+        const int L = begin + (over >= 0 ? whole + (over >> cut) : place);
         GroupedTile t;
-        t.n0 = (L % row_tiles) * PR;
         if (LISTED) {
-            t.e = __builtin_amdgcn_readfirstlane(a.tiles[3 * s]);
-            t.first = __builtin_amdgcn_readfirstlane(a.tiles[3 * s + 1]);
-            t.ns = __builtin_amdgcn_readfirstlane(min(max(a.tiles[3 * s + 2], 0), LISTED_SLOTS));
+            const int s = __builtin_amdgcn_readfirstlane(L / row_tiles);       // which slot tile
+            t.n0 = (L - s * row_tiles) * PR;
+            const int2 ef = scalar_pair(a.tiles + 3 * (size_t)s);
+            t.e = ef.x;
+            t.first = ef.y;
+            t.ns = min(max(scalar_word(a.tiles + 3 * (size_t)s + 2), 0), LISTED_SLOTS);
             return t;
         }
-        int lo = 0, hi = a.E;                                       // tiles_before[lo] <= s < tiles_before[hi]
-        while (hi - lo > 1) {
-            const int m = (lo + hi) >> 1;
-            if (__builtin_amdgcn_readfirstlane(tiles_before[m]) <= s) lo = m;
-            else hi = m;
+        int e = from & ~63;                                         // side[e] row_tiles <= L < side[e + 1] row_tiles, 64 experts at a time
+        for (;;) {
+            const int before = __popcll(__ballot(e + lane < a.E && side[min(e + lane, a.E - 1) + 1] * row_tiles <= L));
+            e += before;
+            if (before < 64) break;
         }
-        const int skip = __builtin_amdgcn_readfirstlane(tiles_before[lo]), first = a.offsets[lo] + (s - skip) * PS + part * size;
-        t.e = lo;
-        t.first = __builtin_amdgcn_readfirstlane(first);
-        t.ns = __builtin_amdgcn_readfirstlane(min(size, a.offsets[lo + 1] - first));   // (none or less: a part behind the expert's last slot)
+        e = __builtin_amdgcn_readfirstlane(e);
+        const int skip = __builtin_amdgcn_readfirstlane(side[e]), slots = __builtin_amdgcn_readfirstlane(side[e + 1]) - skip;
+        const int2 off = scalar_pair(a.offsets + e);
+        const int l = L - skip * row_tiles, band = l / (BAND * slots), high = min(BAND, row_tiles - BAND * band), in = l - band * BAND * slots;
+        const int s = __builtin_amdgcn_readfirstlane(in / high);
+        t.e = e;
+        t.n0 = __builtin_amdgcn_readfirstlane((BAND * band + in - s * high) * PR);
+        t.first = __builtin_amdgcn_readfirstlane(off.x + s * PS + part * size);
+        t.ns = __builtin_amdgcn_readfirstlane(min(size, off.y - t.first));   // (none or less: a part behind the expert's last slot)
         return t;
     };
-    // copies: wave w brings rows 32 w .. 32 w + 31 of the weights and of the inputs, eight rows (of 128 bytes) per instruction
-    const int piece = ((lane & 7) ^ (lane >> 3)) * 16;
-    auto x_slot = [&](const GroupedTile& t, int j) __attribute__((always_inline)) {
+    // Copies: of an operand half wave w brings rows 16 w .. 16 w + 15, eight (of 128 bytes) per instruction.  Request (h, j): half h, j of 2.
+    auto x_row = [&](const GroupedTile& t, int r) __attribute__((always_inline)) { return t.first + min(r, max(t.ns, 1) - 1); };
+    // (the lane's number is taken anew where a tile ends, so that nothing made of it is kept through the steps)
+    auto fresh_lane = [&]() __attribute__((always_inline)) {
+        int l = threadIdx.x & 63;
+        asm volatile("" : "+v"(l));
+        return l;
+    };
+    auto x_slot = [&](const GroupedTile& t, int h, int j, int lane) __attribute__((always_inline)) {
         if (LISTED && t.ns <= 0) return 0;                          // (an empty tile of the list: nothing is read or stored)
-        const int s = t.first + min(32 * w + 8 * j + (lane >> 3), t.ns - 1);
+        const int s = x_row(t, 128 * h + 16 * w + 8 * j + (lane >> 3));
         if (LISTED) return a.x_index ? (int)a.x_index[s] : s;
         return a.order ? a.order[s] : s;
     };
-    const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(lds_ptr)buf) + (unsigned)w * 4096u;
-    GroupedTile t = tile_at(at);
-    if (!LISTED && t.ns <= 0) return;                                        // (parts are the last places: nothing follows)
-    const bf16_t* W0 = a.W + ((size_t)t.e * a.N + t.n0) * (size_t)a.K;
+    const bool indexed = LISTED ? a.x_index != nullptr : a.order != nullptr;
+    const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(lds_ptr)buf) + (unsigned)w * 2048u;
+    const unsigned ahead0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(lds_ptr)side) + (unsigned)(AHEAD + 64 * w) * 4u;
+    const int steps = a.K / KS, V = max(steps, 2);                  // (one step: a second one that copies and multiplies nothing)
+    // the next tile's input rows come through LDS where there is room and time for it: nothing that is in flight is waited for
+    const bool early = V >= 6 && indexed && (LISTED || a.E < AHEAD);
+    GroupedTile t = tile_at(at, 0);
+    if (!LISTED && t.ns <= 0) return;                               // (parts are the last places: nothing follows)
+    const bf16_t* W0;
     unsigned woff[4];
     const unsigned char* xrow[4];
-    int rows_here = 0;                                              // inputs of the tile that is being copied, from this wave's first on
-    auto point = [&](const GroupedTile& g, const int (&slot)[4]) __attribute__((always_inline)) {
+    int rows_here, steps_here;                                      // of the tile that is being copied: inputs from this wave's first on, steps (none: 0)
+    auto point = [&](const GroupedTile& g, bool more, bool staged) __attribute__((always_inline)) {
+        steps_here = __builtin_amdgcn_readfirstlane(more ? steps : 0);
+        if (!more) return;                                          // (the requests that only count go to the last tile's addresses)
+        const int lane = fresh_lane(), piece = ((lane & 7) ^ (lane >> 3)) * 16;
         W0 = a.W + ((size_t)g.e * a.N + g.n0) * (size_t)a.K;
-        rows_here = g.ns - 32 * w;
+        rows_here = __builtin_amdgcn_readfirstlane(g.ns - 16 * w);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            woff[j] = (unsigned)min(32 * w + 8 * j + (lane >> 3), a.N - 1 - g.n0) * (unsigned)a.K * 2u + piece;
-            xrow[j] = (const unsigned char*)(a.X + (size_t)(slot[j] / a.div) * (size_t)a.K) + piece;
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                woff[2 * h + j] = (unsigned)min(128 * h + 16 * w + 8 * j + (lane >> 3), a.N - 1 - g.n0) * (unsigned)a.K * 2u + piece;
+                const int slot = staged ? side[AHEAD + 64 * w + 16 * h + 8 * j + (lane >> 3)] : x_slot(g, h, j, lane);
+                xrow[2 * h + j] = (const unsigned char*)(a.X + (size_t)(a.div == 1 ? slot : slot / a.div) * (size_t)a.K) + piece;
+                if (LISTED && g.ns <= 0) xrow[2 * h + j] = (const unsigned char*)W0 + woff[2 * h + j];   // (no input need exist)
+            }
+    };
+    auto copy_w = [&](int h, unsigned to, int step) __attribute__((always_inline)) {
+        const int k0 = step < steps ? step * KS : 0;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) lds_copy16(lds0 + to + h * HALF + 1024 * j, W0 + k0, woff[2 * h + j], step - steps_here);
+    };
+    auto copy_x = [&](int h, unsigned to, int step) __attribute__((always_inline)) {
+        const int k0 = step < steps ? step * KS : 0;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int left = (step - steps_here) & (128 * h + 8 * j - rows_here);
+            lds_copy16(lds0 + to + (2 + h) * HALF + 1024 * j, xrow[2 * h + j] + (size_t)k0 * 2, left);
         }
     };
-    auto copy = [&](int j, int which, int k0) __attribute__((always_inline)) {   // one of the wave's eight copies of a step
-        if (j < 4) lds_copy16(lds0 + which * PBUF + 1024 * j, W0 + k0, woff[j]);
-        else if (8 * (j - 4) < rows_here) lds_copy16(lds0 + which * PBUF + PR * 128 + 1024 * (j - 4), xrow[j - 4] + (size_t)k0 * 2);
-    };
-    {
-        int slot[4];
+    point(t, true, false);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) slot[j] = x_slot(t, j);
-        point(t, slot);
+    for (int i = 0; i < 8; ++i) {                              // (in the order of the phases that read them)
+        const int to = i / 4 * PBUF;
+        if (i % 4 == 0) copy_x(0, to, i / 4);
+        if (i % 4 == 1) copy_w(0, to, i / 4);
+        if (i % 4 == 2) copy_x(1, to, i / 4);
+        if (i % 4 == 3) copy_w(1, to, i / 4);
     }
-#pragma unroll
-    for (int j = 0; j < 8; ++j) copy(j, 0, 0);
-    const int col = lane & 15, g4 = lane >> 4, wr = w & 3, ws = w >> 2;
-    const int steps = a.K / KS;
-    int which = 0;
+    wait_copies<6>();                 // (as in front of every tile's epilogue)
+    const int col = lane & 15, g4 = lane >> 4, group = w >> 2, q = w & 3;
+    const bool wide = a.N % 16 == 0;
+    int stored = 0;                                                 // stores behind the last tile, at least
+    unsigned which = 0;                                             // the half of buf that holds the step
+    const int p0 = (g4 ^ (col & 7)) << 4, p1 = ((4 + g4) ^ (col & 7)) << 4;
 
-    auto run_tile = [&](auto nts) __attribute__((always_inline)) {
-        constexpr int NTS = decltype(nts)::value;
+    auto run_tile = [&](auto na_, auto nb_, auto nt_) __attribute__((always_inline)) {
+        constexpr int NA = decltype(na_)::value, NB = decltype(nb_)::value, NT = decltype(nt_)::value;   // row halves, slot halves, slots / 16 of a wave
         const int next = at + per_xcd;
-        const GroupedTile u = next < last ? tile_at(next) : t;
-        const bool more = next < last && (LISTED || u.ns > 0);
-        int slot[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) slot[j] = x_slot(more ? u : t, j);
-        v4f acc[4][NTS];
-#pragma unroll
-        for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-            for (int nt = 0; nt < NTS; ++nt) acc[mt][nt] = v4f{0.f, 0.f, 0.f, 0.f};
-        const int s_wave = ws * 16 * NTS;
-        for (int i = 0; i < steps; ++i) {
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            __builtin_amdgcn_s_barrier();                           // this step has landed; the other half has been read by everyone
-            asm volatile("" ::: "memory");
-            const unsigned char* A = buf + which * PBUF + (64 * wr + col) * 128;
-            const unsigned char* B = buf + which * PBUF + (PR + s_wave + col) * 128;
-            const int p0 = (g4 ^ (col & 7)) << 4, p1 = ((4 + g4) ^ (col & 7)) << 4;
-            int k_next = (i + 1) * KS;
-            bool bring = true;
-            if (i + 1 == steps) {                                   // the next tile's first step
-                k_next = 0;
-                bring = more;
-                if (more) point(u, slot);
+        GroupedTile u = t;
+        bool more = false;
+        auto look = [&]() __attribute__((always_inline)) {
+            if (next < last) {
+                u = tile_at(next, t.e);
+                more = LISTED || u.ns > 0;
             }
-            which ^= 1;
-            // 2 NTS groups of four products; group g's inputs are requested three groups ahead, the weights' second half and the copies
-            // of the next step in between (the order is the source's: left alone, the compiler reads each operand just before its use)
-            v4u av[2][4], bv[4];
-            auto read_b = [&](int g) __attribute__((always_inline)) { bv[g & 3] = *(const v4u*)(B + 2048 * (g % NTS) + (g < NTS ? p0 : p1)); };
+        };
+        if (!early) look();
+        v4f acc[NA][NB][4][NT];
 #pragma unroll
-            for (int mt = 0; mt < 4; ++mt) av[0][mt] = *(const v4u*)(A + 2048 * mt + p0);
-            read_b(0), read_b(1), read_b(2);
-            __builtin_amdgcn_sched_barrier(0);
+        for (int i = 0; i < NA * NB * 4 * NT; ++i) (&acc[0][0][0][0])[i] = v4f{0.f, 0.f, 0.f, 0.f};
+        const unsigned char* A = buf + (64 * group + col) * 128;
+        const unsigned char* B = buf + 2 * HALF + (16 * NT * q + col) * 128;
+        v4u av[2][4], b0[2][NT], b1[2][NT];
+        auto read_a = [&](int h) __attribute__((always_inline)) {
 #pragma unroll
-            for (int g = 0; g < 2 * NTS; ++g) {
-                if (g + 3 < 2 * NTS) read_b(g + 3);
-#pragma unroll
-                for (int mt = 0; mt < 4; ++mt)
-                    if (mt * NTS / 4 == g) av[1][mt] = *(const v4u*)(A + 2048 * mt + p1);
-                if (bring) {
-#pragma unroll
-                    for (int j = 0; j < 8; ++j)
-                        if (j * (NTS < 4 ? 2 * NTS : 8) / 8 == g) copy(j, which, k_next);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int mt = 0; mt < 4; ++mt)
-                    acc[mt][g % NTS] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, av[g / NTS][mt]), __builtin_bit_cast(bf8, bv[g & 3]),
-                                                                               acc[mt][g % NTS], 0, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);
+            for (int mt = 0; mt < 4; ++mt) {
+                av[0][mt] = *(const v4u*)(A + which + h * HALF + 2048 * mt + p0);
+                av[1][mt] = *(const v4u*)(A + which + h * HALF + 2048 * mt + p1);
             }
+        };
+        auto read_b = [&](v4u(&b)[2][NT], unsigned from, int h) __attribute__((always_inline)) {
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                b[0][nt] = *(const v4u*)(B + from + h * HALF + 2048 * nt + p0);
+                b[1][nt] = *(const v4u*)(B + from + h * HALF + 2048 * nt + p1);
+            }
+        };
+        auto multiply = [&](v4f(&c)[4][NT], const v4u(&b)[2][NT]) __attribute__((always_inline)) {
+            __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                    for (int mt = 0; mt < 4; ++mt)
+                        c[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, av[ks][mt]), __builtin_bit_cast(bf8, b[ks][nt]), c[mt][nt], 0, 0, 0);
+            __builtin_amdgcn_s_setprio(0);
+        };
+        // One K step.  Phase by phase: read, request, wait (12 requests are younger than what the next phase reads), barrier, multiply, barrier.  c holds the
+        // step's first slot half on entry; the next step's goes to d, whose second half is used up by then.
+        auto settle = [&](int i, auto p_) __attribute__((always_inline)) {
+            constexpr int p = decltype(p_)::value;
+            if (p < 3 && i == 0) wait_copies<63>();
+            else if ((p == 3 ? i == 0 : p < 2 && i == 1) && stored) {     // requested before the last tile's stores: these may be under way still
+                if (stored >= 16) wait_copies<12 + 16>();
+                else if (stored >= 8) wait_copies<12 + 8>();
+                else if (stored >= 4) wait_copies<12 + 4>();
+                else wait_copies<12>();
+            } else wait_copies<12>();
+            step_barrier();
+        };
+        typedef std::integral_constant<int, 0> P0;
+        typedef std::integral_constant<int, 1> P1;
+        typedef std::integral_constant<int, 2> P2;
+        typedef std::integral_constant<int, 3> P3;
+        auto step = [&](int i, v4u(&c)[2][NT], v4u(&d)[2][NT]) __attribute__((always_inline)) {
+            const bool live = V == steps || i < steps;
+            const int k = i + 2 < V ? i + 2 : i + 2 - V;
+            read_a(0);
+            if (i == V - 2) point(u, more, early);
+            copy_x(0, which, k);
+            settle(i, P0());
+            if (live) multiply(acc[0][0], c);
+            step_barrier();
+
+            if (NB == 2) read_b(d, which, 1);
+            copy_w(0, which, k);
+            settle(i, P1());
+            if (NB == 2 && live) multiply(acc[0][NB - 1], d);
+            step_barrier();
+
+            if (NA == 2) read_a(1);
+            copy_x(1, which, k);
+            settle(i, P2());
+            if (NA == 2 && NB == 2 && live) multiply(acc[NA - 1][NB - 1], d);
+            step_barrier();
+
+            if (i + 1 < V) read_b(d, which ^ PBUF, 0);
+            copy_w(1, which, k);
+            if (early && i == 0) look();
+            if (early && i == 1 && more && u.ns > 0) {
+                const int lane = fresh_lane();
+                const int s = x_row(u, 128 * ((lane >> 4) & 1) + 16 * w + (lane & 15));
+                lds_copy4(ahead0, LISTED ? (const void*)(a.x_index + s) : (const void*)(a.order + s));
+            }
+            settle(i, P3());
+            if (NA == 2 && live) multiply(acc[NA - 1][0], c);
+            step_barrier();
+            which ^= PBUF;
+        };
+        step_barrier();                                             // every wave's requests for the first phases have landed
+        read_b(b0, which, 0);
+        wait_copies<63>();
+        step_barrier();
+        if (group) step_barrier();
+        int i = 0;
+        for (; i + 1 < V; i += 2) {
+            step(i, b0, b1);
+            step(i + 1, b1, b0);
         }
-        grouped_store<ACT, LISTED, NTS>(a, t, 64 * wr, s_wave, lane, acc);
+        if (i < V) step(i, b0, b1);
+        if (!group) step_barrier();
+        // (what the next tile's first step reads, and the first slot half of its second; the stores below are younger)
+        wait_copies<6>();
+        const int lane = fresh_lane(), col = lane & 15;
+        const int n0 = t.n0 + 64 * group, sl0 = 16 * NT * q;
+        stored = 0;
+        float iw[NB][NT];                                           // the expert works on iw * input
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                iw[b][nt] = 1.0f;
+                const int sl = 128 * b + sl0 + 16 * nt + col;
+                if (a.in_weight && sl < t.ns) {
+                    const int s = t.first + sl;
+                    iw[b][nt] = a.in_weight[LISTED ? (a.x_index ? a.x_index[s] : s) : (a.order ? a.order[s] : s)];
+                }
+            }
+#pragma unroll
+        for (int h = 0; h < NA; ++h)
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                if (wide) stored += grouped_store_wide<ACT, NT>(a, t, n0 + 128 * h, 128 * b + sl0, lane, iw[b], acc[h][b]);
+                else grouped_store<ACT, NT>(a, t, n0 + 128 * h, 128 * b + sl0, lane, iw[b], acc[h][b]);
+            }
         asm volatile("" ::: "memory");                              // (the stores' branches join here: what follows stays uniform)
         if (more) t = u;
         at = next;
         return more;
     };
+    typedef std::integral_constant<int, 1> One;
+    typedef std::integral_constant<int, 2> Two;
     for (;;) {
-        const bool more = t.ns > PS / 2   ? run_tile(std::integral_constant<int, 8>())
-                          : t.ns > PS / 4 ? run_tile(std::integral_constant<int, 4>())
-                                          : run_tile(std::integral_constant<int, 2>());
+        bool more;
+        if (t.n0 + PR / 2 < a.N) more = t.ns > PS / 2 ? run_tile(Two(), Two(), Two()) : t.ns > PS / 4 ? run_tile(Two(), One(), Two()) : run_tile(Two(), One(), One());
+        else more = t.ns > PS / 2 ? run_tile(One(), Two(), Two()) : t.ns > PS / 4 ? run_tile(One(), One(), Two()) : run_tile(One(), One(), One());
         if (!more) break;
     }
 }

@@ -104,6 +104,37 @@ def test_grouped_form(ops, T, top, E, ident, D, ff, crowd, act, weigh):
     check(o, T, top, E, ident, D, ff, act, weigh, crowd)
 
 
+# one step; runs of steps around the two that are requested ahead and the six from which a tile's rows come through LDS; rows in and out of 16; empty, full
+# and nearly empty tiles; the gather through slot / div and rows as they lie; experts on both sides of the room for staged rows
+@pytest.mark.parametrize("K", [64, 128, 192, 320, 384, 448])
+@pytest.mark.parametrize("N, E, div", [(4, 14, 1), (132, 14, 3), (260, 14, 0), (528, 14, 2), (128, 7679, 1), (272, 7680, 1)])
+def test_grouped_products_of_sorted_runs(ops, K, N, E, div):
+    g, dev = torch.Generator().manual_seed(K + N), "cuda:0"
+    counts = torch.tensor([0, 1, 63, 64, 65, 0, 127, 128, 129, 255, 256, 257, 600, 0])
+    counts = torch.cat([counts[:7], counts.new_zeros(E - 14), counts[7:]])
+    n = int(counts.sum())
+    off = torch.cat([counts.new_zeros(1), counts.cumsum(0)]).int()
+    order = torch.randperm(n, generator=g).int() if div else torch.arange(n, dtype=torch.int32)
+    x, w14 = torch.randn(-(-n // max(div, 1)), K, generator=g).bfloat16(), (torch.randn(14, N, K, generator=g) / K ** 0.5).bfloat16()
+    w = torch.empty(E, N, K, dtype=torch.bfloat16, device=dev)          # (empty experts' weights are never read)
+    w[:7], w[-7:] = w14[:7].to(dev), w14[7:].to(dev)
+    xd, od, offd = x.to(dev), order.to(dev), off.to(dev)
+    out = torch.full((n + 1, N), 3.0, dtype=torch.bfloat16, device=dev)
+    for _ in range(2):                                                  # (a second launch finds what the first one left in LDS)
+        ops.check(ops.L.qsv_grouped_gemm_sorted(out.data_ptr(), xd.data_ptr(), od.data_ptr() if div else None, max(div, 1), w.data_ptr(), offd.data_ptr(),
+                                                E, N, K, 0, 0.0, None, torch.cuda.current_stream().cuda_stream), "grouped")
+    y, rows = out.cpu(), x.double()[order.long() // max(div, 1)]
+    at = 0
+    for e in range(E):
+        c = int(counts[e])
+        if c:
+            ref = rows[at:at + c] @ w14[e if e < 7 else e - (E - 14)].double().T
+            # half a unit in the last of bfloat16's 8 digits; float sums of K products of order K^-1/2
+            assert ((y[at:at + c].double() - ref).abs() <= 2.0 ** -8 * ref.abs() + K * 2.0 ** -22).all(), (e, c)
+        at += c
+    assert (y[n] == 3.0).all()
+
+
 @pytest.mark.parametrize("E", [1025, 1600, 8064])
 def test_grouped_form_of_many_experts(ops, E):
     check(ops, 600, 2, E, 3, 64, 64, "relu_sq", "input", 0.1)

@@ -50,6 +50,12 @@ int qsv_add_rms_norm(float* x, void* h, const void* a, const void* b, const void
 int qsv_scaled_sum_rms_norms(float* x, void* h0, void* h1, const void* a, const void* sa, const void* b, const void* sb, const void* c,
                              const void* sc, const float* g0, const float* g1, const int32_t* tokens, const void* table, float eps,
                              int n_tokens, int width, int dtype, void* stream);
+/* The same with the sum over a mixture's experts in it: x[t] += sa a[t] + slot_scale y[t] + sc c[t] (c may be NULL), y[t] = sum_k weight[t, k] ys[place ? place[t
+ * top_k + k] : t top_k + k], rounded to the storage type (ys: float_rows ? float : storage type rows of `width`; weight NULL: ones; slots whose idx names none of the n_experts
+ * add nothing).  width a multiple of 4, at most 4096. */
+int qsv_scaled_sum_rms_norms_slots(float* x, void* h0, void* h1, const void* a, const void* sa, const void* ys, int float_rows, const int32_t* place,
+                                   const float* weight, const int32_t* idx, int top_k, int n_experts, const void* slot_scale, const void* c,
+                                   const void* sc, const float* g0, const float* g1, float eps, int n_tokens, int width, int dtype, void* stream);
 /* Sublayers between two norms: x[t] += rms_norm(y[t]) * w_post (y == NULL: nothing added), then h[t] = rms_norm(x[t]) * w_next in
  * the storage type (h == NULL: the sum only).  A weight is one gain for all coordinates (its *_wide flag 0) or one per coordinate. */
 int qsv_add_normed_rms_norm(float* x, void* h, const void* y, const void* w_post, int post_wide, const void* w_next, int next_wide,
@@ -101,6 +107,9 @@ int qsv_normed_attention_prep(float* qf, void* pool, int64_t pool_rows, const vo
 /* x[t] += layer_norm(y[t]) * w (no bias; variance = mean of squared deviations); h[t] = x[t] in the storage type. */
 int qsv_add_layer_norm(float* x, void* h, const void* y, const void* w, float eps, int n_tokens, int width, int dtype,
                        void* stream);
+/* The same with y[t] the sum over a mixture's experts (see qsv_scaled_sum_rms_norms_slots; width a multiple of 4, at most 4096). */
+int qsv_add_layer_norm_slots(float* x, void* h, const void* ys, int float_rows, const int32_t* place, const float* weight, const int32_t* idx, int top_k,
+                             int n_experts, const void* w, float eps, int n_tokens, int width, int dtype, void* stream);
 
 /* out[r] = layer_norm(x[rows[r]]) * w in the storage type (rows == NULL: row r). */
 int qsv_layer_norm_rows(void* out, const float* x, const int32_t* rows, const void* w, float eps, int n_rows, int width,
@@ -298,6 +307,9 @@ int qsv_hc_read(void* h, const float* x, const float* w_in, const void* norm_w, 
  * sublayer's input from the new streams, h_next[t] = tanh(alpha * sum_r w_in_next[r] x[t, r]) * norm_w + norm_b (no token shift). */
 int qsv_hc_write(float* x, const void* y, const float* mix, const float* w_out, int n_tokens, int streams, int width, void* h_next,
                  const float* w_in_next, const void* norm_w, const void* norm_b, float alpha, int dtype, void* stream);
+/* The same (without h_next) with y[t] the sum over a mixture's experts (see qsv_scaled_sum_rms_norms_slots; width a multiple of 4). */
+int qsv_hc_write_slots(float* x, const void* ys, int float_rows, const int32_t* place, const float* weight, const int32_t* idx, int top_k, int n_experts,
+                       const float* mix, const float* w_out, int n_tokens, int streams, int width, int dtype, void* stream);
 /* out[r] = tanh(alpha * sum_s x[rows[r], s]) * norm_w + norm_b  (rows == NULL: row r). */
 int qsv_dyt_sum_rows(void* out, const float* x, const int32_t* rows, const void* norm_w, const void* norm_b, float alpha,
                      int n_rows, int streams, int width, int dtype, void* stream);

@@ -122,6 +122,58 @@ __device__ __forceinline__ unsigned token_of(unsigned block, int chunks) { retur
 // an address that 4 elements of its type may be read from at once
 inline bool fits4(const void* p, int dtype) { return (uintptr_t)p % (dtype == QSV_BF16 ? 8 : 16) == 0; }
 
+// What a mixture of experts leaves, a row per slot (t, k), to be summed by the kernel that uses it: y[t] = sum_k weight[t, k] ys[place ? place[t top + k] :
+// t top + k] (weight NULL: ones; slots whose index names none of the experts add nothing).
+struct SlotRows {
+    const void* ys;
+    const int32_t* place;
+    const float* weight;
+    const int32_t* idx;
+    int top, n_experts;
+};
+// a[p] = four columns of y[t] from c + p * step on, p < P (zeros behind D).  The rows of four slots are requested together.
+template <typename Y, int P>
+__device__ __forceinline__ void slot_sum4(const SlotRows& s, size_t t, int D, int c, int step, float (&a)[P][4]) {
+#pragma unroll
+    for (int p = 0; p < P; ++p) a[p][0] = a[p][1] = a[p][2] = a[p][3] = 0.f;
+    for (int k0 = 0; k0 < s.top; k0 += 4) {
+        float v[4][P][4], w[4];
+        bool none[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const size_t slot = t * s.top + min(k0 + q, s.top - 1);
+            none[q] = k0 + q >= s.top || (unsigned)s.idx[slot] >= (unsigned)s.n_experts;
+            w[q] = s.weight ? s.weight[slot] : 1.0f;
+            const size_t row = none[q] ? 0 : s.place ? (size_t)s.place[slot] : slot;      // (no slot's row, but a row)
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                v[q][p][0] = v[q][p][1] = v[q][p][2] = v[q][p][3] = 0.f;
+                if (c + p * step < D) ld4t((const Y*)s.ys, row * D + c + p * step, v[q][p]);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int p = 0; p < P; ++p)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float sum = a[p][j] + w[q] * v[q][p][j];
+                    a[p][j] = none[q] ? a[p][j] : sum;
+                }
+    }
+}
+
+// ... as a tensor of the storage type would hold it
+__device__ __forceinline__ float stored(const float*, float v) { return v; }
+__device__ __forceinline__ float stored(const bf16_t*, float v) { return bf2f(f2bf(v)); }
+template <typename T, int P>
+__device__ __forceinline__ void round_stored(float (&a)[P][4]) {
+#pragma unroll
+    for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) a[p][j] = stored((const T*)nullptr, a[p][j]);
+}
+
 // dtype dispatch of a templated launcher: F<bf16_t>() or F<float>()
 #define QSV_DISPATCH(dtype, what, CALL)                                  \
     do {                                                                 \

@@ -2,6 +2,8 @@
 // latent projections' norms + rotary + cache write, the latent query, the output gate.  Statistics and angles are float.
 #include "serve_common.h"
 
+#include <type_traits>
+
 static thread_local char g_err[512] = "";
 void qsv_set_error(const char* fmt, ...) {
     va_list ap;
@@ -61,10 +63,11 @@ __global__ __launch_bounds__(NT) void add_layer_norm_kernel(float* __restrict__ 
 }
 // The same, and the plain norm below, for rows of up to 1024 P elements, a multiple of four: one trip to memory - every operand is requested
 // before the first sum and stays in registers.  Bound by the row's latency in a step, by HBM in a prompt (64 / 8192 rows of 2048: 8.8 ->
-// 2.7 / 130 -> 33 us).
-template <typename T, int P, bool ADD>
+// 2.7 / 130 -> 33 us).  Y other than void: y is what a mixture of experts left per slot (float or the storage type), summed here and
+// rounded as a tensor would hold it.
+template <typename T, int P, bool ADD, typename Y = void>
 __global__ __launch_bounds__(NT) void layer_norm_vec_kernel(T* __restrict__ h, float* __restrict__ x, const T* __restrict__ y,
-                                                            const int32_t* __restrict__ rows, const T* __restrict__ w, float eps, int D) {
+                                                            const int32_t* __restrict__ rows, const T* __restrict__ w, float eps, int D, SlotRows slots) {
     __shared__ float red[NT / 64 + 1];
     const size_t t = blockIdx.x, from = ADD ? t : rows ? (size_t)rows[t] : t;
     float v[P][4], g[P][4], old[P][4];
@@ -73,10 +76,16 @@ __global__ __launch_bounds__(NT) void layer_norm_vec_kernel(T* __restrict__ h, f
         const int i = (k * NT + threadIdx.x) * 4;
         v[k][0] = v[k][1] = v[k][2] = v[k][3] = 0.f;
         if (i >= D) continue;
-        if (ADD) ld4t(y, t * D + i, v[k]);
-        else ld4t(x, from * D + i, v[k]);
+        if constexpr (std::is_void<Y>::value) {
+            if (ADD) ld4t(y, t * D + i, v[k]);
+            else ld4t(x, from * D + i, v[k]);
+        }
         ld4t(w, i, g[k]);
         if (ADD) ld4t(x, t * D + i, old[k]);
+    }
+    if constexpr (!std::is_void<Y>::value) {
+        slot_sum4<Y>(slots, t, D, threadIdx.x * 4, NT * 4, v);
+        round_stored<T>(v);
     }
     float s = 0.f;
 #pragma unroll
@@ -105,9 +114,16 @@ __global__ __launch_bounds__(NT) void layer_norm_vec_kernel(T* __restrict__ h, f
 }
 template <typename T, bool ADD>
 static void launch_layer_norm_vec(T* h, float* x, const T* y, const int32_t* rows, const T* w, float eps, int n, int D, hipStream_t stream) {
-    if (D <= NT * 4) hipLaunchKernelGGL((layer_norm_vec_kernel<T, 1, ADD>), dim3(n), dim3(NT), 0, stream, h, x, y, rows, w, eps, D);
-    else if (D <= NT * 8) hipLaunchKernelGGL((layer_norm_vec_kernel<T, 2, ADD>), dim3(n), dim3(NT), 0, stream, h, x, y, rows, w, eps, D);
-    else hipLaunchKernelGGL((layer_norm_vec_kernel<T, 4, ADD>), dim3(n), dim3(NT), 0, stream, h, x, y, rows, w, eps, D);
+    const SlotRows none = {};
+    if (D <= NT * 4) hipLaunchKernelGGL((layer_norm_vec_kernel<T, 1, ADD>), dim3(n), dim3(NT), 0, stream, h, x, y, rows, w, eps, D, none);
+    else if (D <= NT * 8) hipLaunchKernelGGL((layer_norm_vec_kernel<T, 2, ADD>), dim3(n), dim3(NT), 0, stream, h, x, y, rows, w, eps, D, none);
+    else hipLaunchKernelGGL((layer_norm_vec_kernel<T, 4, ADD>), dim3(n), dim3(NT), 0, stream, h, x, y, rows, w, eps, D, none);
+}
+template <typename T, typename Y>
+static void launch_layer_norm_slots(T* h, float* x, const T* w, float eps, int n, int D, const SlotRows& slots, hipStream_t stream) {
+    if (D <= NT * 4) hipLaunchKernelGGL((layer_norm_vec_kernel<T, 1, true, Y>), dim3(n), dim3(NT), 0, stream, h, x, (const T*)nullptr, nullptr, w, eps, D, slots);
+    else if (D <= NT * 8) hipLaunchKernelGGL((layer_norm_vec_kernel<T, 2, true, Y>), dim3(n), dim3(NT), 0, stream, h, x, (const T*)nullptr, nullptr, w, eps, D, slots);
+    else hipLaunchKernelGGL((layer_norm_vec_kernel<T, 4, true, Y>), dim3(n), dim3(NT), 0, stream, h, x, (const T*)nullptr, nullptr, w, eps, D, slots);
 }
 static bool layer_norm_fits(const void* x, const void* h, const void* y, const void* w, int D, int dtype) {
     return D % 4 == 0 && D <= NT * 16 && fits4(x, QSV_F32) && fits4(h, dtype) && fits4(y, dtype) && fits4(w, dtype);
@@ -125,6 +141,18 @@ extern "C" int qsv_add_layer_norm(float* x, void* h, const void* y, const void* 
                  hipLaunchKernelGGL(add_layer_norm_kernel<T>, dim3(n), dim3(NT), 0, (hipStream_t)stream, x, (T*)h, (const T*)y,
                                     (const T*)w, eps, D));
     return qsv_launch_status("qsv_add_layer_norm");
+}
+
+extern "C" int qsv_add_layer_norm_slots(float* x, void* h, const void* ys, int float_rows, const int32_t* place, const float* weight, const int32_t* idx, int top_k,
+                                        int n_experts, const void* w, float eps, int n, int D, int dtype, void* stream) {
+    QSV_REQUIRE(x && h && ys && idx && w && n >= 0 && D > 0 && top_k > 0 && n_experts > 0, "qsv_add_layer_norm_slots: bad arguments");
+    QSV_REQUIRE(layer_norm_fits(x, h, h, w, D, dtype) && fits4(ys, float_rows ? QSV_F32 : dtype), "qsv_add_layer_norm_slots: width %d (a multiple of 4, at most %d), rows on four elements",
+                D, NT * 16);
+    if (n == 0) return QSV_OK;
+    const SlotRows slots = {ys, place, weight, idx, top_k, n_experts};
+    if (float_rows) QSV_DISPATCH(dtype, "qsv_add_layer_norm_slots", (launch_layer_norm_slots<T, float>((T*)h, x, (const T*)w, eps, n, D, slots, (hipStream_t)stream)));
+    else QSV_DISPATCH(dtype, "qsv_add_layer_norm_slots", (launch_layer_norm_slots<T, T>((T*)h, x, (const T*)w, eps, n, D, slots, (hipStream_t)stream)));
+    return qsv_launch_status("qsv_add_layer_norm_slots");
 }
 
 template <typename T>
@@ -446,31 +474,60 @@ extern "C" int qsv_add_rms_norm(float* x, void* h, const void* a, const void* b,
 // embedding row.  a, b, c (storage type), their scales and h1 may be NULL; h0 == NULL: the sum only.
 struct ScaledParts {
     const void *y[3], *s[3];
+    const void* slot_scale;
 };
-template <typename T, int VPT>
+// One trip to memory: the NP parts (and, Y other than void, what a mixture of experts left per slot, summed and rounded here as a tensor would hold it,
+// scaled by slot_scale: added behind the first part) are requested before the first is used.
+template <typename T, int VPT, int NP, typename Y = void>
 __global__ __launch_bounds__(NT) void scaled_sum_rms_norms_vec_kernel(float* __restrict__ x, T* __restrict__ h0, T* __restrict__ h1, ScaledParts p,
                                                                       const float* __restrict__ g0, const float* __restrict__ g1,
-                                                                      const int32_t* __restrict__ tokens, const T* __restrict__ table, float eps, int D) {
+                                                                      const int32_t* __restrict__ tokens, const T* __restrict__ table, float eps, int D, SlotRows slots) {
+    constexpr bool SLOTS = !std::is_void<Y>::value;
     __shared__ float red[NT / 64 + 1];
     const size_t t = blockIdx.x;
-    float4 v[VPT];
+    float v[VPT][4], z[VPT][NP ? NP : 1][4], f[VPT][NP ? NP : 1][4], ysum[VPT][4], yf[VPT][4];
+#pragma unroll
+    for (int k = 0; k < VPT; ++k) {
+        const int i = (threadIdx.x + k * NT) * 4;
+        if (i >= D) continue;
+        if (tokens) ld4t(table, (size_t)tokens[t] * D + i, v[k]);
+        else ld4t(x, t * D + i, v[k]);
+#pragma unroll
+        for (int j = 0; j < NP; ++j) {
+            ld4t((const T*)p.y[j], t * D + i, z[k][j]);
+            f[k][j][0] = f[k][j][1] = f[k][j][2] = f[k][j][3] = 1.f;
+            if (p.s[j]) ld4t((const T*)p.s[j], i, f[k][j]);
+        }
+        if (SLOTS) {
+            yf[k][0] = yf[k][1] = yf[k][2] = yf[k][3] = 1.f;
+            if (p.slot_scale) ld4t((const T*)p.slot_scale, i, yf[k]);
+        }
+    }
+    if constexpr (SLOTS) {
+        slot_sum4<Y>(slots, t, D, threadIdx.x * 4, NT * 4, ysum);
+        round_stored<T>(ysum);
+    }
     float s = 0.f;
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
         const int i = (threadIdx.x + k * NT) * 4;
         if (i >= D) continue;
-        v[k] = tokens ? ld4v(table, (size_t)tokens[t] * D + i) : ld4v(x, t * D + i);
-        float4 y = make_float4(0.f, 0.f, 0.f, 0.f);
+        float y[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < 3; ++j)
-            if (p.y[j]) {
-                const float4 z = ld4v((const T*)p.y[j], t * D + i);
-                const float4 f = p.s[j] ? ld4v((const T*)p.s[j], i) : make_float4(1.f, 1.f, 1.f, 1.f);
-                y.x += f.x * z.x; y.y += f.y * z.y; y.z += f.z * z.z; y.w += f.w * z.w;
-            }
-        v[k].x += y.x; v[k].y += y.y; v[k].z += y.z; v[k].w += y.w;
-        st4v(x, t * D + i, v[k]);
-        s += v[k].x * v[k].x + v[k].y * v[k].y + v[k].z * v[k].z + v[k].w * v[k].w;
+        for (int j = 0; j < NP; ++j) {
+            if (SLOTS && j == 1)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) y[e] += yf[k][e] * ysum[k][e];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[e] += f[k][j][e] * z[k][j][e];
+        }
+        if (SLOTS && NP < 2)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[e] += yf[k][e] * ysum[k][e];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[k][e] += y[e];
+        st4t(x, t * D + i, v[k]);
+        s += v[k][0] * v[k][0] + v[k][1] * v[k][1] + v[k][2] * v[k][2] + v[k][3] * v[k][3];
     }
     if (!h0) return;
     const float inv = 1.0f / sqrtf(block_sum<NT>(s, red) / (float)D + eps);
@@ -478,12 +535,19 @@ __global__ __launch_bounds__(NT) void scaled_sum_rms_norms_vec_kernel(float* __r
     for (int k = 0; k < VPT; ++k) {
         const int i = (threadIdx.x + k * NT) * 4;
         if (i >= D) continue;
-        const float4 n = make_float4(v[k].x * inv, v[k].y * inv, v[k].z * inv, v[k].w * inv);
-        const float4 a = ld4v(g0, i);
-        st4v(h0, t * D + i, make_float4(n.x * a.x, n.y * a.y, n.z * a.z, n.w * a.w));
+        float a[4], n[4];
+        ld4t(g0, i, a);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[k][e] *= inv;
+            n[e] = v[k][e] * a[e];
+        }
+        st4t(h0, t * D + i, n);
         if (h1) {
-            const float4 b = ld4v(g1, i);
-            st4v(h1, t * D + i, make_float4(n.x * b.x, n.y * b.y, n.z * b.z, n.w * b.w));
+            ld4t(g1, i, a);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) n[e] = v[k][e] * a[e];
+            st4t(h1, t * D + i, n);
         }
     }
 }
@@ -511,29 +575,59 @@ __global__ __launch_bounds__(NT) void scaled_sum_rms_norms_kernel(float* __restr
         if (h1) st(h1, t * D + i, n * g1[i]);
     }
 }
+template <typename T, int NP, typename Y>
+static void launch_scaled_sum(float* x, T* h0, T* h1, const ScaledParts& p, const float* g0, const float* g1, const int32_t* tokens, const T* table, float eps, int n, int D,
+                              const SlotRows& slots, hipStream_t stream) {
+    const int vecs = (D / 4 + NT - 1) / NT;
+#define QSV_SSN(V) hipLaunchKernelGGL((scaled_sum_rms_norms_vec_kernel<T, V, NP, Y>), dim3(n), dim3(NT), 0, stream, x, h0, h1, p, g0, g1, tokens, table, eps, D, slots)
+    if (vecs <= 1) QSV_SSN(1);
+    else if (vecs <= 2) QSV_SSN(2);
+    else if (vecs <= 4) QSV_SSN(4);
+    else if constexpr (std::is_void<Y>::value) QSV_SSN(8);
+#undef QSV_SSN
+}
 extern "C" int qsv_scaled_sum_rms_norms(float* x, void* h0, void* h1, const void* a, const void* sa, const void* b, const void* sb, const void* c,
                                         const void* sc, const float* g0, const float* g1, const int32_t* tokens, const void* table, float eps,
                                         int n, int D, int dtype, void* stream) {
     QSV_REQUIRE(x && n >= 0 && D > 0 && (!h0 || g0) && (!h1 || (h0 && g1)) && (!tokens || table), "qsv_scaled_sum_rms_norms: bad arguments");
     if (n == 0) return QSV_OK;
-    const ScaledParts p = {{a, b, c}, {sa, sb, sc}};
-    const int vecs = (D / 4 + NT - 1) / NT;
-#define QSV_SSN(V)                                                                                                                 \
-    QSV_DISPATCH(dtype, "qsv_scaled_sum_rms_norms",                                                                                \
-                 hipLaunchKernelGGL((scaled_sum_rms_norms_vec_kernel<T, V>), dim3(n), dim3(NT), 0, (hipStream_t)stream, x, (T*)h0, (T*)h1, p, g0, \
-                                    g1, tokens, (const T*)table, eps, D))
-    if (D % 4 == 0 && vecs <= 8) {
-        if (vecs <= 1) QSV_SSN(1);
-        else if (vecs <= 2) QSV_SSN(2);
-        else if (vecs <= 4) QSV_SSN(4);
-        else QSV_SSN(8);
+    ScaledParts p = {{a, b, c}, {sa, sb, sc}, nullptr};
+    if (D % 4 == 0 && D <= NT * 32) {
+        int np = 0;                                                 // (the parts that there are, in their order)
+        for (int j = 0; j < 3; ++j)
+            if (p.y[j]) {
+                p.y[np] = p.y[j];
+                p.s[np++] = p.s[j];
+            }
+        if (np == 0) QSV_DISPATCH(dtype, "qsv_scaled_sum_rms_norms", (launch_scaled_sum<T, 0, void>(x, (T*)h0, (T*)h1, p, g0, g1, tokens, (const T*)table, eps, n, D, SlotRows{}, (hipStream_t)stream)));
+        else if (np == 1) QSV_DISPATCH(dtype, "qsv_scaled_sum_rms_norms", (launch_scaled_sum<T, 1, void>(x, (T*)h0, (T*)h1, p, g0, g1, tokens, (const T*)table, eps, n, D, SlotRows{}, (hipStream_t)stream)));
+        else if (np == 2) QSV_DISPATCH(dtype, "qsv_scaled_sum_rms_norms", (launch_scaled_sum<T, 2, void>(x, (T*)h0, (T*)h1, p, g0, g1, tokens, (const T*)table, eps, n, D, SlotRows{}, (hipStream_t)stream)));
+        else QSV_DISPATCH(dtype, "qsv_scaled_sum_rms_norms", (launch_scaled_sum<T, 3, void>(x, (T*)h0, (T*)h1, p, g0, g1, tokens, (const T*)table, eps, n, D, SlotRows{}, (hipStream_t)stream)));
     } else {
         QSV_DISPATCH(dtype, "qsv_scaled_sum_rms_norms",
                      hipLaunchKernelGGL(scaled_sum_rms_norms_kernel<T>, dim3(n), dim3(NT), 0, (hipStream_t)stream, x, (T*)h0, (T*)h1, p, g0, g1,
                                         tokens, (const T*)table, eps, D));
     }
-#undef QSV_SSN
     return qsv_launch_status("qsv_scaled_sum_rms_norms");
+}
+// x += sa * a + slot_scale * (the slots' sum) + sc * c (c NULL: none), then as above.
+extern "C" int qsv_scaled_sum_rms_norms_slots(float* x, void* h0, void* h1, const void* a, const void* sa, const void* ys, int float_rows, const int32_t* place,
+                                              const float* weight, const int32_t* idx, int top_k, int n_experts, const void* slot_scale, const void* c, const void* sc,
+                                              const float* g0, const float* g1, float eps, int n, int D, int dtype, void* stream) {
+    QSV_REQUIRE(x && a && ys && idx && n >= 0 && D > 0 && (!h0 || g0) && (!h1 || (h0 && g1)) && top_k > 0 && n_experts > 0, "qsv_scaled_sum_rms_norms_slots: bad arguments");
+    QSV_REQUIRE(D % 4 == 0 && D <= NT * 16 && fits4(ys, float_rows ? QSV_F32 : dtype), "qsv_scaled_sum_rms_norms_slots: width %d (a multiple of 4, at most %d), rows on four elements", D, NT * 16);
+    if (n == 0) return QSV_OK;
+    const ScaledParts p = {{a, c, nullptr}, {sa, sc, nullptr}, slot_scale};
+    const SlotRows slots = {ys, place, weight, idx, top_k, n_experts};
+#define QSV_SLOTS(NP, Y)                                                                                                                    \
+    QSV_DISPATCH(dtype, "qsv_scaled_sum_rms_norms_slots",                                                                                   \
+                 (launch_scaled_sum<T, NP, Y>(x, (T*)h0, (T*)h1, p, g0, g1, nullptr, (const T*)nullptr, eps, n, D, slots, (hipStream_t)stream)))
+    if (c && float_rows) QSV_SLOTS(2, float);
+    else if (c) QSV_SLOTS(2, T);
+    else if (float_rows) QSV_SLOTS(1, float);
+    else QSV_SLOTS(1, T);
+#undef QSV_SLOTS
+    return qsv_launch_status("qsv_scaled_sum_rms_norms_slots");
 }
 
 template <typename T, typename TW>

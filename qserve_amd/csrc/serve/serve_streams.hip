@@ -5,6 +5,8 @@
 // Streams, sums and norms are float; only what leaves for a matrix product is in the storage type.
 #include "serve_common.h"
 
+#include <type_traits>
+
 namespace {
 constexpr int NT = 256;
 constexpr int MAX_STREAMS = 16;
@@ -132,23 +134,28 @@ __global__ __launch_bounds__(NT) void hc_read_vec_kernel(T* __restrict__ h, cons
     }
 }
 
-template <typename T>
+// (Y other than void: y is what a mixture of experts left per slot, float or the storage type; it is summed here, and rounded as a tensor would hold it)
+template <typename T, typename Y = void>
 __global__ __launch_bounds__(NT) void hc_write_vec_kernel(float* __restrict__ x, const T* __restrict__ y, const float* __restrict__ mix,
                                                           const float* __restrict__ w_out, int S, int D, T* __restrict__ h_next,
                                                           const float* __restrict__ w_in_next, const T* __restrict__ nw,
-                                                          const T* __restrict__ nb, float alpha, int chunks) {
+                                                          const T* __restrict__ nb, float alpha, int chunks, SlotRows slots) {
     const size_t t = token_of(blockIdx.x, chunks);
     for (int i = ((blockIdx.x - (unsigned)t * chunks) * NT + threadIdx.x) * 4; i < D; i += chunks * NT * 4) {
-        float old[MAX_STREAMS][4], yv[4], u[4] = {0.f, 0.f, 0.f, 0.f};
+        float old[MAX_STREAMS][4], yv[1][4], u[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int s = 0; s < MAX_STREAMS; ++s)
             if (s < S) ld4t(x, (t * S + s) * D + i, old[s]);
-        ld4t(y, t * D + i, yv);
+        if constexpr (std::is_void<Y>::value) ld4t(y, t * D + i, yv[0]);
+        else {
+            slot_sum4<Y>(slots, t, D, i, 0, yv);
+            round_stored<T>(yv);
+        }
         for (int r = 0; r < S; ++r) {
             float a[4];
             const float wo = w_out[r];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) a[j] = wo * yv[j];
+            for (int j = 0; j < 4; ++j) a[j] = wo * yv[0][j];
 #pragma unroll
             for (int s = 0; s < MAX_STREAMS; ++s)
                 if (s < S) {
@@ -302,12 +309,30 @@ extern "C" int qsv_hc_write(float* x, const void* y, const float* mix, const flo
     if (D % 4 == 0)
         QSV_DISPATCH(dtype, "qsv_hc_write",
                      hipLaunchKernelGGL(hc_write_vec_kernel<T>, dim3((unsigned)(chunks * n)), dim3(NT), 0, (hipStream_t)stream, x, (const T*)y, mix, w_out,
-                                        streams, D, (T*)h_next, w_in_next, (const T*)norm_w, (const T*)norm_b, alpha, chunks));
+                                        streams, D, (T*)h_next, w_in_next, (const T*)norm_w, (const T*)norm_b, alpha, chunks, SlotRows{}));
     else
         QSV_DISPATCH(dtype, "qsv_hc_write",
                      hipLaunchKernelGGL(hc_write_kernel<T>, dim3(n), dim3(NT), 0, (hipStream_t)stream, x, (const T*)y, mix, w_out,
                                         streams, D, (T*)h_next, w_in_next, (const T*)norm_w, (const T*)norm_b, alpha));
     return qsv_launch_status("qsv_hc_write");
+}
+
+extern "C" int qsv_hc_write_slots(float* x, const void* ys, int float_rows, const int32_t* place, const float* weight, const int32_t* idx, int top_k, int n_experts,
+                                  const float* mix, const float* w_out, int n, int streams, int D, int dtype, void* stream) {
+    QSV_REQUIRE(x && ys && idx && mix && w_out && n >= 0 && D > 0 && top_k > 0 && n_experts > 0, "qsv_hc_write_slots: bad arguments");
+    QSV_REQUIRE(streams > 0 && streams <= MAX_STREAMS, "qsv_hc_write_slots: %d streams (at most %d)", streams, MAX_STREAMS);
+    QSV_REQUIRE(D % 4 == 0 && fits4(ys, float_rows ? QSV_F32 : dtype), "qsv_hc_write_slots: width %d (a multiple of 4), rows on four elements", D);
+    if (n == 0) return QSV_OK;
+    const int chunks = stream_chunks(n, 512, D);
+    const SlotRows slots = {ys, place, weight, idx, top_k, n_experts};
+#define QSV_HCW(Y)                                                                                                                              \
+    QSV_DISPATCH(dtype, "qsv_hc_write_slots",                                                                                                   \
+                 hipLaunchKernelGGL((hc_write_vec_kernel<T, Y>), dim3((unsigned)(chunks * n)), dim3(NT), 0, (hipStream_t)stream, x, (const T*)nullptr, mix, w_out, \
+                                    streams, D, (T*)nullptr, (const float*)nullptr, (const T*)nullptr, (const T*)nullptr, 0.f, chunks, slots))
+    if (float_rows) QSV_HCW(float);
+    else QSV_HCW(T);
+#undef QSV_HCW
+    return qsv_launch_status("qsv_hc_write_slots");
 }
 
 extern "C" int qsv_dyt_sum_rows(void* out, const float* x, const int32_t* rows, const void* norm_w, const void* norm_b,

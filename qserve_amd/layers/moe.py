@@ -21,9 +21,10 @@ class GroupedTopKMoE:
         if E % self.groups or not 0 < self.keep <= self.groups or not 0 < self.top_k <= self.keep * (E // self.groups):
             raise ValueError(f"router: {E} experts, {self.groups} groups, keep {self.keep}, top {self.top_k}")
 
-    def __call__(self, h):
+    def __call__(self, h, rows=False):
+        """rows: the caller takes the experts' rows (qserve_amd.layers.ops.ExpertRows) and sums them itself."""
         idx, wt = self.ops.moe_route(h, self.router, self.top_k, self.groups, self.keep)
-        return self.ops.moe_experts(h, self.up, self.down, idx, wt)
+        return self.ops.moe_experts(h, self.up, self.down, idx, wt, rows=rows)
 
 
 def _interleave(gate, up):
@@ -43,7 +44,8 @@ class GatedFeedForward:
             raise ValueError(f"gated feed-forward: activation {act!r}, limit {limit}")
         self.ops, self.w_in, self.w_down, self.act, self.limit = ops, _interleave(gate, up), down.contiguous(), act, float(limit)
 
-    def __call__(self, h):
+    def __call__(self, h, rows=False):
+        """rows: as the mixtures below take it; there is one row per token here, its sum."""
         from .ops import linear
         a = linear(h, self.w_in)
         return linear(self.ops.glu(a) if self.act == "silu" else self.ops.glu(a, self.act, self.limit), self.w_down)
@@ -66,9 +68,10 @@ class TopKGatedMoE:
         if not 0 < self.top_k <= E:
             raise ValueError(f"router: {E} experts, top {self.top_k}")
 
-    def __call__(self, h):
+    def __call__(self, h, rows=False):
+        """rows: the caller takes the experts' rows (qserve_amd.layers.ops.ExpertRows) and sums them itself."""
         idx, wt = self.ops.moe_route(h, self.router, self.top_k, 1, 1, bias=self.bias, renorm=True)
-        return self.ops.moe_experts(h, self.up, self.down, idx, wt, act="swiglu")
+        return self.ops.moe_experts(h, self.up, self.down, idx, wt, act="swiglu", rows=rows)
 
 
 class SigmoidMoE:
@@ -94,10 +97,11 @@ class SigmoidMoE:
         if E % self.groups or not 0 < self.keep <= self.groups or not 0 < self.top_k <= self.keep * (E // self.groups):
             raise ValueError(f"router: {E} experts, {self.groups} groups, keep {self.keep}, top {self.top_k}")
 
-    def __call__(self, h):
+    def __call__(self, h, rows=False):
+        """rows: the caller takes the experts' rows (qserve_amd.layers.ops.ExpertRows) for the routed output and sums them itself."""
         idx, wt = self.ops.moe_route(h, self.router, self.top_k, self.groups, self.keep, score="sigmoid", correction=self.correction,
                                      group_top=2, scale=self.scale)
-        y = [self.ops.moe_experts(h, self.up, self.down, idx, wt, act="swiglu", weigh=self.weigh)]
+        y = [self.ops.moe_experts(h, self.up, self.down, idx, wt, act="swiglu", weigh=self.weigh, rows=rows)]
         if self.shared is not None:
             y.append(self.shared(h))
         return y

@@ -108,6 +108,35 @@ def _head_products(x, w):
     return torch.bmm(x.transpose(0, 1), w).transpose(0, 1).reshape(x.size(0), w.size(0) * w.size(2))
 
 
+class ExpertRows:
+    """What a mixture of experts leaves, a row per slot (t, k), where its user sums them itself (`moe_experts(..., rows=True)`): y[t] = sum_k wt[t, k]
+    ys[place[t K + k]] (wt None: ones; place None: row t K + k).  `dense()` is the sum as a tensor of the storage type."""
+
+    def __init__(self, ops, ys, place, wt, idx, h, experts):
+        self.ops, self.ys, self.place, self.wt, self.idx, self.h, self.experts = ops, ys, place, wt, idx, h, experts
+        self.shape = h.shape
+
+    def args(self):
+        return (self.ys.data_ptr(), int(self.ys.dtype == torch.float32), 0 if self.place is None else self.place.data_ptr(),
+                0 if self.wt is None else self.wt.data_ptr(), self.idx.data_ptr(), self.idx.size(1), self.experts)
+
+    def dense(self):
+        o, (T, D) = self.ops, self.shape
+        y = torch.empty((T, D), dtype=o.dtype, device=self.ys.device)
+        w, K = 0 if self.wt is None else self.wt.data_ptr(), self.idx.size(1)
+        rest = (w, T, K, D, self.idx.data_ptr(), self.h.data_ptr(), self.experts, o.code, o._s())
+        if self.place is None:
+            o.check(o.L.qsv_moe_combine_slots(y.data_ptr(), self.ys.data_ptr(), *rest), "moe_combine_slots")
+        else:
+            o.check(o.L.qsv_moe_combine_sorted(y.data_ptr(), self.ys.data_ptr(), self.place.data_ptr(), *rest), "moe_combine_sorted")
+        return y
+
+
+def _on_four(*ts):
+    """Whether four elements can be read at once from the start of every tensor."""
+    return all(t is None or t.data_ptr() % (4 * t.element_size()) == 0 for t in ts)
+
+
 class HipOps:
     name = "hip"
 
@@ -135,8 +164,17 @@ class HipOps:
         return x, h
 
     def add_layer_norm(self, x, y, w, eps):
-        """x += layer_norm(y) * w in place; returns x in the storage type."""
+        """x += layer_norm(y) * w in place; returns x in the storage type.  y: a tensor or a mixture's ExpertRows (summed here, the same bits as its
+        dense())."""
         h = torch.empty(x.shape, dtype=self.dtype, device=x.device)
+        if isinstance(y, ExpertRows):
+            if x.size(1) % 4 == 0 and x.size(1) <= 4096 and _on_four(x, w):
+                self._need(x, w, y.ys, y.idx)
+                assert y.shape == x.shape and x.dtype == torch.float32 and w.dtype == self.dtype
+                self.check(self.L.qsv_add_layer_norm_slots(x.data_ptr(), h.data_ptr(), *y.args(), w.data_ptr(), eps, x.size(0), x.size(1), self.code, self._s()),
+                           "add_layer_norm_slots")
+                return h
+            y = y.dense()
         self._need(x, y, w)
         assert y.shape == x.shape and y.dtype == self.dtype and x.dtype == torch.float32
         self.check(self.L.qsv_add_layer_norm(x.data_ptr(), h.data_ptr(), y.data_ptr(), w.data_ptr(), eps, x.size(0), x.size(1),
@@ -327,6 +365,13 @@ class HipOps:
         """All streams rewritten in place from the sublayer's output y.  then_read = (w_in, norm) of the NEXT sublayer, if it
         reads without a token shift: its input comes out of the same pass -> h [T, D] (else None)."""
         T, S, D = x.shape
+        if isinstance(y, ExpertRows):                                   # (the same bits as y.dense() gives)
+            if then_read is None and D % 4 == 0 and _on_four(x):
+                self._need(x, y.ys, y.idx, w_mix, w_out)
+                assert y.shape == (T, D) and w_mix.dtype == torch.float32 and w_mix.shape == (S, S)
+                self.check(self.L.qsv_hc_write_slots(x.data_ptr(), *y.args(), w_mix.data_ptr(), w_out.data_ptr(), T, S, D, self.code, self._s()), "hc_write_slots")
+                return None
+            y = y.dense()
         self._need(x, y, w_mix, w_out)
         assert y.shape == (T, D) and y.dtype == self.dtype and w_mix.dtype == torch.float32 and w_mix.shape == (S, S)
         h, nxt = None, [0, 0, 0, 0, 0.0]
@@ -406,8 +451,23 @@ class HipOps:
     def scaled_sum_rms_norms(self, x, parts, gains, eps, tokens=None, table=None):
         """x += sum of scale * y over parts [(y, scale)] (up to three; y storage type, scale per coordinate in the storage type or None) in
         place, or, with tokens, x <- table[tokens] (+ the parts; x None: made here); -> (x, [rms_norm(x) * g in the storage type for the (up to
-        two) float gains g]), all from one statistic."""
+        two) float gains g]), all from one statistic.  The second part may be a mixture's ExpertRows (the same bits as its dense())."""
         assert len(parts) <= 3 and len(gains) <= 2
+        if any(isinstance(y, ExpertRows) for y, _ in parts):
+            T, D = x.shape
+            (a, sa), (e, se), (c, sc) = (list(parts) + [(None, None)] * 2)[:3]
+            if (tokens is None and isinstance(e, ExpertRows) and isinstance(a, torch.Tensor) and not isinstance(c, ExpertRows) and D % 4 == 0 and D <= 4096
+                    and _on_four(x, a, sa, se, c, sc, *gains)):
+                hs = [torch.empty((T, D), dtype=self.dtype, device=x.device) for _ in gains]
+                self._need(x, a, sa, e.ys, e.idx, se, c, sc, *gains)
+                assert x.dtype == torch.float32 and all(g.dtype == torch.float32 and g.numel() == D for g in gains)
+                assert all(y is None or (y.shape == x.shape and (s is None or (s.dtype == self.dtype and s.numel() == D))) for y, s in ((a, sa), (e, se), (c, sc)))
+                p = [0 if v is None else v.data_ptr() for v in (a, sa, se, c, sc)]
+                hp, gp = ([v.data_ptr() for v in vs] + [0] * (2 - len(vs)) for vs in (hs, gains))
+                self.check(self.L.qsv_scaled_sum_rms_norms_slots(x.data_ptr(), *hp, *p[:2], *e.args(), *p[2:], *gp, float(eps), T, D, self.code, self._s()),
+                           "scaled_sum_rms_norms_slots")
+                return x, hs
+            parts = [(y.dense() if isinstance(y, ExpertRows) else y, s) for y, s in parts]
         if tokens is not None and x is None:
             x = torch.empty((tokens.numel(), table.size(1)), dtype=torch.float32, device=table.device)
         T, D = x.shape
@@ -831,14 +891,15 @@ class HipOps:
 
     ACTS = {"none": 0, "relu_sq": 1, "swiglu": 2, "clamped_glu": 3}
 
-    def moe_experts(self, h, up, down, idx, wt, act="relu_sq", limit=0.0, weigh="output"):
+    def moe_experts(self, h, up, down, idx, wt, act="relu_sq", limit=0.0, weigh="output", rows=False):
         """up [E, rows, D], down [E, D, ff]; y[t] = sum_k wt[t, k] * down[idx[t, k]] a(up[idx[t, k]] h[t]).  act "relu_sq":
         a = relu(.)^2, rows = ff; "swiglu": up's rows come in pairs (2f = gate, 2f + 1 = up), a_f = silu(gate_f) up_f, rows = 2 ff;
         "clamped_glu": the same pairs with g = min(gate_f, limit), u = clamp(up_f, -limit, limit), a_f = g sigmoid(1.702 g) (u + 1).
         Indices at or above E (up.size(0)) name identity experts: their output is h[t] itself; below 0: no expert.  weigh "input": the weight multiplies the
-        expert's input, y[t] = sum_k down[..] a(up[..] (wt[t, k] h[t])) (the products' results are scaled, in float)."""
+        expert's input, y[t] = sum_k down[..] a(up[..] (wt[t, k] h[t])) (the products' results are scaled, in float).  rows: the caller takes ExpertRows in
+        place of the sum (where the form has them), and idx names experts of `up` only or none."""
         T, D = h.shape
-        top_k, rows = idx.size(1), up.size(1)
+        lazy, top_k, rows = rows, idx.size(1), up.size(1)
         idx = idx.to(torch.int32).contiguous()
         a = self.ACTS[act]
         ff = rows // 2 if a >= 2 else rows
@@ -846,9 +907,9 @@ class HipOps:
         if major is None:
             major = self.moe_sorted_above if max(D, ff) > 4096 else 896 if self._grouped_takes(up.size(0), rows, D, ff) else 1024
         if self.code == BF16 and self.moe_token_slots < T * top_k <= major and D % 8 == 0 and ff % 8 == 0 and max(D, ff) <= 1 << 25:
-            return self._moe_experts_expert_major(h, up, down, idx, wt, a, limit, weigh)
+            return self._moe_experts_expert_major(h, up, down, idx, wt, a, limit, weigh, lazy)
         if T * top_k > self.moe_sorted_above or (T and max(D, top_k * ff) * 4 > 64 * 1024):     # (the per-token kernels keep a token's rows in 64 KiB of LDS)
-            return self._moe_experts_sorted(h, up, down, idx, wt, a, limit, weigh)
+            return self._moe_experts_sorted(h, up, down, idx, wt, a, limit, weigh, lazy)
         act = torch.empty((T, top_k, ff), dtype=self.dtype, device=h.device)
         y = torch.empty((T, D), dtype=self.dtype, device=h.device)
         self._need(h, up, down, idx, wt)
@@ -900,9 +961,9 @@ class HipOps:
                                           h.data_ptr(), E, self.code, self._s()), "moe_combine")
         return y
 
-    def _moe_experts_expert_major(self, h, up, down, idx, wt, a=1, limit=0.0, weigh="output"):
+    def _moe_experts_expert_major(self, h, up, down, idx, wt, a=1, limit=0.0, weigh="output", lazy=False):
         T, D = h.shape
-        w_in, w_out = self._weights_at(wt, weigh)
+        w_in, _ = self._weights_at(wt, weigh)
         E, rows, K = up.size(0), up.size(1), idx.size(1)
         ff = rows // 2 if a >= 2 else rows
         n = T * K
@@ -910,17 +971,15 @@ class HipOps:
         h, up, down = self._on_16_bytes(h, up, down)
         act = torch.empty((n, ff), dtype=self.dtype, device=h.device)
         ys = torch.empty((n, D), dtype=torch.float32, device=h.device)
-        y = torch.empty((T, D), dtype=self.dtype, device=h.device)
         s = self._s()
         self.check(self.L.qsv_expert_slots(act.data_ptr(), 0, h.data_ptr(), K, up.data_ptr(), idx.data_ptr(), n, E, rows, D, a, float(limit),
                                            w_in, s), "expert_slots(up)")
         self.check(self.L.qsv_expert_slots(ys.data_ptr(), 1, act.data_ptr(), 1, down.data_ptr(), idx.data_ptr(), n, E, D, ff, 0, 0.0, 0, s),
                    "expert_slots(down)")
-        self.check(self.L.qsv_moe_combine_slots(y.data_ptr(), ys.data_ptr(), w_out, T, K, D, idx.data_ptr(), h.data_ptr(), E, self.code, s),
-                   "moe_combine_slots")
-        return y
+        y = ExpertRows(self, ys, None, wt if weigh == "output" else None, idx, h, E)
+        return y if lazy else y.dense()
 
-    def _moe_experts_sorted(self, h, up, down, idx, wt, code=1, limit=0.0, weigh="output"):
+    def _moe_experts_sorted(self, h, up, down, idx, wt, code=1, limit=0.0, weigh="output", lazy=False):
         """code >= 2 (gated units): the grouped kernel folds the two halves of a unit in its epilogue; with vendor products the
         first product leaves both halves ([n, 2 ff]) and `glu` folds them."""
         T, D = h.shape
@@ -937,16 +996,14 @@ class HipOps:
             offsets = torch.empty((E + 1,), dtype=torch.int32, device=h.device)
             act = torch.empty((n, ff), dtype=self.dtype, device=h.device)
             ys = torch.empty((n, D), dtype=self.dtype, device=h.device)
-            y = torch.empty((T, D), dtype=self.dtype, device=h.device)
             s = self._s()
             self.check(L.qsv_moe_sort(order.data_ptr(), place.data_ptr(), offsets.data_ptr(), idx.data_ptr(), n, E, s), "moe_sort")
             self.check(L.qsv_grouped_gemm_sorted(act.data_ptr(), h.data_ptr(), order.data_ptr(), K, up.data_ptr(), offsets.data_ptr(), E, rows, D, code,
                                                  float(limit), w_in, s), "grouped_gemm(up)")
             self.check(L.qsv_grouped_gemm_sorted(ys.data_ptr(), act.data_ptr(), 0, 1, down.data_ptr(), offsets.data_ptr(), E, D, ff, 0, 0.0, 0, s),
                        "grouped_gemm(down)")
-            self.check(L.qsv_moe_combine_sorted(y.data_ptr(), ys.data_ptr(), place.data_ptr(), w_out, T, K, D, idx.data_ptr(), h.data_ptr(), E,
-                                                self.code, s), "moe_combine_sorted")
-            return y
+            y = ExpertRows(self, ys, place, wt if weigh == "output" else None, idx, h, E)
+            return y if lazy else y.dense()
         flat = idx.reshape(-1)
         order = torch.argsort(flat, stable=True)                       # sorted slot -> slot (t K + k)
         counts = torch.bincount(flat, minlength=E).tolist()[:E]        # (host synchronisation: the runs' lengths; identity experts sort last)
@@ -1435,7 +1492,7 @@ class TorchOps:
             m_state[slot] = prev
         return a, b, m
 
-    def moe_experts(self, h, up, down, idx, wt, act="relu_sq", limit=0.0, weigh="output"):
+    def moe_experts(self, h, up, down, idx, wt, act="relu_sq", limit=0.0, weigh="output", rows=False):
         T, D = h.shape
         E = up.size(0)
         y = torch.zeros((T, D), dtype=torch.float32, device=h.device)

@@ -140,7 +140,7 @@ class Mumelix:
                 ops.hc_write(x, y, w_mix, w_out)
             else:                                               # the feed-forward's input comes out of the mixer's stream rewrite
                 h = ops.hc_write(x, y, w_mix, w_out, then_read=(L["hc2"][0], L["norm2"]))
-                ops.hc_write(x, L["ff"](h), L["hc2"][1], L["hc2"][2])
+                ops.hc_write(x, L["ff"](h, rows=True), L["hc2"][1], L["hc2"][2])
             if tap is not None:
                 tap(run, x.sum(1))
         return x

@@ -123,7 +123,7 @@ class Rivolix:
             p0, p1, s0, s1 = self.slices[i]
             parts = [(L["mixer"](hs[0], batch, pools[p0:p1], states[s0:s1]), L["ls1"])]
             if L["ff"] is not None:
-                parts += [(y, L["ls2"]) for y in L["ff"](hs[1])]
+                parts += [(y, L["ls2"]) for y in L["ff"](hs[1], rows=True)]
             # the next layer's two inputs come out of the pass that adds this layer's outputs to the stream
             _, hs = ops.scaled_sum_rms_norms(x, parts, gains(i + 1), self.eps)
             if tap is not None:

@@ -91,7 +91,7 @@ class Vekalorn:
         for i, L in enumerate(self.layers):
             h = ops.add_layer_norm(x, L["mixer"](h, batch, pools[i]), L["norm1"], self.eps)
             if L["ff"] is not None:
-                h = ops.add_layer_norm(x, L["ff"](h), L["norm2"], self.eps)
+                h = ops.add_layer_norm(x, L["ff"](h, rows=True), L["norm2"], self.eps)
             if tap is not None:
                 tap(i, x)
         return x

@@ -16,6 +16,7 @@ SIGNATURES = {
     "qsv_head_product": (_i, [_vp, _vp, _i64, _i64, _vp, _i, _i, _i, _i, _vp]),
     "qsv_latent_query_product": (_i, [_vp, _vp, _vp, _vp, _vp, _f, _i, _i, _i, _i, _i, _i, _vp]),
     "qsv_embed": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _vp]),
+    "qsv_add_layer_norm_slots": (_i, [_vp, _vp, _vp, _i, _vp, _vp, _vp, _i, _i, _vp, _f, _i, _i, _i, _vp]),
     "qsv_add_layer_norm": (_i, [_vp, _vp, _vp, _vp, _f, _i, _i, _i, _vp]),
     "qsv_layer_norm_rows": (_i, [_vp, _vp, _vp, _vp, _f, _i, _i, _i, _vp]),
     "qsv_latent_prep": (_i, [_vp, _i64, _i, _i, _vp, _vp, _i, _i, _vp, _i, _i, _vp, _vp, _vp, _vp, _f, _i, _i, _vp]),
@@ -63,6 +64,7 @@ SIGNATURES = {
     "qsv_moe_down": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp, _i, _i, _vp]),
     "qsv_embed_streams": (_i, [_vp, _vp, _vp, _f, _i, _i, _i, _i, _vp]),
     "qsv_hc_read": (_i, [_vp, _vp, _vp, _vp, _vp, _f, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp]),
+    "qsv_hc_write_slots": (_i, [_vp, _vp, _i, _vp, _vp, _vp, _i, _i, _vp, _vp, _i, _i, _i, _i, _vp]),
     "qsv_hc_write": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _vp, _vp, _vp, _vp, _f, _i, _vp]),
     "qsv_dyt_sum_rows": (_i, [_vp, _vp, _vp, _vp, _vp, _f, _i, _i, _i, _i, _vp]),
     "qsv_rms_pair_mean": (_i, [_vp, _vp, _vp, _vp, _vp, _f, _i, _i, _i, _vp]),
@@ -87,6 +89,7 @@ SIGNATURES = {
     "qsv_embed_sinusoid": (_i, [_vp, _vp, _vp, _vp, _vp, _f, _i, _i, _i, _vp]),
     "qsv_add_rms_norm": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _f, _i, _i, _i, _vp]),
     "qsv_rms_norm_rows": (_i, [_vp, _vp, _vp, _vp, _i, _f, _i, _i, _i, _vp]),
+    "qsv_scaled_sum_rms_norms_slots": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i, _vp, _vp, _vp, _i, _i, _vp, _vp, _vp, _vp, _vp, _f, _i, _i, _i, _vp]),
     "qsv_scaled_sum_rms_norms": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _f, _i, _i, _i, _vp]),
     "qsv_normed_attention_prep": (_i, [_vp, _vp, _i64, _vp, _i64, _i, _i, _i, _i, _i, _i, _i, _vp, _vp, _f, _f, _vp, _i64, _f, _vp, _i,
                                        _i, _vp]),

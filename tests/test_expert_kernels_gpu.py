@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from qserve_amd.layers.ops import make_ops
+from qserve_amd.layers.ops import ExpertRows, make_ops
 
 pytestmark = pytest.mark.gpu
 
@@ -138,6 +138,50 @@ def test_grouped_products_of_sorted_runs(ops, K, N, E, div):
 @pytest.mark.parametrize("E", [1025, 1600, 8064])
 def test_grouped_form_of_many_experts(ops, E):
     check(ops, 600, 2, E, 3, 64, 64, "relu_sq", "input", 0.1)
+
+
+# The sum over a mixture's rows inside the kernel that uses it: float rows (a step) and rows in the storage type found through their places (a prompt), slots
+# without an expert, weights on the inputs, chunks of 1024 columns; and widths that only the sum as a tensor serves.
+@pytest.mark.parametrize("T, top, D, ff", [(1, 1, 8, 8), (3, 4, 72, 40), (5, 5, 1032, 64), (64, 4, 2048, 64), (17, 7, 4096, 64), (3, 2, 4104, 64), (600, 2, 64, 64), (400, 4, 1088, 64)])
+@pytest.mark.parametrize("weigh", ["output", "input"])
+def test_sums_over_experts_inside_their_users(ops, T, top, D, ff, weigh):
+    g = torch.Generator().manual_seed(T + D)
+    dev, E = "cuda:0", 8
+    h, up, down = torch.randn(T, D, generator=g).bfloat16(), (torch.randn(E, ff, D, generator=g) / D ** 0.5).bfloat16(), (torch.randn(E, D, ff, generator=g) / ff ** 0.5).bfloat16()
+    idx, wt = torch.rand(T, E, generator=g).argsort(1)[:, :top].int(), torch.rand(T, top, generator=g)
+    idx[torch.rand(T, top, generator=g) < 0.2] = -1
+    rows = ops.moe_experts(h.to(dev), up.to(dev), down.to(dev), idx.to(dev), wt.to(dev), weigh=weigh, rows=True)
+    assert isinstance(rows, ExpertRows)
+    k = torch.arange(T * top).view(T, top) if rows.place is None else rows.place.cpu().long().view(T, top).clamp(0)
+    w = (wt if weigh == "output" else torch.ones_like(wt)) * (idx >= 0)
+    y = (w.double()[..., None] * rows.ys.double().cpu()[torch.where(idx >= 0, k, torch.zeros_like(k))].where((idx >= 0)[..., None], torch.zeros(()).double())).sum(1)
+    x, a, c = torch.randn(T, D, generator=g), torch.randn(T, D, generator=g).bfloat16(), torch.randn(T, D, generator=g).bfloat16()
+    v, s = torch.randn(D, generator=g).bfloat16(), [torch.randn(D, generator=g).bfloat16() for _ in range(3)]
+    gains = [torch.randn(D, generator=g) for _ in range(2)]
+    near = lambda got, ref, size: ((got.double().cpu() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2.0 ** -18 + 2.0 ** -7 * size).all()    # noqa: E731
+    y = y.bfloat16().double()                                           # (as a tensor holds it; a sum near half a unit may fall the other way)
+    xd = x.to(dev)
+    hd = ops.add_layer_norm(xd, rows, v.to(dev), 1e-5)
+    d = y - y.mean(-1, keepdim=True)
+    scale = 1.0 / (d.pow(2).mean(-1, keepdim=True) + 1e-5).sqrt()
+    ref = x.double() + d * scale * v.double()
+    size = (y.abs().amax(-1, keepdim=True) * scale * v.double().abs() * 4)
+    assert near(xd, ref, size) and near(hd, ref, size)
+    for parts, more in (([(a, s[0]), (rows, s[1]), (c, s[2])], True), ([(a, None), (rows, None)], False)):
+        xd = x.to(dev)
+        _, hs = ops.scaled_sum_rms_norms(xd, [(p if p is rows else p.to(dev), None if f is None else f.to(dev)) for p, f in parts], [t.to(dev) for t in gains], 1e-5)
+        one = torch.ones(D, dtype=torch.float64)
+        ref = x.double() + a.double() * (s[0].double() if more else one) + y * (s[1].double() if more else one) + (c.double() * s[2].double() if more else 0.0)
+        inv = 1.0 / (ref.pow(2).mean(-1, keepdim=True) + 1e-5).sqrt()
+        size = y.abs() * (s[1].double().abs() if more else 1.0) + ref.abs()
+        assert near(xd, ref, size)
+        assert all(near(t, ref * inv * gn.double(), size * inv * gn.double().abs()) for t, gn in zip(hs, gains))
+    S = 3
+    x3, mix, out = torch.randn(T, S, D, generator=g), torch.randn(S, S, generator=g), torch.randn(S, generator=g)
+    xd = x3.to(dev)
+    ops.hc_write(xd, rows, mix.to(dev), out.to(dev))
+    ref = torch.einsum("tsd,sr->trd", x3.double(), mix.double()) + out.double()[None, :, None] * y[:, None]
+    assert near(xd, ref, y.abs()[:, None] * out.abs()[None, :, None] + 4)
 
 
 @pytest.mark.parametrize("T, top, D, ff", [(3, 2, 64, 64), (40, 4, 72, 40), (1200, 2, 64, 128)])

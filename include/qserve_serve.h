@@ -27,6 +27,9 @@ int qsv_skinny_linear(void* out, const void* x, int64_t x_stride, const void* w,
 /* out [T, H, N] = x[t, h] @ w[h], w [H, K, N], bfloat16 with float accumulation, for up to 64 rows; x_tok, x_head: elements from one token / head
  * of x to the next.  K and N multiples of 32, x_tok and x_head of 8, x on 16 bytes. */
 int qsv_head_product(void* out, const void* x, int64_t x_tok, int64_t x_head, const void* w, int T, int H, int K, int N, void* stream);
+/* The same times sigmoid(gate[t, h]) before the rounding; gate: storage type, rows gate_stride (even) elements apart. */
+int qsv_head_product_gated(void* out, const void* x, int64_t x_tok, int64_t x_head, const void* w, int n_tokens, int heads, int K, int N, const void* gate,
+                           int64_t gate_stride, void* stream);
 
 /* The product with w_uk [H, dim, rank] and qsv_latent_query in one (bfloat16, up to 64 rows; dim and rank multiples of 32, dim + rot_dim of 8,
  * rot_dim even): the absorbed part is not rounded in between. */

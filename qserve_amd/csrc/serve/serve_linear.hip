@@ -58,6 +58,8 @@ struct HeadProductArgs {
     const int32_t* pos;
     float scale;
     int dim, rot_dim, rot_n;
+    const bf16_t* gate;              // (not QUERY) the result is multiplied by sigmoid(gate[t, h]) before it is rounded
+    int64_t gate_stride;
 };
 template <int RT, int S, bool QUERY>
 __global__ __launch_bounds__(256) void head_product_kernel(HeadProductArgs a) {
@@ -119,6 +121,7 @@ __global__ __launch_bounds__(256) void head_product_kernel(HeadProductArgs a) {
     for (int r = 0; r < RT; ++r) {
         const int t = 16 * r + (tid >> 4), c = 2 * (tid & 15);
         if (t >= a.T) continue;
+        const unsigned g = !QUERY && a.gate ? *(const unsigned*)(a.gate + t * a.gate_stride + (size_t)h * a.N + n0 + c) : 0u;
         float2 v = make_float2(0.f, 0.f);
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
@@ -127,7 +130,13 @@ __global__ __launch_bounds__(256) void head_product_kernel(HeadProductArgs a) {
             v.y += p.y;
         }
         if (QUERY) *(float2*)((float*)a.out + ((size_t)t * a.H + h) * (a.N + a.rot_dim) + n0 + c) = make_float2(v.x * a.scale, v.y * a.scale);
-        else *(unsigned*)((bf16_t*)a.out + ((size_t)t * a.H + h) * a.N + n0 + c) = (unsigned)f2bf(v.x) | ((unsigned)f2bf(v.y) << 16);
+        else {
+            if (a.gate) {
+                v.x *= 1.0f / (1.0f + expf(-__uint_as_float(g << 16)));
+                v.y *= 1.0f / (1.0f + expf(-__uint_as_float(g & 0xffff0000u)));
+            }
+            *(unsigned*)((bf16_t*)a.out + ((size_t)t * a.H + h) * a.N + n0 + c) = (unsigned)f2bf(v.x) | ((unsigned)f2bf(v.y) << 16);
+        }
     }
 }
 template <int RT, bool QUERY>
@@ -155,8 +164,16 @@ int run_head_product(const HeadProductArgs& a, hipStream_t stream, const char* w
 // out [T, H, N] = x[t, h] @ w[h], x rows x_tok / x_head elements apart, w [H, K, N]
 extern "C" int qsv_head_product(void* out, const void* x, int64_t x_tok, int64_t x_head, const void* w, int T, int H, int K, int N, void* stream) {
     QSV_REQUIRE(out && x && w && head_product_ok(T, x_tok, x_head, x, w, K, N, H) && (uintptr_t)out % 4 == 0, "qsv_head_product: bad arguments");
-    return run_head_product<false>({out, (const bf16_t*)x, (const bf16_t*)w, x_tok, x_head, T, K, N, H, nullptr, nullptr, 1.0f, 0, 0, 0},
+    return run_head_product<false>({out, (const bf16_t*)x, (const bf16_t*)w, x_tok, x_head, T, K, N, H, nullptr, nullptr, 1.0f, 0, 0, 0, nullptr, 0},
                                    (hipStream_t)stream, "qsv_head_product");
+}
+// ... times sigmoid(gate[t, h]), rows of gate gate_stride apart
+extern "C" int qsv_head_product_gated(void* out, const void* x, int64_t x_tok, int64_t x_head, const void* w, int T, int H, int K, int N, const void* gate,
+                                      int64_t gate_stride, void* stream) {
+    QSV_REQUIRE(out && x && w && gate && head_product_ok(T, x_tok, x_head, x, w, K, N, H) && (uintptr_t)out % 4 == 0 && (uintptr_t)gate % 4 == 0 && gate_stride % 2 == 0 &&
+                    gate_stride >= (int64_t)H * N, "qsv_head_product_gated: bad arguments");
+    return run_head_product<false>({out, (const bf16_t*)x, (const bf16_t*)w, x_tok, x_head, T, K, N, H, nullptr, nullptr, 1.0f, 0, 0, 0, (const bf16_t*)gate, gate_stride},
+                                   (hipStream_t)stream, "qsv_head_product_gated");
 }
 
 // qf [T, H, rank + rot_dim] (float) = scale * [q[t, h, :dim] @ w_uk[h] | rotated q[t, h, dim:]], q [T, H, dim + rot_dim], w_uk [H, dim, rank]
@@ -166,7 +183,7 @@ extern "C" int qsv_latent_query_product(float* qf, const void* q, const void* w_
                     rot_dim <= (1 << 20) && rot_dim % 2 == 0 && (uintptr_t)qf % 8 == 0, "qsv_latent_query_product: bad arguments");
     const int64_t row = dim + rot_dim;
     QSV_REQUIRE(head_product_ok(T, row * H, row, q, w_uk, dim, rank, H), "qsv_latent_query_product: sizes or addresses it does not take");
-    return run_head_product<true>({qf, (const bf16_t*)q, (const bf16_t*)w_uk, row * H, row, T, dim, rank, H, rope, pos, scale, dim, rot_dim, rot_n},
+    return run_head_product<true>({qf, (const bf16_t*)q, (const bf16_t*)w_uk, row * H, row, T, dim, rank, H, rope, pos, scale, dim, rot_dim, rot_n, nullptr, 0},
                                   (hipStream_t)stream, "qsv_latent_query_product");
 }
 

@@ -53,7 +53,5 @@ class LatentAttention:
         q = linear(cq, self.w_uq)                                                   # [T, H (dim + rot_dim)]
         qf = ops.latent_queries(q, self.w_uk, rope, batch.pos, self.scale, H, self.dim, self.rot_dim, self.rot_n, self.rank)
         o_lat = ops.latent_attention(qf, pool, batch, self.window, self.rank, self.page)
-        o = ops.head_products(o_lat, self.w_uv_t)                                   # [T, H vdim]
-        if self.gated:
-            ops.sigmoid_gate(o, down[:, self.g_off:self.g_off + H * self.vdim])
-        return linear(o, self.w_o)
+        gate = down[:, self.g_off:self.g_off + H * self.vdim] if self.gated else None
+        return linear(ops.head_products(o_lat, self.w_uv_t, gate), self.w_o)

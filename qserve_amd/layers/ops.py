@@ -231,17 +231,23 @@ class HipOps:
                 and w.size(1) % 32 == 0 and w.size(2) % 32 == 0 and row % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 4 == 0
                 and w.size(0) <= 65535 and w.size(1) * w.size(2) < 2 ** 31)
 
-    def head_products(self, x, w):
-        """x [T, H, K], w [H, K, N] -> [T, H N], head by head: a step's few rows (up to 64) in one launch (16 heads of 512 to 128, 1 / 16 / 64 tokens:
+    def head_products(self, x, w, gate=None):
+        """x [T, H, K], w [H, K, N] -> [T, H N], head by head, times sigmoid(gate [T, H N]) where given (a column slice is fine): a step's few rows (up to 64) in one launch (16 heads of 512 to 128, 1 / 16 / 64 tokens:
         3.1 / 3.5 / 5.3 us, the vendor's with its copy back to rows 9.8 / 12.9 / 13.3), more through the vendor's batched product."""
         T, H, K = x.shape
         if _heads_stream(T, H, K, w.size(2)) and self._head_products_fit(T, x, w, K):
             self._need(x, w)
             assert w.size(0) == H and w.size(1) == K
             out = torch.empty((T, H * w.size(2)), dtype=x.dtype, device=x.device)
+            if gate is not None and gate.data_ptr() % 4 == 0 and gate.stride(0) % 2 == 0:       # (one launch and one rounding fewer)
+                assert gate.is_cuda and gate.shape == out.shape and gate.stride(1) == 1 and gate.dtype == x.dtype
+                self.check(self.L.qsv_head_product_gated(out.data_ptr(), x.data_ptr(), H * K, K, w.data_ptr(), T, H, K, w.size(2), gate.data_ptr(), gate.stride(0),
+                                                         self._s()), "head_products")
+                return out
             self.check(self.L.qsv_head_product(out.data_ptr(), x.data_ptr(), H * K, K, w.data_ptr(), T, H, K, w.size(2), self._s()), "head_products")
-            return out
-        return _head_products(x, w)
+            return out if gate is None else self.sigmoid_gate(out, gate)
+        out = _head_products(x, w)
+        return out if gate is None else self.sigmoid_gate(out, gate)
 
     plain_rows_kernel = True            # exact row sizes without options: the kernel that copies whole rows into LDS
     attention_split_target = 512        # workgroups a launch of the matrix-core attention should at least have
@@ -1094,8 +1100,9 @@ class TorchOps:
     def latent_queries(self, q, w_uk, rope, pos, scale, heads, dim, rot_dim, rot_n, rank):
         return self.latent_query(q, _absorbed(q, w_uk), rope, pos, scale, heads, dim, rot_dim, rot_n, rank)
 
-    def head_products(self, x, w):
-        return _head_products(x, w)
+    def head_products(self, x, w, gate=None):
+        o = _head_products(x, w)
+        return o if gate is None else self.sigmoid_gate(o, gate)
 
     def latent_attention(self, qf, pool, batch, window, rank, page, variant=0, key_splits=None, q_first=0, chunk=None, bias=None,
                          keep_first=0, sink=None, pooled=None, pool_block=0, slopes=None):

@@ -30,6 +30,18 @@ def test_one_product_per_head(T, H, K, N):
     assert ((y - ref).abs() <= 2.0 ** -8 * ref.abs() + 2.0 ** -22 * K * size + 1e-30).all()
 
 
+@pytest.mark.parametrize("T, H, K, N, off", [(1, 1, 32, 32, 0), (17, 3, 128, 160, 2), (64, 16, 512, 128, 1344), (33, 2, 96, 64, 1), (70, 2, 64, 32, 2)])
+def test_gated_product_per_head(T, H, K, N, off):
+    """The gate a column slice: on two elements (inside the product), on an odd one and beyond 64 rows (a launch of its own, one rounding more)."""
+    g = _gen(T)
+    x, w = torch.randn(T, H, K, device=DEV, generator=g).bfloat16(), torch.randn(H, K, N, device=DEV, generator=g).bfloat16()
+    gate = (torch.randn(T, off + H * N + (off & 1), device=DEV, generator=g) * 3).bfloat16()[:, off:off + H * N]
+    y = HipOps(torch.bfloat16).head_products(x, w, gate).double()
+    xc, wc, s = x.double().cpu(), w.double().cpu(), torch.sigmoid(gate.double()).cpu()
+    ref, size = (torch.einsum("thk,hkn->thn", a, b).reshape(T, -1) * s for a, b in ((xc, wc), (xc.abs(), wc.abs())))
+    assert ((y.cpu() - ref).abs() <= (2 if off & 1 or T > 64 else 1) * 2.0 ** -8 * ref.abs() * 1.01 + 2.0 ** -22 * K * size + 1e-30).all()
+
+
 @pytest.mark.parametrize("T, H, dim, rot_dim, rot_n, rank", [(1, 1, 32, 0, 0, 32), (16, 16, 128, 64, 64, 512), (17, 2, 64, 8, 4, 96), (33, 3, 96, 40, 38, 64),
                                                              (64, 16, 128, 64, 32, 256), (65, 16, 128, 64, 64, 512), (70, 2, 20, 12, 8, 24),
                                                              (5, 3, 33, 7, 2, 31)])

@@ -133,6 +133,20 @@ int qsv_latent_prep(const void* down, int64_t down_stride, int q_off, int q_rank
 int qsv_latent_query(float* qf, const void* q, const void* q_abs, const float* rope, const int32_t* pos, float scale,
                      int n_tokens, int heads, int dim, int rot_dim, int rot_n, int rank, int dtype, void* stream);
 
+/* Latent attention of prompts with the heads' keys and values written out (bfloat16; dim = vdim = 128, rot_dim 0 or 64).
+ * gather: rows [n_rows, R] of the runs [n_runs, 4] = (slot, first position, keys, first row), keys padded to a multiple of 8 with zero rows; longest: the
+ * most keys of a run.
+ * prompt: out [T, H, 128] = attention of q [T, H, 128 + rot_dim] (the first rot_n of its last rot_dim dimensions are rotated here) over k [n_rows, H, 128],
+ * vt [H, 128, n_rows] and the rotated key part, columns rank .. of rows [n_rows, rank + rot_dim]; tiles [n_tiles, 8] = (first token, tokens <=
+ * qsv_latent_prompt_tile_tokens, position of the first, position of the run's first key, its row (a multiple of 8), keys of the run, -, -); window 0: none;
+ * times sigmoid(gate [T, H 128], rows gate_stride apart) where given. */
+int qsv_latent_prompt_tile_tokens(void);
+int qsv_latent_prompt_ok(int dim, int rot_dim, int vdim, int rank, int dtype);
+int qsv_latent_gather(void* rows, const void* pool, const int32_t* block_table, int table_stride, const int32_t* runs, int n_runs, int longest, int n_rows,
+                      int R, int page, void* stream);
+int qsv_latent_prompt(void* out, const void* q, const void* k, const void* vt, const void* rows, const int32_t* tiles, int n_tiles, const float* rope, float scale,
+                      int heads, int rot_dim, int rot_n, int rank, int window, int n_rows, const void* gate, int64_t gate_stride, void* stream);
+
 /* Softmax attention of every token over the cached latent rows of its sequence:
  *   score(t, h, j) = qf[t, h] . pool[row(seq[t], j)]   for  max(0, pos[t] - window + 1) <= j <= pos[t]  (window 0: all j <= pos)
  *   out[t, h]      = sum_j softmax_j(score) * pool[row][0 : rank]            (storage type, [T, H, rank])

@@ -4,9 +4,10 @@ Per token: the query goes down to a latent (RMS-normed) and up to H heads of `di
 values come from ONE shared latent row c (RMS-normed, `kv_rank` values) per token, k_h = W_uk,h c and v_h = W_uv,h c, plus an
 optional rotated key part of `rot_dim` values shared by all heads.  Only [c | rotated key part] is cached.
 
-The layer never materialises per-head keys or values: with q'_h = W_uk,h^T q_h the score q_h . k_h equals q'_h . c, and
+A step never materialises per-head keys or values: with q'_h = W_uk,h^T q_h the score q_h . k_h equals q'_h . c, and
 sum_j p_j v_h,j = W_uv,h (sum_j p_j c_j), so attention runs directly on the cached rows and its cost per cached byte grows
-with the number of heads.  Options, all parameters: a sliding window (a query at position i sees i - window < j <= i), a
+with the number of heads.  A prompt that brings its own keys does (`HipOps.latent_prompt_plan` says when): there the products per query and key
+are what costs, and dim + rot_dim + vdim are fewer than twice the rank.  Options, all parameters: a sliding window (a query at position i sees i - window < j <= i), a
 rotary table for the rotated part (first `rot_n` of its dimensions), a sigmoid output gate computed from the layer input.
 """
 import torch
@@ -41,6 +42,7 @@ class LatentAttention:
         self.q_off, self.kv_off, self.g_off = 0, q_rank, q_rank + kv_rank + rot_dim
         self.dq_norm, self.dkv_norm, self.w_uq, self.w_o = w["dq_norm"], w["dkv_norm"], w["uq"], w["o"]
         self.w_uk = w["uk"].view(heads, dim, kv_rank).contiguous()                     # q'_h = q_h @ w_uk[h]
+        self.w_uv = w["uv"].contiguous()
         self.w_uv_t = w["uv"].view(heads, vdim, kv_rank).transpose(1, 2).contiguous()  # o_h = (sum p c) @ w_uv_t[h]
 
     def __call__(self, h, batch, pool):
@@ -51,7 +53,11 @@ class LatentAttention:
         cq = ops.latent_prep(down, self.q_off, self.q_rank, self.dq_norm, self.kv_off, self.rank, self.dkv_norm, self.rot_dim,
                              self.rot_n, rope, pool, batch.slot, batch.pos, self.eps)
         q = linear(cq, self.w_uq)                                                   # [T, H (dim + rot_dim)]
+        gate = down[:, self.g_off:self.g_off + H * self.vdim] if self.gated else None
+        plan = ops.latent_prompt_plan(batch, self.window, H, self.dim, self.rot_dim, self.vdim, self.rank, self.scale)
+        if plan is not None:
+            return linear(ops.latent_prompt(q, pool, batch, plan, self.w_uk.view(H * self.dim, self.rank), self.w_uv, rope, self.scale, H, self.rot_dim,
+                                            self.rot_n, self.rank, self.page, self.window, gate), self.w_o)
         qf = ops.latent_queries(q, self.w_uk, rope, batch.pos, self.scale, H, self.dim, self.rot_dim, self.rot_n, self.rank)
         o_lat = ops.latent_attention(qf, pool, batch, self.window, self.rank, self.page)
-        gate = down[:, self.g_off:self.g_off + H * self.vdim] if self.gated else None
         return linear(ops.head_products(o_lat, self.w_uv_t, gate), self.w_o)

@@ -226,6 +226,40 @@ class HipOps:
         q_abs = _absorbed(q, w_uk)
         return self.latent_query(q, q_abs, rope, pos, scale, heads, dim, rot_dim, rot_n, rank)
 
+    def latent_prompt_plan(self, batch, window, heads, dim, rot_dim, vdim, rank, scale):
+        """What `latent_prompt` is given for this batch, or None where the attention on the latent rows is the better one or the only one.
+        Writing keys and values out costs the keys' products with w_uk and w_uv; the queries' and the results' go, and the attention costs 320 products in place
+        of 1088 per query, key and head (rank 512 + 64).  Whole layer, on the rows / this way, us, 16 heads, rank 512 + 64: runs of 65 / 300 / 1000 new tokens
+        79 / 61, 108 / 75, 177 / 111; 512 behind 512 / 1536: 131 / 96, 154 / 122; 33 behind 67, four of them 92 / 73; 512 beside three single tokens at 1000
+        (7 keys a token) 130 / 118; 128 behind 1024 (9) 98 / 96.  The line is at 4 keys a token, which also bounds what is written out; up to 64
+        tokens the products per head have a kernel of their own."""
+        if not (self.prompt_heads_kernel and scale > 0 and heads <= 1 << 12 and self.L.qsv_latent_prompt_ok(dim, rot_dim, vdim, rank, self.code)):
+            return None
+        plan = batch.key_runs(window, self.L.qsv_latent_prompt_tile_tokens()) if batch.n_tokens > 64 else None
+        return plan if plan is not None and plan[2] <= min(4 * batch.n_tokens, 1 << 23) else None
+
+    def latent_prompt(self, q, pool, batch, plan, w_uk, w_uv, rope, scale, heads, rot_dim, rot_n, rank, page, window, gate=None):
+        """q [T, heads (dim + rot_dim)] attends its runs' cached rows through w_uk [heads dim, rank] and w_uv [heads vdim, rank] -> [T, heads vdim], times
+        sigmoid(gate [T, heads vdim]) where given."""
+        runs, tiles, n_rows, longest = plan
+        T, R = q.size(0), rank + rot_dim
+        self._need(q, pool, batch.block_table, runs, tiles, w_uk, w_uv, rope)
+        assert pool.dim() == 2 and pool.size(1) == R and q.size(1) == heads * (128 + rot_dim) and w_uk.shape == w_uv.shape == (heads * 128, rank)
+        assert rope is None or (rope.dtype == torch.float32 and rope.size(-1) * 2 == rot_n)
+        rows = torch.empty((n_rows, R), dtype=self.dtype, device=q.device)
+        self.check(self.L.qsv_latent_gather(rows.data_ptr(), pool.data_ptr(), batch.block_table.data_ptr(), batch.block_table.stride(0), runs.data_ptr(), runs.size(0),
+                                            longest, n_rows, R, page, self._s()), "latent_gather")
+        k = torch.matmul(rows[:, :rank], w_uk.t())                                # [n_rows, heads dim]
+        vt = torch.matmul(w_uv, rows[:, :rank].t())                               # [heads vdim, n_rows]: keys next to each other, as the product wants them
+        out = torch.empty((T, heads * 128), dtype=self.dtype, device=q.device)
+        if gate is not None and not (gate.data_ptr() % 8 == 0 and gate.stride(0) % 4 == 0 and gate.stride(1) == 1):
+            gate = gate.contiguous()
+        assert gate is None or (gate.is_cuda and gate.shape == out.shape and gate.dtype == self.dtype)
+        self.check(self.L.qsv_latent_prompt(out.data_ptr(), q.data_ptr(), k.data_ptr(), vt.data_ptr(), rows.data_ptr(), tiles.data_ptr(), tiles.size(0),
+                                            0 if rope is None else rope.data_ptr(), scale, heads, rot_dim, rot_n, rank, int(window or 0), n_rows,
+                                            0 if gate is None else gate.data_ptr(), 0 if gate is None else gate.stride(0), self._s()), "latent_prompt")
+        return out
+
     def _head_products_fit(self, T, x, w, row):
         return (_called_plainly(x, w) and 0 < T <= 64 and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous()
                 and w.size(1) % 32 == 0 and w.size(2) % 32 == 0 and row % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 4 == 0
@@ -249,6 +283,7 @@ class HipOps:
         out = _head_products(x, w)
         return out if gate is None else self.sigmoid_gate(out, gate)
 
+    prompt_heads_kernel = True          # latent attention of prompts over the heads' own keys and values
     plain_rows_kernel = True            # exact row sizes without options: the kernel that copies whole rows into LDS
     attention_split_target = 512        # workgroups a launch of the matrix-core attention should at least have
 
@@ -1096,6 +1131,9 @@ class TorchOps:
         T = q.size(0)
         qr = _rotate(q.view(T, heads, dim + rot_dim)[..., dim:].float(), rope, pos, rot_n)
         return (torch.cat([q_abs.transpose(0, 1).float(), qr], dim=-1) * scale).contiguous()
+
+    def latent_prompt_plan(self, batch, window, heads, dim, rot_dim, vdim, rank, scale):
+        return None
 
     def latent_queries(self, q, w_uk, rope, pos, scale, heads, dim, rot_dim, rot_n, rank):
         return self.latent_query(q, _absorbed(q, w_uk), rope, pos, scale, heads, dim, rot_dim, rot_n, rank)

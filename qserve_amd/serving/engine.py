@@ -34,6 +34,7 @@ class StepBatch:
     run_off: torch.Tensor = None    # int32 [T]  index of the token within its run
     state_rd: torch.Tensor = None   # int32 [T]  two-copy state row the token's run reads (-1: the run starts its sequence)
     state_wr: torch.Tensor = None   # int32 [T]  two-copy state row to write, on the LAST token of a run (-1 elsewhere)
+    starts: list = None         # host: position of each run's first token (None: not known on the host)
     _tiles: dict = field(default_factory=dict)
     _runs: torch.Tensor = None
     _single: torch.Tensor = None    # int32 [T, 3] = (slot, token, 1) where every run is one token: the tiles of any size
@@ -74,6 +75,27 @@ class StepBatch:
             self._tiles[key] = both
         both, k = self._tiles[key], sum(1 for run in self.items if run[2] <= n)
         return both[k:], both[:k]
+
+    def key_runs(self, window, tokens_per_tile):
+        """For kernels that lay the keys of whole runs out one behind another: -> (runs int32 [n, 4] = (sequence slot, position of the first key that a
+        token of the run sees, keys, first row), tiles int32 [m, 8] = (first flat token index, tokens <= tokens_per_tile, position of the first, then
+        the run's last three, 0, 0), the longest first, rows (every run's keys padded to a multiple of 8), most keys of a run).  None where the host does not
+        know the positions or every run is one token."""
+        if self.starts is None or self._single is not None:
+            return None
+        key = ("keys", int(window or 0), int(tokens_per_tile))
+        if key not in self._tiles:
+            runs, tiles, rows = [], [], 0
+            for (slot, first, n), start in zip(self.items, self.starts):
+                lo = max(0, start - int(window) + 1) if window else 0
+                keys = start + n - lo
+                runs.append((slot, lo, keys, rows))
+                tiles += [(first + o, min(tokens_per_tile, n - o), start + o, lo, rows, keys, 0, 0) for o in range(0, n, tokens_per_tile)]
+                rows += (keys + 7) // 8 * 8
+            tiles.sort(key=lambda t: -(t[2] + t[1] - max(t[3], t[2] - int(window) + 1 if window else 0)))
+            both = upload(np.array([v for r in runs for v in r] + [v for t in tiles for v in t], dtype=np.int32), self.pos.device)
+            self._tiles[key] = (both[:4 * len(runs)].view(-1, 4), both[4 * len(runs):].view(-1, 8), rows, max(r[2] for r in runs))
+        return self._tiles[key]
 
 
 class Engine:
@@ -133,7 +155,7 @@ class Engine:
 
     def _layout_host(self, items):
         """Host side of a step's batch: extends the sequences' pages, swaps their two-copy states.  -> (everything the device needs as one
-        int32 array, see `_batch_of`; runs [(slot, first flat token, tokens)]; largest position) or None."""
+        int32 array, see `_batch_of`; runs [(slot, first flat token, tokens)]; largest position; every run's first position) or None."""
         if len({slot for slot, t in items if len(t)}) != sum(1 for _, t in items if len(t)):
             raise ValueError("a sequence appears twice in one step")
         cache, runs, cols, T, max_pos = self.cache, [], [], 0, 0
@@ -164,7 +186,7 @@ class Engine:
                 row_of[s], meta[0, s], meta[1, s] = rows, ids, slot
                 meta[2, s], meta[3, s] = np.arange(start, start + n), np.arange(n)
                 meta[4, s], meta[5, s], meta[5, first + n - 1] = rd if start else -1, -1, wr
-        return flat, runs, max_pos
+        return flat, runs, max_pos, [c[1] for c in cols]
 
     def layout(self, items):
         """items: [(slot, tokens)] -> the StepBatch of these tokens on the device (None if there are none).  Part of `execute`;
@@ -172,14 +194,14 @@ class Engine:
         host = self._layout_host(items)
         return None if host is None else self._batch_of(upload(host[0], self.device), *host[1:])
 
-    def _batch_of(self, flat, runs, max_pos):
+    def _batch_of(self, flat, runs, max_pos, starts=None):
         """The StepBatch over one int32 tensor: cache rows (int64 [T]) | token, slot, position, index in run, state row to read, state row to
         write ([6, T]) | runs ([R, 4]) | the tiles of single tokens ([R, 3], where every run is one)."""
         T, R = sum(n for _, _, n in runs), len(runs)
         meta = flat[2 * T:8 * T].view(6, T)
         return StepBatch(tokens=meta[0], seq=meta[1], pos=meta[2], slot=flat[:2 * T].view(torch.int64), block_table=self.cache.block_table(),
                          max_pos=max_pos, n_tokens=T, items=list(runs), run_off=meta[3], state_rd=meta[4], state_wr=meta[5],
-                         _runs=flat[8 * T:8 * T + 4 * R].view(R, 4), _single=flat[8 * T + 4 * R:].view(R, 3) if T == R else None)
+                         starts=starts, _runs=flat[8 * T:8 * T + 4 * R].view(R, 4), _single=flat[8 * T + 4 * R:].view(R, 3) if T == R else None)
 
     @torch.no_grad()
     def execute(self, items, want):
@@ -189,7 +211,7 @@ class Engine:
         if host is None:
             return None
         if self.decode_graphs and all(n == 1 for _, _, n in host[1]):
-            out = self._execute_graph(*host)
+            out = self._execute_graph(*host[:3])
             if out is not None:
                 if not want:
                     return None

@@ -1,0 +1,102 @@
+"""Latent attention of prompts over written-out keys and values: tile edges, later portions, windows, neighbours that hold no numbers, against float64."""
+import math
+
+import pytest
+import torch
+
+from qserve_amd.layers.ops import make_ops
+from qserve_amd.serving.engine import StepBatch
+
+pytestmark = pytest.mark.gpu
+
+
+# runs: (context, new tokens)
+@pytest.mark.parametrize("H, rank, rot_dim, rot_n", [(16, 512, 64, 64), (3, 256, 64, 22), (8, 128, 0, 0)])
+@pytest.mark.parametrize("runs, window, gated", [(((65, 65), (1, 1), (128, 128), (129, 129)), None, False), (((191, 191), (64, 64), (63, 63), (8, 7)), None, True),
+                                                 (((200, 130), (385, 128), (70, 1)), None, True), (((300, 300), (257, 129)), 37, False),
+                                                 (((700, 257), (64, 64)), 64, True), (((333, 333),), 300, False)])
+def test_prompt(H, rank, rot_dim, rot_n, runs, window, gated):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    dev = torch.device("cuda:0")
+    ops = make_ops("hip", torch.bfloat16, dev)
+    g = torch.Generator().manual_seed(rank + H + len(runs))
+    R, pages, scale = rank + rot_dim, sum((c + 63) // 64 for c, _ in runs), 1.0 / math.sqrt(128 + rot_dim)
+    order = torch.randperm(pages + 1, generator=g).tolist()
+    table = torch.full((len(runs), pages), order.pop(), dtype=torch.int32)           # (unused entries: a page of nothing)
+    pool = torch.full(((pages + 1) * 64, R), float("nan"))                           # rows that nobody wrote must not reach a result
+    keys, items, starts, pos, at = [], [], [], [], 0
+    for b, (ctx, n) in enumerate(runs):
+        rows = torch.randn(ctx, R, generator=g).bfloat16()
+        if b == 1:
+            rows[...] = float("nan")                                                 # a neighbour without numbers stays by itself
+        for i in range((ctx + 63) // 64):
+            table[b, i] = order.pop()
+            part = rows[64 * i:64 * i + 64]
+            pool[table[b, i] * 64:table[b, i] * 64 + part.size(0)] = part.float()
+        keys.append(rows.double())
+        items.append((b, at, n))
+        starts.append(ctx - n)
+        pos += range(ctx - n, ctx)
+        at += n
+    # every key and value is an element of its latent row times a power of two, so that the products with these weights are exact
+    pick = lambda: torch.stack([torch.zeros(128, rank).scatter_(1, torch.randint(0, rank, (128, 1), generator=g),       # noqa: E731
+                                                               2.0 ** torch.randint(-1, 2, (128, 1), generator=g)) for _ in range(H)])
+    uk, uv = pick(), pick()
+    q = (torch.randn(at, H, 128 + rot_dim, generator=g) * 1.5).bfloat16()
+    gate = torch.randn(at, 5 + H * 128, generator=g).bfloat16()[:, 5:] if gated else None      # (a column slice off the alignment)
+    angle = torch.rand(max(pos) + 1, max(rot_n // 2, 1), generator=g) * 6.0
+    rope = torch.stack([torch.cos(angle), torch.sin(angle)], 1).contiguous() if rot_n else None
+    batch = StepBatch(tokens=None, seq=None, pos=torch.tensor(pos, dtype=torch.int32, device=dev), slot=None, block_table=table.to(dev), max_pos=max(pos),
+                      n_tokens=at, items=items, starts=starts)
+    plan = batch.key_runs(window, ops.L.qsv_latent_prompt_tile_tokens())
+    to = lambda t: None if t is None else t.to(dev)                                  # noqa: E731
+    out = ops.latent_prompt(to(q.view(at, -1)), to(pool.bfloat16()), batch, plan, to(uk.view(-1, rank).bfloat16()), to(uv.view(-1, rank).bfloat16()), to(rope), scale,
+                            H, rot_dim, rot_n, rank, 64, window, to(gate))
+    out = out.view(at, H, 128).double().cpu()
+    qr = q.double()
+    if rot_n:
+        c, s = (rope[pos, i].double()[:, None] for i in (0, 1))
+        u, v = qr[..., 128:128 + rot_n:2].clone(), qr[..., 129:128 + rot_n:2].clone()
+        qr[..., 128:128 + rot_n:2], qr[..., 129:128 + rot_n:2] = (u * c - v * s).bfloat16().double(), (v * c + u * s).bfloat16().double()
+    for b, first, n in items:
+        if b == 1:
+            continue
+        rows, p = keys[b], torch.tensor(pos[first:first + n])
+        j = torch.arange(rows.size(0))
+        seen = (j[None] <= p[:, None]) & (j[None] > p[:, None] - (window or 1 << 30))
+        for h in range(H):
+            k = torch.cat([rows[:, :rank] @ uk[h].double().t(), rows[:, rank:]], 1)
+            v = rows[:, :rank] @ uv[h].double().t()
+            w = torch.softmax((qr[first:first + n, h] @ k.t() * scale).masked_fill(~seen, -math.inf), 1)
+            ref, spread = w @ v, ((w * w) @ (v * v)).sqrt()
+            if gated:
+                f = torch.sigmoid(gate[first:first + n, 128 * h:128 * h + 128].double())
+                ref, spread = ref * f, spread * f
+            # weights enter the second product as bfloat16 (relative 2^-9 each, independent), so may a rotated query that lies on a tie; the result is
+            # stored as bfloat16
+            bound = 2.0 ** -8 * ref.abs() + 6 * 2.0 ** -9 * spread + 1e-5
+            err = (out[first:first + n, h] - ref).abs()
+            assert (err <= bound).all(), (b, h, (err / bound).max())
+    assert torch.isfinite(out[[i for b, f, n in items if b != 1 for i in range(f, f + n)]]).all()
+
+
+@pytest.mark.parametrize("tokens, starts, taken", [((65,), (0,), True), ((64,), (0,), False), ((128, 1), (0, 40), True), ((128, 1), (0, 4000), False),
+                                                   ((1,) * 80, (0,) * 80, False), ((512,), (1536,), True), ((512,), (1544,), False)])
+def test_where_it_is_taken(tokens, starts, taken):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    dev = torch.device("cuda:0")
+    ops, at, items = make_ops("hip", torch.bfloat16, dev), 0, []
+    for b, n in enumerate(tokens):
+        items.append((b, at, n))
+        at += n
+    single = torch.zeros((at, 3), dtype=torch.int32, device=dev) if at == len(tokens) else None
+    batch = StepBatch(tokens=None, seq=None, pos=torch.zeros(at, dtype=torch.int32, device=dev), slot=None, block_table=None, max_pos=0, n_tokens=at, items=items,
+                      starts=list(starts), _single=single)
+    plan = lambda **k: ops.latent_prompt_plan(batch, None, *(k.get(n, d) for n, d in (("H", 16), ("dim", 128), ("rot", 64), ("vdim", 128), ("rank", 512), ("scale", 0.1))))   # noqa: E731
+    assert (plan() is not None) == taken
+    assert plan(dim=64) is None and plan(vdim=64) is None and plan(rot=32) is None and plan(rank=100) is None and plan(scale=-0.1) is None
+    batch.starts = None
+    batch._tiles.clear()
+    assert plan() is None

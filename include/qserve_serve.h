@@ -282,6 +282,9 @@ int qsv_expert_rows(void* out, const void* X, const int64_t* x_index, int div, c
  * QSV_ACT_NONE only): out is float. */
 int qsv_expert_slots(void* out, int float_out, const void* X, int div, const void* W, const int32_t* idx, int n, int n_experts, int rows, int K,
                      int act, float limit, const float* in_weight, void* stream);
+/* The same with a shared expert in the launch: rows 0 .. sh_n - 1 of sh_X [sh_n, sh_K] through sh_W [sh_rows, sh_K] and the same activation -> sh_out (bfloat16). */
+int qsv_expert_slots_shared(void* out, int float_out, const void* X, int div, const void* W, const int32_t* idx, int n, int n_experts, int rows, int K, int act,
+                            float limit, const float* in_weight, void* sh_out, const void* sh_X, const void* sh_W, int sh_n, int sh_rows, int sh_K, void* stream);
 /* Grouped expert product on the bf16 matrix cores (prompt phase): qsv_moe_sort orders the n slots by expert (order: sorted slot -> slot,
  * place: slot -> sorted slot, offsets [n_experts + 1]: first sorted slot of every expert; indices below 0 and from n_experts on are left out of all
  * three), and the product takes those: out[s, r] = act(W[e][r, :] . X[order ? order[s] / div : s, :]) for the sorted slots of every expert

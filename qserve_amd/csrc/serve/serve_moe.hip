@@ -512,6 +512,16 @@ struct ExpertArgs {
     int n, div, rows, K;
     float limit;
     bool wide;                       // out starts on 16 bytes
+    bool stored;                     // gated units are made from their halves as a tensor would hold them
+};
+// An expert every token goes through, of sizes of its own: X row t, out row t in bfloat16, the bits that the products and the activation give one by one.
+// W NULL: none.  Alone it took four launches, three of them at 4 - 5 us whatever they read (16 experts of 2048 x 1408 and one more, top 4, with the router,
+// 1 / 16 / 64 tokens: 42 / 77 / 85 -> 32 / 63 / 71 us; of 4096 x 2752 106 / 387 / 432 -> 91 / 369 / 409).
+struct SharedArgs {
+    void* out;
+    const bf16_t *X, *W;
+    int n, rows, K;
+    bool wide;
 };
 
 // The four waves' partial sums (through LDS), the weight on the input, the activation, the store: slot of column c by slot_of(c).
@@ -541,6 +551,10 @@ __device__ __forceinline__ void expert_finish(const ExpertArgs& a, int r0, int c
             float u[4] = {v[0], v[1], v[2], v[3]};
             int m = 4, stride = a.rows, at = n0;
             if (ACT == ACT_GLU) {
+                if (a.stored) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) u[q] = bf2f(f2bf(u[q]));
+                }
                 u[0] = glu(u[0], u[1], a.limit);
                 u[1] = glu(u[2], u[3], a.limit);
                 m = 2;
@@ -573,12 +587,32 @@ __device__ __forceinline__ void expert_finish(const ExpertArgs& a, int r0, int c
 }
 
 template <int ACT, bool FOUT>
-__global__ __launch_bounds__(NT, 2) void expert_rows_kernel(ExpertArgs a) {
+__global__ __launch_bounds__(NT, 2) void expert_rows_kernel(ExpertArgs a, SharedArgs sh) {
     __shared__ __attribute__((aligned(128))) unsigned char rings[NW * XRING];
     __shared__ unsigned short list[XLIST];
     __shared__ int listed[NW];
-    const int e = blockIdx.y, lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int r0 = blockIdx.x * XR, rows_here = min(XR, a.rows - r0);
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r0 = blockIdx.x * XR;
+    if (sh.W && blockIdx.y == 0) {                                                 // (first: it has the most inputs)
+        if (r0 >= sh.rows) return;
+        const ExpertArgs b = {sh.out, sh.X, sh.W, nullptr, nullptr, nullptr, nullptr, sh.n, 1, sh.rows, sh.K, a.limit, sh.wide, true};
+        for (int c0 = 0; c0 < sh.n; c0 += 32) {
+            const int c = min(32, sh.n - c0);
+            auto rows = [&](int i) { return sh.X + (size_t)(c0 + min(i, c - 1)) * (size_t)sh.K; };
+            auto slots = [&](int i, int64_t& slot, float&) { slot = c0 + i; };
+            if (c <= 16) {
+                v4f acc[XR / 16][1];
+                stream_products<XR / 16, 1>(sh.W + (size_t)r0 * sh.K, sh.K, min(XR, sh.rows - r0), rings + w * XRING, w, lane, rows, acc);
+                expert_finish<ACT, false, 1>(b, r0, c, rings, w, lane, slots, acc);
+            } else {
+                v4f acc[XR / 16][2];
+                stream_products<XR / 16, 2>(sh.W + (size_t)r0 * sh.K, sh.K, min(XR, sh.rows - r0), rings + w * XRING, w, lane, rows, acc);
+                expert_finish<ACT, false, 2>(b, r0, c, rings, w, lane, slots, acc);
+            }
+        }
+        return;
+    }
+    if (r0 >= a.rows) return;
+    const int e = blockIdx.y - (sh.W ? 1 : 0), rows_here = min(XR, a.rows - r0);
     const bf16_t* W0 = a.W + ((size_t)e * a.rows + r0) * (size_t)a.K;
     unsigned char* ring = rings + w * XRING;
     // `count` inputs: X row by row_of(i), output row (and weight) by slot_of(i)
@@ -701,7 +735,7 @@ extern "C" int qsv_gather_rows(void* out, const void* src, const int64_t* order,
                                     order, div, width));
     return qsv_launch_status("qsv_gather_rows");
 }
-static int launch_expert_rows(const char* what, ExpertArgs a, int n_experts, int act, bool float_out, void* stream) {
+static int launch_expert_rows(const char* what, ExpertArgs a, int n_experts, int act, bool float_out, void* stream, SharedArgs sh = {}) {
     QSV_REQUIRE(a.out && a.X && a.W && n_experts > 0 && a.rows > 0 && a.div > 0, "%s: bad arguments", what);
     QSV_REQUIRE(act == ACT_NONE || act == ACT_RELU_SQ || ((act == ACT_GLU || act == QSV_ACT_CLAMPED_GLU) && a.rows % 2 == 0), "%s: activation %d", what,
                 act);
@@ -713,25 +747,37 @@ static int launch_expert_rows(const char* what, ExpertArgs a, int n_experts, int
     QSV_REQUIRE(n_experts <= 65535, "%s: too many experts", what);
     QSV_REQUIRE(((uintptr_t)a.X | (uintptr_t)a.W) % 16 == 0, "%s: inputs and weights start on 16 bytes", what);
     a.wide = (uintptr_t)a.out % 16 == 0;
-    const dim3 grid((a.rows + XR - 1) / XR, n_experts), block(NT);
-    if (float_out) hipLaunchKernelGGL((expert_rows_kernel<ACT_NONE, true>), grid, block, 0, (hipStream_t)stream, a);
-    else if (act == ACT_RELU_SQ) hipLaunchKernelGGL((expert_rows_kernel<ACT_RELU_SQ, false>), grid, block, 0, (hipStream_t)stream, a);
-    else if (act == ACT_GLU) hipLaunchKernelGGL((expert_rows_kernel<ACT_GLU, false>), grid, block, 0, (hipStream_t)stream, a);
-    else hipLaunchKernelGGL((expert_rows_kernel<ACT_NONE, false>), grid, block, 0, (hipStream_t)stream, a);
+    const dim3 grid(((sh.W && sh.rows > a.rows ? sh.rows : a.rows) + XR - 1) / XR, n_experts + (sh.W ? 1 : 0)), block(NT);
+    if (float_out) hipLaunchKernelGGL((expert_rows_kernel<ACT_NONE, true>), grid, block, 0, (hipStream_t)stream, a, sh);
+    else if (act == ACT_RELU_SQ) hipLaunchKernelGGL((expert_rows_kernel<ACT_RELU_SQ, false>), grid, block, 0, (hipStream_t)stream, a, sh);
+    else if (act == ACT_GLU) hipLaunchKernelGGL((expert_rows_kernel<ACT_GLU, false>), grid, block, 0, (hipStream_t)stream, a, sh);
+    else hipLaunchKernelGGL((expert_rows_kernel<ACT_NONE, false>), grid, block, 0, (hipStream_t)stream, a, sh);
     return qsv_launch_status(what);
 }
 extern "C" int qsv_expert_rows(void* out, const void* X, const int64_t* x_index, int div, const void* W, const int64_t* offsets,
                                int n_experts, int rows, int K, int act, float limit, const float* in_weight, void* stream) {
     QSV_REQUIRE(offsets, "qsv_expert_rows: bad arguments");
-    const ExpertArgs a = {out, (const bf16_t*)X, (const bf16_t*)W, nullptr, x_index, offsets, in_weight, 0, div, rows, K, limit, false};
+    const ExpertArgs a = {out, (const bf16_t*)X, (const bf16_t*)W, nullptr, x_index, offsets, in_weight, 0, div, rows, K, limit, false, false};
     return launch_expert_rows("qsv_expert_rows", a, n_experts, act, false, stream);
 }
 extern "C" int qsv_expert_slots(void* out, int float_out, const void* X, int div, const void* W, const int32_t* idx, int n, int n_experts, int rows,
                                 int K, int act, float limit, const float* in_weight, void* stream) {
     QSV_REQUIRE(idx && n >= 0 && (!float_out || act == ACT_NONE), "qsv_expert_slots: bad arguments");
     if (n == 0) return QSV_OK;
-    const ExpertArgs a = {out, (const bf16_t*)X, (const bf16_t*)W, idx, nullptr, nullptr, in_weight, n, div, rows, K, limit, false};
+    const ExpertArgs a = {out, (const bf16_t*)X, (const bf16_t*)W, idx, nullptr, nullptr, in_weight, n, div, rows, K, limit, false, false};
     return launch_expert_rows("qsv_expert_slots", a, n_experts, act, float_out != 0, stream);
+}
+// ... and every token's row of X through a shared expert of sh_rows x sh_K in the same launch: sh_out [n / div, sh_rows (/ 2 for gated units)]
+extern "C" int qsv_expert_slots_shared(void* out, int float_out, const void* X, int div, const void* W, const int32_t* idx, int n, int n_experts, int rows, int K,
+                                       int act, float limit, const float* in_weight, void* sh_out, const void* sh_X, const void* sh_W, int sh_n, int sh_rows, int sh_K,
+                                       void* stream) {
+    QSV_REQUIRE(idx && n >= 0 && (!float_out || act == ACT_NONE) && sh_out && sh_X && sh_W && sh_n > 0 && sh_rows > 0 && n_experts < 65535, "qsv_expert_slots_shared: bad arguments");
+    QSV_REQUIRE(sh_K > 0 && sh_K % 8 == 0 && sh_K <= 1 << 25 && ((uintptr_t)sh_X | (uintptr_t)sh_W) % 16 == 0, "qsv_expert_slots_shared: inner width %d, rows on 16 bytes", sh_K);
+    QSV_REQUIRE(act == ACT_NONE || act == ACT_RELU_SQ || sh_rows % 2 == 0, "qsv_expert_slots_shared: %d rows of gated units", sh_rows);
+    if (n == 0) return QSV_OK;
+    const ExpertArgs a = {out, (const bf16_t*)X, (const bf16_t*)W, idx, nullptr, nullptr, in_weight, n, div, rows, K, limit, false, false};
+    return launch_expert_rows("qsv_expert_slots_shared", a, n_experts, act, float_out != 0, stream,
+                              {sh_out, (const bf16_t*)sh_X, (const bf16_t*)sh_W, sh_n, sh_rows, sh_K, (uintptr_t)sh_out % 16 == 0});
 }
 extern "C" int qsv_relu_sq(void* a, int64_t n, int dtype, void* stream) {
     QSV_REQUIRE(a && n >= 0 && n < (1ll << 31) * NT, "qsv_relu_sq: bad arguments");

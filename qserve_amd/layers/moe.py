@@ -101,6 +101,10 @@ class SigmoidMoE:
         """rows: the caller takes the experts' rows (qserve_amd.layers.ops.ExpertRows) for the routed output and sums them itself."""
         idx, wt = self.ops.moe_route(h, self.router, self.top_k, self.groups, self.keep, score="sigmoid", correction=self.correction,
                                      group_top=2, scale=self.scale)
+        if type(self.shared) is GatedFeedForward and self.shared.act == "silu":
+            both = self.ops.moe_experts_shared(h, self.up, self.down, idx, wt, self.shared.w_in, self.shared.w_down, weigh=self.weigh, rows=rows)
+            if both is not None:
+                return list(both)
         y = [self.ops.moe_experts(h, self.up, self.down, idx, wt, act="swiglu", weigh=self.weigh, rows=rows)]
         if self.shared is not None:
             y.append(self.shared(h))

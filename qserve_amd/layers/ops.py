@@ -944,10 +944,7 @@ class HipOps:
         idx = idx.to(torch.int32).contiguous()
         a = self.ACTS[act]
         ff = rows // 2 if a >= 2 else rows
-        major = self.moe_expert_major_slots
-        if major is None:
-            major = self.moe_sorted_above if max(D, ff) > 4096 else 896 if self._grouped_takes(up.size(0), rows, D, ff) else 1024
-        if self.code == BF16 and self.moe_token_slots < T * top_k <= major and D % 8 == 0 and ff % 8 == 0 and max(D, ff) <= 1 << 25:
+        if self._expert_major(T * top_k, up.size(0), rows, D, ff):
             return self._moe_experts_expert_major(h, up, down, idx, wt, a, limit, weigh, lazy)
         if T * top_k > self.moe_sorted_above or (T and max(D, top_k * ff) * 4 > 64 * 1024):     # (the per-token kernels keep a token's rows in 64 KiB of LDS)
             return self._moe_experts_sorted(h, up, down, idx, wt, a, limit, weigh, lazy)
@@ -961,6 +958,27 @@ class HipOps:
         self.check(self.L.qsv_moe_down(y.data_ptr(), act.data_ptr(), down.data_ptr(), idx.data_ptr(), w_out, T, top_k, D,
                                        ff, h.data_ptr(), up.size(0), self.code, self._s()), "moe_down")
         return y
+
+    def _expert_major(self, slots, E, rows, D, ff):
+        major = self.moe_expert_major_slots
+        if major is None:
+            major = self.moe_sorted_above if max(D, ff) > 4096 else 896 if self._grouped_takes(E, rows, D, ff) else 1024
+        return self.code == BF16 and self.moe_token_slots < slots <= major and D % 8 == 0 and ff % 8 == 0 and max(D, ff) <= 1 << 25
+
+    # Tokens up to which a shared expert joins the expert-major launches: every 32 tokens stream its rows anew, while the products apart go to the vendor
+    # beyond 64 (apart / joined, us, 64 and 100 tokens: 16 experts of 2048 x 1408 85 / 71, 100 / 80; a shared one of four times that size 101 / 91, 114 / 119)
+    moe_shared_tokens = 64
+
+    def moe_experts_shared(self, h, up, down, idx, wt, sh_up, sh_down, weigh="output", rows=False):
+        """Gated experts as moe_experts (act "swiglu") beside a shared expert sh_up [2 sff, D], sh_down [D, sff] that every token goes through, in the same
+        two launches -> (the experts' result, the shared expert's [T, D]); None where the sizes or the tokens make that the slower or an impossible way."""
+        (T, D), sff = h.shape, sh_down.size(1)
+        if not (0 < T <= self.moe_shared_tokens and self._expert_major(T * idx.size(1), up.size(0), up.size(1), D, up.size(1) // 2) and up.size(0) < 65535
+                and _called_plainly(h, sh_up, sh_down) and sff % 8 == 0 and sff <= 1 << 25 and sh_up.shape == (2 * sff, D) and sh_down.size(0) == D
+                and all(t.dtype == torch.bfloat16 and t.is_cuda and t.is_contiguous() for t in (h, sh_up, sh_down))
+                and all(t.data_ptr() % 16 == 0 for t in (sh_up, sh_down))):
+            return None
+        return self._moe_experts_expert_major(h, up, down, idx.to(torch.int32).contiguous(), wt, self.ACTS["swiglu"], 0.0, weigh, rows, (sh_up, sh_down))
 
     # More (token, expert) slots than this: sort the slots by expert and run each expert as one matrix product.  Below it the
     # per-token kernels above are used: no host synchronisation, a fixed launch sequence.
@@ -1002,7 +1020,7 @@ class HipOps:
                                           h.data_ptr(), E, self.code, self._s()), "moe_combine")
         return y
 
-    def _moe_experts_expert_major(self, h, up, down, idx, wt, a=1, limit=0.0, weigh="output", lazy=False):
+    def _moe_experts_expert_major(self, h, up, down, idx, wt, a=1, limit=0.0, weigh="output", lazy=False, shared=None):
         T, D = h.shape
         w_in, _ = self._weights_at(wt, weigh)
         E, rows, K = up.size(0), up.size(1), idx.size(1)
@@ -1013,6 +1031,15 @@ class HipOps:
         act = torch.empty((n, ff), dtype=self.dtype, device=h.device)
         ys = torch.empty((n, D), dtype=torch.float32, device=h.device)
         s = self._s()
+        if shared is not None:
+            sff = shared[1].size(1)
+            sact, sy = torch.empty((T, sff), dtype=self.dtype, device=h.device), torch.empty((T, D), dtype=self.dtype, device=h.device)
+            self.check(self.L.qsv_expert_slots_shared(act.data_ptr(), 0, h.data_ptr(), K, up.data_ptr(), idx.data_ptr(), n, E, rows, D, a, float(limit), w_in,
+                                                      sact.data_ptr(), h.data_ptr(), shared[0].data_ptr(), T, 2 * sff, D, s), "expert_slots_shared(up)")
+            self.check(self.L.qsv_expert_slots_shared(ys.data_ptr(), 1, act.data_ptr(), 1, down.data_ptr(), idx.data_ptr(), n, E, D, ff, 0, 0.0, 0,
+                                                      sy.data_ptr(), sact.data_ptr(), shared[1].data_ptr(), T, D, sff, s), "expert_slots_shared(down)")
+            y = ExpertRows(self, ys, None, wt if weigh == "output" else None, idx, h, E)
+            return (y if lazy else y.dense()), sy
         self.check(self.L.qsv_expert_slots(act.data_ptr(), 0, h.data_ptr(), K, up.data_ptr(), idx.data_ptr(), n, E, rows, D, a, float(limit),
                                            w_in, s), "expert_slots(up)")
         self.check(self.L.qsv_expert_slots(ys.data_ptr(), 1, act.data_ptr(), 1, down.data_ptr(), idx.data_ptr(), n, E, D, ff, 0, 0.0, 0, s),
@@ -1536,6 +1563,9 @@ class TorchOps:
                 prev = m[t]
             m_state[slot] = prev
         return a, b, m
+
+    def moe_experts_shared(self, h, up, down, idx, wt, sh_up, sh_down, weigh="output", rows=False):
+        return None
 
     def moe_experts(self, h, up, down, idx, wt, act="relu_sq", limit=0.0, weigh="output", rows=False):
         T, D = h.shape

@@ -55,6 +55,7 @@ SIGNATURES = {
     "qsv_moe_up": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _f, _i, _vp, _i, _vp]),
     "qsv_expert_rows": (_i, [_vp, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _i, _f, _vp, _vp]),
     "qsv_expert_slots": (_i, [_vp, _i, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _f, _vp, _vp]),
+    "qsv_expert_slots_shared": (_i, [_vp, _i, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _f, _vp, _vp, _vp, _vp, _i, _i, _i, _vp]),
     "qsv_moe_sort": (_i, [_vp, _vp, _vp, _vp, _i, _i, _vp]),
     "qsv_grouped_gemm_sorted_ok": (_i, [_i, _i, _i]),
     "qsv_grouped_gemm_sorted": (_i, [_vp, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _i, _f, _vp, _vp]),

@@ -78,7 +78,7 @@ def random_weights(cfg, dev, seed=0):
 class OpTimer:
     """HIP events around every call of the ops object's methods and of the vendor products (one step at a time)."""
     NAMES = ("embed", "add_layer_norm", "layer_norm_rows", "latent_prep", "latent_queries", "latent_prompt", "head_products", "latent_attention", "sigmoid_gate",
-             "moe_route", "moe_experts", "embed_streams", "hc_read", "hc_write", "dyt_sum_rows", "rms_pair_mean", "glu",
+             "moe_route", "moe_experts", "moe_experts_shared", "embed_streams", "hc_read", "hc_write", "dyt_sum_rows", "rms_pair_mean", "glu",
              "attention_prep", "rotate_heads", "decay", "conv_silu_unit", "recurrent_scan", "head_rms_gate", "embed_sinusoid",
              "add_rms_norm", "rms_norm_rows", "normed_attention_prep", "max_gates", "add_normed_rms_norm", "qk_norm_rope_prep", "pool_blocks",
              "min_gru_scan", "relu_sq", "embed_rms_norm", "residual_conv", "scaled_add_rms_norm", "rotate_qk", "talking_attention",

@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from qserve_amd.layers.ops import ExpertRows, make_ops
+from qserve_amd.layers.ops import ExpertRows, linear, make_ops
 
 pytestmark = pytest.mark.gpu
 
@@ -266,3 +266,27 @@ def test_router_takes_what_is_not_a_number_last_and_ties_by_index():
     assert idx.cpu()[0].tolist() == [2, 4, 0, 1, 5, 3]
     idx, _ = o.moe_route(torch.full_like(h, float("nan")).to(dev), r.to(dev), 3, 3, 2)
     assert sorted(set(idx.cpu()[0].tolist())) == sorted(idx.cpu()[0].tolist()) and idx.min() >= 0 and idx.max() < 6
+
+
+# a shared expert in the same two launches: edges of 16 / 32 tokens, narrower and wider than the others, remainders of rows and of the reduction
+@pytest.mark.parametrize("T", [1, 2, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("D, ff, sff, weigh", [(256, 128, 128, "input"), (264, 72, 200, "output"), (2048, 64, 24, "output"), (72, 136, 1408, "input")])
+def test_shared_expert_in_the_launch(ops, T, D, ff, sff, weigh):
+    E, top, g = 5, 2, torch.Generator().manual_seed(T + D)
+    mat = lambda *s: (torch.randn(*s, generator=g) / s[-1] ** 0.5).bfloat16()                              # noqa: E731
+    h, up, down, sup, sdown = torch.randn(T, D, generator=g).bfloat16(), mat(E, 2 * ff, D), mat(E, D, ff), mat(2 * sff, D), mat(D, sff)
+    idx, wt = torch.rand(T, E, generator=g).argsort(dim=1)[:, :top].int(), torch.rand(T, top, generator=g)
+    args = [t.cuda() for t in (h, up, down, idx, wt)]
+    both = ops.moe_experts_shared(*args, sup.cuda(), sdown.cuda(), weigh=weigh)
+    assert both is not None and torch.equal(both[0], ops.moe_experts(*args, act="swiglu", weigh=weigh))
+    apart = linear(ops.glu(linear(args[0], sup.cuda())), sdown.cuda())
+    assert torch.equal(both[1], apart)                                  # (these sizes go through the same stream of products: the same bits)
+
+
+def test_shared_expert_where_it_is_left_alone(ops):
+    t = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device="cuda:0")                                  # noqa: E731
+    route = lambda T: (torch.zeros(T, 2, dtype=torch.int32, device="cuda:0"), torch.zeros(T, 2, device="cuda:0"))       # noqa: E731
+    up, down = t(5, 256, 128), t(5, 128, 128)
+    for T, sup, sdown in ((65, t(256, 128), t(128, 128)), (4, t(200, 128), t(128, 100)), (4, t(256, 128).float(), t(128, 128).float()),
+                          (4, t(32769)[1:].view(256, 128), t(128, 128))):
+        assert ops.moe_experts_shared(t(T, 128), up, down, *route(T), sup, sdown) is None

@@ -234,6 +234,21 @@ int qsv_talking_mix(void* out, const float* part_o, const float* part_ml, const 
 /* o[t, i] *= sigmoid(g[t * g_stride + i]),  i < n. */
 int qsv_sigmoid_gate(void* o, const void* g, int64_t g_stride, int n_tokens, int n, int dtype, void* stream);
 
+/* Row kernels of a step that route the row they leave (bfloat16, D a multiple of 8 up to 4096, E <= 64; the router's arguments and results as in
+ * qsv_moe_route, with its bits): qsv_add_layer_norm; qsv_scaled_sum_rms_norms (the rows of h1; a and float rows per slot ys as in
+ * qsv_scaled_sum_rms_norms_slots with c NULL or not, or tokens alone); qsv_hc_write with the next sublayer's input (up to four streams). */
+int qsv_add_layer_norm_route(float* x, void* h, const void* y, const void* w, float eps, int n, int D, int32_t* idx, float* weight, const void* router,
+                             const void* bias, int renorm, int E, int top_k, int G, int keep, int score_fn, const float* correction, int group_top, float scale,
+                             void* stream);
+int qsv_scaled_sum_rms_norms_route(float* x, void* h0, void* h1, const void* a, const void* sa, const float* ys, const int32_t* slot_idx, const float* slot_weight,
+                                   int slot_top, int n_experts, const void* slot_scale, const void* c, const void* sc, const float* g0, const float* g1,
+                                   const int32_t* tokens, const void* table, float eps, int n, int D, int32_t* idx, float* weight, const void* router,
+                                   const void* bias, int renorm, int E, int top_k, int G, int keep, int score_fn, const float* correction, int group_top, float scale,
+                                   void* stream);
+int qsv_hc_write_route(float* x, const void* y, const float* mix, const float* w_out, int n, int streams, int D, void* h_next, const float* w_in_next,
+                       const void* norm_w, const void* norm_b, float alpha, int32_t* idx, float* weight, const void* router, const void* bias, int renorm, int E,
+                       int top_k, int G, int keep, int score_fn, const float* correction, int group_top, float scale, void* stream);
+
 /* Grouped top-k router: scores s = softmax(router . h[t]) over n_experts (score_fn QSV_SCORE_SOFTMAX) or sigmoid(router . h[t])
  * (QSV_SCORE_SIGMOID); the choice goes by c = s + correction (float [n_experts], may be NULL: c = s).  The experts form n_groups
  * equal groups of neighbours, a group's score is its largest c (group_top 1) or the sum of its two largest (group_top 2), only

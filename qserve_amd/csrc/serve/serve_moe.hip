@@ -3,6 +3,7 @@
 // Router scores are float from the first product to the chosen weights.  The expert kernels keep one token's input in LDS
 // and let every wave walk output rows with its lanes spread along the reduction (coalesced weight rows).
 #include "serve_common.h"
+#include "serve_route.h"
 #include "serve_stream.h"
 
 namespace {
@@ -10,19 +11,6 @@ constexpr int NT = 256;
 constexpr int NW = NT / 64;
 constexpr int MAX_EXPERTS = 1024;
 
-__device__ __forceinline__ void load8(const bf16_t* p, float (&v)[8]) {
-    const uint4 u = *(const uint4*)p;
-    const unsigned w[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        v[2 * i] = __uint_as_float(w[i] << 16);
-        v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
-    }
-}
-__device__ __forceinline__ void load8(const float* p, float (&v)[8]) {
-    const float4 a = *(const float4*)p, b = *(const float4*)(p + 4);
-    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-}
 __device__ __forceinline__ void loadv(const bf16_t* p, float (&v)[4]) {
     const uint2 u = *(const uint2*)p;
     v[0] = __uint_as_float(u.x << 16);
@@ -183,30 +171,6 @@ __global__ __launch_bounds__(NT) void moe_route_kernel(int32_t* __restrict__ idx
 // with a barrier each.  Here the four waves split the width and hold EC experts' sums for TT tokens side by side, the sums are reduced and
 // scattered over the lanes in one butterfly, and a lane finds its expert's place by counting the better ones (broadcasts, no search).
 // TT = 4 tokens share the router's rows in prompts; in steps one token per workgroup keeps more workgroups busy.
-__device__ __forceinline__ unsigned order_key(float v) {         // larger key = larger value; -0 = +0, NaN below everything
-    const unsigned u = __float_as_uint(v + 0.0f);
-    return v != v ? 0u : u >> 31 ? ~u : u | 0x80000000u;
-}
-// number of lanes j < n in `mask` whose key is larger (or equal at a lower index): unique per lane of the mask
-__device__ __forceinline__ int place_of(unsigned key, unsigned long long mask, int n, int lane) {
-    int r = 0;
-    for (int j = 0; j < n; ++j) {
-        const unsigned kj = (unsigned)__builtin_amdgcn_readlane((int)key, j);
-        r += (mask >> j & 1) && (kj > key || (kj == key && j < lane));
-    }
-    return r;
-}
-template <typename T>
-struct Piece {
-    typedef uint4 type;
-};
-struct float8 {
-    float4 a, b;
-};
-template <>
-struct Piece<float> {
-    typedef float8 type;
-};
 template <typename T, int TT, int EC>
 __global__ __launch_bounds__(NT, 2) void moe_route_wave_kernel(int32_t* __restrict__ idx, float* __restrict__ weight, const T* __restrict__ h,
                                                             const T* __restrict__ router, const T* __restrict__ bias, int renorm, int n, int D, int E,
@@ -249,62 +213,12 @@ __global__ __launch_bounds__(NT, 2) void moe_route_wave_kernel(int32_t* __restri
     __syncthreads();
     if (w >= TT || t0 + w >= (size_t)n) return;                  // wave w selects for token w (no barrier follows)
     const size_t t = t0 + w;
-    const bool mine = lane < E;
-    float s = -INFINITY;
-    if (mine) {
-        s = 0.f;
+    float s = 0.f;
+    if (lane < E) {
 #pragma unroll
         for (int o = 0; o < NW; ++o) s += part[o][w][lane];
-        if (bias) s += lane_bias;
     }
-    if (score_fn == 0) {
-        const float mx = wave_max(s);
-        s = mine ? expf(s - mx) : 0.f;
-        s *= 1.0f / wave_sum(s);
-    } else {
-        s = 1.0f / (1.0f + expf(-s));
-    }
-    const float c = mine ? (correction ? s + lane_corr : s) : 0.f;
-    unsigned long long ok = E == 64 ? ~0ull : (1ull << E) - 1;   // experts that may be chosen
-    if (keep < G) {
-        cs[w][lane] = c;
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        const int per = E / G;
-        float gs = 0.f;
-        if (lane < G) {
-            float v1 = cs[w][lane * per], v2 = -INFINITY;        // the two largest
-            for (int e = 1; e < per; ++e) {
-                const float v = cs[w][lane * per + e];
-                if (v > v1) {
-                    v2 = v1;
-                    v1 = v;
-                } else if (v > v2) {
-                    v2 = v;
-                }
-            }
-            gs = (group_top == 2 && per > 1) ? v1 + v2 : v1;
-        }
-        const unsigned long long all = G == 64 ? ~0ull : (1ull << G) - 1;
-        const int place = place_of(order_key(gs), all, G, lane);
-        const unsigned long long kept = __ballot(lane < G && place < keep);
-        ok = __ballot(mine && (kept >> (min(lane, E - 1) / per) & 1));
-    }
-    const int place = place_of(order_key(c), ok, E, lane);
-    const bool chosen = mine && (ok >> lane & 1) && place < top_k;
-    float wt = s;
-    if (renorm) {                                                // over the chosen only, summed from the best down
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        if (chosen) cs[w][place] = s;
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        float sum = 0.f;
-        for (int k = 0; k < top_k; ++k) sum += cs[w][k];
-        wt /= sum;
-    }
-    if (renorm || scale != 1.0f) wt *= scale;
-    if (chosen) {
-        idx[t * top_k + place] = lane;
-        weight[t * top_k + place] = wt;
-    }
+    select_experts(s, lane_bias, lane_corr, {idx, weight, router, bias, correction, renorm, E, top_k, G, keep, score_fn, group_top, scale}, t, cs[w], lane);
 }
 
 // Activation of the first expert product.  ACT_GLU: the weight rows come in pairs (2f = gate, 2f + 1 = up) and output f is

@@ -1,6 +1,7 @@
 // serve_rows.hip -- one-workgroup-per-token kernels of the serving engine: embedding, fused residual + layer norm, the
 // latent projections' norms + rotary + cache write, the latent query, the output gate.  Statistics and angles are float.
 #include "serve_common.h"
+#include "serve_route.h"
 
 #include <type_traits>
 
@@ -65,10 +66,13 @@ __global__ __launch_bounds__(NT) void add_layer_norm_kernel(float* __restrict__ 
 // before the first sum and stays in registers.  Bound by the row's latency in a step, by HBM in a prompt (64 / 8192 rows of 2048: 8.8 ->
 // 2.7 / 130 -> 33 us).  Y other than void: y is what a mixture of experts left per slot (float or the storage type), summed here and
 // rounded as a tensor would hold it.
-template <typename T, int P, bool ADD, typename Y = void>
+// EC other than 0: h's row goes through a router on its way out (serve_route.h).
+template <typename T, int P, bool ADD, typename Y = void, int EC = 0>
 __global__ __launch_bounds__(NT) void layer_norm_vec_kernel(T* __restrict__ h, float* __restrict__ x, const T* __restrict__ y,
-                                                            const int32_t* __restrict__ rows, const T* __restrict__ w, float eps, int D, SlotRows slots) {
+                                                            const int32_t* __restrict__ rows, const T* __restrict__ w, float eps, int D, SlotRows slots, RouteArgs route) {
     __shared__ float red[NT / 64 + 1];
+    __shared__ __attribute__((aligned(16))) RouteRoom<T, P, EC> room;
+    RouteHead<T, EC ? EC : 1> head;
     const size_t t = blockIdx.x, from = ADD ? t : rows ? (size_t)rows[t] : t;
     float v[P][4], g[P][4], old[P][4];
 #pragma unroll
@@ -82,6 +86,10 @@ __global__ __launch_bounds__(NT) void layer_norm_vec_kernel(T* __restrict__ h, f
         }
         ld4t(w, i, g[k]);
         if (ADD) ld4t(x, t * D + i, old[k]);
+    }
+    if constexpr (EC > 0) {
+        head.request(route, D);
+        __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (!std::is_void<Y>::value) {
         slot_sum4<Y>(slots, t, D, threadIdx.x * 4, NT * 4, v);
@@ -110,20 +118,25 @@ __global__ __launch_bounds__(NT) void layer_norm_vec_kernel(T* __restrict__ h, f
         for (int j = 0; j < 4; ++j) v[k][j] = (ADD ? old[k][j] : 0.f) + v[k][j] * inv * g[k][j];
         if (ADD) st4t(x, t * D + i, v[k]);
         st4t(h, t * D + i, v[k]);
+        if constexpr (EC > 0) st4t(room.row, i, v[k]);
+    }
+    if constexpr (EC > 0) {
+        __syncthreads();
+        route_row<T, EC>(route, head, t, room.row, D, room.part, room.cs);
     }
 }
 template <typename T, bool ADD>
 static void launch_layer_norm_vec(T* h, float* x, const T* y, const int32_t* rows, const T* w, float eps, int n, int D, hipStream_t stream) {
     const SlotRows none = {};
-    if (D <= NT * 4) hipLaunchKernelGGL((layer_norm_vec_kernel<T, 1, ADD>), dim3(n), dim3(NT), 0, stream, h, x, y, rows, w, eps, D, none);
-    else if (D <= NT * 8) hipLaunchKernelGGL((layer_norm_vec_kernel<T, 2, ADD>), dim3(n), dim3(NT), 0, stream, h, x, y, rows, w, eps, D, none);
-    else hipLaunchKernelGGL((layer_norm_vec_kernel<T, 4, ADD>), dim3(n), dim3(NT), 0, stream, h, x, y, rows, w, eps, D, none);
+    if (D <= NT * 4) hipLaunchKernelGGL((layer_norm_vec_kernel<T, 1, ADD>), dim3(n), dim3(NT), 0, stream, h, x, y, rows, w, eps, D, none, RouteArgs{});
+    else if (D <= NT * 8) hipLaunchKernelGGL((layer_norm_vec_kernel<T, 2, ADD>), dim3(n), dim3(NT), 0, stream, h, x, y, rows, w, eps, D, none, RouteArgs{});
+    else hipLaunchKernelGGL((layer_norm_vec_kernel<T, 4, ADD>), dim3(n), dim3(NT), 0, stream, h, x, y, rows, w, eps, D, none, RouteArgs{});
 }
 template <typename T, typename Y>
 static void launch_layer_norm_slots(T* h, float* x, const T* w, float eps, int n, int D, const SlotRows& slots, hipStream_t stream) {
-    if (D <= NT * 4) hipLaunchKernelGGL((layer_norm_vec_kernel<T, 1, true, Y>), dim3(n), dim3(NT), 0, stream, h, x, (const T*)nullptr, nullptr, w, eps, D, slots);
-    else if (D <= NT * 8) hipLaunchKernelGGL((layer_norm_vec_kernel<T, 2, true, Y>), dim3(n), dim3(NT), 0, stream, h, x, (const T*)nullptr, nullptr, w, eps, D, slots);
-    else hipLaunchKernelGGL((layer_norm_vec_kernel<T, 4, true, Y>), dim3(n), dim3(NT), 0, stream, h, x, (const T*)nullptr, nullptr, w, eps, D, slots);
+    if (D <= NT * 4) hipLaunchKernelGGL((layer_norm_vec_kernel<T, 1, true, Y>), dim3(n), dim3(NT), 0, stream, h, x, (const T*)nullptr, nullptr, w, eps, D, slots, RouteArgs{});
+    else if (D <= NT * 8) hipLaunchKernelGGL((layer_norm_vec_kernel<T, 2, true, Y>), dim3(n), dim3(NT), 0, stream, h, x, (const T*)nullptr, nullptr, w, eps, D, slots, RouteArgs{});
+    else hipLaunchKernelGGL((layer_norm_vec_kernel<T, 4, true, Y>), dim3(n), dim3(NT), 0, stream, h, x, (const T*)nullptr, nullptr, w, eps, D, slots, RouteArgs{});
 }
 static bool layer_norm_fits(const void* x, const void* h, const void* y, const void* w, int D, int dtype) {
     return D % 4 == 0 && D <= NT * 16 && fits4(x, QSV_F32) && fits4(h, dtype) && fits4(y, dtype) && fits4(w, dtype);
@@ -141,6 +154,30 @@ extern "C" int qsv_add_layer_norm(float* x, void* h, const void* y, const void* 
                  hipLaunchKernelGGL(add_layer_norm_kernel<T>, dim3(n), dim3(NT), 0, (hipStream_t)stream, x, (T*)h, (const T*)y,
                                     (const T*)w, eps, D));
     return qsv_launch_status("qsv_add_layer_norm");
+}
+
+// the same, h's rows routed in the same launch (bfloat16)
+extern "C" int qsv_add_layer_norm_route(float* x, void* h, const void* y, const void* w, float eps, int n, int D, int32_t* idx, float* weight, const void* router,
+                                        const void* bias, int renorm, int E, int top_k, int G, int keep, int score_fn, const float* correction, int group_top,
+                                        float scale, void* stream) {
+    QSV_REQUIRE(x && h && y && w && n >= 0 && D > 0 && D % 8 == 0 && layer_norm_fits(x, h, y, w, D, QSV_BF16), "qsv_add_layer_norm_route: bad arguments");
+    const RouteArgs r = {idx, weight, router, bias, correction, renorm, E, top_k, G, keep, score_fn, group_top, scale};
+    QSV_REQUIRE(route_ok(r), "qsv_add_layer_norm_route: %d experts in %d groups, %d groups kept, top %d", E, G, keep, top_k);
+    if (n == 0) return QSV_OK;
+#define QSV_LNR(P, EC)                                                                                                                             \
+    hipLaunchKernelGGL((layer_norm_vec_kernel<bf16_t, P, true, void, EC>), dim3(n), dim3(NT), 0, (hipStream_t)stream, (bf16_t*)h, x, (const bf16_t*)y, nullptr, \
+                       (const bf16_t*)w, eps, D, SlotRows{}, r)
+    if (E <= 8) {
+        if (D <= NT * 4) QSV_LNR(1, 8);
+        else if (D <= NT * 8) QSV_LNR(2, 8);
+        else QSV_LNR(4, 8);
+    } else {
+        if (D <= NT * 4) QSV_LNR(1, 16);
+        else if (D <= NT * 8) QSV_LNR(2, 16);
+        else QSV_LNR(4, 16);
+    }
+#undef QSV_LNR
+    return qsv_launch_status("qsv_add_layer_norm_route");
 }
 
 extern "C" int qsv_add_layer_norm_slots(float* x, void* h, const void* ys, int float_rows, const int32_t* place, const float* weight, const int32_t* idx, int top_k,
@@ -478,12 +515,16 @@ struct ScaledParts {
 };
 // One trip to memory: the NP parts (and, Y other than void, what a mixture of experts left per slot, summed and rounded here as a tensor would hold it,
 // scaled by slot_scale: added behind the first part) are requested before the first is used.
-template <typename T, int VPT, int NP, typename Y = void>
+// EC other than 0: the rows of the second norm go through a router on their way out (serve_route.h).
+template <typename T, int VPT, int NP, typename Y = void, int EC = 0>
 __global__ __launch_bounds__(NT) void scaled_sum_rms_norms_vec_kernel(float* __restrict__ x, T* __restrict__ h0, T* __restrict__ h1, ScaledParts p,
                                                                       const float* __restrict__ g0, const float* __restrict__ g1,
-                                                                      const int32_t* __restrict__ tokens, const T* __restrict__ table, float eps, int D, SlotRows slots) {
+                                                                      const int32_t* __restrict__ tokens, const T* __restrict__ table, float eps, int D, SlotRows slots,
+                                                                      RouteArgs route) {
     constexpr bool SLOTS = !std::is_void<Y>::value;
     __shared__ float red[NT / 64 + 1];
+    __shared__ __attribute__((aligned(16))) RouteRoom<T, VPT, EC> room;
+    RouteHead<T, EC ? EC : 1> head;
     const size_t t = blockIdx.x;
     float v[VPT][4], z[VPT][NP ? NP : 1][4], f[VPT][NP ? NP : 1][4], ysum[VPT][4], yf[VPT][4];
 #pragma unroll
@@ -502,6 +543,10 @@ __global__ __launch_bounds__(NT) void scaled_sum_rms_norms_vec_kernel(float* __r
             yf[k][0] = yf[k][1] = yf[k][2] = yf[k][3] = 1.f;
             if (p.slot_scale) ld4t((const T*)p.slot_scale, i, yf[k]);
         }
+    }
+    if constexpr (EC > 0) {
+        head.request(route, D);
+        __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (SLOTS) {
         slot_sum4<Y>(slots, t, D, threadIdx.x * 4, NT * 4, ysum);
@@ -548,7 +593,12 @@ __global__ __launch_bounds__(NT) void scaled_sum_rms_norms_vec_kernel(float* __r
 #pragma unroll
             for (int e = 0; e < 4; ++e) n[e] = v[k][e] * a[e];
             st4t(h1, t * D + i, n);
+            if constexpr (EC > 0) st4t(room.row, i, n);
         }
+    }
+    if constexpr (EC > 0) {
+        __syncthreads();
+        route_row<T, EC>(route, head, t, room.row, D, room.part, room.cs);
     }
 }
 template <typename T>
@@ -579,7 +629,7 @@ template <typename T, int NP, typename Y>
 static void launch_scaled_sum(float* x, T* h0, T* h1, const ScaledParts& p, const float* g0, const float* g1, const int32_t* tokens, const T* table, float eps, int n, int D,
                               const SlotRows& slots, hipStream_t stream) {
     const int vecs = (D / 4 + NT - 1) / NT;
-#define QSV_SSN(V) hipLaunchKernelGGL((scaled_sum_rms_norms_vec_kernel<T, V, NP, Y>), dim3(n), dim3(NT), 0, stream, x, h0, h1, p, g0, g1, tokens, table, eps, D, slots)
+#define QSV_SSN(V) hipLaunchKernelGGL((scaled_sum_rms_norms_vec_kernel<T, V, NP, Y>), dim3(n), dim3(NT), 0, stream, x, h0, h1, p, g0, g1, tokens, table, eps, D, slots, RouteArgs{})
     if (vecs <= 1) QSV_SSN(1);
     else if (vecs <= 2) QSV_SSN(2);
     else if (vecs <= 4) QSV_SSN(4);
@@ -628,6 +678,43 @@ extern "C" int qsv_scaled_sum_rms_norms_slots(float* x, void* h0, void* h1, cons
     else QSV_SLOTS(1, T);
 #undef QSV_SLOTS
     return qsv_launch_status("qsv_scaled_sum_rms_norms_slots");
+}
+
+// The same for steps (bfloat16), the rows of h1 routed in the same launch: x += sa * a + slot_scale * (the slots' sum) + sc * c with a and ys (float rows per
+// slot) given, c NULL or not; without them x <- table[tokens].
+extern "C" int qsv_scaled_sum_rms_norms_route(float* x, void* h0, void* h1, const void* a, const void* sa, const float* ys, const int32_t* slot_idx, const float* slot_weight,
+                                              int slot_top, int n_experts, const void* slot_scale, const void* c, const void* sc, const float* g0, const float* g1,
+                                              const int32_t* tokens, const void* table, float eps, int n, int D, int32_t* idx, float* weight, const void* router,
+                                              const void* bias, int renorm, int E, int top_k, int G, int keep, int score_fn, const float* correction, int group_top,
+                                              float scale, void* stream) {
+    QSV_REQUIRE(x && h0 && h1 && g0 && g1 && n >= 0 && D > 0 && D % 8 == 0 && D <= NT * 16 && (tokens ? table && !a && !ys && !c : a && ys && slot_idx && slot_top > 0 && n_experts > 0),
+                "qsv_scaled_sum_rms_norms_route: bad arguments");
+    const RouteArgs r = {idx, weight, router, bias, correction, renorm, E, top_k, G, keep, score_fn, group_top, scale};
+    QSV_REQUIRE(route_ok(r), "qsv_scaled_sum_rms_norms_route: %d experts in %d groups, %d groups kept, top %d", E, G, keep, top_k);
+    if (n == 0) return QSV_OK;
+    const ScaledParts p = {{a, c, nullptr}, {sa, sc, nullptr}, slot_scale};
+    const SlotRows slots = {ys, nullptr, slot_weight, slot_idx, slot_top, n_experts};
+#define QSV_SSR(V, NP, Y, EC)                                                                                                                       \
+    hipLaunchKernelGGL((scaled_sum_rms_norms_vec_kernel<bf16_t, V, NP, Y, EC>), dim3(n), dim3(NT), 0, (hipStream_t)stream, x, (bf16_t*)h0, (bf16_t*)h1, p, g0, g1, \
+                       tokens, (const bf16_t*)table, eps, D, slots, r)
+#define QSV_SSR_V(NP, Y, EC)                      \
+    do {                                          \
+        if (D <= NT * 4) QSV_SSR(1, NP, Y, EC);   \
+        else if (D <= NT * 8) QSV_SSR(2, NP, Y, EC); \
+        else QSV_SSR(4, NP, Y, EC);               \
+    } while (0)
+#define QSV_SSR_P(EC)                             \
+    do {                                          \
+        if (tokens) QSV_SSR_V(0, void, EC);       \
+        else if (c) QSV_SSR_V(2, float, EC);      \
+        else QSV_SSR_V(1, float, EC);             \
+    } while (0)
+    if (E <= 8) QSV_SSR_P(8);
+    else QSV_SSR_P(16);
+#undef QSV_SSR
+#undef QSV_SSR_V
+#undef QSV_SSR_P
+    return qsv_launch_status("qsv_scaled_sum_rms_norms_route");
 }
 
 template <typename T, typename TW>

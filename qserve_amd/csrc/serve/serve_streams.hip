@@ -4,6 +4,7 @@
 // sum; and two small row kernels of the same models (RMS-normed mean of two branches, gated-unit activation).
 // Streams, sums and norms are float; only what leaves for a matrix product is in the storage type.
 #include "serve_common.h"
+#include "serve_route.h"
 
 #include <type_traits>
 
@@ -181,6 +182,59 @@ __global__ __launch_bounds__(NT) void hc_write_vec_kernel(float* __restrict__ x,
     }
 }
 
+// The same for a step (bfloat16, up to four streams, a workgroup per token), the next sublayer's input routed on its way out (serve_route.h).  P: groups of four
+// columns a thread holds, all requested before the first is used.
+template <int P, int EC>
+__global__ __launch_bounds__(NT) void hc_write_route_kernel(float* __restrict__ x, const bf16_t* __restrict__ y, const float* __restrict__ mix,
+                                                            const float* __restrict__ w_out, int S, int D, bf16_t* __restrict__ h_next,
+                                                            const float* __restrict__ w_in_next, const bf16_t* __restrict__ nw,
+                                                            const bf16_t* __restrict__ nb, float alpha, RouteArgs route) {
+    __shared__ __attribute__((aligned(16))) RouteRoom<bf16_t, P, EC> room;
+    RouteHead<bf16_t, EC> head;
+    const size_t t = blockIdx.x;
+    float old[P][4][4], yv[P][4], w[P][4], b[P][4];
+#pragma unroll
+    for (int k = 0; k < P; ++k) {
+        const int i = (k * NT + threadIdx.x) * 4;
+        if (i >= D) continue;
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+            if (s < S) ld4t(x, (t * S + s) * D + i, old[k][s]);
+        ld4t(y, t * D + i, yv[k]);
+        ld4t(nw, i, w[k]);
+        ld4t(nb, i, b[k]);
+    }
+    head.request(route, D);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < P; ++k) {
+        const int i = (k * NT + threadIdx.x) * 4;
+        if (i >= D) continue;
+        float u[4] = {0.f, 0.f, 0.f, 0.f}, n[4];
+        for (int r = 0; r < S; ++r) {
+            float a[4];
+            const float wo = w_out[r], wi = w_in_next[r];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) a[j] = wo * yv[k][j];
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                if (s < S) {
+                    const float m = mix[s * S + r];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) a[j] += m * old[k][s][j];
+                }
+            st4t(x, (t * S + r) * D + i, a);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) u[j] += wi * a[j];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) n[j] = tanhf(alpha * u[j]) * w[k][j] + b[k][j];
+        st4t(h_next, t * D + i, n);
+        st4t(room.row, i, n);
+    }
+    __syncthreads();
+    route_row<bf16_t, EC>(route, head, t, room.row, D, room.part, room.cs);
+}
 template <typename T>
 __global__ __launch_bounds__(NT) void dyt_sum_rows_kernel(T* __restrict__ out, const float* __restrict__ x,
                                                           const int32_t* __restrict__ rows, const T* __restrict__ nw,
@@ -315,6 +369,32 @@ extern "C" int qsv_hc_write(float* x, const void* y, const float* mix, const flo
                      hipLaunchKernelGGL(hc_write_kernel<T>, dim3(n), dim3(NT), 0, (hipStream_t)stream, x, (const T*)y, mix, w_out,
                                         streams, D, (T*)h_next, w_in_next, (const T*)norm_w, (const T*)norm_b, alpha));
     return qsv_launch_status("qsv_hc_write");
+}
+
+// the same for a step, h_next's rows routed in the same launch (bfloat16, up to four streams)
+extern "C" int qsv_hc_write_route(float* x, const void* y, const float* mix, const float* w_out, int n, int streams, int D, void* h_next, const float* w_in_next,
+                                  const void* norm_w, const void* norm_b, float alpha, int32_t* idx, float* weight, const void* router, const void* bias, int renorm, int E,
+                                  int top_k, int G, int keep, int score_fn, const float* correction, int group_top, float scale, void* stream) {
+    QSV_REQUIRE(x && y && mix && w_out && h_next && w_in_next && norm_w && norm_b && n >= 0 && D > 0 && D % 8 == 0 && D <= NT * 16 && streams > 0 && streams <= 4,
+                "qsv_hc_write_route: bad arguments");
+    QSV_REQUIRE(fits4(x, QSV_F32) && fits4(y, QSV_BF16) && fits4(h_next, QSV_BF16) && fits4(norm_w, QSV_BF16) && fits4(norm_b, QSV_BF16), "qsv_hc_write_route: rows on four elements");
+    const RouteArgs r = {idx, weight, router, bias, correction, renorm, E, top_k, G, keep, score_fn, group_top, scale};
+    QSV_REQUIRE(route_ok(r), "qsv_hc_write_route: %d experts in %d groups, %d groups kept, top %d", E, G, keep, top_k);
+    if (n == 0) return QSV_OK;
+#define QSV_HCR(P, EC)                                                                                                                         \
+    hipLaunchKernelGGL((hc_write_route_kernel<P, EC>), dim3(n), dim3(NT), 0, (hipStream_t)stream, x, (const bf16_t*)y, mix, w_out, streams, D, (bf16_t*)h_next, \
+                       w_in_next, (const bf16_t*)norm_w, (const bf16_t*)norm_b, alpha, r)
+    if (E <= 8) {
+        if (D <= NT * 4) QSV_HCR(1, 8);
+        else if (D <= NT * 8) QSV_HCR(2, 8);
+        else QSV_HCR(4, 8);
+    } else {
+        if (D <= NT * 4) QSV_HCR(1, 16);
+        else if (D <= NT * 8) QSV_HCR(2, 16);
+        else QSV_HCR(4, 16);
+    }
+#undef QSV_HCR
+    return qsv_launch_status("qsv_hc_write_route");
 }
 
 extern "C" int qsv_hc_write_slots(float* x, const void* ys, int float_rows, const int32_t* place, const float* weight, const int32_t* idx, int top_k, int n_experts,

@@ -21,9 +21,12 @@ class GroupedTopKMoE:
         if E % self.groups or not 0 < self.keep <= self.groups or not 0 < self.top_k <= self.keep * (E // self.groups):
             raise ValueError(f"router: {E} experts, {self.groups} groups, keep {self.keep}, top {self.top_k}")
 
-    def __call__(self, h, rows=False):
-        """rows: the caller takes the experts' rows (qserve_amd.layers.ops.ExpertRows) and sums them itself."""
-        idx, wt = self.ops.moe_route(h, self.router, self.top_k, self.groups, self.keep)
+        self.routing = dict(router=self.router, top_k=self.top_k, groups=self.groups, keep=self.keep)
+
+    def __call__(self, h, rows=False, routed=None):
+        """rows: the caller takes the experts' rows (qserve_amd.layers.ops.ExpertRows) and sums them itself.  routed: what moe_route(h, **routing) returned,
+        where the kernel that made h has routed it."""
+        idx, wt = routed or self.ops.moe_route(h, **self.routing)
         return self.ops.moe_experts(h, self.up, self.down, idx, wt, rows=rows)
 
 
@@ -68,9 +71,11 @@ class TopKGatedMoE:
         if not 0 < self.top_k <= E:
             raise ValueError(f"router: {E} experts, top {self.top_k}")
 
-    def __call__(self, h, rows=False):
-        """rows: the caller takes the experts' rows (qserve_amd.layers.ops.ExpertRows) and sums them itself."""
-        idx, wt = self.ops.moe_route(h, self.router, self.top_k, 1, 1, bias=self.bias, renorm=True)
+        self.routing = dict(router=self.router, top_k=self.top_k, groups=1, keep=1, bias=self.bias, renorm=True)
+
+    def __call__(self, h, rows=False, routed=None):
+        """rows, routed: as above."""
+        idx, wt = routed or self.ops.moe_route(h, **self.routing)
         return self.ops.moe_experts(h, self.up, self.down, idx, wt, act="swiglu", rows=rows)
 
 
@@ -97,10 +102,12 @@ class SigmoidMoE:
         if E % self.groups or not 0 < self.keep <= self.groups or not 0 < self.top_k <= self.keep * (E // self.groups):
             raise ValueError(f"router: {E} experts, {self.groups} groups, keep {self.keep}, top {self.top_k}")
 
-    def __call__(self, h, rows=False):
-        """rows: the caller takes the experts' rows (qserve_amd.layers.ops.ExpertRows) for the routed output and sums them itself."""
-        idx, wt = self.ops.moe_route(h, self.router, self.top_k, self.groups, self.keep, score="sigmoid", correction=self.correction,
-                                     group_top=2, scale=self.scale)
+        self.routing = dict(router=self.router, top_k=self.top_k, groups=self.groups, keep=self.keep, score="sigmoid", correction=self.correction, group_top=2,
+                            scale=self.scale)
+
+    def __call__(self, h, rows=False, routed=None):
+        """rows: the caller takes the experts' rows (qserve_amd.layers.ops.ExpertRows) for the routed output and sums them itself.  routed: as above."""
+        idx, wt = routed or self.ops.moe_route(h, **self.routing)
         if type(self.shared) is GatedFeedForward and self.shared.act == "silu":
             both = self.ops.moe_experts_shared(h, self.up, self.down, idx, wt, self.shared.w_in, self.shared.w_down, weigh=self.weigh, rows=rows)
             if both is not None:

@@ -163,10 +163,39 @@ class HipOps:
                    "embed")
         return x, h
 
-    def add_layer_norm(self, x, y, w, eps):
+    # Rows up to which a row kernel routes what it leaves (a workgroup per token; beyond, tokens share the router's rows in a launch of their own)
+    route_rows = 512
+
+    def _routing(self, route, T, D, *on_four):
+        """route: the arguments of moe_route behind h -> (experts, weights, the row kernels' arguments), or None where the launch of its own is taken."""
+        if route is None or self.code != BF16 or not 0 < T <= self.route_rows or D % 8 or D > 4096 or not _on_four(*on_four):
+            return None
+        o = dict(bias=None, renorm=False, score="softmax", correction=None, group_top=1, scale=1.0)
+        o.update(route)
+        router, bias, corr, G, keep, top_k = o["router"], o["bias"], o["correction"], o["groups"], o["keep"], o["top_k"]
+        E = router.size(0)
+        if not (E <= 64 and G > 0 and E % G == 0 and 0 < keep <= G and 0 < top_k <= keep * (E // G) and router.shape == (E, D) and router.dtype == self.dtype
+                and router.is_cuda and router.is_contiguous() and router.data_ptr() % 16 == 0 and o["score"] in ("softmax", "sigmoid") and o["group_top"] in (1, 2)
+                and (bias is None or (bias.dtype == self.dtype and bias.numel() == E and bias.is_contiguous()))
+                and (corr is None or (corr.dtype == torch.float32 and corr.numel() == E and corr.is_contiguous()))):
+            return None
+        idx = torch.empty((T, top_k), dtype=torch.int32, device=router.device)
+        wt = torch.empty((T, top_k), dtype=torch.float32, device=router.device)
+        return idx, wt, (idx.data_ptr(), wt.data_ptr(), router.data_ptr(), 0 if bias is None else bias.data_ptr(), int(bool(o["renorm"])), E, top_k, G, keep,
+                         int(o["score"] == "sigmoid"), 0 if corr is None else corr.data_ptr(), int(o["group_top"]), float(o["scale"]), self._s())
+
+    def add_layer_norm(self, x, y, w, eps, route=None):
         """x += layer_norm(y) * w in place; returns x in the storage type.  y: a tensor or a mixture's ExpertRows (summed here, the same bits as its
-        dense())."""
+        dense()).  route: the arguments of moe_route behind h: -> (x in the storage type, its (experts, weights) or None where moe_route is to be called)."""
         h = torch.empty(x.shape, dtype=self.dtype, device=x.device)
+        if route is not None:
+            q = None if isinstance(y, ExpertRows) else self._routing(route, x.size(0), x.size(1), x, y, w)
+            if q is None:
+                return self.add_layer_norm(x, y, w, eps), None
+            self._need(x, y, w)
+            assert y.shape == x.shape and y.dtype == self.dtype and x.dtype == torch.float32 and w.dtype == self.dtype and w.numel() == x.size(1)
+            self.check(self.L.qsv_add_layer_norm_route(x.data_ptr(), h.data_ptr(), y.data_ptr(), w.data_ptr(), eps, x.size(0), x.size(1), *q[2]), "add_layer_norm_route")
+            return h, q[:2]
         if isinstance(y, ExpertRows):
             if x.size(1) % 4 == 0 and x.size(1) <= 4096 and _on_four(x, w):
                 self._need(x, w, y.ys, y.idx)
@@ -402,10 +431,22 @@ class HipOps:
                                       T, S, D, self.code, self._s()), "hc_read")
         return h
 
-    def hc_write(self, x, y, w_mix, w_out, then_read=None):
+    def hc_write(self, x, y, w_mix, w_out, then_read=None, route=None):
         """All streams rewritten in place from the sublayer's output y.  then_read = (w_in, norm) of the NEXT sublayer, if it
-        reads without a token shift: its input comes out of the same pass -> h [T, D] (else None)."""
+        reads without a token shift: its input comes out of the same pass -> h [T, D] (else None).  route (with then_read): the arguments of moe_route
+        behind h: -> (h, its (experts, weights) or None where moe_route is to be called)."""
         T, S, D = x.shape
+        if route is not None:
+            w_in, (w, b, alpha) = then_read
+            q = None if isinstance(y, ExpertRows) or S > 4 else self._routing(route, T, D, x, y, w, b)
+            if q is None:
+                return self.hc_write(x, y, w_mix, w_out, then_read), None
+            self._need(x, y, w_mix, w_out, w_in, w, b)
+            assert y.shape == (T, D) and y.dtype == self.dtype and w_mix.dtype == torch.float32 and w_mix.shape == (S, S) and w.dtype == b.dtype == self.dtype
+            h = torch.empty((T, D), dtype=self.dtype, device=x.device)
+            self.check(self.L.qsv_hc_write_route(x.data_ptr(), y.data_ptr(), w_mix.data_ptr(), w_out.data_ptr(), T, S, D, h.data_ptr(), w_in.data_ptr(), w.data_ptr(),
+                                                 b.data_ptr(), float(alpha), *q[2]), "hc_write_route")
+            return h, q[:2]
         if isinstance(y, ExpertRows):                                   # (the same bits as y.dense() gives)
             if then_read is None and D % 4 == 0 and _on_four(x):
                 self._need(x, y.ys, y.idx, w_mix, w_out)
@@ -489,11 +530,32 @@ class HipOps:
                                             dtype_code(w.dtype), float(eps), n, x.size(1), self.code, self._s()), "rms_norm_rows")
         return out
 
-    def scaled_sum_rms_norms(self, x, parts, gains, eps, tokens=None, table=None):
+    def scaled_sum_rms_norms(self, x, parts, gains, eps, tokens=None, table=None, route=None):
         """x += sum of scale * y over parts [(y, scale)] (up to three; y storage type, scale per coordinate in the storage type or None) in
         place, or, with tokens, x <- table[tokens] (+ the parts; x None: made here); -> (x, [rms_norm(x) * g in the storage type for the (up to
-        two) float gains g]), all from one statistic.  The second part may be a mixture's ExpertRows (the same bits as its dense())."""
+        two) float gains g]), all from one statistic.  The second part may be a mixture's ExpertRows (the same bits as its dense()).
+        route: the arguments of moe_route behind the second norm's rows: -> (x, norms, their (experts, weights) or None where moe_route is to be called)."""
         assert len(parts) <= 3 and len(gains) <= 2
+        if route is not None:
+            (a, sa), (e, se), (c, sc) = (list(parts) + [(None, None)] * 3)[:3]
+            T, D = (tokens.numel(), table.size(1)) if tokens is not None else x.shape
+            steps = (tokens is not None and not parts) or (tokens is None and isinstance(a, torch.Tensor) and isinstance(e, ExpertRows) and not isinstance(c, ExpertRows)
+                                                           and e.place is None and e.ys.dtype == torch.float32)
+            q = self._routing(route, T, D, x, a, sa, se, c, sc, table, *gains) if steps and len(gains) == 2 else None
+            if q is None:
+                return (*self.scaled_sum_rms_norms(x, parts, gains, eps, tokens, table), None)
+            if x is None:
+                x = torch.empty((T, D), dtype=torch.float32, device=table.device)
+            hs = [torch.empty((T, D), dtype=self.dtype, device=x.device) for _ in gains]
+            self._need(x, tokens, table, a, sa, se, c, sc, *gains, *((e.ys, e.idx, e.wt) if e is not None else ()))
+            assert x.dtype == torch.float32 and x.shape == (T, D) and all(g.dtype == torch.float32 and g.numel() == D for g in gains)
+            assert all(y is None or (y.shape == x.shape and (s is None or (s.dtype == self.dtype and s.numel() == D))) for y, s in ((a, sa), (e, se), (c, sc)))
+            at = lambda t: 0 if t is None else t.data_ptr()                          # noqa: E731
+            slots = (0, 0, 0, 0, 0) if e is None else (e.ys.data_ptr(), e.idx.data_ptr(), at(e.wt), e.idx.size(1), e.experts)
+            self.check(self.L.qsv_scaled_sum_rms_norms_route(x.data_ptr(), hs[0].data_ptr(), hs[1].data_ptr(), at(a), at(sa), *slots, at(se), at(c), at(sc), gains[0].data_ptr(),
+                                                             gains[1].data_ptr(), at(tokens), at(table) if tokens is not None else 0, float(eps), T, D, *q[2]),
+                       "scaled_sum_rms_norms_route")
+            return x, hs, q[:2]
         if any(isinstance(y, ExpertRows) for y, _ in parts):
             T, D = x.shape
             (a, sa), (e, se), (c, sc) = (list(parts) + [(None, None)] * 2)[:3]
@@ -1135,9 +1197,9 @@ class TorchOps:
         var = ((y - mu) ** 2).mean(-1, keepdim=True)
         return (y - mu) / torch.sqrt(var + eps) * w.float()
 
-    def add_layer_norm(self, x, y, w, eps):
+    def add_layer_norm(self, x, y, w, eps, route=None):
         x += self._ln(y, w, eps)
-        return x.to(self.dtype)
+        return x.to(self.dtype) if route is None else (x.to(self.dtype), None)
 
     def layer_norm_rows(self, x, rows, w, eps):
         return self._ln(x if rows is None else x[rows.long()], w, eps).to(self.dtype)
@@ -1229,7 +1291,9 @@ class TorchOps:
             prev[wr] = n[first + cnt - 1]
         return (n + (before - n) * shift.float()).to(self.dtype)
 
-    def hc_write(self, x, y, w_mix, w_out, then_read=None):
+    def hc_write(self, x, y, w_mix, w_out, then_read=None, route=None):
+        if route is not None:
+            return self.hc_write(x, y, w_mix, w_out, then_read), None
         x.copy_(torch.einsum("sr,tsd->trd", w_mix, x) + w_out[None, :, None] * y.float()[:, None, :])
         return None if then_read is None else self.hc_read(x, then_read[0], then_read[1])
 
@@ -1492,7 +1556,9 @@ class TorchOps:
     def rms_norm_rows(self, x, rows, w, eps):
         return self._rms(x if rows is None else x[rows.long()], w, eps).to(self.dtype)
 
-    def scaled_sum_rms_norms(self, x, parts, gains, eps, tokens=None, table=None):
+    def scaled_sum_rms_norms(self, x, parts, gains, eps, tokens=None, table=None, route=None):
+        if route is not None:
+            return (*self.scaled_sum_rms_norms(x, parts, gains, eps, tokens, table), None)
         if tokens is not None:
             start = table[tokens.long()].float()
             x = start if x is None else x.copy_(start)

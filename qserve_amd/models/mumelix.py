@@ -139,8 +139,13 @@ class Mumelix:
             if L["ff"] is None:
                 ops.hc_write(x, y, w_mix, w_out)
             else:                                               # the feed-forward's input comes out of the mixer's stream rewrite
-                h = ops.hc_write(x, y, w_mix, w_out, then_read=(L["hc2"][0], L["norm2"]))
-                ops.hc_write(x, L["ff"](h, rows=True), L["hc2"][1], L["hc2"][2])
+                then = (L["hc2"][0], L["norm2"])
+                if type(L["ff"]) is TopKGatedMoE:               # ... and through the router
+                    h, routed = ops.hc_write(x, y, w_mix, w_out, then_read=then, route=L["ff"].routing)
+                    y = L["ff"](h, rows=True, routed=routed)
+                else:
+                    y = L["ff"](ops.hc_write(x, y, w_mix, w_out, then_read=then), rows=True)
+                ops.hc_write(x, y, L["hc2"][1], L["hc2"][2])
             if tap is not None:
                 tap(run, x.sum(1))
         return x

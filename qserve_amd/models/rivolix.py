@@ -118,14 +118,20 @@ class Rivolix:
             L = self.layers[i]
             return [L["norm1"]] + ([L["norm2"]] if L["ff"] is not None else [])
 
-        x, hs = ops.scaled_sum_rms_norms(None, [], gains(0), self.eps, tokens=batch.tokens, table=self.embed)
+        def norms(x, parts, i, **start):                       # (a mixture's router runs in the kernel that makes its input)
+            ff = self.layers[i]["ff"] if i < n else None
+            if type(ff) is SigmoidMoE:
+                return ops.scaled_sum_rms_norms(x, parts, gains(i), self.eps, route=ff.routing, **start)
+            return (*ops.scaled_sum_rms_norms(x, parts, gains(i), self.eps, **start), None)
+
+        x, hs, routed = norms(None, [], 0, tokens=batch.tokens, table=self.embed)
         for i, L in enumerate(self.layers):
             p0, p1, s0, s1 = self.slices[i]
             parts = [(L["mixer"](hs[0], batch, pools[p0:p1], states[s0:s1]), L["ls1"])]
             if L["ff"] is not None:
-                parts += [(y, L["ls2"]) for y in L["ff"](hs[1], rows=True)]
+                parts += [(y, L["ls2"]) for y in L["ff"](hs[1], rows=True, routed=routed)]
             # the next layer's two inputs come out of the pass that adds this layer's outputs to the stream
-            _, hs = ops.scaled_sum_rms_norms(x, parts, gains(i + 1), self.eps)
+            _, hs, routed = norms(x, parts, i + 1)
             if tap is not None:
                 tap(i, x)
         return x

@@ -89,9 +89,15 @@ class Vekalorn:
         ops = self.ops
         x, h = ops.embed(batch.tokens, self.embed)
         for i, L in enumerate(self.layers):
-            h = ops.add_layer_norm(x, L["mixer"](h, batch, pools[i]), L["norm1"], self.eps)
-            if L["ff"] is not None:
-                h = ops.add_layer_norm(x, L["ff"](h, rows=True), L["norm2"], self.eps)
+            y = L["mixer"](h, batch, pools[i])
+            if type(L["ff"]) is GroupedTopKMoE:                 # its router runs in the kernel that makes its input
+                h, routed = ops.add_layer_norm(x, y, L["norm1"], self.eps, route=L["ff"].routing)
+                y = L["ff"](h, rows=True, routed=routed)
+            else:
+                h = ops.add_layer_norm(x, y, L["norm1"], self.eps)
+                y = None if L["ff"] is None else L["ff"](h, rows=True)
+            if y is not None:
+                h = ops.add_layer_norm(x, y, L["norm2"], self.eps)
             if tap is not None:
                 tap(i, x)
         return x

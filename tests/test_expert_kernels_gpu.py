@@ -290,3 +290,60 @@ def test_shared_expert_where_it_is_left_alone(ops):
     for T, sup, sdown in ((65, t(256, 128), t(128, 128)), (4, t(200, 128), t(128, 100)), (4, t(256, 128).float(), t(128, 128).float()),
                           (4, t(32769)[1:].view(256, 128), t(128, 128))):
         assert ops.moe_experts_shared(t(T, 128), up, down, *route(T), sup, sdown) is None
+
+
+# Row kernels that route the row they leave: the bits of the two launches one by one; one to four chunks of 1024 columns, parts of one, more experts than are
+# summed side by side, every option of the router.
+ROUTERS = [(16, dict(top_k=4, groups=4, keep=2)), (5, dict(top_k=2, groups=1, keep=1, bias=True, renorm=True)), (64, dict(top_k=6, groups=8, keep=3, score="sigmoid", correction=True,
+           group_top=2, scale=1.5)), (17, dict(top_k=17, groups=1, keep=1, score="sigmoid", group_top=2)), (1, dict(top_k=1, groups=1, keep=1))]
+
+
+@pytest.mark.parametrize("T, D", [(1, 8), (3, 264), (2, 1024), (64, 2048), (5, 2056), (33, 4096)])
+@pytest.mark.parametrize("E, kind", ROUTERS, ids=[str(e) for e, _ in ROUTERS])
+def test_routing_on_the_way_out(ops, T, D, E, kind):
+    g, dev = torch.Generator().manual_seed(T + D + E), "cuda:0"
+    bf = lambda *s: torch.randn(*s, generator=g).bfloat16().to(dev)                                        # noqa: E731
+    fl = lambda *s: torch.randn(*s, generator=g).to(dev)                                                   # noqa: E731
+    route = dict(kind, router=bf(E, D) * (3.0 / D ** 0.5))
+    if kind.get("bias"):
+        route["bias"] = bf(E)
+    if kind.get("correction"):
+        route["correction"] = fl(E)
+
+    def same(fused, apart, x1, x2):
+        h, (idx, wt) = fused
+        i2, w2 = ops.moe_route(apart, **route)
+        assert torch.equal(h, apart) and torch.equal(x1, x2) and torch.equal(idx, i2) and torch.equal(wt, w2)
+
+    x, y, w, b = fl(T, D), bf(T, D), bf(D), bf(D)
+    x1, x2 = x.clone(), x.clone()
+    same(ops.add_layer_norm(x1, y, w, 1e-5, route=route), ops.add_layer_norm(x2, y, w, 1e-5), x1, x2)
+    for S in (1, 2, 4):
+        s1 = fl(T, S, D)
+        s2, mix, out, then = s1.clone(), fl(S, S), fl(S), (fl(S), (w, b, 0.7))
+        same(ops.hc_write(s1, y, mix, out, then_read=then, route=route), ops.hc_write(s2, y, mix, out, then_read=then), s1, s2)
+    gains, table, tokens = [fl(D), fl(D)], bf(11, D), torch.randint(0, 11, (T,), generator=g, dtype=torch.int32).to(dev)
+    x1, hs, routed = ops.scaled_sum_rms_norms(None, [], gains, 1e-5, tokens=tokens, table=table, route=route)
+    x2, apart = ops.scaled_sum_rms_norms(None, [], gains, 1e-5, tokens=tokens, table=table)
+    assert torch.equal(hs[0], apart[0])
+    same((hs[1], routed), apart[1], x1, x2)
+    top = min(2, E)
+    idx = torch.randint(-1, E, (T, top), generator=g, dtype=torch.int32).to(dev)
+    for wt, parts in ((fl(T, top), 2), (None, 3)):
+        rows = ExpertRows(ops, fl(T * top, D), None, wt, idx, y, E)
+        ps = [(bf(T, D), bf(D)), (rows, bf(D)), (bf(T, D), bf(D))][:parts]
+        x1, x2 = x.clone(), x.clone()
+        _, hs, routed = ops.scaled_sum_rms_norms(x1, ps, gains, 1e-5, route=route)
+        _, apart = ops.scaled_sum_rms_norms(x2, ps, gains, 1e-5)
+        assert torch.equal(hs[0], apart[0])
+        same((hs[1], routed), apart[1], x1, x2)
+
+
+def test_routing_apart_where_the_rows_do_not_take_it(ops):
+    t = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device="cuda:0")                                  # noqa: E731
+    for T, D, E, kw in ((513, 64, 8, {}), (2, 4104, 8, {}), (2, 60, 4, {}), (2, 64, 65, {}), (2, 64, 8, dict(groups=3)), (2, 64, 8, dict(top_k=9))):
+        route = dict(dict(top_k=2, groups=1, keep=1), router=t(E, D)) | kw
+        assert ops.add_layer_norm(torch.zeros(T, D, device="cuda:0"), t(T, D), t(D), 1e-5, route=route)[1] is None
+    route = dict(top_k=2, groups=1, keep=1, router=t(8, 64))
+    then = (torch.zeros(5, device="cuda:0"), (t(64), t(64), 1.0))
+    assert ops.hc_write(torch.zeros(2, 5, 64, device="cuda:0"), t(2, 64), torch.zeros(5, 5, device="cuda:0"), torch.zeros(5, device="cuda:0"), then_read=then, route=route)[1] is None

@@ -117,6 +117,29 @@ __device__ __forceinline__ void st4t(float* p, size_t i, const float (&v)[4]) { 
 __device__ __forceinline__ void st4t(bf16_t* p, size_t i, const float (&v)[4]) {
     *(uint2*)(p + i) = make_uint2((unsigned)f2bf(v[0]) | ((unsigned)f2bf(v[1]) << 16), (unsigned)f2bf(v[2]) | ((unsigned)f2bf(v[3]) << 16));
 }
+// The same in two steps, request and use.  A row kernel requests every operand as it lies in memory, at a column inside the row (a lane behind its end repeats
+// the last), and converts behind `requested()`: a conversion beside its load, or in a branch that not every lane takes, makes the wave wait there, and a row
+// of a step would make one trip to memory after another.
+typedef unsigned raw2u __attribute__((ext_vector_type(2)));
+typedef float raw4f __attribute__((ext_vector_type(4)));
+template <typename T>
+struct Raw4;
+template <>
+struct Raw4<bf16_t> {
+    typedef raw2u type;
+};
+template <>
+struct Raw4<float> {
+    typedef raw4f type;
+};
+template <typename T>
+__device__ __forceinline__ typename Raw4<T>::type raw4(const T* p, size_t i) { return *(const typename Raw4<T>::type*)(p + i); }
+__device__ __forceinline__ void widen4(raw4f r, float (&v)[4]) { v[0] = r[0]; v[1] = r[1]; v[2] = r[2]; v[3] = r[3]; }
+__device__ __forceinline__ void widen4(raw2u r, float (&v)[4]) {
+    v[0] = __uint_as_float(r[0] << 16); v[1] = __uint_as_float(r[0] & 0xffff0000u);
+    v[2] = __uint_as_float(r[1] << 16); v[3] = __uint_as_float(r[1] & 0xffff0000u);
+}
+__device__ __forceinline__ void requested() { __builtin_amdgcn_sched_barrier(0); }
 // token of a workgroup where each has `chunks` of them, neighbours (one: no division, which a kernel of 3 us would notice)
 __device__ __forceinline__ unsigned token_of(unsigned block, int chunks) { return chunks == 1 ? block : block / (unsigned)chunks; }
 // an address that 4 elements of its type may be read from at once
@@ -131,36 +154,50 @@ struct SlotRows {
     const int32_t* idx;
     int top, n_experts;
 };
-// a[p] = four columns of y[t] from c + p * step on, p < P (zeros behind D).  The rows of four slots are requested together.
+// a[p] = four columns of y[t] from c + p * step on, p < P (zeros behind D).  The rows of four slots are requested together, beside their weights and indices
+// where a slot's row is its number (a row without an expert holds anything: it is taken out by value).
+template <typename Y, int P, bool PLACED>
+__device__ __forceinline__ void slot_sum4_as(const SlotRows& s, size_t t, int D, int c, int step, float (&a)[P][4]) {
+    const float* weight = s.weight ? s.weight : (const float*)s.idx;           // (none: something that can be read)
+    auto four = [&](int k0) __attribute__((always_inline)) {
+        typename Raw4<Y>::type r[4][P];
+        float w[4];
+        int e[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const size_t slot = t * s.top + min(k0 + q, s.top - 1);
+            e[q] = s.idx[slot];
+            w[q] = weight[slot];
+            const size_t row = !PLACED ? slot : (unsigned)e[q] < (unsigned)s.n_experts ? (size_t)s.place[slot] : 0;      // (no slot's row, but a row)
+#pragma unroll
+            for (int p = 0; p < P; ++p) r[q][p] = raw4((const Y*)s.ys, row * D + min(c + p * step, D - 4));
+        }
+        requested();
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const bool none = k0 + q >= s.top || (unsigned)e[q] >= (unsigned)s.n_experts;
+            const float wq = s.weight ? w[q] : 1.0f;
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                float v[4];
+                widen4(r[q][p], v);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float sum = a[p][j] + wq * v[j];
+                    a[p][j] = none || c + p * step >= D ? a[p][j] : sum;
+                }
+            }
+        }
+    };
+    four(0);                                                                   // (outside the loop, whose head waits for what the caller has requested)
+    for (int k0 = 4; k0 < s.top; k0 += 4) four(k0);
+}
 template <typename Y, int P>
 __device__ __forceinline__ void slot_sum4(const SlotRows& s, size_t t, int D, int c, int step, float (&a)[P][4]) {
 #pragma unroll
     for (int p = 0; p < P; ++p) a[p][0] = a[p][1] = a[p][2] = a[p][3] = 0.f;
-    for (int k0 = 0; k0 < s.top; k0 += 4) {
-        float v[4][P][4], w[4];
-        bool none[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const size_t slot = t * s.top + min(k0 + q, s.top - 1);
-            none[q] = k0 + q >= s.top || (unsigned)s.idx[slot] >= (unsigned)s.n_experts;
-            w[q] = s.weight ? s.weight[slot] : 1.0f;
-            const size_t row = none[q] ? 0 : s.place ? (size_t)s.place[slot] : slot;      // (no slot's row, but a row)
-#pragma unroll
-            for (int p = 0; p < P; ++p) {
-                v[q][p][0] = v[q][p][1] = v[q][p][2] = v[q][p][3] = 0.f;
-                if (c + p * step < D) ld4t((const Y*)s.ys, row * D + c + p * step, v[q][p]);
-            }
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int p = 0; p < P; ++p)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float sum = a[p][j] + w[q] * v[q][p][j];
-                    a[p][j] = none[q] ? a[p][j] : sum;
-                }
-    }
+    if (s.place) slot_sum4_as<Y, P, true>(s, t, D, c, step, a);
+    else slot_sum4_as<Y, P, false>(s, t, D, c, step, a);
 }
 
 // ... as a tensor of the storage type would hold it

@@ -75,25 +75,30 @@ __global__ __launch_bounds__(NT) void layer_norm_vec_kernel(T* __restrict__ h, f
     RouteHead<T, EC ? EC : 1> head;
     const size_t t = blockIdx.x, from = ADD ? t : rows ? (size_t)rows[t] : t;
     float v[P][4], g[P][4], old[P][4];
+    typename Raw4<T>::type ry[P], rg[P];
+    raw4f rx[P];
 #pragma unroll
     for (int k = 0; k < P; ++k) {
-        const int i = (k * NT + threadIdx.x) * 4;
-        v[k][0] = v[k][1] = v[k][2] = v[k][3] = 0.f;
-        if (i >= D) continue;
-        if constexpr (std::is_void<Y>::value) {
-            if (ADD) ld4t(y, t * D + i, v[k]);
-            else ld4t(x, from * D + i, v[k]);
-        }
-        ld4t(w, i, g[k]);
-        if (ADD) ld4t(x, t * D + i, old[k]);
+        const int at = min((k * NT + (int)threadIdx.x) * 4, D - 4);
+        if constexpr (ADD && std::is_void<Y>::value) ry[k] = raw4(y, t * D + at);
+        rx[k] = raw4(x, from * D + at);
+        rg[k] = raw4(w, at);
     }
-    if constexpr (EC > 0) {
-        head.request(route, D);
-        __builtin_amdgcn_sched_barrier(0);
-    }
+    if constexpr (EC > 0) head.request(route, D);
     if constexpr (!std::is_void<Y>::value) {
         slot_sum4<Y>(slots, t, D, threadIdx.x * 4, NT * 4, v);
         round_stored<T>(v);
+    }
+    requested();
+#pragma unroll
+    for (int k = 0; k < P; ++k) {
+        if constexpr (std::is_void<Y>::value) {
+            if constexpr (ADD) widen4(ry[k], v[k]);
+            else widen4(rx[k], v[k]);
+            if ((k * NT + (int)threadIdx.x) * 4 >= D) v[k][0] = v[k][1] = v[k][2] = v[k][3] = 0.f;
+        }
+        widen4(rx[k], old[k]);
+        widen4(rg[k], g[k]);
     }
     float s = 0.f;
 #pragma unroll
@@ -527,30 +532,58 @@ __global__ __launch_bounds__(NT) void scaled_sum_rms_norms_vec_kernel(float* __r
     RouteHead<T, EC ? EC : 1> head;
     const size_t t = blockIdx.x;
     float v[VPT][4], z[VPT][NP ? NP : 1][4], f[VPT][NP ? NP : 1][4], ysum[VPT][4], yf[VPT][4];
+    typename Raw4<T>::type rz[VPT][NP ? NP : 1], rf[VPT][NP ? NP : 1], ryf[VPT], rt[VPT];
+    raw4f rx[VPT], rg0[VPT], rg1[VPT];
+    const bool norms = h0 != nullptr, two = norms && h1 != nullptr;
+    const T* sf[NP ? NP : 1];
+#pragma unroll
+    for (int j = 0; j < NP; ++j) sf[j] = p.s[j] ? (const T*)p.s[j] : (const T*)p.y[j];      // (no scale: a row that there is)
+    const T* sy = SLOTS ? (p.slot_scale ? (const T*)p.slot_scale : (const T*)p.y[0]) : nullptr;
+    const float *first = norms ? g0 : x, *second = two ? g1 : first;
+    if (tokens) {
+        const size_t row = (size_t)tokens[t] * D;
+#pragma unroll
+        for (int k = 0; k < VPT; ++k) rt[k] = raw4(table, row + min(((int)threadIdx.x + k * NT) * 4, D - 4));
+    }
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
-        const int i = (threadIdx.x + k * NT) * 4;
-        if (i >= D) continue;
-        if (tokens) ld4t(table, (size_t)tokens[t] * D + i, v[k]);
-        else ld4t(x, t * D + i, v[k]);
+        const int at = min(((int)threadIdx.x + k * NT) * 4, D - 4);
+        if (!tokens) rx[k] = raw4(x, t * D + at);
 #pragma unroll
         for (int j = 0; j < NP; ++j) {
-            ld4t((const T*)p.y[j], t * D + i, z[k][j]);
-            f[k][j][0] = f[k][j][1] = f[k][j][2] = f[k][j][3] = 1.f;
-            if (p.s[j]) ld4t((const T*)p.s[j], i, f[k][j]);
+            rz[k][j] = raw4((const T*)p.y[j], t * D + at);
+            rf[k][j] = raw4(sf[j], at);
         }
-        if (SLOTS) {
-            yf[k][0] = yf[k][1] = yf[k][2] = yf[k][3] = 1.f;
-            if (p.slot_scale) ld4t((const T*)p.slot_scale, i, yf[k]);
-        }
+        if constexpr (SLOTS) ryf[k] = raw4(sy, at);
     }
-    if constexpr (EC > 0) {
-        head.request(route, D);
-        __builtin_amdgcn_sched_barrier(0);
-    }
+    if constexpr (EC > 0) head.request(route, D);
     if constexpr (SLOTS) {
         slot_sum4<Y>(slots, t, D, threadIdx.x * 4, NT * 4, ysum);
         round_stored<T>(ysum);
+    }
+    if constexpr (VPT <= 2) {                                        // (wider rows would hold too much)
+#pragma unroll
+        for (int k = 0; k < VPT; ++k) {
+            const int at = min(((int)threadIdx.x + k * NT) * 4, D - 4);
+            rg0[k] = raw4(first, at);
+            rg1[k] = raw4(second, at);
+        }
+    }
+    requested();
+#pragma unroll
+    for (int k = 0; k < VPT; ++k) {
+        if (tokens) widen4(rt[k], v[k]);
+        else widen4(rx[k], v[k]);
+#pragma unroll
+        for (int j = 0; j < NP; ++j) {
+            widen4(rz[k][j], z[k][j]);
+            widen4(rf[k][j], f[k][j]);
+            if (!p.s[j]) f[k][j][0] = f[k][j][1] = f[k][j][2] = f[k][j][3] = 1.f;
+        }
+        if constexpr (SLOTS) {
+            widen4(ryf[k], yf[k]);
+            if (!p.slot_scale) yf[k][0] = yf[k][1] = yf[k][2] = yf[k][3] = 1.f;
+        }
     }
     float s = 0.f;
 #pragma unroll
@@ -581,7 +614,8 @@ __global__ __launch_bounds__(NT) void scaled_sum_rms_norms_vec_kernel(float* __r
         const int i = (threadIdx.x + k * NT) * 4;
         if (i >= D) continue;
         float a[4], n[4];
-        ld4t(g0, i, a);
+        if constexpr (VPT <= 2) widen4(rg0[k], a);
+        else ld4t(g0, i, a);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             v[k][e] *= inv;
@@ -589,7 +623,8 @@ __global__ __launch_bounds__(NT) void scaled_sum_rms_norms_vec_kernel(float* __r
         }
         st4t(h0, t * D + i, n);
         if (h1) {
-            ld4t(g1, i, a);
+            if constexpr (VPT <= 2) widen4(rg1[k], a);
+            else ld4t(g1, i, a);
 #pragma unroll
             for (int e = 0; e < 4; ++e) n[e] = v[k][e] * a[e];
             st4t(h1, t * D + i, n);

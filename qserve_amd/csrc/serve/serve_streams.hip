@@ -89,9 +89,31 @@ __global__ __launch_bounds__(NT) void hc_write_kernel(float* __restrict__ x, con
 // reading kernel (8192 of 2 x 2048, shifted: 47 us against 51; 1023 of 4 x 2048 spread: 6.9 against 7.9), above 512 for the writing one, which keeps more
 // in registers (1023 of 2 x 4096: 17.6 us against 19.4).
 inline int stream_chunks(int n, int most, int D) { return n > most ? 1 : (int)(((int64_t)D + 4 * NT - 1) / (4 * NT)); }
+template <int MS, class More>
 __device__ __forceinline__ void stream_sum4(const float* __restrict__ x, const float* __restrict__ w_in, size_t t, int S, int D, int i,
-                                            float (&u)[4]) {
+                                            float (&u)[4], More more) {
     u[0] = u[1] = u[2] = u[3] = 0.f;
+    if constexpr (MS <= 4) {                                               // all at once (a stream that there is not repeats the last)
+        raw4f r[MS];
+        float w[MS];
+#pragma unroll
+        for (int s = 0; s < MS; ++s) {
+            r[s] = raw4(x, (t * S + min(s, S - 1)) * D + i);
+            w[s] = w_in[min(s, S - 1)];
+        }
+        more();
+        requested();
+#pragma unroll
+        for (int s = 0; s < MS; ++s)
+            if (s < S) {
+                float v[4];
+                widen4(r[s], v);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) u[j] += w[s] * v[j];
+            }
+        return;
+    }
+    more();
     for (int s = 0; s < S; ++s) {
         float v[4];
         ld4t(x, (t * S + s) * D + i, v);
@@ -101,7 +123,7 @@ __device__ __forceinline__ void stream_sum4(const float* __restrict__ x, const f
     }
 }
 
-template <typename T>
+template <typename T, int MS = MAX_STREAMS>
 __global__ __launch_bounds__(NT) void hc_read_vec_kernel(T* __restrict__ h, const float* __restrict__ x, const float* __restrict__ w_in,
                                                          const T* __restrict__ nw, const T* __restrict__ nb, float alpha,
                                                          const T* __restrict__ shift, float* __restrict__ prev,
@@ -110,24 +132,29 @@ __global__ __launch_bounds__(NT) void hc_read_vec_kernel(T* __restrict__ h, cons
     const size_t t = token_of(blockIdx.x, chunks);
     const bool shifted = shift != nullptr;
     const int off = shifted ? run_off[t] : 0, rd = shifted ? state_rd[t] : -1, wr = shifted ? state_wr[t] : -1;
+    const T* mus = shifted ? shift : nw;
     for (int i = ((blockIdx.x - (unsigned)t * chunks) * NT + threadIdx.x) * 4; i < D; i += chunks * NT * 4) {
         float w[4], b[4], u[4], n[4];
-        ld4t(nw, i, w);
-        ld4t(nb, i, b);
-        stream_sum4(x, w_in, t, S, D, i, u);
+        raw4f rp;
+        const auto rw = raw4(nw, i), rb = raw4(nb, i), rm = raw4(mus, i);
+        stream_sum4<MS>(x, w_in, t, S, D, i, u, [&] {                       // (behind the streams' requests)
+            if (off == 0 && rd >= 0) rp = raw4(prev, (size_t)rd * D + i);
+        });
+        widen4(rw, w);
+        widen4(rb, b);
 #pragma unroll
         for (int j = 0; j < 4; ++j) n[j] = tanhf(alpha * u[j]) * w[j] + b[j];
         if (shifted) {
             float before[4] = {0.f, 0.f, 0.f, 0.f}, mu[4];
             if (off > 0) {
-                stream_sum4(x, w_in, t - 1, S, D, i, u);
+                stream_sum4<MS>(x, w_in, t - 1, S, D, i, u, [] {});
 #pragma unroll
                 for (int j = 0; j < 4; ++j) before[j] = tanhf(alpha * u[j]) * w[j] + b[j];
             } else if (rd >= 0) {
-                ld4t(prev, (size_t)rd * D + i, before);
+                widen4(rp, before);
             }
             if (wr >= 0) st4t(prev, (size_t)wr * D + i, n);
-            ld4t(shift, i, mu);
+            widen4(rm, mu);
 #pragma unroll
             for (int j = 0; j < 4; ++j) n[j] += (before[j] - n[j]) * mu[j];
         }
@@ -136,55 +163,83 @@ __global__ __launch_bounds__(NT) void hc_read_vec_kernel(T* __restrict__ h, cons
 }
 
 // (Y other than void: y is what a mixture of experts left per slot, float or the storage type; it is summed here, and rounded as a tensor would hold it)
-template <typename T, typename Y = void>
+// MS: streams at most; up to four of them are requested at once, with the mix beside them (a stream that there is not repeats the last).
+template <typename T, typename Y = void, int MS = MAX_STREAMS>
 __global__ __launch_bounds__(NT) void hc_write_vec_kernel(float* __restrict__ x, const T* __restrict__ y, const float* __restrict__ mix,
                                                           const float* __restrict__ w_out, int S, int D, T* __restrict__ h_next,
                                                           const float* __restrict__ w_in_next, const T* __restrict__ nw,
                                                           const T* __restrict__ nb, float alpha, int chunks, SlotRows slots) {
     const size_t t = token_of(blockIdx.x, chunks);
-    for (int i = ((blockIdx.x - (unsigned)t * chunks) * NT + threadIdx.x) * 4; i < D; i += chunks * NT * 4) {
-        float old[MAX_STREAMS][4], yv[1][4], u[4] = {0.f, 0.f, 0.f, 0.f};
+    const float* w_in = h_next ? w_in_next : w_out;
+    const T *pw = h_next ? nw : y, *pb = h_next ? nb : y;              // (no next input: nothing of these is used)
+    float m[MS <= 4 ? MS : 1][MS <= 4 ? MS : 1], wo[MS <= 4 ? MS : 1], wi[MS <= 4 ? MS : 1];
+    if constexpr (MS <= 4) {
 #pragma unroll
-        for (int s = 0; s < MAX_STREAMS; ++s)
-            if (s < S) ld4t(x, (t * S + s) * D + i, old[s]);
-        if constexpr (std::is_void<Y>::value) ld4t(y, t * D + i, yv[0]);
-        else {
+        for (int r = 0; r < MS; ++r) {
+            wo[r] = w_out[min(r, S - 1)];
+            wi[r] = w_in[min(r, S - 1)];
+#pragma unroll
+            for (int a = 0; a < MS; ++a) m[a][r] = mix[min(a, S - 1) * S + min(r, S - 1)];
+        }
+    }
+    for (int i = ((blockIdx.x - (unsigned)t * chunks) * NT + threadIdx.x) * 4; i < D; i += chunks * NT * 4) {
+        raw4f rx[MS];
+        typename Raw4<T>::type ry, rw, rb;
+        float old[MS][4], yv[1][4], u[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < MS; ++q)
+            if (MS <= 4 || q < S) rx[q] = raw4(x, (t * S + min(q, S - 1)) * D + i);
+        if constexpr (std::is_void<Y>::value) {
+            ry = raw4(y, t * D + i);
+            rw = raw4(pw, i);
+            rb = raw4(pb, i);
+        } else {
             slot_sum4<Y>(slots, t, D, i, 0, yv);
             round_stored<T>(yv);
         }
-        for (int r = 0; r < S; ++r) {
+        requested();
+        if constexpr (std::is_void<Y>::value) widen4(ry, yv[0]);
+#pragma unroll
+        for (int q = 0; q < MS; ++q) widen4(rx[q], old[q]);
+        auto stream = [&](int r, auto mix_of, float wor, float wir) __attribute__((always_inline)) {
             float a[4];
-            const float wo = w_out[r];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) a[j] = wo * yv[0][j];
+            for (int j = 0; j < 4; ++j) a[j] = wor * yv[0][j];
 #pragma unroll
-            for (int s = 0; s < MAX_STREAMS; ++s)
-                if (s < S) {
-                    const float m = mix[s * S + r];
+            for (int q = 0; q < MS; ++q)
+                if (q < S) {
+                    const float mq = mix_of(q);
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) a[j] += m * old[s][j];
+                    for (int j = 0; j < 4; ++j) a[j] += mq * old[q][j];
                 }
             st4t(x, (t * S + r) * D + i, a);
             if (h_next) {
-                const float wi = w_in_next[r];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) u[j] += wi * a[j];
+                for (int j = 0; j < 4; ++j) u[j] += wir * a[j];
             }
-        }
-        if (h_next) {
-            float w[4], b[4], n[4];
-            ld4t(nw, i, w);
-            ld4t(nb, i, b);
+        };
+        if constexpr (MS <= 4) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) n[j] = tanhf(alpha * u[j]) * w[j] + b[j];
-            st4t(h_next, t * D + i, n);
+            for (int r = 0; r < MS; ++r)
+                if (r < S) stream(r, [&](int q) { return m[q][r]; }, wo[r], wi[r]);
+        } else {
+            for (int r = 0; r < S; ++r) stream(r, [&](int q) { return mix[q * S + r]; }, w_out[r], h_next ? w_in_next[r] : 0.f);
         }
+        if constexpr (std::is_void<Y>::value)
+            if (h_next) {
+                float w[4], b[4], n[4];
+                widen4(rw, w);
+                widen4(rb, b);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) n[j] = tanhf(alpha * u[j]) * w[j] + b[j];
+                st4t(h_next, t * D + i, n);
+            }
     }
 }
 
 // The same for a step (bfloat16, up to four streams, a workgroup per token), the next sublayer's input routed on its way out (serve_route.h).  P: groups of four
 // columns a thread holds, all requested before the first is used.
-template <int P, int EC>
+template <int P, int MS, int EC>
 __global__ __launch_bounds__(NT) void hc_write_route_kernel(float* __restrict__ x, const bf16_t* __restrict__ y, const float* __restrict__ mix,
                                                             const float* __restrict__ w_out, int S, int D, bf16_t* __restrict__ h_next,
                                                             const float* __restrict__ w_in_next, const bf16_t* __restrict__ nw,
@@ -192,43 +247,55 @@ __global__ __launch_bounds__(NT) void hc_write_route_kernel(float* __restrict__ 
     __shared__ __attribute__((aligned(16))) RouteRoom<bf16_t, P, EC> room;
     RouteHead<bf16_t, EC> head;
     const size_t t = blockIdx.x;
-    float old[P][4][4], yv[P][4], w[P][4], b[P][4];
+    raw4f rx[P][MS];
+    raw2u ry[P], rw[P], rb[P];
+    float m[MS][MS], wo[MS], wi[MS];
 #pragma unroll
     for (int k = 0; k < P; ++k) {
-        const int i = (k * NT + threadIdx.x) * 4;
-        if (i >= D) continue;
+        const int at = min((k * NT + (int)threadIdx.x) * 4, D - 4);
 #pragma unroll
-        for (int s = 0; s < 4; ++s)
-            if (s < S) ld4t(x, (t * S + s) * D + i, old[k][s]);
-        ld4t(y, t * D + i, yv[k]);
-        ld4t(nw, i, w[k]);
-        ld4t(nb, i, b[k]);
+        for (int q = 0; q < MS; ++q) rx[k][q] = raw4(x, (t * S + min(q, S - 1)) * D + at);
+        ry[k] = raw4(y, t * D + at);
+        rw[k] = raw4(nw, at);
+        rb[k] = raw4(nb, at);
+    }
+#pragma unroll
+    for (int r = 0; r < MS; ++r) {
+        wo[r] = w_out[min(r, S - 1)];
+        wi[r] = w_in_next[min(r, S - 1)];
+#pragma unroll
+        for (int q = 0; q < MS; ++q) m[q][r] = mix[min(q, S - 1) * S + min(r, S - 1)];
     }
     head.request(route, D);
-    __builtin_amdgcn_sched_barrier(0);
+    requested();
 #pragma unroll
     for (int k = 0; k < P; ++k) {
         const int i = (k * NT + threadIdx.x) * 4;
         if (i >= D) continue;
-        float u[4] = {0.f, 0.f, 0.f, 0.f}, n[4];
-        for (int r = 0; r < S; ++r) {
+        float old[MS][4], yv[4], w[4], b[4], u[4] = {0.f, 0.f, 0.f, 0.f}, n[4];
+#pragma unroll
+        for (int q = 0; q < MS; ++q) widen4(rx[k][q], old[q]);
+        widen4(ry[k], yv);
+        widen4(rw[k], w);
+        widen4(rb[k], b);
+#pragma unroll
+        for (int r = 0; r < MS; ++r) {
+            if (r >= S) continue;
             float a[4];
-            const float wo = w_out[r], wi = w_in_next[r];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) a[j] = wo * yv[k][j];
+            for (int j = 0; j < 4; ++j) a[j] = wo[r] * yv[j];
 #pragma unroll
-            for (int s = 0; s < 4; ++s)
-                if (s < S) {
-                    const float m = mix[s * S + r];
+            for (int q = 0; q < MS; ++q)
+                if (q < S) {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) a[j] += m * old[k][s][j];
+                    for (int j = 0; j < 4; ++j) a[j] += m[q][r] * old[q][j];
                 }
             st4t(x, (t * S + r) * D + i, a);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) u[j] += wi * a[j];
+            for (int j = 0; j < 4; ++j) u[j] += wi[r] * a[j];
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) n[j] = tanhf(alpha * u[j]) * w[k][j] + b[k][j];
+        for (int j = 0; j < 4; ++j) n[j] = tanhf(alpha * u[j]) * w[j] + b[j];
         st4t(h_next, t * D + i, n);
         st4t(room.row, i, n);
     }
@@ -247,14 +314,78 @@ __global__ __launch_bounds__(NT) void dyt_sum_rows_kernel(T* __restrict__ out, c
         st(out, r * D + i, tanhf(alpha * u) * ld(nw, i) + ld(nb, i));
     }
 }
+// The same for widths that are multiples of four and up to four streams: a thread's four columns in one trip to memory, `chunks` workgroups per row.
+template <typename T, int MS>
+__global__ __launch_bounds__(NT) void dyt_sum_rows_vec_kernel(T* __restrict__ out, const float* __restrict__ x, const int32_t* __restrict__ rows,
+                                                              const T* __restrict__ nw, const T* __restrict__ nb, float alpha, int S, int D, int chunks) {
+    const size_t r = token_of(blockIdx.x, chunks);
+    const int i = ((blockIdx.x - (unsigned)r * chunks) * NT + threadIdx.x) * 4;
+    if (i >= D) return;
+    const auto rw = raw4(nw, i), rb = raw4(nb, i);
+    const size_t t = rows ? (size_t)rows[r] : r;
+    raw4f rx[MS];
+#pragma unroll
+    for (int s = 0; s < MS; ++s) rx[s] = raw4(x, (t * S + min(s, S - 1)) * D + i);
+    requested();
+    float u[4] = {0.f, 0.f, 0.f, 0.f}, w[4], b[4], n[4];
+#pragma unroll
+    for (int s = 0; s < MS; ++s)
+        if (s < S) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) u[j] += rx[s][j];
+        }
+    widen4(rw, w);
+    widen4(rb, b);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) n[j] = tanhf(alpha * u[j]) * w[j] + b[j];
+    st4t(out, r * D + i, n);
+}
 
 // out[t] = (a[t] / rms(a[t]) * wa + b[t] / rms(b[t]) * wb) / 2
-template <typename T, bool VEC>
+// P other than 0: rows of up to 1024 P elements, a multiple of four, read once.
+template <typename T, bool VEC, int P>
 __global__ __launch_bounds__(NT) void rms_pair_mean_kernel(T* __restrict__ out, const T* __restrict__ a, const T* __restrict__ wa,
                                                            const T* __restrict__ b, const T* __restrict__ wb, float eps, int D) {
     __shared__ float red[NT / 64 + 1];
     const size_t t = blockIdx.x;
     float sa = 0.f, sb = 0.f;
+    if constexpr (P > 0) {
+        typename Raw4<T>::type ra[P], rb[P], rwa[P], rwb[P];
+#pragma unroll
+        for (int k = 0; k < P; ++k) {
+            const int at = min((k * NT + (int)threadIdx.x) * 4, D - 4);
+            ra[k] = raw4(a, t * D + at);
+            rb[k] = raw4(b, t * D + at);
+            rwa[k] = raw4(wa, at);
+            rwb[k] = raw4(wb, at);
+        }
+        requested();
+        float u[P][4], v[P][4], wu[4], wv[4], y[4];
+#pragma unroll
+        for (int k = 0; k < P; ++k) {
+            widen4(ra[k], u[k]);
+            widen4(rb[k], v[k]);
+            if ((k * NT + (int)threadIdx.x) * 4 >= D) continue;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                sa += u[k][j] * u[k][j];
+                sb += v[k][j] * v[k][j];
+            }
+        }
+        const float ia = 1.0f / sqrtf(block_sum<NT>(sa, red) / (float)D + eps);
+        const float ib = 1.0f / sqrtf(block_sum<NT>(sb, red) / (float)D + eps);
+#pragma unroll
+        for (int k = 0; k < P; ++k) {
+            const int i = (k * NT + (int)threadIdx.x) * 4;
+            if (i >= D) continue;
+            widen4(rwa[k], wu);
+            widen4(rwb[k], wv);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) y[j] = 0.5f * (u[k][j] * ia * wu[j] + v[k][j] * ib * wv[j]);
+            st4t(out, t * D + i, y);
+        }
+        return;
+    }
     if (VEC) {                                                           // D % 4 == 0
         for (int i = threadIdx.x * 4; i < D; i += NT * 4) {
             float u[4], v[4];
@@ -341,15 +472,20 @@ extern "C" int qsv_hc_read(void* h, const float* x, const float* w_in, const voi
     QSV_REQUIRE(!shift || (prev && run_off && state_rd && state_wr), "qsv_hc_read: token shift without its state");
     if (n == 0) return QSV_OK;
     const int chunks = stream_chunks(n, 1023, D);
-    if (D % 4 == 0)
-        QSV_DISPATCH(dtype, "qsv_hc_read",
-                     hipLaunchKernelGGL(hc_read_vec_kernel<T>, dim3((unsigned)(chunks * n)), dim3(NT), 0, (hipStream_t)stream, (T*)h, x, w_in,
-                                        (const T*)norm_w, (const T*)norm_b, alpha, (const T*)shift, prev, run_off, state_rd, state_wr,
-                                        streams, D, chunks));
-    else
+    if (D % 4 == 0) {
+#define QSV_HCRD(MS)                                                                                                                           \
+    QSV_DISPATCH(dtype, "qsv_hc_read",                                                                                                        \
+                 hipLaunchKernelGGL((hc_read_vec_kernel<T, MS>), dim3((unsigned)(chunks * n)), dim3(NT), 0, (hipStream_t)stream, (T*)h, x, w_in,       \
+                                    (const T*)norm_w, (const T*)norm_b, alpha, (const T*)shift, prev, run_off, state_rd, state_wr, streams, D, chunks))
+        if (streams <= 2) QSV_HCRD(2);
+        else if (streams <= 4) QSV_HCRD(4);
+        else QSV_HCRD(MAX_STREAMS);
+#undef QSV_HCRD
+    } else {
         QSV_DISPATCH(dtype, "qsv_hc_read",
                      hipLaunchKernelGGL(hc_read_kernel<T>, dim3(n), dim3(NT), 0, (hipStream_t)stream, (T*)h, x, w_in, (const T*)norm_w,
                                         (const T*)norm_b, alpha, (const T*)shift, prev, run_off, state_rd, state_wr, streams, D));
+    }
     return qsv_launch_status("qsv_hc_read");
 }
 
@@ -360,14 +496,20 @@ extern "C" int qsv_hc_write(float* x, const void* y, const float* mix, const flo
     QSV_REQUIRE(streams > 0 && streams <= MAX_STREAMS, "qsv_hc_write: %d streams (at most %d)", streams, MAX_STREAMS);
     if (n == 0) return QSV_OK;
     const int chunks = stream_chunks(n, 512, D);
-    if (D % 4 == 0)
-        QSV_DISPATCH(dtype, "qsv_hc_write",
-                     hipLaunchKernelGGL(hc_write_vec_kernel<T>, dim3((unsigned)(chunks * n)), dim3(NT), 0, (hipStream_t)stream, x, (const T*)y, mix, w_out,
-                                        streams, D, (T*)h_next, w_in_next, (const T*)norm_w, (const T*)norm_b, alpha, chunks, SlotRows{}));
-    else
+    if (D % 4 == 0) {
+#define QSV_HCV(MS)                                                                                                                            \
+    QSV_DISPATCH(dtype, "qsv_hc_write",                                                                                                       \
+                 hipLaunchKernelGGL((hc_write_vec_kernel<T, void, MS>), dim3((unsigned)(chunks * n)), dim3(NT), 0, (hipStream_t)stream, x, (const T*)y, mix, w_out, \
+                                    streams, D, (T*)h_next, w_in_next, (const T*)norm_w, (const T*)norm_b, alpha, chunks, SlotRows{}))
+        if (streams <= 2) QSV_HCV(2);
+        else if (streams <= 4) QSV_HCV(4);
+        else QSV_HCV(MAX_STREAMS);
+#undef QSV_HCV
+    } else {
         QSV_DISPATCH(dtype, "qsv_hc_write",
                      hipLaunchKernelGGL(hc_write_kernel<T>, dim3(n), dim3(NT), 0, (hipStream_t)stream, x, (const T*)y, mix, w_out,
                                         streams, D, (T*)h_next, w_in_next, (const T*)norm_w, (const T*)norm_b, alpha));
+    }
     return qsv_launch_status("qsv_hc_write");
 }
 
@@ -381,19 +523,21 @@ extern "C" int qsv_hc_write_route(float* x, const void* y, const float* mix, con
     const RouteArgs r = {idx, weight, router, bias, correction, renorm, E, top_k, G, keep, score_fn, group_top, scale};
     QSV_REQUIRE(route_ok(r), "qsv_hc_write_route: %d experts in %d groups, %d groups kept, top %d", E, G, keep, top_k);
     if (n == 0) return QSV_OK;
-#define QSV_HCR(P, EC)                                                                                                                         \
-    hipLaunchKernelGGL((hc_write_route_kernel<P, EC>), dim3(n), dim3(NT), 0, (hipStream_t)stream, x, (const bf16_t*)y, mix, w_out, streams, D, (bf16_t*)h_next, \
+#define QSV_HCR(P, MS, EC)                                                                                                                     \
+    hipLaunchKernelGGL((hc_write_route_kernel<P, MS, EC>), dim3(n), dim3(NT), 0, (hipStream_t)stream, x, (const bf16_t*)y, mix, w_out, streams, D, (bf16_t*)h_next, \
                        w_in_next, (const bf16_t*)norm_w, (const bf16_t*)norm_b, alpha, r)
-    if (E <= 8) {
-        if (D <= NT * 4) QSV_HCR(1, 8);
-        else if (D <= NT * 8) QSV_HCR(2, 8);
-        else QSV_HCR(4, 8);
-    } else {
-        if (D <= NT * 4) QSV_HCR(1, 16);
-        else if (D <= NT * 8) QSV_HCR(2, 16);
-        else QSV_HCR(4, 16);
-    }
+#define QSV_HCR_P(MS, EC)                         \
+    do {                                          \
+        if (D <= NT * 4) QSV_HCR(1, MS, EC);      \
+        else if (D <= NT * 8) QSV_HCR(2, MS, EC); \
+        else QSV_HCR(4, MS, EC);                  \
+    } while (0)
+    if (streams <= 2 && E <= 8) QSV_HCR_P(2, 8);
+    else if (streams <= 2) QSV_HCR_P(2, 16);
+    else if (E <= 8) QSV_HCR_P(4, 8);
+    else QSV_HCR_P(4, 16);
 #undef QSV_HCR
+#undef QSV_HCR_P
     return qsv_launch_status("qsv_hc_write_route");
 }
 
@@ -405,13 +549,20 @@ extern "C" int qsv_hc_write_slots(float* x, const void* ys, int float_rows, cons
     if (n == 0) return QSV_OK;
     const int chunks = stream_chunks(n, 512, D);
     const SlotRows slots = {ys, place, weight, idx, top_k, n_experts};
-#define QSV_HCW(Y)                                                                                                                              \
+#define QSV_HCW(Y, MS)                                                                                                                          \
     QSV_DISPATCH(dtype, "qsv_hc_write_slots",                                                                                                   \
-                 hipLaunchKernelGGL((hc_write_vec_kernel<T, Y>), dim3((unsigned)(chunks * n)), dim3(NT), 0, (hipStream_t)stream, x, (const T*)nullptr, mix, w_out, \
+                 hipLaunchKernelGGL((hc_write_vec_kernel<T, Y, MS>), dim3((unsigned)(chunks * n)), dim3(NT), 0, (hipStream_t)stream, x, (const T*)nullptr, mix, w_out, \
                                     streams, D, (T*)nullptr, (const float*)nullptr, (const T*)nullptr, (const T*)nullptr, 0.f, chunks, slots))
-    if (float_rows) QSV_HCW(float);
-    else QSV_HCW(T);
+#define QSV_HCW_S(Y)                          \
+    do {                                      \
+        if (streams <= 2) QSV_HCW(Y, 2);      \
+        else if (streams <= 4) QSV_HCW(Y, 4); \
+        else QSV_HCW(Y, MAX_STREAMS);         \
+    } while (0)
+    if (float_rows) QSV_HCW_S(float);
+    else QSV_HCW_S(T);
 #undef QSV_HCW
+#undef QSV_HCW_S
     return qsv_launch_status("qsv_hc_write_slots");
 }
 
@@ -419,6 +570,17 @@ extern "C" int qsv_dyt_sum_rows(void* out, const float* x, const int32_t* rows, 
                                 float alpha, int n_rows, int streams, int D, int dtype, void* stream) {
     QSV_REQUIRE(out && x && norm_w && norm_b && n_rows >= 0 && D > 0 && streams > 0, "qsv_dyt_sum_rows: bad arguments");
     if (n_rows == 0) return QSV_OK;
+    const int64_t chunks = ((int64_t)D / 4 + NT - 1) / NT;
+    if (D % 4 == 0 && streams <= 4 && fits4(out, dtype) && fits4(x, QSV_F32) && fits4(norm_w, dtype) && fits4(norm_b, dtype) && chunks * n_rows < (1ll << 31)) {
+#define QSV_DSR(MS)                                                                                                                           \
+    QSV_DISPATCH(dtype, "qsv_dyt_sum_rows",                                                                                                   \
+                 hipLaunchKernelGGL((dyt_sum_rows_vec_kernel<T, MS>), dim3((unsigned)(chunks * n_rows)), dim3(NT), 0, (hipStream_t)stream, (T*)out, x, rows, \
+                                    (const T*)norm_w, (const T*)norm_b, alpha, streams, D, (int)chunks))
+        if (streams <= 2) QSV_DSR(2);
+        else QSV_DSR(4);
+#undef QSV_DSR
+        return qsv_launch_status("qsv_dyt_sum_rows");
+    }
     QSV_DISPATCH(dtype, "qsv_dyt_sum_rows",
                  hipLaunchKernelGGL(dyt_sum_rows_kernel<T>, dim3(n_rows), dim3(NT), 0, (hipStream_t)stream, (T*)out, x, rows,
                                     (const T*)norm_w, (const T*)norm_b, alpha, streams, D));
@@ -429,14 +591,16 @@ extern "C" int qsv_rms_pair_mean(void* out, const void* a, const void* wa, const
                                  int dtype, void* stream) {
     QSV_REQUIRE(out && a && wa && b && wb && n >= 0 && D > 0, "qsv_rms_pair_mean: bad arguments");
     if (n == 0) return QSV_OK;
-    if (D % 4 == 0)
-        QSV_DISPATCH(dtype, "qsv_rms_pair_mean",
-                     hipLaunchKernelGGL((rms_pair_mean_kernel<T, true>), dim3(n), dim3(NT), 0, (hipStream_t)stream, (T*)out, (const T*)a,
-                                        (const T*)wa, (const T*)b, (const T*)wb, eps, D));
-    else
-        QSV_DISPATCH(dtype, "qsv_rms_pair_mean",
-                     hipLaunchKernelGGL((rms_pair_mean_kernel<T, false>), dim3(n), dim3(NT), 0, (hipStream_t)stream, (T*)out, (const T*)a,
-                                        (const T*)wa, (const T*)b, (const T*)wb, eps, D));
+#define QSV_RPM(VEC, P)                                                                                                                       \
+    QSV_DISPATCH(dtype, "qsv_rms_pair_mean",                                                                                                  \
+                 hipLaunchKernelGGL((rms_pair_mean_kernel<T, VEC, P>), dim3(n), dim3(NT), 0, (hipStream_t)stream, (T*)out, (const T*)a, (const T*)wa, (const T*)b, \
+                                    (const T*)wb, eps, D))
+    if (D % 4) QSV_RPM(false, 0);
+    else if (D <= NT * 4) QSV_RPM(true, 1);
+    else if (D <= NT * 8) QSV_RPM(true, 2);
+    else if (D <= NT * 16) QSV_RPM(true, 4);
+    else QSV_RPM(true, 0);
+#undef QSV_RPM
     return qsv_launch_status("qsv_rms_pair_mean");
 }
 

@@ -122,6 +122,42 @@ __global__ __launch_bounds__(NT) void conv_heads_kernel(T* __restrict__ q, T* __
     }
     conv_store<V>(q, pool, a, t, c, y, query_factor(a, a.pos[t]));
 }
+// The same for a step's tokens, four channels per thread and PAST = taps - 1 known: every tap requested before the first is used.
+template <typename T, int PAST>
+__global__ __launch_bounds__(NT) void conv_heads_step_kernel(T* __restrict__ q, T* __restrict__ pool, const T* __restrict__ proj, ConvHeads a) {
+    const size_t t = blockIdx.x;
+    const int c = ((int)blockIdx.y * NT + (int)threadIdx.x) * 4;
+    if (c >= a.C) return;
+    const int i = a.run_off[t], rd = a.rd[t], wr = a.wr[t];
+    typename Raw4<T>::type rx[PAST + 1];
+    raw4f rw[PAST + 1], rh[PAST];                        // rx, rw[d]: d tokens back
+#pragma unroll
+    for (int d = 0; d <= PAST; ++d) {
+        rx[d] = raw4(proj, (t - min(d, min(i, PAST))) * (size_t)a.stride + c);
+        rw[d] = raw4(a.w, (size_t)(PAST - d) * a.C + c);
+    }
+    if (i < PAST && rd >= 0) {                           // (the same for the whole workgroup)
+#pragma unroll
+        for (int d = 1; d <= PAST; ++d) rh[d - 1] = raw4(a.hist, ((size_t)rd * PAST + min(max(PAST + i - d, 0), PAST - 1)) * a.C + c);
+    }
+    const float factor = query_factor(a, a.pos[t]);
+    requested();
+    Vec<4> y, u[PAST + 1];
+#pragma unroll
+    for (int d = 0; d <= PAST; ++d) {
+        float x[4], h[4], w[4];
+        widen4(rx[d], x);
+        widen4(rh[d > 0 ? d - 1 : 0], h);
+        widen4(rw[d], w);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            u[d].v[e] = d <= i ? x[e] : rd >= 0 ? h[e] : 0.f;
+            y.v[e] = d == 0 ? w[e] * u[d].v[e] : y.v[e] + w[e] * u[d].v[e];
+        }
+        if (wr >= 0 && d < PAST) stv<4>(a.hist, ((size_t)wr * PAST + (PAST - 1 - d)) * a.C + c, u[d]);
+    }
+    conv_store<4>(q, pool, a, t, c, y, factor);
+}
 // The same for PAST = taps - 1 known: a workgroup walks TB consecutive tokens of four channels per thread with the last PAST rows in
 // registers; rows of another run are replaced by the run's history (or zeros).
 constexpr int TB = 8;
@@ -832,6 +868,16 @@ extern "C" int qsv_conv_heads_cache(void* q, void* pool, int64_t pool_rows, cons
         else if (taps == 3) QSV_CHR(2);
         else QSV_CHR(3);
 #undef QSV_CHR
+        return qsv_launch_status("qsv_conv_heads_cache");
+    }
+    if (vec && taps >= 2 && taps <= 4) {
+        const dim3 grid(n, (a.C / 4 + NT - 1) / NT);
+#define QSV_CHS(P) \
+    QSV_DISPATCH(dtype, "qsv_conv_heads_cache", hipLaunchKernelGGL((conv_heads_step_kernel<T, P>), grid, dim3(NT), 0, (hipStream_t)stream, (T*)q, (T*)pool, (const T*)proj, a))
+        if (taps == 2) QSV_CHS(1);
+        else if (taps == 3) QSV_CHS(2);
+        else QSV_CHS(3);
+#undef QSV_CHS
         return qsv_launch_status("qsv_conv_heads_cache");
     }
 #define QSV_CH(V)                                                                                                                      \

@@ -23,6 +23,30 @@ __global__ __launch_bounds__(NT) void decay_kernel(float* __restrict__ out, cons
     }
 }
 
+// The same, four channels per thread, `chunks` workgroups per token.
+template <typename T>
+__global__ __launch_bounds__(NT) void decay_vec_kernel(float* __restrict__ out, const T* __restrict__ z, int64_t z_stride, const T* __restrict__ bias,
+                                                       const float* __restrict__ a_log, float inv_tau, int dim, int n, int chunks) {
+    const size_t t = token_of(blockIdx.x, chunks);
+    const int c = ((blockIdx.x - (unsigned)t * chunks) * NT + threadIdx.x) * 4;
+    if (c >= n) return;
+    const auto rz = raw4(z, t * z_stride + c), rb = raw4(bias, c);
+    float a[4] = {0.f, 0.f, 0.f, 0.f}, v[4], b[4];
+    if (a_log) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) a[j] = a_log[(c + j) / dim];
+    }
+    requested();
+    widen4(rz, v);
+    widen4(rb, b);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        v[j] += b[j];
+        v[j] = a_log ? expf(-expf(a[j]) * softplusf(v[j])) : expf(-softplusf(-v[j]) * inv_tau);
+    }
+    st4t(out, t * n + c, v);
+}
+
 // ---- causal convolution over time + silu (act 0: no activation), unit norm of the leading groups -----------------------------------------------------
 // Workgroup = token.  Tap j (last column = the current token) reads the input taps - 1 - j tokens back: a row of this batch
 // inside the run, the sequence's history state before the run's start, zero before the sequence's start.  The last token of a
@@ -100,14 +124,25 @@ __global__ __launch_bounds__(NT) void conv_silu_unit_vec_kernel(float* __restric
     const int from = in ? c : 0;                                   // (lanes behind the end stay for the sums below)
     const int i = run_off[t], rd = state_rd[t], wr = state_wr[t];
     float x[TAPS][4], wt[TAPS][4];
+    typename Raw4<T>::type rx[TAPS];
+    raw4f rh[PAST];
 #pragma unroll
     for (int j = 0; j < TAPS; ++j) ld4t(w, (size_t)from * TAPS + 4 * j, wt[j]);
 #pragma unroll
+    for (int j = 0; j < TAPS; ++j) rx[j] = raw4(proj, (size_t)(t - min(PAST - j, min(i, PAST))) * stride + off + from);
+    if (i < PAST && rd >= 0) {                                      // (the same for the whole workgroup)
+#pragma unroll
+        for (int j = 0; j < PAST; ++j) rh[j] = raw4(hist, ((size_t)rd * PAST + min(i + j, PAST - 1)) * C + from);
+    }
+    requested();
+#pragma unroll
     for (int j = 0; j < TAPS; ++j) {
         const int d = PAST - j;
-        x[j][0] = x[j][1] = x[j][2] = x[j][3] = 0.f;
-        if (d <= i) ld4t(proj, (size_t)(t - d) * stride + off + from, x[j]);
-        else if (rd >= 0) ld4t(hist, ((size_t)rd * PAST + (PAST + i - d)) * C + from, x[j]);
+        float a[4], b[4];
+        widen4(rx[j], a);
+        widen4(rh[min(j, PAST - 1)], b);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[j][q] = d <= i ? a[q] : rd >= 0 ? b[q] : 0.f;
     }
     float y[4], s = 0.f;
 #pragma unroll
@@ -654,30 +689,50 @@ __global__ __launch_bounds__(256) void recurrent_step_wide_kernel(float* __restr
     float S[P][8][4], kc[P][8], qc[P][8], gc[P][8], vc[4];
     const float kb = kscale ? kscale[t * H + h] : 1.0f;
     const float hd = head_decay == 2 ? decay[h] : head_decay ? decay[t * H + h] : 0.f;
+    // every operand as it lies in memory, rows and columns clamped into the state: one trip
+    typename Raw4<TQ>::type rk[P][2], rq[P][2];
+    raw4f rg4[P][2];
+    TQ rv[4];
+    TB rb = TB();
 #pragma unroll
     for (int p = 0; p < P; ++p) {
-        const int r0 = p * 64 + rg * 8;
-        const bool ok = r0 < dim;                                   // (dim is a multiple of 8)
+        const int r0 = min(p * 64 + rg * 8, dim - 8);               // (dim is a multiple of 8)
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            rk[p][x] = raw4(k, t * k_stride + (size_t)qh * dim + r0 + 4 * x);
+            rq[p][x] = raw4(q, t * q_stride + (size_t)qh * dim + r0 + 4 * x);
+            if (!head_decay) rg4[p][x] = raw4(decay, (t * H + h) * (size_t)dim + r0 + 4 * x);
+        }
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             S[p][i][0] = S[p][i][1] = S[p][i][2] = S[p][i][3] = 0.f;
-            if (ok && col_ok && !fresh) ld4t(Sg, (size_t)(r0 + i) * vdim, S[p][i]);
-        }
-#pragma unroll
-        for (int i = 0; i < 8; i += 4) {
-            float a[4] = {0.f, 0.f, 0.f, 0.f}, b[4] = {0.f, 0.f, 0.f, 0.f}, g[4] = {hd, hd, hd, hd};
-            if (ok) {
-                ld4t(k, t * k_stride + (size_t)qh * dim + r0 + i, a);
-                ld4t(q, t * q_stride + (size_t)qh * dim + r0 + i, b);
-                if (!head_decay) ld4t(decay, (t * H + h) * (size_t)dim + r0 + i, g);
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) kc[p][i + e] = a[e], qc[p][i + e] = b[e], gc[p][i + e] = g[e];
+            if (p * 64 + rg * 8 < dim && col_ok && !fresh) ld4t(Sg, (size_t)(r0 + i) * vdim, S[p][i]);
         }
     }
 #pragma unroll
-    for (int c = 0; c < 4; ++c) vc[c] = j + c < v_cols ? ld(v, t * v_stride + (size_t)h * v_cols + j + c) : j + c == v_cols ? 1.0f : 0.f;
-    const float rate = DELTA ? 1.0f / (1.0f + expf(-ld(beta, t * beta_stride + h))) : 0.f;
+    for (int c = 0; c < 4; ++c) rv[c] = v[t * v_stride + (size_t)h * v_cols + min(j + c, v_cols - 1)];
+    if (DELTA) rb = beta[t * beta_stride + h];
+    requested();
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const bool ok = p * 64 + rg * 8 < dim;
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            float a[4], b[4], g[4];
+            widen4(rk[p][x], a);
+            widen4(rq[p][x], b);
+            widen4(rg4[p][x], g);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                kc[p][4 * x + e] = ok ? a[e] : 0.f;
+                qc[p][4 * x + e] = ok ? b[e] : 0.f;
+                gc[p][4 * x + e] = head_decay || !ok ? hd : g[e];
+            }
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) vc[c] = j + c < v_cols ? ld(&rv[c], 0) : j + c == v_cols ? 1.0f : 0.f;
+    const float rate = DELTA ? 1.0f / (1.0f + expf(-ld(&rb, 0))) : 0.f;
     // sum over the workgroup's rows; every thread gets its columns'
     auto row_sum = [&](float (&a)[4], int buffer) {
 #pragma unroll
@@ -914,12 +969,33 @@ __global__ __launch_bounds__(NT) void attention_prep_vec_kernel(float* __restric
 }
 
 // o[t, h, :n] turned by sign * pos[t] in place
-template <typename T>
+template <typename T, bool V4>
 __global__ __launch_bounds__(NT) void rotate_heads_kernel(T* __restrict__ o, const float* __restrict__ rope,
                                                           const int32_t* __restrict__ pos, float sign, int H, int n) {
     const size_t t = blockIdx.x;
     const int half = n >> 1;
     const float* cs = rope + (size_t)pos[t] * n;
+    if (V4) {
+        for (int idx = threadIdx.x * 4; idx < H * half; idx += NT * 4) {
+            const int h = idx / half, p = idx - h * half;
+            T* vec = o + (t * H + h) * (size_t)n;
+            const auto ra = raw4((const T*)vec, p), rb = raw4((const T*)vec, p + half);
+            const auto rc = raw4(cs, p), rs = raw4(cs, half + p);
+            requested();
+            float a[4], b[4], x[4], y[4];
+            widen4(ra, a);
+            widen4(rb, b);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float c = rc[j], s = rs[j] * sign;
+                x[j] = a[j] * c - b[j] * s;
+                y[j] = b[j] * c + a[j] * s;
+            }
+            st4t(vec, p, x);
+            st4t(vec, p + half, y);
+        }
+        return;
+    }
     for (int idx = threadIdx.x; idx < H * half; idx += NT) {
         const int h = idx / half, p = idx - h * half;
         T* vec = o + (t * H + h) * (size_t)n;
@@ -936,6 +1012,14 @@ extern "C" int qsv_decay(float* out, const void* z, int64_t z_stride, const void
                 "qsv_decay: bad arguments");
     QSV_REQUIRE(a_log || tau > 0.f, "qsv_decay: a power-sigmoid decay needs tau > 0");
     if (n_tokens == 0) return QSV_OK;
+    const int width = heads * dim;
+    const int64_t chunks = ((int64_t)width / 4 + NT - 1) / NT;
+    if (width % 4 == 0 && z_stride % 4 == 0 && fits4(out, QSV_F32) && fits4(z, dtype) && fits4(bias, dtype) && chunks * n_tokens < (1ll << 31)) {
+        QSV_DISPATCH(dtype, "qsv_decay",
+                     hipLaunchKernelGGL(decay_vec_kernel<T>, dim3((unsigned)(chunks * n_tokens)), dim3(NT), 0, (hipStream_t)stream, out, (const T*)z, z_stride,
+                                        (const T*)bias, a_log, a_log ? 0.f : 1.0f / tau, dim, width, (int)chunks));
+        return qsv_launch_status("qsv_decay");
+    }
     QSV_DISPATCH(dtype, "qsv_decay",
                  hipLaunchKernelGGL(decay_kernel<T>, dim3(n_tokens), dim3(NT), 0, (hipStream_t)stream, out, (const T*)z, z_stride,
                                     (const T*)bias, a_log, a_log ? 0.f : 1.0f / tau, dim, heads * dim));
@@ -1215,8 +1299,12 @@ extern "C" int qsv_rotate_heads(void* o, const float* rope, const int32_t* pos, 
                                 int dtype, void* stream) {
     QSV_REQUIRE(o && rope && pos && n_tokens >= 0 && heads > 0 && n > 0 && n % 2 == 0, "qsv_rotate_heads: bad arguments");
     if (n_tokens == 0) return QSV_OK;
-    QSV_DISPATCH(dtype, "qsv_rotate_heads",
-                 hipLaunchKernelGGL(rotate_heads_kernel<T>, dim3(n_tokens), dim3(NT), 0, (hipStream_t)stream, (T*)o, rope, pos, sign,
+    if (n % 8 == 0 && fits4(o, dtype) && fits4(rope, QSV_F32))
+        QSV_DISPATCH(dtype, "qsv_rotate_heads",
+                     hipLaunchKernelGGL((rotate_heads_kernel<T, true>), dim3(n_tokens), dim3(NT), 0, (hipStream_t)stream, (T*)o, rope, pos, sign, heads, n));
+    else
+        QSV_DISPATCH(dtype, "qsv_rotate_heads",
+                 hipLaunchKernelGGL((rotate_heads_kernel<T, false>), dim3(n_tokens), dim3(NT), 0, (hipStream_t)stream, (T*)o, rope, pos, sign,
                                     heads, n));
     return qsv_launch_status("qsv_rotate_heads");
 }

@@ -270,6 +270,84 @@ __global__ __launch_bounds__(NT) void latent_prep_kernel(const T* __restrict__ d
         st(dst, kv_rank + i, v);
     }
 }
+// The same for sizes and addresses that are multiples of four: a thread owns groups of four columns of the row [query latent | key-value latent | rotated key],
+// all requested before the first sum; the two sums meet in one exchange.  Bound by the row's latency in a step, by memory in a prompt.
+template <typename T, int P>
+__global__ __launch_bounds__(NT) void latent_prep_vec_kernel(const T* __restrict__ down, int64_t down_stride, int q_off, int q_rank, const T* __restrict__ q_w,
+                                                             T* __restrict__ cq, int kv_off, int kv_rank, const T* __restrict__ kv_w, int rot_dim, int rot_n,
+                                                             const float* __restrict__ rope, T* __restrict__ pool, const int64_t* __restrict__ slot,
+                                                             const int32_t* __restrict__ pos, float eps) {
+    __shared__ float red[2][NT / 64];
+    const size_t t = blockIdx.x;
+    const T* row = down + t * down_stride;
+    const int width = q_rank + kv_rank + rot_dim, half = rot_n / 2;
+    typename Raw4<T>::type rx[P], rw[P];
+    float co[P][2], sn[P][2];
+    const float* cs = rope ? rope + (size_t)pos[t] * (size_t)rot_n : nullptr;
+    T* dst = pool + (size_t)slot[t] * (size_t)(kv_rank + rot_dim);
+#pragma unroll
+    for (int k = 0; k < P; ++k) {
+        const int c = min((k * NT + (int)threadIdx.x) * 4, width - 4);
+        rx[k] = raw4(row, c < q_rank ? q_off + c : kv_off + c - q_rank);
+        rw[k] = raw4(c < q_rank ? q_w : kv_w, c < q_rank ? c : min(c - q_rank, kv_rank - 4));     // (no weight on the rotated part)
+    }
+    if (rope) {
+#pragma unroll
+        for (int k = 0; k < P; ++k) {                               // (a group's first pair may be rotated and its second not)
+            const int d = (k * NT + (int)threadIdx.x) * 4 - q_rank - kv_rank, p = max(0, min(d, rot_n - 2)) / 2, q = max(0, min(d + 2, rot_n - 2)) / 2;
+            co[k][0] = cs[p];
+            sn[k][0] = cs[half + p];
+            co[k][1] = cs[q];
+            sn[k][1] = cs[half + q];
+        }
+    }
+    requested();
+    float v[P][4], sq = 0.f, sk = 0.f;
+#pragma unroll
+    for (int k = 0; k < P; ++k) {
+        const int c = (k * NT + (int)threadIdx.x) * 4;
+        widen4(rx[k], v[k]);
+        const float s = v[k][0] * v[k][0] + v[k][1] * v[k][1] + v[k][2] * v[k][2] + v[k][3] * v[k][3];
+        if (c < q_rank) sq += s;
+        else if (c < q_rank + kv_rank) sk += s;
+    }
+    sq = wave_sum(sq);
+    sk = wave_sum(sk);
+    if ((threadIdx.x & 63) == 0) {
+        red[0][threadIdx.x >> 6] = sq;
+        red[1][threadIdx.x >> 6] = sk;
+    }
+    __syncthreads();
+    sq = sk = 0.f;
+#pragma unroll
+    for (int i = 0; i < NT / 64; ++i) {
+        sq += red[0][i];
+        sk += red[1][i];
+    }
+    const float qinv = 1.0f / sqrtf(sq / (float)q_rank + eps), kinv = 1.0f / sqrtf(sk / (float)kv_rank + eps);
+#pragma unroll
+    for (int k = 0; k < P; ++k) {
+        const int c = (k * NT + (int)threadIdx.x) * 4, d = c - q_rank - kv_rank;
+        if (c >= width) continue;
+        float w[4];
+        widen4(rw[k], w);
+        if (d < 0) {
+            const float inv = c < q_rank ? qinv : kinv;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[k][j] = v[k][j] * inv * w[j];
+        } else {
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                if (d + 2 * j < rot_n) {
+                    const float a = v[k][2 * j], b = v[k][2 * j + 1];
+                    v[k][2 * j] = a * co[k][j] - b * sn[k][j];
+                    v[k][2 * j + 1] = b * co[k][j] + a * sn[k][j];
+                }
+        }
+        if (c < q_rank) st4t(cq, t * q_rank + c, v[k]);
+        else st4t(dst, c - q_rank, v[k]);
+    }
+}
 extern "C" int qsv_latent_prep(const void* down, int64_t down_stride, int q_off, int q_rank, const void* q_w, void* cq,
                                int kv_off, int kv_rank, const void* kv_w, int rot_dim, int rot_n, const float* rope,
                                void* pool, const int64_t* slot, const int32_t* pos, float eps, int n, int dtype, void* stream) {
@@ -280,6 +358,19 @@ extern "C" int qsv_latent_prep(const void* down, int64_t down_stride, int q_off,
     QSV_REQUIRE(q_off >= 0 && kv_off >= 0 && q_off + q_rank <= down_stride && kv_off + kv_rank + rot_dim <= down_stride,
                 "qsv_latent_prep: the slices do not fit a row of %lld elements", (long long)down_stride);
     if (n == 0) return QSV_OK;
+    const int width = q_rank + kv_rank + rot_dim;
+    if (q_rank % 4 == 0 && kv_rank % 4 == 0 && rot_dim % 4 == 0 && q_off % 4 == 0 && kv_off % 4 == 0 && down_stride % 4 == 0 && width <= NT * 16 && fits4(down, dtype) &&
+        fits4(q_w, dtype) && fits4(cq, dtype) && fits4(kv_w, dtype) && fits4(pool, dtype)) {
+#define QSV_LPV(P)                                                                                                                            \
+    QSV_DISPATCH(dtype, "qsv_latent_prep",                                                                                                    \
+                 hipLaunchKernelGGL((latent_prep_vec_kernel<T, P>), dim3(n), dim3(NT), 0, (hipStream_t)stream, (const T*)down, down_stride, q_off, q_rank, \
+                                    (const T*)q_w, (T*)cq, kv_off, kv_rank, (const T*)kv_w, rot_dim, rot_n, rot_n ? rope : nullptr, (T*)pool, slot, pos, eps))
+        if (width <= NT * 4) QSV_LPV(1);
+        else if (width <= NT * 8) QSV_LPV(2);
+        else QSV_LPV(4);
+#undef QSV_LPV
+        return qsv_launch_status("qsv_latent_prep");
+    }
     QSV_DISPATCH(dtype, "qsv_latent_prep",
                  hipLaunchKernelGGL(latent_prep_kernel<T>, dim3(n), dim3(NT), 0, (hipStream_t)stream, (const T*)down, down_stride,
                                     q_off, q_rank, (const T*)q_w, (T*)cq, kv_off, kv_rank, (const T*)kv_w, rot_dim, rot_n, rope,
@@ -976,31 +1067,65 @@ __global__ __launch_bounds__(NT) void qk_norm_rope_prep_kernel(float* __restrict
     float* nq = sm;                                    // [NH][dim]
     const TI* qrow = q + t * q_stride;
     const TI* krow = k ? k + t * k_stride : nullptr;
+    // (the first pair's turn is requested with the row)
+    const int half = rot_n / 2, i_first = rope ? (int)threadIdx.x % half : 0;
+    const float* cs = rope ? rope + (size_t)pos[t] * rot_n : nullptr;
+    float c_first = 0.f, s_first = 0.f;
+    if (rope) {
+        c_first = cs[i_first];
+        s_first = cs[half + i_first];
+    }
     if (VEC && per_head) {
         const int e = (lane & (lph - 1)) * 4;
-        for (int h0 = threadIdx.x / lph; h0 - lane / lph < NH; h0 += NT / lph) {      // (a wave stays together: its lanes exchange sums)
-            const bool ok = h0 < NH && e < dim, isq = h0 < H;
-            const int hh = isq ? h0 : h0 - H;
-            float4 u = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (ok) {
-                u = ld4v(isq ? qrow : krow, (size_t)hh * dim + e);
-                const T* bias = isq ? q_b : k_b;
-                if (bias) {
-                    const float4 b = ld4v(bias, (size_t)hh * dim + e);
-                    u.x += b.x; u.y += b.y; u.z += b.z; u.w += b.w;
-                }
+        // (a wave stays together: its lanes exchange sums; up to four of its rounds of heads in one trip to memory)
+        const int step = NT / lph, at = min(e, dim - 4);
+        typename Raw4<T>::type rqw, rkw;
+        if (q_w) {
+            rqw = raw4(q_w, at);
+            rkw = raw4(k ? k_w : q_w, at);
+        }
+        for (int b0 = threadIdx.x / lph; b0 - lane / lph < NH; b0 += 4 * step) {
+            typename Raw4<TI>::type ru[4];
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+                const int h0 = min(b0 + x * step, NH - 1);
+                ru[x] = raw4(h0 < H ? qrow : krow, (size_t)(h0 < H ? h0 : h0 - H) * dim + at);
             }
-            float s;
-            if (rot_gain > 0.f)
-                s = (e < rot_n ? rot_gain : 1.f) * u.x * u.x + (e + 1 < rot_n ? rot_gain : 1.f) * u.y * u.y +
-                    (e + 2 < rot_n ? rot_gain : 1.f) * u.z * u.z + (e + 3 < rot_n ? rot_gain : 1.f) * u.w * u.w;
-            else
-                s = u.x * u.x + u.y * u.y + u.z * u.z + u.w * u.w;
-            for (int o = lph >> 1; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-            const float inv = 1.0f / sqrtf(s / (float)dim + eps);
-            if (ok) {
-                const float4 g = q_w ? ld4v(isq ? q_w : k_w, e) : make_float4(1.f, 1.f, 1.f, 1.f);
-                *(float4*)(nq + h0 * dim + e) = make_float4(u.x * (inv * g.x), u.y * (inv * g.y), u.z * (inv * g.z), u.w * (inv * g.w));
+            requested();
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+                const int h0 = b0 + x * step;
+                if (h0 - lane / lph >= NH) continue;                                        // (the whole wave)
+                const bool ok = h0 < NH && e < dim, isq = h0 < H;
+                const int hh = isq ? h0 : h0 - H;
+                float u4[4];
+                widen4(ru[x], u4);
+                float4 u = ok ? make_float4(u4[0], u4[1], u4[2], u4[3]) : make_float4(0.f, 0.f, 0.f, 0.f);
+                if (ok) {
+                    const T* bias = isq ? q_b : k_b;
+                    if (bias) {
+                        const float4 b = ld4v(bias, (size_t)hh * dim + e);
+                        u.x += b.x; u.y += b.y; u.z += b.z; u.w += b.w;
+                    }
+                }
+                float s;
+                if (rot_gain > 0.f)
+                    s = (e < rot_n ? rot_gain : 1.f) * u.x * u.x + (e + 1 < rot_n ? rot_gain : 1.f) * u.y * u.y +
+                        (e + 2 < rot_n ? rot_gain : 1.f) * u.z * u.z + (e + 3 < rot_n ? rot_gain : 1.f) * u.w * u.w;
+                else
+                    s = u.x * u.x + u.y * u.y + u.z * u.z + u.w * u.w;
+                for (int o = lph >> 1; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+                const float inv = 1.0f / sqrtf(s / (float)dim + eps);
+                if (ok) {
+                    float g4[4] = {1.f, 1.f, 1.f, 1.f}, a[4], b[4];
+                    widen4(rqw, a);
+                    widen4(rkw, b);
+                    if (q_w) {
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) g4[j] = isq ? a[j] : b[j];
+                    }
+                    *(float4*)(nq + h0 * dim + e) = make_float4(u.x * (inv * g4[0]), u.y * (inv * g4[1]), u.z * (inv * g4[2]), u.w * (inv * g4[3]));
+                }
             }
         }
     } else if (per_head) {
@@ -1041,11 +1166,13 @@ __global__ __launch_bounds__(NT) void qk_norm_rope_prep_kernel(float* __restrict
     }
     __syncthreads();
     if (rope) {                                        // each pair by one thread
-        const int half = rot_n / 2;
-        const float* cs = rope + (size_t)pos[t] * rot_n;
         for (int idx = threadIdx.x; idx < NH * half; idx += NT) {
             const int hh = idx / half, i = idx - hh * half;
-            const float c = cs[i], sn = cs[half + i];
+            float c = c_first, sn = s_first;
+            if (i != i_first) {
+                c = cs[i];
+                sn = cs[half + i];
+            }
             const int i0 = hh * dim + (halves ? i : 2 * i), i1 = i0 + (halves ? half : 1);
             const float a = nq[i0], b = nq[i1];
             nq[i0] = a * c - b * sn;

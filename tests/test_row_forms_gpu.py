@@ -1,0 +1,104 @@
+"""Row kernels that take four columns a thread against their forms for any width and address: the same operands a few elements off the alignment."""
+import pytest
+import torch
+
+from qserve_amd.layers.ops import make_ops
+from qserve_amd.serving.engine import StepBatch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+TYPES = pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
+
+
+def make(dtype):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return make_ops("hip", dtype, torch.device(DEV))
+
+
+def off(t):
+    """The same values, the storage starting one element late."""
+    return torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape)
+
+
+def ints(v):
+    return torch.tensor(v, dtype=torch.int32, device=DEV)
+
+
+@TYPES
+@pytest.mark.parametrize("T, q_rank, kv_rank, rot_dim, rot_n", [(1, 4, 4, 0, 0), (3, 768, 512, 64, 64), (5, 768, 512, 64, 22), (2, 8, 1024, 4, 2), (65, 1536, 2000, 64, 64), (2, 2056, 2040, 0, 0)])
+def test_latent_prep(dtype, T, q_rank, kv_rank, rot_dim, rot_n):
+    ops, g = make(dtype), torch.Generator().manual_seed(T + q_rank)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(dtype).to(DEV)                                        # noqa: E731
+    R = kv_rank + rot_dim
+    down, qw, kw = rnd(T, q_rank + R + 8), rnd(q_rank), rnd(kv_rank)
+    rope = torch.randn(T + 1, 2, rot_n // 2, generator=g).to(DEV) if rot_n else None
+    pos, slot = ints(list(range(T, 0, -1))), torch.randperm(2 * T, generator=g)[:T].to(DEV)
+    out = []
+    for q in (qw, off(qw)):                                              # (off the alignment: a column at a time)
+        pool = torch.zeros(2 * T, R, dtype=dtype, device=DEV)
+        out.append((ops.latent_prep(down, 0, q_rank, q, q_rank + 4, kv_rank, kw, rot_dim, rot_n, rope, pool, slot, pos, 1e-5), pool))
+    for a, b in zip(*out):
+        # sums of squares in another order, and a turn's second product rounded or not before the sum (terms below 10: 2^-24 of each): the last bit
+        a, b = a.double(), b.double()
+        assert ((a - b).abs() <= (2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -20) * b.abs() + 2e-6).all()
+        assert (a != b).float().mean() < 0.02 or dtype == torch.float32
+
+
+@TYPES
+@pytest.mark.parametrize("T, H, dim", [(1, 1, 4), (3, 5, 12), (16, 16, 64), (65, 3, 1028)])
+@pytest.mark.parametrize("log", [False, True])
+def test_decay_and_rotation(dtype, T, H, dim, log):
+    ops, g = make(dtype), torch.Generator().manual_seed(T + dim)
+    z, b = (torch.randn(T, H * dim + 8, generator=g).to(dtype).to(DEV), torch.randn(H * dim, generator=g).to(dtype).to(DEV))
+    a = torch.randn(H, generator=g).to(DEV) if log else None
+    z = z[:, 4:4 + H * dim]
+    assert torch.equal(ops.decay(z, b, a, 16.0, H, dim), ops.decay(z, off(b), a, 16.0, H, dim))
+    n = dim // 4 * 8
+    o, pos, rope = torch.randn(T, H, n, generator=g).to(dtype).to(DEV), ints(list(range(T))), torch.randn(T, 2, n // 2, generator=g).to(DEV)
+    assert torch.equal(ops.rotate_heads(o.clone(), rope, pos, -1.0), ops.rotate_heads(off(o), rope, pos, -1.0))
+
+
+@TYPES
+@pytest.mark.parametrize("T, S, D", [(1, 1, 4), (3, 2, 1028), (16, 3, 2048), (5, 4, 4096), (2, 5, 72)])
+def test_streams_norm_and_branches(dtype, T, S, D):
+    ops, g = make(dtype), torch.Generator().manual_seed(T + D)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(dtype).to(DEV)                                        # noqa: E731
+    x, w, b, rows = torch.randn(T, S, D, generator=g).to(DEV), rnd(D), rnd(D), ints(list(range(T))[::-1])
+    assert torch.equal(ops.dyt_sum_rows(x, rows, (w, b, 0.6)), ops.dyt_sum_rows(x, rows, (off(w), b, 0.6)))
+    u, v = rnd(T, D), rnd(T, D)
+    ref = 0.5 * sum(t.double() / (t.double().pow(2).mean(-1, keepdim=True) + 1e-5).sqrt() * f.double() for t, f in ((u, w), (v, b)))
+    got = ops.rms_pair_mean(u, w, v, b, 1e-5).double()
+    assert ((got - ref).abs() <= (2.0 ** -8 if dtype == torch.bfloat16 else 0.0) * ref.abs() + 2e-5).all()
+
+
+# runs: (first position, tokens); a run behind its first token reads the history
+@TYPES
+@pytest.mark.parametrize("taps", [2, 3, 4])
+@pytest.mark.parametrize("runs", [((0, 1), (7, 1), (1, 1)), ((0, 5), (3, 2)), ((2, 3), (0, 2), (9, 4))])
+def test_convolved_heads(dtype, taps, runs):
+    ops, g = make(dtype), torch.Generator().manual_seed(taps + len(runs))
+    T, qc, G, kd, vd = sum(n for _, n in runs), 40, 2, 8, 12
+    C, past = qc + G * (kd + vd), taps - 1
+    proj, w = torch.randn(T, C + 4, generator=g).to(dtype).to(DEV), torch.randn(taps, C, generator=g).to(DEV)
+    hist = torch.randn(2 * len(runs), past, C, generator=g).to(DEV)
+    off_, rd, wr, pos, items, at = [], [], [], [], [], 0
+    for r, (start, n) in enumerate(runs):
+        off_ += range(n)
+        rd += [2 * r if start else -1] * n
+        wr += [-1] * (n - 1) + [2 * r + 1]
+        pos += range(start, start + n)
+        items.append((r, at, n))
+        at += n
+    batch = StepBatch(tokens=None, seq=None, pos=ints(pos), slot=torch.arange(T, device=DEV), block_table=None, max_pos=max(pos), n_tokens=T, items=items,
+                      run_off=ints(off_), state_rd=ints(rd), state_wr=ints(wr))
+    out = []
+    for f in (w, off(w)):
+        h, pool = hist.clone(), torch.zeros(G, T, vd + kd, dtype=dtype, device=DEV)
+        out.append((ops.conv_heads_cache(proj, f, h, batch, qc, G, kd, vd, pool, 0.3, (0.1, 4.0)), pool, h))
+    assert all(torch.equal(a, b) for a, b in zip(*out))
+    # ... and the convolution in front of a recurrence
+    h1, h2, taps_of = hist.clone(), hist.clone(), w.t().contiguous()
+    a, b = ops.conv_silu_unit(proj, 0, taps_of, h1, batch, 4, 8), ops.conv_silu_unit(proj, 0, off(taps_of), h2, batch, 4, 8)
+    # eight squares added in another order, four products: some units of 2^-24 of values below 16
+    assert ((a - b).abs() <= 1e-5).all() and torch.equal(h1, h2)

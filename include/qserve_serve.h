@@ -23,6 +23,11 @@ const char* qsv_last_error(void);
 /* out [n_rows, N] = x [n_rows, K] @ w [N, K]^T, bfloat16 with float accumulation, for few rows (a decoding step); x_stride: elements from one
  * row of x to the next.  K and x_stride multiples of 8, x and w on 16 bytes. */
 int qsv_skinny_linear(void* out, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K, void* stream);
+/* The same values in float. */
+int qsv_skinny_linear_widened(float* out, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K, void* stream);
+/* decay [n_rows, N] = qsv_decay of x @ w^T (bias [N], a_log [N / dim] or NULL and tau), and, with gate_N > 0, gate = gate_x @ gate_w^T, in one launch. */
+int qsv_decay_products(float* decay, const void* x, int64_t x_stride, const void* w, int N, int K, const void* bias, const float* a_log, float tau, int dim,
+                       void* gate, const void* gate_x, int64_t gate_x_stride, const void* gate_w, int gate_N, int gate_K, int n_rows, void* stream);
 
 /* out [T, H, N] = x[t, h] @ w[h], w [H, K, N], bfloat16 with float accumulation, for up to 64 rows; x_tok, x_head: elements from one token / head
  * of x to the next.  K and N multiples of 32, x_tok and x_head of 8, x on 16 bytes. */

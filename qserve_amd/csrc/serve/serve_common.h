@@ -200,6 +200,12 @@ __device__ __forceinline__ void slot_sum4(const SlotRows& s, size_t t, int D, in
     else slot_sum4_as<Y, P, false>(s, t, D, c, step, a);
 }
 
+// A recurrence's decay from its gate z: sigmoid(z)^(1 / tau) = exp(-softplus(-z) / tau), or, with a log rate, exp(-exp(a) softplus(z))
+__device__ __forceinline__ float softplusf(float z) { return z > 20.f ? z : log1pf(expf(z)); }
+__device__ __forceinline__ float gate_decay(float z, bool with_rate, float a, float inv_tau) {
+    return with_rate ? expf(-expf(a) * softplusf(z)) : expf(-softplusf(-z) * inv_tau);
+}
+
 // ... as a tensor of the storage type would hold it
 __device__ __forceinline__ float stored(const float*, float v) { return v; }
 __device__ __forceinline__ float stored(const bf16_t*, float v) { return bf2f(f2bf(v)); }

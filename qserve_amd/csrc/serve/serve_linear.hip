@@ -8,17 +8,29 @@
 #include "serve_stream.h"
 
 namespace {
-template <int RB, int SG>
-__global__ __launch_bounds__(64 * STREAM_WAVES, 2) void skinny_linear_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ X, int64_t x_stride,
-                                                                            const bf16_t* __restrict__ W, int T, int N, int K, int wide) {
-    __shared__ __attribute__((aligned(128))) unsigned char rings[STREAM_WAVES * XRING];
+// What becomes of a product x [T, K] @ w [N, K]^T: rounded to bfloat16 it is stored, stored as float (a caller that would widen it), or, as a decay's gate, turned
+// into the decay (float) with bias [N] and the log rate of its head, a_log [N / dim] or NULL.
+enum { AS_IS, WIDENED, DECAY };
+struct SkinnyJob {
+    void* out;
+    const bf16_t* X;
+    int64_t x_stride;
+    const bf16_t* W;
+    int T, N, K, wide;
+    const bf16_t* bias;
+    const float* a_log;
+    float inv_tau;
+    int dim;
+};
+template <int RB, int SG, int HOW>
+__device__ __forceinline__ void skinny_product(const SkinnyJob& a, int block, unsigned char* rings) {
     constexpr int TILES = RB * SG;
     static_assert(STREAM_WAVES * TILES * 1024 <= STREAM_WAVES * XRING, "");
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int r0 = blockIdx.x * 16 * RB, t0 = blockIdx.y * 16 * SG, count = min(16 * SG, T - t0);
+    const int r0 = block * 16 * RB, t0 = blockIdx.y * 16 * SG, count = min(16 * SG, a.T - t0);
     v4f acc[RB][SG];
-    stream_products<RB, SG>(W + (size_t)r0 * K, K, min(16 * RB, N - r0), rings + w * XRING, w, lane,
-                            [&](int i) { return X + (size_t)(t0 + min(i, count - 1)) * (size_t)x_stride; }, acc);
+    stream_products<RB, SG>(a.W + (size_t)r0 * a.K, a.K, min(16 * RB, a.N - r0), rings + w * XRING, w, lane,
+                            [&](int i) { return a.X + (size_t)(t0 + min(i, count - 1)) * (size_t)a.x_stride; }, acc);
     v4f* red = (v4f*)rings;                                         // [wave][tile][lane]
     __syncthreads();                                                // every wave is done with its ring
 #pragma unroll
@@ -26,20 +38,58 @@ __global__ __launch_bounds__(64 * STREAM_WAVES, 2) void skinny_linear_kernel(bf1
 #pragma unroll
         for (int g = 0; g < SG; ++g) red[(w * TILES + r * SG + g) * 64 + lane] = acc[r][g];
     __syncthreads();
+    if constexpr (HOW == DECAY) {                                   // (some hundred instructions a value: every wave takes one of a lane's four)
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            const int c = 16 * (t % SG) + (lane & 15), n = r0 + 16 * (t / SG) + 4 * (lane >> 4) + w;
+            if (c >= count || n >= a.N) continue;
+            const float* p = (const float*)(red + t * 64 + lane) + w;
+            float v = p[0];
+#pragma unroll
+            for (int o = 1; o < STREAM_WAVES; ++o) v += p[o * TILES * 256];
+            v = gate_decay(bf2f(f2bf(v)) + bf2f(a.bias[n]), a.a_log != nullptr, a.a_log ? a.a_log[n / a.dim] : 0.f, a.inv_tau);
+            ((float*)a.out)[(size_t)(t0 + c) * a.N + n] = v;
+        }
+        return;
+    }
     for (int t = w; t < TILES; t += STREAM_WAVES) {
         const int c = 16 * (t % SG) + (lane & 15), n = r0 + 16 * (t / SG) + 4 * (lane >> 4);
         if (c >= count) continue;
         v4f v = red[t * 64 + lane];
 #pragma unroll
         for (int o = 1; o < STREAM_WAVES; ++o) v += red[(o * TILES + t) * 64 + lane];
-        bf16_t* p = out + (size_t)(t0 + c) * N + n;
-        if (wide && n + 4 <= N) {
-            *(uint2*)p = make_uint2((unsigned)f2bf(v[0]) | ((unsigned)f2bf(v[1]) << 16), (unsigned)f2bf(v[2]) | ((unsigned)f2bf(v[3]) << 16));
+        const size_t at = (size_t)(t0 + c) * a.N + n;
+        const bool whole = a.wide && n + 4 <= a.N;
+        if constexpr (HOW == AS_IS) {
+            bf16_t* p = (bf16_t*)a.out + at;
+            if (whole) {
+                *(uint2*)p = make_uint2((unsigned)f2bf(v[0]) | ((unsigned)f2bf(v[1]) << 16), (unsigned)f2bf(v[2]) | ((unsigned)f2bf(v[3]) << 16));
+            } else {
+                for (int q = 0; q < 4; ++q)
+                    if (n + q < a.N) p[q] = f2bf(v[q]);
+            }
         } else {
-            for (int q = 0; q < 4; ++q)
-                if (n + q < N) p[q] = f2bf(v[q]);
+            float* p = (float*)a.out + at;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] = bf2f(f2bf(v[q]));
+            if (whole) *(v4f*)p = v;
+            else
+                for (int q = 0; q < 4; ++q)
+                    if (n + q < a.N) p[q] = v[q];
         }
     }
+}
+template <int RB, int SG, int HOW>
+__global__ __launch_bounds__(64 * STREAM_WAVES, 2) void skinny_linear_kernel(SkinnyJob a) {
+    __shared__ __attribute__((aligned(128))) unsigned char rings[STREAM_WAVES * XRING];
+    skinny_product<RB, SG, HOW>(a, blockIdx.x, rings);
+}
+// A recurrence's two second stages in one launch: the decay's product (its first `blocks` workgroups) and the output gate's (N 0: none)
+template <int SG>
+__global__ __launch_bounds__(64 * STREAM_WAVES, 2) void decay_products_kernel(SkinnyJob decay, SkinnyJob gate, int blocks) {
+    __shared__ __attribute__((aligned(128))) unsigned char rings[STREAM_WAVES * XRING];
+    if ((int)blockIdx.x < blocks) skinny_product<1, SG, DECAY>(decay, blockIdx.x, rings);
+    else skinny_product<1, SG, AS_IS>(gate, blockIdx.x - blocks, rings);
 }
 
 // ---- one product per head: y[t, h] = x[t, h] @ W[h], W [H, K, N] with N contiguous -------------------------------------------------------
@@ -187,22 +237,51 @@ extern "C" int qsv_latent_query_product(float* qf, const void* q, const void* w_
                                   (hipStream_t)stream, "qsv_latent_query_product");
 }
 
-extern "C" int qsv_skinny_linear(void* out, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K, void* stream) {
-    QSV_REQUIRE(out && x && w && n_rows >= 0 && N > 0 && K > 0 && K % 8 == 0 && x_stride % 8 == 0 && x_stride >= 0, "qsv_skinny_linear: bad arguments");
-    QSV_REQUIRE(((uintptr_t)x | (uintptr_t)w) % 16 == 0, "qsv_skinny_linear: inputs and weights start on 16 bytes");
-    QSV_REQUIRE(K <= (1 << 25) && n_rows <= 65535 * 16, "qsv_skinny_linear: %d inputs of %d", n_rows, K);
-    if (n_rows == 0) return QSV_OK;
-    const int wide = N % 4 == 0 && (uintptr_t)out % 8 == 0;
+static int skinny_fits(const char* what, const void* out, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K) {
+    QSV_REQUIRE(out && x && w && n_rows >= 0 && N > 0 && K > 0 && K % 8 == 0 && x_stride % 8 == 0 && x_stride >= 0, "%s: bad arguments", what);
+    QSV_REQUIRE(((uintptr_t)x | (uintptr_t)w) % 16 == 0, "%s: inputs and weights start on 16 bytes", what);
+    QSV_REQUIRE(K <= (1 << 25) && n_rows <= 65535 * 16, "%s: %d inputs of %d", what, n_rows, K);
+    return QSV_OK;
+}
+template <int HOW>
+static int launch_skinny(const char* what, void* out, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K, void* stream) {
+    const int rc = skinny_fits(what, out, x, x_stride, w, n_rows, N, K);
+    if (rc != QSV_OK || n_rows == 0) return rc;
+    const SkinnyJob a = {out, (const bf16_t*)x, x_stride, (const bf16_t*)w, n_rows, N, K, N % 4 == 0 && (uintptr_t)out % (HOW == AS_IS ? 8 : 16) == 0, nullptr, nullptr, 0.f, 1};
     // 16 weight rows per workgroup where 32 would leave CUs without one, or need a second round for a few (8256 x 2048: 11.4 -> 10.5 us); else 32,
     // which reads the inputs half as often (6144 x 2048: 8.2 -> 7.4 us)
     const bool few = n_rows <= 16, small = N < 5120 || (N > 8192 && N <= 16384 && n_rows <= 32);
 #define QSV_SKINNY(RB, SG)                                                                                                                    \
-    hipLaunchKernelGGL((skinny_linear_kernel<RB, SG>), dim3((N + 16 * RB - 1) / (16 * RB), (n_rows + 16 * SG - 1) / (16 * SG)),               \
-                       dim3(64 * STREAM_WAVES), 0, (hipStream_t)stream, (bf16_t*)out, (const bf16_t*)x, x_stride, (const bf16_t*)w, n_rows, N, K, wide)
+    hipLaunchKernelGGL((skinny_linear_kernel<RB, SG, HOW>), dim3((N + 16 * RB - 1) / (16 * RB), (n_rows + 16 * SG - 1) / (16 * SG)),          \
+                       dim3(64 * STREAM_WAVES), 0, (hipStream_t)stream, a)
     if (few && small) QSV_SKINNY(1, 1);
     else if (few) QSV_SKINNY(2, 1);
     else if (small) QSV_SKINNY(1, 2);
     else QSV_SKINNY(2, 2);
 #undef QSV_SKINNY
-    return qsv_launch_status("qsv_skinny_linear");
+    return qsv_launch_status(what);
+}
+extern "C" int qsv_skinny_linear(void* out, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K, void* stream) {
+    return launch_skinny<AS_IS>("qsv_skinny_linear", out, x, x_stride, w, n_rows, N, K, stream);
+}
+// the same values in float
+extern "C" int qsv_skinny_linear_widened(float* out, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K, void* stream) {
+    return launch_skinny<WIDENED>("qsv_skinny_linear_widened", out, x, x_stride, w, n_rows, N, K, stream);
+}
+// decay [n_rows, N] (float) of z = x @ w^T as qsv_decay makes it, and, with gate_N > 0, gate [n_rows, gate_N] = gate_x @ gate_w^T
+extern "C" int qsv_decay_products(float* decay, const void* x, int64_t x_stride, const void* w, int N, int K, const void* bias, const float* a_log, float tau, int dim,
+                                  void* gate, const void* gate_x, int64_t gate_x_stride, const void* gate_w, int gate_N, int gate_K, int n_rows, void* stream) {
+    int rc = skinny_fits("qsv_decay_products", decay, x, x_stride, w, n_rows, N, K);
+    if (rc == QSV_OK && gate_N) rc = skinny_fits("qsv_decay_products (gate)", gate, gate_x, gate_x_stride, gate_w, n_rows, gate_N, gate_K);
+    if (rc != QSV_OK) return rc;
+    QSV_REQUIRE(bias && dim > 0 && N % dim == 0 && gate_N >= 0 && (a_log || tau > 0.f), "qsv_decay_products: %d decays of heads of %d", N, dim);
+    if (n_rows == 0) return QSV_OK;
+    const SkinnyJob a = {decay, (const bf16_t*)x, x_stride, (const bf16_t*)w, n_rows, N, K, N % 4 == 0 && (uintptr_t)decay % 16 == 0, (const bf16_t*)bias, a_log,
+                         a_log ? 0.f : 1.0f / tau, dim};
+    const SkinnyJob g = {gate, (const bf16_t*)gate_x, gate_x_stride, (const bf16_t*)gate_w, n_rows, gate_N, gate_N ? gate_K : 8, gate_N % 4 == 0 && (uintptr_t)gate % 8 == 0,
+                         nullptr, nullptr, 0.f, 1};
+    const int blocks = (N + 15) / 16, more = (gate_N + 15) / 16;
+    if (n_rows <= 16) hipLaunchKernelGGL(decay_products_kernel<1>, dim3(blocks + more, 1), dim3(64 * STREAM_WAVES), 0, (hipStream_t)stream, a, g, blocks);
+    else hipLaunchKernelGGL(decay_products_kernel<2>, dim3(blocks + more, (n_rows + 31) / 32), dim3(64 * STREAM_WAVES), 0, (hipStream_t)stream, a, g, blocks);
+    return qsv_launch_status("qsv_decay_products");
 }

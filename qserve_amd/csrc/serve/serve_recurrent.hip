@@ -8,10 +8,7 @@ namespace {
 constexpr int NT = 256;
 constexpr int NW = NT / 64;
 
-__device__ __forceinline__ float softplusf(float z) { return z > 20.f ? z : log1pf(expf(z)); }
-
-// ---- decays ---------------------------------------------------------------------------------------------------------------
-// mode 0: sigmoid(z + bias)^(1 / tau) = exp(-softplus(-(z + bias)) / tau);  mode 1: exp(-exp(a_log[head]) softplus(z + bias))
+// ---- decays (gate_decay) ---------------------------------------------------------------------------------------------------
 template <typename T>
 __global__ __launch_bounds__(NT) void decay_kernel(float* __restrict__ out, const T* __restrict__ z, int64_t z_stride,
                                                    const T* __restrict__ bias, const float* __restrict__ a_log, float inv_tau,
@@ -19,7 +16,7 @@ __global__ __launch_bounds__(NT) void decay_kernel(float* __restrict__ out, cons
     const size_t t = blockIdx.x;
     for (int c = threadIdx.x; c < n; c += NT) {
         const float v = ld(z, t * z_stride + c) + ld(bias, c);
-        out[t * n + c] = a_log ? expf(-expf(a_log[c / dim]) * softplusf(v)) : expf(-softplusf(-v) * inv_tau);
+        out[t * n + c] = gate_decay(v, a_log != nullptr, a_log ? a_log[c / dim] : 0.f, inv_tau);
     }
 }
 
@@ -41,8 +38,7 @@ __global__ __launch_bounds__(NT) void decay_vec_kernel(float* __restrict__ out, 
     widen4(rb, b);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        v[j] += b[j];
-        v[j] = a_log ? expf(-expf(a[j]) * softplusf(v[j])) : expf(-softplusf(-v[j]) * inv_tau);
+        v[j] = gate_decay(v[j] + b[j], a_log != nullptr, a[j], inv_tau);
     }
     st4t(out, t * n + c, v);
 }

@@ -30,9 +30,29 @@ __global__ __launch_bounds__(NT) void embed_kernel(float* __restrict__ x, T* __r
         st(h, t * D + i, v);
     }
 }
+// The same, four columns per thread, `chunks` workgroups per token.
+template <typename T>
+__global__ __launch_bounds__(NT) void embed_vec_kernel(float* __restrict__ x, T* __restrict__ h, const T* __restrict__ table, const int32_t* __restrict__ tokens, int D,
+                                                       int chunks) {
+    const size_t t = token_of(blockIdx.x, chunks);
+    const int i = ((blockIdx.x - (unsigned)t * chunks) * NT + threadIdx.x) * 4;
+    if (i >= D) return;
+    const auto r = raw4(table, (size_t)tokens[t] * D + i);
+    float v[4];
+    widen4(r, v);
+    st4t(x, t * D + i, v);
+    *(typename Raw4<T>::type*)(h + t * D + i) = r;
+}
 extern "C" int qsv_embed(float* x, void* h, const void* table, const int32_t* tokens, int n, int D, int dtype, void* stream) {
     QSV_REQUIRE(x && h && table && tokens && n >= 0 && D > 0, "qsv_embed: bad arguments");
     if (n == 0) return QSV_OK;
+    const int64_t chunks = ((int64_t)D / 4 + NT - 1) / NT;
+    if (D % 4 == 0 && fits4(x, QSV_F32) && fits4(h, dtype) && fits4(table, dtype) && chunks * n < (1ll << 31)) {
+        QSV_DISPATCH(dtype, "qsv_embed",
+                     hipLaunchKernelGGL(embed_vec_kernel<T>, dim3((unsigned)(chunks * n)), dim3(NT), 0, (hipStream_t)stream, x, (T*)h, (const T*)table, tokens, D,
+                                        (int)chunks));
+        return qsv_launch_status("qsv_embed");
+    }
     QSV_DISPATCH(dtype, "qsv_embed",
                  hipLaunchKernelGGL(embed_kernel<T>, dim3(n), dim3(NT), 0, (hipStream_t)stream, x, (T*)h, (const T*)table, tokens, D));
     return qsv_launch_status("qsv_embed");

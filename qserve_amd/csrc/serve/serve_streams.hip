@@ -23,6 +23,20 @@ __global__ __launch_bounds__(NT) void embed_streams_kernel(float* __restrict__ x
     }
 }
 
+// The same, four columns per thread, `chunks` workgroups per token.
+template <typename T>
+__global__ __launch_bounds__(NT) void embed_streams_vec_kernel(float* __restrict__ x, const T* __restrict__ table, const int32_t* __restrict__ tokens, float scale, int S,
+                                                               int D, int chunks) {
+    const size_t t = token_of(blockIdx.x, chunks);
+    const int i = ((blockIdx.x - (unsigned)t * chunks) * NT + threadIdx.x) * 4;
+    if (i >= D) return;
+    float v[4];
+    ld4t(table, (size_t)tokens[t] * D + i, v);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] *= scale;
+    for (int s = 0; s < S; ++s) st4t(x, (t * S + s) * D + i, v);
+}
+
 __device__ __forceinline__ float stream_sum(const float* __restrict__ x, const float* __restrict__ w_in, size_t t, int S, int D,
                                             int i) {
     float u = 0.f;
@@ -459,6 +473,13 @@ extern "C" int qsv_embed_streams(float* x, const void* table, const int32_t* tok
                                  int dtype, void* stream) {
     QSV_REQUIRE(x && table && tokens && n >= 0 && D > 0 && streams > 0, "qsv_embed_streams: bad arguments");
     if (n == 0) return QSV_OK;
+    const int64_t chunks = ((int64_t)D / 4 + NT - 1) / NT;
+    if (D % 4 == 0 && fits4(x, QSV_F32) && fits4(table, dtype) && chunks * n < (1ll << 31)) {
+        QSV_DISPATCH(dtype, "qsv_embed_streams",
+                     hipLaunchKernelGGL(embed_streams_vec_kernel<T>, dim3((unsigned)(chunks * n)), dim3(NT), 0, (hipStream_t)stream, x, (const T*)table, tokens, scale,
+                                        streams, D, (int)chunks));
+        return qsv_launch_status("qsv_embed_streams");
+    }
     QSV_DISPATCH(dtype, "qsv_embed_streams",
                  hipLaunchKernelGGL(embed_streams_kernel<T>, dim3(n), dim3(NT), 0, (hipStream_t)stream, x, (const T*)table, tokens,
                                     scale, streams, D));

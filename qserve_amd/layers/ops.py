@@ -82,20 +82,36 @@ def _called_plainly(*ts):
             and not (torch.is_grad_enabled() and any(t.requires_grad for t in ts)))
 
 
-def linear(x, w):
-    """x [T, in] @ w [out, in]^T in the storage type, float accumulation: the few rows of a decoding step (bfloat16 on a GPU) through
-    qsv_skinny_linear, everything else through hipBLASLt / rocBLAS."""
-    if (type(x) is torch.Tensor and type(w) in (torch.Tensor, torch.nn.Parameter) and x.is_cuda and _called_plainly(x, w) and x.dim() == 2 and w.dim() == 2
+def _streams(x, w):
+    """Whether x @ w^T goes through the kernel for the few rows of a decoding step."""
+    return (type(x) is torch.Tensor and type(w) in (torch.Tensor, torch.nn.Parameter) and x.is_cuda and _called_plainly(x, w) and x.dim() == 2 and w.dim() == 2
             and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and w.is_contiguous() and 0 < x.size(0) and x.size(1) == w.size(1)
             and x.size(1) and w.size(0) and _skinny(x.size(0), w.size(0), w.size(1))
             and x.stride(1) == 1 and x.size(1) % 8 == 0 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-            and x.device == w.device and x.device.index == torch.cuda.current_device()):
+            and x.device == w.device and x.device.index == torch.cuda.current_device())
+
+
+def linear(x, w):
+    """x [T, in] @ w [out, in]^T in the storage type, float accumulation: the few rows of a decoding step (bfloat16 on a GPU) through
+    qsv_skinny_linear, everything else through hipBLASLt / rocBLAS."""
+    if _streams(x, w):
         from ..serving._lib import check, lib
         out = torch.empty((x.size(0), w.size(0)), dtype=x.dtype, device=x.device)
         check(lib().qsv_skinny_linear(out.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(), x.size(0), w.size(0), x.size(1),
                                       torch.cuda.current_stream(x.device).cuda_stream), "skinny_linear")
         return out
     return torch.matmul(x, w.t())
+
+
+def float_linear(x, w):
+    """linear(x, w).float(): a step's few rows in one launch."""
+    if _streams(x, w):
+        from ..serving._lib import check, lib
+        out = torch.empty((x.size(0), w.size(0)), dtype=torch.float32, device=x.device)
+        check(lib().qsv_skinny_linear_widened(out.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(), x.size(0), w.size(0), x.size(1),
+                                              torch.cuda.current_stream(x.device).cuda_stream), "skinny_linear_widened")
+        return out
+    return torch.matmul(x, w.t()).float()
 
 
 def _absorbed(q, w_uk):
@@ -918,6 +934,22 @@ class HipOps:
                                     float(tau), T, heads, dim, self.code, self._s()), "decay")
         return out
 
+    def decay_products(self, z, w, bias, a_log, tau, heads, dim, gate=None, w_gate=None):
+        """-> (decay(z w^T, bias, a_log, tau), gate w_gate^T or None): the second stages of a recurrence's low-rank decay and output gate, a step's few rows in
+        one launch."""
+        if (z.dtype == self.dtype == torch.bfloat16 and _streams(z, w) and (gate is None or _streams(gate, w_gate)) and (a_log is not None or tau > 0)
+                and w.size(0) == heads * dim):
+            T, N = z.size(0), w.size(0)
+            self._need(bias, a_log)
+            assert bias.dtype == self.dtype and bias.numel() == N and (a_log is None or (a_log.dtype == torch.float32 and a_log.numel() == heads))
+            out = torch.empty((T, N), dtype=torch.float32, device=z.device)
+            g = None if gate is None else torch.empty((T, w_gate.size(0)), dtype=self.dtype, device=z.device)
+            more = (0, 0, 0, 0, 0, 0) if gate is None else (g.data_ptr(), gate.data_ptr(), gate.stride(0), w_gate.data_ptr(), w_gate.size(0), w_gate.size(1))
+            self.check(self.L.qsv_decay_products(out.data_ptr(), z.data_ptr(), z.stride(0), w.data_ptr(), N, w.size(1), bias.data_ptr(),
+                                                 0 if a_log is None else a_log.data_ptr(), float(tau), dim, *more, T, self._s()), "decay_products")
+            return out, g
+        return self.decay(linear(z, w), bias, a_log, tau, heads, dim), None if gate is None else linear(gate, w_gate)
+
     def conv_silu_unit(self, proj, off, conv_w, hist, batch, n_unit, unit_dim, act="silu"):
         """Causal convolution over time of the columns [off, off + C) of proj with per-channel taps conv_w [C, taps], then silu
         (act "none": nothing), then the first n_unit groups of unit_dim channels made unit vectors.  hist: two-copy state, the last
@@ -1441,6 +1473,9 @@ class TorchOps:
             return torch.exp(-torch.nn.functional.softplus(-z) / tau).contiguous()          # sigmoid(z) ^ (1 / tau)
         rate = torch.exp(a_log.float()).repeat_interleave(dim)
         return torch.exp(-rate * torch.nn.functional.softplus(z)).contiguous()
+
+    def decay_products(self, z, w, bias, a_log, tau, heads, dim, gate=None, w_gate=None):
+        return self.decay(linear(z, w), bias, a_log, tau, heads, dim), None if gate is None else linear(gate, w_gate)
 
     def conv_silu_unit(self, proj, off, conv_w, hist, batch, n_unit, unit_dim, act="silu"):
         C, taps = conv_w.shape

@@ -48,8 +48,7 @@ class GatedLinearAttention:
         ops, H, d, dv = self.ops, self.H, self.dim, self.vdim
         proj = linear(h, self.w_in)
         o_q, o_k, o_v, o_g, o_a = 0, H * d, 2 * H * d, 2 * H * d + H * dv, 2 * H * d + 2 * H * dv
-        z = linear(proj[:, o_a:o_a + self.r], self.w_a2)
-        a = ops.decay(z, self.b_a2, None, self.tau, H, d)
+        a, _ = ops.decay_products(proj[:, o_a:o_a + self.r], self.w_a2, self.b_a2, None, self.tau, H, d)
         o = ops.recurrent_scan(proj[:, o_q:o_k], proj[:, o_k:o_v], proj[:, o_v:o_g], a, None, states[0], batch, H, H, d, dv,
                                d ** -0.5)
         return linear(ops.head_rms_gate(o, self.norm, proj[:, o_g:o_a], "silu", self.eps), self.w_o)
@@ -99,15 +98,16 @@ class GatedDeltaRule:
         o_b = self.C
         o_a, o_g = o_b + H, o_b + H + self.r
         qkv = ops.conv_silu_unit(proj, 0, self.conv, states[1], batch, 2 * G, d)       # float [T, C]: q | k (unit) | v
-        z = proj[:, o_a:o_g]
+        z, gate = proj[:, o_a:o_g], proj[:, o_g:o_g + self.rg]
         if self.head_decay:
             g = ops.decay(z, self.dt_bias, self.a_log, 0.0, H, 1)                      # float [T, H]
+            gate = linear(gate, self.w_g2) if self.low_gate else gate
         else:
-            g = ops.decay(linear(z, self.w_a2), self.dt_bias, self.a_log, 0.0, H, d)
+            g, low = ops.decay_products(z, self.w_a2, self.dt_bias, self.a_log, 0.0, H, d, *((gate, self.w_g2) if self.low_gate else ()))
+            gate = low if self.low_gate else gate
         o = ops.recurrent_scan(qkv[:, :G * d], qkv[:, G * d:2 * G * d], qkv[:, 2 * G * d:], g, proj[:, o_b:o_a], states[0], batch,
                                H, G, d, dv, d ** -0.5)
-        gate = proj[:, o_g:o_g + self.rg]
-        return linear(ops.head_rms_gate(o, self.norm, linear(gate, self.w_g2) if self.low_gate else gate, self.gate, self.eps), self.w_o)
+        return linear(ops.head_rms_gate(o, self.norm, gate, self.gate, self.eps), self.w_o)
 
 
 class Retention:

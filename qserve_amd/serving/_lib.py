@@ -13,6 +13,8 @@ SIGNATURES = {
     "qsv_arch": (C.c_char_p, []),
     "qsv_last_error": (C.c_char_p, []),
     "qsv_skinny_linear": (_i, [_vp, _vp, _i64, _vp, _i, _i, _i, _vp]),
+    "qsv_skinny_linear_widened": (_i, [_vp, _vp, _i64, _vp, _i, _i, _i, _vp]),
+    "qsv_decay_products": (_i, [_vp, _vp, _i64, _vp, _i, _i, _vp, _vp, _f, _i, _vp, _vp, _i64, _vp, _i, _i, _i, _vp]),
     "qsv_head_product_gated": (_i, [_vp, _vp, _i64, _i64, _vp, _i, _i, _i, _i, _vp, _i64, _vp]),
     "qsv_head_product": (_i, [_vp, _vp, _i64, _i64, _vp, _i, _i, _i, _i, _vp]),
     "qsv_latent_query_product": (_i, [_vp, _vp, _vp, _vp, _vp, _f, _i, _i, _i, _i, _i, _i, _vp]),

@@ -102,3 +102,31 @@ def test_convolved_heads(dtype, taps, runs):
     a, b = ops.conv_silu_unit(proj, 0, taps_of, h1, batch, 4, 8), ops.conv_silu_unit(proj, 0, off(taps_of), h2, batch, 4, 8)
     # eight squares added in another order, four products: some units of 2^-24 of values below 16
     assert ((a - b).abs() <= 1e-5).all() and torch.equal(h1, h2)
+
+
+# a recurrence's second stages in one launch: the bits of the launches one by one; edges of 16 and 32 rows, widths off the alignment, both kinds of decay
+@pytest.mark.parametrize("T", [1, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("H, dim, r, gate, rg, log", [(16, 64, 64, 0, 0, False), (3, 5, 24, 0, 0, True), (16, 128, 16, 2048, 136, True), (1, 17, 8, 40, 72, False)])
+def test_decay_products(T, H, dim, r, gate, rg, log):
+    from qserve_amd.layers.ops import float_linear, linear
+    ops, g = make(torch.bfloat16), torch.Generator().manual_seed(T + dim)
+    rnd = lambda *s: torch.randn(*s, generator=g).bfloat16().to(DEV)                                       # noqa: E731
+    proj, w, b, wg = rnd(T, r + rg + 16), rnd(H * dim, r) * 0.3, rnd(H * dim), rnd(gate, rg) if gate else None
+    a = torch.randn(H, generator=g).to(DEV) if log else None
+    z, x = proj[:, 8:8 + r], proj[:, 8 + r:8 + r + rg] if gate else None
+    d, y = ops.decay_products(z, w, b, a, 16.0, H, dim, x, wg)
+    assert torch.equal(d, ops.decay(linear(z, w), b, a, 16.0, H, dim)) and (y is None if not gate else torch.equal(y, linear(x, wg)))
+    assert torch.equal(float_linear(z, w), linear(z, w).float())
+    # ... and behind what the one launch takes
+    z = rnd(T, r)[:, 1:r - 7 + 1] if r > 16 else rnd(65, r)
+    w = w[:, :z.size(1)].contiguous()
+    assert torch.equal(ops.decay_products(z, w, b, a, 16.0, H, dim)[0], ops.decay(linear(z, w), b, a, 16.0, H, dim))
+
+
+@TYPES
+@pytest.mark.parametrize("T, D", [(1, 4), (3, 1028), (70, 2048)])
+def test_embeddings(dtype, T, D):
+    ops, g = make(dtype), torch.Generator().manual_seed(T + D)
+    table, tokens = torch.randn(9, D, generator=g).to(dtype).to(DEV), torch.randint(0, 9, (T,), generator=g, dtype=torch.int32).to(DEV)
+    assert all(torch.equal(a, b) for a, b in zip(ops.embed(tokens, table), ops.embed(tokens, off(table))))
+    assert torch.equal(ops.embed_streams(tokens, table, 1.7, 3), ops.embed_streams(tokens, off(table), 1.7, 3))

@@ -61,6 +61,7 @@ class PagedCache:
         self.pages = {}                                                # slot -> [page ids]
         self.length = {}                                               # slot -> tokens held
         self.table_host = torch.zeros((self.max_seqs, self.num_pages), dtype=torch.int32)
+        self.table_rows = self.table_host.numpy()                      # the same memory: [slot, page of the sequence] -> page id
         self.table = self.table_host.to(device)
         self._dirty = False
 
@@ -82,7 +83,7 @@ class PagedCache:
             raise CacheFull(f"{need} more pages needed, {len(self.free_pages)} free of {self.num_pages}")
         for _ in range(need):
             p = self.free_pages.pop()
-            self.table_host[slot, len(have)] = p
+            self.table_rows[slot, len(have)] = p                       # (an element of a tensor takes 40 times as long)
             have.append(p)
             self._dirty = True
         self.length[slot] = start + n
@@ -95,9 +96,21 @@ class PagedCache:
 
     def extend_array(self, slot, n):
         """`extend` for many tokens: the row indices as an int64 array."""
-        have, start = self._grow(slot, n)
-        j = np.arange(start, start + n, dtype=np.int64)
-        return np.array(have, dtype=np.int64)[j // self.page] * self.page + j % self.page
+        start = self._grow(slot, n)[1]
+        return self.rows_of(slot, np.arange(start, start + n, dtype=np.int64))
+
+    def extend_one(self, slot):
+        """`extend` for one token: -> (its row index, its position)."""
+        start = self.length[slot]
+        at = start % self.page
+        if not at:
+            return self.extend(slot, 1)[0], start
+        self.length[slot] = start + 1
+        return self.pages[slot][start // self.page] * self.page + at, start
+
+    def rows_of(self, slots, positions):
+        """The flat row indices of positions that sequences hold, slots and positions as arrays."""
+        return self.table_rows[slots, positions // self.page].astype(np.int64) * self.page + positions % self.page
 
     def step_rows(self, slot):
         """-> (row to read, row to write) of the two-copy states for this step of `slot`; the next step reads what this one

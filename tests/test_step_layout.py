@@ -129,3 +129,23 @@ def test_wanted_rows_are_whatever_int_takes(want):
     e.execute([(slots[0][0], [1, 2, 3])], want)
     assert seen[0].dtype == torch.int32 and seen[0].tolist() == [2, 0]
     assert e.execute([(slots[0][0], [4])], []) is None and len(seen) == 1
+
+
+@pytest.mark.parametrize("kinds", [(list, list), (list, tuple, np.array), (list, torch.tensor), (list, lambda t: [float(v) for v in t]), (list, lambda t: [_OnAnotherDevice(v) for v in t]),
+                                   (list, lambda t: [np.uint64(v) for v in t]), (list, lambda t: [str(v) for v in t])])
+@pytest.mark.parametrize("n", [1, 3])
+def test_runs_of_different_kinds_of_tokens(kinds, n):
+    e, plain, slots = _pair()
+    for step in range(3):
+        runs = [[(7 * i + 3 * step + j) % 100 for j in range(n)] for i in range(len(kinds))]
+        flat, *rest = e._layout_host([(slots[i][0], k(t)) for i, (k, t) in enumerate(zip(kinds, runs))])
+        T = n * len(kinds)
+        assert flat[2 * T:3 * T].tolist() == [v for t in runs for v in t]
+        assert flat[:2 * T].view(np.int64).tolist() == [r for i in range(len(kinds)) for r in plain.extend(slots[i][1], n)]
+        assert rest[2] == [n * step] * len(kinds)
+    before = [e.cache.length[s] for s, _ in slots]
+    with pytest.raises(ValueError, match="vocabulary"):
+        e._layout_host([(slots[0][0], [1] * n), (slots[1][0], [2] * (n - 1) + [100])])
+    assert [e.cache.length[s] for s, _ in slots] == before          # (nothing of a refused step stays)
+    with pytest.raises(KeyError):
+        e._layout_host([(slots[0][0], [1]), (77, [])])

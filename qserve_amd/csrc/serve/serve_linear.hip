@@ -22,14 +22,14 @@ struct SkinnyJob {
     float inv_tau;
     int dim;
 };
-template <int RB, int SG, int HOW>
+template <int RB, int SG, int HOW, bool ONCE>
 __device__ __forceinline__ void skinny_product(const SkinnyJob& a, int block, unsigned char* rings) {
     constexpr int TILES = RB * SG;
     static_assert(STREAM_WAVES * TILES * 1024 <= STREAM_WAVES * XRING, "");
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r0 = block * 16 * RB, t0 = blockIdx.y * 16 * SG, count = min(16 * SG, a.T - t0);
     v4f acc[RB][SG];
-    stream_products<RB, SG>(a.W + (size_t)r0 * a.K, a.K, min(16 * RB, a.N - r0), rings + w * XRING, w, lane,
+    stream_products<RB, SG, ONCE>(a.W + (size_t)r0 * a.K, a.K, min(16 * RB, a.N - r0), rings + w * XRING, w, lane,
                             [&](int i) { return a.X + (size_t)(t0 + min(i, count - 1)) * (size_t)a.x_stride; }, acc);
     v4f* red = (v4f*)rings;                                         // [wave][tile][lane]
     __syncthreads();                                                // every wave is done with its ring
@@ -79,17 +79,17 @@ __device__ __forceinline__ void skinny_product(const SkinnyJob& a, int block, un
         }
     }
 }
-template <int RB, int SG, int HOW>
+template <int RB, int SG, int HOW, bool ONCE>
 __global__ __launch_bounds__(64 * STREAM_WAVES, 2) void skinny_linear_kernel(SkinnyJob a) {
     __shared__ __attribute__((aligned(128))) unsigned char rings[STREAM_WAVES * XRING];
-    skinny_product<RB, SG, HOW>(a, blockIdx.x, rings);
+    skinny_product<RB, SG, HOW, ONCE>(a, blockIdx.x, rings);
 }
 // A recurrence's two second stages in one launch: the decay's product (its first `blocks` workgroups) and the output gate's (N 0: none)
 template <int SG>
 __global__ __launch_bounds__(64 * STREAM_WAVES, 2) void decay_products_kernel(SkinnyJob decay, SkinnyJob gate, int blocks) {
     __shared__ __attribute__((aligned(128))) unsigned char rings[STREAM_WAVES * XRING];
-    if ((int)blockIdx.x < blocks) skinny_product<1, SG, DECAY>(decay, blockIdx.x, rings);
-    else skinny_product<1, SG, AS_IS>(gate, blockIdx.x - blocks, rings);
+    if ((int)blockIdx.x < blocks) skinny_product<1, SG, DECAY, false>(decay, blockIdx.x, rings);
+    else skinny_product<1, SG, AS_IS, false>(gate, blockIdx.x - blocks, rings);
 }
 
 // ---- one product per head: y[t, h] = x[t, h] @ W[h], W [H, K, N] with N contiguous -------------------------------------------------------
@@ -251,9 +251,15 @@ static int launch_skinny(const char* what, void* out, const void* x, int64_t x_s
     // 16 weight rows per workgroup where 32 would leave CUs without one, or need a second round for a few (8256 x 2048: 11.4 -> 10.5 us); else 32,
     // which reads the inputs half as often (6144 x 2048: 8.2 -> 7.4 us)
     const bool few = n_rows <= 16, small = N < 5120 || (N > 8192 && N <= 16384 && n_rows <= 32);
+    // every weight is read once, or twice at the same time
+    const bool once = streams_once(w, N, K);
 #define QSV_SKINNY(RB, SG)                                                                                                                    \
-    hipLaunchKernelGGL((skinny_linear_kernel<RB, SG, HOW>), dim3((N + 16 * RB - 1) / (16 * RB), (n_rows + 16 * SG - 1) / (16 * SG)),          \
-                       dim3(64 * STREAM_WAVES), 0, (hipStream_t)stream, a)
+    do {                                                                                                                                      \
+        const dim3 grid((N + 16 * RB - 1) / (16 * RB), (n_rows + 16 * SG - 1) / (16 * SG)), block(64 * STREAM_WAVES);                         \
+        if (once && (grid.y == 1 || (int64_t)grid.x * grid.y <= 256))                                                                        \
+            hipLaunchKernelGGL((skinny_linear_kernel<RB, SG, HOW, true>), grid, block, 0, (hipStream_t)stream, a);                            \
+        else hipLaunchKernelGGL((skinny_linear_kernel<RB, SG, HOW, false>), grid, block, 0, (hipStream_t)stream, a);                          \
+    } while (0)
     if (few && small) QSV_SKINNY(1, 1);
     else if (few) QSV_SKINNY(2, 1);
     else if (small) QSV_SKINNY(1, 2);

@@ -6,6 +6,8 @@
 #include "serve_route.h"
 #include "serve_stream.h"
 
+#include <type_traits>
+
 namespace {
 constexpr int NT = 256;
 constexpr int NW = NT / 64;
@@ -427,6 +429,7 @@ struct ExpertArgs {
     float limit;
     bool wide;                       // out starts on 16 bytes
     bool stored;                     // gated units are made from their halves as a tensor would hold them
+    bool once;                       // weights that one reading may stream past the caches
 };
 // An expert every token goes through, of sizes of its own: X row t, out row t in bfloat16, the bits that the products and the activation give one by one.
 // W NULL: none.  Alone it took four launches, three of them at 4 - 5 us whatever they read (16 experts of 2048 x 1408 and one more, top 4, with the router,
@@ -435,7 +438,7 @@ struct SharedArgs {
     void* out;
     const bf16_t *X, *W;
     int n, rows, K;
-    bool wide;
+    bool wide, once;
 };
 
 // The four waves' partial sums (through LDS), the weight on the input, the activation, the store: slot of column c by slot_of(c).
@@ -508,21 +511,25 @@ __global__ __launch_bounds__(NT, 2) void expert_rows_kernel(ExpertArgs a, Shared
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r0 = blockIdx.x * XR;
     if (sh.W && blockIdx.y == 0) {                                                 // (first: it has the most inputs)
         if (r0 >= sh.rows) return;
-        const ExpertArgs b = {sh.out, sh.X, sh.W, nullptr, nullptr, nullptr, nullptr, sh.n, 1, sh.rows, sh.K, a.limit, sh.wide, true};
-        for (int c0 = 0; c0 < sh.n; c0 += 32) {
+        const ExpertArgs b = {sh.out, sh.X, sh.W, nullptr, nullptr, nullptr, nullptr, sh.n, 1, sh.rows, sh.K, a.limit, sh.wide, true, false};
+        auto chunk = [&](int c0, auto once) __attribute__((always_inline)) {
+            constexpr bool ONCE = decltype(once)::value;
             const int c = min(32, sh.n - c0);
             auto rows = [&](int i) { return sh.X + (size_t)(c0 + min(i, c - 1)) * (size_t)sh.K; };
             auto slots = [&](int i, int64_t& slot, float&) { slot = c0 + i; };
             if (c <= 16) {
                 v4f acc[XR / 16][1];
-                stream_products<XR / 16, 1>(sh.W + (size_t)r0 * sh.K, sh.K, min(XR, sh.rows - r0), rings + w * XRING, w, lane, rows, acc);
+                stream_products<XR / 16, 1, ONCE>(sh.W + (size_t)r0 * sh.K, sh.K, min(XR, sh.rows - r0), rings + w * XRING, w, lane, rows, acc);
                 expert_finish<ACT, false, 1>(b, r0, c, rings, w, lane, slots, acc);
             } else {
                 v4f acc[XR / 16][2];
-                stream_products<XR / 16, 2>(sh.W + (size_t)r0 * sh.K, sh.K, min(XR, sh.rows - r0), rings + w * XRING, w, lane, rows, acc);
+                stream_products<XR / 16, 2, ONCE>(sh.W + (size_t)r0 * sh.K, sh.K, min(XR, sh.rows - r0), rings + w * XRING, w, lane, rows, acc);
                 expert_finish<ACT, false, 2>(b, r0, c, rings, w, lane, slots, acc);
             }
-        }
+        };
+        if (sh.n <= 32 && sh.once) chunk(0, std::true_type());
+        else
+            for (int c0 = 0; c0 < sh.n; c0 += 32) chunk(c0, std::false_type());
         return;
     }
     if (r0 >= a.rows) return;
@@ -531,20 +538,25 @@ __global__ __launch_bounds__(NT, 2) void expert_rows_kernel(ExpertArgs a, Shared
     unsigned char* ring = rings + w * XRING;
     // `count` inputs: X row by row_of(i), output row (and weight) by slot_of(i)
     auto walk = [&](int count, auto row_of, auto slot_of) {
-        for (int c0 = 0; c0 < count; c0 += 32) {
+        auto chunk = [&](int c0, auto once) __attribute__((always_inline)) {
+            constexpr bool ONCE = decltype(once)::value;
             const int c = min(32, count - c0);
             auto rows = [&](int i) { return a.X + (size_t)row_of(c0 + min(i, c - 1)) * (size_t)a.K; };
             auto slots = [&](int i, int64_t& slot, float& iw) { slot_of(c0 + i, slot, iw); };
             if (c <= 16) {
                 v4f acc[XR / 16][1];
-                stream_products<XR / 16, 1>(W0, a.K, rows_here, ring, w, lane, rows, acc);
+                stream_products<XR / 16, 1, ONCE>(W0, a.K, rows_here, ring, w, lane, rows, acc);
                 expert_finish<ACT, FOUT, 1>(a, r0, c, rings, w, lane, slots, acc);
             } else {
                 v4f acc[XR / 16][2];
-                stream_products<XR / 16, 2>(W0, a.K, rows_here, ring, w, lane, rows, acc);
+                stream_products<XR / 16, 2, ONCE>(W0, a.K, rows_here, ring, w, lane, rows, acc);
                 expert_finish<ACT, FOUT, 2>(a, r0, c, rings, w, lane, slots, acc);
             }
-        }
+        };
+        if (count <= 0) return;
+        if (count <= 32 && a.once) chunk(0, std::true_type());
+        else
+            for (int c0 = 0; c0 < count; c0 += 32) chunk(c0, std::false_type());
     };
     if (a.offsets) {
         const int64_t s0 = a.offsets[e];
@@ -661,6 +673,8 @@ static int launch_expert_rows(const char* what, ExpertArgs a, int n_experts, int
     QSV_REQUIRE(n_experts <= 65535, "%s: too many experts", what);
     QSV_REQUIRE(((uintptr_t)a.X | (uintptr_t)a.W) % 16 == 0, "%s: inputs and weights start on 16 bytes", what);
     a.wide = (uintptr_t)a.out % 16 == 0;
+    a.once = streams_once(a.W, (int64_t)n_experts * a.rows, a.K);
+    sh.once = streams_once(sh.W, sh.rows, sh.K);
     const dim3 grid(((sh.W && sh.rows > a.rows ? sh.rows : a.rows) + XR - 1) / XR, n_experts + (sh.W ? 1 : 0)), block(NT);
     if (float_out) hipLaunchKernelGGL((expert_rows_kernel<ACT_NONE, true>), grid, block, 0, (hipStream_t)stream, a, sh);
     else if (act == ACT_RELU_SQ) hipLaunchKernelGGL((expert_rows_kernel<ACT_RELU_SQ, false>), grid, block, 0, (hipStream_t)stream, a, sh);
@@ -671,14 +685,14 @@ static int launch_expert_rows(const char* what, ExpertArgs a, int n_experts, int
 extern "C" int qsv_expert_rows(void* out, const void* X, const int64_t* x_index, int div, const void* W, const int64_t* offsets,
                                int n_experts, int rows, int K, int act, float limit, const float* in_weight, void* stream) {
     QSV_REQUIRE(offsets, "qsv_expert_rows: bad arguments");
-    const ExpertArgs a = {out, (const bf16_t*)X, (const bf16_t*)W, nullptr, x_index, offsets, in_weight, 0, div, rows, K, limit, false, false};
+    const ExpertArgs a = {out, (const bf16_t*)X, (const bf16_t*)W, nullptr, x_index, offsets, in_weight, 0, div, rows, K, limit, false, false, false};
     return launch_expert_rows("qsv_expert_rows", a, n_experts, act, false, stream);
 }
 extern "C" int qsv_expert_slots(void* out, int float_out, const void* X, int div, const void* W, const int32_t* idx, int n, int n_experts, int rows,
                                 int K, int act, float limit, const float* in_weight, void* stream) {
     QSV_REQUIRE(idx && n >= 0 && (!float_out || act == ACT_NONE), "qsv_expert_slots: bad arguments");
     if (n == 0) return QSV_OK;
-    const ExpertArgs a = {out, (const bf16_t*)X, (const bf16_t*)W, idx, nullptr, nullptr, in_weight, n, div, rows, K, limit, false, false};
+    const ExpertArgs a = {out, (const bf16_t*)X, (const bf16_t*)W, idx, nullptr, nullptr, in_weight, n, div, rows, K, limit, false, false, false};
     return launch_expert_rows("qsv_expert_slots", a, n_experts, act, float_out != 0, stream);
 }
 // ... and every token's row of X through a shared expert of sh_rows x sh_K in the same launch: sh_out [n / div, sh_rows (/ 2 for gated units)]
@@ -689,9 +703,9 @@ extern "C" int qsv_expert_slots_shared(void* out, int float_out, const void* X, 
     QSV_REQUIRE(sh_K > 0 && sh_K % 8 == 0 && sh_K <= 1 << 25 && ((uintptr_t)sh_X | (uintptr_t)sh_W) % 16 == 0, "qsv_expert_slots_shared: inner width %d, rows on 16 bytes", sh_K);
     QSV_REQUIRE(act == ACT_NONE || act == ACT_RELU_SQ || sh_rows % 2 == 0, "qsv_expert_slots_shared: %d rows of gated units", sh_rows);
     if (n == 0) return QSV_OK;
-    const ExpertArgs a = {out, (const bf16_t*)X, (const bf16_t*)W, idx, nullptr, nullptr, in_weight, n, div, rows, K, limit, false, false};
+    const ExpertArgs a = {out, (const bf16_t*)X, (const bf16_t*)W, idx, nullptr, nullptr, in_weight, n, div, rows, K, limit, false, false, false};
     return launch_expert_rows("qsv_expert_slots_shared", a, n_experts, act, float_out != 0, stream,
-                              {sh_out, (const bf16_t*)sh_X, (const bf16_t*)sh_W, sh_n, sh_rows, sh_K, (uintptr_t)sh_out % 16 == 0});
+                              {sh_out, (const bf16_t*)sh_X, (const bf16_t*)sh_W, sh_n, sh_rows, sh_K, (uintptr_t)sh_out % 16 == 0, false});
 }
 extern "C" int qsv_relu_sq(void* a, int64_t n, int dtype, void* stream) {
     QSV_REQUIRE(a && n >= 0 && n < (1ll << 31) * NT, "qsv_relu_sq: bad arguments");

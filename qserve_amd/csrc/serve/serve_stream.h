@@ -25,16 +25,24 @@ template <int N>
 __device__ __forceinline__ void wait_vm() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
+// ONCE: nothing reads these lines again (non-temporal: they leave the caches to what is read again)
+template <bool ONCE>
 __device__ __forceinline__ void lds_copy16(unsigned dst, const void* base, unsigned off) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(dst) : "memory");
+    if constexpr (ONCE) asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(off), "s"(base), "s"(dst) : "memory");
+    else asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(dst) : "memory");
 }
 __device__ __forceinline__ void lds_copy16(unsigned dst, const void* from) {
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(dst) : "memory");
 }
 
+// ONCE: the launch reads every weight once, so non-temporally: a large stream gets 4 - 10 % faster (92 / 185 MB of experts 21.5 / 39.1 -> 19.5 / 36.8 us, 4096 x 4096
+// 8.9 -> 8.5; weights that a cache holds from step to step, less than 200 MB in all, lose as much).  Where workgroups read the same rows one after another, or rows
+// start inside a line of 128 bytes, whose halves two requests would fetch, it loses (2560 x 5120 read twice 16.1 -> 20.7).
+// Under 1 MB, which a cache keeps beside anything, it loses too (64 x 2048 of 64 inputs 5.0 -> 5.6).
+inline bool streams_once(const void* w, int64_t rows, int K) { return K % 64 == 0 && (uintptr_t)w % 128 == 0 && rows * K >= 1 << 19; }
 // acc[r][g]: this wave's share of the products of weight rows W0 + 16 r + .. (rows_here of them, K elements each) with inputs 16 g + ..;
 // input(i): where input i starts.  w (the wave) is wave-uniform; `ring`: its XRING bytes of LDS.
-template <int RB, int SG, class Input>
+template <int RB, int SG, bool ONCE, class Input>
 __device__ __forceinline__ void stream_products(const bf16_t* W0, int K, int rows_here, unsigned char* ring, int w, int lane, Input input,
                                                 v4f (&acc)[RB][SG]) {
     typedef StreamRing<RB, SG> R;
@@ -56,7 +64,7 @@ __device__ __forceinline__ void stream_products(const bf16_t* W0, int K, int row
         const unsigned po = k0 + piece * 8 < K ? (unsigned)piece * 16u : 0u;       // (beyond the row: any valid piece, masked below)
         const unsigned dst = lds0 + (unsigned)(i % R::DEPTH) * R::STAGE;
 #pragma unroll
-        for (int j = 0; j < 2 * RB; ++j) lds_copy16(dst + 1024 * j, W0 + k0, woff[j] + po);
+        for (int j = 0; j < 2 * RB; ++j) lds_copy16<ONCE>(dst + 1024 * j, W0 + k0, woff[j] + po);
 #pragma unroll
         for (int j = 0; j < 2 * SG; ++j) lds_copy16(dst + 1024 * (2 * RB + j), (const unsigned char*)(xrow[j] + k0) + po);
     };

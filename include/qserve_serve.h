@@ -41,6 +41,13 @@ int qsv_head_product_gated(void* out, const void* x, int64_t x_tok, int64_t x_he
 int qsv_latent_query_product(float* qf, const void* q, const void* w_uk, const float* rope, const int32_t* pos, float scale, int n_tokens, int heads,
                              int dim, int rot_dim, int rot_n, int rank, void* stream);
 
+/* out[0 .. n) (device, 32-bit words) = host_words[0 .. n), which may change when the call returns: they travel in the launches' arguments (at most
+ * qsv_step_words_most).  qsv_copy_words: the same between device addresses on 16 bytes, any n. */
+int qsv_step_words_most(void);
+int qsv_set_words(void* out, const void* host_pairs, int n, void* stream);    /* out[place] = word for n <= 480 pairs, no place twice */
+int qsv_step_words(void* out, const void* host_words, int n, void* stream);
+int qsv_copy_words(void* out, const void* in, int64_t n, void* stream);
+
 /* x[t] = table[tokens[t]] (float) and h[t] = the same row in the storage type. */
 int qsv_embed(float* x, void* h, const void* table, const int32_t* tokens, int n_tokens, int width, int dtype, void* stream);
 

@@ -3,6 +3,8 @@
 #include "serve_common.h"
 #include "serve_route.h"
 
+#include <string.h>
+
 #include <type_traits>
 
 static thread_local char g_err[512] = "";
@@ -43,6 +45,51 @@ __global__ __launch_bounds__(NT) void embed_vec_kernel(float* __restrict__ x, T*
     st4t(x, t * D + i, v);
     *(typename Raw4<T>::type*)(h + t * D + i) = r;
 }
+// A step's words (rows, positions, slots ...) travel in the launch's arguments, its logits leave through a kernel: a copy command waits for the stream on both
+// sides (a step of 64 sequences 22 us, of one 10 us).
+constexpr int STEP_WORDS = 960;
+struct StepWords {
+    uint32_t w[STEP_WORDS];
+};
+__global__ __launch_bounds__(NT) void step_words_kernel(uint32_t* __restrict__ out, StepWords words, int n) {
+    for (int i = threadIdx.x; i < n; i += NT) out[i] = words.w[i];
+}
+__global__ __launch_bounds__(NT) void copy_words_kernel(uint32_t* __restrict__ out, const uint32_t* __restrict__ in, int64_t n) {
+    const int64_t i = ((int64_t)blockIdx.x * NT + threadIdx.x) * 4;
+    if (i + 4 <= n) *(uint4*)(out + i) = *(const uint4*)(in + i);
+    else
+        for (int64_t j = i; j < n; ++j) out[j] = in[j];
+}
+__global__ __launch_bounds__(NT) void set_words_kernel(uint32_t* __restrict__ out, StepWords pairs, int n) {
+    for (int i = threadIdx.x; i < n; i += NT) out[pairs.w[2 * i]] = pairs.w[2 * i + 1];
+}
+// out[place] = word for up to STEP_WORDS / 2 pairs (place, word), every place at most once
+extern "C" int qsv_set_words(void* out, const void* host_pairs, int n, void* stream) {
+    QSV_REQUIRE(n >= 0 && n <= STEP_WORDS / 2 && (n == 0 || (out && host_pairs)), "qsv_set_words: %d pairs (at most %d)", n, STEP_WORDS / 2);
+    if (n == 0) return QSV_OK;
+    StepWords pairs;
+    memcpy(pairs.w, host_pairs, 8 * (size_t)n);
+    hipLaunchKernelGGL(set_words_kernel, dim3(1), dim3(NT), 0, (hipStream_t)stream, (uint32_t*)out, pairs, n);
+    return qsv_launch_status("qsv_set_words");
+}
+extern "C" int qsv_step_words_most(void) { return 4 * STEP_WORDS; }
+extern "C" int qsv_step_words(void* out, const void* host_words, int n, void* stream) {
+    QSV_REQUIRE(n >= 0 && n <= 4 * STEP_WORDS && (n == 0 || (out && host_words)), "qsv_step_words: %d words (at most %d)", n, 4 * STEP_WORDS);
+    StepWords words;
+    for (int at = 0; at < n; at += STEP_WORDS) {
+        const int here = n - at < STEP_WORDS ? n - at : STEP_WORDS;
+        memcpy(words.w, (const uint32_t*)host_words + at, 4 * (size_t)here);
+        hipLaunchKernelGGL(step_words_kernel, dim3(1), dim3(NT), 0, (hipStream_t)stream, (uint32_t*)out + at, words, here);
+    }
+    return qsv_launch_status("qsv_step_words");
+}
+extern "C" int qsv_copy_words(void* out, const void* in, int64_t n, void* stream) {
+    QSV_REQUIRE(n >= 0 && n < (1ll << 40) && (n == 0 || (out && in && ((uintptr_t)out | (uintptr_t)in) % 16 == 0)), "qsv_copy_words: bad arguments");
+    if (n == 0) return QSV_OK;
+    hipLaunchKernelGGL(copy_words_kernel, dim3((unsigned)((n + 4 * NT - 1) / (4 * NT))), dim3(NT), 0, (hipStream_t)stream, (uint32_t*)out, (const uint32_t*)in, n);
+    return qsv_launch_status("qsv_copy_words");
+}
+
 extern "C" int qsv_embed(float* x, void* h, const void* table, const int32_t* tokens, int n, int D, int dtype, void* stream) {
     QSV_REQUIRE(x && h && table && tokens && n >= 0 && D > 0, "qsv_embed: bad arguments");
     if (n == 0) return QSV_OK;

@@ -8,6 +8,7 @@
 Conventions: `x` is the float residual stream [T, D]; `h` and every other activation is in the storage type (bfloat16 or
 float32); matrix products (`linear`, the products per head) are own kernels for a step's few rows and the vendor's beyond, with float accumulation.
 """
+import numpy as np
 import torch
 from torch.autograd import forward_ad
 
@@ -169,6 +170,23 @@ class HipOps:
         for t in ts:
             if t is not None and not (t.is_cuda and t.is_contiguous()):
                 raise RuntimeError("serving kernels need contiguous tensors on the GPU")
+
+    def put_words(self, out, words):
+        """out (int32, on the GPU) = words (a numpy int32 array), which the caller may change at once."""
+        n = words.size
+        assert out.dtype == torch.int32 and out.numel() == n and out.is_cuda and out.is_contiguous() and words.dtype == np.int32 and words.flags.c_contiguous
+        if n <= self.L.qsv_step_words_most():
+            self.check(self.L.qsv_step_words(out.data_ptr(), words.ctypes.data, n, self._s()), "step_words")
+        else:
+            out.copy_(torch.empty(words.shape, dtype=torch.int32, pin_memory=True).copy_(torch.from_numpy(words)), non_blocking=True)
+
+    def copied(self, t):
+        """t.clone() of a contiguous tensor of 32-bit elements, by a kernel."""
+        if t.element_size() != 4 or not t.is_contiguous() or t.data_ptr() % 16:
+            return t.clone()
+        out = torch.empty_like(t)
+        self.check(self.L.qsv_copy_words(out.data_ptr(), t.data_ptr(), t.numel(), self._s()), "copy_words")
+        return out
 
     def embed(self, tokens, table):
         T, D = tokens.numel(), table.size(1)

@@ -18,6 +18,10 @@ SIGNATURES = {
     "qsv_head_product_gated": (_i, [_vp, _vp, _i64, _i64, _vp, _i, _i, _i, _i, _vp, _i64, _vp]),
     "qsv_head_product": (_i, [_vp, _vp, _i64, _i64, _vp, _i, _i, _i, _i, _vp]),
     "qsv_latent_query_product": (_i, [_vp, _vp, _vp, _vp, _vp, _f, _i, _i, _i, _i, _i, _i, _vp]),
+    "qsv_step_words_most": (_i, []),
+    "qsv_step_words": (_i, [_vp, _vp, _i, _vp]),
+    "qsv_set_words": (_i, [_vp, _vp, _i, _vp]),
+    "qsv_copy_words": (_i, [_vp, _vp, _i64, _vp]),
     "qsv_embed": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _vp]),
     "qsv_add_layer_norm_slots": (_i, [_vp, _vp, _vp, _i, _vp, _vp, _vp, _i, _i, _vp, _f, _i, _i, _i, _vp]),
     "qsv_add_layer_norm": (_i, [_vp, _vp, _vp, _vp, _f, _i, _i, _i, _vp]),

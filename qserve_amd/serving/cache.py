@@ -16,6 +16,8 @@ A sequence's state is never cleared: kernels take a run that starts at position 
 import numpy as np
 import torch
 
+from ._lib import check, lib
+
 
 def upload(a, device):
     """numpy array -> tensor on `device`.  To a GPU through a pinned buffer and without waiting for the copy (torch hands a pinned buffer
@@ -64,6 +66,7 @@ class PagedCache:
         self.table_rows = self.table_host.numpy()                      # the same memory: [slot, page of the sequence] -> page id
         self.table = self.table_host.to(device)
         self._dirty = False
+        self._entered = {}                                             # place in the table -> page id, since the last upload
 
     def pages_for(self, tokens):
         return (tokens + self.page - 1) // self.page
@@ -84,6 +87,7 @@ class PagedCache:
         for _ in range(need):
             p = self.free_pages.pop()
             self.table_rows[slot, len(have)] = p                       # (an element of a tensor takes 40 times as long)
+            self._entered[slot * self.num_pages + len(have)] = p
             have.append(p)
             self._dirty = True
         self.length[slot] = start + n
@@ -127,9 +131,12 @@ class PagedCache:
     def block_table(self):
         """The device copy of the block table, uploaded if pages were handed out since the last call."""
         if self._dirty:
-            if self.table.is_cuda:                                     # (a pinned copy: the host's table may change before the device has read it)
+            if self.table.is_cuda and len(self._entered) <= 480:       # (a step's few: no copy command, and no more than what is new)
+                new = np.array(list(self._entered.items()), dtype=np.int32)
+                check(lib().qsv_set_words(self.table.data_ptr(), new.ctypes.data, len(new), torch.cuda.current_stream(self.table.device).cuda_stream), "set_words")
+            elif self.table.is_cuda:                                     # (a pinned copy: the host's table may change before the device has read it)
                 self.table.copy_(torch.empty(self.table_host.shape, dtype=torch.int32, pin_memory=True).copy_(self.table_host), non_blocking=True)
             else:
                 self.table.copy_(self.table_host)
-            self._dirty = False
+            self._dirty, self._entered = False, {}
         return self.table

@@ -237,7 +237,7 @@ class Engine:
                 if not want:
                     return None
                 want = [int(v) for v in want]
-                return out.clone() if want == list(range(out.size(0))) else out[upload(np.array(want, dtype=np.int64), self.device)]
+                return self.ops.copied(out) if want == list(range(out.size(0))) else out[upload(np.array(want, dtype=np.int64), self.device)]
         batch = self._batch_of(upload(host[0], self.device), *host[1:])
         x = self._forward(batch)
         if not want:
@@ -290,7 +290,7 @@ class Engine:
                 return None
             self._graphs[key] = G
         else:
-            G["flat"].copy_(torch.empty(flat.shape, dtype=torch.int32, pin_memory=True).copy_(torch.from_numpy(flat)), non_blocking=True)
+            self.ops.put_words(G["flat"], flat)
         self.cache.block_table()
         G["graph"].replay()
         return G["logits"]

@@ -1,4 +1,5 @@
 """Row kernels that take four columns a thread against their forms for any width and address: the same operands a few elements off the alignment."""
+import numpy as np
 import pytest
 import torch
 
@@ -130,3 +131,35 @@ def test_embeddings(dtype, T, D):
     table, tokens = torch.randn(9, D, generator=g).to(dtype).to(DEV), torch.randint(0, 9, (T,), generator=g, dtype=torch.int32).to(DEV)
     assert all(torch.equal(a, b) for a, b in zip(ops.embed(tokens, table), ops.embed(tokens, off(table))))
     assert torch.equal(ops.embed_streams(tokens, table, 1.7, 3), ops.embed_streams(tokens, off(table), 1.7, 3))
+
+
+@pytest.mark.parametrize("n", [0, 1, 255, 960, 961, 3839, 3840, 3841, 9000])
+def test_words_of_a_step(n):
+    ops, g = make(torch.bfloat16), np.random.default_rng(n)
+    out, words = torch.full((n + 1,), -7, dtype=torch.int32, device=DEV), g.integers(-2 ** 31, 2 ** 31, n, dtype=np.int64).astype(np.int32)
+    keep = words.copy()
+    ops.put_words(out[:n], words)
+    words[:] = 0                                                         # (the caller's array is its own again)
+    assert out[:n].tolist() == keep.tolist() and int(out[n]) == -7
+    t = torch.randn(3, n, device=DEV)
+    for v in (t, t.bfloat16(), t.t(), off(t)):
+        c = ops.copied(v)
+        assert torch.equal(c, v) and (n == 0 or c.data_ptr() != v.data_ptr())
+
+
+def test_block_table_on_the_device_is_the_hosts():
+    make(torch.bfloat16)
+    from qserve_amd.serving.cache import PagedCache
+    cache = PagedCache([4], num_pages=1400, max_seqs=5, dtype=torch.bfloat16, device=DEV, page=8)
+    slots = [cache.admit() for _ in range(5)]
+    for step in ([1] * 5, [7, 8, 9, 200, 1], [3840, 8, 0, 3000, 5], [1] * 5, [8] * 5, [8] * 5):       # (one page to more than travel with a launch)
+        for s, n in zip(slots, step):
+            if n:
+                cache.extend(s, n)
+        assert torch.equal(cache.block_table().cpu(), cache.table_host)
+        for _ in range(3):                                               # (the same places again and again, before they are uploaded)
+            cache.release(slots[1])
+            cache.extend(slots[0], 9)
+            slots[1] = cache.admit()
+            cache.extend(slots[1], 17)
+        assert torch.equal(cache.block_table().cpu(), cache.table_host)

@@ -231,11 +231,17 @@ class DecodeEngine:
         self.gate_up_buf = torch.empty((B, 2 * inter), dtype=f16, device=self.dev)
         self.mlp_act = torch.empty((B, inter), dtype=f16, device=self.dev)
         self.final = torch.empty((B, hid), dtype=f16, device=self.dev)
-        # K-slice planes (qserve_amd.fused.gemm_planes): the row-parallel projections named in `planes` (default: QS_PLANES or
-        # "down") leave int32 partial sums per K slice and the add + norm + quant launch behind them finishes the GEMM - where
+        # K-slice planes (qserve_amd.fused.gemm_planes): the row-parallel projections named in `planes` (default: QS_PLANES, else
+        # by rows, below) leave int32 partial sums per K slice and the add + norm + quant launch behind them finishes the GEMM - where
         # the pair fusions are on, on one GPU, for shapes the library has such a launch for
-        if planes is None:
-            planes = tuple(x for x in os.environ.get("QS_PLANES", "down").split(",") if x)
+        if planes is None and os.environ.get("QS_PLANES") is not None:
+            planes = tuple(x for x in os.environ["QS_PLANES"].split(",") if x)
+        elif planes is None:
+            # `o` has few output blocks for the chip (64 of 4096 channels, 256 with four slices), but no seam to save: with few rows the shorter
+            # launch outweighs the planes' bytes, with per-group weights (whose unpacking is the launch) for longer.  Four layers, without /
+            # with, us: per-channel 2 / 8 / 16 / 24 / 128 rows 215 / 211, 222 / 218, 232 / 229, 236 / 238, 395 / 399; groups of 128, 1 / 32 / 64 / 128
+            # rows 278 / 266, 294 / 286, 340 / 337, 455 / 456
+            planes = ("o", "down") if batch <= (64 if group_size != -1 else 16) else ("down",)
         bad = [x for x in planes if x not in ("o", "down")]
         if bad:
             raise ValueError(f"planes / QS_PLANES: {bad} - only the row-parallel projections 'o' and 'down' have a planes form")

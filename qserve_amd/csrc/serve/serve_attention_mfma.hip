@@ -373,6 +373,17 @@ __global__ __launch_bounds__(64 * RW, RT + CT > 24 ? 2 : 4) void latent_rows_ker
                              : "memory");
             }
     };
+    // the query row, whole before anything is rounded: rounded under its condition, every piece waited for the one before
+    float4 q[RT][2];
+    {
+        const float* qrow = qf + ((size_t)t * H + (row_ok ? head : h0)) * (size_t)R + 8 * g4;
+#pragma unroll
+        for (int s = S0; s < RT; ++s) {
+            q[s][0] = *(const float4*)(qrow + 32 * s);
+            q[s][1] = *(const float4*)(qrow + 32 * s + 4);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
     const int Z = gridDim.z, z = blockIdx.z;
     auto page_of = [&](int tile) __attribute__((always_inline)) { return bt[(kstart + min(tile, nT - 1) * BN) / page]; };
     int next_page = 0;
@@ -381,17 +392,10 @@ __global__ __launch_bounds__(64 * RW, RT + CT > 24 ? 2 : 4) void latent_rows_ker
         next_page = page_of(z + Z);
     }
     v4u qfrag[RT];
-    {
-        const float* qrow = qf + ((size_t)t * H + (row_ok ? head : h0)) * (size_t)R;
+    const unsigned kept = row_ok ? ~0u : 0u;
 #pragma unroll
-        for (int s = 0; s < RT; ++s) {
-            qfrag[s] = v4u{0u, 0u, 0u, 0u};
-            if (row_ok && s >= S0) {
-                const float4 a = *(const float4*)(qrow + 32 * s + 8 * g4), b = *(const float4*)(qrow + 32 * s + 8 * g4 + 4);
-                qfrag[s] = v4u{pack_bf2(a.x, a.y), pack_bf2(a.z, a.w), pack_bf2(b.x, b.y), pack_bf2(b.z, b.w)};
-            }
-        }
-    }
+    for (int s = S0; s < RT; ++s)
+        qfrag[s] = v4u{pack_bf2(q[s][0].x, q[s][0].y), pack_bf2(q[s][0].z, q[s][0].w), pack_bf2(q[s][1].x, q[s][1].y), pack_bf2(q[s][1].z, q[s][1].w)} & kept;
     v4f oacc[CT];
 #pragma unroll
     for (int c = 0; c < CT; ++c) oacc[c] = v4f{0.f, 0.f, 0.f, 0.f};
@@ -516,8 +520,13 @@ __global__ __launch_bounds__(64 * RW, RT + CT > 24 ? 2 : 4) void latent_rows_ker
 // rounds of 64 keys, copied as above (two rounds in turn); a wave scores 16 of the keys (its rows of K only), the maximum and the
 // probabilities of a round meet in LDS, and a wave multiplies them with its quarter of the value columns.  Bound by latency at short contexts, by
 // HBM at long ones.
-// Measured (16 heads, 576 / 512, best split each, kernel above -> this one and the merge below): 64 sequences at 128 / 1000 / 2000 positions 15 -> 12 / 31 ->
-// 28 / 44 -> 37 us, 16 at 1000 25 -> 18, one at 300 / 2000 17 -> 13 / 28 -> 16; 256 / 128, 16 heads on 4 pools, 16 sequences at 1000: 15 -> 11.5 us.
+// Its chain is the launch: tiles, positions and pages, the queries, the first keys.  The queries are requested first, all of them, and rounded
+// before the keys' copies are (rounded under their condition, each of the 18 pairs waited for the one before; rounded behind the copies, the wait
+// is for those too); then two rounds are in flight, the next two pages with them: in a step of 64 sequences at 50 - 150 positions 576 / 512 16.5 ->
+// 13.4 us and 512 / 512 15.1 -> 12.3 (13.7 and 12.4 with one round ahead), 16 sequences at 100 - 220 of 256 / 128 8.7 -> 7.2.
+// Measured alone, its queries in the caches (16 heads, 576 / 512, best split each, kernel above -> this one and the merge below): 64 sequences at 128 / 1000 /
+// 2000 positions 15 -> 12.5 / 31 -> 26 / 44 -> 36 us, 16 at 1000 25 -> 18, one at 300 / 2000 17 -> 14.5 / 28 -> 17.5; 256 / 128, 16 heads on 4 pools, 16
+// sequences at 1000: 15 -> 10.8 us.
 constexpr int SW = 4, SN = 64;       // waves, keys of a round
 template <int RT, int CT, int S0>
 __global__ __launch_bounds__(64 * SW, 1) void latent_step_kernel(
@@ -539,6 +548,17 @@ __global__ __launch_bounds__(64 * SW, 1) void latent_step_kernel(
     const int32_t* bt = block_table + (size_t)slot * table_stride;
     const int head = h0 + col;
     const bool row_ok = col < HP && head < h_end;
+    // the query row, whole before anything is rounded: rounded under its condition, every piece waited for the one before
+    float4 q[RT][2];
+    {
+        const float* qrow = qf + ((size_t)t * H + (row_ok ? head : h0)) * (size_t)R + 8 * g4;
+#pragma unroll
+        for (int s = S0; s < RT; ++s) {
+            q[s][0] = *(const float4*)(qrow + 32 * s);
+            q[s][1] = *(const float4*)(qrow + 32 * s + 4);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
     const int p_row = __builtin_amdgcn_readfirstlane(pos[t]), lo_row = window > 0 ? max(0, p_row - window + 1) : 0;
     const int kstart = lo_row / BN * BN, nT = (p_row - kstart) / SN + 1, last_half = (p_row - kstart) / BN;
     const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(lds_ptr)buf);
@@ -559,24 +579,22 @@ __global__ __launch_bounds__(64 * SW, 1) void latent_step_kernel(
     };
     const int Z = gridDim.z, z = blockIdx.z;
     auto page_of = [&](int half) __attribute__((always_inline)) { return bt[(kstart + min(half, last_half) * BN) / page]; };
-    auto copy = [&](int round, int which) __attribute__((always_inline)) {
-        const int a = __builtin_amdgcn_readfirstlane(page_of(2 * round)), b = __builtin_amdgcn_readfirstlane(page_of(2 * round + 1));
-        copy_half(2 * round, a, which * TILE);
-        copy_half(2 * round + 1, b, which * TILE + TILE / 2);
+    auto copy = [&](int round, int which, int page_a, int page_b) __attribute__((always_inline)) {
+        copy_half(2 * round, __builtin_amdgcn_readfirstlane(page_a), which * TILE);
+        copy_half(2 * round + 1, __builtin_amdgcn_readfirstlane(page_b), which * TILE + TILE / 2);
     };
-    if (z < nT) copy(z, 0);
+    const int a0 = page_of(2 * z), b0 = page_of(2 * z + 1), a1 = page_of(2 * (z + Z)), b1 = page_of(2 * (z + Z) + 1);
+    int next_a = page_of(2 * (z + 2 * Z)), next_b = page_of(2 * (z + 2 * Z) + 1);
+    __builtin_amdgcn_sched_barrier(0);
     v4u qfrag[RT];
-    {
-        const float* qrow = qf + ((size_t)t * H + (row_ok ? head : h0)) * (size_t)R;
+    const unsigned kept = row_ok ? ~0u : 0u;
 #pragma unroll
-        for (int s = 0; s < RT; ++s) {
-            qfrag[s] = v4u{0u, 0u, 0u, 0u};
-            if (row_ok && s >= S0) {
-                const float4 a = *(const float4*)(qrow + 32 * s + 8 * g4), b = *(const float4*)(qrow + 32 * s + 8 * g4 + 4);
-                qfrag[s] = v4u{pack_bf2(a.x, a.y), pack_bf2(a.z, a.w), pack_bf2(b.x, b.y), pack_bf2(b.z, b.w)};
-            }
-        }
-    }
+    for (int s = S0; s < RT; ++s)
+        qfrag[s] = v4u{pack_bf2(q[s][0].x, q[s][0].y), pack_bf2(q[s][0].z, q[s][0].w), pack_bf2(q[s][1].x, q[s][1].y), pack_bf2(q[s][1].z, q[s][1].w)} & kept;
+#pragma unroll
+    for (int s = S0; s < RT; ++s) asm volatile("" : "+v"(qfrag[s]));               // (before the copies: behind them its wait would be for them too)
+    if (z < nT) copy(z, 0, a0, b0);
+    if (z + Z < nT) copy(z + Z, 1, a1, b1);
     v4f oacc[WC];
 #pragma unroll
     for (int c = 0; c < WC; ++c) oacc[c] = v4f{0.f, 0.f, 0.f, 0.f};
@@ -592,12 +610,11 @@ __global__ __launch_bounds__(64 * SW, 1) void latent_step_kernel(
     }
     int which = 0;
     for (int round = z; round < nT; round += Z) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();                                           // these keys have landed; the other half has been read by everyone
+        if (round + Z < nT) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NJ) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();                                           // these keys have landed
         asm volatile("" ::: "memory");
         const unsigned char* T = buf + which * TILE;
-        which ^= 1;
-        if (round + Z < nT) copy(round + Z, which);
         v4f sacc[2] = {v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}};
         v4u kf[RT];
 #pragma unroll
@@ -651,6 +668,12 @@ __global__ __launch_bounds__(64 * SW, 1) void latent_step_kernel(
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
+        if (round + 2 * Z < nT) {                                               // (everyone has read these)
+            copy(round + 2 * Z, which, next_a, next_b);
+            next_a = page_of(2 * (round + 3 * Z));
+            next_b = page_of(2 * (round + 3 * Z) + 1);
+        }
+        which ^= 1;
 #pragma unroll
         for (int b = 0; b < 2; ++b) {                                           // 32 keys: k-slot (g4, e) <-> key 16 (e / 4) + 4 g4 + e % 4
             const uint2 p0 = probs[2 * b][lane], p1 = probs[2 * b + 1][lane];

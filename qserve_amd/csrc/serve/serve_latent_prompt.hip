@@ -115,18 +115,28 @@ __global__ __launch_bounds__(64 * PW, 2) void latent_prompt_kernel(PromptArgs a)
         const bf16_t* qr = a.q + ((size_t)(t0 + mine) * a.H + h) * D + 8 * g;
 #pragma unroll
         for (int s = 0; s < NS; ++s) qf[s] = __builtin_bit_cast(bf8, *(const v4u*)(qr + 16 * s));
-        if constexpr (ROT > 0) {
+        if constexpr (ROT > 0)
+        if (a.rot_n > 0) {                                                      // (nothing turned: there need be no table)
+            // cosines and sines, all requested before the first turn (behind its condition, every pair waited for the one before)
             const float* cs = a.rope + (size_t)p_row * a.rot_n;
+            float co[NS - 8][4], sn[NS - 8][4];
+#pragma unroll
+            for (int s = 0; s < NS - 8; ++s)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int c = min(8 * s + 4 * g + e, (a.rot_n >> 1) - 1);
+                    co[s][e] = cs[c];
+                    sn[s][e] = cs[(a.rot_n >> 1) + c];
+                }
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int s = 8; s < NS; ++s) {
                 v4u x = __builtin_bit_cast(v4u, qf[s]);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const int c = 16 * (s - 8) + 8 * g + 2 * e;
-                    if (c < a.rot_n) {
-                        const float co = cs[c >> 1], sn = cs[(a.rot_n >> 1) + (c >> 1)], u = __uint_as_float(x[e] << 16), v = __uint_as_float(x[e] & 0xffff0000u);
-                        x[e] = pack2(u * co - v * sn, v * co + u * sn);
-                    }
+                    const float u = __uint_as_float(x[e] << 16), v = __uint_as_float(x[e] & 0xffff0000u), c = co[s - 8][e], i = sn[s - 8][e];
+                    const unsigned turned = pack2(u * c - v * i, v * c + u * i);
+                    x[e] = 16 * (s - 8) + 8 * g + 2 * e < a.rot_n ? turned : x[e];
                 }
                 qf[s] = __builtin_bit_cast(bf8, x);
             }

@@ -284,15 +284,17 @@ __global__ __launch_bounds__(PT, 2) void grouped_gemm_persistent_kernel(GroupedA
         const int lane = fresh_lane(), piece = ((lane & 7) ^ (lane >> 3)) * 16;
         W0 = a.W + ((size_t)g.e * a.N + g.n0) * (size_t)a.K;
         rows_here = __builtin_amdgcn_readfirstlane(g.ns - 16 * w);
+        int slot[4];                                                // (all four asked for before the first is divided)
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+        for (int i = 0; i < 4; ++i)
+            slot[i] = staged ? side[AHEAD + 64 * w + 16 * (i >> 1) + 8 * (i & 1) + (lane >> 3)] : x_slot(g, i >> 1, i & 1, lane);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                woff[2 * h + j] = (unsigned)min(128 * h + 16 * w + 8 * j + (lane >> 3), a.N - 1 - g.n0) * (unsigned)a.K * 2u + piece;
-                const int slot = staged ? side[AHEAD + 64 * w + 16 * h + 8 * j + (lane >> 3)] : x_slot(g, h, j, lane);
-                xrow[2 * h + j] = (const unsigned char*)(a.X + (size_t)(a.div == 1 ? slot : slot / a.div) * (size_t)a.K) + piece;
-                if (LISTED && g.ns <= 0) xrow[2 * h + j] = (const unsigned char*)W0 + woff[2 * h + j];   // (no input need exist)
-            }
+        for (int i = 0; i < 4; ++i) {
+            woff[i] = (unsigned)min(128 * (i >> 1) + 16 * w + 8 * (i & 1) + (lane >> 3), a.N - 1 - g.n0) * (unsigned)a.K * 2u + piece;
+            xrow[i] = (const unsigned char*)(a.X + (size_t)(a.div == 1 ? slot[i] : slot[i] / a.div) * (size_t)a.K) + piece;
+            if (LISTED && g.ns <= 0) xrow[i] = (const unsigned char*)W0 + woff[i];   // (no input need exist)
+        }
     };
     auto copy_w = [&](int h, unsigned to, int step) __attribute__((always_inline)) {
         const int k0 = step < steps ? step * KS : 0;

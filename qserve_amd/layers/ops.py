@@ -390,8 +390,8 @@ class HipOps:
             wide = R > 320
             if tiles.size(0) == T:              # one token per tile: the kernel for steps
                 # A split costs a trip of its partial result through memory and the merge, 2 - 3 us at two splits, 64 keys about 2 us: none up to 256
-                # keys (16 heads, 576 wide, 64 sequences of 128 / 200 / 500 / 1000 positions, one / two / four splits: 12 / 14 / 16, 15 / 18 / 18, 28 /
-                # 24 / 23, 43 / 32 / 28 us), then 96 keys or more each while the workgroups fit the chip at once (one sequence of 2000: 64 us with
+                # keys (16 heads, 576 wide, 64 sequences of 200 / 256 / 500 / 1000 positions, one / two / four splits: 16 / 17, 16 / 17, 25 / 22 / 21,
+                # 40 / - / 26 us), then 96 keys or more each while the workgroups fit the chip at once (one sequence of 2000: 64 us with
                 # one, 18 with 8, 16 with 16; 256 wide on 4 pools, 64 sequences of 1000, one / two: 23 / 26 us)
                 splits = max(1, min((256 if wide else 384) // max(groups, 1), span // 96, 32)) if span > 256 else 1
             else:

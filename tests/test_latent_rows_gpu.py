@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
                                                   # one token each: rounds of 64 keys, halves of 32
                                                   (tuple((c, 1) for c in (1, 31, 32, 33, 64, 65, 96, 97, 128, 129, 200)), None, 1),
                                                   (tuple((c, 1) for c in (2, 64, 100, 193)), None, 2), (((700, 1), (65, 1), (3, 1)), 64, 3),
-                                                  (((300, 1), (40, 1)), 37, 1), (((1000, 1),), None, 16), (((1200, 1), (63, 1)), None, None)])
+                                                  (((300, 1), (40, 1)), 37, 1), (((321, 1), (450, 1), (5, 1)), None, 1), (((1000, 1),), None, 16), (((1200, 1), (63, 1)), None, None)])
 def test_plain_rows(R, rank, H, G, q_first, runs, window, splits):
     if not torch.cuda.is_available():
         pytest.skip("no GPU")

@@ -394,11 +394,12 @@ struct Rows {                                            // the softmax state of
     v16f o[M][CT];
     float m[M], l[M];
 
-    __device__ __forceinline__ void start(const bf16_t* qrow, bool ok, int hi) {
+    // (the query as it lies in memory, also of rows that are none: any row's; keep() takes those out)
+    __device__ __forceinline__ void start(const bf16_t* qrow, int hi) {
 #pragma unroll
         for (int f = 0; f < M; ++f) {
 #pragma unroll
-            for (int s = 0; s < DT; ++s) qf[f][s] = ok ? *(const v4u*)(qrow + f * S::DIM + 16 * s + 8 * hi) : v4u{0u, 0u, 0u, 0u};
+            for (int s = 0; s < DT; ++s) qf[f][s] = *(const v4u*)(qrow + f * S::DIM + 16 * s + 8 * hi);
 #pragma unroll
             for (int c = 0; c < CT; ++c)
 #pragma unroll
@@ -406,6 +407,17 @@ struct Rows {                                            // the softmax state of
             m[f] = -INFINITY;
             l[f] = 0.f;
         }
+    }
+    // complete before the loop, whose waits count the copies only
+    __device__ __forceinline__ void keep(bool ok) {
+        const unsigned kept = ok ? ~0u : 0u;
+#pragma unroll
+        for (int f = 0; f < M; ++f)
+#pragma unroll
+            for (int s = 0; s < DT; ++s) {
+                qf[f][s] &= kept;
+                asm volatile("" : "+v"(qf[f][s]));
+            }
     }
     // keys k0 .. k0 + 31, staged at `blk`; p_row: this lane's position; mask: some row of the wave does not see the whole block
     __device__ __forceinline__ void block(const unsigned char* blk, int k0, int p_row, bool mask, int lane) {
@@ -540,7 +552,7 @@ __global__ __launch_bounds__(NT, (Shape<DT, CT, M>::PROMPT_OCC)) void maps_promp
     const int t = t0 + (ok ? tok : 0), p_row = p_first + (ok ? tok : 0);
     const int wp_first = p_first + w * a.TQ, wp_last = min(wp_first + a.TQ - 1, p_last);      // (a wave without tokens: wp_first > p_last)
     Rows<DT, CT, M> R;
-    R.start(a.q + ((size_t)t * a.H + (ok ? head : 0)) * (M * S::DIM), ok, hi);
+    R.start(a.q + ((size_t)t * a.H + (ok ? head : 0)) * (M * S::DIM), hi);
     const unsigned lds = (unsigned)(size_t)(lds_ptr)smem;
     const int ntiles = p_last / (2 * BN) + 1;
     PageIds pages(bt, (p_last >> a.page_shift) + 1, lane);
@@ -553,10 +565,7 @@ __global__ __launch_bounds__(NT, (Shape<DT, CT, M>::PROMPT_OCC)) void maps_promp
         copy_rows<S, 2 * BN, NW>(base_of(k0), lds + 2 * buf * S::BLOCK, p_last - k0, w, lane);
     };
     copy_tile(0, 0);
-#pragma unroll
-    for (int f = 0; f < M; ++f)
-#pragma unroll
-        for (int s = 0; s < DT; ++s) asm volatile("" : "+v"(R.qf[f][s]));      // (complete before the loop: its waits count the copies only)
+    R.keep(ok);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     for (int tile = 0; tile < ntiles; ++tile) {
@@ -589,7 +598,15 @@ __global__ __launch_bounds__(NT, (Shape<DT, CT, M>::PROMPT_OCC)) void maps_promp
         f = 1.0f / (R.l[0] + __shfl_xor(R.l[0], 32, 64));
     }
     bf16_t* orow = a.out + ((size_t)t * a.H + head) * S::VDIM;
-    const bf16_t* grow = a.gate ? a.gate + (size_t)t * (size_t)a.gate_stride + (size_t)head * S::VDIM : nullptr;
+    const bf16_t* grow = a.gate ? a.gate + (size_t)t * (size_t)a.gate_stride + (size_t)head * S::VDIM + 4 * hi : nullptr;
+    raw2u rg[CT][4] = {};                                           // (whole before the first store: each would wait for the store before it)
+    if (grow) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) rg[c][j] = raw4(grow, 32 * c + 8 * j);
+    }
+    requested();
 #pragma unroll
     for (int c = 0; c < CT; ++c)
 #pragma unroll
@@ -599,17 +616,29 @@ __global__ __launch_bounds__(NT, (Shape<DT, CT, M>::PROMPT_OCC)) void maps_promp
 #pragma unroll
             for (int r = 0; r < 4; ++r) v[r] = R.o[0][c][4 * j + r] * f;
             if (grow) {
-                const Vec<4> g = ldv<4>(grow, e);
+                float g[4];
+                widen4(rg[c][j], g);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) v[r] *= 1.0f / (1.0f + __expf(-g.v[r]));
+                for (int r = 0; r < 4; ++r) v[r] *= 1.0f / (1.0f + __expf(-g[r]));
             }
             *(v2u*)(orow + e) = v2u{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
         }
 }
 
+// The gate of a row as it lies in memory, for finish_row (no gate: nothing is read).
+template <int VDIM>
+struct GateRow {
+    unsigned v[(VDIM + 63) / 64] = {};                             // (a register each: two in one would be waited for where they meet)
+    __device__ __forceinline__ void request(const MapsArgs& a, size_t t, int head, int lane) {
+        if (!a.gate) return;
+        const bf16_t* row = a.gate + t * (size_t)a.gate_stride + (size_t)head * VDIM;
+#pragma unroll
+        for (int i = 0; i < (VDIM + 63) / 64; ++i) v[i] = row[min(lane + 64 * i, VDIM - 1)];
+    }
+};
 // One row from n partial results: src(i, f) its unnormalised output of map f, ml(i, f) its (maximum, sum); the wave's lanes walk vdim.
 template <int VDIM, int M, typename FO, typename FM>
-__device__ __forceinline__ void finish_row(const MapsArgs& a, int n, FO src, FM ml, size_t t, int head, int lane) {
+__device__ __forceinline__ void finish_row(const MapsArgs& a, int n, FO src, FM ml, size_t t, int head, int lane, const GateRow<VDIM>& gate) {
     constexpr int EO = (VDIM + 63) / 64;
     float o[EO];
 #pragma unroll
@@ -643,7 +672,7 @@ __device__ __forceinline__ void finish_row(const MapsArgs& a, int n, FO src, FM 
         const int e = lane + 64 * i;
         if (e >= VDIM) continue;
         float v = o[i] * inv;
-        if (a.gate) v *= 1.0f / (1.0f + __expf(-bf2f(a.gate[t * (size_t)a.gate_stride + (size_t)head * VDIM + e])));
+        if (a.gate) v *= 1.0f / (1.0f + __expf(-bf2f((bf16_t)gate.v[i])));
         a.out[(t * a.H + head) * (size_t)VDIM + e] = f2bf(v);
     }
 }
@@ -663,8 +692,11 @@ __global__ __launch_bounds__(NT, (Shape<DT, CT, M>::STEP_OCC)) void maps_step_ke
     const int tok = li / a.HP, head = h0 + li % a.HP;
     const bool ok = tok < ntok && head < h_end;
     const int t = t0 + (ok ? tok : 0), p_row = p_first + (ok ? tok : 0);
+    // the gate of the wave's first row (most steps: its only one) ahead of everything: asked for when the row is done, it is a trip to memory at the end
+    GateRow<S::VDIM> gate;
+    if (a.Z == 1) gate.request(a, (size_t)(t0 + min(w / a.HP, ntok - 1)), min(h0 + w % a.HP, h_end - 1), lane);
     Rows<DT, CT, M> R;
-    R.start(a.q + ((size_t)t * a.H + (ok ? head : 0)) * (M * S::DIM), ok, hi);
+    R.start(a.q + ((size_t)t * a.H + (ok ? head : 0)) * (M * S::DIM), hi);
     const unsigned lds = (unsigned)(size_t)(lds_ptr)smem + w * S::BUFS * S::BLOCK;
     const unsigned char* mine = smem + w * S::BUFS * S::BLOCK;
     const int nT = p_last / BN + 1, stride = NW * a.Z, first = z * NW + w;
@@ -675,10 +707,7 @@ __global__ __launch_bounds__(NT, (Shape<DT, CT, M>::STEP_OCC)) void maps_step_ke
                             p_last - k0, 0, lane);
     };
     if (first < nT) copy(first, 0);
-#pragma unroll
-    for (int f = 0; f < M; ++f)
-#pragma unroll
-        for (int s = 0; s < DT; ++s) asm volatile("" : "+v"(R.qf[f][s]));
+    R.keep(ok);
     int i = 0;
     for (int tile = first; tile < nT; tile += stride, ++i) {
         const bool more = tile + stride < nT;
@@ -723,7 +752,8 @@ __global__ __launch_bounds__(NT, (Shape<DT, CT, M>::STEP_OCC)) void maps_step_ke
         auto src = [&](int k, int f) { return so + ((k * M + f) * 32 + row) * S::OROW; };
         auto ml = [&](int k, int f) { return sml + ((k * M + f) * 32 + row) * 2; };
         if (a.Z == 1) {
-            finish_row<S::VDIM, M>(a, NW, src, ml, (size_t)(t0 + rt), rh, lane);
+            if (row != w) gate.request(a, (size_t)(t0 + rt), rh, lane);
+            finish_row<S::VDIM, M>(a, NW, src, ml, (size_t)(t0 + rt), rh, lane, gate);
             continue;
         }
         const size_t at = (((size_t)z * a.n_tiles + blockIdx.x) * gridDim.y + y) * 32 + row;
@@ -762,8 +792,10 @@ __global__ __launch_bounds__(NT) void maps_merge_kernel(MapsArgs a) {
         const int rt = row / a.HP, rh = h0 + row % a.HP;
         if (rt >= ntok || rh >= h_end) continue;
         auto at = [&](int k, int f) { return ((((size_t)k * a.n_tiles + blockIdx.x) * gridDim.y + y) * 32 + row) * M + f; };
+        GateRow<VDIM> gate;
+        gate.request(a, (size_t)(t0 + rt), rh, lane);
         finish_row<VDIM, M>(a, a.Z, [&](int k, int f) { return a.part_o + at(k, f) * VDIM; }, [&](int k, int f) { return a.part_ml + at(k, f) * 2; },
-                            (size_t)(t0 + rt), rh, lane);
+                            (size_t)(t0 + rt), rh, lane, gate);
     }
 }
 

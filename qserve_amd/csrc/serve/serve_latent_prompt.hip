@@ -240,6 +240,14 @@ __global__ __launch_bounds__(64 * PW, 2) void latent_prompt_kernel(PromptArgs a)
     const size_t t = (size_t)(t0 + wq + col);
     bf16_t* out = a.out + (t * a.H + h) * 128 + 4 * g;
     const bf16_t* gate = a.gate ? a.gate + t * a.gate_stride + (size_t)h * 128 + 4 * g : nullptr;
+    raw2u rg[4][4] = {};                                            // (whole before the first store: each would wait for the store before it)
+    if (gate) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) rg[c][j] = raw4(gate, 32 * c + 8 * j);
+    }
+    requested();
 #pragma unroll
     for (int c = 0; c < 4; ++c)
 #pragma unroll
@@ -249,7 +257,7 @@ __global__ __launch_bounds__(64 * PW, 2) void latent_prompt_kernel(PromptArgs a)
             for (int r = 0; r < 4; ++r) v[r] = o[c][4 * j + r] * inv;
             if (gate) {
                 float x[4];
-                ld4t(gate, 32 * c + 8 * j, x);
+                widen4(rg[c][j], x);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) v[r] *= 1.0f / (1.0f + expf(-x[r]));
             }

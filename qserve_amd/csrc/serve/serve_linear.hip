@@ -4,6 +4,7 @@
 // weight streamed through LDS rings (serve_stream.h), the four waves' shares of the reduction added in LDS.
 // Measured against the vendor's product (MI355X, weights from HBM, 1 / 16 / 32 / 64 rows, us): 2048 x 2048 4.5 / 4.7 / 5.5 / 5.6 against 8.1 / 8.2 / 8.4 /
 // 8.8; 6144 x 2048 7.4 / 7.6 / 8.4 / 10.9 against 12.7 / 12.5 / 12.4 / 13.0; 32000 x 2048 27 / 28 / 30 / 47 against 34 / 34 / 35 / 35.
+// (Weights that pass once stream past the caches since: 32000 x 2048 of one or 16 rows 25 - 26 us, 4096 x 4096 8.9 -> 8.5.)
 #include "serve_common.h"
 #include "serve_stream.h"
 
@@ -132,6 +133,12 @@ __global__ __launch_bounds__(256) void head_product_kernel(HeadProductArgs a) {
     const int n0 = blockIdx.x * 32, kq = (lane >> 4) * 8;
     const bf16_t* W = a.w + (size_t)h * a.K * a.N + n0 + 2 * (lane & 15);
     const bf16_t* X = a.x + h * a.x_head;
+    unsigned gate[RT] = {};                                                     // (first: asked for behind the sum, each row's waits for the row before)
+    if (!QUERY && a.gate) {
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+            gate[r] = *(const unsigned*)(a.gate + min(16 * r + (tid >> 4), a.T - 1) * a.gate_stride + (size_t)h * a.N + n0 + 2 * (tid & 15));
+    }
     v4f acc[RT][2];
 #pragma unroll
     for (int r = 0; r < RT; ++r) acc[r][0] = acc[r][1] = (v4f){0.f, 0.f, 0.f, 0.f};
@@ -171,7 +178,6 @@ __global__ __launch_bounds__(256) void head_product_kernel(HeadProductArgs a) {
     for (int r = 0; r < RT; ++r) {
         const int t = 16 * r + (tid >> 4), c = 2 * (tid & 15);
         if (t >= a.T) continue;
-        const unsigned g = !QUERY && a.gate ? *(const unsigned*)(a.gate + t * a.gate_stride + (size_t)h * a.N + n0 + c) : 0u;
         float2 v = make_float2(0.f, 0.f);
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
@@ -182,8 +188,8 @@ __global__ __launch_bounds__(256) void head_product_kernel(HeadProductArgs a) {
         if (QUERY) *(float2*)((float*)a.out + ((size_t)t * a.H + h) * (a.N + a.rot_dim) + n0 + c) = make_float2(v.x * a.scale, v.y * a.scale);
         else {
             if (a.gate) {
-                v.x *= 1.0f / (1.0f + expf(-__uint_as_float(g << 16)));
-                v.y *= 1.0f / (1.0f + expf(-__uint_as_float(g & 0xffff0000u)));
+                v.x *= 1.0f / (1.0f + expf(-__uint_as_float(gate[r] << 16)));
+                v.y *= 1.0f / (1.0f + expf(-__uint_as_float(gate[r] & 0xffff0000u)));
             }
             *(unsigned*)((bf16_t*)a.out + ((size_t)t * a.H + h) * a.N + n0 + c) = (unsigned)f2bf(v.x) | ((unsigned)f2bf(v.y) << 16);
         }

@@ -413,7 +413,10 @@ __global__ __launch_bounds__(NT) void moe_down_vec_kernel(T* __restrict__ y, con
 // Measured per launch in a step (MI355X): 64 tokens, 4 of 16 experts of 2048 x 1408 (92 MB a product) 55.6 / 62.4 us -> 23.8 / 21.1 us (up /
 // down) against the form it replaces, which kept weight rows in registers and paid a wave-wide sum per token and row; 16 tokens with
 // gated units (184 + 92 MB) 42.6 / 26.1 -> 36.5 / 19.3 us (5.0 TB/s); one token 1446 / 3117 us (the per-token kernels) -> 14.0 / 8.8 us.
-// The sort, search and permutation launches in front of it (60 us a layer) are gone.
+// The sort, search and permutation launches in front of it (60 us a layer) are gone.  Streamed past the caches, the shared expert in the same
+// launch: 64 tokens 22.7 / 19.4 us (98 MB), 16 tokens gated 33.8 / 17.6 (196 / 98 MB, 5.7 TB/s), one token 15.3 / 9.5.
+// 32 rows: 16, more evenly spread over the CUs, read the inputs twice as often and are slower everywhere (64 tokens 24.7 / 25.7, 16 tokens 36.3 / 21.4,
+// one 18.7 / 11.7), and so are 64; rings twice as deep give no more.
 constexpr int XR = 32;               // weight rows per workgroup
 constexpr int XLIST = 1024;          // router indices looked at in one go
 

@@ -83,11 +83,13 @@ class OpTimer:
              "add_rms_norm", "rms_norm_rows", "normed_attention_prep", "max_gates", "add_normed_rms_norm", "qk_norm_rope_prep", "pool_blocks",
              "min_gru_scan", "relu_sq", "embed_rms_norm", "residual_conv", "scaled_add_rms_norm", "rotate_qk", "talking_attention",
              "scaled_sum_rms_norms", "conv_heads_cache", "diff_attention", "single_map_attention")
+    # another form of the same operation: its time is that operation's
+    FORMS = {"latent_prompt": "latent_attention", "moe_experts_shared": "moe_experts"}
 
     def __init__(self, ops):
         self.ops, self.events, self.calls, self.on = ops, [], [], False
         for n in self.NAMES:
-            setattr(ops, n, self._wrap(n, getattr(ops, n)))
+            setattr(ops, n, self._wrap(self.FORMS.get(n, n), getattr(ops, n)))
         from ..layers import ops as ops_module                # the vendor products, as the layers call them
         for mod in self._linear_users():
             name = "linear" if hasattr(mod, "linear") else "float_linear"
@@ -174,6 +176,7 @@ def bench_vekalorn(name, s, dev, steps, warmup):
         if i == BP:                                          # one step with events around every launch
             ops_pre, _ = timer.step(lambda: eng.execute(items, want))
             att_pre_ms = timer.replay("latent_attention", 5)
+            over_heads = any(fn.__name__ == "latent_prompt" for _, fn, _, _ in timer.calls)
             continue
         torch.cuda.synchronize()
         t0 = time.perf_counter()
@@ -213,8 +216,11 @@ def bench_vekalorn(name, s, dev, steps, warmup):
     rows = {"latent_attention_2": rank + s["rot_dim"], "latent_attention": rank}
     kinds = [x["type"] for x in cfg["layers"]]
     T = BP * L
-    flops = sum(sum(min(p + 1, s["window"]) if k == "latent_attention" else p + 1 for p in range(L)) * BP * H * (rows[k] + rank) * 2.0
-                for k in kinds)
+    pairs = {k: sum(min(p + 1, s["window"]) if k == "latent_attention" else p + 1 for p in range(L)) * BP * H * 2.0 for k in rows}
+    if over_heads:                                           # (with the heads' keys and values out of the cached rows)
+        flops = sum(pairs[k] * (s["dim"] + rows[k] - rank + s["vdim"]) + T * H * rank * (s["dim"] + s["vdim"]) * 2.0 for k in kinds)
+    else:
+        flops = sum(pairs[k] * (rows[k] + rank) for k in kinds)
     att_pre = flops / (att_pre_ms * 1e-3) / 1e12
     by = sum(NB * (min(ctx, s["window"]) if k == "latent_attention" else ctx) * rows[k] * 2.0 for k in kinds)
     att_dec = by / (att_dec_ms * 1e-3) / 1e9

@@ -625,7 +625,8 @@ __global__ __launch_bounds__(NT, (Shape<DT, CT, M>::PROMPT_OCC)) void maps_promp
         }
 }
 
-// The gate of a row as it lies in memory, for finish_row (no gate: nothing is read).
+// The gate of a row as it lies in memory, for finish_row (no gate: nothing is read).  Bound by the chain of trips to memory: asked for at the kernel's start, beside
+// the query, one sequence of 330 positions, 16 heads on 4 pools, two maps: 12.2 -> 11.3 us; a prompt's, whole before its stores, 2047 tokens 100 -> 96.
 template <int VDIM>
 struct GateRow {
     unsigned v[(VDIM + 63) / 64] = {};                             // (a register each: two in one would be waited for where they meet)

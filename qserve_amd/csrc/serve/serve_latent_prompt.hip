@@ -59,6 +59,7 @@ __device__ __forceinline__ unsigned pack2(float a, float b) {
 // Measured (MI355X, 128 + 64 / 128 dimensions): 8 prompts of 1024, 16 heads 78 / 53 us (550 / 650 TFLOP/s; on the latent rows 350 / 331 us and
 // 99 us for their float queries), one of 4100, 32 heads 204 / 163 us (845 TFLOP/s).  Eight waves that share a tile's copy, one workgroup a CU: 82 /
 // 56 us, 64 prompts of 50 - 100 tokens 34 / 23 -> 46 / 31.
+// In a model, gated, 8 prompts of 1024: 110 -> 94 us with 64 rotated dimensions since their cosines and the gate are requested whole (58 without either).
 template <int ROT>
 __global__ __launch_bounds__(64 * PW, 2) void latent_prompt_kernel(PromptArgs a) {
     constexpr int D = 128 + ROT, NS = D / 16, KB = PK * 256, RB = PK * ROT * 2, TILE = KB + RB + 128 * PK * 2;

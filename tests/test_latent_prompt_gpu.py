@@ -100,3 +100,55 @@ def test_where_it_is_taken(tokens, starts, taken):
     batch.starts = None
     batch._tiles.clear()
     assert plan() is None
+
+
+class _Turned:
+    dims = 64
+
+    def reserve(self, n):
+        a = torch.arange(n)[:, None] * 10.0 ** (-torch.arange(32) / 8.0)
+        return torch.stack([torch.cos(a), torch.sin(a)], 1).cuda()
+
+
+def _layer(H=4, D=256, qr=64, rank=64, rot_dim=64, gated=False, window=None, page=64):
+    from qserve_amd.layers.latent_attention import LatentAttention
+    g = torch.Generator().manual_seed(H + rank)
+    mat = lambda o, i: (torch.randn(o, i, generator=g) / i ** 0.5).bfloat16().cuda()               # noqa: E731
+    one = lambda n: torch.ones(n, dtype=torch.bfloat16, device="cuda")                             # noqa: E731
+    w = dict(dq=mat(qr, D), dq_norm=one(qr), uq=mat(H * (128 + rot_dim), qr), dkv=mat(rank + rot_dim, D), dkv_norm=one(rank), uk=mat(H * 128, rank),
+             uv=mat(H * 128, rank), o=mat(D, H * 128))
+    if gated:
+        w["g"] = mat(H * 128, D)
+    return LatentAttention(make_ops("hip", torch.bfloat16, torch.device("cuda:0")), heads=H, dim=128, vdim=128, kv_rank=rank, q_rank=qr, scale=0.1, eps=1e-5, weights=w,
+                           rot_dim=rot_dim, rotary=_Turned() if rot_dim else None, gated=gated, window=window, page=page)
+
+
+def _step(layer, h, runs, pool, table):
+    """The layer over runs (sequence, first position, tokens) of one step."""
+    dev, at, items, starts, pos, seq = h.device, 0, [], [], [], []
+    for b, start, n in runs:
+        items.append((b, at, n))
+        starts.append(start)
+        pos += range(start, start + n)
+        seq += [b] * n
+        at += n
+    p, s = torch.tensor(pos), torch.tensor(seq)
+    slot = table.cpu()[s, p // layer.page].long() * layer.page + p % layer.page
+    batch = StepBatch(tokens=None, seq=s.int().to(dev), pos=p.int().to(dev), slot=slot.to(dev), block_table=table, max_pos=max(pos), n_tokens=at, items=items, starts=starts)
+    return layer(h, batch, pool)
+
+
+def test_a_pool_off_16_bytes_is_taken():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    layer, g = _layer(page=40), torch.Generator().manual_seed(5)       # (pages that the kernels reading elements one by one serve)
+    h, table = torch.randn(150, 256, generator=g).bfloat16().cuda(), torch.tensor([[2, 0, 3, 1]], dtype=torch.int32, device="cuda")
+    outs = []
+    for off, rule in ((0, False), (1, True), (4, True)):                # (the rule off: on the rows, aligned)
+        pool = torch.zeros(160 * 128 + 8, dtype=torch.bfloat16, device="cuda")[off:][:160 * 128].view(160, 128)
+        layer.ops.prompt_heads_kernel = rule
+        outs.append(_step(layer, h, [(0, 0, 150)], pool, table))
+    # the latents' norms sum their squares in another order where the pool is off four elements, so that a latent may round the other way: 2^-9 of some of them
+    a = outs[0].double()
+    for o in outs[1:]:
+        assert (o.double() - a).norm() <= 2.0 ** -9 * a.norm()

@@ -1,0 +1,30 @@
+"""Which prompts attend over written-out keys and values: the rule alone, on the host."""
+import pytest
+import torch
+
+from qserve_amd.layers.ops import HipOps
+from qserve_amd.serving.engine import StepBatch
+
+
+def _batch(runs):
+    """runs: (first position, tokens)."""
+    at, items = 0, []
+    for b, (_, n) in enumerate(runs):
+        items.append((b, at, n))
+        at += n
+    return StepBatch(tokens=None, seq=None, pos=torch.zeros(at, dtype=torch.int32), slot=None, block_table=None, max_pos=max(s + n for s, n in runs) - 1, n_tokens=at,
+                     items=items, starts=[s for s, _ in runs])
+
+
+def _plan(runs, H=16, rot=64, rank=512, window=None, **more):
+    return HipOps(torch.bfloat16).latent_prompt_plan(_batch(runs), window, H, 128, rot, 128, rank, 0.1, **more)
+
+
+def test_a_pool_off_the_alignment_keeps_its_rows():
+    rows = torch.zeros(64 * 576 + 8, dtype=torch.bfloat16)
+    start = -rows.data_ptr() // 2 % 8                                   # (the first element on 16 bytes)
+    for off in range(8):
+        pool = rows[(start + off) % 8:][:64 * 576].view(64, 576)
+        assert pool.data_ptr() % 16 == 2 * off
+        assert (_plan([(0, 100)], pool=pool) is not None) == (off == 0)
+    assert _plan([(0, 100)]) is not None

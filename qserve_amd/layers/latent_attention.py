@@ -54,7 +54,7 @@ class LatentAttention:
                              self.rot_n, rope, pool, batch.slot, batch.pos, self.eps)
         q = linear(cq, self.w_uq)                                                   # [T, H (dim + rot_dim)]
         gate = down[:, self.g_off:self.g_off + H * self.vdim] if self.gated else None
-        plan = ops.latent_prompt_plan(batch, self.window, H, self.dim, self.rot_dim, self.vdim, self.rank, self.scale, pool)
+        plan = ops.latent_prompt_plan(batch, self.window, H, self.dim, self.rot_dim, self.vdim, self.rank, self.scale, pool, (self.w_uk, self.w_uv))
         if plan is not None:
             return linear(ops.latent_prompt(q, pool, batch, plan, self.w_uk.view(H * self.dim, self.rank), self.w_uv, rope, self.scale, H, self.rot_dim,
                                             self.rot_n, self.rank, self.page, self.window, gate), self.w_o)

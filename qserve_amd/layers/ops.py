@@ -289,16 +289,16 @@ class HipOps:
         q_abs = _absorbed(q, w_uk)
         return self.latent_query(q, q_abs, rope, pos, scale, heads, dim, rot_dim, rot_n, rank)
 
-    def latent_prompt_plan(self, batch, window, heads, dim, rot_dim, vdim, rank, scale, pool=None):
+    def latent_prompt_plan(self, batch, window, heads, dim, rot_dim, vdim, rank, scale, pool=None, weights=()):
         """What `latent_prompt` is given for this batch, or None where the attention on the latent rows is the better one or the only one (also for a pool
-        whose rows do not start on 16 bytes).
+        whose rows do not start on 16 bytes, and where torch would make something else of the products with `weights`, or somebody follows them).
         Writing keys and values out costs the keys' products with w_uk and w_uv; the queries' and the results' go, and the attention costs 320 products in place
         of 1088 per query, key and head (rank 512 + 64).  Whole layer, on the rows / this way, us, 16 heads, rank 512 + 64: runs of 65 / 300 / 1000 new tokens
         79 / 61, 108 / 75, 177 / 111; 512 behind 512 / 1536: 131 / 96, 154 / 122; 33 behind 67, four of them 92 / 73; 512 beside three single tokens at 1000
         (7 keys a token) 130 / 118; 128 behind 1024 (9) 98 / 96.  The line is at 4 keys a token, which also bounds what is written out; up to 64
         tokens the products per head have a kernel of their own."""
         if not (self.prompt_heads_kernel and scale > 0 and heads <= 1 << 12 and self.L.qsv_latent_prompt_ok(dim, rot_dim, vdim, rank, self.code)
-                and (pool is None or pool.data_ptr() % 16 == 0)):
+                and (pool is None or pool.data_ptr() % 16 == 0) and _called_plainly(*weights) and all(w.dtype == self.dtype for w in weights)):
             return None
         plan = batch.key_runs(window, self.L.qsv_latent_prompt_tile_tokens()) if batch.n_tokens > 64 else None
         return plan if plan is not None and plan[2] <= min(4 * batch.n_tokens, 1 << 23) else None
@@ -310,12 +310,15 @@ class HipOps:
         T, R = q.size(0), rank + rot_dim
         self._need(q, pool, batch.block_table, runs, tiles, w_uk, w_uv, rope)
         assert pool.dim() == 2 and pool.size(1) == R and q.size(1) == heads * (128 + rot_dim) and w_uk.shape == w_uv.shape == (heads * 128, rank)
+        assert all(t.dtype == self.dtype for t in (q, pool, w_uk, w_uv))
         assert rope is None or (rope.dtype == torch.float32 and rope.size(-1) * 2 == rot_n)
         rows = torch.empty((n_rows, R), dtype=self.dtype, device=q.device)
         self.check(self.L.qsv_latent_gather(rows.data_ptr(), pool.data_ptr(), batch.block_table.data_ptr(), batch.block_table.stride(0), runs.data_ptr(), runs.size(0),
                                             longest, n_rows, R, page, self._s()), "latent_gather")
         k = torch.matmul(rows[:, :rank], w_uk.t())                                # [n_rows, heads dim]
         vt = torch.matmul(w_uv, rows[:, :rank].t())                               # [heads vdim, n_rows]: keys next to each other, as the product wants them
+        self._need(k, vt)
+        assert k.dtype == vt.dtype == self.dtype                                  # (torch made them: the kernel reads addresses)
         out = torch.empty((T, heads * 128), dtype=self.dtype, device=q.device)
         if gate is not None and not (gate.data_ptr() % 8 == 0 and gate.stride(0) % 4 == 0 and gate.stride(1) == 1):
             gate = gate.contiguous()
@@ -1273,7 +1276,7 @@ class TorchOps:
         qr = _rotate(q.view(T, heads, dim + rot_dim)[..., dim:].float(), rope, pos, rot_n)
         return (torch.cat([q_abs.transpose(0, 1).float(), qr], dim=-1) * scale).contiguous()
 
-    def latent_prompt_plan(self, batch, window, heads, dim, rot_dim, vdim, rank, scale, pool=None):
+    def latent_prompt_plan(self, batch, window, heads, dim, rot_dim, vdim, rank, scale, pool=None, weights=()):
         return None
 
     def latent_queries(self, q, w_uk, rope, pos, scale, heads, dim, rot_dim, rot_n, rank):

@@ -28,3 +28,17 @@ def test_a_pool_off_the_alignment_keeps_its_rows():
         assert pool.data_ptr() % 16 == 2 * off
         assert (_plan([(0, 100)], pool=pool) is not None) == (off == 0)
     assert _plan([(0, 100)]) is not None
+
+
+def test_products_that_torch_would_change_keep_the_rows():
+    w = lambda **k: torch.zeros(8, 8, **dict(dict(dtype=torch.bfloat16), **k))                     # noqa: E731
+    assert _plan([(0, 100)], weights=(w(), w())) is not None
+    assert _plan([(0, 100)], weights=(w(), w(dtype=torch.float16))) is None
+    assert _plan([(0, 100)], weights=(w(requires_grad=True), w())) is None
+    with torch.no_grad():
+        assert _plan([(0, 100)], weights=(w(requires_grad=True), w())) is not None
+    torch.set_autocast_enabled("cuda", True)
+    try:
+        assert _plan([(0, 100)], weights=(w(), w())) is None
+    finally:
+        torch.set_autocast_enabled("cuda", False)

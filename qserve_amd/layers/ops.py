@@ -295,13 +295,17 @@ class HipOps:
         Writing keys and values out costs the keys' products with w_uk and w_uv; the queries' and the results' go, and the attention costs 320 products in place
         of 1088 per query, key and head (rank 512 + 64).  Whole layer, on the rows / this way, us, 16 heads, rank 512 + 64: runs of 65 / 300 / 1000 new tokens
         79 / 61, 108 / 75, 177 / 111; 512 behind 512 / 1536: 131 / 96, 154 / 122; 33 behind 67, four of them 92 / 73; 512 beside three single tokens at 1000
-        (7 keys a token) 130 / 118; 128 behind 1024 (9) 98 / 96.  The line is at 4 keys a token, which also bounds what is written out; up to 64
-        tokens the products per head have a kernel of their own."""
+        (7 keys a token) 130 / 118; 128 behind 1024 (9) 98 / 96.  The line is at 4 keys a token; up to 64 tokens the products per head have a kernel of their own.
+        What is written out, 512 bytes a key and head, is bounded by what the attention on the rows holds at the same time (a token's absorbed query, once
+        in bfloat16 and once in float with its rotated part) or by 256 MB: beyond that no prompt takes more memory this way."""
         if not (self.prompt_heads_kernel and scale > 0 and heads <= 1 << 12 and self.L.qsv_latent_prompt_ok(dim, rot_dim, vdim, rank, self.code)
                 and (pool is None or pool.data_ptr() % 16 == 0) and _called_plainly(*weights) and all(w.dtype == self.dtype for w in weights)):
             return None
         plan = batch.key_runs(window, self.L.qsv_latent_prompt_tile_tokens()) if batch.n_tokens > 64 else None
-        return plan if plan is not None and plan[2] <= min(4 * batch.n_tokens, 1 << 23) else None
+        T = batch.n_tokens
+        if plan is None or plan[2] > min(4 * T, 1 << 23) or plan[2] * heads * 512 > max(1 << 28, T * heads * (6 * rank + 4 * rot_dim)):
+            return None
+        return plan
 
     def latent_prompt(self, q, pool, batch, plan, w_uk, w_uv, rope, scale, heads, rot_dim, rot_n, rank, page, window, gate=None):
         """q [T, heads (dim + rot_dim)] attends its runs' cached rows through w_uk [heads dim, rank] and w_uv [heads vdim, rank] -> [T, heads vdim], times

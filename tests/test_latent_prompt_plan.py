@@ -42,3 +42,13 @@ def test_products_that_torch_would_change_keep_the_rows():
         assert _plan([(0, 100)], weights=(w(), w())) is None
     finally:
         torch.set_autocast_enabled("cuda", False)
+
+
+# 512 bytes a key and head written out against 6 rank + 4 rot_dim bytes a token and head on the rows, beyond 256 MB
+@pytest.mark.parametrize("runs, H, rot, rank, taken", [([(0, 8192)], 128, 64, 512, True), ([(24576, 8192)], 128, 64, 512, True), ([(8192, 8192)], 64, 64, 64, False),
+                                                       ([(0, 8192)], 64, 0, 64, True), ([(0, 8200)], 64, 0, 64, False), ([(0, 4000)], 64, 0, 64, True),
+                                                       ([(4000, 4000)], 128, 0, 128, False), ([(4000, 4000)], 128, 0, 176, True)])
+def test_what_is_written_out_is_bounded(runs, H, rot, rank, taken):
+    plan = _plan(runs, H=H, rot=rot, rank=rank)
+    assert (plan is not None) == taken
+    assert plan is None or plan[2] * H * 512 <= max(1 << 28, sum(n for _, n in runs) * H * (6 * rank + 4 * rot))

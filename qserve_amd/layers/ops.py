@@ -296,16 +296,21 @@ class HipOps:
         of 1088 per query, key and head (rank 512 + 64).  Whole layer, on the rows / this way, us, 16 heads, rank 512 + 64: runs of 65 / 300 / 1000 new tokens
         79 / 61, 108 / 75, 177 / 111; 512 behind 512 / 1536: 131 / 96, 154 / 122; 33 behind 67, four of them 92 / 73; 512 beside three single tokens at 1000
         (7 keys a token) 130 / 118; 128 behind 1024 (9) 98 / 96.  The line is at 4 keys a token; up to 64 tokens the products per head have a kernel of their own.
+        A workgroup walks all keys of 128 tokens and a head, 1.2 us for 64, where the attention on the rows cuts them over the chip.  So one or two heads
+        never (one, rank 512 + 64: 4000 tokens 131 / 149, 1000 behind 3000 83 / 137; rank 128: 89 / 124, 62 / 115; two 106 / 143, 72 / 119), and where a
+        run's tokens see more than 1024 keys on average only with 48 workgroups (three heads, 1000 behind 3000: 124 / 144, 90 / 127; 500 behind 1500, two of
+        them 100 / 106, 73 / 90; 512 behind 512 81 / 72, 58 / 55; 2000 new tokens 132 / 104, 91 / 85; six, 1000 behind 3000 190 / 155, 135 / 132).
         What is written out, 512 bytes a key and head, is bounded by what the attention on the rows holds at the same time (a token's absorbed query, once
         in bfloat16 and once in float with its rotated part) or by 256 MB: beyond that no prompt takes more memory this way."""
-        if not (self.prompt_heads_kernel and scale > 0 and heads <= 1 << 12 and self.L.qsv_latent_prompt_ok(dim, rot_dim, vdim, rank, self.code)
+        if not (self.prompt_heads_kernel and scale > 0 and 2 < heads <= 1 << 12 and self.L.qsv_latent_prompt_ok(dim, rot_dim, vdim, rank, self.code)
                 and (pool is None or pool.data_ptr() % 16 == 0) and _called_plainly(*weights) and all(w.dtype == self.dtype for w in weights)):
             return None
         plan = batch.key_runs(window, self.L.qsv_latent_prompt_tile_tokens()) if batch.n_tokens > 64 else None
         T = batch.n_tokens
         if plan is None or plan[2] > min(4 * T, 1 << 23) or plan[2] * heads * 512 > max(1 << 28, T * heads * (6 * rank + 4 * rot_dim)):
             return None
-        return plan
+        keys = max(start + n // 2 for (_, _, n), start in zip(batch.items, batch.starts))
+        return plan if (min(keys, int(window)) if window else keys) <= 1024 or plan[1].size(0) * heads >= 48 else None
 
     def latent_prompt(self, q, pool, batch, plan, w_uk, w_uv, rope, scale, heads, rot_dim, rot_n, rank, page, window, gate=None):
         """q [T, heads (dim + rot_dim)] attends its runs' cached rows through w_uk [heads dim, rank] and w_uv [heads vdim, rank] -> [T, heads vdim], times

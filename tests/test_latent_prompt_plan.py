@@ -52,3 +52,12 @@ def test_what_is_written_out_is_bounded(runs, H, rot, rank, taken):
     plan = _plan(runs, H=H, rot=rot, rank=rank)
     assert (plan is not None) == taken
     assert plan is None or plan[2] * H * 512 <= max(1 << 28, sum(n for _, n in runs) * H * (6 * rank + 4 * rot))
+
+
+# workgroups (128 tokens and a head each) against the keys that a run's tokens see on average
+@pytest.mark.parametrize("runs, H, window, taken", [([(0, 4000)], 1, None, False), ([(0, 300)], 2, None, False), ([(0, 65)], 3, None, True), ([(0, 2000)], 3, None, True),
+                                                    ([(512, 512)], 3, None, True), ([(775, 500)], 3, None, False), ([(774, 500)], 3, None, True), ([(3000, 1000)], 3, None, False),
+                                                    ([(3000, 1000)], 6, None, True), ([(1500, 500)] * 2, 4, None, False), ([(1500, 500)] * 3, 4, None, True),
+                                                    ([(3000, 1000)], 3, 1024, True), ([(3000, 1000)], 3, 1025, False)])
+def test_long_walks_need_workgroups(runs, H, window, taken):
+    assert (_plan(runs, H=H, window=window) is not None) == taken

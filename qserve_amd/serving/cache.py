@@ -78,6 +78,14 @@ class PagedCache:
         self.pages[s], self.length[s] = [], 0
         return s
 
+    def room_for(self, slots, counts):
+        """Raises CacheFull, with nothing changed, if these sequences cannot all grow by their counts."""
+        if sum(counts) // self.page + len(slots) <= len(self.free_pages):      # (no sequence needs more than n / page + 1)
+            return
+        need = sum(self.pages_for(self.length[s] + n) - len(self.pages[s]) for s, n in zip(slots, counts))
+        if need > len(self.free_pages):
+            raise CacheFull(f"{need} more pages needed, {len(self.free_pages)} free of {self.num_pages}")
+
     def _grow(self, slot, n):
         """Pages for n more tokens of `slot`.  -> (its pages, tokens it held before)."""
         have, start = self.pages[slot], self.length[slot]

@@ -177,6 +177,7 @@ class Engine:
             return None
         ids = self._all_ids([t for (_, t), n in zip(items, counts) if n])
         counts = [n for n in counts if n]
+        cache.room_for(slots, counts)                                  # (a step that is refused leaves every sequence as it was)
         R, T = len(slots), len(ids)
         single = T == R
         flat = np.empty(8 * T + (7 if single else 4) * R, dtype=np.int32)

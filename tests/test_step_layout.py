@@ -149,3 +149,25 @@ def test_runs_of_different_kinds_of_tokens(kinds, n):
     assert [e.cache.length[s] for s, _ in slots] == before          # (nothing of a refused step stays)
     with pytest.raises(KeyError):
         e._layout_host([(slots[0][0], [1]), (77, [])])
+
+
+@pytest.mark.parametrize("filled, step", [((8, 8, 8), (1, 1, 1)), ((8, 7, 8), (1, 1, 1)), ((1, 1, 1), (8, 8, 16)), ((3, 9, 0), (5, 8, 1)), ((8, 8, 0), (1, 0, 9))])
+def test_a_step_without_room_leaves_every_sequence_as_it_was(filled, step):
+    for pages, room in ((0, False), (1, False), (2, None), (3, None), (40, True)):       # (free pages; None: as the counts say)
+        e, _, slots = _pair(pages=sum(-(-n // 8) for n in filled) + pages)
+        c = e.cache
+        for (s, _), n in zip(slots, filled):
+            if n:
+                e.layout([(s, [1] * n)])
+        need = sum(-(-(a + b) // 8) - -(-a // 8) for a, b in zip(filled, step))
+        state = lambda: (dict(c.length), {k: list(v) for k, v in c.pages.items()}, list(c.free_pages), list(c.parity), c.table_host.clone().tolist())     # noqa: E731
+        before, items = state(), [(s, [2] * n) for (s, _), n in zip(slots, step)]
+        assert len(c.free_pages) == pages and (room is None or room == (need <= pages))
+        if need <= pages:
+            assert e.layout(items).n_tokens == sum(step)
+            continue
+        with pytest.raises(CacheFull):
+            e.layout(items)
+        assert state() == before
+        e.close_sequence(slots[4][0])                                    # ... and goes on
+        assert e.layout([(slots[0][0], [3] * (-filled[0] % 8))]) is not None or filled[0] % 8 == 0

@@ -136,13 +136,17 @@ class PagedCache:
         del self.length[slot]
         self.free_slots.append(slot)
 
+    def _new_by_kernel(self):
+        """Whether a launch's arguments carry what is new in the table: few entries, places that 32 bits hold, the device that launches go to."""
+        return (self.table.is_cuda and len(self._entered) <= 480 and self.table.numel() <= 2 ** 31 and self.table.device.index == torch.cuda.current_device())
+
     def block_table(self):
         """The device copy of the block table, uploaded if pages were handed out since the last call."""
         if self._dirty:
-            if self.table.is_cuda and len(self._entered) <= 480:       # (a step's few: no copy command, and no more than what is new)
+            if self._new_by_kernel():                                  # (a step's few: no copy command, and no more than what is new)
                 new = np.array(list(self._entered.items()), dtype=np.int32)
                 check(lib().qsv_set_words(self.table.data_ptr(), new.ctypes.data, len(new), torch.cuda.current_stream(self.table.device).cuda_stream), "set_words")
-            elif self.table.is_cuda:                                     # (a pinned copy: the host's table may change before the device has read it)
+            elif self.table.is_cuda:                                   # (a pinned copy: the host's table may change before the device has read it)
                 self.table.copy_(torch.empty(self.table_host.shape, dtype=torch.int32, pin_memory=True).copy_(self.table_host), non_blocking=True)
             else:
                 self.table.copy_(self.table_host)

@@ -171,3 +171,12 @@ def test_a_step_without_room_leaves_every_sequence_as_it_was(filled, step):
         assert state() == before
         e.close_sequence(slots[4][0])                                    # ... and goes on
         assert e.layout([(slots[0][0], [3] * (-filled[0] % 8))]) is not None or filled[0] % 8 == 0
+
+
+@pytest.mark.parametrize("entries, size, index, taken", [(480, 2 ** 31, 0, True), (481, 100, 0, False), (1, 2 ** 31 + 64, 0, False), (1, 100, 1, False)])
+def test_when_new_places_of_the_table_travel_with_a_launch(monkeypatch, entries, size, index, taken):
+    e, _, _ = _pair()
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    e.cache._entered = dict.fromkeys(range(entries), 1)
+    e.cache.table = type("T", (), {"is_cuda": True, "numel": lambda self: size, "device": torch.device("cuda", index)})()
+    assert e.cache._new_by_kernel() == taken

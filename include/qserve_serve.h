@@ -25,6 +25,8 @@ const char* qsv_last_error(void);
 int qsv_skinny_linear(void* out, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K, void* stream);
 /* The same values in float. */
 int qsv_skinny_linear_widened(float* out, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K, void* stream);
+/* Either of them (widened: in float) with weights that are to stay in the caches; qsv_skinny_linear lets large ones that it reads once stream past them. */
+int qsv_skinny_linear_kept(void* out, int widened, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K, void* stream);
 /* decay [n_rows, N] = qsv_decay of x @ w^T (bias [N], a_log [N / dim] or NULL and tau), and, with gate_N > 0, gate = gate_x @ gate_w^T, in one launch. */
 int qsv_decay_products(float* decay, const void* x, int64_t x_stride, const void* w, int N, int K, const void* bias, const float* a_log, float tau, int dim,
                        void* gate, const void* gate_x, int64_t gate_x_stride, const void* gate_w, int gate_N, int gate_K, int n_rows, void* stream);
@@ -312,6 +314,9 @@ int qsv_expert_slots(void* out, int float_out, const void* X, int div, const voi
 /* The same with a shared expert in the launch: rows 0 .. sh_n - 1 of sh_X [sh_n, sh_K] through sh_W [sh_rows, sh_K] and the same activation -> sh_out (bfloat16). */
 int qsv_expert_slots_shared(void* out, int float_out, const void* X, int div, const void* W, const int32_t* idx, int n, int n_experts, int rows, int K, int act,
                             float limit, const float* in_weight, void* sh_out, const void* sh_X, const void* sh_W, int sh_n, int sh_rows, int sh_K, void* stream);
+/* Either of them (sh_W NULL: no shared expert) with weights that are to stay in the caches; see qsv_skinny_linear_kept. */
+int qsv_expert_slots_kept(void* out, int float_out, const void* X, int div, const void* W, const int32_t* idx, int n, int n_experts, int rows, int K, int act,
+                          float limit, const float* in_weight, void* sh_out, const void* sh_X, const void* sh_W, int sh_n, int sh_rows, int sh_K, void* stream);
 /* Grouped expert product on the bf16 matrix cores (prompt phase): qsv_moe_sort orders the n slots by expert (order: sorted slot -> slot,
  * place: slot -> sorted slot, offsets [n_experts + 1]: first sorted slot of every expert; indices below 0 and from n_experts on are left out of all
  * three), and the product takes those: out[s, r] = act(W[e][r, :] . X[order ? order[s] / div : s, :]) for the sorted slots of every expert

@@ -250,7 +250,7 @@ static int skinny_fits(const char* what, const void* out, const void* x, int64_t
     return QSV_OK;
 }
 template <int HOW>
-static int launch_skinny(const char* what, void* out, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K, void* stream) {
+static int launch_skinny(const char* what, void* out, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K, void* stream, bool kept = false) {
     const int rc = skinny_fits(what, out, x, x_stride, w, n_rows, N, K);
     if (rc != QSV_OK || n_rows == 0) return rc;
     const SkinnyJob a = {out, (const bf16_t*)x, x_stride, (const bf16_t*)w, n_rows, N, K, N % 4 == 0 && (uintptr_t)out % (HOW == AS_IS ? 8 : 16) == 0, nullptr, nullptr, 0.f, 1};
@@ -258,7 +258,7 @@ static int launch_skinny(const char* what, void* out, const void* x, int64_t x_s
     // which reads the inputs half as often (6144 x 2048: 8.2 -> 7.4 us)
     const bool few = n_rows <= 16, small = N < 5120 || (N > 8192 && N <= 16384 && n_rows <= 32);
     // every weight is read once, or twice at the same time
-    const bool once = streams_once(w, N, K);
+    const bool once = !kept && streams_once(w, N, K);
 #define QSV_SKINNY(RB, SG)                                                                                                                    \
     do {                                                                                                                                      \
         const dim3 grid((N + 16 * RB - 1) / (16 * RB), (n_rows + 16 * SG - 1) / (16 * SG)), block(64 * STREAM_WAVES);                         \
@@ -279,6 +279,11 @@ extern "C" int qsv_skinny_linear(void* out, const void* x, int64_t x_stride, con
 // the same values in float
 extern "C" int qsv_skinny_linear_widened(float* out, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K, void* stream) {
     return launch_skinny<WIDENED>("qsv_skinny_linear_widened", out, x, x_stride, w, n_rows, N, K, stream);
+}
+// either of them with weights that are to stay in the caches
+extern "C" int qsv_skinny_linear_kept(void* out, int widened, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K, void* stream) {
+    return widened ? launch_skinny<WIDENED>("qsv_skinny_linear_kept", out, x, x_stride, w, n_rows, N, K, stream, true)
+                   : launch_skinny<AS_IS>("qsv_skinny_linear_kept", out, x, x_stride, w, n_rows, N, K, stream, true);
 }
 // decay [n_rows, N] (float) of z = x @ w^T as qsv_decay makes it, and, with gate_N > 0, gate [n_rows, gate_N] = gate_x @ gate_w^T
 extern "C" int qsv_decay_products(float* decay, const void* x, int64_t x_stride, const void* w, int N, int K, const void* bias, const float* a_log, float tau, int dim,

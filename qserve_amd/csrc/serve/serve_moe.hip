@@ -664,7 +664,7 @@ extern "C" int qsv_gather_rows(void* out, const void* src, const int64_t* order,
                                     order, div, width));
     return qsv_launch_status("qsv_gather_rows");
 }
-static int launch_expert_rows(const char* what, ExpertArgs a, int n_experts, int act, bool float_out, void* stream, SharedArgs sh = {}) {
+static int launch_expert_rows(const char* what, ExpertArgs a, int n_experts, int act, bool float_out, void* stream, SharedArgs sh = {}, bool kept = false) {
     QSV_REQUIRE(a.out && a.X && a.W && n_experts > 0 && a.rows > 0 && a.div > 0, "%s: bad arguments", what);
     QSV_REQUIRE(act == ACT_NONE || act == ACT_RELU_SQ || ((act == ACT_GLU || act == QSV_ACT_CLAMPED_GLU) && a.rows % 2 == 0), "%s: activation %d", what,
                 act);
@@ -676,8 +676,8 @@ static int launch_expert_rows(const char* what, ExpertArgs a, int n_experts, int
     QSV_REQUIRE(n_experts <= 65535, "%s: too many experts", what);
     QSV_REQUIRE(((uintptr_t)a.X | (uintptr_t)a.W) % 16 == 0, "%s: inputs and weights start on 16 bytes", what);
     a.wide = (uintptr_t)a.out % 16 == 0;
-    a.once = streams_once(a.W, (int64_t)n_experts * a.rows, a.K);
-    sh.once = streams_once(sh.W, sh.rows, sh.K);
+    a.once = !kept && streams_once(a.W, (int64_t)n_experts * a.rows, a.K);
+    sh.once = !kept && streams_once(sh.W, sh.rows, sh.K);
     const dim3 grid(((sh.W && sh.rows > a.rows ? sh.rows : a.rows) + XR - 1) / XR, n_experts + (sh.W ? 1 : 0)), block(NT);
     if (float_out) hipLaunchKernelGGL((expert_rows_kernel<ACT_NONE, true>), grid, block, 0, (hipStream_t)stream, a, sh);
     else if (act == ACT_RELU_SQ) hipLaunchKernelGGL((expert_rows_kernel<ACT_RELU_SQ, false>), grid, block, 0, (hipStream_t)stream, a, sh);
@@ -698,17 +698,33 @@ extern "C" int qsv_expert_slots(void* out, int float_out, const void* X, int div
     const ExpertArgs a = {out, (const bf16_t*)X, (const bf16_t*)W, idx, nullptr, nullptr, in_weight, n, div, rows, K, limit, false, false, false};
     return launch_expert_rows("qsv_expert_slots", a, n_experts, act, float_out != 0, stream);
 }
-// ... and every token's row of X through a shared expert of sh_rows x sh_K in the same launch: sh_out [n / div, sh_rows (/ 2 for gated units)]
+// ... and, with sh_W, every token's row of X through a shared expert of sh_rows x sh_K in the same launch: sh_out [n / div, sh_rows (/ 2 for gated units)]
+static int expert_slots_shared(const char* what, bool kept, void* out, int float_out, const void* X, int div, const void* W, const int32_t* idx, int n, int n_experts,
+                               int rows, int K, int act, float limit, const float* in_weight, void* sh_out, const void* sh_X, const void* sh_W, int sh_n, int sh_rows,
+                               int sh_K, void* stream) {
+    QSV_REQUIRE(idx && n >= 0 && (!float_out || act == ACT_NONE) && n_experts < 65535, "%s: bad arguments", what);
+    if (sh_W) {
+        QSV_REQUIRE(sh_out && sh_X && sh_n > 0 && sh_rows > 0, "%s: bad arguments", what);
+        QSV_REQUIRE(sh_K > 0 && sh_K % 8 == 0 && sh_K <= 1 << 25 && ((uintptr_t)sh_X | (uintptr_t)sh_W) % 16 == 0, "%s: inner width %d, rows on 16 bytes", what, sh_K);
+        QSV_REQUIRE(act == ACT_NONE || act == ACT_RELU_SQ || sh_rows % 2 == 0, "%s: %d rows of gated units", what, sh_rows);
+    }
+    if (n == 0) return QSV_OK;
+    const ExpertArgs a = {out, (const bf16_t*)X, (const bf16_t*)W, idx, nullptr, nullptr, in_weight, n, div, rows, K, limit, false, false, false};
+    const SharedArgs sh = {sh_out, (const bf16_t*)sh_X, (const bf16_t*)sh_W, sh_n, sh_rows, sh_K, (uintptr_t)sh_out % 16 == 0, false};
+    return launch_expert_rows(what, a, n_experts, act, float_out != 0, stream, sh_W ? sh : SharedArgs{}, kept);
+}
 extern "C" int qsv_expert_slots_shared(void* out, int float_out, const void* X, int div, const void* W, const int32_t* idx, int n, int n_experts, int rows, int K,
                                        int act, float limit, const float* in_weight, void* sh_out, const void* sh_X, const void* sh_W, int sh_n, int sh_rows, int sh_K,
                                        void* stream) {
-    QSV_REQUIRE(idx && n >= 0 && (!float_out || act == ACT_NONE) && sh_out && sh_X && sh_W && sh_n > 0 && sh_rows > 0 && n_experts < 65535, "qsv_expert_slots_shared: bad arguments");
-    QSV_REQUIRE(sh_K > 0 && sh_K % 8 == 0 && sh_K <= 1 << 25 && ((uintptr_t)sh_X | (uintptr_t)sh_W) % 16 == 0, "qsv_expert_slots_shared: inner width %d, rows on 16 bytes", sh_K);
-    QSV_REQUIRE(act == ACT_NONE || act == ACT_RELU_SQ || sh_rows % 2 == 0, "qsv_expert_slots_shared: %d rows of gated units", sh_rows);
-    if (n == 0) return QSV_OK;
-    const ExpertArgs a = {out, (const bf16_t*)X, (const bf16_t*)W, idx, nullptr, nullptr, in_weight, n, div, rows, K, limit, false, false, false};
-    return launch_expert_rows("qsv_expert_slots_shared", a, n_experts, act, float_out != 0, stream,
-                              {sh_out, (const bf16_t*)sh_X, (const bf16_t*)sh_W, sh_n, sh_rows, sh_K, (uintptr_t)sh_out % 16 == 0, false});
+    QSV_REQUIRE(sh_W, "qsv_expert_slots_shared: bad arguments");
+    return expert_slots_shared("qsv_expert_slots_shared", false, out, float_out, X, div, W, idx, n, n_experts, rows, K, act, limit, in_weight, sh_out, sh_X, sh_W, sh_n,
+                               sh_rows, sh_K, stream);
+}
+// either of them (sh_W NULL: no shared expert) with weights that are to stay in the caches
+extern "C" int qsv_expert_slots_kept(void* out, int float_out, const void* X, int div, const void* W, const int32_t* idx, int n, int n_experts, int rows, int K, int act,
+                                     float limit, const float* in_weight, void* sh_out, const void* sh_X, const void* sh_W, int sh_n, int sh_rows, int sh_K, void* stream) {
+    return expert_slots_shared("qsv_expert_slots_kept", true, out, float_out, X, div, W, idx, n, n_experts, rows, K, act, limit, in_weight, sh_out, sh_X, sh_W, sh_n, sh_rows,
+                               sh_K, stream);
 }
 extern "C" int qsv_relu_sq(void* a, int64_t n, int dtype, void* stream) {
     QSV_REQUIRE(a && n >= 0 && n < (1ll << 31) * NT, "qsv_relu_sq: bad arguments");

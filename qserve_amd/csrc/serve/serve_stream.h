@@ -36,9 +36,12 @@ __device__ __forceinline__ void lds_copy16(unsigned dst, const void* from) {
 }
 
 // ONCE: the launch reads every weight once, so non-temporally: a large stream gets 4 - 10 % faster (92 / 185 MB of experts 21.5 / 39.1 -> 19.5 / 36.8 us, 4096 x 4096
-// 8.9 -> 8.5; weights that a cache holds from step to step, less than 200 MB in all, lose as much).  Where workgroups read the same rows one after another, or rows
-// start inside a line of 128 bytes, whose halves two requests would fetch, it loses (2560 x 5120 read twice 16.1 -> 20.7).
-// Under 1 MB, which a cache keeps beside anything, it loses too (64 x 2048 of 64 inputs 5.0 -> 5.6).
+// 8.9 -> 8.5).  Where workgroups read the same rows one after another, or rows start inside a line of 128 bytes, whose halves two requests would fetch, it loses
+// (2560 x 5120 read twice 16.1 -> 20.7).  Under 1 MB, which a cache keeps beside anything, it loses too (64 x 2048 of 64 inputs 5.0 -> 5.6).
+// A model whose weights the caches hold from step to step loses by it with many rows (the forms *_kept, which the engine asks for): whole steps of four layers, 74 /
+// 116 / 187 / 194 / 234 MB of weights, non-temporally -> kept, us: 8 rows 234 -> 246, 204 -> 208, 223 -> 225, 227 -> 226, 224 -> 228, 24 rows 250 -> 255, 222 -> 218,
+// 240 -> 235, 245 -> 240, 243 -> 244, 32 rows 258 -> 257, 227 -> 220, 243 -> 238, 253 -> 243, 248 -> 247, 64 rows 290 -> 287, 260 -> 255, 268 -> 266, 287 -> 284, 270 ->
+// 270.  So up to 200 MB they are kept in steps of more than 24 rows.  Larger ones lose by that at any number (24 layers of 43 MB: 17 / 32 rows 1340 -> 1446, 1377 -> 1477).
 inline bool streams_once(const void* w, int64_t rows, int K) { return K % 64 == 0 && (uintptr_t)w % 128 == 0 && rows * K >= 1 << 19; }
 // acc[r][g]: this wave's share of the products of weight rows W0 + 16 r + .. (rows_here of them, K elements each) with inputs 16 g + ..;
 // input(i): where input i starts.  w (the wave) is wave-uniform; `ring`: its XRING bytes of LDS.

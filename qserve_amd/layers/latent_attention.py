@@ -12,7 +12,6 @@ rotary table for the rotated part (first `rot_n` of its dimensions), a sigmoid o
 """
 import torch
 
-from .ops import linear
 
 
 class LatentAttention:
@@ -49,15 +48,15 @@ class LatentAttention:
         """h [T, D] (storage type) -> mixer output [T, D]; writes this step's rows into `pool` ([rows, row_width])."""
         ops, T, H = self.ops, h.size(0), self.H
         rope = self.rotary.reserve(batch.max_pos + 1) if self.rot_n else None
-        down = linear(h, self.w_down)
+        down = self.ops.linear(h, self.w_down)
         cq = ops.latent_prep(down, self.q_off, self.q_rank, self.dq_norm, self.kv_off, self.rank, self.dkv_norm, self.rot_dim,
                              self.rot_n, rope, pool, batch.slot, batch.pos, self.eps)
-        q = linear(cq, self.w_uq)                                                   # [T, H (dim + rot_dim)]
+        q = self.ops.linear(cq, self.w_uq)                                                   # [T, H (dim + rot_dim)]
         gate = down[:, self.g_off:self.g_off + H * self.vdim] if self.gated else None
         plan = ops.latent_prompt_plan(batch, self.window, H, self.dim, self.rot_dim, self.vdim, self.rank, self.scale, pool, (self.w_uk, self.w_uv))
         if plan is not None:
-            return linear(ops.latent_prompt(q, pool, batch, plan, self.w_uk.view(H * self.dim, self.rank), self.w_uv, rope, self.scale, H, self.rot_dim,
+            return self.ops.linear(ops.latent_prompt(q, pool, batch, plan, self.w_uk.view(H * self.dim, self.rank), self.w_uv, rope, self.scale, H, self.rot_dim,
                                             self.rot_n, self.rank, self.page, self.window, gate), self.w_o)
         qf = ops.latent_queries(q, self.w_uk, rope, batch.pos, self.scale, H, self.dim, self.rot_dim, self.rot_n, self.rank)
         o_lat = ops.latent_attention(qf, pool, batch, self.window, self.rank, self.page)
-        return linear(ops.head_products(o_lat, self.w_uv_t, gate), self.w_o)
+        return self.ops.linear(ops.head_products(o_lat, self.w_uv_t, gate), self.w_o)

@@ -49,9 +49,8 @@ class GatedFeedForward:
 
     def __call__(self, h, rows=False):
         """rows: as the mixtures below take it; there is one row per token here, its sum."""
-        from .ops import linear
-        a = linear(h, self.w_in)
-        return linear(self.ops.glu(a) if self.act == "silu" else self.ops.glu(a, self.act, self.limit), self.w_down)
+        a = self.ops.linear(h, self.w_in)
+        return self.ops.linear(self.ops.glu(a) if self.act == "silu" else self.ops.glu(a, self.act, self.limit), self.w_down)
 
 
 class TopKGatedMoE:
@@ -134,8 +133,7 @@ class ReluSquaredFeedForward:
         self.ops, self.w_up, self.w_down = ops, up.contiguous(), down.contiguous()
 
     def __call__(self, h):
-        from .ops import linear
-        return linear(self.ops.relu_sq(linear(h, self.w_up)), self.w_down)
+        return self.ops.linear(self.ops.relu_sq(self.ops.linear(h, self.w_up)), self.w_down)
 
 
 class IdentityExpertMoE:

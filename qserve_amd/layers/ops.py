@@ -92,26 +92,31 @@ def _streams(x, w):
             and x.device == w.device and x.device.index == torch.cuda.current_device())
 
 
-def linear(x, w):
+def _stream_product(x, w, out, kept):
+    from ..serving._lib import check, lib
+    L, widened = lib(), out.dtype == torch.float32
+    rest = (x.data_ptr(), x.stride(0), w.data_ptr(), x.size(0), w.size(0), x.size(1), torch.cuda.current_stream(x.device).cuda_stream)
+    if kept:
+        check(L.qsv_skinny_linear_kept(out.data_ptr(), int(widened), *rest), "skinny_linear_kept")
+    elif widened:
+        check(L.qsv_skinny_linear_widened(out.data_ptr(), *rest), "skinny_linear_widened")
+    else:
+        check(L.qsv_skinny_linear(out.data_ptr(), *rest), "skinny_linear")
+    return out
+
+
+def linear(x, w, kept=False):
     """x [T, in] @ w [out, in]^T in the storage type, float accumulation: the few rows of a decoding step (bfloat16 on a GPU) through
-    qsv_skinny_linear, everything else through hipBLASLt / rocBLAS."""
+    qsv_skinny_linear, everything else through hipBLASLt / rocBLAS.  kept: w is to stay in the caches (see HipOps.kept_above)."""
     if _streams(x, w):
-        from ..serving._lib import check, lib
-        out = torch.empty((x.size(0), w.size(0)), dtype=x.dtype, device=x.device)
-        check(lib().qsv_skinny_linear(out.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(), x.size(0), w.size(0), x.size(1),
-                                      torch.cuda.current_stream(x.device).cuda_stream), "skinny_linear")
-        return out
+        return _stream_product(x, w, torch.empty((x.size(0), w.size(0)), dtype=x.dtype, device=x.device), kept)
     return torch.matmul(x, w.t())
 
 
-def float_linear(x, w):
+def float_linear(x, w, kept=False):
     """linear(x, w).float(): a step's few rows in one launch."""
     if _streams(x, w):
-        from ..serving._lib import check, lib
-        out = torch.empty((x.size(0), w.size(0)), dtype=torch.float32, device=x.device)
-        check(lib().qsv_skinny_linear_widened(out.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(), x.size(0), w.size(0), x.size(1),
-                                              torch.cuda.current_stream(x.device).cuda_stream), "skinny_linear_widened")
-        return out
+        return _stream_product(x, w, torch.empty((x.size(0), w.size(0)), dtype=torch.float32, device=x.device), kept)
     return torch.matmul(x, w.t()).float()
 
 
@@ -170,6 +175,18 @@ class HipOps:
         for t in ts:
             if t is not None and not (t.is_cuda and t.is_contiguous()):
                 raise RuntimeError("serving kernels need contiguous tensors on the GPU")
+
+    # Rows beyond which a step's weights are left in the caches (None: never; the engine sets it for a model that they hold, see serve_stream.h's streams_once)
+    kept_above = None
+
+    def _kept(self, rows):
+        return self.kept_above is not None and rows > self.kept_above
+
+    def linear(self, x, w):
+        return linear(x, w, self._kept(x.size(0)))
+
+    def float_linear(self, x, w):
+        return float_linear(x, w, self._kept(x.size(0)))
 
     def put_words(self, out, words):
         """out (int32, on the GPU) = words (a numpy int32 array), which the caller may change at once."""
@@ -980,7 +997,7 @@ class HipOps:
             self.check(self.L.qsv_decay_products(out.data_ptr(), z.data_ptr(), z.stride(0), w.data_ptr(), N, w.size(1), bias.data_ptr(),
                                                  0 if a_log is None else a_log.data_ptr(), float(tau), dim, *more, T, self._s()), "decay_products")
             return out, g
-        return self.decay(linear(z, w), bias, a_log, tau, heads, dim), None if gate is None else linear(gate, w_gate)
+        return self.decay(self.linear(z, w), bias, a_log, tau, heads, dim), None if gate is None else self.linear(gate, w_gate)
 
     def conv_silu_unit(self, proj, off, conv_w, hist, batch, n_unit, unit_dim, act="silu"):
         """Causal convolution over time of the columns [off, off + C) of proj with per-channel taps conv_w [C, taps], then silu
@@ -1157,21 +1174,21 @@ class HipOps:
         act = torch.empty((n, ff), dtype=self.dtype, device=h.device)
         ys = torch.empty((n, D), dtype=torch.float32, device=h.device)
         s = self._s()
+        kept = self._kept(T)
+        sff, sy, first, second = 0, None, (0, 0, 0, 0, 0, 0), (0, 0, 0, 0, 0, 0)
         if shared is not None:
             sff = shared[1].size(1)
             sact, sy = torch.empty((T, sff), dtype=self.dtype, device=h.device), torch.empty((T, D), dtype=self.dtype, device=h.device)
-            self.check(self.L.qsv_expert_slots_shared(act.data_ptr(), 0, h.data_ptr(), K, up.data_ptr(), idx.data_ptr(), n, E, rows, D, a, float(limit), w_in,
-                                                      sact.data_ptr(), h.data_ptr(), shared[0].data_ptr(), T, 2 * sff, D, s), "expert_slots_shared(up)")
-            self.check(self.L.qsv_expert_slots_shared(ys.data_ptr(), 1, act.data_ptr(), 1, down.data_ptr(), idx.data_ptr(), n, E, D, ff, 0, 0.0, 0,
-                                                      sy.data_ptr(), sact.data_ptr(), shared[1].data_ptr(), T, D, sff, s), "expert_slots_shared(down)")
-            y = ExpertRows(self, ys, None, wt if weigh == "output" else None, idx, h, E)
-            return (y if lazy else y.dense()), sy
-        self.check(self.L.qsv_expert_slots(act.data_ptr(), 0, h.data_ptr(), K, up.data_ptr(), idx.data_ptr(), n, E, rows, D, a, float(limit),
-                                           w_in, s), "expert_slots(up)")
-        self.check(self.L.qsv_expert_slots(ys.data_ptr(), 1, act.data_ptr(), 1, down.data_ptr(), idx.data_ptr(), n, E, D, ff, 0, 0.0, 0, s),
-                   "expert_slots(down)")
+            first = (sact.data_ptr(), h.data_ptr(), shared[0].data_ptr(), T, 2 * sff, D)
+            second = (sy.data_ptr(), sact.data_ptr(), shared[1].data_ptr(), T, D, sff)
+        launch = self.L.qsv_expert_slots_kept if kept else self.L.qsv_expert_slots_shared if shared is not None else self.L.qsv_expert_slots
+        if not kept and shared is None:
+            first = second = ()
+        self.check(launch(act.data_ptr(), 0, h.data_ptr(), K, up.data_ptr(), idx.data_ptr(), n, E, rows, D, a, float(limit), w_in, *first, s), "expert_slots(up)")
+        self.check(launch(ys.data_ptr(), 1, act.data_ptr(), 1, down.data_ptr(), idx.data_ptr(), n, E, D, ff, 0, 0.0, 0, *second, s), "expert_slots(down)")
         y = ExpertRows(self, ys, None, wt if weigh == "output" else None, idx, h, E)
-        return y if lazy else y.dense()
+        y = y if lazy else y.dense()
+        return y if shared is None else (y, sy)
 
     def _moe_experts_sorted(self, h, up, down, idx, wt, code=1, limit=0.0, weigh="output", lazy=False):
         """code >= 2 (gated units): the grouped kernel folds the two halves of a unit in its epilogue; with vendor products the
@@ -1249,6 +1266,14 @@ class TorchOps:
     def __init__(self, dtype):
         self.dtype = dtype
         dtype_code(dtype)
+
+    @staticmethod
+    def linear(x, w):
+        return linear(x, w)
+
+    @staticmethod
+    def float_linear(x, w):
+        return float_linear(x, w)
 
     def embed(self, tokens, table):
         h = table[tokens.long()]

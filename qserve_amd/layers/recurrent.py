@@ -17,7 +17,6 @@ that own its columns) and, for the convolution, the last taps - 1 inputs (two co
 import torch
 
 from ..serving.cache import StateSpec
-from .ops import linear
 
 
 def pad_rows(w, to=8):
@@ -46,12 +45,12 @@ class GatedLinearAttention:
 
     def __call__(self, h, batch, pools, states):
         ops, H, d, dv = self.ops, self.H, self.dim, self.vdim
-        proj = linear(h, self.w_in)
+        proj = self.ops.linear(h, self.w_in)
         o_q, o_k, o_v, o_g, o_a = 0, H * d, 2 * H * d, 2 * H * d + H * dv, 2 * H * d + 2 * H * dv
         a, _ = ops.decay_products(proj[:, o_a:o_a + self.r], self.w_a2, self.b_a2, None, self.tau, H, d)
         o = ops.recurrent_scan(proj[:, o_q:o_k], proj[:, o_k:o_v], proj[:, o_v:o_g], a, None, states[0], batch, H, H, d, dv,
                                d ** -0.5)
-        return linear(ops.head_rms_gate(o, self.norm, proj[:, o_g:o_a], "silu", self.eps), self.w_o)
+        return self.ops.linear(ops.head_rms_gate(o, self.norm, proj[:, o_g:o_a], "silu", self.eps), self.w_o)
 
 
 class GatedDeltaRule:
@@ -94,20 +93,20 @@ class GatedDeltaRule:
         """proj: h's product with w_in, where the caller has it already (a column slice is fine)."""
         ops, H, G, d, dv = self.ops, self.H, self.G, self.dim, self.vdim
         if proj is None:
-            proj = linear(h, self.w_in)
+            proj = self.ops.linear(h, self.w_in)
         o_b = self.C
         o_a, o_g = o_b + H, o_b + H + self.r
         qkv = ops.conv_silu_unit(proj, 0, self.conv, states[1], batch, 2 * G, d)       # float [T, C]: q | k (unit) | v
         z, gate = proj[:, o_a:o_g], proj[:, o_g:o_g + self.rg]
         if self.head_decay:
             g = ops.decay(z, self.dt_bias, self.a_log, 0.0, H, 1)                      # float [T, H]
-            gate = linear(gate, self.w_g2) if self.low_gate else gate
+            gate = self.ops.linear(gate, self.w_g2) if self.low_gate else gate
         else:
             g, low = ops.decay_products(z, self.w_a2, self.dt_bias, self.a_log, 0.0, H, d, *((gate, self.w_g2) if self.low_gate else ()))
             gate = low if self.low_gate else gate
         o = ops.recurrent_scan(qkv[:, :G * d], qkv[:, G * d:2 * G * d], qkv[:, 2 * G * d:], g, proj[:, o_b:o_a], states[0], batch,
                                H, G, d, dv, d ** -0.5)
-        return linear(ops.head_rms_gate(o, self.norm, gate, self.gate, self.eps), self.w_o)
+        return self.ops.linear(ops.head_rms_gate(o, self.norm, gate, self.gate, self.eps), self.w_o)
 
 
 class Retention:
@@ -131,12 +130,12 @@ class Retention:
 
     def __call__(self, h, batch, pools, states):
         ops, H, d, dv = self.ops, self.H, self.dim, self.vdim
-        proj = linear(h, self.w_in)
+        proj = self.ops.linear(h, self.w_in)
         o_v, o_g = 2 * H * d, 2 * H * d + H * dv
         rope = self.rotary.reserve(batch.max_pos + 1) if self.rotary is not None else None
         qkv = ops.rotate_qk(proj, H, d, dv, rope, self.rotary.dims if rope is not None else 0, batch)          # float [T, q | k | v]
         o = ops.recurrent_scan(qkv[:, :H * d], qkv[:, H * d:o_v], qkv[:, o_v:], self.decay, None, states[0], batch, H, H, d, dv, d ** -0.5)
-        return linear(ops.head_rms_gate(o, self.norm, proj[:, o_g:o_g + H * dv], "silu", self.eps), self.w_o)
+        return self.ops.linear(ops.head_rms_gate(o, self.norm, proj[:, o_g:o_g + H * dv], "silu", self.eps), self.w_o)
 
 
 class ParallelMixer:
@@ -156,7 +155,7 @@ class ParallelMixer:
     def __call__(self, h, batch, pools, states):
         pl = pr = {}
         if self.w_in is not None:
-            proj = linear(h, self.w_in)
+            proj = self.ops.linear(h, self.w_in)
             pl, pr = {"proj": proj[:, :self._cut]}, {"proj": proj[:, self._cut:]}
         a = self.left(h, batch, pools[:self._np], states[:self._ns], **pl)
         b = self.right(h, batch, pools[self._np:], states[self._ns:], **pr)
@@ -185,12 +184,12 @@ class MatrixLSTM:
 
     def __call__(self, h, batch, pools, states, carry=None):
         ops, H, d, dv = self.ops, self.H, self.dim, self.vdim
-        proj = linear(h, self.w_in)
+        proj = self.ops.linear(h, self.w_in)
         o_k, o_v, o_g, o_i = H * d, 2 * H * d, 2 * H * d + H * dv, 2 * H * d + 2 * H * dv
         a, b, m = ops.max_gates(proj, o_i, o_i + H, self.b_i, self.b_f, self.cap, states[1], batch, H)
         o = ops.recurrent_scan(proj[:, :o_k], proj[:, o_k:o_v], proj[:, o_v:o_g], a, None, states[0], batch, H, H, d, self.cols,
                                d ** -0.5, kscale=b, v_cols=dv)
-        return linear(ops.head_rms_gate(o, self.norm, proj[:, o_g:o_i], "sigmoid", self.eps, vdim=dv, den_m=m), self.w_o)
+        return self.ops.linear(ops.head_rms_gate(o, self.norm, proj[:, o_g:o_i], "sigmoid", self.eps, vdim=dv, den_m=m), self.w_o)
 
 
 class MinGRU:
@@ -210,5 +209,5 @@ class MinGRU:
 
     def __call__(self, h, batch, pools, states, carry=None):
         n = self.width
-        proj = linear(h, self.w_in)
-        return linear(self.ops.min_gru_scan(proj, 0, n, 2 * n, self.b_z, self.b_x, states[0], batch, n), self.w_o)
+        proj = self.ops.linear(h, self.w_in)
+        return self.ops.linear(self.ops.min_gru_scan(proj, 0, n, 2 * n, self.b_z, self.b_x, states[0], batch, n), self.w_o)

@@ -19,7 +19,6 @@ import math
 
 import torch
 
-from .ops import linear
 
 
 class RotatedValueAttention:
@@ -41,12 +40,12 @@ class RotatedValueAttention:
         ops, T, H, G = self.ops, h.size(0), self.H, self.G
         pool = pools[0]                                                    # [G, rows, vdim + dim]
         n = batch.max_pos + 1
-        proj = linear(h, self.w_in)
+        proj = self.ops.linear(h, self.w_in)
         qf = ops.attention_prep(proj, 0, H * self.dim, (H + G) * self.dim, H, G, self.dim, self.vdim, self.rot_n,
                                 self.rope_k.reserve(n), self.rope_v.reserve(n), self.scale, pool, batch)
         o = ops.latent_attention(qf, pool, batch, None, self.vdim, self.page, q_first=self.vdim)      # head h reads pool h // (H / G)
         ops.rotate_heads(o, self.rope_v.table, batch.pos, -1.0)
-        return linear(o.view(T, H * self.vdim), self.w_o)
+        return self.ops.linear(o.view(T, H * self.vdim), self.w_o)
 
 
 def distance_bucket(n, rows, far):
@@ -107,7 +106,7 @@ class NormedChunkAttention:
     def __call__(self, h, batch, pools, states, carry=None):
         ops, T, H, G = self.ops, h.size(0), self.H, self.G
         pool = pools[0]                                                    # [G, rows, vdim + dim]
-        proj = linear(h, self.w_in)
+        proj = self.ops.linear(h, self.w_in)
         o_k, o_v = H * self.dim, (H + G) * self.dim
         own = proj[:, o_v:o_v + G * self.vdim]
         v_first = None
@@ -120,7 +119,7 @@ class NormedChunkAttention:
         qf = ops.normed_attention_prep(proj, 0, o_k, o_v, H, G, self.dim, self.vdim, self.q_norm, self.k_norm, self.eps, self.scale,
                                        v_first, self.mix or 0.0, pool, batch)
         o = ops.latent_attention(qf, pool, batch, None, self.vdim, self.page, q_first=self.vdim, chunk=self.chunk, bias=self.bias)
-        return linear(o.view(T, H * self.vdim), self.w_o)
+        return self.ops.linear(o.view(T, H * self.vdim), self.w_o)
 
 
 class SinkWindowAttention:
@@ -195,7 +194,7 @@ class SinkWindowAttention:
 
     def __call__(self, h, batch, pools, states, carry=None):
         ops, T, H, G, d, dv = self.ops, h.size(0), self.H, self.G, self.dim, self.vdim
-        proj = linear(h, self.w_in)
+        proj = self.ops.linear(h, self.w_in)
         if self.taps and self.taps > 1:
             proj = ops.conv_silu_unit(proj, 0, self.conv, states[0], batch, 0, 1, act="none")          # float [T, C]
         elif self.taps:
@@ -214,7 +213,7 @@ class SinkWindowAttention:
             ops.pool_blocks(pool, pooled, batch, self.pool_block, self.page)
         o = ops.latent_attention(qf, pool, batch, self.window, dv, self.page, q_first=dv, keep_first=self.keep_first, sink=self.sink,
                                  slopes=self.slopes, pooled=pooled, pool_block=self.pool_block or 0)
-        return linear(o.view(T, H * dv), self.w_o)
+        return self.ops.linear(o.view(T, H * dv), self.w_o)
 
 
 def distance_slopes(heads):
@@ -257,14 +256,14 @@ class TalkingHeadsAttention:
         """proj: h's product with w_in, where the caller has it already (a column slice is fine)."""
         ops, H, G, d, pool = self.ops, self.H, self.G, self.dim, pools[0]
         if proj is None:
-            proj = linear(h, self.w_in)
+            proj = self.ops.linear(h, self.w_in)
         o_k, o_g = H * d, (H + G) * d
         k = proj[:, o_k:o_g]
         rope = self.rotary.reserve(batch.max_pos + 1) if self.rotary is not None else None
         qf = ops.qk_norm_rope_prep(proj[:, :o_k], k, k, H, G, d, d, self.q_norm, self.k_norm, True, self.eps, rope,
                                    self.rotary.dims if rope is not None else 0, self.scale, pool, batch, q_b=self.q_b, k_b=self.k_b,
                                    v_b=self.k_b, halves=True, head_scale=self.temp, q_pad=0)
-        return linear(ops.talking_attention(qf, pool, batch, self.talk, proj[:, o_g:o_g + H], d, self.page, cap=self.cap), self.w_o)
+        return self.ops.linear(ops.talking_attention(qf, pool, batch, self.talk, proj[:, o_g:o_g + H], d, self.page, cap=self.cap), self.w_o)
 
 
 class DifferentialAttention:
@@ -308,11 +307,11 @@ class DifferentialAttention:
 
     def __call__(self, h, batch, pools, states):
         ops, H, d, dv, pool = self.ops, self.H, self.dim, self.vdim, pools[0]
-        proj = linear(h, self.w_in)
+        proj = self.ops.linear(h, self.w_in)
         q = ops.conv_heads_cache(proj, self.conv, states[0] if self.taps > 1 else None, batch, 2 * H * d, 0 if self.shared_kv else self.G, 2 * d, dv,
                                  pool, self.scale, self.temperature)
         o = ops.diff_attention(q, pool, batch, H, d, dv, self.lam, self.out_scale, self.eps, proj[:, self.C:self.C + H * dv], self.page)
-        return linear(o, self.w_o)
+        return self.ops.linear(o, self.w_o)
 
 
 class TiedRotaryAttention:
@@ -336,7 +335,7 @@ class TiedRotaryAttention:
 
     def __call__(self, h, batch, pools, states):
         ops, T, H, G, d, pool, rot = self.ops, h.size(0), self.H, self.G, self.dim, pools[0], self.rotary
-        proj = linear(h, self.w_in)
+        proj = self.ops.linear(h, self.w_in)
         k = proj[:, H * d:]
         rope = rot.reserve(batch.max_pos + 1) if rot is not None else None
         plain = ops.maps_attention_ok(d, d, 1, self.page)        # queries in the storage type without the zeros in front
@@ -344,6 +343,6 @@ class TiedRotaryAttention:
                                   self.scale, pool, batch, halves=True, rot_gain=rot.magnitude ** 2 if rot is not None else 0.0,
                                   q_pad=0 if plain else d, q_store=plain)
         if plain:
-            return linear(ops.single_map_attention(q, pool, batch, H, d, d, self.page), self.w_o)
+            return self.ops.linear(ops.single_map_attention(q, pool, batch, H, d, d, self.page), self.w_o)
         o = ops.latent_attention(q, pool, batch, None, d, self.page, q_first=d)
-        return linear(o.view(T, H * d), self.w_o)
+        return self.ops.linear(o.view(T, H * d), self.w_o)

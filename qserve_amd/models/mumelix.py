@@ -17,7 +17,6 @@ layers: [{type, mixer: {...}, mlp: {kind: dense | moe, ...} | null}]}.
 import torch
 
 from ..layers.moe import GatedFeedForward, TopKGatedMoE
-from ..layers.ops import float_linear
 from ..layers.recurrent import GatedDeltaRule, GatedLinearAttention, ParallelMixer
 from ..layers.rotary import RotaryTable
 from ..layers.softmax_attention import RotatedValueAttention
@@ -151,4 +150,4 @@ class Mumelix:
         return x
 
     def logits(self, x, rows):
-        return float_linear(self.ops.dyt_sum_rows(x, rows, self.final_norm), self.head)
+        return self.ops.float_linear(self.ops.dyt_sum_rows(x, rows, self.final_norm), self.head)

@@ -14,7 +14,6 @@ l<i>.mix.left.{q, k, v, o, q.norm, k.norm, q.conv, k.conv, v.conv, sink, out} + 
 l<i>.mlp.{up, down} or l<i>.mlp.{router, correction, e<k>.{gate, up, down}}.
 """
 from ..layers.moe import IdentityExpertMoE, ReluSquaredFeedForward
-from ..layers.ops import float_linear
 from ..layers.recurrent import MinGRU, ParallelMixer
 from ..layers.rotary import RotaryTable
 from ..layers.softmax_attention import SinkWindowAttention
@@ -147,4 +146,4 @@ class Pemolorn:
         return x
 
     def logits(self, x, rows):
-        return float_linear(self.ops.rms_norm_rows(x, rows, self.final_norm, self.eps), self.head)
+        return self.ops.float_linear(self.ops.rms_norm_rows(x, rows, self.final_norm, self.eps), self.head)

@@ -12,7 +12,6 @@ Tensor names: embed, final.norm, l<i>.norm1 / ls1 / norm2 / ls2, l<i>.mix.{q, k,
 v and their convolutions with kv_from) or l<i>.mix.{q, k, o} (attention_2), l<i>.mlp.{router, e<k>.{gate, up, down}, shared.{gate, up, down}}.
 """
 from ..layers.moe import GatedFeedForward, SigmoidMoE
-from ..layers.ops import float_linear
 from ..layers.rotary import RotaryTable
 from ..layers.softmax_attention import DifferentialAttention, TiedRotaryAttention
 from ..serving.registry import register_model
@@ -137,4 +136,4 @@ class Rivolix:
         return x
 
     def logits(self, x, rows):
-        return float_linear(self.ops.rms_norm_rows(x, rows, self.final_gain, self.eps), self.embed)
+        return self.ops.float_linear(self.ops.rms_norm_rows(x, rows, self.final_gain, self.eps), self.embed)

@@ -16,7 +16,6 @@ k.conv, v.conv, b, A_log, norm, a, dt_bias, g, o, out} (parallel), l<i>.mlp.{gat
 import torch
 
 from ..layers.moe import GatedFeedForward
-from ..layers.ops import float_linear
 from ..layers.recurrent import GatedDeltaRule, ParallelMixer, Retention
 from ..layers.rotary import RotaryTable
 from ..layers.softmax_attention import SinkWindowAttention, TalkingHeadsAttention, distance_slopes
@@ -142,4 +141,4 @@ class Sagupel:
         return x
 
     def logits(self, x, rows):
-        return float_linear(self.ops.rms_norm_rows(x, rows, self.final_norm, self.eps), self.embed)
+        return self.ops.float_linear(self.ops.rms_norm_rows(x, rows, self.final_norm, self.eps), self.embed)

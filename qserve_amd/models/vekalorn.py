@@ -14,7 +14,6 @@ import torch
 
 from ..layers.latent_attention import LatentAttention
 from ..layers.moe import GroupedTopKMoE
-from ..layers.ops import float_linear
 from ..layers.rotary import RotaryTable
 from ..serving.registry import register_model
 
@@ -103,4 +102,4 @@ class Vekalorn:
         return x
 
     def logits(self, x, rows):
-        return float_linear(self.ops.layer_norm_rows(x, rows, self.final_norm, self.eps), self.head)
+        return self.ops.float_linear(self.ops.layer_norm_rows(x, rows, self.final_norm, self.eps), self.head)

@@ -14,7 +14,6 @@ norm, i, i.b, f, f.b}, l<i>.mlp.{gate, up, down} or l<i>.mlp.{router, correction
 import torch
 
 from ..layers.moe import CorrectedSigmoidMoE, GatedFeedForward
-from ..layers.ops import float_linear
 from ..layers.recurrent import MatrixLSTM
 from ..layers.softmax_attention import NormedChunkAttention
 from ..serving.registry import register_model
@@ -116,4 +115,4 @@ class Vepolix:
         return x
 
     def logits(self, x, rows):
-        return float_linear(self.ops.rms_norm_rows(x, rows, self.final_norm, self.eps), self.head)
+        return self.ops.float_linear(self.ops.rms_norm_rows(x, rows, self.final_norm, self.eps), self.head)

@@ -14,6 +14,7 @@ SIGNATURES = {
     "qsv_last_error": (C.c_char_p, []),
     "qsv_skinny_linear": (_i, [_vp, _vp, _i64, _vp, _i, _i, _i, _vp]),
     "qsv_skinny_linear_widened": (_i, [_vp, _vp, _i64, _vp, _i, _i, _i, _vp]),
+    "qsv_skinny_linear_kept": (_i, [_vp, _i, _vp, _i64, _vp, _i, _i, _i, _vp]),
     "qsv_decay_products": (_i, [_vp, _vp, _i64, _vp, _i, _i, _vp, _vp, _f, _i, _vp, _vp, _i64, _vp, _i, _i, _i, _vp]),
     "qsv_head_product_gated": (_i, [_vp, _vp, _i64, _i64, _vp, _i, _i, _i, _i, _vp, _i64, _vp]),
     "qsv_head_product": (_i, [_vp, _vp, _i64, _i64, _vp, _i, _i, _i, _i, _vp]),
@@ -65,6 +66,7 @@ SIGNATURES = {
     "qsv_expert_rows": (_i, [_vp, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _i, _f, _vp, _vp]),
     "qsv_expert_slots": (_i, [_vp, _i, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _f, _vp, _vp]),
     "qsv_expert_slots_shared": (_i, [_vp, _i, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _f, _vp, _vp, _vp, _vp, _i, _i, _i, _vp]),
+    "qsv_expert_slots_kept": (_i, [_vp, _i, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _f, _vp, _vp, _vp, _vp, _i, _i, _i, _vp]),
     "qsv_moe_sort": (_i, [_vp, _vp, _vp, _vp, _i, _i, _vp]),
     "qsv_grouped_gemm_sorted_ok": (_i, [_i, _i, _i]),
     "qsv_grouped_gemm_sorted": (_i, [_vp, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _i, _f, _vp, _vp]),

@@ -76,31 +76,25 @@ def random_weights(cfg, dev, seed=0):
 
 
 class OpTimer:
-    """HIP events around every call of the ops object's methods and of the vendor products (one step at a time)."""
+    """HIP events around every call of the ops object's methods (one step at a time)."""
     NAMES = ("embed", "add_layer_norm", "layer_norm_rows", "latent_prep", "latent_queries", "latent_prompt", "head_products", "latent_attention", "sigmoid_gate",
              "moe_route", "moe_experts", "moe_experts_shared", "embed_streams", "hc_read", "hc_write", "dyt_sum_rows", "rms_pair_mean", "glu",
              "attention_prep", "rotate_heads", "decay", "decay_products", "conv_silu_unit", "recurrent_scan", "head_rms_gate", "embed_sinusoid",
              "add_rms_norm", "rms_norm_rows", "normed_attention_prep", "max_gates", "add_normed_rms_norm", "qk_norm_rope_prep", "pool_blocks",
              "min_gru_scan", "relu_sq", "embed_rms_norm", "residual_conv", "scaled_add_rms_norm", "rotate_qk", "talking_attention",
-             "scaled_sum_rms_norms", "conv_heads_cache", "diff_attention", "single_map_attention")
+             "scaled_sum_rms_norms", "conv_heads_cache", "diff_attention", "single_map_attention", "linear", "float_linear")
     # another form of the same operation: its time is that operation's
-    FORMS = {"latent_prompt": "latent_attention", "moe_experts_shared": "moe_experts"}
+    FORMS = {"latent_prompt": "latent_attention", "moe_experts_shared": "moe_experts", "float_linear": "linear"}
 
     def __init__(self, ops):
         self.ops, self.events, self.calls, self.on = ops, [], [], False
         for n in self.NAMES:
             setattr(ops, n, self._wrap(self.FORMS.get(n, n), getattr(ops, n)))
-        from ..layers import ops as ops_module                # the vendor products, as the layers call them
-        for mod in self._linear_users():
-            name = "linear" if hasattr(mod, "linear") else "float_linear"
-            setattr(mod, name, self._wrap("linear", getattr(ops_module, name)))
 
     @staticmethod
     def _linear_users():
-        import importlib
-        return [importlib.import_module("qserve_amd." + m) for m in
-                ("layers.latent_attention", "layers.moe", "layers.recurrent", "layers.softmax_attention", "models.vekalorn",
-                 "models.mumelix", "models.vepolix", "models.pemolorn", "models.sagupel", "models.rivolix")]
+        """Modules whose products are not the ops object's: none (layers and models call its `linear` and `float_linear`)."""
+        return []
 
     def _wrap(self, name, fn):
         def timed(*a, **k):

@@ -17,7 +17,16 @@ from .cache import PagedCache, upload
 from .sampler import SamplingParams, sample
 from .scheduler import Request, Scheduler
 
+# Weights that the last cache (256 MB) holds from step to step beside the rest; kernels then leave them there in steps of more than 24 rows (streams_once
+# in csrc/serve/serve_stream.h has both sides' times)
+KEPT_WEIGHTS = 200_000_000
 DTYPES = {"bfloat16": torch.bfloat16, "float32": torch.float32}
+
+
+def kept_above(weights, dtype):
+    """HipOps.kept_above for a model of these checkpoint tensors (a step reads a few rows of an embedding that is not the head too)."""
+    read = sum(w.numel() for n, w in weights.items() if isinstance(w, torch.Tensor) and not (n == "embed" and "head" in weights))
+    return 24 if read * dtype.itemsize <= KEPT_WEIGHTS else None
 
 
 @dataclass
@@ -109,6 +118,7 @@ class Engine:
             torch.backends.cuda.matmul.allow_tf32 = False          # float32 means float32 products
             torch.backends.cudnn.allow_tf32 = False
         self.ops = make_ops(backend, self.dtype, self.device)
+        self.ops.kept_above = kept_above(weights, self.dtype)
         self.model = model_cls.from_config(config, weights, self.ops, self.device, self.dtype, page=page)
         self.cache = PagedCache(self.model.cache_rows, (int(max_tokens) + page - 1) // page, max_seqs, self.dtype, self.device,
                                 page=page, states=getattr(self.model, "state_specs", ()))

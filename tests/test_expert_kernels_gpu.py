@@ -347,3 +347,23 @@ def test_routing_apart_where_the_rows_do_not_take_it(ops):
     route = dict(top_k=2, groups=1, keep=1, router=t(8, 64))
     then = (torch.zeros(5, device="cuda:0"), (t(64), t(64), 1.0))
     assert ops.hc_write(torch.zeros(2, 5, 64, device="cuda:0"), t(2, 64), torch.zeros(5, 5, device="cuda:0"), torch.zeros(5, device="cuda:0"), then_read=then, route=route)[1] is None
+
+
+# weights left in the caches: the same products from the same launches, only how the weights are asked for differs
+@pytest.mark.parametrize("T", [1, 16, 17, 33, 64])
+@pytest.mark.parametrize("D, ff, sff", [(256, 128, 64), (2048, 384, 1408), (72, 136, 200)])
+def test_weights_kept_in_the_caches(ops, T, D, ff, sff):
+    from qserve_amd.layers.ops import float_linear
+    kept, g, E, top = make_ops("hip", torch.bfloat16, torch.device("cuda:0")), torch.Generator().manual_seed(T + D), 5, 3
+    mat = lambda *s: (torch.randn(*s, generator=g) / s[-1] ** 0.5).bfloat16().cuda()                       # noqa: E731
+    h, up, down, sup, sdown = mat(T, D), mat(E, 2 * ff, D), mat(E, D, ff), mat(2 * sff, D), mat(D, sff)
+    idx, wt = torch.rand(T, E, generator=g).argsort(1)[:, :top].int().cuda(), torch.rand(T, top, generator=g).cuda()
+    idx[0, 0] = -1
+    assert kept.kept_above is None and not kept._kept(64)
+    kept.kept_above = 0
+    assert torch.equal(kept.linear(h, sup), linear(h, sup)) and torch.equal(kept.float_linear(h, sup), float_linear(h, sup))
+    for act, u in (("swiglu", up), ("relu_sq", up[:, :ff].contiguous())):
+        for weigh in ("input", "output"):
+            assert torch.equal(kept.moe_experts(h, u, down, idx, wt, act=act, weigh=weigh), ops.moe_experts(h, u, down, idx, wt, act=act, weigh=weigh))
+    a, b = (o.moe_experts_shared(h, up, down, idx, wt, sup, sdown) for o in (kept, ops))
+    assert (a is None) == (b is None) and (a is None or all(torch.equal(x, y) for x, y in zip(a, b)))

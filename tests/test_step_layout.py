@@ -180,3 +180,11 @@ def test_when_new_places_of_the_table_travel_with_a_launch(monkeypatch, entries,
     e.cache._entered = dict.fromkeys(range(entries), 1)
     e.cache.table = type("T", (), {"is_cuda": True, "numel": lambda self: size, "device": torch.device("cuda", index)})()
     assert e.cache._new_by_kernel() == taken
+
+
+@pytest.mark.parametrize("sizes, dtype, kept", [(dict(a=10 ** 8), torch.bfloat16, 24), (dict(a=10 ** 8, b=1), torch.bfloat16, None), (dict(a=5 * 10 ** 7), torch.float32, 24),
+                                                (dict(a=5 * 10 ** 7 + 1), torch.float32, None), (dict(embed=10 ** 8, head=10 ** 8), torch.bfloat16, 24),
+                                                (dict(embed=10 ** 8, a=1), torch.bfloat16, None), ({}, torch.bfloat16, 24)])
+def test_weights_that_the_caches_hold(sizes, dtype, kept):
+    from qserve_amd.serving.engine import kept_above
+    assert kept_above({n: torch.empty(s, device="meta") for n, s in sizes.items()} | {"scale": 0.5}, dtype) == kept

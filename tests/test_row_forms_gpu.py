@@ -163,3 +163,28 @@ def test_block_table_on_the_device_is_the_hosts():
             slots[1] = cache.admit()
             cache.extend(slots[1], 17)
         assert torch.equal(cache.block_table().cpu(), cache.table_host)
+
+
+def close(got, ref, size, dtype):
+    """Within half a unit of the storage type's last place (or a rounding that falls the other way) and float sums whose terms are of `size`."""
+    return ((got.double() - ref).abs() <= (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -22) * ref.abs() + 2.0 ** -19 * size).all()
+
+
+# one wave and two, groups of 1024 columns, rows in one trip and in two; parts with and without a scale, the rows of a table, no norm, one and two
+@TYPES
+@pytest.mark.parametrize("D", [4, 256, 260, 512, 516, 1024, 2052, 3072, 3076, 4100, 5120, 6144, 6148, 8192, 8196])
+@pytest.mark.parametrize("parts, norms, table", [(0, 2, True), (1, 1, False), (2, 2, False), (3, 2, False), (3, 0, True)])
+def test_scaled_sums(dtype, D, parts, norms, table):
+    ops, g, T = make(dtype), torch.Generator().manual_seed(D + parts), 5
+    rnd = lambda *s: torch.randn(*s, generator=g).to(dtype).to(DEV)                                        # noqa: E731
+    x, rows, tokens = torch.randn(T, D, generator=g).to(DEV), rnd(9, D), ints([3, 0, 8, 8, 1])
+    ps = [(rnd(T, D), None if j == 1 else rnd(D)) for j in range(parts)]
+    gains = [torch.randn(D, generator=g).to(DEV) for _ in range(norms)]
+    start = rows[tokens.long()].double() if table else x.double()
+    terms = [y.double() * (1.0 if f is None else f.double()) for y, f in ps]
+    ref = start + sum(terms)
+    size = start.abs() + sum(t.abs() for t in terms)
+    got, hs = ops.scaled_sum_rms_norms(x, ps, gains, 1e-5, **(dict(tokens=tokens, table=rows) if table else {}))
+    assert len(hs) == norms and close(got, ref, size, torch.float32)
+    inv = 1.0 / (ref.pow(2).mean(-1, keepdim=True) + 1e-5).sqrt()
+    assert all(close(h, ref * inv * w.double(), size * inv * w.double().abs(), dtype) for h, w in zip(hs, gains))

@@ -1136,7 +1136,7 @@ extern "C" int qsv_add_normed_rms_norm(float* x, void* h, const void* y, const v
 // on normed values staged in LDS (a pair's two values may sit in different threads).  Dynamic LDS: (heads + kv_heads) * dim floats.
 // VEC (every size, stride and address a multiple of four elements, dim <= 256): four elements per lane, dim / 4 lanes (rounded up to a
 // power of two, `lph`) per head for the per-head statistics, 16-byte stores.
-template <typename T, typename TI, bool VEC>
+template <typename T, typename TI, bool VEC, int ROUNDS>
 __global__ __launch_bounds__(NT) void qk_norm_rope_prep_kernel(float* __restrict__ qf, const TI* __restrict__ q, int64_t q_stride,
                                                                const TI* __restrict__ k, int64_t k_stride, const TI* __restrict__ v,
                                                                int64_t v_stride, int H, int G, int dim, int vdim,
@@ -1157,7 +1157,7 @@ __global__ __launch_bounds__(NT) void qk_norm_rope_prep_kernel(float* __restrict
     const TI* qrow = q + t * q_stride;
     const TI* krow = k ? k + t * k_stride : nullptr;
     // (the first pair's turn is requested with the row)
-    const int half = rot_n / 2, i_first = rope ? (int)threadIdx.x % half : 0;
+    const int half = rot_n / 2, i_first = !rope ? 0 : half & (half - 1) ? (int)threadIdx.x % half : (int)threadIdx.x & (half - 1);
     const float* cs = rope ? rope + (size_t)pos[t] * rot_n : nullptr;
     float c_first = 0.f, s_first = 0.f;
     if (rope) {
@@ -1166,23 +1166,23 @@ __global__ __launch_bounds__(NT) void qk_norm_rope_prep_kernel(float* __restrict
     }
     if (VEC && per_head) {
         const int e = (lane & (lph - 1)) * 4;
-        // (a wave stays together: its lanes exchange sums; up to four of its rounds of heads in one trip to memory)
+        // (a wave stays together: its lanes exchange sums; ROUNDS of its rounds of heads in one trip to memory)
         const int step = NT / lph, at = min(e, dim - 4);
         typename Raw4<T>::type rqw, rkw;
         if (q_w) {
             rqw = raw4(q_w, at);
             rkw = raw4(k ? k_w : q_w, at);
         }
-        for (int b0 = threadIdx.x / lph; b0 - lane / lph < NH; b0 += 4 * step) {
-            typename Raw4<TI>::type ru[4];
+        for (int b0 = threadIdx.x / lph; b0 - lane / lph < NH; b0 += ROUNDS * step) {
+            typename Raw4<TI>::type ru[ROUNDS];
 #pragma unroll
-            for (int x = 0; x < 4; ++x) {
+            for (int x = 0; x < ROUNDS; ++x) {
                 const int h0 = min(b0 + x * step, NH - 1);
                 ru[x] = raw4(h0 < H ? qrow : krow, (size_t)(h0 < H ? h0 : h0 - H) * dim + at);
             }
             requested();
 #pragma unroll
-            for (int x = 0; x < 4; ++x) {
+            for (int x = 0; x < ROUNDS; ++x) {
                 const int h0 = b0 + x * step;
                 if (h0 - lane / lph >= NH) continue;                                        // (the whole wave)
                 const bool ok = h0 < NH && e < dim, isq = h0 < H;
@@ -1343,19 +1343,29 @@ extern "C" int qsv_qk_norm_rope_prep(void* qf, const void* q, int64_t q_stride, 
                      (!k || (k_stride % 4 == 0 && v_stride % 4 == 0 && al(k, el) && al(v, el) && al(k_w, es) && al(k_b, es) && al(v_b, es) && al(pool, es)));
     int lph = 1;
     while (lph * 4 < dim) lph <<= 1;
-#define QSV_QKP(TI, VEC)                                                                                                         \
+#define QSV_QKP(TI, VEC, RO)                                                                                                     \
     QSV_DISPATCH(dtype, "qsv_qk_norm_rope_prep",                                                                                 \
-                 hipLaunchKernelGGL((qk_norm_rope_prep_kernel<T, TI, VEC>), dim3(n), dim3(NT), lds, (hipStream_t)stream, q_store ? nullptr : (float*)qf, (const TI*)q, \
+                 hipLaunchKernelGGL((qk_norm_rope_prep_kernel<T, TI, VEC, RO>), dim3(n), dim3(NT), lds, (hipStream_t)stream, q_store ? nullptr : (float*)qf, (const TI*)q, \
                                     q_stride, (const TI*)k, k_stride, (const TI*)v, v_stride, heads, kv_heads, dim, vdim,          \
                                     (const T*)q_w, (const T*)k_w, per_head, eps, rope, rot_n, scale, (T*)pool, pool_rows, slot, pos,  \
                                     (const T*)q_b, (const T*)k_b, (const T*)v_b, halves, head_scale, q_pad, lph, rot_gain,              \
                                     q_store ? (T*)qf : nullptr))
     if (vec) {
-        if (qkv_dtype == QSV_F32) QSV_QKP(float, true);
-        else QSV_QKP(bf16_t, true);
+        // (rounds of heads in a trip: no more than there are, those behind the last head would be requested all the same: 4 + 4 heads of 64, 2048 tokens,
+        // one / four 7.7 / 8.1 us)
+        const int step = NT / lph, all = k ? heads + kv_heads : heads;
+        if (qkv_dtype == QSV_F32) {
+            if (!per_head || all <= step) QSV_QKP(float, true, 1);
+            else if (all <= 2 * step) QSV_QKP(float, true, 2);
+            else QSV_QKP(float, true, 4);
+        } else {
+            if (!per_head || all <= step) QSV_QKP(bf16_t, true, 1);
+            else if (all <= 2 * step) QSV_QKP(bf16_t, true, 2);
+            else QSV_QKP(bf16_t, true, 4);
+        }
     } else {
-        if (qkv_dtype == QSV_F32) QSV_QKP(float, false);
-        else QSV_QKP(bf16_t, false);
+        if (qkv_dtype == QSV_F32) QSV_QKP(float, false, 1);
+        else QSV_QKP(bf16_t, false, 1);
     }
 #undef QSV_QKP
     return qsv_launch_status("qsv_qk_norm_rope_prep");

@@ -188,3 +188,37 @@ def test_scaled_sums(dtype, D, parts, norms, table):
     assert len(hs) == norms and close(got, ref, size, torch.float32)
     inv = 1.0 / (ref.pow(2).mean(-1, keepdim=True) + 1e-5).sqrt()
     assert all(close(h, ref * inv * w.double(), size * inv * w.double().abs(), dtype) for h, w in zip(hs, gains))
+
+
+# heads in one round of the workgroup, two, four and more; a head's lanes a power of two and not
+@TYPES
+@pytest.mark.parametrize("dim", [8, 40, 64, 128, 256])
+@pytest.mark.parametrize("extra", [0, 1])
+@pytest.mark.parametrize("rounds", [1, 2, 4])
+def test_head_norms_by_rounds(dtype, dim, extra, rounds):
+    ops, g, T = make(dtype), torch.Generator().manual_seed(dim + rounds), 3
+    lanes = 1
+    while lanes * 4 < dim:
+        lanes *= 2
+    G = 2
+    H = rounds * (256 // lanes) + extra - G
+    if (H + G) * dim * 4 > 64 * 1024:
+        pytest.skip("more heads than the launch takes")
+    rnd = lambda *s: torch.randn(*s, generator=g).to(dtype).to(DEV)                                        # noqa: E731
+    q, k, v, qw, kw = rnd(T, H * dim), rnd(T, G * dim), rnd(T, G * dim), rnd(dim), rnd(dim)
+    rot = dim // 8 * 8 - (4 if dim == 40 else 0)
+    rope, pos = torch.randn(T + 2, 2, rot // 2, generator=g).to(DEV), [4, 0, 2]
+    batch = StepBatch(tokens=None, seq=None, pos=ints(pos), slot=torch.tensor([2, 0, 1], device=DEV), block_table=None, max_pos=4, n_tokens=T, items=[(i, i, 1) for i in range(T)])
+    pool = torch.zeros(G, T, 2 * dim, dtype=dtype, device=DEV)
+    qf = ops.qk_norm_rope_prep(q, k, v, H, G, dim, dim, qw, kw, True, 1e-5, rope, rot, 0.5, pool, batch, q_pad=0)
+
+    def ref(u, w):
+        u = u.double().view(T, -1, dim)
+        n = u / (u.pow(2).mean(-1, keepdim=True) + 1e-5).sqrt() * w.double()
+        c, s = (rope[pos, i].double()[:, None] for i in (0, 1))
+        a, b = n[..., 0:rot:2].clone(), n[..., 1:rot:2].clone()
+        n[..., 0:rot:2], n[..., 1:rot:2] = a * c - b * s, b * c + a * s
+        return n
+    assert close(qf, ref(q, qw) * 0.5, 16.0, torch.float32)
+    rows = pool[:, [2, 0, 1]].transpose(0, 1)
+    assert torch.equal(rows[..., :dim], v.view(T, G, dim)) and close(rows[..., dim:], ref(k, kw), 16.0, dtype)

@@ -222,3 +222,14 @@ def test_head_norms_by_rounds(dtype, dim, extra, rounds):
     assert close(qf, ref(q, qw) * 0.5, 16.0, torch.float32)
     rows = pool[:, [2, 0, 1]].transpose(0, 1)
     assert torch.equal(rows[..., :dim], v.view(T, G, dim)) and close(rows[..., dim:], ref(k, kw), 16.0, dtype)
+
+
+@TYPES
+@pytest.mark.parametrize("T", [128, 129, 1023, 1024])
+@pytest.mark.parametrize("S, D", [(1, 4), (2, 1028), (3, 64), (4, 1024)])
+def test_streams_read_by_number_of_rows(dtype, T, S, D):
+    ops, g = make(dtype), torch.Generator().manual_seed(T + D)
+    x, w_in = torch.randn(T, S, D, generator=g).to(DEV), torch.randn(S, generator=g).to(DEV)
+    w, b = (torch.randn(D, generator=g).to(dtype).to(DEV) for _ in range(2))
+    ref = torch.tanh(0.6 * torch.einsum("s,tsd->td", w_in.double(), x.double())) * w.double() + b.double()
+    assert close(ops.hc_read(x, w_in, (w, b, 0.6)), ref, 16.0, dtype)

@@ -1010,7 +1010,8 @@ extern "C" int qsv_decay(float* out, const void* z, int64_t z_stride, const void
     if (n_tokens == 0) return QSV_OK;
     const int width = heads * dim;
     const int64_t chunks = ((int64_t)width / 4 + NT - 1) / NT;
-    if (width % 4 == 0 && z_stride % 4 == 0 && fits4(out, QSV_F32) && fits4(z, dtype) && fits4(bias, dtype) && chunks * n_tokens < (1ll << 31)) {
+    // (below 1024 channels the general kernel has a thread for each, and a thread's four would come one after another: 256 channels, 1 - 512 tokens 3.3 against 4.3 us)
+    if (width >= 4 * NT && width % 4 == 0 && z_stride % 4 == 0 && fits4(out, QSV_F32) && fits4(z, dtype) && fits4(bias, dtype) && chunks * n_tokens < (1ll << 31)) {
         QSV_DISPATCH(dtype, "qsv_decay",
                      hipLaunchKernelGGL(decay_vec_kernel<T>, dim3((unsigned)(chunks * n_tokens)), dim3(NT), 0, (hipStream_t)stream, out, (const T*)z, z_stride,
                                         (const T*)bias, a_log, a_log ? 0.f : 1.0f / tau, dim, width, (int)chunks));

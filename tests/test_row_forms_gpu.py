@@ -233,3 +233,20 @@ def test_streams_read_by_number_of_rows(dtype, T, S, D):
     w, b = (torch.randn(D, generator=g).to(dtype).to(DEV) for _ in range(2))
     ref = torch.tanh(0.6 * torch.einsum("s,tsd->td", w_in.double(), x.double())) * w.double() + b.double()
     assert close(ops.hc_read(x, w_in, (w, b, 0.6)), ref, 16.0, dtype)
+
+
+# below 1024 channels one a thread, from there four
+@TYPES
+@pytest.mark.parametrize("H, dim", [(1, 4), (2, 128), (255, 4), (256, 4), (257, 4), (3, 341)])
+@pytest.mark.parametrize("log", [False, True])
+def test_decay_by_width(dtype, H, dim, log):
+    ops, g, T = make(dtype), torch.Generator().manual_seed(H * dim), 17
+    z, b = torch.randn(T, H * dim + 4, generator=g).to(dtype).to(DEV)[:, 4:], torch.randn(H * dim, generator=g).to(dtype).to(DEV)
+    a = torch.randn(H, generator=g).to(DEV) if log else None
+    u = z.double() + b.double()
+    if log:
+        power = -a.double().exp().repeat_interleave(dim) * torch.nn.functional.softplus(u)
+    else:
+        power = -torch.nn.functional.softplus(-u) / 16.0
+    # a power of e that carries some units of 2^-24 of itself, exponentials of a few more
+    assert ((ops.decay(z, b, a, 16.0, H, dim).double() - power.exp()).abs() <= 2.0 ** -20 * (1.0 + power.abs()) * power.exp() + 1e-30).all()

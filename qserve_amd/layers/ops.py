@@ -513,7 +513,9 @@ class HipOps:
                                                  b.data_ptr(), float(alpha), *q[2]), "hc_write_route")
             return h, q[:2]
         if isinstance(y, ExpertRows):                                   # (the same bits as y.dense() gives)
-            if then_read is None and D % 4 == 0 and _on_four(x):
+            # More than four slots are summed in two rounds of requests, which a large prompt's streams wait for; 2 streams, summed here / apart, us: 8192 tokens
+            # of 2048, top 4 / 5 / 8 62 / 80, 122 / 96, 146 / 121, 4096 of 4096 62 / 86, 128 / 97, 164 / 135, 2048 of 3072, top 5 / 8 40 / 34, 43 / 40; below, here: 1024 of 3072 21 / 21, 23 / 23, 2048 of 1024 16 / 17, 18 / 18
+            if then_read is None and D % 4 == 0 and _on_four(x) and not (y.place is not None and y.idx.size(1) > 4 and T * D >= 1 << 22):
                 self._need(x, y.ys, y.idx, w_mix, w_out)
                 assert y.shape == (T, D) and w_mix.dtype == torch.float32 and w_mix.shape == (S, S)
                 self.check(self.L.qsv_hc_write_slots(x.data_ptr(), *y.args(), w_mix.data_ptr(), w_out.data_ptr(), T, S, D, self.code, self._s()), "hc_write_slots")

@@ -184,6 +184,50 @@ def test_sums_over_experts_inside_their_users(ops, T, top, D, ff, weigh):
     assert near(xd, ref, y.abs()[:, None] * out.abs()[None, :, None] + 4)
 
 
+# ... to the bit what the sum as a tensor gives: slots without an expert, sums in one and two rounds of requests, streams that take the tensor
+# (more than four placed slots, 2^22 elements and more) and the last that do not
+@pytest.mark.parametrize("placed", [False, True])
+@pytest.mark.parametrize("weighed", [False, True])
+@pytest.mark.parametrize("T, top, D", [(1, 1, 4), (5, 4, 256), (3, 5, 516), (17, 8, 1028), (2, 9, 3076), (33, 6, 4096), (1024, 5, 4096), (1023, 5, 4096), (1024, 4, 4096)])
+def test_sums_inside_their_users_have_the_tensors_bits(ops, T, top, D, placed, weighed):
+    g, dev, E = torch.Generator().manual_seed(T + D + top), "cuda:0", 6
+    bf = lambda *s: torch.randn(*s, generator=g).bfloat16().to(dev)                                        # noqa: E731
+    fl = lambda *s: torch.randn(*s, generator=g).to(dev)                                                   # noqa: E731
+    idx = torch.randint(-1, E, (T, top), generator=g, dtype=torch.int32).to(dev)
+    place = torch.randperm(T * top, generator=g).int().to(dev) if placed else None
+    wt, ys, h = fl(T, top) if weighed else None, bf(T * top, D) if placed else fl(T * top, D), bf(T, D)
+    rows = ExpertRows(ops, ys, place, wt, idx, h, E)
+    y = rows.dense()
+    at = torch.arange(T * top, device=dev) if place is None else place.long()
+    terms = ys[at].view(T, top, D).double() * (idx >= 0)[..., None] * (1.0 if wt is None else wt.double()[..., None])
+    ref, size = terms.sum(1), terms.abs().sum(1)
+    # half a unit in the last of bfloat16's 8 digits (or a rounding that falls the other way), a float sum of `top` products
+    assert ((y.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + (top + 1) * 2.0 ** -24 * size).all()
+    del terms, ref
+    x, a, c, w, f = fl(T, D), bf(T, D), bf(T, D), bf(D), [bf(D) for _ in range(3)]
+    x1, x2 = x.clone(), x.clone()
+    assert torch.equal(ops.add_layer_norm(x1, rows, w, 1e-5), ops.add_layer_norm(x2, y, w, 1e-5)) and torch.equal(x1, x2)
+    for parts in ([(a, f[0]), (y, f[1]), (c, f[2])], [(a, None), (y, None)]):
+        x1, x2, gains = x.clone(), x.clone(), [fl(D), fl(D)]
+        _, h1 = ops.scaled_sum_rms_norms(x1, [(rows if p is y else p, v) for p, v in parts], gains, 1e-5)
+        _, h2 = ops.scaled_sum_rms_norms(x2, parts, gains, 1e-5)
+        assert torch.equal(x1, x2) and all(map(torch.equal, h1, h2))
+        ref, size = x.double(), x.double().abs()
+        for p, v in parts:
+            t = p.double() * (1.0 if v is None else v.double())
+            ref, size = ref + t, size + t.abs()
+        assert ((x1.double() - ref).abs() <= 2.0 ** -22 * size).all()
+    for S in (2, 5):
+        s1, mix, out = fl(T, S, D), fl(S, S), fl(S)
+        s2, s0 = s1.clone(), s1.double()
+        ops.hc_write(s1, rows, mix, out)
+        ops.hc_write(s2, y, mix, out)
+        assert torch.equal(s1, s2)
+        ref = s0.transpose(1, 2) @ mix.double() + y.double()[..., None] * out.double()
+        size = s0.abs().transpose(1, 2) @ mix.abs().double() + y.abs().double()[..., None] * out.abs().double()
+        assert ((s1.double() - ref.transpose(1, 2)).abs() <= (S + 2) * 2.0 ** -24 * size.transpose(1, 2)).all()
+
+
 @pytest.mark.parametrize("T, top, D, ff", [(3, 2, 64, 64), (40, 4, 72, 40), (1200, 2, 64, 128)])
 @pytest.mark.parametrize("knobs", [{}, dict(moe_token_slots=10 ** 9, moe_sorted_above=10 ** 9)], ids=["rule", "per token"])
 def test_slots_without_an_expert_add_nothing(T, top, D, ff, knobs):

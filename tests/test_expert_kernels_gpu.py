@@ -104,8 +104,8 @@ def test_grouped_form(ops, T, top, E, ident, D, ff, crowd, act, weigh):
     check(o, T, top, E, ident, D, ff, act, weigh, crowd)
 
 
-# one step; runs of steps around the two that are requested ahead and the six from which a tile's rows come through LDS; rows in and out of 16; empty, full
-# and nearly empty tiles; the gather through slot / div and rows as they lie; experts on both sides of the room for staged rows
+# a tile a workgroup at most: one step and runs of steps around the two that are requested ahead; rows in and out of 16; empty, full and nearly empty tiles; the
+# gather through slot / div and rows as they lie
 @pytest.mark.parametrize("K", [64, 128, 192, 320, 384, 448])
 @pytest.mark.parametrize("N, E, div", [(4, 14, 1), (132, 14, 3), (260, 14, 0), (528, 14, 2), (128, 7679, 1), (272, 7680, 1)])
 def test_grouped_products_of_sorted_runs(ops, K, N, E, div):
@@ -133,6 +133,56 @@ def test_grouped_products_of_sorted_runs(ops, K, N, E, div):
             assert ((y[at:at + c].double() - ref).abs() <= 2.0 ** -8 * ref.abs() + K * 2.0 ** -22).all(), (e, c)
         at += c
     assert (y[n] == 3.0).all()
+
+
+# ... and workgroups that take a second and a third tile: an odd and an even number of steps (the half of the buffer that a tile starts in), input rows of the
+# next tile through LDS (from six steps on, up to 7679 experts) and not, stores of 16 and of 8 bytes, rows folded in pairs; the callers' own tiles, whose gather is of 64-bit numbers
+@pytest.mark.parametrize("K", [64, 192, 320, 384, 448, 1088])
+@pytest.mark.parametrize("N, E, div, act, times, listed", [(8192, 14, 3, 0, 1, False), (12300, 14, 1, 0, 1, False), (8192, 14, 2, 2, 1, False), (5120, 14, 0, 1, 1, False),
+                                                           (272, 7679, 2, 0, 20, False), (272, 7680, 2, 0, 20, False), (8192, 14, 3, 0, 1, True), (5120, 14, 0, 2, 1, True)])
+def test_grouped_products_of_many_tiles(ops, K, N, E, div, act, times, listed):
+    gen, dev = torch.Generator(device="cuda:0").manual_seed(K + N), "cuda:0"
+    counts = [times * c for c in (0, 1, 63, 64, 65, 0, 127, 128, 129, 255, 256, 257, 600, 0)]
+    n, names = sum(counts), list(range(7)) + list(range(E - 7, E))
+    first = [sum(counts[:i]) for i in range(14)]
+    order = torch.randperm(n, generator=gen, device=dev) if div else torch.arange(n, device=dev)
+    x = torch.randn(-(-n // max(div, 1)), K, generator=gen, device=dev).bfloat16()
+    w = torch.empty(E, N, K, dtype=torch.bfloat16, device=dev)          # (empty experts' weights are never read)
+    for e, c in zip(names, counts):
+        if c:
+            w[e] = torch.randn(N, K, generator=gen, device=dev) / K ** 0.5
+    wide, s = N // 2 if act == 2 else N, torch.cuda.current_stream().cuda_stream
+    out = torch.full((n + 1, wide), 3.0, dtype=torch.bfloat16, device=dev)
+    if listed:
+        size = ops.L.qsv_grouped_gemm_tile_slots()
+        tiles = [(e, f + o, min(size, c - o)) for e, f, c in zip(names, first, counts) for o in range(0, max(c, 1), size)]
+        td = torch.tensor(tiles, dtype=torch.int32, device=dev)
+        many = len(tiles) * -(-N // 256)
+        call = lambda: ops.L.qsv_grouped_gemm(out.data_ptr(), x.data_ptr(), order.data_ptr() if div else None, max(div, 1), w.data_ptr(), td.data_ptr(), len(tiles),      # noqa: E731
+                                              N, K, act, 0.0, None, s)
+    else:
+        at = torch.zeros(E + 1, dtype=torch.int32)
+        for e, c in zip(names, counts):
+            at[e + 1] = c
+        at, od = at.cumsum(0).int().to(dev), order.int()
+        many = sum(-(-c // 256) for c in counts) * -(-N // 256)
+        call = lambda: ops.L.qsv_grouped_gemm_sorted(out.data_ptr(), x.data_ptr(), od.data_ptr() if div else None, max(div, 1), w.data_ptr(), at.data_ptr(),             # noqa: E731
+                                                     E, N, K, act, 0.0, None, s)
+    assert many > 256                                                   # (a workgroup for each of 256 CUs)
+    for _ in range(2):
+        ops.check(call(), "grouped")
+    for e, f, c in zip(names, first, counts):
+        if not c:
+            continue
+        # float sums of K products of order K^-1/2; half a unit in the last of bfloat16's 8 digits (or a rounding that falls the other way)
+        a, d = x[order[f:f + c] // max(div, 1)].double() @ w[e].double().t(), K * 2.0 ** -22
+        if act == 2:
+            g, u = a[:, 0::2], a[:, 1::2]
+            a, d = _silu(g) * u, d * (1.1 * u.abs() + g.abs()) + 2.0 ** -20 * (_silu(g) * u).abs()
+        elif act == 1:
+            a, d = torch.relu(a) ** 2, 2.0 * d * a.abs() + d * d
+        assert ((out[f:f + c].double() - a).abs() <= 2.0 ** -8 * a.abs() + d).all(), (e, c)
+    assert (out[n] == 3.0).all()
 
 
 @pytest.mark.parametrize("E", [1025, 1600, 8064])

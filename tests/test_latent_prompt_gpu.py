@@ -152,3 +152,60 @@ def test_a_pool_off_16_bytes_is_taken():
     a = outs[0].double()
     for o in outs[1:]:
         assert (o.double() - a).norm() <= 2.0 ** -9 * a.norm()
+
+
+def _wide(layer, h, window):
+    """The layer over one sequence in float64, all of its tokens at once."""
+    H, n, d = layer.H, h.size(0), lambda t: t.double()
+    down = d(h) @ d(layer.w_down).t()
+    norm = lambda t, w: t / (t.pow(2).mean(-1, keepdim=True) + layer.eps).sqrt() * d(w)            # noqa: E731
+    q = (norm(down[:, :layer.q_rank], layer.dq_norm) @ d(layer.w_uq).t()).view(n, H, 128 + layer.rot_dim)
+    kv = down[:, layer.kv_off:layer.kv_off + layer.row_width]
+    c, kr = norm(kv[:, :layer.rank], layer.dkv_norm), kv[:, layer.rank:]
+
+    def turned(u):
+        if not layer.rot_dim:
+            return u
+        cos, sin = (layer.rotary.reserve(n)[:, i].double().view(n, *[1] * (u.dim() - 2), -1) for i in (0, 1))
+        a, b = u[..., 0::2], u[..., 1::2]
+        return torch.stack([a * cos - b * sin, b * cos + a * sin], -1).flatten(-2)
+    qr, kr = turned(q[..., 128:]), turned(kr)
+    i = torch.arange(n, device=h.device)
+    seen = (i[None] <= i[:, None]) & (i[None] > i[:, None] - (window or n))
+    outs = []
+    for j in range(H):
+        s = q[:, j, :128] @ (c @ d(layer.w_uk[j]).t()).t() + qr[:, j] @ kr.t()
+        outs.append(torch.softmax((s * layer.scale).masked_fill(~seen, -math.inf), 1) @ (c @ d(layer.w_uv[128 * j:128 * j + 128]).t()))
+    o = torch.cat(outs, 1)
+    return (o * torch.sigmoid(down[:, layer.g_off:]) if layer.gated else o) @ d(layer.w_o).t()
+
+
+# two sequences in portions (sequence, first position, tokens), step after step: up to 64 tokens and behind more than three times as many keys on the rows, between
+# them over written-out heads, both kinds of run in one step, one head too few
+@pytest.mark.parametrize("H, rank, rot_dim, gated, window", [(4, 64, 64, False, None), (3, 512, 64, True, None), (5, 128, 0, True, 96), (2, 64, 64, False, None)])
+def test_portions_on_both_sides_of_the_line(H, rank, rot_dim, gated, window):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    layer, g = _layer(H=H, rank=rank, rot_dim=rot_dim, gated=gated, window=window), torch.Generator().manual_seed(H)
+    steps = [([(0, 0, 200)], True), ([(0, 200, 40)], False), ([(0, 240, 70)], None if window else False), ([(0, 310, 110), (1, 0, 65)], True), ([(0, 420, 1), (1, 65, 1)], False),
+             ([(1, 66, 170), (0, 421, 1)], True), ([(0, 422, 129)], None if window else False), ([(0, 551, 300), (1, 236, 3)], True)]
+    h = [torch.randn(n, 256, generator=g).bfloat16().cuda() for n in (851, 239)]
+    table = torch.randperm(18, generator=g)[:18].int().view(1, -1).cuda()
+    table = torch.cat([table[:, :14], torch.cat([table[:, 14:], table[:, :10]], 1)])        # (the second sequence's pages: the last four; the rest is never reached)
+    pool = torch.full((18 * 64, rank + rot_dim), float("nan"), dtype=torch.bfloat16, device="cuda")
+    plan, taken = layer.ops.latent_prompt_plan, []
+    layer.ops.latent_prompt_plan = lambda *a: taken.append(plan(*a)) or taken[-1]
+    got = [torch.zeros(t.size(0), 256, dtype=torch.float64, device="cuda") for t in h]
+    for runs, heads_form in steps:
+        out, at = _step(layer, torch.cat([h[b][s:s + n] for b, s, n in runs]), runs, pool, table), 0
+        assert heads_form is None or (taken[-1] is not None) == (heads_form and H > 2)
+        for b, s, n in runs:
+            got[b][s:s + n] = out[at:at + n].double()
+            at += n
+    for b in (0, 1):
+        ref = _wide(layer, h[b], window)
+        # ten roundings to bfloat16 on the way of the values (2^-9 of what they round at most, 0.6 of that in the mean, independent), four on the way of scores of
+        # up to 4, which scale their weights: (10 + 4 4^2)^0.5 0.6 2^-9 < 2^-6.5 of a portion's size
+        for s, n in [(s, n) for runs, _ in steps for q, s, n in runs if q == b]:
+            err = (got[b][s:s + n] - ref[s:s + n]).norm() / ref[s:s + n].norm()
+            assert err <= 2.0 ** -6.5, (b, s, n, err)

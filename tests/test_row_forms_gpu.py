@@ -250,3 +250,75 @@ def test_decay_by_width(dtype, H, dim, log):
         power = -torch.nn.functional.softplus(-u) / 16.0
     # a power of e that carries some units of 2^-24 of itself, exponentials of a few more
     assert ((ops.decay(z, b, a, 16.0, H, dim).double() - power.exp()).abs() <= 2.0 ** -20 * (1.0 + power.abs()) * power.exp() + 1e-30).all()
+
+
+# The forms of four columns a thread against their statements in 64 bits: rotated pairs, norms of a latent row, sums of streams, embeddings
+@TYPES
+@pytest.mark.parametrize("T, n", [(1, 4), (3, 64), (65, 260), (2, 2052)])
+def test_rows_against_64_bits(dtype, T, n):
+    ops, g = make(dtype), torch.Generator().manual_seed(T + n)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(dtype).to(DEV)                                        # noqa: E731
+    rms = lambda t, w: t.double() / (t.double().pow(2).mean(-1, keepdim=True) + 1e-5).sqrt() * w.double()  # noqa: E731
+    pos, slot = torch.randperm(T, generator=g), torch.randperm(2 * T, generator=g)[:T].to(DEV)
+    # a latent row: query latent, key-value latent and rotated key with neighbours as pairs
+    rot_n = min(n, 64) // 4 * 2
+    down, qw, kw, rope = rnd(T, 3 * n + 4), rnd(n), rnd(n), torch.randn(T + 1, 2, rot_n // 2, generator=g).to(DEV)
+    pool = torch.zeros(2 * T, 2 * n, dtype=dtype, device=DEV)
+    cq = ops.latent_prep(down, 0, n, qw, n + 4, n, kw, n, rot_n, rope, pool, slot, pos.int().to(DEV), 1e-5)
+    c, s = (rope[pos, i].double() for i in (0, 1))
+    kr = down[:, 2 * n + 4:].double()
+    a, b = kr[:, 0:rot_n:2].clone(), kr[:, 1:rot_n:2].clone()
+    kr[:, 0:rot_n:2], kr[:, 1:rot_n:2] = a * c - b * s, b * c + a * s
+    assert close(cq, rms(down[:, :n], qw), 16.0, dtype)
+    assert close(pool[slot][:, :n], rms(down[:, n + 4:2 * n + 4], kw), 16.0, dtype) and close(pool[slot][:, n:], kr, 16.0, dtype)
+    # pairs half a head apart, turned back
+    o, rope = rnd(T, 3, 2 * n), torch.randn(T, 2, n, generator=g).to(DEV)
+    c, s = (rope[pos, i].double()[:, None] for i in (0, 1))
+    a, b = o.double()[..., :n], o.double()[..., n:]
+    assert close(ops.rotate_heads(o.clone(), rope, pos.int().to(DEV), -1.0), torch.cat([a * c + b * s, b * c - a * s], -1), 16.0, dtype)
+    x, w, b, rows = torch.randn(T, 3, n, generator=g).to(DEV), rnd(n), rnd(n), ints(pos.tolist())
+    assert close(ops.dyt_sum_rows(x, rows, (w, b, 0.6)), torch.tanh(0.6 * x[rows.long()].double().sum(1)) * w.double() + b.double(), 16.0, dtype)
+    table, tokens = rnd(9, n), torch.randint(0, 9, (T,), generator=g).to(DEV)
+    h, t = ops.embed(tokens.int(), table)
+    assert torch.equal(h, table[tokens].float()) and torch.equal(t, table[tokens])
+    streams = ops.embed_streams(tokens.int(), table, 1.7, 3)
+    assert close(streams, (1.7 * table[tokens].double())[:, None].expand(T, 3, n), 0.0, torch.float32)
+
+
+# ... convolutions over time: runs with and without a history, the histories that they leave
+@TYPES
+@pytest.mark.parametrize("taps", [2, 3, 4])
+@pytest.mark.parametrize("runs", [((0, 1), (7, 1), (1, 1)), ((2, 3), (0, 2), (9, 4))])
+def test_convolutions_against_64_bits(dtype, taps, runs):
+    ops, g = make(dtype), torch.Generator().manual_seed(taps + len(runs))
+    T, qc, G, kd, vd = sum(n for _, n in runs), 40, 2, 8, 12
+    C, past = qc + G * (kd + vd), taps - 1
+    proj, w = torch.randn(T, C + 4, generator=g).to(dtype).to(DEV), torch.randn(taps, C, generator=g).to(DEV)
+    hist = torch.randn(2 * len(runs), past, C, generator=g).to(DEV)
+    off_, rd, wr, pos, items, at, y, left = [], [], [], [], [], 0, [], hist.double()
+    for r, (start, n) in enumerate(runs):
+        off_ += range(n)
+        rd += [2 * r if start else -1] * n
+        wr += [-1] * (n - 1) + [2 * r + 1]
+        pos += range(start, start + n)
+        items.append((r, at, n))
+        seq = torch.cat([hist[2 * r].double() if start else torch.zeros(past, C, device=DEV), proj[at:at + n, :C].double()])
+        y.append(sum(seq[j:j + n] * w[j].double() for j in range(taps)))
+        left[2 * r + 1] = seq[n:]
+        at += n
+    y = torch.cat(y)
+    batch = StepBatch(tokens=None, seq=None, pos=ints(pos), slot=torch.arange(T, device=DEV), block_table=None, max_pos=max(pos), n_tokens=T, items=items,
+                      run_off=ints(off_), state_rd=ints(rd), state_wr=ints(wr))
+    h, pool = hist.clone(), torch.zeros(G, T, vd + kd, dtype=dtype, device=DEV)
+    q = ops.conv_heads_cache(proj, w, h, batch, qc, G, kd, vd, pool, 0.3, (0.1, 4.0))
+    warm = 1.0 + 0.1 * torch.log(((torch.tensor(pos, device=DEV).double() + 1.0) / 4.0).floor() + 1.0)
+    assert close(q, 0.3 * y[:, :qc] * warm[:, None], 16.0, dtype) and torch.equal(h.double(), left)
+    k, v = y[:, qc:qc + G * kd].view(T, G, kd).transpose(0, 1), y[:, qc + G * kd:].view(T, G, vd).transpose(0, 1)
+    assert close(pool[..., :vd], v, 16.0, dtype) and close(pool[..., vd:], k, 16.0, dtype)
+    h = hist.clone()
+    got, ref = ops.conv_silu_unit(proj, 0, w.t().contiguous(), h, batch, 4, 8), y * torch.sigmoid(y)
+    u = ref[:, :32].reshape(-1, 8)
+    ref = torch.cat([(u / (u.pow(2).sum(-1, keepdim=True) + 1e-6).sqrt()).view(T, 32), ref[:, 32:]], 1)
+    # unit vectors: float products of up to 16 over a length that may be small
+    size = torch.cat([(1.0 + 1.0 / (u.pow(2).sum(-1, keepdim=True) + 1e-6).sqrt()).expand_as(u).reshape(T, 32), torch.ones_like(ref[:, 32:])], 1) * 16.0
+    assert ((got.double() - ref).abs() <= 2.0 ** -20 * (ref.abs() + size)).all() and torch.equal(h.double(), left)

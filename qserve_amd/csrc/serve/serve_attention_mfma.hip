@@ -526,7 +526,9 @@ __global__ __launch_bounds__(64 * RW, RT + CT > 24 ? 2 : 4) void latent_rows_ker
 // 13.4 us and 512 / 512 15.1 -> 12.3 (13.7 and 12.4 with one round ahead), 16 sequences at 100 - 220 of 256 / 128 8.7 -> 7.2.
 // Measured alone, its queries in the caches (16 heads, 576 / 512, best split each, kernel above -> this one and the merge below): 64 sequences at 128 / 1000 /
 // 2000 positions 15 -> 12.5 / 31 -> 26 / 44 -> 36 us, 16 at 1000 25 -> 18, one at 300 / 2000 17 -> 14.5 / 28 -> 17.5; 256 / 128, 16 heads on 4 pools, 16
-// sequences at 1000: 15 -> 10.8 us.
+// sequences at 1000: 15 -> 10.8 us.  The queries' early requests are for a step, whose queries come from memory: alone, short contexts lose 0.5 us by them (64 at 128
+// 12 -> 12.5, one at 300 / 2000 14 -> 14.5 / 17 -> 17.5), inside a step of one sequence at 300 / 2000 positions 576 / 512 takes 16.4 -> 12.7 / 16.5 -> 13.1 us and
+// 512 / 512 14.8 -> 11.8 / 15.2 -> 12.1.
 constexpr int SW = 4, SN = 64;       // waves, keys of a round
 template <int RT, int CT, int S0>
 __global__ __launch_bounds__(64 * SW, 1) void latent_step_kernel(

@@ -39,7 +39,9 @@ __device__ __forceinline__ unsigned pack_bf2(float a, float b) { return (unsigne
 // Measured (MI355X, one product, the form before -> now in one call; before: eight waves in step, one barrier and a wait for every request per K step, rows
 // first): 32768 slots x 4096 x 4096 1014 -> 866 us (1270 TFLOP/s; hipBLASLt's dense product of that size 740), 28480 slots over 32 experts gated
 // 5504 x 4096 1380 -> 1230 (1045), 4096 x 2752 686 -> 587 (1095), 32768 over 16 of 1408 x 2048 204 -> 203, 2048 x 1408 201 -> 185, 8188 over 16 gated 2816 x 2048
-// 118 -> 115, 2048 x 1408 63.6 -> 64.5, 1300 over 16 of these 44.4 -> 42.4, 28.9 -> 29.8.  A K step takes 1.5 us, which is the card's power: the same
+// 118 -> 115, 2048 x 1408 63.6 -> 64.5, 1300 over 16 of these 44.4 -> 42.4, 28.9 -> 29.8.  Small layers, both products with sort and sum, weights out of memory / left in the caches by the call before: 4
+// gated of 2048 x 1408, 1024 slots 84 -> 75 / 67 -> 75, 8 of them, 1200 92 -> 83 / 72 -> 81, 8 of 1024 x 512 49 -> 46 / 40 -> 45, 4 of 512 x 2048 63 -> 57 / 45 -> 56:
+// a layer's weights are in the caches only where the whole model is one small layer; from 4096 x 2752 on 0.77 - 0.93 of before either way.  A K step takes 1.5 us, which is the card's power: the same
 // instructions on constant data take 1.1.  How far ahead the requests run (3 - 7 phases) and bands of 4 - 12 make no difference.
 constexpr int PR = 256, PS = 256, PWAVES = 8, PT = 64 * PWAVES;
 constexpr int PBUF = (PR + PS) * 128;               // bytes of one K step

@@ -27,11 +27,13 @@ def _skinny(T, N, K):
     """Whether the kernel that streams the weight beats the vendor's product for T rows.  Every line is from both sides' times, measured from HBM
     for T 1 - 64, N 8 - 152064, K 64 - 29568 (vendor / own below, us); beyond 64 rows never.
     * It has one workgroup per 16 or 32 weight rows, each reading the inputs again, so it loses where a second round of workgroups is nearly
-      empty (4608 x 5120, 16 tokens 15.3 / 16.6) or the inputs outweigh its lead (4096 x 3072, 33 tokens 11.2 / 12.3, 64: 16.1 / 12.9).
-    * It does not split the reduction; the vendor's product does for few outputs and long rows of a multiple of 512 (64 x 8192 8.4 / 10.6, 1024 x 6144
-      33 tokens 10.6 / 11.5; but 512 x 11008 33 / 14, 2048 x 18944 56 / 27).
-    * Rows a multiple of 16 KB apart slow the stream (8192 x 8192 31 / 36, 152064 x 8192 449 / 531).
-    Otherwise its lead is the start of the stream: 2048 x 2048 8.2 / 4.7, 4096 x 4096 15.5 / 9.2, 4096 x 11008 39 / 22, 27648 x 5120 81 / 58."""
+      empty (4608 x 5120, 16 tokens 15.5 / 16.3) or the inputs outweigh its lead (4096 x 3072, 48 tokens 11.4 / 13.1, 64: 16.1 / 13.3).
+    * It does not split the reduction; the vendor's product does for few outputs and long rows of a multiple of 512 (64 x 8192 8.5 / 10.6, 1024 x 6144
+      48 tokens 10.9 / 11.9; but 512 x 11008 33 / 14, 2048 x 18944 57 / 27).
+    * Rows a multiple of 16 KB apart slow the stream (8192 x 8192 33 / 36, 48 tokens 37 / 56).
+    Otherwise its lead is the start of the stream: 2048 x 2048 8.3 / 4.8, 4096 x 4096 15.8 / 8.8, 4096 x 11008 39 / 21.
+    Over 1938 sizes with the weights past the caches the lines leave 25 to the slower kernel by 3 % and more, most of them outputs of rows of 64 (65536 x 64,
+    16 tokens 5.4 / 8.2), and give the vendor 191 that the stream would win by 10 %, most of them 33 - 64 tokens of rows beyond 7168 (1024 x 18944 77 / 31)."""
     if T <= 16:
         if K <= 4864:
             return K <= 2048 or N * K <= 135_000_000
@@ -1136,10 +1138,12 @@ class HipOps:
     # one workgroup per token walks a whole product (one token at 2048 x 1408, 4 of 16 experts: 4.6 ms against 0.04 ms) - serve
     # float storage and widths the others do not take.
     moe_token_slots = 0
-    # None: 896 (crossover measured: 16 experts of 2048 x 1408 at 1000 (relu^2) and 850 slots (gated), 32 of 4096 x 2752 at 850; it moves with the
-    # slots per expert: 2 of 2048 x 1408 at 450, 8 of 4096 x 2752 at 320, 128 and 256 of 2048 x 768 / 512 at 1000); 1024 where the grouped kernel does
-    # not take the sizes - the vendor products wait for the runs' lengths and cannot be captured; 64 (moe_sorted_above) for rows longer than 4096 (8 of
-    # 5120 x 5632, gated, 64 / 256 / 512 slots: 235 / 338 / 523 us, grouped 371 / 381 / 402; 16 of 8192 x 4096 64 / 256: 429 / 440, grouped 388 / 396)
+    # None: 896.  Crossover measured, slots (expert-major / sorted around it, us): 16 experts of 2048 x 1408 relu^2 at 900 (896 77 / 79, 1024 97 / 81), gated at
+    # 580 (512 77 / 85, 640 94 / 86), 32 of 4096 x 2752 at 800 (768 400 / 401, 896 429 / 404), 64 of 2048 x 1408, 128 of 2048 x 768 and 256 of 2048 x 512 above
+    # 1024 (222 / 239 and 310 / 311 there), 8 of 1024 x 512 and 64 of 1024 x 256 at 1200.  It moves with the slots per expert: 2 and 4 of 2048 x 1408 at 540 and
+    # 600 (640 77 / 68 and 71 / 68; 2 of them at 896 104 / 69), 16 and 8 of 4096 x 2752 at 450 and 220 (512 284 / 256, 256 168 / 143).
+    # 1024 where the grouped kernel does not take the sizes - the vendor products wait for the runs' lengths and cannot be captured; 64 (moe_sorted_above) for
+    # rows longer than 4096 (16 of 8192 x 4096, 64 slots 611 / 577; but 8 of 5120 x 5632, gated, 64 / 192 / 256: 210 / 294, 250 / 294, 360 / 296)
     moe_expert_major_slots = None
 
     def _grouped_takes(self, E, rows, D, ff):

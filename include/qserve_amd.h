@@ -74,6 +74,14 @@ int qs_w4a8_per_group_gemm(const int8_t* in_feats, const int8_t* kernel, const i
                            const int8_t* scales_i8, const void* wscales, const void* ascales, void* out_feats,
                            int M, int N, int K, qs_stream_t stream);
 
+/* The same with scratch of the caller's, for products of many tokens: the weights are widened to int8 into it once and multiplied from there (two launches,
+ * the same bits).  qs_w4a8_per_group_scratch_bytes: what the call wants (N K bytes, on 16; 0: nothing, the plain entry is the faster one - or the shape
+ * does not fit).  With less than that, or with operands that do not start on 16 bytes, the call is the plain entry.  The scratch holds nothing
+ * afterwards and may be given to any later work of the same stream. */
+long long qs_w4a8_per_group_scratch_bytes(int M, int N, int K);
+int qs_w4a8_per_group_gemm_scratch(const int8_t* in_feats, const int8_t* kernel, const int8_t* zeros, const int8_t* scales_i8, const void* wscales,
+                                   const void* ascales, void* out_feats, int M, int N, int K, void* scratch, long long scratch_bytes, qs_stream_t stream);
+
 /* gate_up GEMM + silu_and_mul in one launch (engine-side fusion, like the pairs further down; no reference op of its
  * own: LlamaMLP.forward, llama_w4a8_unpad.py:69-93, issues gate_up_proj, then SiluAndMulQuant = silu_and_mul ; invoke_quant).
  *   kernel   the stacked gate_up weight [N, K/2], rows 0 .. N/2-1 = gate, N/2 .. N-1 = up (load_weights' row
@@ -89,6 +97,10 @@ int qs_w4a8_per_chn_gemm_silu_mul(const int8_t* in_feats, const int8_t* kernel, 
 int qs_w4a8_per_group_gemm_silu_mul(const int8_t* in_feats, const int8_t* kernel, const int8_t* zeros,
                                     const int8_t* scales_i8, const void* wscales, const void* ascales, void* out_act,
                                     void* tmp, int M, int N, int K, qs_stream_t stream);
+
+int qs_w4a8_per_group_gemm_silu_mul_scratch(const int8_t* in_feats, const int8_t* kernel, const int8_t* zeros, const int8_t* scales_i8, const void* wscales,
+                                            const void* ascales, void* out_act, void* tmp, int M, int N, int K, void* scratch, long long scratch_bytes,
+                                            qs_stream_t stream);
 
 /* Debug/parity entry points: same kernels, but the raw INT32 accumulators are written to acc_out [M,N]
  * instead of the fp16 epilogue (the reference keeps them in registers: gemm_cuda.cu:327). */

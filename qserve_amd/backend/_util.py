@@ -50,3 +50,17 @@ def expect(t, dtype, name, contiguous=True):
         raise RuntimeError(f"{name} must be on CUDA")   # wording of the reference's CHECK_DEVICE
     if contiguous and not t.is_contiguous():
         raise RuntimeError(f"{name} must be contiguous")
+
+
+def widened_scratch(M, N, K, like):
+    """Scratch for a per-group product of many tokens (include/qserve_amd.h, qs_w4a8_per_group_scratch_bytes), or None: the product needs none - a decode
+    step is not asked -, or there is no memory left for it."""
+    if M <= 256:
+        return None
+    need = lib.qs_w4a8_per_group_scratch_bytes(M, N, K)
+    if need <= 0:
+        return None
+    try:
+        return torch.empty((need,), dtype=torch.uint8, device=like.device)
+    except torch.OutOfMemoryError:
+        return None

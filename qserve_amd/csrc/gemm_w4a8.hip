@@ -402,6 +402,9 @@ int qs_launch_gemm_tiled(int mode, int outk, const int8_t* A, const uint8_t* W, 
 int qs_launch_gemm_wide(int mode, int outk, const int8_t* A, const uint8_t* W, const int8_t* zeros,
                         const int8_t* scales8, const void* wscales, const void* ascales, const void* wszs,
                         const void* assums, void* out, int M, int N, int K, int persist_mode, hipStream_t stream);
+// per-group products of prompts over weights widened into the caller's scratch (gemm_w4a8_unpacked.hip)
+int qs_launch_gemm_unpacked(bool act, const int8_t* A, const uint8_t* W, const int8_t* zeros, const int8_t* scales8, const void* wscales, const void* ascales,
+                            void* out, int M, int N, int K, void* scratch, hipStream_t stream);
 extern qs_flag g_tiled_order;   // gemm_w4a8_tiled.hip
 namespace {
 
@@ -733,11 +736,58 @@ extern "C" int qs_w4a8_per_chn_gemm_silu_mul(const int8_t* in_feats, const int8_
                            stream);
 }
 
+// Per-group products of many tokens over weights widened to int8 in scratch of the caller's (gemm_w4a8_unpacked.hip): the level-2 dequant once a weight in place
+// of once a weight and 256 tokens, and a last round of tiles that is cut.  us, plain -> widened, MI355X, weights out of memory:
+//  * 8192 tokens: 12288 x 4096 389 -> 329, 4096 x 11008 311 -> 279, 28672 x 4096 + silu 880 -> 769; 5331: 253 -> 224, 274 -> 218, 634 -> 529; 1300: 118 -> 96, 180 -> 97,
+//    201 -> 183; 2048 x 2048 30 -> 26.  Not where the four-wave tile needs one round of the chip only (12288 x 4096, 1152 tokens 67 -> 72), nor up to 2 M weights (512 x 4096
+//    26 -> 33, 1024 x 1024 13 -> 17).
+//  * up to 1024 tokens the widening is a larger share: not in one round of any kernel (28672 x 4096, 512 tokens 68 -> 86), not up to 4096 x 4096 (1024 tokens
+//    39 -> 41; 6144 x 4096 54 -> 47, 4096 x 14336 110 -> 100), not beyond 128 M weights (57344 x 8192, 1024 tokens 472 -> 510; 28672 x 4096 133 -> 133); up to 512 only
+//    beside two rounds of 128-token tiles (22016 x 4096, 300 tokens 104 -> 73; the ring kernel's two: 8192 x 8192, 512 tokens 68 -> 71).
+extern "C" long long qs_w4a8_per_group_scratch_bytes(int M, int N, int K) {
+    if (g_variant != QS_GEMM_DEFAULT || M <= 256 || N <= 0 || K <= 0 || N % 256 != 0 || K % 128 != 0 || K >= (1 << 24) || (size_t)M * K >= (1ull << 32) ||
+        (size_t)N * K >= (1ull << 32))
+        return 0;
+    const long long need = (long long)N * K, million = 1 << 20;
+    if (need < 4 * million || (M <= 1024 && (need < 20 * million || need > 128 * million))) return 0;
+    int plan[5];
+    if (qs_w4a8_gemm_plan(1, M, N, K, plan) != QS_OK) return 0;
+    const bool ring = plan[0] == 3, tiled = plan[0] == 4, wide = plan[0] == 5;
+    const long long groups = ring ? (long long)plan[3] * (N / (64 * plan[2])) * plan[4]                            // token blocks x channels x K slices
+                             : tiled || wide ? (long long)((M + 32 * plan[1] - 1) / (32 * plan[1])) * (N / 256) : 0;
+    if (M <= 512 ? !(tiled && groups > 256) : M <= 1024 ? (ring || tiled || wide) && groups <= 256 : wide && groups <= 256) return 0;
+    return need;
+}
+namespace {
+bool unpack_fits(const void* in_feats, const void* kernel, const void* zeros, const void* scales_i8, const void* wscales, const void* ascales, const void* out,
+                 int M, int N, int K, const void* scratch, long long scratch_bytes) {
+    const long long need = qs_w4a8_per_group_scratch_bytes(M, N, K);
+    return need > 0 && scratch && scratch_bytes >= need && in_feats && kernel && zeros && scales_i8 && wscales && ascales && out &&
+           ((uintptr_t)in_feats | (uintptr_t)kernel | (uintptr_t)out | (uintptr_t)scratch) % 16 == 0 && ((uintptr_t)zeros | (uintptr_t)scales_i8) % 4 == 0;
+}
+}  // namespace
+extern "C" int qs_w4a8_per_group_gemm_scratch(const int8_t* in_feats, const int8_t* kernel, const int8_t* zeros, const int8_t* scales_i8, const void* wscales,
+                                              const void* ascales, void* out_feats, int M, int N, int K, void* scratch, long long scratch_bytes, qs_stream_t stream) {
+    if (!unpack_fits(in_feats, kernel, zeros, scales_i8, wscales, ascales, out_feats, M, N, K, scratch, scratch_bytes))
+        return qs_w4a8_per_group_gemm(in_feats, kernel, zeros, scales_i8, wscales, ascales, out_feats, M, N, K, stream);
+    return qs_launch_gemm_unpacked(false, in_feats, reinterpret_cast<const uint8_t*>(kernel), zeros, scales_i8, wscales, ascales, out_feats, M, N, K, scratch,
+                                   (hipStream_t)stream);
+}
+
 extern "C" int qs_w4a8_per_group_gemm_silu_mul(const int8_t* in_feats, const int8_t* kernel, const int8_t* zeros,
                                                const int8_t* scales_i8, const void* wscales, const void* ascales,
                                                void* out_act, void* tmp, int M, int N, int K, qs_stream_t stream) {
     return gate_up_silu<1>(in_feats, kernel, zeros, scales_i8, wscales, ascales, nullptr, nullptr, out_act, tmp, M, N, K,
                            stream);
+}
+
+extern "C" int qs_w4a8_per_group_gemm_silu_mul_scratch(const int8_t* in_feats, const int8_t* kernel, const int8_t* zeros, const int8_t* scales_i8,
+                                                       const void* wscales, const void* ascales, void* out_act, void* tmp, int M, int N, int K, void* scratch,
+                                                       long long scratch_bytes, qs_stream_t stream) {
+    if (g_act_off || !unpack_fits(in_feats, kernel, zeros, scales_i8, wscales, ascales, out_act, M, N, K, scratch, scratch_bytes))
+        return qs_w4a8_per_group_gemm_silu_mul(in_feats, kernel, zeros, scales_i8, wscales, ascales, out_act, tmp, M, N, K, stream);
+    return qs_launch_gemm_unpacked(true, in_feats, reinterpret_cast<const uint8_t*>(kernel), zeros, scales_i8, wscales, ascales, out_act, M, N, K, scratch,
+                                   (hipStream_t)stream);
 }
 
 // ---- K-slice planes (round 4) ---------------------------------------------------------------------------------------------

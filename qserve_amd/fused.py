@@ -11,7 +11,7 @@ they exist because at decode batch sizes each row kernel is a fixed ~5 us latenc
 """
 import torch
 
-from .backend._util import check, expect, guard, lib, ptr, stream
+from .backend._util import check, expect, guard, lib, ptr, stream, widened_scratch
 
 
 def add_residual_rms_norm_general(out, hidden, delta, weight, scaling, epsilon, input_sum=None):
@@ -77,6 +77,12 @@ def _gemm_silu(per_group, in_feats, kernel, rest, out_act, tmp):
             raise RuntimeError(f"gemm_silu_and_mul: tmp has {tmp.numel()} elements, needs {M} x {N}")
     fn = lib.qs_w4a8_per_group_gemm_silu_mul if per_group else lib.qs_w4a8_per_chn_gemm_silu_mul
     with guard(out_act):
+        scratch = widened_scratch(M, N, K, in_feats) if per_group else None
+        if scratch is not None:
+            check(lib.qs_w4a8_per_group_gemm_silu_mul_scratch(ptr(in_feats), ptr(kernel), *[ptr(t) for t in rest], ptr(out_act),
+                                                              ptr(tmp) if tmp is not None else 0, M, N, K, ptr(scratch), scratch.numel(), stream()),
+                  "fused.gemm_silu_and_mul")
+            return
         check(fn(ptr(in_feats), ptr(kernel), *[ptr(t) for t in rest], ptr(out_act), ptr(tmp) if tmp is not None else 0,
                  M, N, K, stream()), "fused.gemm_silu_and_mul")
 

@@ -76,6 +76,21 @@ void gemm_per_group(torch::Tensor in_feats, torch::Tensor kernel, torch::Tensor 
         TORCH_CHECK(wscales.numel() >= N && ascales.numel() >= out_feats.size(-2), "wscales / ascales: one value per channel / token");
     }
     const DeviceGuard guard(in_feats.device());
+    const int M = (int)out_feats.size(-2), N = (int)out_feats.size(-1), K = (int)in_feats.size(1);
+    // scratch for the widened weights of a product of many tokens; without memory for it the product runs without
+    torch::Tensor scratch;
+    const long long wanted = M > 256 ? qs_w4a8_per_group_scratch_bytes(M, N, K) : 0;
+    if (wanted > 0) {
+        try {
+            scratch = torch::empty({(int64_t)wanted}, in_feats.options());
+        } catch (const c10::OutOfMemoryError&) {
+        }
+    }
+    if (scratch.defined()) {
+        QS_CALL(qs_w4a8_per_group_gemm_scratch(in_feats.data_ptr<int8_t>(), kernel.data_ptr<int8_t>(), zeros.data_ptr<int8_t>(), scales_i8.data_ptr<int8_t>(),
+                                               wscales.data_ptr(), ascales.data_ptr(), out_feats.data_ptr(), M, N, K, scratch.data_ptr(), wanted, cur_stream()));
+        return;
+    }
     QS_CALL(qs_w4a8_per_group_gemm(in_feats.data_ptr<int8_t>(), kernel.data_ptr<int8_t>(), zeros.data_ptr<int8_t>(),
                                    scales_i8.data_ptr<int8_t>(), wscales.data_ptr(), ascales.data_ptr(), out_feats.data_ptr(),
                                    (int)out_feats.size(-2), (int)out_feats.size(-1), (int)in_feats.size(1), cur_stream()));

@@ -29,7 +29,6 @@ constexpr int NWV = 4;
 constexpr int BN = 32;          // keys per tile
 constexpr int VS = BN + 4;      // row stride (elements) of the transposed tile: 18 dwords, 8-byte reads of 32 lanes hit 64 banks
 
-__device__ __forceinline__ unsigned pack_bf2(float a, float b) { return (unsigned)f2bf(a) | ((unsigned)f2bf(b) << 16); }
 
 // RT: 32-element steps along a cache row (R <= 32 RT); CT: 16-column tiles of the output (rank <= 16 CT).
 template <int RT, int CT>

@@ -29,12 +29,13 @@ static inline int qsv_launch_status(const char* what) {
 typedef uint16_t bf16_t;   // storage only: arithmetic is float
 
 __device__ __forceinline__ float bf2f(bf16_t v) { return __uint_as_float((uint32_t)v << 16); }
-__device__ __forceinline__ bf16_t f2bf(float f) {   // round to nearest even; NaN stays NaN
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return (bf16_t)0x7fc0;
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (bf16_t)(u >> 16);
-}
+// Round to nearest even; NaN stays NaN.  v_cvt_pk_bf16_f32: one instruction for two values, where bit arithmetic takes eight for each: a grouped product's epilogue
+// (128 values a lane) 4.1 -> 3.5 us, a model's step of 64 tokens 2 % (64 sequences of Vekalorn 12.98 -> 12.68 ms).  Over all 2^32 floats the same bits but for a NaN's sign
+// and payload.
+typedef float pair_f32 __attribute__((ext_vector_type(2)));
+typedef __bf16 pair_bf16 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ bf16_t f2bf(float f) { return __builtin_bit_cast(bf16_t, (__bf16)f); }
+__device__ __forceinline__ uint32_t pack_bf2(float a, float b) { return __builtin_bit_cast(uint32_t, __builtin_convertvector((pair_f32{a, b}), pair_bf16)); }
 __device__ __forceinline__ float ld(const float* p, size_t i) { return p[i]; }
 __device__ __forceinline__ float ld(const bf16_t* p, size_t i) { return bf2f(p[i]); }
 __device__ __forceinline__ void st(float* p, size_t i, float v) { p[i] = v; }
@@ -115,7 +116,7 @@ __device__ __forceinline__ void ld4t(const bf16_t* p, size_t i, float (&v)[4]) {
 }
 __device__ __forceinline__ void st4t(float* p, size_t i, const float (&v)[4]) { *(float4*)(p + i) = make_float4(v[0], v[1], v[2], v[3]); }
 __device__ __forceinline__ void st4t(bf16_t* p, size_t i, const float (&v)[4]) {
-    *(uint2*)(p + i) = make_uint2((unsigned)f2bf(v[0]) | ((unsigned)f2bf(v[1]) << 16), (unsigned)f2bf(v[2]) | ((unsigned)f2bf(v[3]) << 16));
+    *(uint2*)(p + i) = make_uint2(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]));
 }
 // The same in two steps, request and use.  A row kernel requests every operand as it lies in memory, at a column inside the row (a lane behind its end repeats
 // the last), and converts behind `requested()`: a conversion beside its load, or in a branch that not every lane takes, makes the wave wait there, and a row

@@ -71,8 +71,8 @@ template <int V>
 __device__ __forceinline__ void stv(bf16_t* p, size_t i, const Vec<V>& x) {
     if constexpr (V == 4) {
         uint2 u;
-        u.x = (uint32_t)f2bf(x.v[0]) | ((uint32_t)f2bf(x.v[1]) << 16);
-        u.y = (uint32_t)f2bf(x.v[2]) | ((uint32_t)f2bf(x.v[3]) << 16);
+        u.x = pack_bf2(x.v[0], x.v[1]);
+        u.y = pack_bf2(x.v[2], x.v[3]);
         *(uint2*)(p + i) = u;
     } else {
         for (int e = 0; e < V; ++e) p[i + e] = f2bf(x.v[e]);
@@ -333,8 +333,6 @@ __global__ __launch_bounds__(NT) void diff_attention_wave_kernel(T* __restrict__
 // * step kernel (runs of at most TQ tokens: decoding): the four waves own the SAME rows and walk different key blocks, each through buffers of
 //   its own without any barrier, and merge at the end; key splits over workgroups leave partial results for a merge launch.
 typedef float v16f __attribute__((ext_vector_type(16)));
-typedef float f2v __attribute__((ext_vector_type(2)));
-typedef __bf16 b2v __attribute__((ext_vector_type(2)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 typedef unsigned int v2u __attribute__((ext_vector_type(2)));
@@ -343,7 +341,6 @@ typedef __attribute__((address_space(3))) s4* lds_s4;
 typedef __attribute__((address_space(3))) void* lds_ptr;
 
 constexpr int BN = 32;                                   // keys per block
-__device__ __forceinline__ unsigned pack_bf2(float a, float b) { return __builtin_bit_cast(unsigned, __builtin_convertvector((f2v{a, b}), b2v)); }
 
 template <int DT, int CT, int M>
 struct Shape {

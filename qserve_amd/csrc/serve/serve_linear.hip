@@ -64,7 +64,7 @@ __device__ __forceinline__ void skinny_product(const SkinnyJob& a, int block, un
         if constexpr (HOW == AS_IS) {
             bf16_t* p = (bf16_t*)a.out + at;
             if (whole) {
-                *(uint2*)p = make_uint2((unsigned)f2bf(v[0]) | ((unsigned)f2bf(v[1]) << 16), (unsigned)f2bf(v[2]) | ((unsigned)f2bf(v[3]) << 16));
+                *(uint2*)p = make_uint2(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]));
             } else {
                 for (int q = 0; q < 4; ++q)
                     if (n + q < a.N) p[q] = f2bf(v[q]);
@@ -191,7 +191,7 @@ __global__ __launch_bounds__(256) void head_product_kernel(HeadProductArgs a) {
                 v.x *= 1.0f / (1.0f + expf(-__uint_as_float(gate[r] << 16)));
                 v.y *= 1.0f / (1.0f + expf(-__uint_as_float(gate[r] & 0xffff0000u)));
             }
-            *(unsigned*)((bf16_t*)a.out + ((size_t)t * a.H + h) * a.N + n0 + c) = (unsigned)f2bf(v.x) | ((unsigned)f2bf(v.y) << 16);
+            *(unsigned*)((bf16_t*)a.out + ((size_t)t * a.H + h) * a.N + n0 + c) = pack_bf2(v.x, v.y);
         }
     }
 }

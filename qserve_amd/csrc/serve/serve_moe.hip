@@ -27,7 +27,7 @@ __device__ __forceinline__ void loadv(const float* p, float (&v)[4]) {
 template <typename T>
 __device__ __forceinline__ void loadv(const T* p, float (&v)[1]) { v[0] = ld(p, 0); }
 __device__ __forceinline__ void storev(bf16_t* p, const float (&v)[4]) {
-    *(uint2*)p = make_uint2((unsigned)f2bf(v[0]) | ((unsigned)f2bf(v[1]) << 16), (unsigned)f2bf(v[2]) | ((unsigned)f2bf(v[3]) << 16));
+    *(uint2*)p = make_uint2(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]));
 }
 __device__ __forceinline__ void storev(float* p, const float (&v)[4]) { *(float4*)p = make_float4(v[0], v[1], v[2], v[3]); }
 template <typename T>
@@ -492,10 +492,10 @@ __device__ __forceinline__ void expert_finish(const ExpertArgs& a, int r0, int c
                         if (at + q < stride) o[q] = u[q];
             } else {
                 bf16_t* o = (bf16_t*)a.out + (size_t)slot * stride + at;
-                const unsigned lo = (unsigned)f2bf(u[0]) | ((unsigned)f2bf(u[1]) << 16);
+                const unsigned lo = pack_bf2(u[0], u[1]);
                 if (a.wide && stride % m == 0 && at + m <= stride) {
                     if (m == 2) *(unsigned*)o = lo;
-                    else *(uint2*)o = make_uint2(lo, (unsigned)f2bf(u[2]) | ((unsigned)f2bf(u[3]) << 16));
+                    else *(uint2*)o = make_uint2(lo, pack_bf2(u[2], u[3]));
                 } else {
                     for (int q = 0; q < m; ++q)
                         if (at + q < stride) o[q] = f2bf(u[q]);

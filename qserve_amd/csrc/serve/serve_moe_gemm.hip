@@ -17,7 +17,6 @@ typedef unsigned int v2u __attribute__((ext_vector_type(2)));
 
 constexpr int KS = 64;       // reduction elements per step
 
-__device__ __forceinline__ unsigned pack_bf2(float a, float b) { return (unsigned)f2bf(a) | ((unsigned)f2bf(b) << 16); }
 
 // Tiles of 256 weight rows x 256 slots (128 or 64 where an expert has no more left).  Bound by the matrix cores.
 //

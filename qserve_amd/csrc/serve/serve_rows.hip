@@ -603,8 +603,8 @@ __device__ __forceinline__ float4 ld4v(const bf16_t* p, size_t i) {
 __device__ __forceinline__ void st4v(float* p, size_t i, float4 v) { *(float4*)(p + i) = v; }
 __device__ __forceinline__ void st4v(bf16_t* p, size_t i, float4 v) {
     uint2 u;
-    u.x = (uint32_t)f2bf(v.x) | ((uint32_t)f2bf(v.y) << 16);
-    u.y = (uint32_t)f2bf(v.z) | ((uint32_t)f2bf(v.w) << 16);
+    u.x = pack_bf2(v.x, v.y);
+    u.y = pack_bf2(v.z, v.w);
     *(uint2*)(p + i) = u;
 }
 template <typename T, int VPT>

@@ -125,7 +125,6 @@ typedef short s4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s4* lds_s4;
 constexpr int BN = 32;             // keys per tile
 
-__device__ __forceinline__ unsigned pack_bf2(float a, float b) { return (unsigned)f2bf(a) | ((unsigned)f2bf(b) << 16); }
 __host__ __device__ constexpr int k_row(int dt) { return 32 * dt + 8; }                       // LDS row strides (elements): the 16 rows of a
 __host__ __device__ inline int v_row(int cols) { return ((cols + 127) & ~127) + 16; }          // read spread over all banks
 

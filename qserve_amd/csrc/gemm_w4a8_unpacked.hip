@@ -65,11 +65,11 @@ __global__ __launch_bounds__(128) void unpack_kernel(int8_t* __restrict__ out, c
 // Tiles of 256 channels x 256 tokens (128 or 64 where no more are left).  Bound by the matrix cores.
 //
 // Eight waves, two per SIMD: waves 0 - 3 and 4 - 7 are half a phase apart, so that one of a SIMD's two always multiplies while the other reads its next
-// operands.  A K step of 128 has four phases, one per quarter of the tile (halves of 128 channels x halves of 128 tokens; in each a wave has 64 channels x
-// 32 tokens: 16 instructions); a phase reads ONE operand half (8 or 4 reads of 16 bytes a lane), requests the same half of the step after the next one into the
-// place that the half read a phase earlier left (global_load_lds, whole 128-byte lines of a row; pieces permuted by the row's number: reads without bank
-// conflicts), and waits for what the next phase reads, requested seven phases before: 96 - 112 KiB in flight a CU.  Of tokens that a tile does not
-// have every wave issues the same requests with one lane, so that the counted waits hold whatever the tile's size.
+// operands.  A K step of 128 has two phases, one per half of the tile's channels; in each a wave has 64 channels x 64 tokens: 32 instructions.  The first reads a
+// weight half and both token halves (16 reads of 16 bytes a lane), the second the other weight half (8).  What every wave has read is requested anew for the
+// step after the next (global_load_lds, whole 128-byte lines of a row; pieces permuted by the row's number: reads without bank conflicts), and a phase waits
+// for what the next one reads, requested three phases before: 64 - 112 KiB in flight a CU.  Of tokens that a tile does not have every wave issues the same
+// requests with one lane, so that the counted waits hold whatever the tile's size.
 //
 // Workgroups are persistent, one per CU; the last two steps of a tile request the first two of the next.  An XCD walks bands of 8 channel tiles and through
 // the tokens inside a band; the tiles of its last, part-empty round are cut by tokens into as many parts (two or four) as it has workgroups for.
@@ -197,7 +197,7 @@ __global__ __launch_bounds__(PT, 2) void gemm_i8_kernel(I8Args a) {
         if (i % 4 == 2) copy_x(1, to, i / 4);
         if (i % 4 == 3) copy_w(1, to, i / 4);
     }
-    wait_copies<6>();                 // (as in front of every tile's epilogue)
+    wait_copies<8>();                 // (as in front of every tile's epilogue)
     const int col = lane & 15, g4 = lane >> 4, group = w >> 2, q = w & 3;
     int stored = 0;                                                 // stores behind the last tile
     unsigned which = 0;                                             // the half of buf that holds the step
@@ -217,7 +217,7 @@ __global__ __launch_bounds__(PT, 2) void gemm_i8_kernel(I8Args a) {
         for (int i = 0; i < 2 * NB * 4 * NT; ++i) (&acc[0][0][0][0])[i] = v4i{0, 0, 0, 0};
         const unsigned char* A = buf + (64 * group + col) * KS;
         const unsigned char* B = buf + 2 * HALF + (16 * NT * q + col) * KS;
-        v4i av[2][4], b0[2][NT], b1[2][NT];
+        v4i av[2][4], b[NB][2][NT];
         auto read_a = [&](int h) __attribute__((always_inline)) {
 #pragma unroll
             for (int mt = 0; mt < 4; ++mt) {
@@ -225,84 +225,74 @@ __global__ __launch_bounds__(PT, 2) void gemm_i8_kernel(I8Args a) {
                 av[1][mt] = *(const v4i*)(A + which + h * HALF + 2048 * mt + p1);
             }
         };
-        auto read_b = [&](v4i(&b)[2][NT], unsigned from, int h) __attribute__((always_inline)) {
+        auto read_b = [&](int h) __attribute__((always_inline)) {
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
-                b[0][nt] = *(const v4i*)(B + from + h * HALF + 2048 * nt + p0);
-                b[1][nt] = *(const v4i*)(B + from + h * HALF + 2048 * nt + p1);
+                b[h][0][nt] = *(const v4i*)(B + which + h * HALF + 2048 * nt + p0);
+                b[h][1][nt] = *(const v4i*)(B + which + h * HALF + 2048 * nt + p1);
             }
         };
-        auto multiply = [&](v4i(&c)[4][NT], const v4i(&b)[2][NT]) __attribute__((always_inline)) {
-            __builtin_amdgcn_s_setprio(1);
+        auto multiply = [&](v4i(&c)[NB][4][NT]) __attribute__((always_inline)) {
 #pragma unroll
             for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-                for (int nt = 0; nt < NT; ++nt)
+                for (int h = 0; h < NB; ++h)
 #pragma unroll
-                    for (int mt = 0; mt < 4; ++mt) c[mt][nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[ks][mt], b[ks][nt], c[mt][nt], 0, 0, 0);
-            __builtin_amdgcn_s_setprio(0);
+                    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                        for (int mt = 0; mt < 4; ++mt) c[h][mt][nt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[ks][mt], b[h][ks][nt], c[h][mt][nt], 0, 0, 0);
         };
-        // One K step.  Phase by phase: read, request, wait (12 requests are younger than what the next phase reads), barrier, multiply, barrier.  c holds the
-        // step's first token half on entry; the next step's goes to d, whose second half is used up by then.
-        auto settle = [&](int i, auto p_) __attribute__((always_inline)) {
-            constexpr int p = decltype(p_)::value;
-            if (p < 3 && i == 0) wait_copies<63>();
-            else if ((p == 3 ? i == 0 : p < 2 && i == 1) && stored) {     // requested before the last tile's stores: these may be under way still
-                if (stored >= 16) wait_copies<12 + 16>();
-                else if (stored >= 8) wait_copies<12 + 8>();
-                else if (stored >= 4) wait_copies<12 + 4>();
-                else wait_copies<12>();
-            } else wait_copies<12>();
+        // Requests come in the order x0 w0 x1 w1 (halves of a step), a phase's as soon as every wave has read what they replace; eight are younger than what the
+        // next phase reads.  `late`: what the phase reads was requested before the last tile's stores, which may be under way still.
+        auto settle = [&](bool late) __attribute__((always_inline)) {
+            if (late && stored) {
+                if (stored >= 16) wait_copies<8 + 16>();
+                else if (stored >= 8) wait_copies<8 + 8>();
+                else if (stored >= 4) wait_copies<8 + 4>();
+                else wait_copies<8>();
+            } else wait_copies<8>();
             step_barrier();
         };
-        typedef std::integral_constant<int, 0> P0;
-        typedef std::integral_constant<int, 1> P1;
-        typedef std::integral_constant<int, 2> P2;
-        typedef std::integral_constant<int, 3> P3;
-        auto step = [&](int i, v4i(&c)[2][NT], v4i(&d)[2][NT]) __attribute__((always_inline)) {
-            const bool live = V == steps || i < steps;
-            const int k = i + 2 < V ? i + 2 : i + 2 - V;
+        auto step = [&](auto edge_, int i) __attribute__((always_inline)) {
+            constexpr bool EDGE = decltype(edge_)::value;              // (the first two steps and the last two: the others hold no branch)
+            const bool live = !EDGE || V == steps || i < steps;
+            const int k = !EDGE || i + 2 < V ? i + 2 : i + 2 - V;
             read_a(0);
-            if (i == V - 2) point(u, more);
-            if (i == 0) copy_side(t);                               // (every wave is past the last tile's epilogue)
-            copy_x(0, which, k);
-            settle(i, P0());
-            if (live) multiply(acc[0][0], c);
-            step_barrier();
-
-            if (NB == 2) read_b(d, which, 1);
-            copy_w(0, which, k);
-            settle(i, P1());
-            if (NB == 2 && live) multiply(acc[0][NB - 1], d);
+#pragma unroll
+            for (int h = 0; h < NB; ++h) read_b(h);
+            if (!EDGE || i) copy_w(1, which ^ PBUF, !EDGE || i + 1 < V ? i + 1 : i + 1 - V);
+            if (EDGE && i == 0) {                                   // (all of the first step has landed)
+                wait_copies<63>();
+                step_barrier();
+            } else settle(EDGE && i == 1);
+            if (live) multiply(acc[0]);
             step_barrier();
 
             read_a(1);
+            if (EDGE && i == 0) copy_side(t);                       // (every wave is past the last tile's epilogue)
+            if (EDGE && i == V - 2) point(u, more);
+            copy_x(0, which, k);
+            copy_w(0, which, k);
             copy_x(1, which, k);
-            settle(i, P2());
-            if (NB == 2 && live) multiply(acc[1][NB - 1], d);
-            step_barrier();
-
-            if (i + 1 < V) read_b(d, which ^ PBUF, 0);
-            copy_w(1, which, k);
-            settle(i, P3());
-            if (live) multiply(acc[1][0], c);
+            settle(EDGE && i == 0);
+            if (live) multiply(acc[1]);
             step_barrier();
             which ^= PBUF;
         };
-        step_barrier();                                             // every wave's requests for the first phases have landed
-        read_b(b0, which, 0);
-        wait_copies<63>();
-        step_barrier();
+        typedef std::integral_constant<bool, true> Edge;
+        typedef std::integral_constant<bool, false> Inner;
+        step_barrier();                                             // every wave's requests for the first step have landed
         if (group) step_barrier();
         int i = 0;
-        for (; i + 1 < V; i += 2) {
-            step(i, b0, b1);
-            step(i + 1, b1, b0);
-        }
-        if (i < V) step(i, b0, b1);
+        do {
+            if (i == 2)
+                for (; i + 2 < V; ++i) step(Inner(), i);
+            step(Edge(), i++);
+        } while (i < V);
         if (!group) step_barrier();
-        // (what the next tile's first step reads, and the first token half of its second; the stores below are younger)
-        wait_copies<6>();
+        copy_w(1, which ^ PBUF, 1);
+        // (what the next tile's first step reads; the stores below are younger)
+        wait_copies<8>();
         const int lane = fresh_lane(), col = lane & 15, g = lane >> 4;
         stored = 0;
 #pragma unroll

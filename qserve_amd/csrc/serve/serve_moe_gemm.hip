@@ -20,13 +20,12 @@ constexpr int KS = 64;       // reduction elements per step
 
 // Tiles of 256 weight rows x 256 slots (128 or 64 where an expert has no more left).  Bound by the matrix cores.
 //
-// Eight waves, two per SIMD: waves 0 - 3 and 4 - 7 are half a phase apart, so that one of a SIMD's two always multiplies while the other reads
-// its next operands.  A K step of 64 has four phases, one per quarter of the tile (halves of 128 rows x halves of 128 slots; in each a wave has 64
-// rows x 32 slots: 16 instructions); a phase reads ONE operand half (8 or 4 reads of 16 bytes a lane), requests the same half of the step after the
-// next one into the place that the half read a phase earlier left (global_load_lds, whole 128-byte lines of a row; pieces permuted by the row's number:
-// 16-byte reads without bank conflicts), and waits for what the next phase reads, which was requested seven phases before: 96 - 112 KiB in flight
-// a CU, no wait for the youngest requests.  Every wave issues the same requests in every phase - of rows that a tile does not have with no
-// lane active - so that the counted waits hold whatever the tile's size.
+// Eight waves, two per SIMD: waves 0 - 3 and 4 - 7 are half a phase apart, so that one of a SIMD's two always multiplies while the other reads its next
+// operands.  A K step of 64 has two phases, one per half of the tile's rows; in each a wave has 64 rows x 64 slots: 32 instructions.  The first reads a weight half
+// and both input halves (16 reads of 16 bytes a lane), the second the other weight half (8).  What every wave has read is requested anew for the step after
+// the next (global_load_lds, whole 128-byte lines of a row; pieces permuted by the row's number: 16-byte reads without bank conflicts), and a phase waits
+// for what the next one reads, which was requested three phases before: 64 - 112 KiB in flight a CU, no wait for the youngest requests.  Every wave issues the
+// same requests in every phase - of rows that a tile does not have with one lane active - so that the counted waits hold whatever the tile's size.
 //
 // Workgroups are persistent (one per CU): each finds its tiles from the experts' offsets - no tile list, no count reaches the host -, the last
 // two steps of a tile request the first two of the next one, so the epilogue's stores have something to hide behind.  An XCD's workgroups walk
@@ -35,13 +34,16 @@ constexpr int KS = 64;       // reduction elements per step
 // halves where at most half of its 32 workgroups have one, into quarters where at most a quarter have: with more than half nothing is cut, and
 // fewer than eight tiles leave workgroups idle.  The XCDs' shares are ceil(tiles / 8) each, so the last of them can be short or empty.
 //
-// Measured (MI355X, one product, the form before -> now in one call; before: eight waves in step, one barrier and a wait for every request per K step, rows
-// first): 32768 slots x 4096 x 4096 1014 -> 866 us (1270 TFLOP/s; hipBLASLt's dense product of that size 740), 28480 slots over 32 experts gated
-// 5504 x 4096 1380 -> 1230 (1045), 4096 x 2752 686 -> 587 (1095), 32768 over 16 of 1408 x 2048 204 -> 203, 2048 x 1408 201 -> 185, 8188 over 16 gated 2816 x 2048
-// 118 -> 115, 2048 x 1408 63.6 -> 64.5, 1300 over 16 of these 44.4 -> 42.4, 28.9 -> 29.8.  Small layers, both products with sort and sum, weights out of memory / left in the caches by the call before: 4
-// gated of 2048 x 1408, 1024 slots 84 -> 75 / 67 -> 75, 8 of them, 1200 92 -> 83 / 72 -> 81, 8 of 1024 x 512 49 -> 46 / 40 -> 45, 4 of 512 x 2048 63 -> 57 / 45 -> 56:
-// a layer's weights are in the caches only where the whole model is one small layer; from 4096 x 2752 on 0.77 - 0.93 of before either way.  A K step takes 1.5 us, which is the card's power: the same
-// instructions on constant data take 1.1.  How far ahead the requests run (3 - 7 phases) and bands of 4 - 12 make no difference.
+// Measured (MI355X, one product out of memory, us, the form before -> now in one call; before: four phases of a quarter each, conditions in every step): 32768 slots of one
+// expert of 4096 x 4096 835 -> 745 (1480 TFLOP/s; hipBLASLt's dense product of that size 700), 890 slots for each of 32 experts of 5504 x 4096 1200 -> 1114 (1155),
+// 2048 of 16 of 1408 x 2048 171 -> 159, of 2048 x 1408 172 -> 164, 550 of 16 of 2816 x 2048 138 -> 124, 512 107 -> 101, 300 94 -> 84; of 64 - 128 slots the same (the weights out
+// of memory).  The card's power bounds it: it holds 1.5 GHz over random numbers and 2.1 over ones (745 -> 620 us).  What counts there is cycles, not bytes: the branches
+// that a step held for the first and the last ones alone took 8 % (they are the forms with EDGE now), halving the barriers 2 %; operands that never miss L2
+// give 4 %, requests and reads left out altogether 18 and 8 %.  Eight waves without the half phase between them 785, four waves of 128 x 128 970 (one wave a SIMD has nothing
+// beside its own barriers and requests); tiles of 192 rows cost 0.89 of 256 (a step's time is its requests and reads as much as its products); another order of the
+// matrix instructions, a raised priority and requests without masks: no difference.
+// Small layers, both products with sort and sum, weights out of memory / left in the caches by the call before: 4 gated of 2048 x 1408, 1024 slots 75 / 75 us, 8 of
+// them, 1200 83 / 81, 8 of 1024 x 512 46 / 45, 4 of 512 x 2048 57 / 56 (before this set of forms).
 constexpr int PR = 256, PS = 256, PWAVES = 8, PT = 64 * PWAVES;
 constexpr int PBUF = (PR + PS) * 128;               // bytes of one K step
 constexpr int HALF = 128 * 128;                     // of an operand half of it
@@ -323,7 +325,7 @@ __global__ __launch_bounds__(PT, 2) void grouped_gemm_persistent_kernel(GroupedA
         if (i % 4 == 2) copy_x(1, to, i / 4);
         if (i % 4 == 3) copy_w(1, to, i / 4);
     }
-    wait_copies<6>();                 // (as in front of every tile's epilogue)
+    wait_copies<8>();                 // (as in front of every tile's epilogue)
     const int col = lane & 15, g4 = lane >> 4, group = w >> 2, q = w & 3;
     const bool wide = a.N % 16 == 0;
     int stored = 0;                                                 // stores behind the last tile, at least
@@ -347,7 +349,7 @@ __global__ __launch_bounds__(PT, 2) void grouped_gemm_persistent_kernel(GroupedA
         for (int i = 0; i < NA * NB * 4 * NT; ++i) (&acc[0][0][0][0])[i] = v4f{0.f, 0.f, 0.f, 0.f};
         const unsigned char* A = buf + (64 * group + col) * 128;
         const unsigned char* B = buf + 2 * HALF + (16 * NT * q + col) * 128;
-        v4u av[2][4], b0[2][NT], b1[2][NT];
+        v4u av[2][4], b[NB][2][NT];
         auto read_a = [&](int h) __attribute__((always_inline)) {
 #pragma unroll
             for (int mt = 0; mt < 4; ++mt) {
@@ -355,90 +357,80 @@ __global__ __launch_bounds__(PT, 2) void grouped_gemm_persistent_kernel(GroupedA
                 av[1][mt] = *(const v4u*)(A + which + h * HALF + 2048 * mt + p1);
             }
         };
-        auto read_b = [&](v4u(&b)[2][NT], unsigned from, int h) __attribute__((always_inline)) {
+        auto read_b = [&](int h) __attribute__((always_inline)) {
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
-                b[0][nt] = *(const v4u*)(B + from + h * HALF + 2048 * nt + p0);
-                b[1][nt] = *(const v4u*)(B + from + h * HALF + 2048 * nt + p1);
+                b[h][0][nt] = *(const v4u*)(B + which + h * HALF + 2048 * nt + p0);
+                b[h][1][nt] = *(const v4u*)(B + which + h * HALF + 2048 * nt + p1);
             }
         };
-        auto multiply = [&](v4f(&c)[4][NT], const v4u(&b)[2][NT]) __attribute__((always_inline)) {
-            __builtin_amdgcn_s_setprio(1);
+        auto multiply = [&](v4f(&c)[NB][4][NT]) __attribute__((always_inline)) {
 #pragma unroll
             for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-                for (int nt = 0; nt < NT; ++nt)
+                for (int h = 0; h < NB; ++h)
 #pragma unroll
-                    for (int mt = 0; mt < 4; ++mt)
-                        c[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, av[ks][mt]), __builtin_bit_cast(bf8, b[ks][nt]), c[mt][nt], 0, 0, 0);
-            __builtin_amdgcn_s_setprio(0);
+                    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                        for (int mt = 0; mt < 4; ++mt)
+                            c[h][mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, av[ks][mt]), __builtin_bit_cast(bf8, b[h][ks][nt]), c[h][mt][nt], 0, 0, 0);
         };
-        // One K step.  Phase by phase: read, request, wait (12 requests are younger than what the next phase reads), barrier, multiply, barrier.  c holds the
-        // step's first slot half on entry; the next step's goes to d, whose second half is used up by then.
-        auto settle = [&](int i, auto p_) __attribute__((always_inline)) {
-            constexpr int p = decltype(p_)::value;
-            if (p < 3 && i == 0) wait_copies<63>();
-            else if ((p == 3 ? i == 0 : p < 2 && i == 1) && stored) {     // requested before the last tile's stores: these may be under way still
-                if (stored >= 16) wait_copies<12 + 16>();
-                else if (stored >= 8) wait_copies<12 + 8>();
-                else if (stored >= 4) wait_copies<12 + 4>();
-                else wait_copies<12>();
-            } else wait_copies<12>();
+        // Requests come in the order x0 w0 x1 w1 (halves of a step), a phase's as soon as every wave has read what they replace; eight are younger than what the
+        // next phase reads.  `late`: what the phase reads was requested before the last tile's stores, which may be under way still.
+        auto settle = [&](bool late) __attribute__((always_inline)) {
+            if (late && stored) {
+                if (stored >= 16) wait_copies<8 + 16>();
+                else if (stored >= 8) wait_copies<8 + 8>();
+                else if (stored >= 4) wait_copies<8 + 4>();
+                else wait_copies<8>();
+            } else wait_copies<8>();
             step_barrier();
         };
-        typedef std::integral_constant<int, 0> P0;
-        typedef std::integral_constant<int, 1> P1;
-        typedef std::integral_constant<int, 2> P2;
-        typedef std::integral_constant<int, 3> P3;
-        auto step = [&](int i, v4u(&c)[2][NT], v4u(&d)[2][NT]) __attribute__((always_inline)) {
-            const bool live = V == steps || i < steps;
-            const int k = i + 2 < V ? i + 2 : i + 2 - V;
+        auto step = [&](auto edge_, int i) __attribute__((always_inline)) {
+            constexpr bool EDGE = decltype(edge_)::value;              // (the first two steps and the last two: the others hold no branch)
+            const bool live = !EDGE || V == steps || i < steps;
+            const int k = !EDGE || i + 2 < V ? i + 2 : i + 2 - V;
             read_a(0);
-            if (i == V - 2) point(u, more, early);
-            copy_x(0, which, k);
-            settle(i, P0());
-            if (live) multiply(acc[0][0], c);
-            step_barrier();
-
-            if (NB == 2) read_b(d, which, 1);
-            copy_w(0, which, k);
-            settle(i, P1());
-            if (NB == 2 && live) multiply(acc[0][NB - 1], d);
+#pragma unroll
+            for (int h = 0; h < NB; ++h) read_b(h);
+            if (!EDGE || i) copy_w(1, which ^ PBUF, !EDGE || i + 1 < V ? i + 1 : i + 1 - V);
+            if (EDGE && i == 0) {                                           // (all of the first step has landed)
+                wait_copies<63>();
+                step_barrier();
+            } else settle(EDGE && i == 1);
+            if (live) multiply(acc[0]);
             step_barrier();
 
             if (NA == 2) read_a(1);
+            if (EDGE && i == V - 2) point(u, more, early);
+            copy_x(0, which, k);
+            copy_w(0, which, k);
             copy_x(1, which, k);
-            settle(i, P2());
-            if (NA == 2 && NB == 2 && live) multiply(acc[NA - 1][NB - 1], d);
-            step_barrier();
-
-            if (i + 1 < V) read_b(d, which ^ PBUF, 0);
-            copy_w(1, which, k);
-            if (early && i == 0) look();
-            if (early && i == 1 && more && u.ns > 0) {
+            if (EDGE && early && i == 0) look();
+            if (EDGE && early && i == 1 && more && u.ns > 0) {
                 const int lane = fresh_lane();
                 const int s = x_row(u, 128 * ((lane >> 4) & 1) + 16 * w + (lane & 15));
                 lds_copy4(ahead0, LISTED ? (const void*)(a.x_index + s) : (const void*)(a.order + s));
             }
-            settle(i, P3());
-            if (NA == 2 && live) multiply(acc[NA - 1][0], c);
+            settle(EDGE && i == 0);
+            if (NA == 2 && live) multiply(acc[NA - 1]);
             step_barrier();
             which ^= PBUF;
         };
         step_barrier();                                             // every wave's requests for the first phases have landed
-        read_b(b0, which, 0);
-        wait_copies<63>();
-        step_barrier();
         if (group) step_barrier();
+        typedef std::integral_constant<bool, true> Edge;
+        typedef std::integral_constant<bool, false> Inner;
         int i = 0;
-        for (; i + 1 < V; i += 2) {
-            step(i, b0, b1);
-            step(i + 1, b1, b0);
-        }
-        if (i < V) step(i, b0, b1);
+        do {
+            if (i == 2)
+                for (; i + 2 < V; ++i) step(Inner(), i);
+            step(Edge(), i++);
+        } while (i < V);
         if (!group) step_barrier();
-        // (what the next tile's first step reads, and the first slot half of its second; the stores below are younger)
-        wait_copies<6>();
+        copy_w(1, which ^ PBUF, 1);
+        // (what the next tile's first step reads; the stores below are younger)
+        wait_copies<8>();
         const int lane = fresh_lane(), col = lane & 15;
         const int n0 = t.n0 + 64 * group, sl0 = 16 * NT * q;
         stored = 0;

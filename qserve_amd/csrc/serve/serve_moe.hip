@@ -414,7 +414,7 @@ __global__ __launch_bounds__(NT) void moe_down_vec_kernel(T* __restrict__ y, con
 // down) against the form it replaces, which kept weight rows in registers and paid a wave-wide sum per token and row; 16 tokens with
 // gated units (184 + 92 MB) 42.6 / 26.1 -> 36.5 / 19.3 us (5.0 TB/s); one token 1446 / 3117 us (the per-token kernels) -> 14.0 / 8.8 us.
 // The sort, search and permutation launches in front of it (60 us a layer) are gone.  Streamed past the caches, the shared expert in the same
-// launch: 64 tokens 22.7 / 19.4 us (98 MB), 16 tokens gated 33.8 / 17.6 (196 / 98 MB, 5.7 TB/s), one token 15.3 / 9.5.
+// launch: 64 tokens 22.7 / 19.4 us (98 MB), 16 tokens gated 33.8 / 17.6 (196 / 98 MB, 5.7 TB/s), one token 15.3 / 9.5 (before its workgroups were the slots').
 // 32 rows: 16, more evenly spread over the CUs, read the inputs twice as often and are slower everywhere (64 tokens 24.7 / 25.7, 16 tokens 36.3 / 21.4,
 // one 18.7 / 11.7), and so are 64; rings twice as deep give no more.
 constexpr int XR = 32;               // weight rows per workgroup
@@ -433,6 +433,7 @@ struct ExpertArgs {
     bool wide;                       // out starts on 16 bytes
     bool stored;                     // gated units are made from their halves as a tensor would hold them
     bool once;                       // weights that one reading may stream past the caches
+    int by_slot;                     // workgroups by slot in place of expert (of this many experts; 0: by expert)
 };
 // An expert every token goes through, of sizes of its own: X row t, out row t in bfloat16, the bits that the products and the activation give one by one.
 // W NULL: none.  Alone it took four launches, three of them at 4 - 5 us whatever they read (16 experts of 2048 x 1408 and one more, top 4, with the router,
@@ -514,7 +515,7 @@ __global__ __launch_bounds__(NT, 2) void expert_rows_kernel(ExpertArgs a, Shared
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r0 = blockIdx.x * XR;
     if (sh.W && blockIdx.y == 0) {                                                 // (first: it has the most inputs)
         if (r0 >= sh.rows) return;
-        const ExpertArgs b = {sh.out, sh.X, sh.W, nullptr, nullptr, nullptr, nullptr, sh.n, 1, sh.rows, sh.K, a.limit, sh.wide, true, false};
+        const ExpertArgs b = {sh.out, sh.X, sh.W, nullptr, nullptr, nullptr, nullptr, sh.n, 1, sh.rows, sh.K, a.limit, sh.wide, true, false, 0};
         auto chunk = [&](int c0, auto once) __attribute__((always_inline)) {
             constexpr bool ONCE = decltype(once)::value;
             const int c = min(32, sh.n - c0);
@@ -536,7 +537,12 @@ __global__ __launch_bounds__(NT, 2) void expert_rows_kernel(ExpertArgs a, Shared
         return;
     }
     if (r0 >= a.rows) return;
-    const int e = blockIdx.y - (sh.W ? 1 : 0), rows_here = min(XR, a.rows - r0);
+    const int which = blockIdx.y - (sh.W ? 1 : 0), rows_here = min(XR, a.rows - r0);
+    int e = which;
+    if (a.by_slot) {                                                               // the expert of slot `which`, by its first slot
+        e = a.idx[which];
+        if ((unsigned)e >= (unsigned)a.by_slot) return;
+    }
     const bf16_t* W0 = a.W + ((size_t)e * a.rows + r0) * (size_t)a.K;
     unsigned char* ring = rings + w * XRING;
     // `count` inputs: X row by row_of(i), output row (and weight) by slot_of(i)
@@ -599,6 +605,7 @@ __global__ __launch_bounds__(NT, 2) void expert_rows_kernel(ExpertArgs a, Shared
             at += __popcll(hit[q]);
         }
         __syncthreads();
+        if (a.by_slot && list[0] != which) return;                                 // (an earlier slot's workgroups do this expert)
         walk(count, [&](int i) { return (int64_t)((n0 + list[i]) / a.div); },
              [&](int i, int64_t& slot, float& iw) {
                  slot = n0 + list[i];
@@ -678,7 +685,13 @@ static int launch_expert_rows(const char* what, ExpertArgs a, int n_experts, int
     a.wide = (uintptr_t)a.out % 16 == 0;
     a.once = !kept && streams_once(a.W, (int64_t)n_experts * a.rows, a.K);
     sh.once = !kept && streams_once(sh.W, sh.rows, sh.K);
-    const dim3 grid(((sh.W && sh.rows > a.rows ? sh.rows : a.rows) + XR - 1) / XR, n_experts + (sh.W ? 1 : 0)), block(NT);
+    // Few slots: workgroups by slot, so that those of experts without one are not there.  Measured for both products of a token, us before and after: 1 token of 4 of
+    // 16 experts of 2048 x 1408 gated with a shared one 24.2 -> 20.3 (1496 and 1088 workgroups, of which 440 and 320 have rows), 2 tokens 29.2 -> 27.5, 1 token of
+    // 8 of 64 of 2048 x 768 35.0 -> 21.1.  The line: slots past half of the experts gain little and lose up to 4 % (3 tokens of the first: 37.3 -> 38.8, the empty
+    // workgroups between the others' are then few), and a grid that fits the chip at once loses .2 us to the load of the slot's expert.
+    const int tiles = ((sh.W && sh.rows > a.rows ? sh.rows : a.rows) + XR - 1) / XR;
+    a.by_slot = a.idx && a.n <= XLIST && 2 * a.n <= n_experts && (int64_t)n_experts * tiles > 512 ? n_experts : 0;
+    const dim3 grid(tiles, (a.by_slot ? a.n : n_experts) + (sh.W ? 1 : 0)), block(NT);
     if (float_out) hipLaunchKernelGGL((expert_rows_kernel<ACT_NONE, true>), grid, block, 0, (hipStream_t)stream, a, sh);
     else if (act == ACT_RELU_SQ) hipLaunchKernelGGL((expert_rows_kernel<ACT_RELU_SQ, false>), grid, block, 0, (hipStream_t)stream, a, sh);
     else if (act == ACT_GLU) hipLaunchKernelGGL((expert_rows_kernel<ACT_GLU, false>), grid, block, 0, (hipStream_t)stream, a, sh);
@@ -688,14 +701,14 @@ static int launch_expert_rows(const char* what, ExpertArgs a, int n_experts, int
 extern "C" int qsv_expert_rows(void* out, const void* X, const int64_t* x_index, int div, const void* W, const int64_t* offsets,
                                int n_experts, int rows, int K, int act, float limit, const float* in_weight, void* stream) {
     QSV_REQUIRE(offsets, "qsv_expert_rows: bad arguments");
-    const ExpertArgs a = {out, (const bf16_t*)X, (const bf16_t*)W, nullptr, x_index, offsets, in_weight, 0, div, rows, K, limit, false, false, false};
+    const ExpertArgs a = {out, (const bf16_t*)X, (const bf16_t*)W, nullptr, x_index, offsets, in_weight, 0, div, rows, K, limit, false, false, false, 0};
     return launch_expert_rows("qsv_expert_rows", a, n_experts, act, false, stream);
 }
 extern "C" int qsv_expert_slots(void* out, int float_out, const void* X, int div, const void* W, const int32_t* idx, int n, int n_experts, int rows,
                                 int K, int act, float limit, const float* in_weight, void* stream) {
     QSV_REQUIRE(idx && n >= 0 && (!float_out || act == ACT_NONE), "qsv_expert_slots: bad arguments");
     if (n == 0) return QSV_OK;
-    const ExpertArgs a = {out, (const bf16_t*)X, (const bf16_t*)W, idx, nullptr, nullptr, in_weight, n, div, rows, K, limit, false, false, false};
+    const ExpertArgs a = {out, (const bf16_t*)X, (const bf16_t*)W, idx, nullptr, nullptr, in_weight, n, div, rows, K, limit, false, false, false, 0};
     return launch_expert_rows("qsv_expert_slots", a, n_experts, act, float_out != 0, stream);
 }
 // ... and, with sh_W, every token's row of X through a shared expert of sh_rows x sh_K in the same launch: sh_out [n / div, sh_rows (/ 2 for gated units)]
@@ -709,7 +722,7 @@ static int expert_slots_shared(const char* what, bool kept, void* out, int float
         QSV_REQUIRE(act == ACT_NONE || act == ACT_RELU_SQ || sh_rows % 2 == 0, "%s: %d rows of gated units", what, sh_rows);
     }
     if (n == 0) return QSV_OK;
-    const ExpertArgs a = {out, (const bf16_t*)X, (const bf16_t*)W, idx, nullptr, nullptr, in_weight, n, div, rows, K, limit, false, false, false};
+    const ExpertArgs a = {out, (const bf16_t*)X, (const bf16_t*)W, idx, nullptr, nullptr, in_weight, n, div, rows, K, limit, false, false, false, 0};
     const SharedArgs sh = {sh_out, (const bf16_t*)sh_X, (const bf16_t*)sh_W, sh_n, sh_rows, sh_K, (uintptr_t)sh_out % 16 == 0, false};
     return launch_expert_rows(what, a, n_experts, act, float_out != 0, stream, sh_W ? sh : SharedArgs{}, kept);
 }

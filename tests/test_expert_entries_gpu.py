@@ -65,3 +65,36 @@ def test_runs_that_the_caller_sorted(counts, top, N, K, indexed, weighted, act, 
     check(lib().qsv_expert_rows(out.data_ptr(), X.data_ptr(), None if order is None else order.data_ptr(), top, W.data_ptr(), offsets.data_ptr(), len(counts), N, K,
                                 act, limit, None if wt is None else wt.data_ptr(), torch.cuda.current_stream().cuda_stream), "expert_rows")
     _close(out, ref, K)
+
+
+# As many slots as half of the experts (workgroups by slot) and one more (by expert), against the same slots among enough without an expert to be done by expert
+# whatever their number; an expert twice, slots without one, rows that do not fill 32, the shared expert's rows fewer and more than the others'
+@pytest.mark.parametrize("n, E, top, N, K, shared", [(1, 1030, 1, 34, 64, 0), (8, 16, 4, 1066, 136, 1100), (9, 17, 3, 1066, 136, 700), (9, 18, 3, 1066, 136, 700), (40, 80, 8, 256, 1032, 0)])
+@ACTS
+def test_few_slots(n, E, top, N, K, shared, act, limit):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    g = torch.Generator().manual_seed(n + E)
+    idx = torch.randint(0, E, (n,), generator=g, dtype=torch.int32)
+    if n > 4:
+        idx[[1, 4]] = E - 1
+        idx[2], idx[3] = -1, E
+    T = (n + top - 1) // top
+    X = torch.randn(3 * E, K, generator=g).bfloat16().cuda()
+    W, sW = ((torch.randn(e, r, K, generator=g) / K ** 0.5).bfloat16().cuda() for e, r in ((E, N), (1, max(shared, 1))))
+    out_of = lambda rows, r: torch.full((rows, r // 2 if act >= 2 else r), float("nan"), dtype=torch.bfloat16, device="cuda")          # noqa: E731
+
+    def run(idx):
+        out, own, s = out_of(len(idx), N), out_of(3 * E, shared), torch.cuda.current_stream().cuda_stream
+        args = out.data_ptr(), 0, X.data_ptr(), top, W.data_ptr(), idx.data_ptr(), len(idx), E, N, K, act, limit, None
+        if shared:
+            check(lib().qsv_expert_slots_shared(*args, own.data_ptr(), X.data_ptr(), sW.data_ptr(), T, shared, K, s), "expert_slots_shared")
+        else:
+            check(lib().qsv_expert_slots(*args, s), "expert_slots")
+        return out[:n], own[:T]
+
+    few, few_shared = run(idx.cuda())
+    by_expert, shared_too = run(torch.cat([idx, torch.full((2 * E,), -1, dtype=torch.int32)]).cuda())
+    there = ((idx >= 0) & (idx < E)).cuda()
+    assert not few[there].isnan().any() and few[~there].isnan().all()
+    assert torch.equal(few[there], by_expert[there]) and torch.equal(few_shared, shared_too)

@@ -70,6 +70,24 @@ __device__ __forceinline__ u32 unpack_hi(u32 raw, u32 s, u32 zb) {
     if (MODE == 1) u = vadd4(u * s, zb);
     return u;
 }
+// The same operand bytes where no byte product carries, 15 s <= 255: two 16-bit multiply-adds, one for the even and one for the odd bytes, whose wrapped sums end in
+// bits 0-7 and 8-15.  v_pk_mad_u16 issues at the full rate, v_mul_lo_u32 at a quarter of it: 11 cycles of 4 for both nibble halves of a word in place of 21.
+// (Measured where it is used.  Zeros and scales quantised as the method quantises them, to at most 119 in size before the second level, have s <= 16.)
+typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+struct Level2 {
+    us2 s, z, z8;                                    // [s, s], [z, z] and [z << 8, z << 8] of one channel
+};
+__device__ __forceinline__ bool level2_carries(u32 sdw) { return ((sdw + 0x6E6E6E6Eu) | sdw) & 0x80808080u; }   // a scale above 17 among four
+__device__ __forceinline__ Level2 level2_of(u32 sdw, u32 zdw, int byte) {
+    const u32 lo = 0x0C000C00u + 0x00010001u * byte, hi = 0x000C000Cu + 0x01000100u * byte;
+    return {__builtin_bit_cast(us2, __builtin_amdgcn_perm(0, sdw, lo)), __builtin_bit_cast(us2, __builtin_amdgcn_perm(0, zdw, lo)),
+            __builtin_bit_cast(us2, __builtin_amdgcn_perm(0, zdw, hi))};
+}
+__device__ __forceinline__ u32 unpack_level2(u32 raw, bool high, const Level2& q) {
+    if (high) raw >>= 4;
+    const us2 even = __builtin_bit_cast(us2, raw & 0x000F000Fu) * q.s + q.z, odd = __builtin_bit_cast(us2, raw & 0x0F000F00u) * q.s + q.z8;
+    return (__builtin_bit_cast(u32, even) & 0x00FF00FFu) | __builtin_bit_cast(u32, odd);
+}
 // fp32 epilogues with the reference's evaluation order (oracle/w4a8.py epilogue_*).
 // per-channel, w4a8_per_chn/gemm_cuda.cu:586-587: (acc * wscale) * ascale - w_sz * a_ssum.  `fma` selects the CONVENTION
 // (qs_set_gemm_epilogue, include/qserve_amd.h): 0 = every operation rounded separately (the library's default; what the

@@ -25,7 +25,7 @@
 
 // A/B switches (qs_set_gemm_variant(5000 + bits); every setting computes the same results):
 //   1 = weight DMA with the default cache policy everywhere, 2 = non-temporal everywhere (default: non-temporal unless several
-//       token blocks share the weight bytes of a channel block and N <= 8192 - see launch_ring and `issue`)
+//       token blocks share the weight bytes of a channel block and N <= 8192 - see launch_ring and `issue`; the host's switch)
 //   4 / 8 = (QS_TIMING libraries only) no cross-group reduction / leave behind the k loop: the price of the tail (round 5)
 //   32 / 64 = (libraries built with -DQS_TIMING only; ignored by the shipped library) timing only, WRONG RESULTS: no MFMA /
 //        no LDS operand reads (what is left is the DMA + barrier pipeline:
@@ -80,6 +80,13 @@ constexpr int ring_gstage() {
     return 16 * MT * 64 + WN * 2048 + (MODE == 1 ? 2 * (WN > 2 ? 256 : 128) : 0);
 }
 
+// ring slots of a group where the reduction is long enough: see launch_ring_as
+template <int MT, int WN, int MODE>
+constexpr int ring_depth() {
+    constexpr int d = 144 * 1024 / (8 / WN * ring_gstage<MT, WN, MODE>());
+    return d > 5 ? 5 : d < 3 ? 3 : d;
+}
+
 // workgroup -> (channel block, token block, K slice); token blocks of one channel block sit on ONE XCD (b % 8) so that the
 // weights are fetched from HBM once and re-served by that XCD's L2; K slices (ksplit > 1) likewise
 struct RingCoords {
@@ -131,8 +138,8 @@ __device__ __forceinline__ RingCoords ring_coords(int b, int N, int wn, int mblo
     return c;
 }
 
-// The GEMM proper.
-template <int MT, int WN, int MODE, int OUTK, bool KSPLIT>
+// The GEMM proper.  NT: non-temporal weight requests (`issue`).
+template <int MT, int WN, int MODE, int OUTK, bool KSPLIT, bool NT>
 __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const uint8_t* __restrict__ W,
                                          const int8_t* __restrict__ zeros, const int8_t* __restrict__ scales8,
                                          const __half* __restrict__ wscales, const __half* __restrict__ ascales,
@@ -232,7 +239,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
     };
     // weights that exactly ONE workgroup reads (one token block per channel block) are non-temporal (MI355X_MICROARCH.md
     // "nt-weights": issued -> landed -18 %); with several token blocks the same bytes are wanted again by the neighbours on the
-    // XCD a moment later, and a streamed line may be gone by then: default policy there (launch_ring sets flags bit 0; round 4,
+    // XCD a moment later, and a streamed line may be gone by then: default policy there (launch_ring;
     // in-run A/B at M = 64: qkv (2 token blocks) 8.45 -> 7.84 us, o (4) 6.66 -> 6.48, down (2 x 4 K slices) 14.05 -> 13.98,
     // gate_up (1 block) 16.97 -> 17.05 the other way; M = 128: qkv 11.70 -> 11.28, o 7.94 -> 7.70).  Measured exception: the
     // 28 672-channel gate_up stream stays 2-3 % faster non-temporal at every M, shared or not (M = 128: 24.56 vs 25.06, g128 35.24
@@ -250,7 +257,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
             const void* sb = p_isw[j] ? static_cast<const void*>(W + (size_t)u * 1024)
                                       : static_cast<const void*>(A + (size_t)(u - hf) * 64);   // the pair's line
             static_assert(MT % WN == 0, "piece kind must be a compile-time function of j");
-            if (j >= MT / WN && !(flags & 1)) dma16_nt(p_off[j], sb, dst + p_lds[j]);   // (p = wn + j*WN >= MT: a weight piece)
+            if (NT && j >= MT / WN) dma16_nt(p_off[j], sb, dst + p_lds[j]);   // (p = wn + j*WN >= MT: a weight piece)
             else dma16(p_off[j], sb, dst + p_lds[j]);
         }
         if (MODE == 1) {
@@ -309,7 +316,12 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
     // ---- prologue: stages 0..ns-2 in flight, operands of stage 0 in registers ---------------------------------------
     QS_STAMP(15);
     for (int j = 0; j < ns - 1; ++j)
-        if (j < nloc) issue(j, j);
+        if (j < nloc) {
+            issue(j, j);
+            // (128 cycles apart: the first stage's lines are then not queued behind the later ones' of other waves.  6144 x 4096, 1 / 16 tokens 6.44 / 7.04 ->
+            //  6.18 / 6.82 us, per group 9.13 / 9.42 -> 8.96 / 9.30)
+            __builtin_amdgcn_s_sleep(2);
+        }
     QS_STAMP(1);
     // Everything the k loop needs but the first requests do not - operand reader addresses, accumulators - is computed BEHIND
     // the prologue (round 4, timeline trace: the first request left 1 200-1 400 cycles after kernel entry; with two waves per
@@ -388,6 +400,21 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
         }
         return a;
     };
+    // per-group: the cheap form wherever no scale of the wave's 64 channels lets byte products carry
+    auto carries = [&](const Raw& q) { return MODE == 1 && __builtin_amdgcn_ballot_w64(level2_carries(q.sdw)) != 0; };
+    auto build_all = [&](const Raw& q, v4i (&a)[4]) __attribute__((always_inline)) {
+        if (MODE == 1 && !carries(q)) {
+#pragma unroll
+            for (int cl = 0; cl < 4; ++cl) {
+                const Level2 l2 = level2_of(q.sdw, q.zdw, cl);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) a[cl][e] = (int)unpack_level2((cl & 1) ? q.r[e].y : q.r[e].x, cl & 2, l2);
+            }
+        } else {
+#pragma unroll
+            for (int cl = 0; cl < 4; ++cl) a[cl] = build(q, cl);
+        }
+    };
 
     v4i acc[MT][4];
 #pragma unroll
@@ -413,15 +440,37 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
         const Raw q0 = read_raw(0);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) o0.b[mt] = read_b(0, mt);
-#pragma unroll
-        for (int cl = 0; cl < 4; ++cl) o0.a[cl] = build(q0, cl);
+        build_all(q0, o0.a);
     }
 
+    // (`steady`: the ring has its full depth and stage i + ns - 1 exists - nothing to ask)
+    constexpr int DEPTH = ring_depth<MT, WN, MODE>();
     // One round: MFMAs of stage i from `cur`; meanwhile operands of stage i+1 -> `nxt`, DMA of stage i+ns-1.
-    auto round = [&](int i, int slot, const Ops& cur, Ops& nxt) {
-        const int slot_n = slot + 1 == ns ? 0 : slot + 1;
-        const int slot_d = slot == 0 ? ns - 1 : slot - 1;
+    auto round = [&](int i, int slot, const Ops& cur, Ops& nxt, auto steady) __attribute__((always_inline)) {
+        constexpr bool STEADY = decltype(steady)::value;
+        const int ns_ = STEADY ? DEPTH : ns;
+        const int slot_n = slot + 1 == ns_ ? 0 : slot + 1;
+        const int slot_d = slot == 0 ? ns_ - 1 : slot - 1;
         Raw qn;
+        if constexpr (MT == 8 && MODE == 1) {
+            // one set of activation operands, each read again behind its last product: two sets and the cheap unpacking do not fit the registers (128 tokens of
+            // gate_up 30.2 us with two sets and the exact form, 28.7 with this; where half of the waves unpack later, so that a SIMD's two waves alternate, 33.7)
+            qn = read_raw(slot_n);
+            if (STEADY || i + ns - 1 < nloc) issue(i + ns - 1, slot_d);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+#pragma unroll
+                for (int cl = 0; cl < 4; ++cl)
+                    acc[mt][cl] = __builtin_amdgcn_mfma_i32_16x16x64_i8(cur.a[cl], o0.b[mt], acc[mt][cl], 0, 0, 0);
+                o0.b[mt] = read_b(slot_n, mt);
+                if (mt == 0) {
+                    build_all(qn, nxt.a);
+#pragma unroll
+                    for (int cl = 0; cl < 4; ++cl) asm volatile("" ::"v"(nxt.a[cl]));
+                }
+            }
+            return;
+        }
 #ifdef QS_TIMING
         const bool t_reads = !(flags & 64), t_mfma = !(flags & 32);   // timing builds only: results wrong by design
 #else
@@ -432,7 +481,27 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) nxt.b[mt] = read_b(slot_n, mt);
         }
-        if (i + ns - 1 < nloc) issue(i + ns - 1, slot_d);
+        if (STEADY || i + ns - 1 < nloc) issue(i + ns - 1, slot_d);
+        if (STEADY && MODE == 0) {
+            // the requests and the reads first, then one product after the other with the next operands' unpacking between them
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int cl = 0; cl < 4; ++cl)
+                    acc[mt][cl] = __builtin_amdgcn_mfma_i32_16x16x64_i8(cur.a[cl], cur.b[mt], acc[mt][cl], 0, 0, 0);
+            build_all(qn, nxt.a);
+            if (MT > 1) {
+                __builtin_amdgcn_sched_group_barrier(0x8, 4, 0);
+#pragma unroll
+                for (int x = 0; x < 4 * MT - 4; ++x) {
+                    __builtin_amdgcn_sched_group_barrier(0x2, MT > 1 ? (48 + 4 * MT - 5) / (4 * MT - 4) : 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            return;
+        }
         if (t_mfma) {
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
@@ -440,8 +509,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
                 for (int cl = 0; cl < 4; ++cl)
                     acc[mt][cl] = __builtin_amdgcn_mfma_i32_16x16x64_i8(cur.a[cl], cur.b[mt], acc[mt][cl], 0, 0, 0);
                 if (mt == 0) {
-#pragma unroll
-                    for (int cl = 0; cl < 4; ++cl) nxt.a[cl] = build(qn, cl);
+                    build_all(qn, nxt.a);
                 }
             }
             // Per-group (round 6): the operands built for the NEXT round must be finished INSIDE this round, under its MFMAs.  Left to
@@ -465,8 +533,24 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
         else if (young == 1) wait_vm<1 * NDMA>();
         else wait_vm<0>();
     };
-    int slot = 0;
-    for (int i = 0; i < nloc; i += 2) {               // two rounds per trip (operand registers ping-pong); nloc may be odd
+    int slot = 0, i = 0;
+    // Two rounds per trip (operand registers ping-pong).  While requests are left to make every wait is the same and nothing is asked inside a trip: with the
+    // general rounds below for all of them a round had twelve branches, between the barrier and the operands it needs.  Before and after, us: 33 tokens 12288 x 4096
+    // 11.6 -> 10.6, gate_up 28672 x 4096 17.2 -> 16.3, 128 tokens gate_up 27.4 -> 23.6, one token of 4096 x 11008 22.8 -> 18.0; per group 64 tokens gate_up 21.8 ->
+    // 19.7, 12288 x 4096 34.1 -> 29.1 with 256 (with the cheap unpacking; scales with carries 18.1 -> 17.1, 16 tokens of gate_up).
+    if (ns == DEPTH) {
+        for (; i + DEPTH < nloc; i += 2) {
+            wait_vm<(DEPTH - 3) * NDMA>();
+            raw_barrier();
+            round(i, slot, o0, o1, std::true_type());
+            slot = slot + 1 == DEPTH ? 0 : slot + 1;
+            wait_vm<(DEPTH - 3) * NDMA>();
+            raw_barrier();
+            round(i + 1, slot, o1, o0, std::true_type());
+            slot = slot + 1 == DEPTH ? 0 : slot + 1;
+        }
+    }
+    for (; i < nloc; i += 2) {                        // (nloc may be odd)
 #ifdef QS_RING_TRACE
         unsigned long long ta = __builtin_amdgcn_s_memtime();
 #endif
@@ -476,7 +560,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
         QS_ACC(t_wait, ta);
         ta = __builtin_amdgcn_s_memtime();
 #endif
-        round(i, slot, o0, o1);
+        round(i, slot, o0, o1, std::false_type());
 #ifdef QS_RING_TRACE
         QS_ACC(t_round, ta);
         ta = __builtin_amdgcn_s_memtime();
@@ -489,7 +573,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
             QS_ACC(t_wait, ta);
             ta = __builtin_amdgcn_s_memtime();
 #endif
-            round(i + 1, slot, o1, o0);
+            round(i + 1, slot, o1, o0, std::false_type());
 #ifdef QS_RING_TRACE
             QS_ACC(t_round, ta);
 #endif
@@ -757,7 +841,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
 // dequant of a weight byte serves 128 tokens, ring depth 3-4, reduction through LDS in two passes); WN units per workgroup;
 // KG = 8 / WN K-groups.
 // KSPLIT = false folds every K-slice path away (the un-split launches keep exactly their earlier code).
-template <int MT, int WN, int MODE, int OUTK, bool KSPLIT>
+template <int MT, int WN, int MODE, int OUTK, bool KSPLIT, bool NT>
 __global__ __launch_bounds__(512, 1) void w4a8_gemm_ring(const int8_t* __restrict__ A, const uint8_t* __restrict__ W,
                                                          const int8_t* __restrict__ zeros,
                                                          const int8_t* __restrict__ scales8,
@@ -769,23 +853,22 @@ __global__ __launch_bounds__(512, 1) void w4a8_gemm_ring(const int8_t* __restric
                                                          int* __restrict__ slabs, unsigned* __restrict__ counters,
                                                          int flags) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    ring_body<MT, WN, MODE, OUTK, KSPLIT>(A, W, zeros, scales8, wscales, ascales, wszs, assums, out, M, N, K, mblocks, ns,
+    ring_body<MT, WN, MODE, OUTK, KSPLIT, NT>(A, W, zeros, scales8, wscales, ascales, wszs, assums, out, M, N, K, mblocks, ns,
                                           ksplit_arg, slabs, counters, flags, smem);
 }
 
-template <int MT, int WN, int MODE, int OUTK, bool KSPLIT>
-int launch_ring(const int8_t* A, const uint8_t* W, const int8_t* zeros, const int8_t* scales8, const void* wscales,
+template <int MT, int WN, int MODE, int OUTK, bool KSPLIT, bool NT>
+int launch_ring_as(const int8_t* A, const uint8_t* W, const int8_t* zeros, const int8_t* scales8, const void* wscales,
                 const void* ascales, const void* wszs, const void* assums, void* out, int M, int N, int K,
                 int mblocks, int ksplit, int* slabs, unsigned* counters, hipStream_t stream) {
-    auto kern = w4a8_gemm_ring<MT, WN, MODE, OUTK, KSPLIT>;
+    auto kern = w4a8_gemm_ring<MT, WN, MODE, OUTK, KSPLIT, NT>;
     constexpr int KG = 8 / WN;
     constexpr int GSTAGE = ring_gstage<MT, WN, MODE>();
     // ring depth: as deep as 144 KiB of LDS allows, never deeper than a group's stage count + 1.  At most 5: every
     // stage layer carries 16 KiB of weights per CU, and beyond 4 layers (64 KiB per CU, 16 MB over the chip) in flight
     // the stream no longer gains while the pipeline fill gets longer (depth sweep 3 / 4 / 5 / 6 at M = 16: o 8.9 / 6.7 /
     // 6.45 / 6.66 us, gate_up 18.7 / 13.8 / 13.6 / 13.9 us; M = 64: o 9.2 / 7.1 / 6.74 / 6.96 us; depth 3 costs 25-40 %)
-    int ns = (144 * 1024) / (KG * GSTAGE);
-    if (ns > 5) ns = 5;
+    int ns = ring_depth<MT, WN, MODE>();
     const int nloc = (K / 64) / ksplit / KG;
     if (ns > nloc + 1) ns = nloc + 1;
     if (const int f = (g_ring_flags >> 8) & 7) {       // A/B: forced depth (sensitivity to the bytes in flight)
@@ -832,9 +915,17 @@ int launch_ring(const int8_t* A, const uint8_t* W, const int8_t* zeros, const in
                        reinterpret_cast<const __half*>(wscales), reinterpret_cast<const __half*>(ascales),
                        reinterpret_cast<const __half*>(wszs), reinterpret_cast<const __half*>(assums), out, M, N, K,
                        mblocks, ns, ksplit, slabs, counters,
-                       (g_ring_flags & ~(3 | 16 | 128 | 2048 | 4096)) | inject | (g_epi_fma ? 16 : 0) | (kxcd ? 2048 : 0) |
-                           ((g_ring_flags & 1) || (mblocks > 1 && N <= 8192 && !(g_ring_flags & 2)) ? 1 : 0));
+                       (g_ring_flags & ~(3 | 16 | 128 | 2048 | 4096)) | inject | (g_epi_fma ? 16 : 0) | (kxcd ? 2048 : 0));
     return qs_launch_status("w4a8 gemm (ring)");
+}
+template <int MT, int WN, int MODE, int OUTK, bool KSPLIT>
+int launch_ring(const int8_t* A, const uint8_t* W, const int8_t* zeros, const int8_t* scales8, const void* wscales,
+                const void* ascales, const void* wszs, const void* assums, void* out, int M, int N, int K,
+                int mblocks, int ksplit, int* slabs, unsigned* counters, hipStream_t stream) {
+    // (the policy of the weight requests is the kernel's own constant: as a branch around every request it cost the k loop a tenth of its instructions)
+    const bool shared = (g_ring_flags & 1) || (mblocks > 1 && N <= 8192 && !(g_ring_flags & 2));
+    const auto go = shared ? launch_ring_as<MT, WN, MODE, OUTK, KSPLIT, false> : launch_ring_as<MT, WN, MODE, OUTK, KSPLIT, true>;
+    return go(A, W, zeros, scales8, wscales, ascales, wszs, assums, out, M, N, K, mblocks, ksplit, slabs, counters, stream);
 }
 
 }  // namespace

@@ -1,7 +1,8 @@
 """Mirror of `qserve_backend.qgemm_w4a8_per_group` (kernels/csrc/qgemm/w4a8_per_group/pybind.cpp:13-16)."""
 import torch
 
-from ._util import check, expect, guard, lib, ptr, stream, widened_scratch
+from ._util import check, expect, guard, lib, ptr, stream
+from ._util import widened_scratch as _widened_scratch
 
 
 def gemm_forward_cuda(in_feats, kernel, zeros, scales_i8, wscales, ascales, out_feats):
@@ -15,7 +16,7 @@ def gemm_forward_cuda(in_feats, kernel, zeros, scales_i8, wscales, ascales, out_
     expect(out_feats, torch.float16, "out_feats")
     M, N, K = out_feats.size(-2), out_feats.size(-1), in_feats.size(1)
     with guard(in_feats):
-        scratch = widened_scratch(M, N, K, in_feats)
+        scratch = _widened_scratch(M, N, K, in_feats)
         if scratch is not None:
             check(lib.qs_w4a8_per_group_gemm_scratch(ptr(in_feats), ptr(kernel), ptr(zeros), ptr(scales_i8), ptr(wscales), ptr(ascales), ptr(out_feats),
                                                      M, N, K, ptr(scratch), scratch.numel(), stream()), "qgemm_w4a8_per_group.gemm_forward_cuda")

@@ -394,6 +394,20 @@ int qs_launch_gemm_ring(int mode, int outk, int mt, int wn, const int8_t* A, con
                         const int8_t* scales8, const void* wscales, const void* ascales, const void* wszs,
                         const void* assums, void* out, int M, int N, int K, int mblocks, int ksplit, int* slabs,
                         unsigned* counters, hipStream_t stream);
+// k that a workgroup of `wn` units and one of `ks` K slices spends rounds on; 0: the ring kernel does not take it.  The slices are whole pairs of 64-k stages, shared
+// out over 8 / wn groups.  Where that leaves groups without a stage in the last round, at least two rounds have to be full and at most an eighth may be lost:
+// Llama-2-7B's down_proj (K = 11 008, 172 stages) then has four slices of 43 where only 32 workgroups of two units fitted before, 18.2 -> 9.7 us for one token and 30.9 ->
+// 11.8 per group (whole steps of that model: 1 token 248 -> 210 / 336 -> 255 us, 64 tokens 405 -> 381 / 491 -> 436).  Over K = 1152 .. 18 944, N = 2048 .. 8192: 1 and 16
+// tokens 2.0 - 2.3 times as fast, none slower.  With more tokens the model's costs of slices with lost rounds are a quarter too low (at their plain cost 100 tokens of
+// 8192 x 11 008 took 26.3 us in place of 20.9; with it none of 64 shapes a size is slower): callers add it.
+static long qs_ring_fits(int K, int ks, int mt, int wn, bool act) {
+    const int kg = 8 / wn;
+    if (K % 64 == 0 && (K / 64) % ks == 0 && (K / 64 / ks) % kg == 0) return K / ks;
+    if (K % 128 || mt == 8 || act) return 0;          // (those kernels have even shares only)
+    const int pairs = K / 128, low = 2 * (pairs / ks), high = 2 * ((pairs + ks - 1) / ks);
+    const long k = (long)(high + kg - 1) / kg * kg * 64;
+    return low >= 2 * kg && 8 * k * ks <= 9L * K ? k : 0;
+}
 // compute-bound tiled kernel (gemm_w4a8_tiled.hip)
 int qs_launch_gemm_tiled(int mode, int outk, const int8_t* A, const uint8_t* W, const int8_t* zeros,
                          const int8_t* scales8, const void* wscales, const void* ascales, const void* wszs,
@@ -481,7 +495,7 @@ int dispatch(const int8_t* A, const int8_t* W, const int8_t* zeros, const int8_t
         if (act && ks > 1) return QS_UNFUSED;
         QS_REQUIRE((mt == 1 || mt == 2 || mt == 4 || mt == 8) && (wn == 1 || wn == 2 || (wn == 4 && mt == 4)) &&
                        !(mt == 1 && wn == 2) && !(mt == 8 && wn != 2) &&
-                       N % (64 * wn) == 0 && (K / 64) % ks == 0 && (K / 64 / ks) % (8 / wn) == 0 && (ks == 1 || K / ks <= 32768),
+                       N % (64 * wn) == 0 && qs_ring_fits(K, ks, mt, wn, act) && (ks == 1 || qs_ring_fits(K, ks, mt, wn, act) <= 32768),
                    "w4a8 gemm: forced ring geometry mt=%d wn=%d ksplit=%d does not fit M=%d N=%d K=%d", mt, wn, ks, M, N,
                    K);
         int* slabs = nullptr;
@@ -521,16 +535,17 @@ int dispatch(const int8_t* A, const int8_t* W, const int8_t* zeros, const int8_t
             for (int i = 0; i < 7; ++i) {
                 const int mt = geo[i][0], wn = geo[i][1];
                 if (mt == 8 && (MODE != 1 || ks > 1 || mt_all <= 4 || mt_all > 8 || g_variant == QS_GEMM_RING_NO_MT8)) continue;   // (65 .. 128 tokens)
-                if (N % (64 * wn) != 0 || (K / 64) % ks != 0 || (K / 64 / ks) % (8 / wn) != 0) continue;
-                if (ks > 1 && K / ks > 32768) continue;        // the seam's sentinel must stay out of reach of a partial sum
+                const long slice = qs_ring_fits(K, ks, mt, wn, act);
+                if (N % (64 * wn) != 0 || !slice) continue;
+                if (ks > 1 && slice > 32768) continue;        // the seam's sentinel must stay out of reach of a partial sum
                 const int mb = (mt_all + mt - 1) / mt;
                 const long blocks = (long)mb * (N / (64 * wn)) * ks;
                 if (ks > 1 && (long)mb * (N / (64 * wn)) > 256) continue;   // K slices are for under-filled grids only
                 // per-group: the level-2 dequant is VALU work per weight byte a workgroup streams (measured at M = 128, g128:
                 // qkv 16.0 us with (4,1) against 18.2 with the equal-bytes (2,2)) - charged as a quarter of the weight bytes
                 const long pg = MODE == 1 && g_variant != QS_GEMM_RING_NO_GROUP_TERM ? 8 * wn : 0;
-                const long cost = ((blocks + 255) / 256) * (16 * mt + 32 * wn + pg) * (long)(K / ks) * (ks > 1 ? 11 : 10) / 10 +
-                                  seam(ks, mt);
+                long cost = ((blocks + 255) / 256) * (16 * mt + 32 * wn + pg) * slice * (ks > 1 ? 11 : 10) / 10 + seam(ks, mt);
+                if (slice * ks != K && M > 16) cost += cost / 4;       // (qs_ring_fits)
                 if (best < 0 || cost < best) best = cost, bmt = mt, bwn = wn, bks = ks;
             }
         // Measured override of the byte model (round 4, scripts/gpu_plan_check.sh, weights from HBM): where the model takes
@@ -566,7 +581,7 @@ int dispatch(const int8_t* A, const int8_t* W, const int8_t* zeros, const int8_t
                 bks = 1;
                 for (int i = 0; i < 6; ++i) {
                     const int mt = geo[i][0], wn = geo[i][1];
-                    if (N % (64 * wn) != 0 || (K / 64) % (8 / wn) != 0) continue;
+                    if (N % (64 * wn) != 0 || !qs_ring_fits(K, 1, mt, wn, act)) continue;
                     const long blocks = (long)((mt_all + mt - 1) / mt) * (N / (64 * wn));
                     const long cost = ((blocks + 255) / 256) * (16 * mt + 32 * wn);
                     if (best < 0 || cost < best) best = cost, bmt = mt, bwn = wn;
@@ -813,13 +828,15 @@ bool planes_geometry(int mode, int M, int N, int K, PlanesGeo& g) {
         for (int i = 0; i < 7; ++i) {
             const int mt = geo[i][0], wn = geo[i][1];
             if (mt == 8 && force < 0) continue;         // (measured: the 128-token geometry never wins as planes)
-            if (N % (64 * wn) != 0 || (K / 64) % ks != 0 || (K / 64 / ks) % (8 / wn) != 0) continue;
+            const long slice = qs_ring_fits(K, ks, mt, wn, false);
+            if (N % (64 * wn) != 0 || !slice) continue;
             if (force >= 0 && force != 100 * (ks - 1) + 10 * mt + wn) continue;
             const int mb = (mt_all + mt - 1) / mt;
             const long blocks = (long)mb * (N / (64 * wn)) * ks;
             const long pg = mode == 1 ? 8 * wn : 0;
             const long planes = (long)ks * M * N * 8 / 256 * 23 / 10;
-            const long cost = ((blocks + 255) / 256) * (16 * mt + 32 * wn + pg) * (long)(K / ks) * (ks > 1 ? 11 : 10) / 10 + planes;
+            long cost = ((blocks + 255) / 256) * (16 * mt + 32 * wn + pg) * slice * (ks > 1 ? 11 : 10) / 10 + planes;
+            if (slice * ks != K && M > 16) cost += cost / 4;
             if (best < 0 || cost < best) best = cost, g = {mt, wn, ks, mb};
         }
     return best >= 0;

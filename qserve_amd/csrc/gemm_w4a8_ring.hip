@@ -139,7 +139,7 @@ __device__ __forceinline__ RingCoords ring_coords(int b, int N, int wn, int mblo
 }
 
 // The GEMM proper.  NT: non-temporal weight requests (`issue`).
-template <int MT, int WN, int MODE, int OUTK, bool KSPLIT, bool NT>
+template <int MT, int WN, int MODE, int OUTK, int KS, bool NT>
 __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const uint8_t* __restrict__ W,
                                          const int8_t* __restrict__ zeros, const int8_t* __restrict__ scales8,
                                          const __half* __restrict__ wscales, const __half* __restrict__ ascales,
@@ -147,6 +147,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
                                          void* __restrict__ out, int M, int N, int K, int mblocks, int ns, int ksplit_arg,
                                          int* __restrict__ slabs, unsigned* __restrict__ counters, int flags,
                                          uint8_t* smem) {
+    constexpr bool KSPLIT = KS != 0;
     const int ksplit = KSPLIT ? ksplit_arg : 1;
     constexpr int KG = 8 / WN;
     constexpr int ASTAGE = 16 * MT * 64;              // activation bytes per stage (64 k)
@@ -180,10 +181,21 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
     auto chan32 = [&](int unit, int t) { return ACT ? (t ? N / 2 + 32 * unit : 32 * unit) : unit * 64 + 32 * t; };
     const int m0 = mblk * (16 * MT);
     const int KT = K >> 5;
-    unsigned nst_rem;
-    const int nst = (int)udivmod((unsigned)(K >> 6), (unsigned)ksplit, nst_rem);   // 64-k stages of this workgroup's K slice
-    const int u0 = kq * nst;                          // first global stage
-    const int nloc = nst / KG;                        // stages per group (dispatcher: (K/64/ksplit) % KG == 0)
+    // 64-k stages of this workgroup's K slice, shared out over the groups.  KS == 2: in whole pairs (an activation line feeds two groups), and where they are not a
+    // multiple of the groups some pairs of groups have one more (the dispatcher's qs_ring_fits has what that may cost)
+    int u0, nst;                                      // first global stage, stages
+    if (KS == 2) {
+        unsigned rem0, rem1;
+        const unsigned pairs = (unsigned)K >> 7;
+        u0 = 2 * (int)udivmod(pairs * kq, (unsigned)ksplit, rem0);
+        nst = 2 * (int)udivmod(pairs * (kq + 1), (unsigned)ksplit, rem1) - u0;
+    } else {
+        unsigned nst_rem;
+        nst = (int)udivmod((unsigned)(K >> 6), (unsigned)ksplit, nst_rem);
+        u0 = kq * nst;
+    }
+    const int whole = nst / KG;                       // rounds in which every group has a stage
+    const int mine = KS == 2 ? (nst - kg + KG - 1) / KG : whole;        // stages of this group
 
     uint8_t* const ring = smem + kg * ns * GSTAGE;    // this group's ring: slot s = [A | W | meta]
     const u32 ring_lds = (u32)(size_t)(lptr_t)ring;
@@ -316,7 +328,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
     // ---- prologue: stages 0..ns-2 in flight, operands of stage 0 in registers ---------------------------------------
     QS_STAMP(15);
     for (int j = 0; j < ns - 1; ++j)
-        if (j < nloc) {
+        if (j < mine) {
             issue(j, j);
             // (128 cycles apart: the first stage's lines are then not queued behind the later ones' of other waves.  6144 x 4096, 1 / 16 tokens 6.44 / 7.04 ->
             //  6.18 / 6.82 us, per group 9.13 / 9.42 -> 8.96 / 9.30)
@@ -422,9 +434,9 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
 #pragma unroll
         for (int cl = 0; cl < 4; ++cl) acc[mt][cl] = (v4i){0, 0, 0, 0};
 
-    // wait for stage 0: younger stages outstanding = min(ns-1, nloc) - 1
+    // wait for stage 0: younger stages outstanding = min(ns-1, mine) - 1
     {
-        const int young = (nloc < ns - 1 ? nloc : ns - 1) - 1;
+        const int young = (mine < ns - 1 ? mine : ns - 1) - 1;
         if (young >= 3) wait_vm<3 * NDMA>();
         else if (young == 2) wait_vm<2 * NDMA>();
         else if (young == 1) wait_vm<1 * NDMA>();
@@ -456,7 +468,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
             // one set of activation operands, each read again behind its last product: two sets and the cheap unpacking do not fit the registers (128 tokens of
             // gate_up 30.2 us with two sets and the exact form, 28.7 with this; where half of the waves unpack later, so that a SIMD's two waves alternate, 33.7)
             qn = read_raw(slot_n);
-            if (STEADY || i + ns - 1 < nloc) issue(i + ns - 1, slot_d);
+            if (STEADY || i + ns - 1 < mine) issue(i + ns - 1, slot_d);
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
@@ -481,7 +493,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) nxt.b[mt] = read_b(slot_n, mt);
         }
-        if (STEADY || i + ns - 1 < nloc) issue(i + ns - 1, slot_d);
+        if (STEADY || i + ns - 1 < mine) issue(i + ns - 1, slot_d);
         if (STEADY && MODE == 0) {
             // the requests and the reads first, then one product after the other with the next operands' unpacking between them
             __builtin_amdgcn_sched_barrier(0);
@@ -526,7 +538,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
     // barrier(i): stage i+1 landed for every wave of the group (own pieces by the counted wait), everybody is done
     // reading stage i-1 (its slot is refilled by the DMA issued in round i)
     auto wait_next = [&](int i) {
-        const int rem = nloc - 1 - i;                 // stages after i
+        const int rem = mine - 1 - i;                 // stages after i
         const int young = (rem < ns - 2 ? rem : ns - 2) - 1;   // stages allowed to stay in flight beyond i+1
         if (young >= 3) wait_vm<3 * NDMA>();
         else if (young == 2) wait_vm<2 * NDMA>();
@@ -539,7 +551,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
     // 11.6 -> 10.6, gate_up 28672 x 4096 17.2 -> 16.3, 128 tokens gate_up 27.4 -> 23.6, one token of 4096 x 11008 22.8 -> 18.0; per group 64 tokens gate_up 21.8 ->
     // 19.7, 12288 x 4096 34.1 -> 29.1 with 256 (with the cheap unpacking; scales with carries 18.1 -> 17.1, 16 tokens of gate_up).
     if (ns == DEPTH) {
-        for (; i + DEPTH < nloc; i += 2) {
+        for (; i + DEPTH < whole; i += 2) {
             wait_vm<(DEPTH - 3) * NDMA>();
             raw_barrier();
             round(i, slot, o0, o1, std::true_type());
@@ -550,7 +562,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
             slot = slot + 1 == DEPTH ? 0 : slot + 1;
         }
     }
-    for (; i < nloc; i += 2) {                        // (nloc may be odd)
+    for (; i < whole; i += 2) {                       // (`whole` may be odd)
 #ifdef QS_RING_TRACE
         unsigned long long ta = __builtin_amdgcn_s_memtime();
 #endif
@@ -566,7 +578,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
         ta = __builtin_amdgcn_s_memtime();
 #endif
         slot = slot + 1 == ns ? 0 : slot + 1;
-        if (i + 1 < nloc) {
+        if (i + 1 < whole) {
             wait_next(i + 1);
             raw_barrier();
 #ifdef QS_RING_TRACE
@@ -579,6 +591,17 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
 #endif
             slot = slot + 1 == ns ? 0 : slot + 1;
         }
+    }
+    if (KS == 2 && whole < mine) {                    // a stage more than other groups have: its operands are here
+        auto last = [&](const Ops& o) __attribute__((always_inline)) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int cl = 0; cl < 4; ++cl)
+                    acc[mt][cl] = __builtin_amdgcn_mfma_i32_16x16x64_i8(o.a[cl], o.b[mt], acc[mt][cl], 0, 0, 0);
+        };
+        if (whole & 1) last(o1);
+        else last(o0);
     }
     QS_STAMP(3);
 #ifdef QS_RING_TRACE
@@ -840,8 +863,9 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
 // MT m-tiles (16 tokens each) per wave = tokens per workgroup / 16 (1, 2, 4; 8 = 128-token workgroups, round 5: one level-2
 // dequant of a weight byte serves 128 tokens, ring depth 3-4, reduction through LDS in two passes); WN units per workgroup;
 // KG = 8 / WN K-groups.
-// KSPLIT = false folds every K-slice path away (the un-split launches keep exactly their earlier code).
-template <int MT, int WN, int MODE, int OUTK, bool KSPLIT, bool NT>
+// KS = 0 folds every K-slice path away, 1 has K slices that the groups share out evenly, 2 any (also one).  (As one kernel 1 and 2 cost whole steps of one
+// and sixteen tokens .4 - .8 %.)
+template <int MT, int WN, int MODE, int OUTK, int KS, bool NT>
 __global__ __launch_bounds__(512, 1) void w4a8_gemm_ring(const int8_t* __restrict__ A, const uint8_t* __restrict__ W,
                                                          const int8_t* __restrict__ zeros,
                                                          const int8_t* __restrict__ scales8,
@@ -853,15 +877,16 @@ __global__ __launch_bounds__(512, 1) void w4a8_gemm_ring(const int8_t* __restric
                                                          int* __restrict__ slabs, unsigned* __restrict__ counters,
                                                          int flags) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    ring_body<MT, WN, MODE, OUTK, KSPLIT, NT>(A, W, zeros, scales8, wscales, ascales, wszs, assums, out, M, N, K, mblocks, ns,
+    ring_body<MT, WN, MODE, OUTK, KS, NT>(A, W, zeros, scales8, wscales, ascales, wszs, assums, out, M, N, K, mblocks, ns,
                                           ksplit_arg, slabs, counters, flags, smem);
 }
 
-template <int MT, int WN, int MODE, int OUTK, bool KSPLIT, bool NT>
+template <int MT, int WN, int MODE, int OUTK, int KS, bool NT>
 int launch_ring_as(const int8_t* A, const uint8_t* W, const int8_t* zeros, const int8_t* scales8, const void* wscales,
                 const void* ascales, const void* wszs, const void* assums, void* out, int M, int N, int K,
                 int mblocks, int ksplit, int* slabs, unsigned* counters, hipStream_t stream) {
-    auto kern = w4a8_gemm_ring<MT, WN, MODE, OUTK, KSPLIT, NT>;
+    auto kern = w4a8_gemm_ring<MT, WN, MODE, OUTK, KS, NT>;
+    constexpr bool KSPLIT = KS != 0;
     constexpr int KG = 8 / WN;
     constexpr int GSTAGE = ring_gstage<MT, WN, MODE>();
     // ring depth: as deep as 144 KiB of LDS allows, never deeper than a group's stage count + 1.  At most 5: every
@@ -869,7 +894,7 @@ int launch_ring_as(const int8_t* A, const uint8_t* W, const int8_t* zeros, const
     // the stream no longer gains while the pipeline fill gets longer (depth sweep 3 / 4 / 5 / 6 at M = 16: o 8.9 / 6.7 /
     // 6.45 / 6.66 us, gate_up 18.7 / 13.8 / 13.6 / 13.9 us; M = 64: o 9.2 / 7.1 / 6.74 / 6.96 us; depth 3 costs 25-40 %)
     int ns = ring_depth<MT, WN, MODE>();
-    const int nloc = (K / 64) / ksplit / KG;
+    const int nloc = ((K / 128 + ksplit - 1) / ksplit * 2 + KG - 1) / KG;
     if (ns > nloc + 1) ns = nloc + 1;
     if (const int f = (g_ring_flags >> 8) & 7) {       // A/B: forced depth (sensitivity to the bytes in flight)
         if (f >= 3 && (size_t)KG * f * GSTAGE <= SC_OFF && f <= nloc + 1) ns = f;
@@ -918,13 +943,13 @@ int launch_ring_as(const int8_t* A, const uint8_t* W, const int8_t* zeros, const
                        (g_ring_flags & ~(3 | 16 | 128 | 2048 | 4096)) | inject | (g_epi_fma ? 16 : 0) | (kxcd ? 2048 : 0));
     return qs_launch_status("w4a8 gemm (ring)");
 }
-template <int MT, int WN, int MODE, int OUTK, bool KSPLIT>
+template <int MT, int WN, int MODE, int OUTK, int KS>
 int launch_ring(const int8_t* A, const uint8_t* W, const int8_t* zeros, const int8_t* scales8, const void* wscales,
                 const void* ascales, const void* wszs, const void* assums, void* out, int M, int N, int K,
                 int mblocks, int ksplit, int* slabs, unsigned* counters, hipStream_t stream) {
     // (the policy of the weight requests is the kernel's own constant: as a branch around every request it cost the k loop a tenth of its instructions)
     const bool shared = (g_ring_flags & 1) || (mblocks > 1 && N <= 8192 && !(g_ring_flags & 2));
-    const auto go = shared ? launch_ring_as<MT, WN, MODE, OUTK, KSPLIT, false> : launch_ring_as<MT, WN, MODE, OUTK, KSPLIT, true>;
+    const auto go = shared ? launch_ring_as<MT, WN, MODE, OUTK, KS, false> : launch_ring_as<MT, WN, MODE, OUTK, KS, true>;
     return go(A, W, zeros, scales8, wscales, ascales, wszs, assums, out, M, N, K, mblocks, ksplit, slabs, counters, stream);
 }
 
@@ -939,27 +964,27 @@ extern "C" int qs_debug_ring_trace(void* buf) {
 
 namespace {
 template <int MT, int WN, int MODE, int OUTK>
-int ring_go(bool ks, const int8_t* A, const uint8_t* W, const int8_t* zeros, const int8_t* scales8, const void* wscales,
+int ring_go(int ks, const int8_t* A, const uint8_t* W, const int8_t* zeros, const int8_t* scales8, const void* wscales,
             const void* ascales, const void* wszs, const void* assums, void* out, int M, int N, int K, int mblocks,
             int ksplit, int* slabs, unsigned* counters, hipStream_t stream) {
-    if constexpr (OUTK == 3) {                        // planes exist in the K-sliced instantiation only (one slice = OUTK 1)
-        return launch_ring<MT, WN, MODE, OUTK, true>(A, W, zeros, scales8, wscales, ascales, wszs, assums, out, M, N, K, mblocks,
-                                                     ksplit, nullptr, nullptr, stream);
-    } else {
-        if constexpr (OUTK != 2) {
-            if (ks)
-                return launch_ring<MT, WN, MODE, OUTK, true>(A, W, zeros, scales8, wscales, ascales, wszs, assums, out, M, N, K,
-                                                             mblocks, ksplit, slabs, counters, stream);
-        }
-        return launch_ring<MT, WN, MODE, OUTK, false>(A, W, zeros, scales8, wscales, ascales, wszs, assums, out, M, N, K,
-                                                      mblocks, 1, nullptr, nullptr, stream);
+    auto go = [&](auto kind) {
+        constexpr int KS = decltype(kind)::value;
+        return launch_ring<MT, WN, MODE, OUTK, KS>(A, W, zeros, scales8, wscales, ascales, wszs, assums, out, M, N, K, mblocks, KS ? ksplit : 1,
+                                                   OUTK == 3 || !KS ? nullptr : slabs, OUTK == 3 || !KS ? nullptr : counters, stream);
+    };
+    if constexpr (OUTK != 2) {                        // the activation epilogue exists un-split only, 128-token workgroups in even shares only
+        if constexpr (MT != 8)
+            if (ks == 2) return go(std::integral_constant<int, 2>());
+        if (ks || OUTK == 3) return go(std::integral_constant<int, 1>());      // planes exist in the K-sliced form only (one slice = OUTK 1)
     }
+    if constexpr (OUTK != 3) return go(std::integral_constant<int, 0>());
+    else return QS_ENOSUP;
 }
 }  // namespace
 
 // Entry used by the dispatcher in gemm_w4a8.hip.  mt = m-tiles per workgroup (1, 2, 4), wn = units per workgroup
 // (1, 2, 4); ksplit = K slices (1 = none; > 1 needs the slab / counter workspace: (N/64) * mblocks * ksplit * mt KiB * 4 and
-// (N/64) * mblocks counters); preconditions (checked there): N % (64*wn) == 0, (K/64/ksplit) % (8/wn) == 0,
+// (N/64) * mblocks counters); preconditions (checked there): N % (64*wn) == 0, qs_ring_fits,
 // M*K and N*K/2 below 4 GiB.
 int qs_launch_gemm_ring(int mode, int outk, int mt, int wn, const int8_t* A, const uint8_t* W, const int8_t* zeros,
                         const int8_t* scales8, const void* wscales, const void* ascales, const void* wszs,
@@ -979,7 +1004,12 @@ int qs_launch_gemm_ring(int mode, int outk, int mt, int wn, const int8_t* A, con
         qs_set_error("w4a8 gemm: wscales / w_szs must be 4-byte aligned");
         return QS_EINVAL;
     }
-    const bool ks = ksplit > 1;
+    const bool even = (K / 64) % ksplit == 0 && (K / 64 / ksplit) % (8 / wn) == 0;
+    if (!even && (outk == 2 || mt == 8)) {
+        qs_set_error("w4a8 gemm (ring): the stages of K=%d do not divide over the groups", K);
+        return QS_ENOSUP;
+    }
+    const int ks = !even ? 2 : ksplit > 1;
 #define QS_R(MTV, WNV, MODEV, OUTV)                                                                                  \
     return ring_go<MTV, WNV, MODEV, OUTV>(ks, A, W, zeros, scales8, wscales, ascales, wszs, assums, out, M, N, K, \
                                           mblocks, ksplit, slabs, counters, stream)

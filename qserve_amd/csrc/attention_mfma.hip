@@ -1083,9 +1083,11 @@ struct SplitWs {
 };
 SplitWs g_ws[16][QS_MAX_STREAM_SLOTS];   // [device][scratch slot] (common.h)
 }  // namespace
-// second phase of split-KV, shared with the KV8 kernel (attention_mfma8.hip)
+// second phase of split-KV, shared with the KV8 kernel (attention_mfma8.hip); with invoke_quant where the caller asked for it (fused_small.hip)
+bool qs_launch_attention_merge_quant(const float* ws, _Float16* out, int H, int Hkv, int G, int nsplit, int batch, hipStream_t st);
 void qs_launch_attention_merge(const float* ws, _Float16* out, int H, int Hkv, int G, int nsplit, int batch,
                                hipStream_t st) {
+    if (qs_launch_attention_merge_quant(ws, out, H, Hkv, G, nsplit, batch, st)) return;
     hipLaunchKernelGGL(decode_attention_merge_kernel, dim3(H, batch), dim3(DH), 0, st, ws, out, H, Hkv, G, nsplit);
 }
 float* qs_split_workspace(size_t bytes, hipStream_t st) {
@@ -1285,7 +1287,6 @@ int qs_launch_decode_mfma(int G, dim3 grid, hipStream_t st, const _Float16* q, c
             return QS_ENOSUP;
     }
 #undef QS_LAUNCH_G
-    if (nsplit > 1)
-        hipLaunchKernelGGL(decode_attention_merge_kernel, dim3(H, grid.y), dim3(DH), 0, st, ws, out, H, Hkv, G, nsplit);
+    if (nsplit > 1) qs_launch_attention_merge(ws, out, H, Hkv, G, nsplit, (int)grid.y, st);
     return qs_launch_status("single_query_attention");
 }

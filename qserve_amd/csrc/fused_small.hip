@@ -255,6 +255,61 @@ extern "C" int qs_set_row_sum_order(int order) {
 }
 extern "C" int qs_get_row_sum_order(void) { return g_row_refsum; }
 
+// Split attention's second phase and invoke_quant(_fuse_sum) of the finished row in one launch: workgroup = sequence, thread = 8 values.  Bound by latency (8 parts of
+// 32 heads are 133 KB a workgroup, requested together).  As two launches, one workgroup per head and one per row, 4.7 + 4.4 us for 8 sequences of 32 heads; whole steps of
+// four layers 325.6 -> 315.6 us (8 sequences of 7700 tokens, 8-bit cache), 265 -> 250 (1 of 7700), 244 -> 231 (2 of 3000, 4-bit), 327 -> 319 (16 of 4000).  With 256
+// threads of two times 8 values 318.8, 254, 236, 321.
+// Same bits: the parts are added in the merge kernel's order (attention_mfma.hip), and the row's sum does not depend on the number of threads.
+constexpr int MERGE_SPLITS = 8, MERGE_DH = 128, MERGE_NT = 512;
+__global__ __launch_bounds__(MERGE_NT) void merge_quant_kernel(const float* __restrict__ ws, _Float16* __restrict__ out, int8_t* __restrict__ qout,
+                                                               __half* __restrict__ sum_out, __half* __restrict__ scale_out, int H, int Hkv, int G, int nsplit) {
+    __shared__ float sm[2 * (MERGE_NT / 64)];
+    __shared__ __attribute__((aligned(16))) _Float16 row[MERGE_NT * 8];
+    const int hidden = H * MERGE_DH, b = blockIdx.x, i = (int)threadIdx.x * 8, hq = i / MERGE_DH, d = i % MERGE_DH;
+    if (i < hidden) {
+        const size_t zs = (size_t)G * (MERGE_DH + 2);
+        const float* base = ws + (((size_t)b * Hkv + hq / G) * nsplit * G + hq % G) * (MERGE_DH + 2);
+        float2 md[MERGE_SPLITS], part[MERGE_SPLITS][4];
+#pragma unroll
+        for (int z = 0; z < MERGE_SPLITS; ++z)
+            if (z < nsplit) {
+                md[z] = *reinterpret_cast<const float2*>(base + z * zs + MERGE_DH);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) part[z][e] = *reinterpret_cast<const float2*>(base + z * zs + d + 2 * e);
+            }
+        float M = -3.0e38f, den = 0.f, num[8] = {};
+#pragma unroll
+        for (int z = 0; z < MERGE_SPLITS; ++z)
+            if (z < nsplit) M = fmaxf(M, md[z].x);
+#pragma unroll
+        for (int z = 0; z < MERGE_SPLITS; ++z)
+            if (z < nsplit) {
+                const float f = __expf(md[z].x - M);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    num[2 * e] += f * part[z][e].x;
+                    num[2 * e + 1] += f * part[z][e].y;
+                }
+                den += f * md[z].y;
+            }
+        h8 v;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = (_Float16)(num[e] / (den + 1.e-6f));
+        *reinterpret_cast<h8*>(row + i) = v;
+        *reinterpret_cast<h8*>(out + (size_t)b * hidden + i) = v;
+    }
+    qs_row::quant_row<1, MERGE_NT / 64, MERGE_NT / 64, false>(qout + (size_t)b * hidden, row, sum_out ? sum_out + b : nullptr, scale_out + b, hidden, sm,
+                                                              (int)threadIdx.x);
+}
+bool qs_launch_attention_merge_quant(const float* ws, _Float16* out, int H, int Hkv, int G, int nsplit, int batch, hipStream_t st) {
+    QsAttnQuant& q = g_qs_attn_quant;
+    // (the rule of splits gives at most 8 parts; the reference's order of the sum stays with the pair)
+    if (!q.qout || H * MERGE_DH > MERGE_NT * 8 || nsplit > MERGE_SPLITS || (qs_get_row_sum_order() && q.qsum)) return false;
+    hipLaunchKernelGGL(merge_quant_kernel, dim3(batch), dim3(MERGE_NT), 0, st, ws, out, q.qout, (__half*)q.qsum, (__half*)q.qscale, H, Hkv, G, nsplit);
+    q.done = 1;
+    return true;
+}
+
 extern "C" int qs_invoke_quant(int8_t* out, const void* input, void* input_sum, void* scale, int num_tokens,
                                int hidden, qs_stream_t stream) {
     QS_REQUIRE(out && input && scale, "invoke_quant: null pointer");

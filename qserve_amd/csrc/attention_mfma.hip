@@ -1133,8 +1133,8 @@ int qs_attn_choose_splits(int blocks, int pages, int kv8, int fused_quant) {
         if (n > 1 && pages / n < 2) break;
         const long rounds = ((long)blocks * n + 255) / 256;
         const long per_cu = rounds * pages * t_cu / n, chip = (long)blocks * pages * t_hbm_ps / 1000;
-        // (fused_quant: qs_single_query_attention_quant - only the un-split launch can finish the row itself; a split one is
-        // followed by the quantiser as a launch of its own, 3.2 us + boundary)
+        // (fused_quant: qs_single_query_attention_quant.  The charge was fitted when a split launch was followed by the merge and the quantiser, two launches;
+        // they are one now, but 0, 1000 or 2000 in its place change whole steps of 1 - 32 sequences at 300 - 4000 tokens by 1.7 % at most, either way)
         const long cost = rounds * F + (per_cu > chip ? per_cu : chip) + (n > 1 ? 2500 + 300 * n + (fused_quant ? 3500 : 0) : 0);
         if (best < 0 || cost < best) best = cost, best_n = n;
     }

@@ -514,7 +514,7 @@ int dispatch(const int8_t* A, const int8_t* W, const int8_t* zeros, const int8_t
         const int mt_all = (M + 15) / 16;
         // <8,2> = 128-token workgroups (round 5): PER-GROUP only, un-split, from 65 tokens on - one level-2 dequant of a weight byte
         // serves 128 tokens instead of being repeated per 64-token block.  Measured (scripts/gpu_mt8_ab.sh, weights from HBM, g128):
-        // gate_up 28 672 x 4096 at M = 128: 30.6 us against 35.6 for <4,4> x 2 token blocks (M = 96: 29.6 / 35.2); per-channel
+        // gate_up 28 672 x 4096 at M = 128: 30.6 us (28.7 since its loop has no branches) against 35.6 for <4,4> x 2 token blocks (M = 96: 29.6 / 35.2); per-channel
         // the same geometry LOSES (28.5 vs 25.4 us: ring depth 3 instead of 5, nothing to share), K-sliced or four-unit forms of it
         // lose everywhere (<8,4>: 60 us), and for N <= 6144 the 64-token geometries fill the chip better (qkv 28.7 vs 15.9 us).
         // Variant 4004 keeps it out (A/B).

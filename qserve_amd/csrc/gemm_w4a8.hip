@@ -757,7 +757,7 @@ extern "C" int qs_w4a8_per_chn_gemm_silu_mul(const int8_t* in_feats, const int8_
 //    201 -> 183; 2048 x 2048 30 -> 26.  Not where the four-wave tile needs one round of the chip only (12288 x 4096, 1152 tokens 67 -> 72), nor up to 2 M weights (512 x 4096
 //    26 -> 33, 1024 x 1024 13 -> 17).
 //  * up to 1024 tokens the widening is a larger share: not in one round of any kernel (28672 x 4096, 512 tokens 68 -> 86), not up to 4096 x 4096 (1024 tokens
-//    39 -> 41; 6144 x 4096 54 -> 47, 4096 x 14336 110 -> 100), not beyond 128 M weights (57344 x 8192, 1024 tokens 472 -> 510; 28672 x 4096 133 -> 133); up to 512 only
+//    39 -> 41; 6144 x 4096, 768 tokens 53 -> 42), not in place of the ring kernel's K slices (4096 x 14336, 600 / 768 tokens 92 / 97 -> 101), not beyond 128 M weights (57344 x 8192, 1024 tokens 472 -> 510; 28672 x 4096 133 -> 133); up to 512 only
 //    beside two rounds of 128-token tiles (22016 x 4096, 300 tokens 104 -> 73; the ring kernel's two: 8192 x 8192, 512 tokens 68 -> 71).
 extern "C" long long qs_w4a8_per_group_scratch_bytes(int M, int N, int K) {
     if (g_variant != QS_GEMM_DEFAULT || M <= 256 || N <= 0 || K <= 0 || N % 256 != 0 || K % 128 != 0 || K >= (1 << 24) || (size_t)M * K >= (1ull << 32) ||
@@ -770,7 +770,7 @@ extern "C" long long qs_w4a8_per_group_scratch_bytes(int M, int N, int K) {
     const bool ring = plan[0] == 3, tiled = plan[0] == 4, wide = plan[0] == 5;
     const long long groups = ring ? (long long)plan[3] * (N / (64 * plan[2])) * plan[4]                            // token blocks x channels x K slices
                              : tiled || wide ? (long long)((M + 32 * plan[1] - 1) / (32 * plan[1])) * (N / 256) : 0;
-    if (M <= 512 ? !(tiled && groups > 256) : M <= 1024 ? (ring || tiled || wide) && groups <= 256 : wide && groups <= 256) return 0;
+    if (M <= 512 ? !(tiled && groups > 256) : M <= 1024 ? (ring && plan[4] > 1) || ((ring || tiled || wide) && groups <= 256) : wide && groups <= 256) return 0;
     return need;
 }
 namespace {

@@ -27,7 +27,7 @@
 //   1 = weight DMA with the default cache policy everywhere, 2 = non-temporal everywhere (default: non-temporal unless several
 //       token blocks share the weight bytes of a channel block and N <= 8192 - see launch_ring and `issue`; the host's switch)
 //   4 / 8 = (QS_TIMING libraries only) no cross-group reduction / leave behind the k loop: the price of the tail (round 5)
-//   32 / 64 = (libraries built with -DQS_TIMING only; ignored by the shipped library) timing only, WRONG RESULTS: no MFMA /
+//   32 / 64 = (libraries built with -DQS_TIMING only; ignored by the shipped library and by 128-token workgroups per group) timing only, WRONG RESULTS: no MFMA /
 //        no LDS operand reads (what is left is the DMA + barrier pipeline:
 //        gate_up at M = 64 17.5 us -> 16.3 / 16.8, both off 15.9 us = 4.2 us of head and tail + 512 KB per CU at 44 GB/s,
 //        the rate scripts/microbench_cufill.hip measures for this L2 + HBM mix with nothing else going on)
@@ -550,6 +550,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
     // general rounds below for all of them a round had twelve branches, between the barrier and the operands it needs.  Before and after, us: 33 tokens 12288 x 4096
     // 11.6 -> 10.6, gate_up 28672 x 4096 17.2 -> 16.3, 128 tokens gate_up 27.4 -> 23.6, one token of 4096 x 11008 22.8 -> 18.0; per group 64 tokens gate_up 21.8 ->
     // 19.7, 12288 x 4096 34.1 -> 29.1 with 256 (with the cheap unpacking; scales with carries 18.1 -> 17.1, 16 tokens of gate_up).
+#ifndef QS_TIMING                                         // (timing builds keep the general rounds, which have their switches)
     if (ns == DEPTH) {
         for (; i + DEPTH < whole; i += 2) {
             wait_vm<(DEPTH - 3) * NDMA>();
@@ -562,6 +563,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
             slot = slot + 1 == DEPTH ? 0 : slot + 1;
         }
     }
+#endif
     for (; i < whole; i += 2) {                       // (`whole` may be odd)
 #ifdef QS_RING_TRACE
         unsigned long long ta = __builtin_amdgcn_s_memtime();

@@ -98,3 +98,33 @@ def test_few_slots(n, E, top, N, K, shared, act, limit):
     there = ((idx >= 0) & (idx < E)).cuda()
     assert not few[there].isnan().any() and few[~there].isnan().all()
     assert torch.equal(few[there], by_expert[there]) and torch.equal(few_shared, shared_too)
+
+
+# Gates over their whole range, products that are sums of one term: the units of a prompt's kernel are a step's, and within a rounding of the exact ones
+@pytest.mark.parametrize("act, limit", [(2, 0.0), (3, 7.0), (3, 100.0)])
+def test_units_over_the_range_of_their_gates(act, limit):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    g = torch.arange(0x3A80, 0x42C9, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)          # 2^-10 .. 100, every bfloat16
+    g = torch.cat([g, -g])
+    X = torch.zeros(len(g), 64, dtype=torch.bfloat16)
+    X[:, 0], X[:, 1], X[:, 2] = g, 1.0, -0.40625
+    W = torch.zeros(1, 4, 64, dtype=torch.bfloat16)
+    W[0, 0, 0] = W[0, 1, 1] = W[0, 2, 0] = W[0, 3, 2] = 1.0                                          # (gate, 1), (gate, -0.40625)
+    X, W = X.cuda(), W.cuda()
+    L, s, n = lib(), torch.cuda.current_stream().cuda_stream, len(g)
+    listed, sorted_, rows = (torch.full((n, 2), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(3))
+    tiles = torch.tensor([(0, o, min(L.qsv_grouped_gemm_tile_slots(), n - o)) for o in range(0, n, L.qsv_grouped_gemm_tile_slots())], dtype=torch.int32, device="cuda")
+    check(L.qsv_grouped_gemm(listed.data_ptr(), X.data_ptr(), None, 1, W.data_ptr(), tiles.data_ptr(), tiles.size(0), 4, 64, act, limit, None, s), "grouped_gemm")
+    order, offsets = torch.arange(n, dtype=torch.int32, device="cuda"), torch.tensor([0, n], dtype=torch.int32, device="cuda")
+    check(L.qsv_grouped_gemm_sorted(sorted_.data_ptr(), X.data_ptr(), order.data_ptr(), 1, W.data_ptr(), offsets.data_ptr(), 1, 4, 64, act, limit, None, s), "sorted")
+    check(L.qsv_expert_rows(rows.data_ptr(), X.data_ptr(), None, 1, W.data_ptr(), offsets.long().data_ptr(), 1, 4, 64, act, limit, None, s), "expert_rows")
+    assert torch.equal(listed.view(torch.int16), rows.view(torch.int16)) and torch.equal(sorted_.view(torch.int16), rows.view(torch.int16))
+    z, u = g.double()[:, None], torch.tensor([1.0, -0.40625], dtype=torch.float64)
+    if act == 3:
+        z, u = z.clamp(max=limit), u.clamp(-limit, limit) + 1.0
+    c = 1.702 if act == 3 else 1.0
+    want, near = z * torch.sigmoid(c * z) * u, (c * z > -87.0).expand(-1, 2)                          # (below, 1 + exp leaves a float's range)
+    # one rounding to the 8 bits of a bfloat16 (2^-8); before it the exponential, a sum, a quotient and a product: 2^-24 each, the exponent's own rounding (1.702 g) times |c z|
+    bound = want.abs() * (2.0 ** -8 + (4 + c * z.abs()) * 2.0 ** -23)
+    assert ((listed.double().cpu() - want).abs() <= bound)[near].all()

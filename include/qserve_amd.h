@@ -22,7 +22,8 @@
  *     graph: such a call runs the variant that needs no scratch) and is NEVER freed, moved or grown afterwards, so a
  *     hipGraph that captured its address stays valid for the life of the process.  Requests beyond the fixed capacity
  *     fall back to the un-split variants.  The scratch areas exist once per device (the CURRENT device of the calling thread),
- *     shared by every stream: launches that use them (split-KV attention, K-sliced GEMMs, the split argmax, the fused attention
+ *     shared by every stream: launches that use them (split-KV attention, K-sliced GEMMs - reductions whose stages divide evenly, the
+ *     others are sliced on bound streams only -, the split argmax, the fused attention
  *     quantiser's hand-over) must not run concurrently on different streams of one device (the reference's engine is
  *     single-stream) - UNLESS the extra streams were given scratch of their own with qs_stream_scratch_bind() (below: up to 7
  *     streams per device; launches issued on, or captured on, a bound stream use that stream's areas).

@@ -529,6 +529,14 @@ int dispatch(const int8_t* A, const int8_t* W, const int8_t* zeros, const int8_t
             if (ks <= 1) return 0;
             return ((ks == 2 ? 150L : 250L) + (mt > 2 ? 40L * (ks - 2) : 0)) * 1024;
         };
+        // Slices that the groups do not share out evenly meet only in scratch that is the stream's own (qs_stream_scratch_bind): these reductions kept to one slice
+        // before there was such a form, and streams that share the device's scratch may run them side by side.  Without: 4096 x 11 008, one token 9.5 -> 10.9 us, per group
+        // 11.4 -> 17.3 (22.8 and 37.7 before the form); the planes form, which meets in its caller's buffer, has its slices on every stream.
+        int own = -1;
+        auto own_scratch = [&]() {
+            if (own < 0) own = !g_qs_plan.active && qs_scratch_slot(stream) > 0;
+            return own == 1;
+        };
         long best = -1;
         int bmt = 0, bwn = 0, bks = 1;
         for (int ks = 1; ks <= (g_variant == QS_GEMM_RING_NO_KSLICES || act ? 1 : 4); ks *= 2)
@@ -538,6 +546,7 @@ int dispatch(const int8_t* A, const int8_t* W, const int8_t* zeros, const int8_t
                 const long slice = qs_ring_fits(K, ks, mt, wn, act);
                 if (N % (64 * wn) != 0 || !slice) continue;
                 if (ks > 1 && slice > 32768) continue;        // the seam's sentinel must stay out of reach of a partial sum
+                if (ks > 1 && slice * ks != K && !own_scratch()) continue;
                 const int mb = (mt_all + mt - 1) / mt;
                 const long blocks = (long)mb * (N / (64 * wn)) * ks;
                 if (ks > 1 && (long)mb * (N / (64 * wn)) > 256) continue;   // K slices are for under-filled grids only
@@ -559,8 +568,8 @@ int dispatch(const int8_t* A, const int8_t* W, const int8_t* zeros, const int8_t
             (K / 64) % 2 == 0 && (K / 64 / 2) % 8 == 0 && g_variant != QS_GEMM_RING_NO_DOWN_OVERRIDE)
             bwn = 1, bks = 2;
         // the older register-staged split-K kernel takes any K and cuts the tokens down to 16 per workgroup: same byte
-        // model, ~20 % slower at equal bytes (measured) - it wins where K leaves the ring kernel only coarse geometries
-        // (Llama-2-7B down_proj: K = 11 008 = 172 stages, two-unit workgroups only)
+        // model, ~20 % slower at equal bytes (measured) - it wins where K leaves the ring kernel only coarse geometries or shares that do not divide
+        // (Llama-2-7B down_proj, K = 11 008 = 172 stages, at 17 - 128 tokens; up to 16 the ring's one-unit workgroups do)
         if (best >= 0 && !act && units < 256 && units % 8 == 0 && M > 16 && M <= 128) {
             int mto = 1;
             for (int cand = 4; cand >= 1; cand >>= 1)

@@ -2,6 +2,7 @@
 measured heuristics of DESIGN.md 5.1 - a change here must come with new measurements (scripts/bench_gemm_shard.py)."""
 import pytest
 
+from qserve_amd.fused import gemm_planes_plan
 from qserve_amd.plan import attention_plan, gemm_plan
 
 
@@ -61,6 +62,23 @@ def test_awkward_k_falls_back_or_uses_two_unit_workgroups():
     assert gemm_plan(64, 5120, 13824)["family"] == "ring"        # Llama-2-13B down_proj: 216 stages = 4 groups x 54
     assert gemm_plan(64, 4096, 512)["family"] == "splitk"        # short K at decode batch: fixed costs
     assert gemm_plan(512, 4096, 1792)["family"] in ("ring", "pair")
+
+
+@pytest.mark.parametrize("per_group", [False, True])
+def test_shares_that_do_not_divide_keep_one_slice_in_shared_scratch(per_group):
+    """172 stages: slices of whole pairs that eight groups do not share out evenly.  In the device's shared scratch they would make streams race that could run side by
+    side before; the planes form meets in the caller's buffer and has them."""
+    for M in (1, 4, 16):
+        assert gemm_plan(M, 4096, 11008, per_group) == ring(1, 1, 1)
+    for M in (17, 33, 64, 128):
+        assert gemm_plan(M, 4096, 11008, per_group)["family"] == "splitk"
+    for M in range(1, 1025, 61):
+        for N in (1024, 4096, 8192):
+            for K in (1152, 1920, 3456, 5504, 6912, 11008, 13824, 18944):
+                p = gemm_plan(M, N, K, per_group)
+                if p["family"] == "ring" and p["k_slices"] > 1:
+                    assert K // 64 % p["k_slices"] == 0 and K // 64 // p["k_slices"] % (8 // p["units"]) == 0, (M, N, K, p)
+    assert [gemm_planes_plan(M, 4096, 11008, per_group) for M in (1, 16, 64)] == [4, 4, 4]
 
 
 @pytest.mark.parametrize("tp", [2, 4, 8])

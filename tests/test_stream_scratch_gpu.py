@@ -97,6 +97,33 @@ def test_k_sliced_gemms_on_two_streams_at_once(gpu, variant, M, N, K):
         _unbind(s1)
 
 
+@pytest.mark.parametrize("M, bound", [(1, False), (16, False), (40, False), (1, True), (16, True)])
+def test_shares_that_do_not_divide_on_two_streams_at_once(gpu, M, bound):
+    """K = 11 008 (172 stages): one slice, nothing shared, on streams without scratch of their own; K slices in it where both have it."""
+    import qserve_backend.qgemm_w4a8_per_chn as op
+    N, K = 256, 11008
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    try:
+        assert not bound or all(_bind(s) == 0 for s in streams)
+        probs = [_gemm_problem(31 + j, M, N, K) for j in range(2)]
+        outs = [[torch.empty((M, N), dtype=torch.float16, device=gpu) for _ in range(40)] for _ in range(2)]
+        torch.cuda.synchronize()
+        graphs = []
+        for j, s in enumerate(streams):
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g, stream=s):
+                for i in range(40):
+                    op.gemm_forward_cuda(*probs[j][0], outs[j][i])
+            graphs.append(g)
+        _replay_together(graphs, streams)
+        for j in range(2):
+            for i in range(40):
+                assert np.array_equal(outs[j][i].cpu().numpy().view(np.uint16), probs[j][1].view(np.uint16)), (j, i)
+    finally:
+        for s in streams:
+            _unbind(s)
+
+
 def test_decode_engines_on_two_streams_at_once(gpu):
     """Two tiny decode engines (attention + quant hand-over through the slot's exchange rows, split argmax, the GEMM families of the
     tiny widths), one per stream, stepping concurrently: each reproduces the tokens it generates alone."""

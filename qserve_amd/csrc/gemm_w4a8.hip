@@ -762,12 +762,17 @@ extern "C" int qs_w4a8_per_chn_gemm_silu_mul(const int8_t* in_feats, const int8_
 
 // Per-group products of many tokens over weights widened to int8 in scratch of the caller's (gemm_w4a8_unpacked.hip): the level-2 dequant once a weight in place
 // of once a weight and 256 tokens, and a last round of tiles that is cut.  us, plain -> widened, MI355X, weights out of memory:
-//  * 8192 tokens: 12288 x 4096 389 -> 329, 4096 x 11008 311 -> 279, 28672 x 4096 + silu 880 -> 769; 5331: 253 -> 224, 274 -> 218, 634 -> 529; 1300: 118 -> 96, 180 -> 97,
-//    201 -> 183; 2048 x 2048 30 -> 26.  Not where the four-wave tile needs one round of the chip only (12288 x 4096, 1152 tokens 67 -> 72), nor up to 2 M weights (512 x 4096
-//    26 -> 33, 1024 x 1024 13 -> 17).
+//  * 8192 tokens: 12288 x 4096 389 -> 329, 4096 x 11008 311 -> 279, 28672 x 4096 + silu 880 -> 769, 57344 x 8192 3363 -> 2716; 5331: 253 -> 224, 274 -> 218, 634 -> 529; 1300:
+//    118 -> 96, 180 -> 97, 201 -> 183; 2048 x 2048 30 -> 26.  Not up to 2 M weights (512 x 4096 26 -> 33, 1024 x 1024 13 -> 17), and not in place of one round of the chip, whose
+//    workgroups unpack beside each other: of four-wave tiles (12288 x 4096, 1152 tokens 67 -> 72), of 128-channel x 64-token pairs (256 x 16384, 1025 tokens 82 -> 96; 512 x 8192, 4096
+//    tokens 46 -> 52, 6000 86 -> 53; two rounds of them and a short reduction: 2816 x 1536, 1300 tokens 22.8 -> 23.1), of 128-token tiles with a reduction below 2048
+//    (4096 x 1024, 2048 tokens 20 -> 22; 4096 x 1536 25 -> 27; 2048 x 2048, 4096 tokens 31 -> 28).
 //  * up to 1024 tokens the widening is a larger share: not in one round of any kernel (28672 x 4096, 512 tokens 68 -> 86), not up to 4096 x 4096 (1024 tokens
-//    39 -> 41; 6144 x 4096, 768 tokens 53 -> 42), not in place of the ring kernel's K slices (4096 x 14336, 600 / 768 tokens 92 / 97 -> 101), not beyond 128 M weights (57344 x 8192, 1024 tokens 472 -> 510; 28672 x 4096 133 -> 133); up to 512 only
+//    39 -> 41; 6144 x 4096, 768 tokens 53 -> 42), not in place of the ring kernel's K slices (4096 x 14336, 600 / 768 tokens 92 / 97 -> 101) or its 32-token workgroups
+//    (2560 x 8192, 800 tokens 50 -> 57; 64-token ones 5120 x 4352 52 -> 41), not beside two full rounds of four-wave tiles and a short reduction (29696 x 2560, 1000 tokens
+//    86 -> 92), not beyond 128 M weights (57344 x 8192, 1024 tokens 472 -> 510; 28672 x 4096 133 -> 133); up to 512 only
 //    beside two rounds of 128-token tiles (22016 x 4096, 300 tokens 104 -> 73; the ring kernel's two: 8192 x 8192, 512 tokens 68 -> 71).
+//  Of 5400 random shapes that this takes 8 are more than a percent slower than the plain entry, by 4 % at most.
 extern "C" long long qs_w4a8_per_group_scratch_bytes(int M, int N, int K) {
     if (g_variant != QS_GEMM_DEFAULT || M <= 256 || N <= 0 || K <= 0 || N % 256 != 0 || K % 128 != 0 || K >= (1 << 24) || (size_t)M * K >= (1ull << 32) ||
         (size_t)N * K >= (1ull << 32))
@@ -776,11 +781,16 @@ extern "C" long long qs_w4a8_per_group_scratch_bytes(int M, int N, int K) {
     if (need < 4 * million || (M <= 1024 && (need < 20 * million || need > 128 * million))) return 0;
     int plan[5];
     if (qs_w4a8_gemm_plan(1, M, N, K, plan) != QS_OK) return 0;
-    const bool ring = plan[0] == 3, tiled = plan[0] == 4, wide = plan[0] == 5;
+    const bool pair = plan[0] == 2, ring = plan[0] == 3, tiled = plan[0] == 4, wide = plan[0] == 5;
     const long long groups = ring ? (long long)plan[3] * (N / (64 * plan[2])) * plan[4]                            // token blocks x channels x K slices
-                             : tiled || wide ? (long long)((M + 32 * plan[1] - 1) / (32 * plan[1])) * (N / 256) : 0;
-    if (M <= 512 ? !(tiled && groups > 256) : M <= 1024 ? (ring && plan[4] > 1) || ((ring || tiled || wide) && groups <= 256) : wide && groups <= 256) return 0;
-    return need;
+                             : tiled || wide ? (long long)((M + 32 * plan[1] - 1) / (32 * plan[1])) * (N / 256)
+                             : pair ? (long long)((M + 63) / 64) * (N / 128) : 0;
+    const bool one = (pair || ring || tiled || wide) && groups <= 256;
+    bool plain;
+    if (M <= 512) plain = !tiled || one;
+    else if (M <= 1024) plain = one || (ring && (plan[4] > 1 || plan[1] < 4)) || (wide && groups >= 448 && groups <= 512 && K < 4096);
+    else plain = ((pair || wide) && one) || (K < 2048 && ((tiled && one) || (pair && groups <= 512)));
+    return plain ? 0 : need;
 }
 namespace {
 bool unpack_fits(const void* in_feats, const void* kernel, const void* zeros, const void* scales_i8, const void* wscales, const void* ascales, const void* out,

@@ -76,7 +76,7 @@ int qs_w4a8_per_group_gemm(const int8_t* in_feats, const int8_t* kernel, const i
                            int M, int N, int K, qs_stream_t stream);
 
 /* The same with scratch of the caller's, for products of many tokens: the weights are widened to int8 into it once and multiplied from there (two launches,
- * the same bits).  qs_w4a8_per_group_scratch_bytes: what the call wants (N K bytes, on 16; 0: nothing, the plain entry is the faster one - or the shape
+ * the same bits).  qs_w4a8_per_group_scratch_bytes: what the call wants (N K bytes, on 16, 512 MiB at most; 0: nothing, the plain entry is the faster one - or the shape
  * does not fit).  With less than that, or with operands that do not start on 16 bytes, the call is the plain entry.  The scratch holds nothing
  * afterwards and may be given to any later work of the same stream. */
 long long qs_w4a8_per_group_scratch_bytes(int M, int N, int K);

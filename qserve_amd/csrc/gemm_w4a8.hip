@@ -773,9 +773,10 @@ extern "C" int qs_w4a8_per_chn_gemm_silu_mul(const int8_t* in_feats, const int8_
 //    86 -> 92), not beyond 128 M weights (57344 x 8192, 1024 tokens 472 -> 510; 28672 x 4096 133 -> 133); up to 512 only
 //    beside two rounds of 128-token tiles (22016 x 4096, 300 tokens 104 -> 73; the ring kernel's two: 8192 x 8192, 512 tokens 68 -> 71).
 //  Of 5400 random shapes that this takes 8 are more than a percent slower than the plain entry, by 4 % at most.
+//  * the scratch is 512 MiB at most; the widening's grid has a row of workgroups for every 32 channels.
 extern "C" long long qs_w4a8_per_group_scratch_bytes(int M, int N, int K) {
     if (g_variant != QS_GEMM_DEFAULT || M <= 256 || N <= 0 || K <= 0 || N % 256 != 0 || K % 128 != 0 || K >= (1 << 24) || (size_t)M * K >= (1ull << 32) ||
-        (size_t)N * K >= (1ull << 32))
+        (size_t)N * K > (512u << 20) || N / 32 > 65535)
         return 0;
     const long long need = (long long)N * K, million = 1 << 20;
     if (need < 4 * million || (M <= 1024 && (need < 20 * million || need > 128 * million))) return 0;
@@ -793,11 +794,17 @@ extern "C" long long qs_w4a8_per_group_scratch_bytes(int M, int N, int K) {
     return plain ? 0 : need;
 }
 namespace {
+// (wscales on 4 bytes: the ring kernel wants it, and what the plain entry refuses is refused here)
 bool unpack_fits(const void* in_feats, const void* kernel, const void* zeros, const void* scales_i8, const void* wscales, const void* ascales, const void* out,
                  int M, int N, int K, const void* scratch, long long scratch_bytes) {
     const long long need = qs_w4a8_per_group_scratch_bytes(M, N, K);
     return need > 0 && scratch && scratch_bytes >= need && in_feats && kernel && zeros && scales_i8 && wscales && ascales && out &&
-           ((uintptr_t)in_feats | (uintptr_t)kernel | (uintptr_t)out | (uintptr_t)scratch) % 16 == 0 && ((uintptr_t)zeros | (uintptr_t)scales_i8) % 4 == 0;
+           ((uintptr_t)in_feats | (uintptr_t)kernel | (uintptr_t)out | (uintptr_t)scratch) % 16 == 0 && ((uintptr_t)zeros | (uintptr_t)scales_i8 | (uintptr_t)wscales) % 4 == 0;
+}
+// where the plain gate_up + silu takes two launches through `tmp`
+bool needs_tmp(int M, int N, int K) {
+    int plan[5];
+    return qs_w4a8_gemm_plan(1, M, N, K, plan) != QS_OK || plan[0] < 3;
 }
 }  // namespace
 extern "C" int qs_w4a8_per_group_gemm_scratch(const int8_t* in_feats, const int8_t* kernel, const int8_t* zeros, const int8_t* scales_i8, const void* wscales,
@@ -818,7 +825,7 @@ extern "C" int qs_w4a8_per_group_gemm_silu_mul(const int8_t* in_feats, const int
 extern "C" int qs_w4a8_per_group_gemm_silu_mul_scratch(const int8_t* in_feats, const int8_t* kernel, const int8_t* zeros, const int8_t* scales_i8,
                                                        const void* wscales, const void* ascales, void* out_act, void* tmp, int M, int N, int K, void* scratch,
                                                        long long scratch_bytes, qs_stream_t stream) {
-    if (g_act_off || !unpack_fits(in_feats, kernel, zeros, scales_i8, wscales, ascales, out_act, M, N, K, scratch, scratch_bytes))
+    if (g_act_off || !unpack_fits(in_feats, kernel, zeros, scales_i8, wscales, ascales, out_act, M, N, K, scratch, scratch_bytes) || (!tmp && needs_tmp(M, N, K)))
         return qs_w4a8_per_group_gemm_silu_mul(in_feats, kernel, zeros, scales_i8, wscales, ascales, out_act, tmp, M, N, K, stream);
     return qs_launch_gemm_unpacked(true, in_feats, reinterpret_cast<const uint8_t*>(kernel), zeros, scales_i8, wscales, ascales, out_act, M, N, K, scratch,
                                    (hipStream_t)stream);

@@ -1,4 +1,4 @@
-"""Which per-group products of many tokens ask for scratch (qs_w4a8_per_group_scratch_bytes), without a GPU.  Every shape was measured on both
+"""Which per-group products of many tokens ask for scratch (qs_w4a8_per_group_scratch_bytes) and what their entries refuse, without a GPU.  Every shape was measured on both
 sides (figures beside the rule)."""
 import pytest
 
@@ -21,3 +21,22 @@ def test_where_the_plain_entry_is_the_faster_one(M, N, K):
 @pytest.mark.parametrize("M, N, K", FASTER)
 def test_where_the_widened_weights_are(M, N, K):
     assert lib.qs_w4a8_per_group_scratch_bytes(M, N, K) == N * K
+
+
+def test_the_scratch_and_the_grid_are_bounded():
+    assert lib.qs_w4a8_per_group_scratch_bytes(2048, 65536, 8192) == 512 << 20
+    assert lib.qs_w4a8_per_group_scratch_bytes(2048, 65792, 8192) == 0
+    assert lib.qs_w4a8_per_group_scratch_bytes(2048, 32 * 65528, 128) == 32 * 65528 * 128 and lib.qs_w4a8_per_group_scratch_bytes(2048, 32 * 65536, 128) == 0
+
+
+P256 = 256                                                           # an address that nothing reads: both calls are refused before a launch
+
+
+def test_what_the_plain_entry_refuses_stays_refused():
+    M, N, K = 800, 5120, 4352                                        # the ring kernel, which reads channel scales in pairs
+    ops = [P256] * 4
+    for fn, tail in ((lib.qs_w4a8_per_group_gemm, ()), (lib.qs_w4a8_per_group_gemm_scratch, (P256, N * K))):
+        assert fn(*ops, P256 + 2, P256, P256, M, N, K, *tail, None) == -1 and b"4-byte" in lib.qs_last_error()
+    M, N, K = 1300, 4096, 1024                                       # channel pairs, which have no activation epilogue
+    for fn, tail in ((lib.qs_w4a8_per_group_gemm_silu_mul, ()), (lib.qs_w4a8_per_group_gemm_silu_mul_scratch, (P256, N * K))):
+        assert fn(*ops, P256, P256, P256, None, M, N, K, *tail, None) == -1 and b"tmp" in lib.qs_last_error()

@@ -52,6 +52,11 @@ def expect(t, dtype, name, contiguous=True):
         raise RuntimeError(f"{name} must be contiguous")
 
 
+# A device that had no memory for the scratch is not asked again for this many products: every such request makes torch's allocator give back what it holds.
+WITHOUT_SCRATCH = 63
+_without = {}                       # device -> products left (a count that threads lose costs a request more or less)
+
+
 def widened_scratch(M, N, K, like):
     """Scratch for a per-group product of many tokens (include/qserve_amd.h, qs_w4a8_per_group_scratch_bytes), or None: the product needs none - a decode
     step is not asked -, or there is no memory left for it."""
@@ -60,7 +65,12 @@ def widened_scratch(M, N, K, like):
     need = lib.qs_w4a8_per_group_scratch_bytes(M, N, K)
     if need <= 0:
         return None
+    left = _without.get(like.device, 0)
+    if left:
+        _without[like.device] = left - 1
+        return None
     try:
         return torch.empty((need,), dtype=torch.uint8, device=like.device)
     except torch.OutOfMemoryError:
+        _without[like.device] = WITHOUT_SCRATCH
         return None

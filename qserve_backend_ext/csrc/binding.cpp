@@ -15,6 +15,8 @@
 //   activation_ops.silu_and_mul .............................................. kernels/csrc/activation.cpp:25-39
 // The W8A8-only functions (invoke_dequant*, gelu_*, per-tensor-scale overloads) are out of scope:
 // they exist as names and raise.
+#include <atomic>
+
 #include <torch/extension.h>
 #include <ATen/hip/HIPContext.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
@@ -77,13 +79,21 @@ void gemm_per_group(torch::Tensor in_feats, torch::Tensor kernel, torch::Tensor 
     }
     const DeviceGuard guard(in_feats.device());
     const int M = (int)out_feats.size(-2), N = (int)out_feats.size(-1), K = (int)in_feats.size(1);
-    // scratch for the widened weights of a product of many tokens; without memory for it the product runs without
+    // scratch for the widened weights of a product of many tokens; without memory for it the product runs without, and so do the next 63 of the device (every such
+    // request makes the allocator give back what it holds)
+    static std::atomic<int> without[64];
     torch::Tensor scratch;
     const long long wanted = M > 256 ? qs_w4a8_per_group_scratch_bytes(M, N, K) : 0;
     if (wanted > 0) {
-        try {
-            scratch = torch::empty({(int64_t)wanted}, in_feats.options());
-        } catch (const c10::OutOfMemoryError&) {
+        std::atomic<int>& left = without[in_feats.get_device() & 63];
+        if (left.load(std::memory_order_relaxed) > 0) {
+            left.fetch_sub(1, std::memory_order_relaxed);
+        } else {
+            try {
+                scratch = torch::empty({(int64_t)wanted}, in_feats.options());
+            } catch (const c10::OutOfMemoryError&) {
+                left.store(63, std::memory_order_relaxed);
+            }
         }
     }
     if (scratch.defined()) {

@@ -891,7 +891,7 @@ __global__ __launch_bounds__(NWT * 64, 4) void decode_attention_mfma_kernel(
             }
         } else {
             // cache-missing loads through the buffer builtin (the compiler counts them; an asm load inside a retry loop is not
-            // safe - gemm_w4a8_ring.hip, the K-slice seam)
+            // safe - gemm_w4a8_ring.h, the K-slice seam)
             const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(xrow, 0, QS_ATTNQ_ROW * 4, 0x00020000);
             v4u raw[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
             if (tid2 < 256) {

@@ -389,7 +389,7 @@ int launch_splitk(const int8_t* A, const uint8_t* W, const int8_t* zeros, const 
 int qs_launch_gemm_pair(int mode, int outk, const int8_t* A, const uint8_t* W, const int8_t* zeros,
                         const int8_t* scales8, const void* wscales, const void* ascales, const void* wszs,
                         const void* assums, void* out, int M, int N, int K, hipStream_t stream);
-// decode ring kernel (gemm_w4a8_ring.hip)
+// decode ring kernel (gemm_w4a8_ring.h)
 int qs_launch_gemm_ring(int mode, int outk, int mt, int wn, const int8_t* A, const uint8_t* W, const int8_t* zeros,
                         const int8_t* scales8, const void* wscales, const void* ascales, const void* wszs,
                         const void* assums, void* out, int M, int N, int K, int mblocks, int ksplit, int* slabs,
@@ -474,7 +474,7 @@ int dispatch(const int8_t* A, const int8_t* W, const int8_t* zeros, const int8_t
             return qs_launch_gemm_tiled(MODE, outk, A, Wu, zeros, scales8, wscales, ascales, wszs, assums, out, M, N, K,
                                         tmt, stream);
     }
-    // decode shapes: LDS-DMA ring kernel with operands read one stage ahead (gemm_w4a8_ring.hip); variant 4000
+    // decode shapes: LDS-DMA ring kernel with operands read one stage ahead (gemm_w4a8_ring.h); variant 4000
     // disables it (A/B tests against the two older decode kernels below)
     // K slices need the slab / counter workspace: tiles * ksplit * (mt KiB * 4) bytes, one counter per tile
     auto ring_ws = [&](int mt, int mb, int ks, int** slabs, unsigned** counters) -> bool {
@@ -560,7 +560,7 @@ int dispatch(const int8_t* A, const int8_t* W, const int8_t* zeros, const int8_t
         // Measured override of the byte model (round 4, scripts/gpu_plan_check.sh, weights from HBM): where the model takes
         // <2,2> x 4 K slices over two token blocks and <2,1> x 2 slices fills the chip with the same 256 workgroups, the latter
         // is 3-7 % faster - a third of the slab traffic (stored, read, restored) on a launch that is HBM-bound, and since round 4
-        // the two token blocks share their weight stream in L2 (default cache policy, gemm_w4a8_ring.hip).  Llama-3-8B down_proj
+        // the two token blocks share their weight stream in L2 (default cache policy, gemm_w4a8_ring.h).  Llama-3-8B down_proj
         // (N = 4096, K = 14336) at 33-64 tokens: 14.4-14.7 vs 15.3-15.8 us per-channel, 19.6-19.9 vs 20.6-20.9 g128.  The byte
         // model puts the two 1 KB apart and cannot be tuned to separate them without flipping M = 32 (measured the other way).
         // (Inside the decode step the two are equal, 2.809 vs 2.813 ms: kept for the traffic - one slab per tile instead of three.)
@@ -836,7 +836,7 @@ extern "C" int qs_w4a8_per_group_gemm_silu_mul_scratch(const int8_t* in_feats, c
 // + norm + quant).  In this form the GEMM leaves its K slices as int32 planes [k_slices][M][N] - no cross-workgroup seam, no
 // epilogue - and qs_add_residual_rms_norm_general_planes sums the planes and applies the GEMM's epilogue arithmetic itself:
 // the kernel boundary that is there anyway is the hand-off (in-launch it costs a 2.4-3 us round trip under load, see
-// gemm_w4a8_ring.hip).  Geometry by the ring kernel's byte model with the seam replaced by the planes' traffic (written once,
+// gemm_w4a8_ring.h).  Geometry by the ring kernel's byte model with the seam replaced by the planes' traffic (written once,
 // read once: 8 bytes per element and slice, weighted by the CU : HBM rate ratio).
 namespace {
 struct PlanesGeo {

@@ -136,7 +136,7 @@ __global__ __launch_bounds__(512, 1) void w4a8_gemm_tiled(const int8_t* __restri
             (void)wid;
         }
     };
-    // OUTK == 2 (gate_up + silu * mul, see gemm_w4a8_ring.hip): N stacks [gate | up]; unit j = gate channels 32 j .. as its
+    // OUTK == 2 (gate_up + silu * mul, see gemm_w4a8_ring.h): N stacks [gate | up]; unit j = gate channels 32 j .. as its
     // tile row t = 0 and up channels N/2 + 32 j .. as t = 1; the workgroup writes 128 channels of the [M, N/2] result
     constexpr bool ACT = OUTK == 2;
     auto trow = [&](int unit, int t) { return ACT ? (t ? N / 64 + unit : unit) : unit * 2 + t; };

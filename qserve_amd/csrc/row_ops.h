@@ -34,7 +34,7 @@ constexpr int WIDE_ROW = 4096;
 __device__ __forceinline__ h8 load8(const _Float16* p) { return *reinterpret_cast<const h8*>(p); }
 
 // 16-byte loads that bypass the caches (sc0 sc1): rows another workgroup of the SAME launch published with write-through
-// stores (the fence-free seam of gemm_w4a8_ring.hip / attention_mfma.hip).  Buffer loads through the BUILTIN (aux 17 =
+// stores (the fence-free seam of gemm_w4a8_ring.h / attention_mfma.hip).  Buffer loads through the BUILTIN (aux 17 =
 // sc0 | sc1): the compiler counts them and waits before the first use.  (An inline-asm load would be invisible to it: the
 // first version of this file had one, and hipcc copied its destination registers before the data had landed -
 // cdna_hip_programming.md 5.7 item 1.)  `row` must be wave-uniform.

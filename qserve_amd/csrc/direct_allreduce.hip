@@ -65,7 +65,7 @@ __device__ __forceinline__ v4u ld16_sys(const uint8_t* p) {
     return v;
 }
 __device__ __forceinline__ void st16_sys(uint8_t* p, v4u v) {
-    asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" ::"v"(p), "v"(v) : "memory");
+    asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
 }
 
 // bounded wait for `*p` to reach epoch `ep` (wrap-safe); false on timeout

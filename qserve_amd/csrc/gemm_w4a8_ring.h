@@ -742,7 +742,9 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
                         const int pc = q * KG + kg;
                         if (NP % KG != 0 && pc >= NP) continue;
                         v4i* const dst = slab + ((size_t)kq * NP + pc) * 64;
-                        asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" ::"v"(dst), "v"(sum[q]) : "memory");
+                        // (s_nop 1: the store reads its four registers over several cycles, and the compiler, which does not look inside, may give
+                        // them to the very next instruction: two wait states are due.  -DQS_TIMING libraries did, rows 8 - 15 of a tile were wrong)
+                        asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" ::"v"(dst), "v"(sum[q]) : "memory");
                     }
                 }
                 return;
@@ -808,7 +810,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
                             if (NP % KG != 0 && pc >= NP) continue;
                             sum[q] += t[jb][q];
                             v4i* const dst = slab + ((size_t)z * NP + pc) * 64;
-                            asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" ::"v"(dst), "v"(sent) : "memory");
+                            asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" ::"v"(dst), "v"(sent) : "memory");
                         }
                     }
                 }

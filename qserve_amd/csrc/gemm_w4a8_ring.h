@@ -445,7 +445,12 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
     // per-group: the cheap form wherever no scale of the wave's 64 channels lets byte products carry
     auto carries = [&](const Raw& q) { return MODE == 1 && __builtin_amdgcn_ballot_w64(level2_carries(q.sdw)) != 0; };
     auto build_all = [&](const Raw& q, v4i (&a)[4]) __attribute__((always_inline)) {
-        if (MODE == 1 && !carries(q)) {
+#ifdef QS_TIMING
+        const bool exact = flags & 8192;                             // (build has the switch)
+#else
+        constexpr bool exact = false;
+#endif
+        if (MODE == 1 && !exact && !carries(q)) {
 #pragma unroll
             for (int cl = 0; cl < 4; ++cl) {
                 const Level2 l2 = level2_of(q.sdw, q.zdw, cl);
@@ -494,18 +499,25 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
         const int slot_n = slot + 1 == ns_ ? 0 : slot + 1;
         const int slot_d = slot == 0 ? ns_ - 1 : slot - 1;
         Raw qn;
+#ifdef QS_TIMING
+        const bool t_reads = !(flags & 64), t_mfma = !(flags & 32);   // timing builds only: results wrong by design
+#else
+        constexpr bool t_reads = true, t_mfma = true;
+#endif
         if constexpr (MT == 8 && MODE == 1) {
             // one set of activation operands, each read again behind its last product: two sets and the cheap unpacking do not fit the registers (128 tokens of
             // gate_up 30.2 us with two sets and the exact form, 28.7 with this; where half of the waves unpack later, so that a SIMD's two waves alternate, 33.7)
-            qn = read_raw(slot_n);
+            if (t_reads) qn = read_raw(slot_n);
             if (STEADY || i + ns - 1 < mine) issue(i + ns - 1, slot_d);
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
+                if (t_mfma) {
 #pragma unroll
-                for (int cl = 0; cl < 4; ++cl)
-                    acc[mt][cl] = __builtin_amdgcn_mfma_i32_16x16x64_i8(cur.a[cl], o0.b[mt], acc[mt][cl], 0, 0, 0);
-                o0.b[mt] = read_b(slot_n, mt);
-                if (mt == 0) {
+                    for (int cl = 0; cl < 4; ++cl)
+                        acc[mt][cl] = __builtin_amdgcn_mfma_i32_16x16x64_i8(cur.a[cl], o0.b[mt], acc[mt][cl], 0, 0, 0);
+                }
+                if (t_reads) o0.b[mt] = read_b(slot_n, mt);
+                if (mt == 0 && t_mfma) {
                     build_all(qn, nxt.a);
 #pragma unroll
                     for (int cl = 0; cl < 4; ++cl) asm volatile("" ::"v"(nxt.a[cl]));
@@ -513,18 +525,13 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
             }
             return;
         }
-#ifdef QS_TIMING
-        const bool t_reads = !(flags & 64), t_mfma = !(flags & 32);   // timing builds only: results wrong by design
-#else
-        constexpr bool t_reads = true, t_mfma = true;
-#endif
         if (t_reads) {
             qn = read_raw(slot_n);
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) nxt.b[mt] = read_b(slot_n, mt);
         }
         if (STEADY || i + ns - 1 < mine) issue(i + ns - 1, slot_d);
-        if (STEADY && MODE == 0) {
+        if (STEADY && MODE == 0 && t_mfma) {
             // the requests and the reads first, then one product after the other with the next operands' unpacking between them
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -580,7 +587,6 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
     // general rounds below for all of them a round had twelve branches, between the barrier and the operands it needs.  Before and after, us: 33 tokens 12288 x 4096
     // 11.6 -> 10.6, gate_up 28672 x 4096 17.2 -> 16.3, 128 tokens gate_up 27.4 -> 23.6, one token of 4096 x 11008 22.8 -> 18.0; per group 64 tokens gate_up 21.8 ->
     // 19.7, 12288 x 4096 34.1 -> 29.1 with 256 (with the cheap unpacking; scales with carries 18.1 -> 17.1, 16 tokens of gate_up).
-#ifndef QS_TIMING                                         // (timing builds keep the general rounds, which have their switches)
     if (ns == DEPTH) {
         for (; i + DEPTH < whole; i += 2) {
             wait_vm<(DEPTH - 3) * NDMA>();
@@ -593,7 +599,6 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
             slot = slot + 1 == DEPTH ? 0 : slot + 1;
         }
     }
-#endif
     for (; i < whole; i += 2) {                       // (`whole` may be odd)
 #ifdef QS_RING_TRACE
         unsigned long long ta = __builtin_amdgcn_s_memtime();

@@ -397,9 +397,8 @@ int qs_launch_gemm_ring(int mode, int outk, int mt, int wn, const int8_t* A, con
 // k that a workgroup of `wn` units and one of `ks` K slices spends rounds on; 0: the ring kernel does not take it.  The slices are whole pairs of 64-k stages, shared
 // out over 8 / wn groups.  Where that leaves groups without a stage in the last round, at least two rounds have to be full and at most an eighth may be lost:
 // Llama-2-7B's down_proj (K = 11 008, 172 stages) then has four slices of 43 where only 32 workgroups of two units fitted before, 18.2 -> 9.7 us for one token and 30.9 ->
-// 11.8 per group (whole steps of that model: 1 token 248 -> 210 / 336 -> 255 us, 64 tokens 405 -> 381 / 491 -> 436).  Over K = 1152 .. 18 944, N = 2048 .. 8192: 1 and 16
-// tokens 2.0 - 2.3 times as fast, none slower.  With more tokens the model's costs of slices with lost rounds are a quarter too low (at their plain cost 100 tokens of
-// 8192 x 11 008 took 26.3 us in place of 20.9; with it none of 64 shapes a size is slower): callers add it.
+// 11.8 per group (whole steps of that model: 1 token 248 -> 210 / 336 -> 255 us, 64 tokens 405 -> 381 / 491 -> 436).  With more than 16
+// tokens the model's costs of such shares are a quarter too low (at their plain cost 100 tokens of 8192 x 11 008 took 26.3 us in place of 20.9): callers add it.
 static long qs_ring_fits(int K, int ks, int mt, int wn, bool act) {
     const int kg = 8 / wn;
     if (K % 64 == 0 && (K / 64) % ks == 0 && (K / 64 / ks) % kg == 0) return K / ks;
@@ -407,6 +406,19 @@ static long qs_ring_fits(int K, int ks, int mt, int wn, bool act) {
     const int pairs = K / 128, low = 2 * (pairs / ks), high = 2 * ((pairs + ks - 1) / ks);
     const long k = (long)(high + kg - 1) / kg * kg * 64;
     return low >= 2 * kg && 8 * k * ks <= 9L * K ? k : 0;
+}
+// Shares that do not divide, in one slice, where no even geometry fits: the ring kernel or the register-staged split-K kernel, whose workgroups take any K and share a
+// CU?  By 10 600 random shapes of N = 512 .. 28 800, K = 1152 .. 21 632, 1 - 1024 tokens, ring / split-K in median and at worst:
+//  * 1 - 16 tokens: per channel from nine rounds on (K > 4096) 1.17 / .97 times as fast, shorter ones 1.06 / .86 and two-unit workgroups .8 - .9; per group 1.00 / .55, never;
+//  * 17 - 32: one-unit workgroups 1.1 - 1.5 / .97 (above 256 units and K < 2048 .98, .90 per group), two-unit ones .90 - .96;
+//  * 33 - 64: up to 256 units 1.3 - 2.2 / 1.03, above 1.0 / .88;
+//  * beyond: two- and four-unit workgroups 1.1 - 1.8 / 1.05; one-unit ones 1.2 - 2.5 up to 160 units and 128 tokens, 63 units and 256,
+//    47 units (per group 23); above .94 - 1.3 / .82.
+static bool qs_ring_over_splitk(int mode, int M, int units, int K, int wn) {
+    if (M <= 16) return mode == 0 && wn == 1 && K > 4096 && (units <= 256 || K >= 5120);
+    if (M <= 32) return wn == 1 && (units <= 256 || K >= 2048);
+    if (M <= 64) return units <= 256;
+    return wn > 1 || units <= (M <= 128 ? 160 : M <= 256 ? 63 : mode == 0 ? 47 : 23);
 }
 // compute-bound tiled kernel (gemm_w4a8_tiled.hip)
 int qs_launch_gemm_tiled(int mode, int outk, const int8_t* A, const uint8_t* W, const int8_t* zeros,
@@ -537,26 +549,34 @@ int dispatch(const int8_t* A, const int8_t* W, const int8_t* zeros, const int8_t
             if (own < 0) own = !g_qs_plan.active && qs_scratch_slot(stream) > 0;
             return own == 1;
         };
+        // ... (with: 1.0 - 4 times as fast, but for more than 256 units and up to 16 tokens, .81 - 1.05.)  In one slice: faster than any coarser even geometry and
+        // than the channel pairs further down (at worst 1.01), by qs_ring_over_splitk where neither would run.  (15 000 and 6 500 random shapes.)
         long best = -1;
         int bmt = 0, bwn = 0, bks = 1;
-        for (int ks = 1; ks <= (g_variant == QS_GEMM_RING_NO_KSLICES || act ? 1 : 4); ks *= 2)
-            for (int i = 0; i < 7; ++i) {
-                const int mt = geo[i][0], wn = geo[i][1];
-                if (mt == 8 && (MODE != 1 || ks > 1 || mt_all <= 4 || mt_all > 8 || g_variant == QS_GEMM_RING_NO_MT8)) continue;   // (65 .. 128 tokens)
-                const long slice = qs_ring_fits(K, ks, mt, wn, act);
-                if (N % (64 * wn) != 0 || !slice) continue;
-                if (ks > 1 && slice > 32768) continue;        // the seam's sentinel must stay out of reach of a partial sum
-                if (ks > 1 && slice * ks != K && !own_scratch()) continue;
-                const int mb = (mt_all + mt - 1) / mt;
-                const long blocks = (long)mb * (N / (64 * wn)) * ks;
-                if (ks > 1 && (long)mb * (N / (64 * wn)) > 256) continue;   // K slices are for under-filled grids only
-                // per-group: the level-2 dequant is VALU work per weight byte a workgroup streams (measured at M = 128, g128:
-                // qkv 16.0 us with (4,1) against 18.2 with the equal-bytes (2,2)) - charged as a quarter of the weight bytes
-                const long pg = MODE == 1 && g_variant != QS_GEMM_RING_NO_GROUP_TERM ? 8 * wn : 0;
-                long cost = ((blocks + 255) / 256) * (16 * mt + 32 * wn + pg) * slice * (ks > 1 ? 11 : 10) / 10 + seam(ks, mt);
-                if (slice * ks != K && M > 16) cost += cost / 4;       // (qs_ring_fits)
-                if (best < 0 || cost < best) best = cost, bmt = mt, bwn = wn, bks = ks;
-            }
+        bool splitk_next = false;
+        auto consider = [&](bool uneven) {
+            for (int ks = 1; ks <= (g_variant == QS_GEMM_RING_NO_KSLICES || act ? 1 : 4); ks *= 2)
+                for (int i = 0; i < 7; ++i) {
+                    const int mt = geo[i][0], wn = geo[i][1];
+                    if (mt == 8 && (MODE != 1 || ks > 1 || mt_all <= 4 || mt_all > 8 || g_variant == QS_GEMM_RING_NO_MT8)) continue;   // (65 .. 128 tokens)
+                    const long slice = qs_ring_fits(K, ks, mt, wn, act);
+                    if (N % (64 * wn) != 0 || !slice || (slice * ks != K) != uneven) continue;
+                    if (ks > 1 && slice > 32768) continue;        // the seam's sentinel must stay out of reach of a partial sum
+                    if (uneven && (ks > 1 ? !own_scratch() || (units > 256 && M <= 16) : splitk_next && !qs_ring_over_splitk(MODE, M, units, K, wn))) continue;
+                    const int mb = (mt_all + mt - 1) / mt;
+                    const long blocks = (long)mb * (N / (64 * wn)) * ks;
+                    if (ks > 1 && (long)mb * (N / (64 * wn)) > 256) continue;   // K slices are for under-filled grids only
+                    // per-group: the level-2 dequant is VALU work per weight byte a workgroup streams (measured at M = 128, g128:
+                    // qkv 16.0 us with (4,1) against 18.2 with the equal-bytes (2,2)) - charged as a quarter of the weight bytes
+                    const long pg = MODE == 1 && g_variant != QS_GEMM_RING_NO_GROUP_TERM ? 8 * wn : 0;
+                    long cost = ((blocks + 255) / 256) * (16 * mt + 32 * wn + pg) * slice * (ks > 1 ? 11 : 10) / 10 + seam(ks, mt);
+                    if (uneven && M > 16) cost += cost / 4;       // (qs_ring_fits)
+                    if (best < 0 || cost < best) best = cost, bmt = mt, bwn = wn, bks = ks;
+                }
+        };
+        consider(false);
+        splitk_next = best < 0 && !(((units >= 256 && M > 16) || M >= 384) && N % 128 == 0);
+        consider(true);
         // Measured override of the byte model (round 4, scripts/gpu_plan_check.sh, weights from HBM): where the model takes
         // <2,2> x 4 K slices over two token blocks and <2,1> x 2 slices fills the chip with the same 256 workgroups, the latter
         // is 3-7 % faster - a third of the slab traffic (stored, read, restored) on a launch that is HBM-bound, and since round 4
@@ -856,6 +876,7 @@ bool planes_geometry(int mode, int M, int N, int K, PlanesGeo& g) {
             if (mt == 8 && force < 0) continue;         // (measured: the 128-token geometry never wins as planes)
             const long slice = qs_ring_fits(K, ks, mt, wn, false);
             if (N % (64 * wn) != 0 || !slice) continue;
+            if (slice * ks != K && N > 8192 && force < 0) continue;     // (above, up to 16 tokens .74 - .95 of the even geometry's speed; below 1.1 - 3.7 times as fast)
             if (force >= 0 && force != 100 * (ks - 1) + 10 * mt + wn) continue;
             const int mb = (mt_all + mt - 1) / mt;
             const long blocks = (long)mb * (N / (64 * wn)) * ks;

@@ -81,6 +81,32 @@ def test_shares_that_do_not_divide_keep_one_slice_in_shared_scratch(per_group):
     assert [gemm_planes_plan(M, 4096, 11008, per_group) for M in (1, 16, 64)] == [4, 4, 4]
 
 
+# shapes measured on both sides (figures beside the rule): without an even geometry the split-K kernel's workgroups, which share a CU, are often the faster ones
+SPLIT_K = [(1, 576, 2304, 0), (2, 896, 1664, 0), (1, 17472, 1408, 0), (1, 6528, 4480, 1), (3, 25664, 1920, 1), (16, 1920, 2688, 1), (3, 16448, 20224, 1), (23, 896, 2176, 0),
+           (31, 25024, 1408, 1), (35, 22336, 1408, 0), (38, 26432, 1920, 1), (69, 11584, 10496, 0), (66, 25024, 1408, 0), (138, 6976, 7552, 0), (322, 8256, 4224, 0),
+           (344, 25280, 1920, 1), (449, 2240, 1408, 1)]
+RING = [(1, 640, 4864, 0), (8, 1344, 7808, 0), (1, 20160, 6528, 0), (17, 640, 1408, 0), (19, 15488, 4864, 1), (37, 1152, 1408, 0), (48, 12096, 16512, 0), (90, 896, 1152, 0),
+        (115, 4608, 4736, 0), (173, 3008, 20864, 0), (331, 11136, 1920, 0), (911, 832, 20864, 0), (706, 960, 19584, 1)]
+
+
+@pytest.mark.parametrize("M, N, K, per_group", SPLIT_K)
+def test_shares_that_do_not_divide_leave_these_to_split_k(M, N, K, per_group):
+    assert gemm_plan(M, N, K, bool(per_group))["family"] == "splitk"
+
+
+@pytest.mark.parametrize("M, N, K, per_group", RING)
+def test_shares_that_do_not_divide_are_taken_here(M, N, K, per_group):
+    p = gemm_plan(M, N, K, bool(per_group))
+    assert p["family"] == "ring" and p["k_slices"] == 1 and K // 64 % (8 // p["units"])
+
+
+def test_planes_above_8192_channels_keep_even_shares():
+    for per_group in (False, True):
+        assert gemm_planes_plan(13, 8192, 5632, per_group) == 2
+        for N, K in ((8512, 5632), (24576, 2816), (11968, 9728), (9280, 11264)):
+            assert gemm_planes_plan(5, N, K, per_group) == 1, (N, K)
+
+
 @pytest.mark.parametrize("tp", [2, 4, 8])
 def test_tensor_parallel_shards_use_the_ring_kernel(tp):
     M = 64 * tp

@@ -266,9 +266,10 @@ int qs_single_query_attention(const void* q, const void* k, const void* v, const
 /* Pair fusion for the decode loop (no reference counterpart): single_query_attention followed by
  * invoke_quant(_fuse_sum) of its output (llama_w4a8_unpad.py:253-282) as ONE call.  `out` receives the fp16 attention
  * output exactly as above; quant_out int8 [B, H*Dh], quant_scale half [B], quant_sum half [B] (may be NULL) receive what
- * qs_invoke_quant(quant_out, out, quant_sum, quant_scale, B, H*Dh) would write - BIT-IDENTICAL.  Where the chosen
- * attention kernel can finish the row itself (matrix-core KV4 kernel, no KV split, H*Dh <= 4096) this is one launch,
- * otherwise the two launches are issued here.  Uses the per-device arrival-counter scratch (same stream rule as above). */
+ * qs_invoke_quant(quant_out, out, quant_sum, quant_scale, B, H*Dh) would write - BIT-IDENTICAL.  Rows of H*Dh <= 4096 in this library's
+ * order of the row sum (qs_set_row_sum_order(0), or no quant_sum): the matrix-core KV4 kernel without a KV split finishes the row
+ * itself (one launch; uses the per-device arrival-counter scratch, same stream rule as above), and both matrix-core kernels with 2 to 8
+ * KV splits are followed by one launch that merges and quantises.  Otherwise attention (with its merge) and qs_invoke_quant are issued here. */
 int qs_single_query_attention_quant(const void* q, const void* k, const void* v, const int64_t* kv_pointers,
                                     const int32_t* length_per_sample, void* out, int8_t* quant_out, void* quant_sum,
                                     void* quant_scale, int batch, int num_heads, int num_kv_heads, int head_dim,

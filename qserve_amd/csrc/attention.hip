@@ -647,9 +647,9 @@ thread_local QsAttnPlan g_qs_attn_plan = {0, 0, 0, 0};
 thread_local QsAttnQuant g_qs_attn_quant = {nullptr, nullptr, nullptr, 0};
 
 // single_query_attention followed by invoke_quant(_fuse_sum) of its output, as ONE call (decode loop of
-// llama_w4a8_unpad.py:253-282: attention, reshape, self.invoke_quant).  Results are bit-identical to the two calls; where
-// the chosen attention kernel can finish the row itself (matrix-core KV4 kernel, no KV split, rows <= 4096) the row
-// kernel and a kernel boundary disappear, otherwise the two launches are issued here.
+// llama_w4a8_unpad.py:253-282: attention, reshape, self.invoke_quant).  Results are bit-identical to the two calls.  Rows of up to 4096
+// values in this library's order of the sum: the matrix-core KV4 kernel without a KV split finishes the row itself (attention_mfma.hip), and where there are
+// 2 to 8 KV splits, of either matrix-core kernel, merge and quantiser are one launch (fused_small.hip, merge_quant_kernel).  Otherwise the launches are issued here.
 extern "C" int qs_single_query_attention_quant(const void* q, const void* k, const void* v, const int64_t* kv_pointers,
                                                const int32_t* length_per_sample, void* out, int8_t* quant_out,
                                                void* quant_sum, void* quant_scale, int batch, int num_heads,

@@ -3,7 +3,7 @@
 //
 // For per-group weights, whose level-2 dequant is vector work beside the matrix instructions wherever it is done in the loop: once a weight here, in the four-wave
 // tile (gemm_w4a8_wide.hip) once a weight and 256 tokens.  Both are bound by the card's power under matrix load: 8192 tokens x 28672 x 4096 + silu 880 -> 769 us
-// (2.19 -> 2.50 POP/s; of the 769 35 are the widening, at 5.5 TB/s), 5331 x 12288 x 4096 253 -> 224, 5331 x 4096 x 11008 274 -> 218 (the last round of tiles cut),
+// (2.19 -> 2.50 POP/s; of the 769 30 are the widening, 178 MB at 5.9 TB/s), 5331 x 12288 x 4096 253 -> 224, 5331 x 4096 x 11008 274 -> 218 (the last round of tiles cut),
 // 1100 x 4096 x 14336 228 -> 117.  Per-channel weights gain nothing (8192 x 28672 x 4096 670 -> 700: the nibbles need no arithmetic, and packed they halve what LDS
 // delivers), 32 x 32 x 32 instructions lose (769 -> 791 with random data).  Where it is taken: qs_w4a8_per_group_scratch_bytes in gemm_w4a8.hip.
 //

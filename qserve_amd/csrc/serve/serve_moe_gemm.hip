@@ -37,7 +37,8 @@ constexpr int KS = 64;       // reduction elements per step
 // Measured (MI355X, one product out of memory, us, the form before -> now in one call; before: four phases of a quarter each, conditions in every step): 32768 slots of one
 // expert of 4096 x 4096 835 -> 745 (1480 TFLOP/s; hipBLASLt's dense product of that size 700), 890 slots for each of 32 experts of 5504 x 4096 1200 -> 1114 (1155),
 // 2048 of 16 of 1408 x 2048 171 -> 159, of 2048 x 1408 172 -> 164, 550 of 16 of 2816 x 2048 138 -> 124, 512 107 -> 101, 300 94 -> 84; of 64 - 128 slots the same (the weights out
-// of memory).  The card's power bounds it: it holds 1.5 GHz over random numbers and 2.1 over ones (745 -> 620 us).  What counts there is cycles, not bytes: the branches
+// of memory).  12 000 random shapes: in median 1.10 times as fast, gated 1.08; slower where few tiles wait for long reductions (up to 64 tiles and more than 3500 elements, by up to
+// 13 %; experts of up to 128 rows and more than 2500, 22 %: less is in flight).  The card's power bounds it: it holds 1.5 GHz over random numbers and 2.1 over ones (745 -> 620 us).  What counts there is cycles, not bytes: the branches
 // that a step held for the first and the last ones alone took 8 % (they are the forms with EDGE now), halving the barriers 2 %; operands that never miss L2
 // give 4 %, requests and reads left out altogether 18 and 8 %.  Eight waves without the half phase between them 785, four waves of 128 x 128 970 (one wave a SIMD has nothing
 // beside its own barriers and requests); tiles of 192 rows cost 0.89 of 256 (a step's time is its requests and reads as much as its products); another order of the
@@ -110,8 +111,8 @@ template <int ACT>
 __device__ __forceinline__ v2u grouped_result(v4f v, float limit) {
     if (ACT == 2) {
         // (the arithmetic of the steps' kernel and of the activation by itself, bit for bit.  It is 4.2 us of vector work a tile, three steps of its loop: with the hardware's
-        // exp2 and reciprocal the epilogue is 2.7 us in place of 6.9 and 8188 slots over 16 experts gated 2816 x 2048 take 107 us in place of 120, but exp2 of a rounded
-        // product loses a bit for every doubling of |x|, the reciprocal is 0 for gates below -87.3, and a prompt's units differ from a step's)
+        // exp2 and reciprocal 512 slots for each of 16 experts gated 2816 x 2048 take 97 us in place of 104 and 890 for each of 32 of 5504 x 4096 1133 in place of 1157, but
+        // exp2 of a rounded product loses a bit for every doubling of |x|, the reciprocal is 0 for gates below -87.3, and a prompt's units differ from a step's)
         float u0, u1;
         if (limit > 0.f) {                                          // clamped units: g sigmoid(1.702 g) (u + 1) (uniform over the launch)
             const float ga = fminf(v[0], limit), gb = fminf(v[2], limit);

@@ -48,12 +48,16 @@ def test_products_without_memory_for_scratch(gpu, compiled, monkeypatch):
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
     total = torch.cuda.get_device_properties(0).total_memory
-    before = torch.cuda.memory_stats()["num_ooms"]
     torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (1 << 20)) / total)
     try:
+        held = []                                                    # (what earlier tests left free inside segments of theirs)
+        with pytest.raises(torch.OutOfMemoryError):
+            while True:
+                held.append(torch.empty(N * K, dtype=torch.uint8, device=gpu))
+        before = torch.cuda.memory_stats()["num_ooms"]
         for out in outs[1:]:
             op.gemm_forward_cuda(X, W, z8, s8, ws, sa, out)
+        assert torch.cuda.memory_stats()["num_ooms"] - before == 1
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
-    assert torch.cuda.memory_stats()["num_ooms"] - before == 1
     assert all(torch.equal(outs[0].view(torch.int16), out.view(torch.int16)) for out in outs[1:])

@@ -32,7 +32,7 @@
 // A/B switches (qs_set_gemm_variant(5000 + bits); every setting computes the same results):
 //   1 = weight DMA with the default cache policy everywhere, 2 = non-temporal everywhere (default: non-temporal unless several
 //       token blocks share the weight bytes of a channel block and N <= 8192 - see launch_ring and `issue`)
-//   4 / 8 = (QS_TIMING libraries only) no cross-group reduction / leave behind the k loop: the price of the tail (round 5)
+//   4 / 8 = (QS_TIMING libraries only) no cross-group reduction / leave behind the k loop: the price of the tail
 //   32 / 64 = (libraries built with -DQS_TIMING only; ignored by the shipped library) timing only, WRONG RESULTS: no MFMA /
 //        no LDS operand reads (what is left is the DMA + barrier pipeline:
 //        gate_up at M = 64 17.5 us -> 16.3 / 16.8, both off 15.9 us = 4.2 us of head and tail + 512 KB per CU at 44 GB/s,
@@ -41,7 +41,7 @@
 //   128 = (set by the launcher) the armed one-shot fault of qs_debug_inject_fault: tile 0's K-slice producers do not deliver
 //   256 * d = ring depth d (3..6, if 160 KiB allow): sensitivity to the bytes in flight
 //   2048 = (set by the launcher) K slices across the XCDs (ring_coords); 4096 = keep every slice of a channel block on one XCD
-//        (the mapping of rounds 3-5; A/B of the activation traffic)
+//        (A/B of the activation traffic)
 //   8192 = (QS_TIMING libraries only, WRONG RESULTS) per-group launches without the level-2 dequant arithmetic
 extern qs_flag g_ring_flags;   // gemm_w4a8_ring.hip
 struct RingCall {
@@ -121,7 +121,7 @@ struct RingCoords {
 };
 // wave-uniform unsigned division by a small run-time divisor that is almost always a power of two (token blocks, K slices): a
 // shift then; the general form costs ~35 dependent scalar / vector instructions each - three of them stood in front of a
-// workgroup's first memory request (round 4, timeline trace: 1 200-1 400 cycles from kernel entry to the first request)
+// workgroup's first memory request (timeline trace: 1 200-1 400 cycles from kernel entry to the first request)
 __device__ __forceinline__ unsigned udivmod(unsigned x, unsigned d, unsigned& rem) {
     if ((d & (d - 1)) == 0) {
         const unsigned sh = (unsigned)__builtin_ctz(d);
@@ -136,7 +136,7 @@ __device__ __forceinline__ RingCoords ring_coords(int b, int N, int wn, int mblo
     const int per = mblocks * ksplit;                 // workgroups per channel block
     if (per > 1) {
         if (kxcd) {
-            // K slices ACROSS the XCDs (round 6; launch_ring sets it when ksplit is 2 / 4 / 8 and the channel blocks divide): XCD x
+            // K slices ACROSS the XCDs (launch_ring sets it when ksplit is 2 / 4 / 8 and the channel blocks divide): XCD x
             // = b % 8 serves K slice x / xs (xs = 8 / ksplit XCDs per slice) of the channel blocks j = x % xs (mod xs), every
             // token block of a channel block on the same XCD as before (its weights come from that L2) - so an L2 holds only ITS
             // K slice of the activation matrix instead of all of it: down_proj's [64, 14336] int8 matrix was fetched once per XCD
@@ -235,7 +235,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
     // (P >= MT), same ring slot.  Inside a piece, half hf of row 2a + b sits at 64-byte position 4a + 2(hf ^ (a & 1)) + b
     // and chunk c at 16-byte position c ^ ((-(row >> 2)) & 3): every 16 consecutive lanes of the DMA fetch two whole
     // lines, and the ds_read_b128 of one stage (lane (li, g): row li, chunk g of its half) is bank-conflict free for
-    // the instruction's lane groups {0-3, 12-15, 20-27}, {4-11, 16-19, 28-31}, ... (MI355X_MICROARCH.md, LDS; measured
+    // the instruction's lane groups {0-3, 12-15, 20-27}, {4-11, 16-19, 28-31}, ... (measured
     // 2.3 ns per wave read against 3.4 ns for the round-1 image, scripts/microbench_cufill.hip).
     auto aswz = [&](int j) { return (0 - j) & 3; };
     static_assert(KG % 2 == 0, "groups pair up for the activation image");
@@ -279,8 +279,8 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_addr)
                      : "memory");
     };
-    // weights that exactly ONE workgroup reads (one token block per channel block) are non-temporal (MI355X_MICROARCH.md
-    // "nt-weights": issued -> landed -18 %); with several token blocks the same bytes are wanted again by the neighbours on the
+    // weights that exactly ONE workgroup reads (one token block per channel block) are non-temporal (in a copy of the stream alone
+    // issued -> landed -18 %); with several token blocks the same bytes are wanted again by the neighbours on the
     // XCD a moment later, and a streamed line may be gone by then: default policy there (launch_ring;
     // in-run A/B at M = 64: qkv (2 token blocks) 8.45 -> 7.84 us, o (4) 6.66 -> 6.48, down (2 x 4 K slices) 14.05 -> 13.98,
     // gate_up (1 block) 16.97 -> 17.05 the other way; M = 128: qkv 11.70 -> 11.28, o 7.94 -> 7.70).  Measured exception: the
@@ -309,7 +309,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
         }
     };
 
-    // ---- epilogue operands (round 4): the per-channel / per-token scale vectors of the workgroup's tile are requested HERE,
+    // ---- epilogue operands: the per-channel / per-token scale vectors of the workgroup's tile are requested HERE,
     // by LDS-DMA into the top 2 KiB of the LDS window (above every ring and reduction area), by wave 0, ahead of the first
     // ring stage in its in-order queue (the counted ring waits are unaffected: the extra requests are OLDER than any stage).
     // Before, every lane loaded its own values from memory after the k loop - a dependent memory round trip between the last
@@ -366,7 +366,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
         }
     QS_STAMP(1);
     // Everything the k loop needs but the first requests do not - operand reader addresses, accumulators - is computed BEHIND
-    // the prologue (round 4, timeline trace: the first request left 1 200-1 400 cycles after kernel entry; with two waves per
+    // the prologue (timeline trace: the first request left 1 200-1 400 cycles after kernel entry; with two waves per
     // SIMD every instruction in front of it costs 4-5 cycles of a launch whose data is ~2.5 us away).  Nothing may be hoisted
     // back above the requests:
     __builtin_amdgcn_sched_barrier(0);
@@ -419,7 +419,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
         u32 s = 0, zb = 0;
 #ifdef QS_TIMING
         // timing builds only, WRONG RESULTS (flags & 8192): per-group launches keep their meta DMA and LDS reads but skip the level-2
-        // arithmetic - what the dequant VALU costs on top of the per-channel stream (round 6, config 3 decomposition)
+        // arithmetic - what the dequant VALU costs on top of the per-channel stream
         if (MODE == 1 && (flags & 8192)) {
             v4i a;
 #pragma unroll
@@ -561,7 +561,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
                     build_all(qn, nxt.a);
                 }
             }
-            // Per-group (round 6): the operands built for the NEXT round must be finished INSIDE this round, under its MFMAs.  Left to
+            // Per-group: the operands built for the NEXT round must be finished INSIDE this round, under its MFMAs.  Left to
             // itself the compiler sinks the second round's level-2 dequant (20 multiplies, ~120 VALU instructions) across the loop's
             // back edge to its use - in front of the first round's MFMAs: one round then carries 240 VALU instructions and its
             // MFMAs wait for them, the other round's 16 MFMAs run with nothing beside them (seen in the ISA: blocks of 16 MFMAs +
@@ -654,8 +654,8 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
     constexpr int NP = MT * 4;                         // 16 x 16 result pieces per wave: piece pc = mt*4 + cl
     // DISTRIBUTED: piece pc is finished by K-group pc % KG - every group sums, scales and converts a 1/KG share of the tile
     // instead of groups 1..KG-1 handing everything to group 0 and leaving (timeline trace, scripts/trace_gemm.py: reduction +
-    // epilogue on two of eight waves = 3 us of a 19 us launch at gate_up size; in-run A/B against the group-0 form in the r2
-    // builds: qkv 9.8 -> 8.7, o 7.5 -> 7.2, gate_up 19.5 -> 18.1 us).  Since round 4 the K-sliced launches take this form as
+    // epilogue on two of eight waves = 3 us of a 19 us launch at gate_up size; in-run A/B against the group-0 form in
+    // one run: qkv 9.8 -> 8.7, o 7.5 -> 7.2, gate_up 19.5 -> 18.1 us).  The K-sliced launches take this form as
     // well: all eight waves carry the seam's traffic (below).
     {
         constexpr int PPG = (NP + KG - 1) / KG;        // pieces per owning group
@@ -668,7 +668,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
                                                        // workgroup's 32 WN result channels in one row
         uint8_t* const st = smem + (size_t)KG * WN * (KG - 1) * PPP * 1024 + (ACT ? wn * 64 : wn * (16 * MT * RS));
         // The pieces this wave finishes are pc = q KG + kg, q < PPG.  Their accumulators are picked by wave-uniform SELECTS, not by
-        // branches (round 4: with one basic block per (q, kk) the four pieces of a gate_up wave ran one after the other, each
+        // branches (with one basic block per (q, kk) the four pieces of a gate_up wave ran one after the other, each
         // a chain LDS read -> sum -> scale -> exp / rcp -> LDS write with nothing to overlap it: 4 400 cycles between the two
         // barriers in the timeline trace; as straight-line code the reads of all pieces are in flight together).
         v4i sum[PPG];
@@ -725,13 +725,13 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
         QS_STAMP(11);
 #endif
         // ---- K-split seam (per wave: its own pieces of unit wn's tile) ------------------------------------------------------
-        // Round 4: no ticket, and every wave takes part.  The slabs hold a SENTINEL word (QS_SLAB_SENTINEL, a value no partial
+        // No ticket, and every wave takes part.  The slabs hold a SENTINEL word (QS_SLAB_SENTINEL, a value no partial
         // sum of an admitted K slice can take) wherever no partial has been delivered.  Slices 0 .. ksplit-2 store their
         // pieces (system-scope write-through, fire and forget) and leave; the LAST slice - dispatched last, so every slice it
         // waits for already holds a CU - loads the other slices' pieces with cache-missing loads, repeats the load while any
         // word still shows the sentinel, adds, and puts the sentinel back for the next launch (ordered by the kernel
         // boundary).  Before: acknowledged stores -> device-scope ticket -> loads by the last arriver, three dependent round
-        // trips, the last one 48 KB through ONE wave per unit (MI355X_MICROARCH.md handoff-payload: "one wave reading a fresh
+        // trips, the last one 48 KB through ONE wave per unit ("one wave reading a fresh
         // 64 KB slot = 4.9 us") - 9 000 cycles in the timeline trace at down's shape.
         // No fences (an agent-scope release / acquire writes back and invalidates the XCD's whole L2 under every other
         // workgroup's feet, measured +10 us): the slab traffic bypasses the caches (sc0 sc1), and the data is its own flag - a
@@ -754,7 +754,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
                 }
                 return;
             }
-            // BOUNDED (round 5): after `spin_cap` polls the wave stops waiting, reports through the device error word (`counters`
+            // BOUNDED: after `spin_cap` polls the wave stops waiting, reports through the device error word (`counters`
             // = qs_gemm_error_word()) and finishes with what it has - a wrong tile and a status bit instead of a hung GPU, if the
             // dispatch-order assumption above ever fails or the slabs were left without their sentinel (include/qserve_amd.h)
             const int spin_cap = (flags & 128) ? 4096 : QS_SPIN_CAP;
@@ -765,7 +765,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
             // cache-missing loads through the buffer BUILTIN (aux 17 = sc0 | sc1): the compiler counts them and waits before
             // the first use.  An inline-asm load is invisible to it - inside this retry loop the loaded registers are loop-
             // carried, and hipcc copied them BEFORE the asm's own s_waitcnt (seen in the ISA; the MT = 1 geometry returned
-            // garbage; cdna_hip_programming.md 5.7 item 1)
+            // garbage)
             const __amdgpu_buffer_rsrc_t srs = __builtin_amdgcn_make_buffer_rsrc(slabs, 0, 0x7FFFFFFF, 0x00020000);
             const u32 sl_off = (u32)((tile * ksplit * (size_t)(NP * 64) + lane) * 16);   // (the workspace is 48 MiB)
             for (int j0 = 0; j0 < ksplit - 1; j0 += ZB) {
@@ -829,7 +829,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
             if (NP % KG != 0 && pc >= NP) continue;    // (fewer pieces than groups: MT = 1 with eight K-groups)
             const int mt = pc >> 2, cl = pc & 3;
             if (OUTK == 1 || OUTK == 3) {
-                // OUTK == 3 (round 4): K-slice PLANES - every slice leaves its own int32 partial tile in plane kq of
+                // OUTK == 3: K-slice PLANES - every slice leaves its own int32 partial tile in plane kq of
                 // out [ksplit][M][N]; no seam at all: the consumer (the row kernel that follows, qs_add_residual_rms_norm_general_planes)
                 // sums the planes and applies this kernel's epilogue itself, and the kernel boundary is the hand-off
                 const int m = m0 + 16 * mt + li;
@@ -899,7 +899,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
     }
 }
 
-// MT m-tiles (16 tokens each) per wave = tokens per workgroup / 16 (1, 2, 4; 8 = 128-token workgroups, round 5: one level-2
+// MT m-tiles (16 tokens each) per wave = tokens per workgroup / 16 (1, 2, 4; 8 = 128-token workgroups: one level-2
 // dequant of a weight byte serves 128 tokens, ring depth 3-4, reduction through LDS in two passes); WN units per workgroup;
 // KG = 8 / WN K-groups.
 // KS = 0 folds every K-slice path away, 1 has K slices that the groups share out evenly, 2 any (also one).  (As one kernel 1 and 2 cost whole steps of one

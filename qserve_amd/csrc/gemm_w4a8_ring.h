@@ -279,7 +279,7 @@ __device__ __forceinline__ void ring_body(const int8_t* __restrict__ A, const ui
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_addr)
                      : "memory");
     };
-    // weights that exactly ONE workgroup reads (one token block per channel block) are non-temporal (in a copy of the stream alone
+    // weights that exactly ONE workgroup reads (one token block per channel block) are non-temporal (a stream by itself:
     // issued -> landed -18 %); with several token blocks the same bytes are wanted again by the neighbours on the
     // XCD a moment later, and a streamed line may be gone by then: default policy there (launch_ring;
     // in-run A/B at M = 64: qkv (2 token blocks) 8.45 -> 7.84 us, o (4) 6.66 -> 6.48, down (2 x 4 K slices) 14.05 -> 13.98,

@@ -20,9 +20,23 @@ int qsv_version(void);
 const char* qsv_arch(void);
 const char* qsv_last_error(void);
 
+/* The arguments of qsv_expert_slots_shared / _kept (sh_W NULL: no shared expert; kept: weights that are to stay in the caches), for launches that run the
+ * experts beside something that does not depend on them. */
+typedef struct {
+    void* out;
+    const void *X, *W;
+    const int32_t* idx;
+    const float* in_weight;
+    void* sh_out;
+    const void *sh_X, *sh_W;
+    int float_out, div, n, n_experts, rows, K, act, sh_n, sh_rows, sh_K, kept;
+    float limit;
+} qsv_expert_job;
 /* out [n_rows, N] = x [n_rows, K] @ w [N, K]^T, bfloat16 with float accumulation, for few rows (a decoding step); x_stride: elements from one
  * row of x to the next.  K and x_stride multiples of 8, x and w on 16 bytes. */
 int qsv_skinny_linear(void* out, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K, void* stream);
+/* The same beside the second products of a mixture's experts (float_out) that reads none of its results, in one launch.  kept: see qsv_skinny_linear_kept. */
+int qsv_skinny_linear_beside(void* out, int kept, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K, const qsv_expert_job* experts, void* stream);
 /* The same values in float. */
 int qsv_skinny_linear_widened(float* out, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K, void* stream);
 /* Either of them (widened: in float) with weights that are to stay in the caches; qsv_skinny_linear lets large ones that it reads once stream past them. */
@@ -397,6 +411,13 @@ int qsv_maps_attention(void* out, const void* q, const void* pool, const int32_t
                        const int32_t* prompt_tiles, int n_prompt, const int32_t* step_tiles, int n_step, int H, int G, int dim, int vdim,
                        int maps, int page, int64_t pool_stride, float lambda, float out_scale, float eps, const void* gate,
                        int64_t gate_stride, int key_splits, float* part_o, float* part_ml, void* stream);
+/* The step form (tiles of ONE token) beside the first products of a mixture of gated experts (act QSV_ACT_GLU or _CLAMPED_GLU) that reads none of its results, in
+ * one launch; the same results as two.  _ok: 1 where qsv_maps_attention_ok takes the sizes and two such workgroups fit a CU. */
+int qsv_maps_beside_ok(int dim, int vdim, int maps, int heads_per_pool);
+int qsv_maps_attention_beside(void* out, const void* q, const void* pool, const int32_t* block_table, int table_stride, const int32_t* pos,
+                              const int32_t* step_tiles, int n_step, int H, int G, int dim, int vdim, int maps, int page, int64_t pool_stride, float lambda,
+                              float out_scale, float eps, const void* gate, int64_t gate_stride, int key_splits, float* part_o, float* part_ml,
+                              const qsv_expert_job* experts, void* stream);
 /* q [T, H, 2, dim] (scaled), cache rows [v (vdim) | k_1 (dim) | k_2 (dim)] in G pools (head h reads pool h / (H / G)), keys 0 .. pos[t]:
  * a_m = softmax(q_m . k_m) v, o = a_1 - lambda a_2, out[t, h] = o / sqrt(mean(o^2) + eps) * out_scale * sigmoid(gate[t, h]) (gate NULL: no
  * gate); [T, H, vdim].  Any sizes up to dim 512 and vdim 1024. */

@@ -6,6 +6,7 @@
 // maps read the same rows in one pass; the combination, the norm and the gate are the epilogue.  With one map: plain causal attention.
 // Scores, maxima, sums, the outputs and their combination are float.
 #include "serve_common.h"
+#include "serve_expert_rows.h"
 
 #include <type_traits>
 #include <utility>
@@ -357,6 +358,10 @@ struct Shape {
     static constexpr int REGS = 16 * M * CT + 4 * M * DT;                            // accumulators + query fragments
     static constexpr int PROMPT_OCC = PROMPT_LDS <= 80 * 1024 && REGS <= 168 ? 2 : 1;
     static constexpr int STEP_OCC = STEP_LDS <= 80 * 1024 && REGS <= 168 ? 2 : 1;
+    // beside expert products: in their LDS, two workgroups a CU
+    static constexpr bool BESIDE = NW * BLOCK <= EXPERT_LDS && REGS <= 168;
+    static constexpr int BESIDE_BUFS = 2 * NW * BLOCK <= EXPERT_LDS ? 2 : 1;
+    static constexpr int beside_merge(int slots) { return NW * M * slots * (OROW + 2) * 4; }
 };
 
 struct MapsArgs {
@@ -675,15 +680,15 @@ __device__ __forceinline__ void finish_row(const MapsArgs& a, int n, FO src, FM 
     }
 }
 
-template <int DT, int CT, int M>
-__global__ __launch_bounds__(NT, (Shape<DT, CT, M>::STEP_OCC)) void maps_step_kernel(MapsArgs a) {
+// Workgroup (tile_at, y of ny, z) of a step.  BUFS: block buffers of a wave; the merge of the waves holds `slots` of the 32 rows (all of the tile's tokens'), its
+// maxima and sums behind them at smem + ml_at.
+template <int DT, int CT, int M, int BUFS>
+__device__ __forceinline__ void maps_step_block(const MapsArgs& a, int tile_at, int y, int ny, int z, unsigned char* smem, int slots, int ml_at) {
     using S = Shape<DT, CT, M>;
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int li = lane & 31, hi = lane >> 5;
-    const int y = blockIdx.y, z = blockIdx.z;
     const int pool_id = y / a.HG, h0 = pool_id * a.per + (y % a.HG) * 32, h_end = pool_id * a.per + a.per;
-    const int slot = a.tiles[3 * blockIdx.x], t0 = a.tiles[3 * blockIdx.x + 1], ntok = a.tiles[3 * blockIdx.x + 2];
+    const int slot = a.tiles[3 * tile_at], t0 = a.tiles[3 * tile_at + 1], ntok = a.tiles[3 * tile_at + 2];
     const bf16_t* pool = a.pool + (size_t)pool_id * (size_t)a.pool_stride;
     const int32_t* bt = a.block_table + (size_t)slot * a.table_stride;
     const int p_first = a.pos[t0], p_last = p_first + ntok - 1;
@@ -695,8 +700,8 @@ __global__ __launch_bounds__(NT, (Shape<DT, CT, M>::STEP_OCC)) void maps_step_ke
     if (a.Z == 1) gate.request(a, (size_t)(t0 + min(w / a.HP, ntok - 1)), min(h0 + w % a.HP, h_end - 1), lane);
     Rows<DT, CT, M> R;
     R.start(a.q + ((size_t)t * a.H + (ok ? head : 0)) * (M * S::DIM), hi);
-    const unsigned lds = (unsigned)(size_t)(lds_ptr)smem + w * S::BUFS * S::BLOCK;
-    const unsigned char* mine = smem + w * S::BUFS * S::BLOCK;
+    const unsigned lds = (unsigned)(size_t)(lds_ptr)smem + w * BUFS * S::BLOCK;
+    const unsigned char* mine = smem + w * BUFS * S::BLOCK;
     const int nT = p_last / BN + 1, stride = NW * a.Z, first = z * NW + w;
     PageIds pages(bt, (p_last >> a.page_shift) + 1, lane);
     auto copy = [&](int tile, int buf) {
@@ -709,28 +714,28 @@ __global__ __launch_bounds__(NT, (Shape<DT, CT, M>::STEP_OCC)) void maps_step_ke
     int i = 0;
     for (int tile = first; tile < nT; tile += stride, ++i) {
         const bool more = tile + stride < nT;
-        if (S::BUFS == 2 && more) {
+        if (BUFS == 2 && more) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");           // (the other buffer has been read)
             copy(tile + stride, (i + 1) & 1);
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"(S::PPR / 2) : "memory");    // this block has landed, the next one may be on its way
         } else {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
-        R.block(mine + (S::BUFS == 2 ? (i & 1) : 0) * S::BLOCK, tile * BN, p_row, tile * BN + BN - 1 > p_first, lane);
-        if (S::BUFS == 1 && more) {
+        R.block(mine + (BUFS == 2 ? (i & 1) : 0) * S::BLOCK, tile * BN, p_row, tile * BN + BN - 1 > p_first, lane);
+        if (BUFS == 1 && more) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             copy(tile + stride, 0);
         }
     }
     // ---- merge the four waves ----
-    float* so = (float*)smem;                                            // [NW][M][32][OROW]
-    float* sml = (float*)(smem + S::STEP_LDS - S::ML);                   // [NW][M][32][2]
+    float* so = (float*)smem;                                            // [NW][M][slots][OROW]
+    float* sml = (float*)(smem + ml_at);                                 // [NW][M][slots][2]
     __syncthreads();                                                     // every wave has read its last block
     if (ok) {
 #pragma unroll
         for (int f = 0; f < M; ++f) {
             const float l = R.l[f] + __shfl_xor(R.l[f], 32, 64);
-            const int row = (w * M + f) * 32 + li;
+            const int row = (w * M + f) * slots + li;
             if (hi == 0) {
                 sml[2 * row] = R.m[f];
                 sml[2 * row + 1] = l;
@@ -747,14 +752,14 @@ __global__ __launch_bounds__(NT, (Shape<DT, CT, M>::STEP_OCC)) void maps_step_ke
     for (int row = w; row < 32; row += NW) {
         const int rt = row / a.HP, rh = h0 + row % a.HP;
         if (rt >= ntok || rh >= h_end) continue;                         // (wave-uniform)
-        auto src = [&](int k, int f) { return so + ((k * M + f) * 32 + row) * S::OROW; };
-        auto ml = [&](int k, int f) { return sml + ((k * M + f) * 32 + row) * 2; };
+        auto src = [&](int k, int f) { return so + ((k * M + f) * slots + row) * S::OROW; };
+        auto ml = [&](int k, int f) { return sml + ((k * M + f) * slots + row) * 2; };
         if (a.Z == 1) {
             if (row != w) gate.request(a, (size_t)(t0 + rt), rh, lane);
             finish_row<S::VDIM, M>(a, NW, src, ml, (size_t)(t0 + rt), rh, lane, gate);
             continue;
         }
-        const size_t at = (((size_t)z * a.n_tiles + blockIdx.x) * gridDim.y + y) * 32 + row;
+        const size_t at = (((size_t)z * a.n_tiles + tile_at) * ny + y) * 32 + row;
 #pragma unroll
         for (int f = 0; f < M; ++f) {
             float mx = -INFINITY, L = 0.f;
@@ -781,6 +786,32 @@ __global__ __launch_bounds__(NT, (Shape<DT, CT, M>::STEP_OCC)) void maps_step_ke
     }
 }
 
+template <int DT, int CT, int M>
+__global__ __launch_bounds__(NT, (Shape<DT, CT, M>::STEP_OCC)) void maps_step_kernel(MapsArgs a) {
+    using S = Shape<DT, CT, M>;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    maps_step_block<DT, CT, M, S::BUFS>(a, blockIdx.x, blockIdx.y, gridDim.y, blockIdx.z, smem, 32, S::STEP_LDS - S::ML);
+}
+// A step's attention (its first `blocks` workgroups) beside the first products of a mixture of gated experts that reads nothing of it.  The one is a chain of
+// trips to memory on a few CUs, the other the weights' stream on all: in one launch the shorter costs nothing.  Sized for the experts - their LDS, 256 registers,
+// two workgroups a CU -, so the attention has one block buffer a wave where two take more, and keeps only its own heads' rows for the merge of its waves.
+// Attention, output product and experts apart -> both products' launches shared (MI355X, us, 16 heads on 4 pools, two maps of 64 over values of 128, 4 of 16 experts of
+// 2048 x 1408 and a shared one): 1 token behind 64 / 333 / 4000 positions 30.0 -> 19.5, 35.6 -> 21.7, 47.6 -> 35.1; 16 behind 300 72.6 -> 56.4; 64 behind 100 /
+// 1000 / 3000 77 -> 70, 99 -> 83, 153 -> 129; 4 of 32 experts of 4096 x 2752, 1 / 16 / 64 behind 333 / 300 / 8000 83 -> 69, 370 -> 353, 582 -> 544.  Faster at every size tried, so
+// wherever the sizes fit (maps of 128 over values of 128 need more registers, 32 heads a pool over wide values more LDS: those run apart).
+template <int DT, int CT, int M>
+__global__ __launch_bounds__(NT, 2) void maps_beside_experts_kernel(MapsArgs a, ExpertArgs e, SharedArgs sh, int blocks, int ny, int tiles) {
+    using S = Shape<DT, CT, M>;
+    __shared__ __attribute__((aligned(128))) unsigned char lds[EXPERT_LDS];
+    int b = blockIdx.x;
+    if (b < blocks) {
+        maps_step_block<DT, CT, M, S::BESIDE_BUFS>(a, b % a.n_tiles, b / a.n_tiles % ny, ny, b / a.n_tiles / ny, lds, a.HP, NW * M * a.HP * S::OROW * 4);
+        return;
+    }
+    b -= blocks;
+    expert_rows_block<ACT_GLU, false>(e, sh, b % tiles, b / tiles, lds);
+}
+
 template <int VDIM, int M>
 __global__ __launch_bounds__(NT) void maps_merge_kernel(MapsArgs a) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, y = blockIdx.y;
@@ -798,9 +829,30 @@ __global__ __launch_bounds__(NT) void maps_merge_kernel(MapsArgs a) {
 }
 
 template <int DT, int CT, int M>
-int launch_maps(MapsArgs a, const int32_t* prompt_tiles, int n_prompt, const int32_t* step_tiles, int n_step, int G, hipStream_t st) {
+int launch_maps(MapsArgs a, const int32_t* prompt_tiles, int n_prompt, const int32_t* step_tiles, int n_step, int G, hipStream_t st, const qsv_expert_job* beside) {
     using S = Shape<DT, CT, M>;
     const int gy = G * a.HG;
+    if (beside) {
+        if constexpr (S::BESIDE) {
+            ExpertArgs e;
+            SharedArgs sh;
+            dim3 grid;
+            int act = beside->act, rc = expert_slots_args("qsv_maps_attention_beside", *beside, e, sh);
+            if (rc == QSV_OK) rc = plan_expert_rows("qsv_maps_attention_beside", e, sh, beside->n_experts, act, beside->kept != 0, grid);
+            if (rc != QSV_OK) return rc;
+            const int64_t blocks = (int64_t)n_step * gy * a.Z, all = blocks + (int64_t)grid.x * grid.y;
+            QSV_REQUIRE(act == ACT_GLU && !beside->float_out && beside->n > 0 && n_prompt == 0 && n_step > 0 && all < (1ll << 31) && S::beside_merge(a.HP) <= EXPERT_LDS,
+                        "qsv_maps_attention_beside: not these experts or tiles");
+            a.tiles = step_tiles;
+            a.n_tiles = n_step;
+            hipLaunchKernelGGL((maps_beside_experts_kernel<DT, CT, M>), dim3((unsigned)all), dim3(NT), 0, st, a, e, sh, (int)blocks, gy, (int)grid.x);
+            rc = qsv_launch_status("qsv_maps_attention_beside");
+            if (rc != QSV_OK) return rc;
+            if (a.Z > 1) hipLaunchKernelGGL((maps_merge_kernel<S::VDIM, M>), dim3(n_step, gy), dim3(NT), 0, st, a);
+            return qsv_launch_status("qsv_maps_attention_beside (merge)");
+        }
+        QSV_REQUIRE(false, "qsv_maps_attention_beside: sizes it does not take");
+    }
     if (n_prompt > 0) {
         a.tiles = prompt_tiles;
         a.n_tiles = n_prompt;
@@ -848,10 +900,11 @@ extern "C" int qsv_maps_attention_tile_tokens(int heads_per_pool) { return heads
 // Rows of the step tiles' partial results per (tile, pool): 32 per head group of 32.
 extern "C" int qsv_maps_attention_head_groups(int heads_per_pool) { return heads_per_pool > 0 ? (heads_per_pool + 31) / 32 : 0; }
 
-extern "C" int qsv_maps_attention(void* out, const void* q, const void* pool, const int32_t* block_table, int table_stride, const int32_t* pos,
-                                  const int32_t* prompt_tiles, int n_prompt, const int32_t* step_tiles, int n_step, int H, int G, int dim,
-                                  int vdim, int maps, int page, int64_t pool_stride, float lambda, float out_scale, float eps, const void* gate,
-                                  int64_t gate_stride, int key_splits, float* part_o, float* part_ml, void* stream) {
+static int maps_attention(void* out, const void* q, const void* pool, const int32_t* block_table, int table_stride, const int32_t* pos,
+                          const int32_t* prompt_tiles, int n_prompt, const int32_t* step_tiles, int n_step, int H, int G, int dim,
+                          int vdim, int maps, int page, int64_t pool_stride, float lambda, float out_scale, float eps, const void* gate,
+                          int64_t gate_stride, int key_splits, float* part_o, float* part_ml, void* stream,
+                          const qsv_expert_job* beside) {
     QSV_REQUIRE(out && q && pool && block_table && pos && n_prompt >= 0 && n_step >= 0 && (!n_prompt || prompt_tiles) && (!n_step || step_tiles),
                 "qsv_maps_attention: null argument");
     QSV_REQUIRE(H > 0 && G > 0 && H % G == 0 && table_stride > 0 && pool_stride >= 0, "qsv_maps_attention: %d heads over %d", H, G);
@@ -866,10 +919,35 @@ extern "C" int qsv_maps_attention(void* out, const void* q, const void* pool, co
                   gate_stride, table_stride, 0, H, per, __builtin_ctz(page), head_slots(per), 32 / head_slots(per), HG, key_splits, lambda, out_scale, eps};
 #define QSV_MAPS_RUN(DT, CT, M)                      \
     if (dim == 16 * DT && vdim == 32 * CT && maps == M) \
-        return launch_maps<DT, CT, M>(a, prompt_tiles, n_prompt, step_tiles, n_step, G, (hipStream_t)stream);
+        return launch_maps<DT, CT, M>(a, prompt_tiles, n_prompt, step_tiles, n_step, G, (hipStream_t)stream, beside);
     QSV_MAPS_SHAPES(QSV_MAPS_RUN)
 #undef QSV_MAPS_RUN
     return QSV_EINVAL;
+}
+
+extern "C" int qsv_maps_attention(void* out, const void* q, const void* pool, const int32_t* block_table, int table_stride, const int32_t* pos,
+                                  const int32_t* prompt_tiles, int n_prompt, const int32_t* step_tiles, int n_step, int H, int G, int dim,
+                                  int vdim, int maps, int page, int64_t pool_stride, float lambda, float out_scale, float eps, const void* gate,
+                                  int64_t gate_stride, int key_splits, float* part_o, float* part_ml, void* stream) {
+    return maps_attention(out, q, pool, block_table, table_stride, pos, prompt_tiles, n_prompt, step_tiles, n_step, H, G, dim, vdim, maps, page, pool_stride, lambda,
+                          out_scale, eps, gate, gate_stride, key_splits, part_o, part_ml, stream, nullptr);
+}
+// 1 if the step kernel runs beside expert products for these sizes (that qsv_maps_attention_ok takes) with one token a tile
+extern "C" int qsv_maps_beside_ok(int dim, int vdim, int maps, int heads_per_pool) {
+    if (heads_per_pool <= 0) return 0;
+#define QSV_MAPS_BESIDE(DT, CT, M) \
+    if (dim == 16 * DT && vdim == 32 * CT && maps == M) return Shape<DT, CT, M>::BESIDE && Shape<DT, CT, M>::beside_merge(head_slots(heads_per_pool)) <= EXPERT_LDS;
+    QSV_MAPS_SHAPES(QSV_MAPS_BESIDE)
+#undef QSV_MAPS_BESIDE
+    return 0;
+}
+extern "C" int qsv_maps_attention_beside(void* out, const void* q, const void* pool, const int32_t* block_table, int table_stride, const int32_t* pos,
+                                         const int32_t* step_tiles, int n_step, int H, int G, int dim, int vdim, int maps, int page, int64_t pool_stride,
+                                         float lambda, float out_scale, float eps, const void* gate, int64_t gate_stride, int key_splits, float* part_o,
+                                         float* part_ml, const qsv_expert_job* experts, void* stream) {
+    QSV_REQUIRE(experts, "qsv_maps_attention_beside: null argument");
+    return maps_attention(out, q, pool, block_table, table_stride, pos, nullptr, 0, step_tiles, n_step, H, G, dim, vdim, maps, page, pool_stride, lambda, out_scale,
+                          eps, gate, gate_stride, key_splits, part_o, part_ml, stream, experts);
 }
 
 extern "C" int qsv_conv_heads_cache(void* q, void* pool, int64_t pool_rows, const void* proj, int64_t stride, const float* w, int taps, float* hist,

@@ -6,6 +6,7 @@
 // 8.8; 6144 x 2048 7.4 / 7.6 / 8.4 / 10.9 against 12.7 / 12.5 / 12.4 / 13.0; 32000 x 2048 27 / 28 / 30 / 47 against 34 / 34 / 35 / 35.
 // (Weights that pass once stream past the caches since: 32000 x 2048 of one or 16 rows 25 - 26 us, 4096 x 4096 8.9 -> 8.5.)
 #include "serve_common.h"
+#include "serve_expert_rows.h"
 #include "serve_stream.h"
 
 namespace {
@@ -24,11 +25,11 @@ struct SkinnyJob {
     int dim;
 };
 template <int RB, int SG, int HOW, bool ONCE>
-__device__ __forceinline__ void skinny_product(const SkinnyJob& a, int block, unsigned char* rings) {
+__device__ __forceinline__ void skinny_product(const SkinnyJob& a, int block, int inputs, unsigned char* rings) {
     constexpr int TILES = RB * SG;
     static_assert(STREAM_WAVES * TILES * 1024 <= STREAM_WAVES * XRING, "");
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int r0 = block * 16 * RB, t0 = blockIdx.y * 16 * SG, count = min(16 * SG, a.T - t0);
+    const int r0 = block * 16 * RB, t0 = inputs * 16 * SG, count = min(16 * SG, a.T - t0);
     v4f acc[RB][SG];
     stream_products<RB, SG, ONCE>(a.W + (size_t)r0 * a.K, a.K, min(16 * RB, a.N - r0), rings + w * XRING, w, lane,
                             [&](int i) { return a.X + (size_t)(t0 + min(i, count - 1)) * (size_t)a.x_stride; }, acc);
@@ -83,14 +84,24 @@ __device__ __forceinline__ void skinny_product(const SkinnyJob& a, int block, un
 template <int RB, int SG, int HOW, bool ONCE>
 __global__ __launch_bounds__(64 * STREAM_WAVES, 2) void skinny_linear_kernel(SkinnyJob a) {
     __shared__ __attribute__((aligned(128))) unsigned char rings[STREAM_WAVES * XRING];
-    skinny_product<RB, SG, HOW, ONCE>(a, blockIdx.x, rings);
+    skinny_product<RB, SG, HOW, ONCE>(a, blockIdx.x, blockIdx.y, rings);
 }
 // A recurrence's two second stages in one launch: the decay's product (its first `blocks` workgroups) and the output gate's (N 0: none)
 template <int SG>
 __global__ __launch_bounds__(64 * STREAM_WAVES, 2) void decay_products_kernel(SkinnyJob decay, SkinnyJob gate, int blocks) {
     __shared__ __attribute__((aligned(128))) unsigned char rings[STREAM_WAVES * XRING];
-    if ((int)blockIdx.x < blocks) skinny_product<1, SG, DECAY, false>(decay, blockIdx.x, rings);
-    else skinny_product<1, SG, AS_IS, false>(gate, blockIdx.x - blocks, rings);
+    if ((int)blockIdx.x < blocks) skinny_product<1, SG, DECAY, false>(decay, blockIdx.x, blockIdx.y, rings);
+    else skinny_product<1, SG, AS_IS, false>(gate, blockIdx.x - blocks, blockIdx.y, rings);
+}
+// A product (its first `blocks` workgroups, `columns` of them for the same inputs) beside the second products of a mixture's experts, which read nothing of it: a
+// launch and its start less (2048 x 2048 beside 4 of 16 experts of 2048 x 1408 and a shared one, 1 / 16 / 64 tokens 3.9 / 5.6 / 4.5 us; figures of a whole layer at
+// maps_beside_experts_kernel).
+template <int RB, int SG, bool ONCE>
+__global__ __launch_bounds__(64 * STREAM_WAVES, 2) void skinny_beside_experts_kernel(SkinnyJob a, ExpertArgs e, SharedArgs sh, int blocks, int columns, int tiles) {
+    __shared__ __attribute__((aligned(128))) unsigned char lds[EXPERT_LDS];
+    const int b = blockIdx.x;
+    if (b < blocks) skinny_product<RB, SG, AS_IS, ONCE>(a, b % columns, b / columns, lds);
+    else expert_rows_block<ACT_NONE, true>(e, sh, (b - blocks) % tiles, (b - blocks) / tiles, lds);
 }
 
 // ---- one product per head: y[t, h] = x[t, h] @ W[h], W [H, K, N] with N contiguous -------------------------------------------------------
@@ -250,9 +261,18 @@ static int skinny_fits(const char* what, const void* out, const void* x, int64_t
     return QSV_OK;
 }
 template <int HOW>
-static int launch_skinny(const char* what, void* out, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K, void* stream, bool kept = false) {
+static int launch_skinny(const char* what, void* out, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K, void* stream, bool kept = false, const qsv_expert_job* beside = nullptr) {
     const int rc = skinny_fits(what, out, x, x_stride, w, n_rows, N, K);
     if (rc != QSV_OK || n_rows == 0) return rc;
+    ExpertArgs e = {};
+    SharedArgs sh = {};
+    dim3 experts;
+    if (beside) {
+        int act = beside->act, rc2 = expert_slots_args(what, *beside, e, sh);
+        if (rc2 == QSV_OK) rc2 = plan_expert_rows(what, e, sh, beside->n_experts, act, beside->kept != 0, experts);
+        if (rc2 != QSV_OK) return rc2;
+        QSV_REQUIRE(beside->float_out && beside->n > 0 && (int64_t)experts.x * experts.y < (1ll << 30), "%s: not these experts", what);
+    }
     const SkinnyJob a = {out, (const bf16_t*)x, x_stride, (const bf16_t*)w, n_rows, N, K, N % 4 == 0 && (uintptr_t)out % (HOW == AS_IS ? 8 : 16) == 0, nullptr, nullptr, 0.f, 1};
     // 16 weight rows per workgroup where 32 would leave CUs without one, or need a second round for a few (8256 x 2048: 11.4 -> 10.5 us); else 32,
     // which reads the inputs half as often (6144 x 2048: 8.2 -> 7.4 us)
@@ -262,7 +282,15 @@ static int launch_skinny(const char* what, void* out, const void* x, int64_t x_s
 #define QSV_SKINNY(RB, SG)                                                                                                                    \
     do {                                                                                                                                      \
         const dim3 grid((N + 16 * RB - 1) / (16 * RB), (n_rows + 16 * SG - 1) / (16 * SG)), block(64 * STREAM_WAVES);                         \
-        if (once && (grid.y == 1 || (int64_t)grid.x * grid.y <= 256))                                                                        \
+        const bool past = once && (grid.y == 1 || (int64_t)grid.x * grid.y <= 256);                                                          \
+        if (beside) {                                                                                                                         \
+            if constexpr (HOW == AS_IS) {                                                                                                     \
+                const int64_t blocks = (int64_t)grid.x * grid.y, all = blocks + (int64_t)experts.x * experts.y;                               \
+                QSV_REQUIRE(all < (1ll << 31), "%s: too many workgroups", what);                                                              \
+                auto kernel = past ? skinny_beside_experts_kernel<RB, SG, true> : skinny_beside_experts_kernel<RB, SG, false>;                \
+                hipLaunchKernelGGL(kernel, dim3((unsigned)all), block, 0, (hipStream_t)stream, a, e, sh, (int)blocks, (int)grid.x, (int)experts.x); \
+            }                                                                                                                                 \
+        } else if (past)                                                                                                                      \
             hipLaunchKernelGGL((skinny_linear_kernel<RB, SG, HOW, true>), grid, block, 0, (hipStream_t)stream, a);                            \
         else hipLaunchKernelGGL((skinny_linear_kernel<RB, SG, HOW, false>), grid, block, 0, (hipStream_t)stream, a);                          \
     } while (0)
@@ -275,6 +303,12 @@ static int launch_skinny(const char* what, void* out, const void* x, int64_t x_s
 }
 extern "C" int qsv_skinny_linear(void* out, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K, void* stream) {
     return launch_skinny<AS_IS>("qsv_skinny_linear", out, x, x_stride, w, n_rows, N, K, stream);
+}
+// ... beside expert products into float (kept: w is to stay in the caches)
+extern "C" int qsv_skinny_linear_beside(void* out, int kept, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K, const qsv_expert_job* experts,
+                                        void* stream) {
+    QSV_REQUIRE(experts && n_rows > 0, "qsv_skinny_linear_beside: bad arguments");
+    return launch_skinny<AS_IS>("qsv_skinny_linear_beside", out, x, x_stride, w, n_rows, N, K, stream, kept != 0, experts);
 }
 // the same values in float
 extern "C" int qsv_skinny_linear_widened(float* out, const void* x, int64_t x_stride, const void* w, int n_rows, int N, int K, void* stream) {

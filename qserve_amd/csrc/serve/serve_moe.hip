@@ -3,10 +3,8 @@
 // Router scores are float from the first product to the chosen weights.  The expert kernels keep one token's input in LDS
 // and let every wave walk output rows with its lanes spread along the reduction (coalesced weight rows).
 #include "serve_common.h"
+#include "serve_expert_rows.h"
 #include "serve_route.h"
-#include "serve_stream.h"
-
-#include <type_traits>
 
 namespace {
 constexpr int NT = 256;
@@ -223,23 +221,6 @@ __global__ __launch_bounds__(NT, 2) void moe_route_wave_kernel(int32_t* __restri
     select_experts(s, lane_bias, lane_corr, {idx, weight, router, bias, correction, renorm, E, top_k, G, keep, score_fn, group_top, scale}, t, cs[w], lane);
 }
 
-// Activation of the first expert product.  ACT_GLU: the weight rows come in pairs (2f = gate, 2f + 1 = up) and output f is
-// silu(gate) * up, so the output is half as wide as the product.
-constexpr int ACT_NONE = 0, ACT_RELU_SQ = 1, ACT_GLU = 2;
-// (QSV_ACT_CLAMPED_GLU runs the ACT_GLU kernels with limit > 0: g = min(gate, limit), u = clamp(up, -limit, limit), g sigmoid(1.702 g) (u + 1))
-__device__ __forceinline__ float relu_sq(float d) {
-    const float a = fmaxf(d, 0.f);
-    return a * a;
-}
-__device__ __forceinline__ float glu(float g, float u, float limit) {
-    if (limit > 0.f) {                                       // (uniform over the launch)
-        g = fminf(g, limit);
-        u = fminf(fmaxf(u, -limit), limit);
-        return g / (1.0f + expf(-1.702f * g)) * (u + 1.0f);
-    }
-    return g / (1.0f + expf(-g)) * u;
-}
-
 // One workgroup per (token, chosen expert): act = relu(up_e . h)^2 (or the gated unit).  Dynamic LDS: D floats.  ff: weight rows.
 template <typename T, int ACT>
 __global__ __launch_bounds__(NT) void moe_up_kernel(T* __restrict__ act, const T* __restrict__ h, const T* __restrict__ up,
@@ -403,216 +384,11 @@ __global__ __launch_bounds__(NT) void moe_down_vec_kernel(T* __restrict__ y, con
     }
 }
 
-// ---- expert-major form (decoding and short portions, bfloat16): workgroup = (32 weight rows, expert), every weight read once per step
-// however many tokens share the expert.  Bound by HBM (the chosen experts' weights) and, below that, by launch latency.
-// * The slots (token t's k-th choice: slot t top_k + k) of an expert are found by the workgroup itself from the router's indices - no
-//   sort, no counts on the host - or given as sorted runs (`offsets`).
-// * The weights stream through per-wave LDS rings (serve_stream.h); the expert's inputs are read once per workgroup.
-// * The partial sums of the four waves meet in LDS; more than 32 slots per expert are walked in chunks (the weights then come from L2).
-// Two workgroups per CU keep up to 96 KiB of weights in flight.
-// Measured per launch in a step (MI355X): 64 tokens, 4 of 16 experts of 2048 x 1408 (92 MB a product) 55.6 / 62.4 us -> 23.8 / 21.1 us (up /
-// down) against the form it replaces, which kept weight rows in registers and paid a wave-wide sum per token and row; 16 tokens with
-// gated units (184 + 92 MB) 42.6 / 26.1 -> 36.5 / 19.3 us (5.0 TB/s); one token 1446 / 3117 us (the per-token kernels) -> 14.0 / 8.8 us.
-// The sort, search and permutation launches in front of it (60 us a layer) are gone.  Streamed past the caches, the shared expert in the same
-// launch: 64 tokens 22.7 / 19.4 us (98 MB), 16 tokens gated 33.8 / 17.6 (196 / 98 MB, 5.7 TB/s), one token 15.3 / 9.5 (before its workgroups were the slots').
-// 32 rows: 16, more evenly spread over the CUs, read the inputs twice as often and are slower everywhere (64 tokens 24.7 / 25.7, 16 tokens 36.3 / 21.4,
-// one 18.7 / 11.7), and so are 64; rings twice as deep give no more.
-constexpr int XR = 32;               // weight rows per workgroup
-constexpr int XLIST = 1024;          // router indices looked at in one go
-
-struct ExpertArgs {
-    void* out;                       // bf16, or float (no activation)
-    const bf16_t* X;
-    const bf16_t* W;
-    const int32_t* idx;              // the router's indices [n] (or NULL)
-    const int64_t* x_index;          // sorted runs: sorted slot -> slot (or NULL: itself)
-    const int64_t* offsets;
-    const float* in_weight;
-    int n, div, rows, K;
-    float limit;
-    bool wide;                       // out starts on 16 bytes
-    bool stored;                     // gated units are made from their halves as a tensor would hold them
-    bool once;                       // weights that one reading may stream past the caches
-    int by_slot;                     // workgroups by slot in place of expert (of this many experts; 0: by expert)
-};
-// An expert every token goes through, of sizes of its own: X row t, out row t in bfloat16, the bits that the products and the activation give one by one.
-// W NULL: none.  Alone it took four launches, three of them at 4 - 5 us whatever they read (16 experts of 2048 x 1408 and one more, top 4, with the router,
-// 1 / 16 / 64 tokens: 42 / 77 / 85 -> 32 / 63 / 71 us; of 4096 x 2752 106 / 387 / 432 -> 91 / 369 / 409).
-struct SharedArgs {
-    void* out;
-    const bf16_t *X, *W;
-    int n, rows, K;
-    bool wide, once;
-};
-
-// The four waves' partial sums (through LDS), the weight on the input, the activation, the store: slot of column c by slot_of(c).
-template <int ACT, bool FOUT, int SG, class Slot>
-__device__ __forceinline__ void expert_finish(const ExpertArgs& a, int r0, int count, unsigned char* rings, int w, int lane, Slot slot_of,
-                                              const v4f (&acc)[XR / 16][SG]) {
-    constexpr int TILES = XR / 16 * SG;
-    v4f* red = (v4f*)rings;                                                        // [wave][tile][lane]
-    __syncthreads();                                                               // every wave is done with its ring
-#pragma unroll
-    for (int r = 0; r < XR / 16; ++r)
-#pragma unroll
-        for (int g = 0; g < SG; ++g) red[(w * TILES + r * SG + g) * 64 + lane] = acc[r][g];
-    __syncthreads();
-#pragma unroll
-    for (int t0 = 0; t0 < TILES; t0 += NW) {
-        const int t = t0 + w, r = t / SG, c = 16 * (t % SG) + (lane & 15);
-        if (t < TILES && c < count) {
-            v4f v = red[t * 64 + lane];
-#pragma unroll
-            for (int o = 1; o < NW; ++o) v += red[(o * TILES + t) * 64 + lane];
-            const int n0 = r0 + 16 * r + 4 * (lane >> 4);
-            int64_t slot;
-            float iw = 1.0f;                                                       // the expert works on weight * input
-            slot_of(c, slot, iw);
-            v *= iw;
-            float u[4] = {v[0], v[1], v[2], v[3]};
-            int m = 4, stride = a.rows, at = n0;
-            if (ACT == ACT_GLU) {
-                if (a.stored) {
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) u[q] = bf2f(f2bf(u[q]));
-                }
-                u[0] = glu(u[0], u[1], a.limit);
-                u[1] = glu(u[2], u[3], a.limit);
-                m = 2;
-                stride /= 2;
-                at /= 2;
-            } else if (ACT == ACT_RELU_SQ) {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) u[q] = relu_sq(u[q]);
-            }
-            if (FOUT) {
-                float* o = (float*)a.out + (size_t)slot * stride + at;
-                if (a.wide && stride % 4 == 0 && at + 4 <= stride) *(v4f*)o = v4f{u[0], u[1], u[2], u[3]};
-                else
-                    for (int q = 0; q < m; ++q)
-                        if (at + q < stride) o[q] = u[q];
-            } else {
-                bf16_t* o = (bf16_t*)a.out + (size_t)slot * stride + at;
-                const unsigned lo = pack_bf2(u[0], u[1]);
-                if (a.wide && stride % m == 0 && at + m <= stride) {
-                    if (m == 2) *(unsigned*)o = lo;
-                    else *(uint2*)o = make_uint2(lo, pack_bf2(u[2], u[3]));
-                } else {
-                    for (int q = 0; q < m; ++q)
-                        if (at + q < stride) o[q] = f2bf(u[q]);
-                }
-            }
-        }
-    }
-    __syncthreads();                                                               // (the rings are free again)
-}
-
+// expert_rows_block (serve_expert_rows.h) as a launch of its own
 template <int ACT, bool FOUT>
 __global__ __launch_bounds__(NT, 2) void expert_rows_kernel(ExpertArgs a, SharedArgs sh) {
-    __shared__ __attribute__((aligned(128))) unsigned char rings[NW * XRING];
-    __shared__ unsigned short list[XLIST];
-    __shared__ int listed[NW];
-    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r0 = blockIdx.x * XR;
-    if (sh.W && blockIdx.y == 0) {                                                 // (first: it has the most inputs)
-        if (r0 >= sh.rows) return;
-        const ExpertArgs b = {sh.out, sh.X, sh.W, nullptr, nullptr, nullptr, nullptr, sh.n, 1, sh.rows, sh.K, a.limit, sh.wide, true, false, 0};
-        auto chunk = [&](int c0, auto once) __attribute__((always_inline)) {
-            constexpr bool ONCE = decltype(once)::value;
-            const int c = min(32, sh.n - c0);
-            auto rows = [&](int i) { return sh.X + (size_t)(c0 + min(i, c - 1)) * (size_t)sh.K; };
-            auto slots = [&](int i, int64_t& slot, float&) { slot = c0 + i; };
-            if (c <= 16) {
-                v4f acc[XR / 16][1];
-                stream_products<XR / 16, 1, ONCE>(sh.W + (size_t)r0 * sh.K, sh.K, min(XR, sh.rows - r0), rings + w * XRING, w, lane, rows, acc);
-                expert_finish<ACT, false, 1>(b, r0, c, rings, w, lane, slots, acc);
-            } else {
-                v4f acc[XR / 16][2];
-                stream_products<XR / 16, 2, ONCE>(sh.W + (size_t)r0 * sh.K, sh.K, min(XR, sh.rows - r0), rings + w * XRING, w, lane, rows, acc);
-                expert_finish<ACT, false, 2>(b, r0, c, rings, w, lane, slots, acc);
-            }
-        };
-        if (sh.n <= 32 && sh.once) chunk(0, std::true_type());
-        else
-            for (int c0 = 0; c0 < sh.n; c0 += 32) chunk(c0, std::false_type());
-        return;
-    }
-    if (r0 >= a.rows) return;
-    const int which = blockIdx.y - (sh.W ? 1 : 0), rows_here = min(XR, a.rows - r0);
-    int e = which;
-    if (a.by_slot) {                                                               // the expert of slot `which`, by its first slot
-        e = a.idx[which];
-        if ((unsigned)e >= (unsigned)a.by_slot) return;
-    }
-    const bf16_t* W0 = a.W + ((size_t)e * a.rows + r0) * (size_t)a.K;
-    unsigned char* ring = rings + w * XRING;
-    // `count` inputs: X row by row_of(i), output row (and weight) by slot_of(i)
-    auto walk = [&](int count, auto row_of, auto slot_of) {
-        auto chunk = [&](int c0, auto once) __attribute__((always_inline)) {
-            constexpr bool ONCE = decltype(once)::value;
-            const int c = min(32, count - c0);
-            auto rows = [&](int i) { return a.X + (size_t)row_of(c0 + min(i, c - 1)) * (size_t)a.K; };
-            auto slots = [&](int i, int64_t& slot, float& iw) { slot_of(c0 + i, slot, iw); };
-            if (c <= 16) {
-                v4f acc[XR / 16][1];
-                stream_products<XR / 16, 1, ONCE>(W0, a.K, rows_here, ring, w, lane, rows, acc);
-                expert_finish<ACT, FOUT, 1>(a, r0, c, rings, w, lane, slots, acc);
-            } else {
-                v4f acc[XR / 16][2];
-                stream_products<XR / 16, 2, ONCE>(W0, a.K, rows_here, ring, w, lane, rows, acc);
-                expert_finish<ACT, FOUT, 2>(a, r0, c, rings, w, lane, slots, acc);
-            }
-        };
-        if (count <= 0) return;
-        if (count <= 32 && a.once) chunk(0, std::true_type());
-        else
-            for (int c0 = 0; c0 < count; c0 += 32) chunk(c0, std::false_type());
-    };
-    if (a.offsets) {
-        const int64_t s0 = a.offsets[e];
-        walk((int)(a.offsets[e + 1] - s0),
-             [&](int i) {
-                 const int64_t s = s0 + i;
-                 return a.x_index ? a.x_index[s] / a.div : s;
-             },
-             [&](int i, int64_t& slot, float& iw) {
-                 slot = s0 + i;
-                 if (a.in_weight) iw = a.in_weight[a.x_index ? a.x_index[slot] : slot];
-             });
-        return;
-    }
-    for (int n0 = 0; n0 < a.n; n0 += XLIST) {
-        // this expert's slots among the next XLIST, in order: wave w looks at a quarter of them
-        const int len = min(XLIST, a.n - n0), span = (len + NT - 1) / NT * 64;
-        int found = 0;
-        unsigned long long hit[XLIST / NT];
-#pragma unroll
-        for (int q = 0; q < XLIST / NT; ++q) {
-            const int i = w * span + 64 * q + lane;
-            hit[q] = __ballot(64 * q < span && i < len && a.idx[n0 + i] == e);
-            found += __popcll(hit[q]);
-        }
-        if (lane == 0) listed[w] = found;
-        __syncthreads();
-        int at = 0, count = 0;
-#pragma unroll
-        for (int o = 0; o < NW; ++o) {
-            at += o < w ? listed[o] : 0;
-            count += listed[o];
-        }
-#pragma unroll
-        for (int q = 0; q < XLIST / NT; ++q) {
-            if (hit[q] >> lane & 1) list[at + __popcll(hit[q] & ((1ull << lane) - 1))] = (unsigned short)(w * span + 64 * q + lane);
-            at += __popcll(hit[q]);
-        }
-        __syncthreads();
-        if (a.by_slot && list[0] != which) return;                                 // (an earlier slot's workgroups do this expert)
-        walk(count, [&](int i) { return (int64_t)((n0 + list[i]) / a.div); },
-             [&](int i, int64_t& slot, float& iw) {
-                 slot = n0 + list[i];
-                 if (a.in_weight) iw = a.in_weight[slot];
-             });
-        __syncthreads();
-    }
+    __shared__ __attribute__((aligned(128))) unsigned char lds[EXPERT_LDS];
+    expert_rows_block<ACT, FOUT>(a, sh, blockIdx.x, blockIdx.y, lds);
 }
 
 // ---- expert-sorted form (many tokens): the products are the vendor's, per expert over contiguous runs of sorted slots; these
@@ -672,26 +448,10 @@ extern "C" int qsv_gather_rows(void* out, const void* src, const int64_t* order,
     return qsv_launch_status("qsv_gather_rows");
 }
 static int launch_expert_rows(const char* what, ExpertArgs a, int n_experts, int act, bool float_out, void* stream, SharedArgs sh = {}, bool kept = false) {
-    QSV_REQUIRE(a.out && a.X && a.W && n_experts > 0 && a.rows > 0 && a.div > 0, "%s: bad arguments", what);
-    QSV_REQUIRE(act == ACT_NONE || act == ACT_RELU_SQ || ((act == ACT_GLU || act == QSV_ACT_CLAMPED_GLU) && a.rows % 2 == 0), "%s: activation %d", what,
-                act);
-    QSV_REQUIRE(act != QSV_ACT_CLAMPED_GLU || a.limit > 0.f, "%s: clamped units need a positive limit", what);
-    if (act == QSV_ACT_CLAMPED_GLU) act = ACT_GLU;
-    else a.limit = 0.f;
-    // (a workgroup's rows within 32-bit byte offsets)
-    QSV_REQUIRE(a.K > 0 && a.K % 8 == 0 && a.K <= 1 << 25, "%s: inner width %d (a multiple of 8, at most 2^25)", what, a.K);
-    QSV_REQUIRE(n_experts <= 65535, "%s: too many experts", what);
-    QSV_REQUIRE(((uintptr_t)a.X | (uintptr_t)a.W) % 16 == 0, "%s: inputs and weights start on 16 bytes", what);
-    a.wide = (uintptr_t)a.out % 16 == 0;
-    a.once = !kept && streams_once(a.W, (int64_t)n_experts * a.rows, a.K);
-    sh.once = !kept && streams_once(sh.W, sh.rows, sh.K);
-    // Few slots: workgroups by slot, so that those of experts without one are not there.  Measured for both products of a token, us before and after: 1 token of 4 of
-    // 16 experts of 2048 x 1408 gated with a shared one 24.2 -> 20.3 (1496 and 1088 workgroups, of which 440 and 320 have rows), 2 tokens 29.2 -> 27.5, 1 token of
-    // 8 of 64 of 2048 x 768 35.0 -> 21.1.  The line: slots past half of the experts gain little and lose up to 4 % (3 tokens of the first: 37.3 -> 38.8, the empty
-    // workgroups between the others' are then few), and a grid that fits the chip at once loses .2 us to the load of the slot's expert.
-    const int tiles = ((sh.W && sh.rows > a.rows ? sh.rows : a.rows) + XR - 1) / XR;
-    a.by_slot = a.idx && a.n <= XLIST && 2 * a.n <= n_experts && (int64_t)n_experts * tiles > 512 ? n_experts : 0;
-    const dim3 grid(tiles, (a.by_slot ? a.n : n_experts) + (sh.W ? 1 : 0)), block(NT);
+    dim3 grid;
+    const int rc = plan_expert_rows(what, a, sh, n_experts, act, kept, grid);
+    if (rc != QSV_OK) return rc;
+    const dim3 block(NT);
     if (float_out) hipLaunchKernelGGL((expert_rows_kernel<ACT_NONE, true>), grid, block, 0, (hipStream_t)stream, a, sh);
     else if (act == ACT_RELU_SQ) hipLaunchKernelGGL((expert_rows_kernel<ACT_RELU_SQ, false>), grid, block, 0, (hipStream_t)stream, a, sh);
     else if (act == ACT_GLU) hipLaunchKernelGGL((expert_rows_kernel<ACT_GLU, false>), grid, block, 0, (hipStream_t)stream, a, sh);
@@ -712,32 +472,25 @@ extern "C" int qsv_expert_slots(void* out, int float_out, const void* X, int div
     return launch_expert_rows("qsv_expert_slots", a, n_experts, act, float_out != 0, stream);
 }
 // ... and, with sh_W, every token's row of X through a shared expert of sh_rows x sh_K in the same launch: sh_out [n / div, sh_rows (/ 2 for gated units)]
-static int expert_slots_shared(const char* what, bool kept, void* out, int float_out, const void* X, int div, const void* W, const int32_t* idx, int n, int n_experts,
-                               int rows, int K, int act, float limit, const float* in_weight, void* sh_out, const void* sh_X, const void* sh_W, int sh_n, int sh_rows,
-                               int sh_K, void* stream) {
-    QSV_REQUIRE(idx && n >= 0 && (!float_out || act == ACT_NONE) && n_experts < 65535, "%s: bad arguments", what);
-    if (sh_W) {
-        QSV_REQUIRE(sh_out && sh_X && sh_n > 0 && sh_rows > 0, "%s: bad arguments", what);
-        QSV_REQUIRE(sh_K > 0 && sh_K % 8 == 0 && sh_K <= 1 << 25 && ((uintptr_t)sh_X | (uintptr_t)sh_W) % 16 == 0, "%s: inner width %d, rows on 16 bytes", what, sh_K);
-        QSV_REQUIRE(act == ACT_NONE || act == ACT_RELU_SQ || sh_rows % 2 == 0, "%s: %d rows of gated units", what, sh_rows);
-    }
-    if (n == 0) return QSV_OK;
-    const ExpertArgs a = {out, (const bf16_t*)X, (const bf16_t*)W, idx, nullptr, nullptr, in_weight, n, div, rows, K, limit, false, false, false, 0};
-    const SharedArgs sh = {sh_out, (const bf16_t*)sh_X, (const bf16_t*)sh_W, sh_n, sh_rows, sh_K, (uintptr_t)sh_out % 16 == 0, false};
-    return launch_expert_rows(what, a, n_experts, act, float_out != 0, stream, sh_W ? sh : SharedArgs{}, kept);
+static int launch_expert_slots(const char* what, const qsv_expert_job& j, void* stream) {
+    QSV_REQUIRE(j.n_experts < 65535, "%s: bad arguments", what);
+    ExpertArgs a;
+    SharedArgs sh;
+    const int rc = expert_slots_args(what, j, a, sh);
+    return rc != QSV_OK || j.n == 0 ? rc : launch_expert_rows(what, a, j.n_experts, j.act, j.float_out != 0, stream, sh, j.kept != 0);
 }
 extern "C" int qsv_expert_slots_shared(void* out, int float_out, const void* X, int div, const void* W, const int32_t* idx, int n, int n_experts, int rows, int K,
                                        int act, float limit, const float* in_weight, void* sh_out, const void* sh_X, const void* sh_W, int sh_n, int sh_rows, int sh_K,
                                        void* stream) {
     QSV_REQUIRE(sh_W, "qsv_expert_slots_shared: bad arguments");
-    return expert_slots_shared("qsv_expert_slots_shared", false, out, float_out, X, div, W, idx, n, n_experts, rows, K, act, limit, in_weight, sh_out, sh_X, sh_W, sh_n,
-                               sh_rows, sh_K, stream);
+    return launch_expert_slots("qsv_expert_slots_shared", {out, X, W, idx, in_weight, sh_out, sh_X, sh_W, float_out, div, n, n_experts, rows, K, act, sh_n, sh_rows, sh_K, 0,
+                                                           limit}, stream);
 }
 // either of them (sh_W NULL: no shared expert) with weights that are to stay in the caches
 extern "C" int qsv_expert_slots_kept(void* out, int float_out, const void* X, int div, const void* W, const int32_t* idx, int n, int n_experts, int rows, int K, int act,
                                      float limit, const float* in_weight, void* sh_out, const void* sh_X, const void* sh_W, int sh_n, int sh_rows, int sh_K, void* stream) {
-    return expert_slots_shared("qsv_expert_slots_kept", true, out, float_out, X, div, W, idx, n, n_experts, rows, K, act, limit, in_weight, sh_out, sh_X, sh_W, sh_n, sh_rows,
-                               sh_K, stream);
+    return launch_expert_slots("qsv_expert_slots_kept", {out, X, W, idx, in_weight, sh_out, sh_X, sh_W, float_out, div, n, n_experts, rows, K, act, sh_n, sh_rows, sh_K, 1,
+                                                         limit}, stream);
 }
 extern "C" int qsv_relu_sq(void* a, int64_t n, int dtype, void* stream) {
     QSV_REQUIRE(a && n >= 0 && n < (1ll << 31) * NT, "qsv_relu_sq: bad arguments");

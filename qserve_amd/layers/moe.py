@@ -104,6 +104,14 @@ class SigmoidMoE:
         self.routing = dict(router=self.router, top_k=self.top_k, groups=self.groups, keep=self.keep, score="sigmoid", correction=self.correction, group_top=2,
                             scale=self.scale)
 
+    def pending(self, h, routed=None):
+        """The call with rows=True, its launches left to be made beside others' (qserve_amd.layers.ops.PendingExperts); None where it has to be called."""
+        plain = type(self.shared) is GatedFeedForward and self.shared.act == "silu"
+        if self.shared is not None and not plain:
+            return None
+        idx, wt = routed or self.ops.moe_route(h, **self.routing)
+        return self.ops.moe_experts_pending(h, self.up, self.down, idx, wt, *((self.shared.w_in, self.shared.w_down) if plain else (None, None)), weigh=self.weigh)
+
     def __call__(self, h, rows=False, routed=None):
         """rows: the caller takes the experts' rows (qserve_amd.layers.ops.ExpertRows) for the routed output and sums them itself.  routed: as above."""
         idx, wt = routed or self.ops.moe_route(h, **self.routing)

@@ -107,11 +107,19 @@ def _stream_product(x, w, out, kept):
     return out
 
 
-def linear(x, w, kept=False):
+def linear(x, w, kept=False, beside=None):
     """x [T, in] @ w [out, in]^T in the storage type, float accumulation: the few rows of a decoding step (bfloat16 on a GPU) through
-    qsv_skinny_linear, everything else through hipBLASLt / rocBLAS.  kept: w is to stay in the caches (see HipOps.kept_above)."""
+    qsv_skinny_linear, everything else through hipBLASLt / rocBLAS.  kept: w is to stay in the caches (see HipOps.kept_above).
+    beside: PendingExperts whose second products run in the same launch where there is one of ours."""
     if _streams(x, w):
-        return _stream_product(x, w, torch.empty((x.size(0), w.size(0)), dtype=x.dtype, device=x.device), kept)
+        out = torch.empty((x.size(0), w.size(0)), dtype=x.dtype, device=x.device)
+        job = None if beside is None else beside.take(1)
+        if job is None:
+            return _stream_product(x, w, out, kept)
+        from ..serving._lib import check, lib
+        check(lib().qsv_skinny_linear_beside(out.data_ptr(), int(kept), x.data_ptr(), x.stride(0), w.data_ptr(), x.size(0), w.size(0), x.size(1), job,
+                                             torch.cuda.current_stream(x.device).cuda_stream), "skinny_linear_beside")
+        return out
     return torch.matmul(x, w.t())
 
 
@@ -156,6 +164,32 @@ class ExpertRows:
         return y
 
 
+class PendingExperts:
+    """The two launches of a mixture's experts in a decoding step, not made yet: a kernel that reads nothing of them may take one along (`take`), and `results`
+    makes those that nobody took.  The second product reads the first one's results, so taking it makes the first if need be.  Everything happens on the stream
+    that was current when the object was made; it keeps the inputs alive until then."""
+
+    def __init__(self, ops, jobs, keeps, results):
+        self.ops, self.jobs, self.keeps, self._results, self.made, self.stream = ops, jobs, keeps, results, 0, ops._s()
+
+    def take(self, i):
+        """The arguments of launch i for the caller's own; None where it has been made already or another stream is current."""
+        if self.made > i or self.ops._s() != self.stream:
+            return None
+        self._make(i)
+        self.made = i + 1
+        return self.jobs[i]
+
+    def _make(self, n):
+        while self.made < n:
+            self.ops.expert_launch(self.jobs[self.made])
+            self.made += 1
+
+    def results(self):
+        self._make(2)
+        return list(self._results)
+
+
 def _on_four(*ts):
     """Whether four elements can be read at once from the start of every tensor."""
     return all(t is None or t.data_ptr() % (4 * t.element_size()) == 0 for t in ts)
@@ -184,8 +218,8 @@ class HipOps:
     def _kept(self, rows):
         return self.kept_above is not None and rows > self.kept_above
 
-    def linear(self, x, w):
-        return linear(x, w, self._kept(x.size(0)))
+    def linear(self, x, w, beside=None):
+        return linear(x, w, self._kept(x.size(0)), beside)
 
     def float_linear(self, x, w):
         return float_linear(x, w, self._kept(x.size(0)))
@@ -930,16 +964,16 @@ class HipOps:
         """Whether the matrix-core kernels of one or two key maps take these sizes."""
         return bool(self.L.qsv_maps_attention_ok(dim, vdim, maps, page, self.code))
 
-    def single_map_attention(self, q, pool, batch, heads, dim, vdim, page, key_splits=None):
+    def single_map_attention(self, q, pool, batch, heads, dim, vdim, page, key_splits=None, beside=None):
         """q [T, heads * dim] (storage type, scaled), pool [G, rows, vdim + dim] of rows [v | k]: causal softmax attention -> [T, heads * vdim];
         only for sizes that `maps_attention_ok` takes."""
         T = q.size(0)
         self._need(q, pool, batch.block_table, batch.pos)
         assert q.numel() == T * heads * dim and q.dtype == self.dtype == pool.dtype and pool.size(2) == vdim + dim and heads % pool.size(0) == 0
         out = torch.empty((T, heads * vdim), dtype=self.dtype, device=q.device)
-        return self._maps_attention(out, q, pool, batch, heads, dim, vdim, 1, page, (0.0, 1.0, 0.0, 0, 0), key_splits)
+        return self._maps_attention(out, q, pool, batch, heads, dim, vdim, 1, page, (0.0, 1.0, 0.0, 0, 0), key_splits, beside)
 
-    def _maps_attention(self, out, q, pool, batch, heads, dim, vdim, maps, page, epilogue, key_splits):
+    def _maps_attention(self, out, q, pool, batch, heads, dim, vdim, maps, page, epilogue, key_splits, beside=None):
         G, bt = pool.size(0), batch.block_table
         per = heads // G
         prompt, step = batch.split_tiles(self.L.qsv_maps_attention_tile_tokens(per))
@@ -950,13 +984,22 @@ class HipOps:
         if splits > 1:
             po = torch.empty((splits, n, groups, 32, maps, vdim), dtype=torch.float32, device=q.device)
             pm = torch.empty((splits, n, groups, 32, maps, 2), dtype=torch.float32, device=q.device)
+        job = None
+        if beside is not None and n == q.size(0) and self.L.qsv_maps_beside_ok(dim, vdim, maps, per):
+            job = beside.take(0)
+        if job is not None:
+            self.check(self.L.qsv_maps_attention_beside(out.data_ptr(), q.data_ptr(), pool.data_ptr(), bt.data_ptr(), bt.stride(0), batch.pos.data_ptr(),
+                                                        step.data_ptr(), n, heads, G, dim, vdim, maps, page, pool.stride(0), *epilogue, splits,
+                                                        0 if po is None else po.data_ptr(), 0 if pm is None else pm.data_ptr(), job, self._s()),
+                       "maps_attention_beside")
+            return out
         self.check(self.L.qsv_maps_attention(out.data_ptr(), q.data_ptr(), pool.data_ptr(), bt.data_ptr(), bt.stride(0), batch.pos.data_ptr(),
                                              prompt.data_ptr() if prompt.size(0) else 0, prompt.size(0), step.data_ptr() if n else 0, n, heads, G,
                                              dim, vdim, maps, page, pool.stride(0), *epilogue, splits, 0 if po is None else po.data_ptr(),
                                              0 if pm is None else pm.data_ptr(), self._s()), "maps_attention")
         return out
 
-    def diff_attention(self, q, pool, batch, heads, dim, vdim, lam, out_scale, eps, gate, page, variant=0, key_splits=None):
+    def diff_attention(self, q, pool, batch, heads, dim, vdim, lam, out_scale, eps, gate, page, variant=0, key_splits=None, beside=None):
         """q [T, heads * 2 * dim] (storage type, scaled; per head map 1, map 2), pool [G, rows, vdim + 2 dim] of rows [v | k_1 | k_2]: with a_m the
         softmax attention of map m over the keys up to the token, o = a_1 - lam a_2; -> o / sqrt(mean(o^2) + eps) * out_scale * sigmoid(gate) [T,
         heads * vdim] (gate [T, heads * vdim], a column slice is fine, or None).  variant: 0 = the matrix-core kernels where they take the
@@ -968,7 +1011,7 @@ class HipOps:
         out = torch.empty((T, heads * vdim), dtype=self.dtype, device=q.device)
         bt, ep = batch.block_table, (float(lam), float(out_scale), float(eps), 0 if gate is None else gate.data_ptr(), 0 if gate is None else gate.stride(0))
         if variant == 0 and self.maps_attention_ok(dim, vdim, 2, page) and (gate is None or (gate.stride(0) % 4 == 0 and gate.data_ptr() % 8 == 0)):
-            return self._maps_attention(out, q, pool, batch, heads, dim, vdim, 2, page, ep, key_splits)
+            return self._maps_attention(out, q, pool, batch, heads, dim, vdim, 2, page, ep, key_splits, beside)
         self.check(self.L.qsv_diff_attention(out.data_ptr(), q.data_ptr(), pool.data_ptr(), bt.data_ptr(), bt.stride(0), batch.seq.data_ptr(),
                                              batch.pos.data_ptr(), T, heads, G, dim, vdim, page, pool.stride(0), *ep, self.code, self._s()),
                    "diff_attention")
@@ -1119,11 +1162,7 @@ class HipOps:
     def moe_experts_shared(self, h, up, down, idx, wt, sh_up, sh_down, weigh="output", rows=False):
         """Gated experts as moe_experts (act "swiglu") beside a shared expert sh_up [2 sff, D], sh_down [D, sff] that every token goes through, in the same
         two launches -> (the experts' result, the shared expert's [T, D]); None where the sizes or the tokens make that the slower or an impossible way."""
-        (T, D), sff = h.shape, sh_down.size(1)
-        if not (0 < T <= self.moe_shared_tokens and self._expert_major(T * idx.size(1), up.size(0), up.size(1), D, up.size(1) // 2) and up.size(0) < 65535
-                and _called_plainly(h, sh_up, sh_down) and sff % 8 == 0 and sff <= 1 << 25 and sh_up.shape == (2 * sff, D) and sh_down.size(0) == D
-                and all(t.dtype == torch.bfloat16 and t.is_cuda and t.is_contiguous() for t in (h, sh_up, sh_down))
-                and all(t.data_ptr() % 16 == 0 for t in (sh_up, sh_down))):
+        if not self._shared_joins(h, up, down, idx, sh_up, sh_down):
             return None
         return self._moe_experts_expert_major(h, up, down, idx.to(torch.int32).contiguous(), wt, self.ACTS["swiglu"], 0.0, weigh, rows, (sh_up, sh_down))
 
@@ -1145,6 +1184,38 @@ class HipOps:
     # 1024 where the grouped kernel does not take the sizes - the vendor products wait for the runs' lengths and cannot be captured; 64 (moe_sorted_above) for
     # rows longer than 4096 (16 of 8192 x 4096, 64 slots 611 / 577; but 8 of 5120 x 5632, gated, 64 / 192 / 256: 210 / 294, 250 / 294, 360 / 296)
     moe_expert_major_slots = None
+
+    def _shared_joins(self, h, up, down, idx, sh_up, sh_down):
+        """Whether moe_experts_shared takes these."""
+        (T, D), sff = h.shape, sh_down.size(1)
+        return (0 < T <= self.moe_shared_tokens and self._expert_major(T * idx.size(1), up.size(0), up.size(1), D, up.size(1) // 2) and up.size(0) < 65535
+                and _called_plainly(h, sh_up, sh_down) and sff % 8 == 0 and sff <= 1 << 25 and sh_up.shape == (2 * sff, D) and sh_down.size(0) == D
+                and all(t.dtype == torch.bfloat16 and t.is_cuda and t.is_contiguous() for t in (h, sh_up, sh_down))
+                and all(t.data_ptr() % 16 == 0 for t in (sh_up, sh_down)))
+
+    def moe_experts_pending(self, h, up, down, idx, wt, sh_up, sh_down, weigh="output"):
+        """moe_experts_shared(..., rows=True) or, sh_up None, moe_experts(..., act "swiglu", rows=True), with its launches left to be made: -> PendingExperts
+        whose results() are [the experts' rows(, the shared expert's)]; None where that takes other launches than two by slot."""
+        T, D = h.shape
+        E, rows = up.size(0), up.size(1)
+        if not (T and E < 65535 and _called_plainly(h) and self._expert_major(T * idx.size(1), E, rows, D, rows // 2)):
+            return None
+        if sh_up is not None:
+            return self._shared_joins(h, up, down, idx, sh_up, sh_down) and self._moe_experts_expert_major(
+                h, up, down, idx.to(torch.int32).contiguous(), wt, self.ACTS["swiglu"], 0.0, weigh, True, (sh_up, sh_down), pending=True) or None
+        return self._moe_experts_expert_major(h, up, down, idx.to(torch.int32).contiguous(), wt, self.ACTS["swiglu"], 0.0, weigh, True, pending=True)
+
+    def expert_launch(self, job):
+        """One launch of qsv_expert_job's experts."""
+        j, s = job, self._s()
+        args = (j.out, j.float_out, j.X, j.div, j.W, j.idx, j.n, j.n_experts, j.rows, j.K, j.act, j.limit, j.in_weight)
+        shared = (j.sh_out, j.sh_X, j.sh_W, j.sh_n, j.sh_rows, j.sh_K)
+        if j.kept:
+            self.check(self.L.qsv_expert_slots_kept(*args, *shared, s), "expert_slots")
+        elif j.sh_W:
+            self.check(self.L.qsv_expert_slots_shared(*args, *shared, s), "expert_slots")
+        else:
+            self.check(self.L.qsv_expert_slots(*args, s), "expert_slots")
 
     def _grouped_takes(self, E, rows, D, ff):
         L = self.L
@@ -1169,7 +1240,7 @@ class HipOps:
                                           h.data_ptr(), E, self.code, self._s()), "moe_combine")
         return y
 
-    def _moe_experts_expert_major(self, h, up, down, idx, wt, a=1, limit=0.0, weigh="output", lazy=False, shared=None):
+    def _moe_experts_expert_major(self, h, up, down, idx, wt, a=1, limit=0.0, weigh="output", lazy=False, shared=None, pending=False):
         T, D = h.shape
         w_in, _ = self._weights_at(wt, weigh)
         E, rows, K = up.size(0), up.size(1), idx.size(1)
@@ -1179,20 +1250,25 @@ class HipOps:
         h, up, down = self._on_16_bytes(h, up, down)
         act = torch.empty((n, ff), dtype=self.dtype, device=h.device)
         ys = torch.empty((n, D), dtype=torch.float32, device=h.device)
-        s = self._s()
-        kept = self._kept(T)
-        sff, sy, first, second = 0, None, (0, 0, 0, 0, 0, 0), (0, 0, 0, 0, 0, 0)
+        kept = int(self._kept(T))
+        sy, first, second = None, (0, 0, 0), (0, 0, 0)
+        sff = 0
+        keeps = [h, up, down, idx, wt, act, ys]
         if shared is not None:
             sff = shared[1].size(1)
             sact, sy = torch.empty((T, sff), dtype=self.dtype, device=h.device), torch.empty((T, D), dtype=self.dtype, device=h.device)
-            first = (sact.data_ptr(), h.data_ptr(), shared[0].data_ptr(), T, 2 * sff, D)
-            second = (sy.data_ptr(), sact.data_ptr(), shared[1].data_ptr(), T, D, sff)
-        launch = self.L.qsv_expert_slots_kept if kept else self.L.qsv_expert_slots_shared if shared is not None else self.L.qsv_expert_slots
-        if not kept and shared is None:
-            first = second = ()
-        self.check(launch(act.data_ptr(), 0, h.data_ptr(), K, up.data_ptr(), idx.data_ptr(), n, E, rows, D, a, float(limit), w_in, *first, s), "expert_slots(up)")
-        self.check(launch(ys.data_ptr(), 1, act.data_ptr(), 1, down.data_ptr(), idx.data_ptr(), n, E, D, ff, 0, 0.0, 0, *second, s), "expert_slots(down)")
+            first = (sact.data_ptr(), h.data_ptr(), shared[0].data_ptr())
+            second = (sy.data_ptr(), sact.data_ptr(), shared[1].data_ptr())
+            keeps += [sact, sy, *shared]
+        sn = T if shared is not None else 0
+        from ..serving._lib import ExpertJob
+        jobs = (ExpertJob(act.data_ptr(), h.data_ptr(), up.data_ptr(), idx.data_ptr(), w_in, *first, 0, K, n, E, rows, D, a, sn, 2 * sff, D if sn else 0, kept, float(limit)),
+                ExpertJob(ys.data_ptr(), act.data_ptr(), down.data_ptr(), idx.data_ptr(), 0, *second, 1, 1, n, E, D, ff, 0, sn, D if sn else 0, sff, kept, 0.0))
         y = ExpertRows(self, ys, None, wt if weigh == "output" else None, idx, h, E)
+        if pending:
+            return PendingExperts(self, jobs, keeps, [y] if shared is None else [y, sy])
+        for job in jobs:
+            self.expert_launch(job)
         y = y if lazy else y.dense()
         return y if shared is None else (y, sy)
 
@@ -1274,7 +1350,7 @@ class TorchOps:
         dtype_code(dtype)
 
     @staticmethod
-    def linear(x, w):
+    def linear(x, w, beside=None):
         return linear(x, w)
 
     @staticmethod
@@ -1688,7 +1764,7 @@ class TorchOps:
     def maps_attention_ok(self, dim, vdim, maps, page):
         return False
 
-    def diff_attention(self, q, pool, batch, heads, dim, vdim, lam, out_scale, eps, gate, page, variant=0, key_splits=None):
+    def diff_attention(self, q, pool, batch, heads, dim, vdim, lam, out_scale, eps, gate, page, variant=0, key_splits=None, beside=None):
         T, G = q.size(0), pool.size(0)
         q, per, bt = q.view(T, heads, 2, dim).float(), heads // G, batch.block_table.long()
         o = torch.empty((T, heads, vdim), device=q.device)
@@ -1729,6 +1805,9 @@ class TorchOps:
         return a, b, m
 
     def moe_experts_shared(self, h, up, down, idx, wt, sh_up, sh_down, weigh="output", rows=False):
+        return None
+
+    def moe_experts_pending(self, *args, **kw):
         return None
 
     def moe_experts(self, h, up, down, idx, wt, act="relu_sq", limit=0.0, weigh="output", rows=False):

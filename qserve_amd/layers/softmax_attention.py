@@ -305,13 +305,13 @@ class DifferentialAttention:
         self.cache_rows = [] if shared_kv else [(kv_heads, vdim + 2 * dim)]
         self.state_specs = [StateSpec((taps - 1, self.C), copies=2)] if taps > 1 else []
 
-    def __call__(self, h, batch, pools, states):
+    def __call__(self, h, batch, pools, states, beside=None):
         ops, H, d, dv, pool = self.ops, self.H, self.dim, self.vdim, pools[0]
         proj = self.ops.linear(h, self.w_in)
         q = ops.conv_heads_cache(proj, self.conv, states[0] if self.taps > 1 else None, batch, 2 * H * d, 0 if self.shared_kv else self.G, 2 * d, dv,
                                  pool, self.scale, self.temperature)
-        o = ops.diff_attention(q, pool, batch, H, d, dv, self.lam, self.out_scale, self.eps, proj[:, self.C:self.C + H * dv], self.page)
-        return self.ops.linear(o, self.w_o)
+        o = ops.diff_attention(q, pool, batch, H, d, dv, self.lam, self.out_scale, self.eps, proj[:, self.C:self.C + H * dv], self.page, beside=beside)
+        return self.ops.linear(o, self.w_o, beside)
 
 
 class TiedRotaryAttention:
@@ -333,7 +333,7 @@ class TiedRotaryAttention:
         self.w_in, self.w_o = torch.cat([w["q"], w["k"]], dim=0).contiguous(), w["o"].contiguous()
         self.cache_rows, self.state_specs = [(kv_heads, 2 * dim)], []
 
-    def __call__(self, h, batch, pools, states):
+    def __call__(self, h, batch, pools, states, beside=None):
         ops, T, H, G, d, pool, rot = self.ops, h.size(0), self.H, self.G, self.dim, pools[0], self.rotary
         proj = self.ops.linear(h, self.w_in)
         k = proj[:, H * d:]
@@ -343,6 +343,6 @@ class TiedRotaryAttention:
                                   self.scale, pool, batch, halves=True, rot_gain=rot.magnitude ** 2 if rot is not None else 0.0,
                                   q_pad=0 if plain else d, q_store=plain)
         if plain:
-            return self.ops.linear(ops.single_map_attention(q, pool, batch, H, d, d, self.page), self.w_o)
+            return self.ops.linear(ops.single_map_attention(q, pool, batch, H, d, d, self.page, beside=beside), self.w_o, beside)
         o = ops.latent_attention(q, pool, batch, None, d, self.page, q_first=d)
         return self.ops.linear(o.view(T, H * d), self.w_o)

@@ -126,9 +126,12 @@ class Rivolix:
         x, hs, routed = norms(None, [], 0, tokens=batch.tokens, table=self.embed)
         for i, L in enumerate(self.layers):
             p0, p1, s0, s1 = self.slices[i]
-            parts = [(L["mixer"](hs[0], batch, pools[p0:p1], states[s0:s1]), L["ls1"])]
+            # neither side reads the other: a step's experts run in the launches of the mixer's attention and output product
+            experts = L["ff"].pending(hs[1], routed) if routed is not None else None
+            parts = [(L["mixer"](hs[0], batch, pools[p0:p1], states[s0:s1], beside=experts), L["ls1"])]
             if L["ff"] is not None:
-                parts += [(y, L["ls2"]) for y in L["ff"](hs[1], rows=True, routed=routed)]
+                ys = L["ff"](hs[1], rows=True, routed=routed) if experts is None else experts.results()
+                parts += [(y, L["ls2"]) for y in ys]
             # the next layer's two inputs come out of the pass that adds this layer's outputs to the stream
             _, hs, routed = norms(x, parts, i + 1)
             if tap is not None:

@@ -8,11 +8,20 @@ import os
 import threading
 
 _vp, _i, _i64, _f, _d = C.c_void_p, C.c_int, C.c_int64, C.c_float, C.c_double
+
+
+class ExpertJob(C.Structure):
+    """qsv_expert_job."""
+    _fields_ = ([(n, _vp) for n in ("out", "X", "W", "idx", "in_weight", "sh_out", "sh_X", "sh_W")]
+                + [(n, _i) for n in ("float_out", "div", "n", "n_experts", "rows", "K", "act", "sh_n", "sh_rows", "sh_K", "kept")] + [("limit", _f)])
+
+
 SIGNATURES = {
     "qsv_version": (_i, []),
     "qsv_arch": (C.c_char_p, []),
     "qsv_last_error": (C.c_char_p, []),
     "qsv_skinny_linear": (_i, [_vp, _vp, _i64, _vp, _i, _i, _i, _vp]),
+    "qsv_skinny_linear_beside": (_i, [_vp, _i, _vp, _i64, _vp, _i, _i, _i, C.POINTER(ExpertJob), _vp]),
     "qsv_skinny_linear_widened": (_i, [_vp, _vp, _i64, _vp, _i, _i, _i, _vp]),
     "qsv_skinny_linear_kept": (_i, [_vp, _i, _vp, _i64, _vp, _i, _i, _i, _vp]),
     "qsv_decay_products": (_i, [_vp, _vp, _i64, _vp, _i, _i, _vp, _vp, _f, _i, _vp, _vp, _i64, _vp, _i, _i, _i, _vp]),
@@ -99,6 +108,9 @@ SIGNATURES = {
     "qsv_maps_attention_head_groups": (_i, [_i]),
     "qsv_maps_attention": (_i, [_vp, _vp, _vp, _vp, _i, _vp, _vp, _i, _vp, _i, _i, _i, _i, _i, _i, _i, _i64, _f, _f, _f, _vp, _i64, _i, _vp, _vp,
                                 _vp]),
+    "qsv_maps_beside_ok": (_i, [_i, _i, _i, _i]),
+    "qsv_maps_attention_beside": (_i, [_vp, _vp, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i64, _f, _f, _f, _vp, _i64, _i, _vp, _vp, C.POINTER(ExpertJob),
+                                       _vp]),
     "qsv_recurrent_scan": (_i, [_vp, _vp, _i64, _vp, _i64, _vp, _i64, _i, _vp, _vp, _i64, _i, _vp, _vp, _i, _i, _i, _i, _i, _i, _f, _vp,
                                 _i, _i, _vp]),
     "qsv_head_rms_gate": (_i, [_vp, _vp, _vp, _vp, _i64, _i, _f, _i, _i, _i, _i, _i, _vp, _i, _vp]),

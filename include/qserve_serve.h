@@ -276,6 +276,11 @@ int qsv_scaled_sum_rms_norms_route(float* x, void* h0, void* h1, const void* a, 
 int qsv_hc_write_route(float* x, const void* y, const float* mix, const float* w_out, int n, int streams, int D, void* h_next, const float* w_in_next,
                        const void* norm_w, const void* norm_b, float alpha, int32_t* idx, float* weight, const void* router, const void* bias, int renorm, int E,
                        int top_k, int G, int keep, int score_fn, const float* correction, int group_top, float scale, void* stream);
+/* ... where y = (rms_norm(a) * wa + rms_norm(b) * wb) / 2, as qsv_rms_pair_mean makes it. */
+int qsv_hc_write_pair_route(float* x, const void* a, const void* wa, const void* b, const void* wb, float eps, const float* mix, const float* w_out, int n, int streams,
+                            int D, void* h_next, const float* w_in_next, const void* norm_w, const void* norm_b, float alpha, int32_t* idx, float* weight,
+                            const void* router, const void* bias, int renorm, int E, int top_k, int G, int keep, int score_fn, const float* correction, int group_top,
+                            float scale, void* stream);
 
 /* Grouped top-k router: scores s = softmax(router . h[t]) over n_experts (score_fn QSV_SCORE_SOFTMAX) or sigmoid(router . h[t])
  * (QSV_SCORE_SIGMOID); the choice goes by c = s + correction (float [n_experts], may be NULL: c = s).  The experts form n_groups
@@ -376,6 +381,11 @@ int qsv_hc_write(float* x, const void* y, const float* mix, const float* w_out, 
 /* The same (without h_next) with y[t] the sum over a mixture's experts (see qsv_scaled_sum_rms_norms_slots; width a multiple of 4). */
 int qsv_hc_write_slots(float* x, const void* ys, int float_rows, const int32_t* place, const float* weight, const int32_t* idx, int top_k, int n_experts,
                        const float* mix, const float* w_out, int n_tokens, int streams, int width, int dtype, void* stream);
+/* The same over a step's float rows (place NULL, every run one token, up to four streams) with the next sublayer's input from the new streams, token-shifted, as
+ * qsv_hc_read makes it. */
+int qsv_hc_write_slots_read(float* x, const float* ys, const float* weight, const int32_t* idx, int top_k, int n_experts, const float* mix, const float* w_out, int n_tokens,
+                            int streams, int width, void* h_next, const float* w_in, const void* norm_w, const void* norm_b, float alpha, const void* shift, float* prev,
+                            const int32_t* state_rd, const int32_t* state_wr, int dtype, void* stream);
 /* out[r] = tanh(alpha * sum_s x[rows[r], s]) * norm_w + norm_b  (rows == NULL: row r). */
 int qsv_dyt_sum_rows(void* out, const float* x, const int32_t* rows, const void* norm_w, const void* norm_b, float alpha,
                      int n_rows, int streams, int width, int dtype, void* stream);
@@ -460,6 +470,12 @@ int qsv_recurrent_scan(float* o, const void* q, int64_t q_stride, const void* k,
                        int64_t v_stride, int qkv_dtype, const float* decay, const void* beta, int64_t beta_stride,
                        int beta_dtype, float* state, const int32_t* runs, int n_runs, int max_run, int heads, int qk_heads,
                        int dim, int vdim, float q_scale, const float* kscale, int head_decay, int v_cols, void* stream);
+/* qsv_recurrent_scan over runs of one token each and qsv_head_rms_gate (bfloat16, one weight row for all heads) of its read-out, in one launch; vdim a power of two up
+ * to 128, dim a multiple of 8 up to 256, strides and addresses multiples of four elements. */
+int qsv_recurrent_step_gated(void* out, const void* q, int64_t q_stride, const void* k, int64_t k_stride, const void* v, int64_t v_stride, int qkv_dtype,
+                             const float* decay, const void* beta, int64_t beta_stride, int beta_dtype, float* state, const int32_t* runs, int n_runs, int heads,
+                             int qk_heads, int dim, int vdim, float q_scale, int head_decay, const void* w, const void* gate, int64_t gate_stride, int gate_kind,
+                             float eps, void* stream);
 /* out[t, h] = o[t, h] / rms(o[t, h]) * w * gate_fn(gate[t, h]) over vdim; gate_kind 0: silu, 1: sigmoid.  o's heads are o_stride
  * floats apart (0: vdim); w is [vdim], shared by the heads, or with w_per_head [heads, vdim].  den_m (float [T, heads], may be
  * NULL): o[t, h] is first divided by max(|o[t, h, vdim]|, exp(-den_m[t, h])) + 1e-6 (o_stride > vdim: the extra column). */

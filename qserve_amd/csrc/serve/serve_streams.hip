@@ -176,15 +176,28 @@ __global__ __launch_bounds__(NT) void hc_read_vec_kernel(T* __restrict__ h, cons
     }
 }
 
+// The next sublayer's input where that reads with a token shift and every run is one token: what hc_read_vec_kernel makes of the streams just written.
+template <typename T>
+struct ShiftedRead {
+    T* h;
+    const float* w_in;
+    const T *nw, *nb, *shift;
+    float* prev;
+    const int32_t *rd, *wr;
+    float alpha;
+};
+
 // (Y other than void: y is what a mixture of experts left per slot, float or the storage type; it is summed here, and rounded as a tensor would hold it)
 // MS: streams at most; up to four of them are requested at once, with the mix beside them (a stream that there is not repeats the last).
-template <typename T, typename Y = void, int MS = MAX_STREAMS>
+// STEP (up to four streams, rows of experts): with the next sublayer's shifted input, a launch less between two layers of a step.
+template <typename T, typename Y = void, int MS = MAX_STREAMS, bool STEP = false>
 __global__ __launch_bounds__(NT) void hc_write_vec_kernel(float* __restrict__ x, const T* __restrict__ y, const float* __restrict__ mix,
                                                           const float* __restrict__ w_out, int S, int D, T* __restrict__ h_next,
                                                           const float* __restrict__ w_in_next, const T* __restrict__ nw,
-                                                          const T* __restrict__ nb, float alpha, int chunks, SlotRows slots) {
+                                                          const T* __restrict__ nb, float alpha, int chunks, SlotRows slots, ShiftedRead<T> next) {
     const size_t t = token_of(blockIdx.x, chunks);
-    const float* w_in = h_next ? w_in_next : w_out;
+    const int rd = STEP ? next.rd[t] : -1, wr = STEP ? next.wr[t] : -1;
+    const float* w_in = STEP ? next.w_in : h_next ? w_in_next : w_out;
     const T *pw = h_next ? nw : y, *pb = h_next ? nb : y;              // (no next input: nothing of these is used)
     float m[MS <= 4 ? MS : 1][MS <= 4 ? MS : 1], wo[MS <= 4 ? MS : 1], wi[MS <= 4 ? MS : 1];
     if constexpr (MS <= 4) {
@@ -197,8 +210,8 @@ __global__ __launch_bounds__(NT) void hc_write_vec_kernel(float* __restrict__ x,
         }
     }
     for (int i = ((blockIdx.x - (unsigned)t * chunks) * NT + threadIdx.x) * 4; i < D; i += chunks * NT * 4) {
-        raw4f rx[MS];
-        typename Raw4<T>::type ry, rw, rb;
+        raw4f rx[MS], rp;
+        typename Raw4<T>::type ry, rw, rb, rm;
         float old[MS][4], yv[1][4], u[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int q = 0; q < MS; ++q)
@@ -208,6 +221,12 @@ __global__ __launch_bounds__(NT) void hc_write_vec_kernel(float* __restrict__ x,
             rw = raw4(pw, i);
             rb = raw4(pb, i);
         } else {
+            if constexpr (STEP) {
+                rw = raw4(next.nw, i);
+                rb = raw4(next.nb, i);
+                rm = raw4(next.shift, i);
+                rp = raw4(next.prev, (size_t)max(rd, 0) * D + i);
+            }
             slot_sum4<Y>(slots, t, D, i, 0, yv);
             round_stored<T>(yv);
         }
@@ -227,7 +246,7 @@ __global__ __launch_bounds__(NT) void hc_write_vec_kernel(float* __restrict__ x,
                     for (int j = 0; j < 4; ++j) a[j] += mq * old[q][j];
                 }
             st4t(x, (t * S + r) * D + i, a);
-            if (h_next) {
+            if (STEP || h_next) {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) u[j] += wir * a[j];
             }
@@ -248,25 +267,52 @@ __global__ __launch_bounds__(NT) void hc_write_vec_kernel(float* __restrict__ x,
                 for (int j = 0; j < 4; ++j) n[j] = tanhf(alpha * u[j]) * w[j] + b[j];
                 st4t(h_next, t * D + i, n);
             }
+        if constexpr (STEP) {
+            float w[4], b[4], n[4], mu[4], before[4];
+            widen4(rw, w);
+            widen4(rb, b);
+            widen4(rm, mu);
+            widen4(rp, before);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                n[j] = tanhf(next.alpha * u[j]) * w[j] + b[j];
+                if (rd < 0) before[j] = 0.f;
+            }
+            if (wr >= 0) st4t(next.prev, (size_t)wr * D + i, n);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) n[j] += (before[j] - n[j]) * mu[j];
+            st4t(next.h, t * D + i, n);
+        }
     }
 }
 
 // The same for a step (bfloat16, up to four streams, a workgroup per token), the next sublayer's input routed on its way out (serve_route.h).  P: groups of four
 // columns a thread holds, all requested before the first is used.
-template <int P, int MS, int EC>
+// PAIR: y is half the sum of two normed rows, made here (rms_pair_mean_kernel's bits, a launch less).
+struct NormedPair {
+    const bf16_t *b, *wa, *wb;
+    float eps;
+};
+template <int P, int MS, int EC, bool PAIR>
 __global__ __launch_bounds__(NT) void hc_write_route_kernel(float* __restrict__ x, const bf16_t* __restrict__ y, const float* __restrict__ mix,
                                                             const float* __restrict__ w_out, int S, int D, bf16_t* __restrict__ h_next,
                                                             const float* __restrict__ w_in_next, const bf16_t* __restrict__ nw,
-                                                            const bf16_t* __restrict__ nb, float alpha, RouteArgs route) {
+                                                            const bf16_t* __restrict__ nb, float alpha, RouteArgs route, NormedPair pair) {
     __shared__ __attribute__((aligned(16))) RouteRoom<bf16_t, P, EC> room;
+    __shared__ float red[NT / 64 + 1];
     RouteHead<bf16_t, EC> head;
     const size_t t = blockIdx.x;
     raw4f rx[P][MS];
-    raw2u ry[P], rw[P], rb[P];
+    raw2u ry[P], rw[P], rb[P], ry2[P], rwa[P], rwb[P];
     float m[MS][MS], wo[MS], wi[MS];
 #pragma unroll
     for (int k = 0; k < P; ++k) {
         const int at = min((k * NT + (int)threadIdx.x) * 4, D - 4);
+        if constexpr (PAIR) {
+            ry2[k] = raw4(pair.b, t * D + at);
+            rwa[k] = raw4(pair.wa, at);
+            rwb[k] = raw4(pair.wb, at);
+        }
 #pragma unroll
         for (int q = 0; q < MS; ++q) rx[k][q] = raw4(x, (t * S + min(q, S - 1)) * D + at);
         ry[k] = raw4(y, t * D + at);
@@ -282,6 +328,24 @@ __global__ __launch_bounds__(NT) void hc_write_route_kernel(float* __restrict__ 
     }
     head.request(route, D);
     requested();
+    float ia = 0.f, ib = 0.f;
+    if constexpr (PAIR) {
+        float sa = 0.f, sb = 0.f;
+#pragma unroll
+        for (int k = 0; k < P; ++k) {
+            float u[4], v[4];
+            widen4(ry[k], u);
+            widen4(ry2[k], v);
+            if ((k * NT + (int)threadIdx.x) * 4 >= D) continue;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                sa += u[j] * u[j];
+                sb += v[j] * v[j];
+            }
+        }
+        ia = 1.0f / sqrtf(block_sum<NT>(sa, red) / (float)D + pair.eps);
+        ib = 1.0f / sqrtf(block_sum<NT>(sb, red) / (float)D + pair.eps);
+    }
 #pragma unroll
     for (int k = 0; k < P; ++k) {
         const int i = (k * NT + threadIdx.x) * 4;
@@ -290,6 +354,14 @@ __global__ __launch_bounds__(NT) void hc_write_route_kernel(float* __restrict__ 
 #pragma unroll
         for (int q = 0; q < MS; ++q) widen4(rx[k][q], old[q]);
         widen4(ry[k], yv);
+        if constexpr (PAIR) {
+            float v[4], wu[4], wv[4];
+            widen4(ry2[k], v);
+            widen4(rwa[k], wu);
+            widen4(rwb[k], wv);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) yv[j] = bf2f(f2bf(0.5f * (yv[j] * ia * wu[j] + v[j] * ib * wv[j])));
+        }
         widen4(rw[k], w);
         widen4(rb[k], b);
 #pragma unroll
@@ -524,7 +596,7 @@ extern "C" int qsv_hc_write(float* x, const void* y, const float* mix, const flo
 #define QSV_HCV(MS)                                                                                                                            \
     QSV_DISPATCH(dtype, "qsv_hc_write",                                                                                                       \
                  hipLaunchKernelGGL((hc_write_vec_kernel<T, void, MS>), dim3((unsigned)(chunks * n)), dim3(NT), 0, (hipStream_t)stream, x, (const T*)y, mix, w_out, \
-                                    streams, D, (T*)h_next, w_in_next, (const T*)norm_w, (const T*)norm_b, alpha, chunks, SlotRows{}))
+                                    streams, D, (T*)h_next, w_in_next, (const T*)norm_w, (const T*)norm_b, alpha, chunks, SlotRows{}, ShiftedRead<T>{}))
         if (streams <= 2) QSV_HCV(2);
         else if (streams <= 4) QSV_HCV(4);
         else QSV_HCV(MAX_STREAMS);
@@ -538,18 +610,18 @@ extern "C" int qsv_hc_write(float* x, const void* y, const float* mix, const flo
 }
 
 // the same for a step, h_next's rows routed in the same launch (bfloat16, up to four streams)
-extern "C" int qsv_hc_write_route(float* x, const void* y, const float* mix, const float* w_out, int n, int streams, int D, void* h_next, const float* w_in_next,
+static int hc_write_route(const char* what, float* x, const void* y, const float* mix, const float* w_out, int n, int streams, int D, void* h_next, const float* w_in_next,
                                   const void* norm_w, const void* norm_b, float alpha, int32_t* idx, float* weight, const void* router, const void* bias, int renorm, int E,
-                                  int top_k, int G, int keep, int score_fn, const float* correction, int group_top, float scale, void* stream) {
+                                  int top_k, int G, int keep, int score_fn, const float* correction, int group_top, float scale, void* stream, const NormedPair* pair) {
     QSV_REQUIRE(x && y && mix && w_out && h_next && w_in_next && norm_w && norm_b && n >= 0 && D > 0 && D % 8 == 0 && D <= NT * 16 && streams > 0 && streams <= 4,
-                "qsv_hc_write_route: bad arguments");
-    QSV_REQUIRE(fits4(x, QSV_F32) && fits4(y, QSV_BF16) && fits4(h_next, QSV_BF16) && fits4(norm_w, QSV_BF16) && fits4(norm_b, QSV_BF16), "qsv_hc_write_route: rows on four elements");
+                "%s: bad arguments", what);
+    QSV_REQUIRE(fits4(x, QSV_F32) && fits4(y, QSV_BF16) && fits4(h_next, QSV_BF16) && fits4(norm_w, QSV_BF16) && fits4(norm_b, QSV_BF16), "%s: rows on four elements", what);
     const RouteArgs r = {idx, weight, router, bias, correction, renorm, E, top_k, G, keep, score_fn, group_top, scale};
-    QSV_REQUIRE(route_ok(r), "qsv_hc_write_route: %d experts in %d groups, %d groups kept, top %d", E, G, keep, top_k);
+    QSV_REQUIRE(route_ok(r), "%s: %d experts in %d groups, %d groups kept, top %d", what, E, G, keep, top_k);
     if (n == 0) return QSV_OK;
 #define QSV_HCR(P, MS, EC)                                                                                                                     \
-    hipLaunchKernelGGL((hc_write_route_kernel<P, MS, EC>), dim3(n), dim3(NT), 0, (hipStream_t)stream, x, (const bf16_t*)y, mix, w_out, streams, D, (bf16_t*)h_next, \
-                       w_in_next, (const bf16_t*)norm_w, (const bf16_t*)norm_b, alpha, r)
+    hipLaunchKernelGGL((pair ? hc_write_route_kernel<P, MS, EC, true> : hc_write_route_kernel<P, MS, EC, false>), dim3(n), dim3(NT), 0, (hipStream_t)stream, x, (const bf16_t*)y, mix, w_out, streams, D, (bf16_t*)h_next, \
+                       w_in_next, (const bf16_t*)norm_w, (const bf16_t*)norm_b, alpha, r, pair ? *pair : NormedPair{})
 #define QSV_HCR_P(MS, EC)                         \
     do {                                          \
         if (D <= NT * 4) QSV_HCR(1, MS, EC);      \
@@ -562,7 +634,24 @@ extern "C" int qsv_hc_write_route(float* x, const void* y, const float* mix, con
     else QSV_HCR_P(4, 16);
 #undef QSV_HCR
 #undef QSV_HCR_P
-    return qsv_launch_status("qsv_hc_write_route");
+    return qsv_launch_status(what);
+}
+
+extern "C" int qsv_hc_write_route(float* x, const void* y, const float* mix, const float* w_out, int n, int streams, int D, void* h_next, const float* w_in_next,
+                                  const void* norm_w, const void* norm_b, float alpha, int32_t* idx, float* weight, const void* router, const void* bias, int renorm, int E,
+                                  int top_k, int G, int keep, int score_fn, const float* correction, int group_top, float scale, void* stream) {
+    return hc_write_route("qsv_hc_write_route", x, y, mix, w_out, n, streams, D, h_next, w_in_next, norm_w, norm_b, alpha, idx, weight, router, bias, renorm, E, top_k, G,
+                          keep, score_fn, correction, group_top, scale, stream, nullptr);
+}
+// ... with y the mean of two normed rows (qsv_rms_pair_mean's)
+extern "C" int qsv_hc_write_pair_route(float* x, const void* a, const void* wa, const void* b, const void* wb, float eps, const float* mix, const float* w_out, int n,
+                                       int streams, int D, void* h_next, const float* w_in_next, const void* norm_w, const void* norm_b, float alpha, int32_t* idx,
+                                       float* weight, const void* router, const void* bias, int renorm, int E, int top_k, int G, int keep, int score_fn,
+                                       const float* correction, int group_top, float scale, void* stream) {
+    QSV_REQUIRE(b && wa && wb && fits4(b, QSV_BF16) && fits4(wa, QSV_BF16) && fits4(wb, QSV_BF16), "qsv_hc_write_pair_route: bad arguments");
+    const NormedPair pair = {(const bf16_t*)b, (const bf16_t*)wa, (const bf16_t*)wb, eps};
+    return hc_write_route("qsv_hc_write_pair_route", x, a, mix, w_out, n, streams, D, h_next, w_in_next, norm_w, norm_b, alpha, idx, weight, router, bias, renorm, E, top_k,
+                          G, keep, score_fn, correction, group_top, scale, stream, &pair);
 }
 
 extern "C" int qsv_hc_write_slots(float* x, const void* ys, int float_rows, const int32_t* place, const float* weight, const int32_t* idx, int top_k, int n_experts,
@@ -576,7 +665,7 @@ extern "C" int qsv_hc_write_slots(float* x, const void* ys, int float_rows, cons
 #define QSV_HCW(Y, MS)                                                                                                                          \
     QSV_DISPATCH(dtype, "qsv_hc_write_slots",                                                                                                   \
                  hipLaunchKernelGGL((hc_write_vec_kernel<T, Y, MS>), dim3((unsigned)(chunks * n)), dim3(NT), 0, (hipStream_t)stream, x, (const T*)nullptr, mix, w_out, \
-                                    streams, D, (T*)nullptr, (const float*)nullptr, (const T*)nullptr, (const T*)nullptr, 0.f, chunks, slots))
+                                    streams, D, (T*)nullptr, (const float*)nullptr, (const T*)nullptr, (const T*)nullptr, 0.f, chunks, slots, ShiftedRead<T>{}))
 #define QSV_HCW_S(Y)                          \
     do {                                      \
         if (streams <= 2) QSV_HCW(Y, 2);      \
@@ -588,6 +677,28 @@ extern "C" int qsv_hc_write_slots(float* x, const void* ys, int float_rows, cons
 #undef QSV_HCW
 #undef QSV_HCW_S
     return qsv_launch_status("qsv_hc_write_slots");
+}
+
+// ... of a step, with the next sublayer's shifted input (one token a run, up to four streams)
+extern "C" int qsv_hc_write_slots_read(float* x, const float* ys, const float* weight, const int32_t* idx, int top_k, int n_experts, const float* mix, const float* w_out,
+                                       int n, int streams, int D, void* h_next, const float* w_in, const void* norm_w, const void* norm_b, float alpha, const void* shift,
+                                       float* prev, const int32_t* state_rd, const int32_t* state_wr, int dtype, void* stream) {
+    QSV_REQUIRE(x && ys && idx && mix && w_out && h_next && w_in && norm_w && norm_b && shift && prev && state_rd && state_wr && n >= 0 && D > 0 && top_k > 0 &&
+                    n_experts > 0 && streams > 0 && streams <= 4, "qsv_hc_write_slots_read: bad arguments");
+    QSV_REQUIRE(D % 4 == 0 && fits4(ys, QSV_F32) && fits4(x, QSV_F32) && fits4(prev, QSV_F32) && fits4(h_next, dtype) && fits4(norm_w, dtype) && fits4(norm_b, dtype) &&
+                    fits4(shift, dtype), "qsv_hc_write_slots_read: width %d (a multiple of 4), rows on four elements", D);
+    if (n == 0) return QSV_OK;
+    const int chunks = stream_chunks(n, 512, D);
+    const SlotRows slots = {ys, nullptr, weight, idx, top_k, n_experts};
+#define QSV_HCWR(MS)                                                                                                                          \
+    QSV_DISPATCH(dtype, "qsv_hc_write_slots_read",                                                                                            \
+                 hipLaunchKernelGGL((hc_write_vec_kernel<T, float, MS, true>), dim3((unsigned)(chunks * n)), dim3(NT), 0, (hipStream_t)stream, x, (const T*)nullptr, \
+                                    mix, w_out, streams, D, (T*)nullptr, (const float*)nullptr, (const T*)nullptr, (const T*)nullptr, 0.f, chunks, slots,            \
+                                    ShiftedRead<T>{(T*)h_next, w_in, (const T*)norm_w, (const T*)norm_b, (const T*)shift, prev, state_rd, state_wr, alpha}))
+    if (streams <= 2) QSV_HCWR(2);
+    else QSV_HCWR(4);
+#undef QSV_HCWR
+    return qsv_launch_status("qsv_hc_write_slots_read");
 }
 
 extern "C" int qsv_dyt_sum_rows(void* out, const float* x, const int32_t* rows, const void* norm_w, const void* norm_b,

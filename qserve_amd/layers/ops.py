@@ -164,6 +164,16 @@ class ExpertRows:
         return y
 
 
+class NormedPair:
+    """rms_pair_mean(a, wa, b, wb, eps) left to its user, who may make it on the way (`hc_write`); `dense()` is the tensor."""
+
+    def __init__(self, ops, a, wa, b, wb, eps):
+        self.ops, self.a, self.wa, self.b, self.wb, self.eps = ops, a, wa, b, wb, eps
+
+    def dense(self):
+        return self.ops.rms_pair_mean(self.a, self.wa, self.b, self.wb, self.eps)
+
+
 class PendingExperts:
     """The two launches of a mixture's experts in a decoding step, not made yet: a kernel that reads nothing of them may take one along (`take`), and `results`
     makes those that nobody took.  The second product reads the first one's results, so taking it makes the first if need be.  Everything happens on the stream
@@ -539,12 +549,19 @@ class HipOps:
         T, S, D = x.shape
         if route is not None:
             w_in, (w, b, alpha) = then_read
-            q = None if isinstance(y, ExpertRows) or S > 4 else self._routing(route, T, D, x, y, w, b)
+            pair = y if isinstance(y, NormedPair) else None
+            rows = (y,) if pair is None else (pair.a, pair.b, pair.wa, pair.wb)
+            q = None if isinstance(y, ExpertRows) or S > 4 else self._routing(route, T, D, x, *rows, w, b)
             if q is None:
-                return self.hc_write(x, y, w_mix, w_out, then_read), None
-            self._need(x, y, w_mix, w_out, w_in, w, b)
-            assert y.shape == (T, D) and y.dtype == self.dtype and w_mix.dtype == torch.float32 and w_mix.shape == (S, S) and w.dtype == b.dtype == self.dtype
+                return self.hc_write(x, y if pair is None else pair.dense(), w_mix, w_out, then_read), None
+            self._need(x, *rows, w_mix, w_out, w_in, w, b)
+            assert all(r.dtype == self.dtype and r.shape == s for r, s in zip(rows, ((T, D), (T, D), (D,), (D,)))) and w_mix.dtype == torch.float32 and w_mix.shape == (S, S) and w.dtype == b.dtype == self.dtype
             h = torch.empty((T, D), dtype=self.dtype, device=x.device)
+            if pair is not None:
+                self.check(self.L.qsv_hc_write_pair_route(x.data_ptr(), pair.a.data_ptr(), pair.wa.data_ptr(), pair.b.data_ptr(), pair.wb.data_ptr(), float(pair.eps),
+                                                          w_mix.data_ptr(), w_out.data_ptr(), T, S, D, h.data_ptr(), w_in.data_ptr(), w.data_ptr(), b.data_ptr(),
+                                                          float(alpha), *q[2]), "hc_write_pair_route")
+                return h, q[:2]
             self.check(self.L.qsv_hc_write_route(x.data_ptr(), y.data_ptr(), w_mix.data_ptr(), w_out.data_ptr(), T, S, D, h.data_ptr(), w_in.data_ptr(), w.data_ptr(),
                                                  b.data_ptr(), float(alpha), *q[2]), "hc_write_route")
             return h, q[:2]
@@ -567,6 +584,24 @@ class HipOps:
         self.check(self.L.qsv_hc_write(x.data_ptr(), y.data_ptr(), w_mix.data_ptr(), w_out.data_ptr(), T, S, D, *nxt, self.code,
                                        self._s()), "hc_write")
         return h
+
+    def hc_write_read(self, x, y, w_mix, w_out, w_in, norm, shift, batch, prev):
+        """hc_write(x, y, w_mix, w_out), then hc_read(x, w_in, norm, shift, batch, prev): a step's experts' rows in one launch."""
+        w, b, alpha = norm
+        T, S, D = x.shape
+        if (isinstance(y, ExpertRows) and y.place is None and y.ys.dtype == torch.float32 and 0 < T == len(batch.items) and S <= 4 and D % 4 == 0
+                and shift is not None and _on_four(x, y.ys, prev, w, b, shift)):
+            h = torch.empty((T, D), dtype=self.dtype, device=x.device)
+            self._need(x, y.ys, y.idx, y.wt, w_mix, w_out, w_in, w, b, shift, prev)
+            assert y.shape == (T, D) and all(v.dtype == torch.float32 for v in (x, prev, w_mix, w_out, w_in)) and w_mix.shape == (S, S) and w_in.numel() == S
+            assert prev.size(-1) == D and shift.dtype == w.dtype == b.dtype == self.dtype
+            self.check(self.L.qsv_hc_write_slots_read(x.data_ptr(), y.ys.data_ptr(), 0 if y.wt is None else y.wt.data_ptr(), y.idx.data_ptr(), y.idx.size(1), y.experts,
+                                                      w_mix.data_ptr(), w_out.data_ptr(), T, S, D, h.data_ptr(), w_in.data_ptr(), w.data_ptr(), b.data_ptr(), float(alpha),
+                                                      shift.data_ptr(), prev.data_ptr(), batch.state_rd.data_ptr(), batch.state_wr.data_ptr(), self.code, self._s()),
+                       "hc_write_slots_read")
+            return h
+        self.hc_write(x, y, w_mix, w_out)
+        return self.hc_read(x, w_in, norm, shift, batch, prev)
 
     def dyt_sum_rows(self, x, rows, norm):
         w, b, alpha = norm
@@ -1087,6 +1122,26 @@ class HipOps:
                                              int(v_cols or 0), self._s()), "recurrent_scan")
         return o
 
+    def recurrent_gated(self, q, k, v, decay, beta, state, batch, heads, qk_heads, dim, vdim, q_scale, w, gate, kind, eps):
+        """head_rms_gate(recurrent_scan(..), w, gate, kind, eps), a step's tokens in one launch."""
+        T, runs = q.size(0), batch.runs()
+        head_decay = 2 if decay.dim() == 1 else int(decay.shape == (T, heads) and dim != 1)
+        if (self.dtype == torch.bfloat16 and T and runs.size(0) == T == len(batch.items) and w.numel() == vdim and w.dtype == gate.dtype == torch.bfloat16 and 4 <= vdim <= 128
+                and vdim & (vdim - 1) == 0 and dim % 8 == 0 and dim <= 256 and q.stride(0) % 4 == 0 and k.stride(0) % 4 == 0 and gate.stride(0) % 4 == 0
+                and _on_four(q, k, decay, state, w, gate)):
+            self._need(decay, state, w)
+            assert q.dtype == k.dtype == v.dtype and q.stride(1) == k.stride(1) == v.stride(1) == gate.stride(1) == 1
+            assert decay.dtype == torch.float32 and (decay.dim() != 1 or decay.numel() == heads) and (head_decay or decay.shape == (T, heads * dim))
+            assert state.shape[1:] == (heads, dim, vdim) and state.dtype == torch.float32 and v.size(1) == heads * vdim == gate.size(1)
+            out = torch.empty((T, heads * vdim), dtype=self.dtype, device=q.device)
+            self.check(self.L.qsv_recurrent_step_gated(out.data_ptr(), q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0), dtype_code(q.dtype),
+                                                       decay.data_ptr(), 0 if beta is None else beta.data_ptr(), 0 if beta is None else beta.stride(0),
+                                                       0 if beta is None else dtype_code(beta.dtype), state.data_ptr(), runs.data_ptr(), T, heads, qk_heads, dim, vdim,
+                                                       float(q_scale), head_decay, w.data_ptr(), gate.data_ptr(), gate.stride(0), {"silu": 0, "sigmoid": 1}[kind],
+                                                       float(eps), self._s()), "recurrent_step_gated")
+            return out
+        return self.head_rms_gate(self.recurrent_scan(q, k, v, decay, beta, state, batch, heads, qk_heads, dim, vdim, q_scale), w, gate, kind, eps)
+
     def head_rms_gate(self, o, w, gate, kind, eps, vdim=None, den_m=None):
         """o float [T, H, n] -> [T, H * vdim] (storage type): per head o[..., :vdim] / its root mean square * w * gate_fn(gate).
         w [vdim] (shared by the heads) or [H * vdim].  den_m float [T, H] (then n > vdim): the read-out is first divided by
@@ -1463,10 +1518,16 @@ class TorchOps:
         return (n + (before - n) * shift.float()).to(self.dtype)
 
     def hc_write(self, x, y, w_mix, w_out, then_read=None, route=None):
+        if isinstance(y, NormedPair):
+            y = y.dense()
         if route is not None:
             return self.hc_write(x, y, w_mix, w_out, then_read), None
         x.copy_(torch.einsum("sr,tsd->trd", w_mix, x) + w_out[None, :, None] * y.float()[:, None, :])
         return None if then_read is None else self.hc_read(x, then_read[0], then_read[1])
+
+    def hc_write_read(self, x, y, w_mix, w_out, w_in, norm, shift, batch, prev):
+        self.hc_write(x, y, w_mix, w_out)
+        return self.hc_read(x, w_in, norm, shift, batch, prev)
 
     def dyt_sum_rows(self, x, rows, norm):
         w, b, alpha = norm
@@ -1664,6 +1725,9 @@ class TorchOps:
                 o[t] = torch.einsum("hdv,hd->hv", S, qf[t])
             state[slot] = S
         return o
+
+    def recurrent_gated(self, q, k, v, decay, beta, state, batch, heads, qk_heads, dim, vdim, q_scale, w, gate, kind, eps):
+        return self.head_rms_gate(self.recurrent_scan(q, k, v, decay, beta, state, batch, heads, qk_heads, dim, vdim, q_scale), w, gate, kind, eps)
 
     def head_rms_gate(self, o, w, gate, kind, eps, vdim=None, den_m=None):
         T, H, n_cols = o.shape

@@ -17,6 +17,7 @@ that own its columns) and, for the convolution, the last taps - 1 inputs (two co
 import torch
 
 from ..serving.cache import StateSpec
+from .ops import NormedPair
 
 
 def pad_rows(w, to=8):
@@ -48,9 +49,9 @@ class GatedLinearAttention:
         proj = self.ops.linear(h, self.w_in)
         o_q, o_k, o_v, o_g, o_a = 0, H * d, 2 * H * d, 2 * H * d + H * dv, 2 * H * d + 2 * H * dv
         a, _ = ops.decay_products(proj[:, o_a:o_a + self.r], self.w_a2, self.b_a2, None, self.tau, H, d)
-        o = ops.recurrent_scan(proj[:, o_q:o_k], proj[:, o_k:o_v], proj[:, o_v:o_g], a, None, states[0], batch, H, H, d, dv,
-                               d ** -0.5)
-        return self.ops.linear(ops.head_rms_gate(o, self.norm, proj[:, o_g:o_a], "silu", self.eps), self.w_o)
+        o = ops.recurrent_gated(proj[:, o_q:o_k], proj[:, o_k:o_v], proj[:, o_v:o_g], a, None, states[0], batch, H, H, d, dv, d ** -0.5, self.norm, proj[:, o_g:o_a],
+                                "silu", self.eps)
+        return self.ops.linear(o, self.w_o)
 
 
 class GatedDeltaRule:
@@ -104,9 +105,9 @@ class GatedDeltaRule:
         else:
             g, low = ops.decay_products(z, self.w_a2, self.dt_bias, self.a_log, 0.0, H, d, *((gate, self.w_g2) if self.low_gate else ()))
             gate = low if self.low_gate else gate
-        o = ops.recurrent_scan(qkv[:, :G * d], qkv[:, G * d:2 * G * d], qkv[:, 2 * G * d:], g, proj[:, o_b:o_a], states[0], batch,
-                               H, G, d, dv, d ** -0.5)
-        return self.ops.linear(ops.head_rms_gate(o, self.norm, gate, self.gate, self.eps), self.w_o)
+        o = ops.recurrent_gated(qkv[:, :G * d], qkv[:, G * d:2 * G * d], qkv[:, 2 * G * d:], g, proj[:, o_b:o_a], states[0], batch, H, G, d, dv, d ** -0.5, self.norm, gate,
+                                self.gate, self.eps)
+        return self.ops.linear(o, self.w_o)
 
 
 class Retention:
@@ -134,8 +135,9 @@ class Retention:
         o_v, o_g = 2 * H * d, 2 * H * d + H * dv
         rope = self.rotary.reserve(batch.max_pos + 1) if self.rotary is not None else None
         qkv = ops.rotate_qk(proj, H, d, dv, rope, self.rotary.dims if rope is not None else 0, batch)          # float [T, q | k | v]
-        o = ops.recurrent_scan(qkv[:, :H * d], qkv[:, H * d:o_v], qkv[:, o_v:], self.decay, None, states[0], batch, H, H, d, dv, d ** -0.5)
-        return self.ops.linear(ops.head_rms_gate(o, self.norm, proj[:, o_g:o_g + H * dv], "silu", self.eps), self.w_o)
+        o = ops.recurrent_gated(qkv[:, :H * d], qkv[:, H * d:o_v], qkv[:, o_v:], self.decay, None, states[0], batch, H, H, d, dv, d ** -0.5, self.norm,
+                                proj[:, o_g:o_g + H * dv], "silu", self.eps)
+        return self.ops.linear(o, self.w_o)
 
 
 class ParallelMixer:
@@ -152,13 +154,16 @@ class ParallelMixer:
             self.w_in, self._cut = torch.cat([left.w_in, right.w_in], dim=0).contiguous(), left.w_in.size(0)
             left.w_in, right.w_in = self.w_in[:self._cut], self.w_in[self._cut:]
 
-    def __call__(self, h, batch, pools, states):
+    def __call__(self, h, batch, pools, states, lazy=False):
+        """lazy: the caller makes the mean of the two outputs itself (qserve_amd.layers.ops.NormedPair)."""
         pl = pr = {}
         if self.w_in is not None:
             proj = self.ops.linear(h, self.w_in)
             pl, pr = {"proj": proj[:, :self._cut]}, {"proj": proj[:, self._cut:]}
         a = self.left(h, batch, pools[:self._np], states[:self._ns], **pl)
         b = self.right(h, batch, pools[self._np:], states[self._ns:], **pr)
+        if lazy:
+            return NormedPair(self.ops, a, self.w_left, b, self.w_right, self.eps)
         return self.ops.rms_pair_mean(a, self.w_left, b, self.w_right, self.eps)
 
 

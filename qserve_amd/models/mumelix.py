@@ -129,22 +129,31 @@ class Mumelix:
         """-> the float residual streams [T, streams, width] after the last layer run; tap(run, sum of streams) after every run."""
         ops = self.ops
         x = ops.embed_streams(batch.tokens, self.embed, self.scale, self.streams)
+
+        def input_of(run):                                      # what a run's first sublayer reads the streams with
+            L = self.layers[self.order[run]]
+            return L["hc1"][0], L["norm1"], L["shift"], batch, states[self.run_slices[run][2]]
+
+        h = ops.hc_read(x, *input_of(0)) if self.order else None
         for run, i in enumerate(self.order):
             L = self.layers[i]
             p0, p1, s0, s1 = self.run_slices[run]
-            w_in, w_mix, w_out = L["hc1"]
-            h = ops.hc_read(x, w_in, L["norm1"], L["shift"], batch, states[s0])
-            y = L["mixer"](h, batch, pools[p0:p1], states[s0 + 1:s1])
-            if L["ff"] is None:
-                ops.hc_write(x, y, w_mix, w_out)
-            else:                                               # the feed-forward's input comes out of the mixer's stream rewrite
+            _, w_mix, w_out = L["hc1"]
+            lazy = {"lazy": True} if type(L["mixer"]) is ParallelMixer and type(L["ff"]) is TopKGatedMoE else {}
+            y = L["mixer"](h, batch, pools[p0:p1], states[s0 + 1:s1], **lazy)
+            if L["ff"] is not None:                             # the feed-forward's input comes out of the mixer's stream rewrite
                 then = (L["hc2"][0], L["norm2"])
                 if type(L["ff"]) is TopKGatedMoE:               # ... and through the router
                     h, routed = ops.hc_write(x, y, w_mix, w_out, then_read=then, route=L["ff"].routing)
                     y = L["ff"](h, rows=True, routed=routed)
                 else:
                     y = L["ff"](ops.hc_write(x, y, w_mix, w_out, then_read=then), rows=True)
-                ops.hc_write(x, y, L["hc2"][1], L["hc2"][2])
+                _, w_mix, w_out = L["hc2"]
+            # the next run's input comes out of the pass that writes this one's output into the streams
+            if run + 1 < len(self.order):
+                h = ops.hc_write_read(x, y, w_mix, w_out, *input_of(run + 1))
+            else:
+                ops.hc_write(x, y, w_mix, w_out)
             if tap is not None:
                 tap(run, x.sum(1))
         return x

@@ -1,0 +1,78 @@
+"""Kernels of a step that make what two launches made: the same bits."""
+import types
+
+import pytest
+import torch
+
+from qserve_amd.layers.ops import ExpertRows, NormedPair, make_ops
+
+pytestmark = pytest.mark.gpu
+DEV, BF = "cuda:0", torch.bfloat16
+
+
+@pytest.fixture
+def ops():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return make_ops("hip", BF, DEV)
+
+
+def _rand(g, *shape, dtype=BF, scale=1.0):
+    return (torch.randn(*shape, generator=g) * scale).to(dtype).to(DEV)
+
+
+def _runs(T, fresh):
+    """T runs of one token on slots in another order; those in `fresh` start their sequence."""
+    rows = [[T - 1 - i, i, 1, 0 if i in fresh else 5 + i] for i in range(T)]
+    return types.SimpleNamespace(items=[(r[0], r[1], 1) for r in rows], runs=lambda r=torch.tensor(rows, dtype=torch.int32, device=DEV): r)
+
+
+# one to four groups of 64 rows, heads that share keys, columns of less than a workgroup, each kind of decay and gate
+@pytest.mark.parametrize("T, H, QH, dim, vdim", [(1, 2, 2, 8, 4), (16, 16, 4, 64, 128), (3, 6, 3, 72, 64), (5, 4, 4, 256, 32), (64, 3, 1, 128, 16)])
+@pytest.mark.parametrize("delta, floats, decays", [(True, True, "channel"), (False, False, "channel"), (True, False, "head"), (False, True, "constant")])
+@pytest.mark.parametrize("kind", ["silu", "sigmoid"])
+def test_recurrence_with_its_norm_and_gate(ops, T, H, QH, dim, vdim, delta, floats, decays, kind):
+    g = torch.Generator().manual_seed(T + dim)
+    q, k = (_rand(g, T, QH * dim + 4, dtype=torch.float32 if floats else BF, scale=dim ** -0.5)[:, 4:] for _ in range(2))
+    v, beta = _rand(g, T, H * vdim, dtype=q.dtype), _rand(g, T, H + 1)[:, 1:] if delta else None
+    decay = torch.rand(*{"channel": (T, H * dim), "head": (T, H), "constant": (H,)}[decays], generator=g).to(DEV)
+    state, w, gate = _rand(g, T, H, dim, vdim, dtype=torch.float32), _rand(g, vdim), _rand(g, T, H * vdim + 4)[:, 4:]
+    batch, other = _runs(T, {0, T - 1}), state.clone()
+    ref = ops.head_rms_gate(ops.recurrent_scan(q, k, v, decay, beta, state, batch, H, QH, dim, vdim, 0.3), w, gate, kind, 1e-5)
+    ops.recurrent_scan = None                                                                    # (one launch, or an error)
+    out = ops.recurrent_gated(q, k, v, decay, beta, other, batch, H, QH, dim, vdim, 0.3, w, gate, kind, 1e-5)
+    assert torch.equal(out, ref) and torch.equal(state, other)
+
+
+# widths of one and several workgroups a token and their remainders, one to four streams, sequences that start, tokens without experts
+@pytest.mark.parametrize("T, S, D", [(1, 1, 4), (5, 2, 2048), (16, 3, 1028), (64, 4, 4096), (600, 2, 1040)])
+@pytest.mark.parametrize("weighted", [True, False])
+def test_streams_written_and_read_shifted(ops, T, S, D, weighted):
+    g = torch.Generator().manual_seed(T + D)
+    f32 = dict(dtype=torch.float32)
+    x, ys, mix = _rand(g, T, S, D, **f32), _rand(g, T * 3, D, **f32), _rand(g, S, S, **f32)
+    idx = torch.randint(-1, 9, (T, 3), generator=g, dtype=torch.int32).to(DEV)
+    y = ExpertRows(ops, ys, None, torch.rand(T, 3, generator=g).to(DEV) if weighted else None, idx, torch.empty(T, D, dtype=BF, device=DEV), 8)
+    w_out, w_in, norm, shift = _rand(g, S, **f32), _rand(g, S, **f32), (_rand(g, D), _rand(g, D), 0.7), _rand(g, D)
+    prev, i32 = _rand(g, 2 * T, D, **f32), lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)             # noqa: E731
+    batch = types.SimpleNamespace(items=[(i, i, 1) for i in range(T)], run_off=i32([0] * T), state_rd=i32([-1 if i % 5 == 0 else 2 * i for i in range(T)]),
+                                  state_wr=i32([2 * i + 1 for i in range(T)]))
+    a, b, pa, pb = x.clone(), x, prev.clone(), prev
+    ops.hc_write(a, y, mix, w_out)
+    ref = ops.hc_read(a, w_in, norm, shift, batch, pa)
+    ops.hc_read = None
+    h = ops.hc_write_read(b, y, mix, w_out, w_in, norm, shift, batch, pb)
+    assert torch.equal(h, ref) and torch.equal(a, b) and torch.equal(pa, pb)
+
+
+@pytest.mark.parametrize("T, S, D", [(1, 2, 8), (16, 2, 2048), (3, 4, 1032), (64, 3, 4096)])
+def test_mean_of_normed_rows_on_the_way_to_the_router(ops, T, S, D):
+    g = torch.Generator().manual_seed(D)
+    x, mix, w_out, w_in = (_rand(g, *s, dtype=torch.float32) for s in ((T, S, D), (S, S), (S,), (S,)))
+    pair = NormedPair(ops, _rand(g, T, D), _rand(g, D), _rand(g, T, D), _rand(g, D), 1e-5)
+    route = dict(router=_rand(g, 16, D, scale=D ** -0.5), top_k=4, groups=1, keep=1, bias=_rand(g, 16), renorm=True)
+    then, other = (w_in, (_rand(g, D), _rand(g, D), 0.7)), x.clone()
+    ref, (idx, wt) = ops.hc_write(x, pair.dense(), mix, w_out, then_read=then, route=route)
+    ops.rms_pair_mean = None
+    h, routed = ops.hc_write(other, pair, mix, w_out, then_read=then, route=route)
+    assert torch.equal(h, ref) and torch.equal(x, other) and torch.equal(routed[0], idx) and torch.equal(routed[1], wt)

@@ -123,6 +123,22 @@ int qs_w4a8_per_chn_gemm_planes(const int8_t* in_feats, const int8_t* kernel, in
 int qs_w4a8_per_group_gemm_planes(const int8_t* in_feats, const int8_t* kernel, const int8_t* zeros, const int8_t* scales_i8,
                                   int32_t* planes, int M, int N, int K, qs_stream_t stream);
 
+/* Products of one to four tokens (a step of few sequences), with the row operation in front of them as their prologue; int32 sums, so the same bits as the
+ * launches they replace.  Per-channel with zeros / scales_i8 (and the sums) NULL, per-group otherwise.
+ *   _ok: 1 if the sizes are taken: M <= 4, N % 64, K % (64 k_slices) (per-group 128), at most 4096 (per-group: 4096) of K per slice.
+ *   qs_w4a8_rows_planes: qs_w4a8_*_gemm_planes in k_slices slices.
+ *   qs_norm_w4a8_rows: qs_add_residual_rms_norm_general_planes (2 or 4 planes, K = 4096) and the product of its rows: out fp16 [M, N], or with silu_mul
+ *     (kernel = gate rows, then up rows) [M, N / 2].  The residual sum goes to hidden_out, another buffer than hidden; the int8 rows, scales and sums stay inside.
+ *   qs_quant_w4a8_rows_planes: qs_invoke_quant (its scale and, per-channel, sum are written) of act fp16 [M, K], 8192 < K <= 16384, and the product's planes. */
+int qs_w4a8_rows_ok(int per_group, int M, int N, int K, int k_slices);
+int qs_w4a8_rows_planes(const int8_t* in_feats, const int8_t* kernel, const int8_t* zeros, const int8_t* scales_i8, int32_t* planes, int M, int N, int K, int k_slices,
+                        qs_stream_t stream);
+int qs_norm_w4a8_rows(void* out, int silu_mul, const void* hidden, void* hidden_out, const int32_t* planes, int plane_slices, int64_t plane_stride,
+                      const void* plane_wscales, const void* plane_wszs, const void* plane_ascales, const void* plane_asums, const void* weight, float epsilon,
+                      const int8_t* kernel, const int8_t* zeros, const int8_t* scales_i8, const void* wscales, const void* wszs, int M, int N, int K, qs_stream_t stream);
+int qs_quant_w4a8_rows_planes(int32_t* planes, const void* act, void* scale, void* input_sum, const int8_t* kernel, const int8_t* zeros, const int8_t* scales_i8, int M,
+                              int N, int K, int k_slices, qs_stream_t stream);
+
 /* W8A8 GEMM (importable-module requirement only).
  * Replaces qserve_backend.qgemm_w8a8.w8a8_gemm_forward_cuda (kernels/csrc/qgemm/w8a8/w8a8_gemm_cuda.h:11).
  *   kernel int8 [N,K] row-major.  out = float(acc) * (wscale[n]*ascale[m]).  N % 16 == 0, K % 64 == 0. */
@@ -350,6 +366,11 @@ int qs_add_residual_rms_norm_general_planes(int8_t* out, void* hidden_io, const 
                                             int64_t plane_stride, const void* wscales, const void* w_szs, const void* ascales,
                                             const void* a_ssums, const void* weight, void* input_sum, void* scaling,
                                             float epsilon, int num_tokens, int hidden, qs_stream_t stream);
+/*   == the same product's delta ; qs_residual_add(hidden_out = hidden + delta) ; qs_rms_norm(out, hidden_out, weight): the norm behind the last layer.  hidden_out may be
+ *   hidden. */
+int qs_add_residual_rms_norm_planes(void* out, const void* hidden, void* hidden_out, const int32_t* planes, int k_slices, int64_t plane_stride, const void* wscales,
+                                    const void* w_szs, const void* ascales, const void* a_ssums, const void* weight, float epsilon, int num_tokens, int hidden_size,
+                                    qs_stream_t stream);
 int qs_silu_and_mul_quant(int8_t* out, const void* input, void* input_sum, void* scale, int num_tokens, int d,
                           qs_stream_t stream);
 

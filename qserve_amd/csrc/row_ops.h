@@ -59,6 +59,9 @@ __device__ __forceinline__ float ln_val(float x, float mean, float rstd, float g
 struct NoHook {
     __device__ __forceinline__ void operator()() const {}
 };
+// Where a row goes if not to its own memory: chunk(i, values, mul, sum) for every chunk of 8 (sum: the residual sum, fp16), row(max, sum) once a thread.
+// want_sum: whether the row sum is asked for.
+struct NoSink {};
 
 // `delta` of norm_quant_row, by where it comes from.  FromRow: an fp16 row in memory (the residual branch's GEMM output).
 // FromPlanes (round 4): the K-slice planes a W4A8 GEMM left instead of its output (qs_w4a8_*_gemm_planes: int32 [KS][M][N]) -
@@ -231,10 +234,10 @@ __device__ __forceinline__ float ref_order_row_sum(const _Float16* hv, int hidde
 // out int8 [hidden], in fp16 [hidden]; sum_out may be null.  sm: (1 + NC) * NVW floats of LDS.  SC: `in` was published by other
 // workgroups of this launch (cache-bypassing loads).  `ready` runs before the first load of `in` (the GEMM tail waits there
 // for the row to be complete).  Every thread of the workgroup must call (barriers); `active` = tid < 64 * PW.
-template <int NC, int NVW, int PW, bool SC, class Hook = NoHook>
+template <int NC, int NVW, int PW, bool SC, class Hook = NoHook, class After = NoHook, class Sink = NoSink>
 __device__ __forceinline__ void quant_row(int8_t* __restrict__ out, const _Float16* __restrict__ in,
                                           __half* __restrict__ sum_out, __half* __restrict__ scale_out, int hidden,
-                                          float* sm, int tid, Hook ready = Hook()) {
+                                          float* sm, int tid, Hook ready = Hook(), After requested = After(), Sink sink = Sink()) {
 #pragma clang fp contract(off)
     constexpr int VPW = NVW / PW, NT = 64 * NVW;
     static_assert(NVW % PW == 0, "virtual waves must split evenly over the physical waves");
@@ -257,6 +260,8 @@ __device__ __forceinline__ void quant_row(int8_t* __restrict__ out, const _Float
                 }
             }
     }
+    requested();
+    if constexpr (!std::is_same<After, NoHook>::value) __builtin_amdgcn_sched_barrier(0);
     float amax[VPW], sum[VPW][NC];
 #pragma unroll
     for (int j = 0; j < VPW; ++j) {
@@ -279,7 +284,7 @@ __device__ __forceinline__ void quant_row(int8_t* __restrict__ out, const _Float
     }
     float mx, s;
     reduce_max_blocksum<NC, NVW, PW>(amax, sum, sm, sm + NVW, sum_out != nullptr, (hidden + 511) / 512, wave, lane, mx, s);
-    if (tid == 0) {
+    if (tid == 0 && scale_out) {
         *scale_out = __float2half_rn(mx / 127.0f);                      // fused_kernels.cu:72
         if (sum_out) *sum_out = __float2half_rn(s);                     // :121
     }
@@ -295,7 +300,8 @@ __device__ __forceinline__ void quant_row(int8_t* __restrict__ out, const _Float
                     float f[8];
 #pragma unroll
                     for (int e = 0; e < 8; ++e) f[e] = (float)v[e];
-                    qs_store_q8(out + i, f, mul);
+                    if constexpr (std::is_same<Sink, NoSink>::value) qs_store_q8(out + i, f, mul);
+                    else sink.chunk(i, f, mul);
                 }
             }
     }
@@ -308,12 +314,12 @@ __device__ __forceinline__ void quant_row(int8_t* __restrict__ out, const _Float
 // REFSUM (round 6): the row sum in the reference's own order (ref_order_row_sum above) instead of this kernel's fp32 chains;
 // `hvbuf` = `hidden` halves of LDS, `sm` then needs 4 * NVW + 32 floats.  Everything else is unchanged, bit for bit.
 template <int NC, int NVW, int PW, bool ADD, bool SC, class Hook = NoHook, class DeltaFn = FromRow, bool FULL = false,
-          bool REFSUM = false>
+          bool REFSUM = false, class After = NoHook, class Sink = NoSink>
 __device__ __forceinline__ void norm_quant_row(int8_t* __restrict__ out, _Float16* __restrict__ hidden_io,
                                                const _Float16* __restrict__ delta, const _Float16* __restrict__ gamma,
                                                __half* __restrict__ sum_out, __half* __restrict__ scale_out, float eps,
                                                int hidden, float* sm, int tid, Hook ready = Hook(), DeltaFn dfn = DeltaFn(),
-                                               _Float16* hvbuf = nullptr) {
+                                               _Float16* hvbuf = nullptr, After requested = After(), Sink sink = Sink()) {
     // FULL: the row is exactly NC * NT * 8 values wide (every chunk of every thread exists): no exec-masked blocks, so the compiler
     // can count the outstanding loads across them and issue the final stores back to back (round 4: with the masks it put a
     // vmcnt(0) - a store acknowledgement - between the two chunks' stores).
@@ -371,6 +377,7 @@ __device__ __forceinline__ void norm_quant_row(int8_t* __restrict__ out, _Float1
                 }
             // (without the exec-masked blocks the scheduler is free to sink a chunk's requests behind the previous chunk's
             //  arithmetic - seen in the ISA: one memory round trip per chunk; nothing may cross this point)
+            requested();
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int j = 0; j < VPW; ++j)
@@ -451,7 +458,10 @@ __device__ __forceinline__ void norm_quant_row(int8_t* __restrict__ out, _Float1
         }
     }
     float mx, sm_row;
-    reduce_max_sum<NVW, PW>(amax, sum, sm + 2 * NVW, sm + 3 * NVW, !REFSUM && sum_out != nullptr, wave, lane, active, mx, sm_row);
+    bool want_sum;
+    if constexpr (std::is_same<Sink, NoSink>::value) want_sum = !REFSUM && sum_out != nullptr;
+    else want_sum = sink.want_sum();
+    reduce_max_sum<NVW, PW>(amax, sum, sm + 2 * NVW, sm + 3 * NVW, want_sum, wave, lane, active, mx, sm_row);
     if (REFSUM) sm_row = ref_order_row_sum(hvbuf, hidden, sm + 4 * NVW, tid);   // (reduce_max_sum's barrier published hvbuf)
     const float mul = 127.f / mx;                                        // :308
     if (active) {
@@ -464,10 +474,18 @@ __device__ __forceinline__ void norm_quant_row(int8_t* __restrict__ out, _Float1
                     float f[8];
 #pragma unroll
                     for (int e = 0; e < 8; ++e) f[e] = ln_val((float)v[j][c][e], mean, rstd_e, (float)g[j][c][e]);   // fp32, :315
-                    qs_store_q8(out + i, f, mul);
-                    if (ADD) *reinterpret_cast<h8*>(hidden_io + i) = v[j][c];
+                    if constexpr (std::is_same<Sink, NoSink>::value) {
+                        qs_store_q8(out + i, f, mul);
+                        if (ADD) *reinterpret_cast<h8*>(hidden_io + i) = v[j][c];
+                    } else {
+                        sink.chunk(i, f, mul, v[j][c]);
+                    }
                 }
             }
+    }
+    if constexpr (!std::is_same<Sink, NoSink>::value) {
+        sink.row(mx, sm_row);
+        return;
     }
     if (tid == 0) {
         *scale_out = __float2half_rn(mx / 127.f);                        // :322

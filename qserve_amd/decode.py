@@ -234,7 +234,8 @@ class DecodeEngine:
         # K-slice planes (qserve_amd.fused.gemm_planes): the row-parallel projections named in `planes` (default: QS_PLANES, else
         # by rows, below) leave int32 partial sums per K slice and the add + norm + quant launch behind them finishes the GEMM - where
         # the pair fusions are on, on one GPU, for shapes the library has such a launch for
-        if planes is None and os.environ.get("QS_PLANES") is not None:
+        chosen = planes is None and os.environ.get("QS_PLANES") is None      # (told which projections leave planes, the engine uses these forms and no others)
+        if planes is None and not chosen:
             planes = tuple(x for x in os.environ["QS_PLANES"].split(",") if x)
         elif planes is None:
             # `o` has few output blocks for the chip (64 of 4096 channels, 256 with four slices), but no seam to save: with few rows the shorter
@@ -253,6 +254,9 @@ class DecodeEngine:
                 ks = {layer[name].planes_slices(B) for layer in self.layers}
                 if len(ks) == 1 and 0 not in ks:
                     self.planes[name] = torch.empty((ks.pop(), B, hid), dtype=torch.int32, device=self.dev)
+        # the norm behind the last layer from down's planes: the product's own epilogue, the add and the norm took three launches
+        self.last_planes = chosen and "down" in self.planes
+        self._choose_rows(chosen)
         self.lengths = torch.full((B,), prompt_len, dtype=torch.int32, device=self.dev)   # context incl. new token
         self.tokens = torch.randint(0, cfg["vocab"], (B,), device=self.dev, generator=gen)
         # Tensor parallel: the (un-quantised) lm_head is cut over the vocabulary - rank r multiplies rows [v0, v0 + V/N)
@@ -272,6 +276,33 @@ class DecodeEngine:
             self.head_cand_res = self.proj_res.view(-1)[:n].view(tp_world, B, 8)  # the sum over the ranks
         self.graph = None
         self.pieces = None
+
+    def _choose_rows(self, chosen):
+        """Which products of a step of few sequences run through the launches that read their weights straight into registers (fused.rows_planes), with the row operation
+        in front of them inside.  Both sides measured for every line, launches replaced / replacing, us (Llama-3-8B's and Llama-2-7B's products, per-channel):
+        * `o` behind the attention, up to 4 rows, two slices: 4.7 / 3.5, 3.7, 4.3, 4.3 (groups of 128: 5.7 / 4.0, 4.4, 5.1, 5.0);
+        * add + norm + quantiser with qkv: 1 row 9.9 / 6.9 (12288 channels 10.9 / 9.8, groups 12.2 / 8.6), 2 rows 10.0 / 9.4 (groups 12.3 / 10.6, but 12288 channels
+          11.1 / 13.9), 3 rows 10.0 / 12.6: every workgroup does every row;
+        * ... with gate_up: 1 row 16.1 / 14.5 (groups 19.6 / 19.2), 2 rows 16.2 / 19.4;
+        * the quantiser with down: 1 row 10.2 / 9.1 (11008 wide 9.6 / 7.9, groups 12.4 / 10.4), 2 rows 10.3 / 12.7."""
+        B, hid, inter = self.B, self.hid, self.inter
+        group = self.group_size != -1
+        self.rows = set()
+        if not (chosen and B <= 4 and hid == 4096 and set(self.planes) == {"o", "down"} and len(self.layers)
+                and fusedmod.rows_ok(B, hid, self.H * 128, 2, group)):
+            return
+        self.rows.add("o")
+        self.rows_planes = {"o": torch.empty((2, B, hid), dtype=torch.int32, device=self.dev)}      # (in their own numbers of slices)
+        plain = all(L[n].bias is None for L in self.layers for n in ("qkv", "gate_up"))
+        if plain and self.planes["down"].size(0) in (2, 4):
+            if (B == 1 or (B == 2 and self.qkv_n <= 8192)) and fusedmod.rows_ok(B, self.qkv_n, hid, 1, group):
+                self.rows.add("qkv")
+            if B == 1 and fusedmod.rows_ok(B, 2 * inter, hid, 1, group):
+                self.rows.add("gate_up")
+        if B == 1 and 8192 < inter <= 16384 and fusedmod.rows_ok(B, hid, inter, 4, group):
+            self.rows.add("down")
+            self.rows_planes["down"] = torch.empty((4, B, hid), dtype=torch.int32, device=self.dev)
+        self.hidden_next = torch.empty_like(self.hidden)      # (a norm inside a product reads one and writes the other)
 
     # ---- fill the cache for positions [0, prompt_len) through the prefill writer (random K/V source) ----------
     def prefill_cache(self, prompt_len, chunk=8):
@@ -416,18 +447,48 @@ class DecodeEngine:
         # kernel that follows sums them and applies the GEMM's epilogue (bit-identical pair fusion; single GPU only - under
         # tensor parallelism the all-reduce sits between the two)
         def proj_add_norm_quant(lin, name, xq, x, w):
-            pl = self.planes.get(name) if fuse and self.tp_world == 1 else None
+            pl = planes_at(name) if fuse and self.tp_world == 1 else None
             if pl is not None:
-                lin.planes(xq, pl)
+                leave_planes(lin, name, xq)
                 lin.add_norm_quant_planes(qa, x, pl, self.q_scale, self.q_sum, w, self.q_scale, cfg["eps"], sums)
                 return True
             return False
 
+        def planes_at(name):
+            return self.rows_planes[name] if name in rows else self.planes.get(name)
+
+        def leave_planes(lin, name, xq):
+            if name == "o" and "o" in rows:
+                fusedmod.rows_planes(xq, lin.qweight, planes_at(name), *level2(lin))
+            elif name != "down" or "down" not in rows:               # (down's are there: made with its quantiser)
+                lin.planes(xq, planes_at(name))
+
+        def level2(lin):
+            return (None, None) if fuse_sum else (lin.s2_zeros, lin.s2_scales)
+
+        def planes_of(lin, name):                                    # the epilogue operands of a product that left planes
+            return dict(planes=planes_at(name), plane_wscales=lin.s1_scales, plane_ascales=self.q_scale, plane_wszs=lin.s1_szeros if fuse_sum else None,
+                        plane_asums=sums)
+
+        def norm_product(lin, out, x, nxt, front, w, silu):          # add + norm + quantiser behind `front`'s planes, and lin's product
+            z, s2 = level2(lin)
+            fusedmod.norm_rows(out, x, nxt, weight=w, epsilon=cfg["eps"], kernel=lin.qweight, wscales=lin.s1_scales, w_szs=lin.s1_szeros if fuse_sum else None, zeros=z,
+                               scales_i8=s2, silu_mul=silu, **front)
+            return nxt, x
+
+        # (the norms inside products add up the row in this library's order)
+        rows = self.rows if fuse and not (self.rows and fuse_sum and _lib.qs_get_row_sum_order()) else set()
+        last_planes = self.last_planes and fuse and self.tp_world == 1
+        nxt, front = getattr(self, "hidden_next", None), None
         nl = len(self.layers)
         for li, L in enumerate(self.layers):
             if li == 0:
                 norm_quant(h, L["ln1"])
-            L["qkv"](qa, self.q_scale, self.q_sum, self.qkv_buf)
+            if front is not None:
+                h, nxt = norm_product(L["qkv"], self.qkv_buf, h, nxt, front, L["ln1"], False)
+                front = None
+            else:
+                L["qkv"](qa, self.q_scale, self.q_sum, self.qkv_buf)
             q, k, v = self.qkv_buf.split([self.H * 128, self.Hkv * 128, self.Hkv * 128], dim=-1)
             if fuse:         # attention + invoke_quant(_fuse_sum) of its output in one call (bit-identical pair fusion)
                 fusedmod.single_query_attention_quant(
@@ -444,7 +505,10 @@ class DecodeEngine:
                     fused_kernels.invoke_quant_fuse_sum(qo, attn, self.q_sum, self.q_scale)
                 else:
                     fused_kernels.invoke_quant(qo, attn, self.q_scale)
-            if not proj_add_norm_quant(L["o"], "o", qo, h, L["ln2"]):
+            if "gate_up" in rows:
+                leave_planes(L["o"], "o", qo)
+                h, nxt = norm_product(L["gate_up"], self.mlp_act, h, nxt, planes_of(L["o"], "o"), L["ln2"], True)
+            elif not proj_add_norm_quant(L["o"], "o", qo, h, L["ln2"]):
                 L["o"](qo, self.q_scale, self.q_sum, self.proj_out)
                 res = self.proj_out
                 if self.tp_world > 1:
@@ -453,11 +517,16 @@ class DecodeEngine:
                     if L["o"].defer_bias and L["o"].bias is not None:
                         res += L["o"].bias                    # once, after the reduce
                 add_norm_quant(h, res, L["ln2"])
-            if fuse and L["gate_up"].bias is None:     # gate_up GEMM with the silu * mul epilogue, then the quantiser
+            if "gate_up" in rows:
+                pass
+            elif fuse and L["gate_up"].bias is None:   # gate_up GEMM with the silu * mul epilogue, then the quantiser
                 L["gate_up"].silu_mul(qa, self.q_scale, self.q_sum, self.mlp_act, self.gate_up_buf)
             else:
                 L["gate_up"](qa, self.q_scale, self.q_sum, self.gate_up_buf)
-            if fuse and L["gate_up"].bias is not None:
+            if "down" in rows:
+                z, s2 = level2(L["down"])
+                fusedmod.quant_rows_planes(planes_at("down"), self.mlp_act, self.q_scale, L["down"].qweight, sums, z, s2)
+            elif fuse and L["gate_up"].bias is not None:
                 fusedmod.silu_and_mul_quant(self.q_mlp, self.gate_up_buf, self.q_scale, sums)
             else:
                 if not fuse:
@@ -466,8 +535,17 @@ class DecodeEngine:
                     fused_kernels.invoke_quant_fuse_sum(self.q_mlp, self.mlp_act, self.q_sum, self.q_scale)
                 else:
                     fused_kernels.invoke_quant(self.q_mlp, self.mlp_act, self.q_scale)
+            if li + 1 < nl and "qkv" in rows:
+                leave_planes(L["down"], "down", self.q_mlp)
+                front = planes_of(L["down"], "down")
+                continue
             if li + 1 < nl and proj_add_norm_quant(L["down"], "down", self.q_mlp, h, self.layers[li + 1]["ln1"]):
                 continue                                             # (next layer's input norm done from the planes)
+            if last_planes:
+                leave_planes(L["down"], "down", self.q_mlp)
+                fusedmod.add_residual_rms_norm_planes(self.final, h, self.hidden, planes_at("down"), L["down"].s1_scales, self.q_scale, self.norm_w, cfg["eps"],
+                                                      L["down"].s1_szeros if fuse_sum else None, sums)
+                break
             L["down"](self.q_mlp, self.q_scale, self.q_sum, self.proj_out)
             res = self.proj_out
             if self.tp_world > 1:
@@ -479,7 +557,8 @@ class DecodeEngine:
                 add_norm_quant(h, res, self.layers[li + 1]["ln1"])   # next layer's input norm
             else:
                 residual_add_(h, res)
-        layernorm_ops.rms_norm(self.final, h, self.norm_w, cfg["eps"])
+        else:
+            layernorm_ops.rms_norm(self.final, h, self.norm_w, cfg["eps"])
         if self.with_lm_head and self.vocab_parallel:
             yield self._head_local()                                 # candidates of the ranks meet in the sum all-reduce
             self._head_finish(self.head_cand_res)

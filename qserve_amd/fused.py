@@ -207,3 +207,86 @@ def add_residual_rms_norm_general_planes(out, hidden, planes, wscales, ascales, 
             ptr(w_szs) if w_szs is not None else 0, ptr(ascales), ptr(a_ssums) if a_ssums is not None else 0, ptr(weight),
             ptr(input_sum) if input_sum is not None else 0, ptr(scaling), float(epsilon), T, hid, stream()),
             "fused.add_residual_rms_norm_general_planes")
+
+
+def add_residual_rms_norm_planes(out, hidden, hidden_out, planes, wscales, ascales, weight, epsilon, w_szs=None, a_ssums=None):
+    """== gemm(..., delta) ; hidden_out = hidden + delta ; rms_norm(out, hidden_out, weight) where the GEMM left planes [k_slices, T, hidden]
+    (k_slices 1, 2 or 4; its epilogue operands as in add_residual_rms_norm_general_planes).  hidden_out may be hidden."""
+    expect(planes, torch.int32, "planes")
+    hid = hidden.size(-1)
+    T = hidden.numel() // hid
+    _whole("add_residual_rms_norm_planes", torch.float16, (out, T * hid), (hidden, T * hid), (hidden_out, T * hid), (wscales, hid), (w_szs, hid), (weight, hid), (ascales, T),
+           (a_ssums, T))
+    if planes.dim() != 3 or planes.size(1) != T or planes.size(2) != hid or not planes.is_contiguous() or (w_szs is None) != (a_ssums is None):
+        raise RuntimeError(f"add_residual_rms_norm_planes: planes {tuple(planes.shape)} vs hidden [{T}, {hid}]")
+    with guard(out):
+        check(lib.qs_add_residual_rms_norm_planes(ptr(out), ptr(hidden), ptr(hidden_out), ptr(planes), planes.size(0), planes.stride(0), ptr(wscales), _or0(w_szs),
+                                                  ptr(ascales), _or0(a_ssums), ptr(weight), float(epsilon), T, hid, stream()), "fused.add_residual_rms_norm_planes")
+
+
+# ---- products of one to four tokens with the row operation in front of them (include/qserve_amd.h, qs_*_w4a8_rows*) ---------------------
+
+def _or0(t):
+    return 0 if t is None else ptr(t)
+
+
+def _whole(what, dtype, *pairs):
+    """Every tensor there is: of this type, contiguous, with at least so many values (the C entries take bare pointers)."""
+    for t, n in pairs:
+        if t is not None:
+            expect(t, dtype, what)
+            if t.numel() < n or not t.is_contiguous():
+                raise RuntimeError(f"{what}: a tensor of {t.numel()} values where {n} contiguous ones are read or written")
+
+
+def _rows_weights(what, kernel, zeros, scales_i8, N, K):
+    _whole(what, torch.int8, (kernel, N * K // 2), (zeros, N * K // 128), (scales_i8, N * K // 128))
+    if (zeros is None) != (scales_i8 is None):
+        raise RuntimeError(f"{what}: zeros and scales_i8 come together or not at all")
+
+
+def rows_ok(M, N, K, k_slices, per_group=False):
+    """Whether the products of few tokens take [M, K] x [N, K] in k_slices slices of K."""
+    return bool(lib.qs_w4a8_rows_ok(int(per_group), int(M), int(N), int(K), int(k_slices)))
+
+
+def rows_planes(in_feats, kernel, planes, zeros=None, scales_i8=None):
+    """planes int32 [k_slices, M, N]: gemm_planes for M <= 4, in as many slices as planes has."""
+    ks, M, N = planes.shape
+    K = in_feats.numel() // M
+    _whole("rows_planes", torch.int8, (in_feats, M * K))
+    _whole("rows_planes", torch.int32, (planes, ks * M * N))
+    _rows_weights("rows_planes", kernel, zeros, scales_i8, N, K)
+    with guard(planes):
+        check(lib.qs_w4a8_rows_planes(ptr(in_feats), ptr(kernel), _or0(zeros), _or0(scales_i8), ptr(planes), M, N, K, ks, stream()), "fused.rows_planes")
+
+
+def norm_rows(out, hidden, hidden_out, planes, plane_wscales, plane_ascales, weight, epsilon, kernel, wscales, plane_wszs=None, plane_asums=None, w_szs=None, zeros=None,
+              scales_i8=None, silu_mul=False):
+    """== add_residual_rms_norm_general_planes (the sum into hidden_out, another tensor than hidden) and the product of its int8 rows with `kernel`: out fp16 [M, N], or
+    with silu_mul silu(gate) * up [M, N / 2] of kernel = [gate rows | up rows]."""
+    M, K = hidden.shape
+    N = kernel.size(0)
+    f16 = torch.float16
+    _whole("norm_rows", f16, (out, M * N // (2 if silu_mul else 1)), (hidden, M * K), (hidden_out, M * K), (plane_wscales, K), (plane_wszs, K), (plane_ascales, M),
+           (plane_asums, M), (weight, K), (wscales, N), (w_szs, N))
+    _whole("norm_rows", torch.int32, (planes, planes.size(0) * M * K))
+    _rows_weights("norm_rows", kernel, zeros, scales_i8, N, K)
+    if planes.dim() != 3 or planes.size(1) != M or planes.size(2) != K:
+        raise RuntimeError(f"norm_rows: planes {tuple(planes.shape)} vs hidden [{M}, {K}]")
+    with guard(out):
+        check(lib.qs_norm_w4a8_rows(ptr(out), int(silu_mul), ptr(hidden), ptr(hidden_out), ptr(planes), planes.size(0), planes.stride(0), ptr(plane_wscales),
+                                    _or0(plane_wszs), ptr(plane_ascales), _or0(plane_asums), ptr(weight), float(epsilon), ptr(kernel), _or0(zeros), _or0(scales_i8),
+                                    ptr(wscales), _or0(w_szs), M, N, K, stream()), "fused.norm_rows")
+
+
+def quant_rows_planes(planes, act, scale, kernel, input_sum=None, zeros=None, scales_i8=None):
+    """== invoke_quant(_fuse_sum) of act [M, K] (scale and, per-channel, input_sum [M] are written) and rows_planes of its int8 rows."""
+    ks, M, N = planes.shape
+    K = act.numel() // M
+    _whole("quant_rows_planes", torch.float16, (act, M * K), (scale, M), (input_sum, M))
+    _whole("quant_rows_planes", torch.int32, (planes, ks * M * N))
+    _rows_weights("quant_rows_planes", kernel, zeros, scales_i8, N, K)
+    with guard(planes):
+        check(lib.qs_quant_w4a8_rows_planes(ptr(planes), ptr(act), ptr(scale), _or0(input_sum), ptr(kernel), _or0(zeros), _or0(scales_i8), M, N, K, ks, stream()),
+              "fused.quant_rows_planes")

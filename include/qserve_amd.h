@@ -129,7 +129,8 @@ int qs_w4a8_per_group_gemm_planes(const int8_t* in_feats, const int8_t* kernel, 
  *   qs_w4a8_rows_planes: qs_w4a8_*_gemm_planes in k_slices slices.
  *   qs_norm_w4a8_rows: qs_add_residual_rms_norm_general_planes (2 or 4 planes, K = 4096) and the product of its rows: out fp16 [M, N], or with silu_mul
  *     (kernel = gate rows, then up rows) [M, N / 2].  The residual sum goes to hidden_out, another buffer than hidden; the int8 rows, scales and sums stay inside.
- *   qs_quant_w4a8_rows_planes: qs_invoke_quant (its scale and, per-channel, sum are written) of act fp16 [M, K], 8192 < K <= 16384, and the product's planes. */
+ *   qs_quant_w4a8_rows_planes: qs_invoke_quant (its scale and, per-channel, sum are written) of act fp16 [M, K], 2048 < K <= 4096 or 8192 < K <= 16384,
+ *     and the product's planes. */
 int qs_w4a8_rows_ok(int per_group, int M, int N, int K, int k_slices);
 int qs_w4a8_rows_planes(const int8_t* in_feats, const int8_t* kernel, const int8_t* zeros, const int8_t* scales_i8, int32_t* planes, int M, int N, int K, int k_slices,
                         qs_stream_t stream);

@@ -21,7 +21,7 @@
 namespace {
 constexpr int TPB = 256, WAVES = TPB / 64;
 constexpr int ROWS_MOST = 4;
-enum { FROM_INT8, FROM_NORM, FROM_ACT };             // what the token rows are made of
+enum { FROM_INT8, FROM_NORM, FROM_ACT, FROM_WIDE_ACT };   // what the token rows are made of (activations of up to 4096 and of 8193 .. 16384 values)
 enum { TO_HALF, TO_SILU, TO_PLANES };
 
 struct RowsArgs {
@@ -40,7 +40,7 @@ struct RowsArgs {
     size_t pstride;
     const __half *psa, *pss;
     float eps;
-    // FROM_ACT
+    // FROM_ACT, FROM_WIDE_ACT
     const _Float16* act;
     __half *scale_out, *sum_out;
 };
@@ -171,7 +171,7 @@ __global__ __launch_bounds__(TPB, 2) void rows_kernel(RowsArgs a) {
             if (m) __syncthreads();                                      // (the statistics' room is free again)
             __half* none = nullptr;
             // (the sum is made by every workgroup: it decides nothing here but the code is one)
-            qs_row::quant_row<2, 16, 4, false>(nullptr, a.act + (size_t)m * a.K, MODE == 0 ? (tell ? a.sum_out + m : reinterpret_cast<__half*>(&s_sum[m])) : none,
+            qs_row::quant_row<2, FROM == FROM_WIDE_ACT ? 16 : 4, 4, false>(nullptr, a.act + (size_t)m * a.K, MODE == 0 ? (tell ? a.sum_out + m : reinterpret_cast<__half*>(&s_sum[m])) : none,
                                                tell ? a.scale_out + m : none, a.K, sm, tid, qs_row::NoHook(), after,
                                                Sink{rows + m * rstride, first * 64, (first + nst) * 64});
         }
@@ -298,7 +298,7 @@ void launch_rows(const RowsArgs& a, hipStream_t stream) {
         else QS_ROWS(S, 4);          \
     } while (0)
     // (the loads of a wave are as many as its template says, those behind its last stage again the last line: the next of four sizes)
-    if constexpr (FROM == FROM_INT8) {
+    if constexpr (FROM == FROM_INT8 || FROM == FROM_ACT) {
         if (per <= 4) {
             QS_ROWS_M(4);
             return;
@@ -372,13 +372,17 @@ extern "C" int qs_quant_w4a8_rows_planes(int32_t* planes, const void* act, void*
                                          int M, int N, int K, int k_slices, qs_stream_t stream) {
     const bool group = zeros != nullptr;
     QS_REQUIRE(planes && act && scale && kernel && group == (scales_i8 != nullptr) && group == (input_sum == nullptr), "quant_w4a8_rows_planes: null pointer");
-    QS_REQUIRE(K > 8192 && K <= 16384 && rows_fit(group, M, N, K, k_slices, false), "quant_w4a8_rows_planes: %d x %d x %d in %d slices", M, N, K, k_slices);
+    const bool wide = K > 8192;                                          // (invoke_quant's two layouts of these widths, row_ops.h)
+    QS_REQUIRE((wide || (K > 2048 && K <= 4096)) && K <= 16384 && rows_fit(group, M, N, K, k_slices, false), "quant_w4a8_rows_planes: %d x %d x %d in %d slices", M, N, K, k_slices);
     QS_REQUIRE(on16(planes) && on16(act) && on16(kernel) && ((uintptr_t)zeros & 3) == 0 && ((uintptr_t)scales_i8 & 3) == 0, "quant_w4a8_rows_planes: unaligned");
     RowsArgs a = {};
     a.W = (const uint8_t*)kernel, a.zeros = zeros, a.scales8 = scales_i8, a.out = planes, a.M = M, a.N = N, a.K = K, a.ks = k_slices;
     a.act = (const _Float16*)act, a.scale_out = (__half*)scale, a.sum_out = (__half*)input_sum;
     a.wscales = a.wszs = (const _Float16*)kernel;                        // (read, not used)
-    if (group) launch_rows<1, FROM_ACT, TO_PLANES, 1>(a, (hipStream_t)stream);
-    else launch_rows<0, FROM_ACT, TO_PLANES, 1>(a, (hipStream_t)stream);
+    const hipStream_t st = (hipStream_t)stream;
+    if (group && wide) launch_rows<1, FROM_WIDE_ACT, TO_PLANES, 1>(a, st);
+    else if (group) launch_rows<1, FROM_ACT, TO_PLANES, 1>(a, st);
+    else if (wide) launch_rows<0, FROM_WIDE_ACT, TO_PLANES, 1>(a, st);
+    else launch_rows<0, FROM_ACT, TO_PLANES, 1>(a, st);
     return qs_launch_status("quant_w4a8_rows_planes");
 }

@@ -16,6 +16,7 @@ served from cache); the KV cache is filled by the prefill writer.  Tensor parall
 H/tp query heads, Hkv/tp KV heads and the matching column / row shards; the partial outputs of o_proj and
 down_proj are summed with one RCCL all-reduce each.
 """
+import ctypes as C
 import os
 
 import torch
@@ -284,6 +285,9 @@ class DecodeEngine:
         * add + norm + quantiser with qkv: 1 row 9.9 / 6.9 (12288 channels 10.9 / 9.8, groups 12.2 / 8.6), 2 rows 10.0 / 9.4 (groups 12.3 / 10.6, but 12288 channels
           11.1 / 13.9), 3 rows 10.0 / 12.6: every workgroup does every row;
         * ... with gate_up: 1 row 16.1 / 14.5 (groups 19.6 / 19.2), 2 rows 16.2 / 19.4;
+        * the quantiser of the attention's rows with o (in place of the attention's own, which its workgroups hand over to each other for), whole steps of four layers where
+          the keys are not cut over workgroups: 1 row 183.1 / 176.9 (Llama-2-7B 185.6 / 178.8, groups 230.6 / 224.0), 2 rows 205.8 / 203.6, 3 rows 208.2 / 210.2; where they
+          are, the merge quantises in its launch: 1 row of 1500 positions 189.7 / 194.4;
         * the quantiser with down: 1 row 10.2 / 9.1 (11008 wide 9.6 / 7.9, groups 12.4 / 10.4), 2 rows 10.3 / 12.7."""
         B, hid, inter = self.B, self.hid, self.inter
         group = self.group_size != -1
@@ -299,10 +303,18 @@ class DecodeEngine:
                 self.rows.add("qkv")
             if B == 1 and fusedmod.rows_ok(B, 2 * inter, hid, 1, group):
                 self.rows.add("gate_up")
+        if B <= 2 and 2048 < self.H * 128 <= 4096 and self._attention_splits() == 1:
+            self.rows.add("attention")
         if B == 1 and 8192 < inter <= 16384 and fusedmod.rows_ok(B, hid, inter, 4, group):
             self.rows.add("down")
             self.rows_planes["down"] = torch.empty((4, B, hid), dtype=torch.int32, device=self.dev)
         self.hidden_next = torch.empty_like(self.hidden)      # (a norm inside a product reads one and writes the other)
+
+    def _attention_splits(self):
+        """Over how many workgroups the decode attention cuts a sequence's keys (0: another kernel than the matrix cores')."""
+        plan = (C.c_int * 3)()
+        _check(_lib.qs_attention_plan(self.B, self.H, self.Hkv, self.tables[0].size(-1), self.max_len, int(self.int4), C.cast(plan, C.c_void_p)), "attention_plan")
+        return plan[1] if plan[0] in (1, 2) else 0
 
     # ---- fill the cache for positions [0, prompt_len) through the prefill writer (random K/V source) ----------
     def prefill_cache(self, prompt_len, chunk=8):
@@ -458,7 +470,10 @@ class DecodeEngine:
             return self.rows_planes[name] if name in rows else self.planes.get(name)
 
         def leave_planes(lin, name, xq):
-            if name == "o" and "o" in rows:
+            if name == "o" and "attention" in rows:
+                z, s2 = level2(lin)
+                fusedmod.quant_rows_planes(planes_at(name), attn.view(B, -1), self.q_scale, lin.qweight, sums, z, s2)
+            elif name == "o" and "o" in rows:
                 fusedmod.rows_planes(xq, lin.qweight, planes_at(name), *level2(lin))
             elif name != "down" or "down" not in rows:               # (down's are there: made with its quantiser)
                 lin.planes(xq, planes_at(name))
@@ -490,7 +505,10 @@ class DecodeEngine:
             else:
                 L["qkv"](qa, self.q_scale, self.q_sum, self.qkv_buf)
             q, k, v = self.qkv_buf.split([self.H * 128, self.Hkv * 128, self.Hkv * 128], dim=-1)
-            if fuse:         # attention + invoke_quant(_fuse_sum) of its output in one call (bit-identical pair fusion)
+            if "attention" in rows:              # (o quantises the attention's rows itself)
+                attn = fused_attention.single_query_attention(q.reshape(B, self.H, 128), k.reshape(B, self.Hkv, 128), v.reshape(B, self.Hkv, 128), self.tables[li], self.lengths, None,
+                                                       8192, 64, self.size_per_token, self.max_len, 128, cfg["rope_theta"], True, self.int4, True)
+            elif fuse:       # attention + invoke_quant(_fuse_sum) of its output in one call (bit-identical pair fusion)
                 fusedmod.single_query_attention_quant(
                     q.reshape(B, self.H, 128), k.reshape(B, self.Hkv, 128), v.reshape(B, self.Hkv, 128), self.tables[li],
                     self.lengths, qo, self.q_scale, 8192, 64, self.size_per_token, self.max_len, 128, cfg["rope_theta"],

@@ -18,6 +18,7 @@ def test_few_sequences(batch, group, inter, heads, kv_heads):
     eng, ref = D.DecodeEngine(cfg, batch, 70, 8, **kw), D.DecodeEngine(cfg, batch, 70, 8, planes=("o", "down"), **kw)
     assert ("o" in eng.rows) and not ref.rows and ("qkv" in eng.rows) == (batch == 1 or (batch == 2 and kv_heads == 8))
     assert ("gate_up" in eng.rows) == (batch == 1) and ("down" in eng.rows) == (batch == 1 and inter > 8192 and (group == -1 or inter % 512 == 0))
+    assert ("attention" in eng.rows) == (batch <= 2)
     for e in (eng, ref):
         e.prefill_cache(70)
         e.tokens.copy_(torch.arange(batch, device="cuda") + 3)

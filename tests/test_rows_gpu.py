@@ -92,7 +92,7 @@ def test_norm_in_front_of_a_product(group, slices, M, N, silu):
 
 @GROUPS
 @pytest.mark.parametrize("M", [1, 2, 3, 4])
-@pytest.mark.parametrize("N, K, ks", [(4096, 14336, 4), (64, 11008, 4), (64, 8704, 4), (64, 16384, 4)])
+@pytest.mark.parametrize("N, K, ks", [(4096, 14336, 4), (64, 11008, 4), (64, 8704, 4), (64, 16384, 4), (4096, 4096, 2), (64, 4096, 4), (64, 2304, 1), (128, 3840, 2)])
 def test_quantiser_in_front_of_planes(group, M, N, K, ks):
     g = _gen(K + M)
     if group != -1 and K % (128 * ks):

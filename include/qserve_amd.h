@@ -372,6 +372,16 @@ int qs_add_residual_rms_norm_general_planes(int8_t* out, void* hidden_io, const 
 int qs_add_residual_rms_norm_planes(void* out, const void* hidden, void* hidden_out, const int32_t* planes, int k_slices, int64_t plane_stride, const void* wscales,
                                     const void* w_szs, const void* ascales, const void* a_ssums, const void* weight, float epsilon, int num_tokens, int hidden_size,
                                     qs_stream_t stream);
+/* The two ends of a prompt phase over `batch` sequences of `tokens` tokens each:
+ *   qs_prompt_layout: seq_lens [batch], cu_seqlens [batch + 1], padding_offsets [batch * tokens] of such sequences (qs_compute_padding_offsets's).
+ *   qs_embed_rms_norm_general: hidden = table[tokens] ; qs_rms_norm_general(out, hidden, ...).  A token outside the table gives NaN.  The row sum has this library's
+ *     order only (qs_set_row_sum_order).
+ *   qs_last_rows_rms_norm: hidden_out[b] = the last row of sequence b of hidden + delta ; qs_rms_norm(out, hidden_out) ; lengths[b] = tokens + 1. */
+int qs_prompt_layout(int32_t* seq_lens, int32_t* cu_seqlens, int32_t* padding_offsets, int batch, int tokens, qs_stream_t stream);
+int qs_embed_rms_norm_general(int8_t* out, void* hidden, const void* table, const int64_t* tokens, int64_t vocab, const void* weight, void* input_sum, void* scaling,
+                              float epsilon, int num_tokens, int hidden_size, qs_stream_t stream);
+int qs_last_rows_rms_norm(void* out, const void* hidden, void* hidden_out, const void* delta, const void* weight, float epsilon, int batch, int tokens, int hidden_size,
+                          int32_t* lengths, qs_stream_t stream);
 int qs_silu_and_mul_quant(int8_t* out, const void* input, void* input_sum, void* scale, int num_tokens, int d,
                           qs_stream_t stream);
 

@@ -41,6 +41,9 @@ SIGNATURES = {
     "qs_norm_w4a8_rows": (_i, [_vp, _i, _vp, _vp, _vp, _i, _i64, _vp, _vp, _vp, _vp, _vp, _f, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp]),
     "qs_quant_w4a8_rows_planes": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp]),
     "qs_add_residual_rms_norm_planes": (_i, [_vp, _vp, _vp, _vp, _i, _i64, _vp, _vp, _vp, _vp, _vp, _f, _i, _i, _vp]),
+    "qs_prompt_layout": (_i, [_vp, _vp, _vp, _i, _i, _vp]),
+    "qs_embed_rms_norm_general": (_i, [_vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _f, _i, _i, _vp]),
+    "qs_last_rows_rms_norm": (_i, [_vp, _vp, _vp, _vp, _vp, _f, _i, _i, _i, _vp, _vp]),
     "qs_set_attention_variant": (None, [_i]),
     "qs_attention_plan": (_i, [_i, _i, _i, _i, _i, _i, _vp]),
     "qs_single_query_attention": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i64, _i64, _i, _i, _i, _i, _i,

@@ -224,6 +224,37 @@ def add_residual_rms_norm_planes(out, hidden, hidden_out, planes, wscales, ascal
                                                   ptr(ascales), _or0(a_ssums), ptr(weight), float(epsilon), T, hid, stream()), "fused.add_residual_rms_norm_planes")
 
 
+# ---- the two ends of a prompt phase over sequences of one length (include/qserve_amd.h) -----------------------------------------------------
+
+def prompt_layout(batch, tokens, device):
+    """-> (lengths int32 [batch], first rows int32 [batch + 1], padding offsets int32 [batch * tokens]) of `batch` sequences of `tokens` tokens."""
+    seq, cu, pad = (torch.empty((n,), dtype=torch.int32, device=device) for n in (batch, batch + 1, batch * tokens))
+    with guard(seq):
+        check(lib.qs_prompt_layout(ptr(seq), ptr(cu), ptr(pad), batch, tokens, stream()), "fused.prompt_layout")
+    return seq, cu, pad
+
+
+def embed_rms_norm_general(out, hidden, table, tokens, weight, scaling, epsilon, input_sum=None):
+    """== hidden = table[tokens] ; rms_norm_general(_fuse_sum)(out, hidden, ...), the row sum in this library's order."""
+    T, hid = hidden.shape
+    _whole("embed_rms_norm_general", torch.int8, (out, T * hid))
+    _whole("embed_rms_norm_general", torch.int64, (tokens, T))
+    _whole("embed_rms_norm_general", torch.float16, (hidden, T * hid), (table, table.size(0) * hid), (weight, hid), (scaling, T), (input_sum, T))
+    with guard(out):
+        check(lib.qs_embed_rms_norm_general(ptr(out), ptr(hidden), ptr(table), ptr(tokens), table.size(0), ptr(weight), _or0(input_sum), ptr(scaling), float(epsilon), T, hid,
+                                            stream()), "fused.embed_rms_norm_general")
+
+
+def last_rows_rms_norm(out, hidden, hidden_out, delta, weight, epsilon, tokens, lengths):
+    """hidden_out [B, hid] = the last of every `tokens` rows of hidden + delta ; rms_norm(out, hidden_out) ; lengths [B] = tokens + 1."""
+    B, hid = hidden_out.shape
+    _whole("last_rows_rms_norm", torch.float16, (out, B * hid), (hidden, B * tokens * hid), (hidden_out, B * hid), (delta, B * tokens * hid), (weight, hid))
+    _whole("last_rows_rms_norm", torch.int32, (lengths, B))
+    with guard(out):
+        check(lib.qs_last_rows_rms_norm(ptr(out), ptr(hidden), ptr(hidden_out), ptr(delta), ptr(weight), float(epsilon), B, tokens, hid, ptr(lengths), stream()),
+              "fused.last_rows_rms_norm")
+
+
 # ---- products of one to four tokens with the row operation in front of them (include/qserve_amd.h, qs_*_w4a8_rows*) ---------------------
 
 def _or0(t):

@@ -156,6 +156,13 @@ int qsv_latent_prep(const void* down, int64_t down_stride, int q_off, int q_rank
                     int kv_off, int kv_rank, const void* kv_w, int rot_dim, int rot_n, const float* rope,
                     void* pool, const int64_t* slot, const int32_t* pos, float eps, int n_tokens, int dtype, void* stream);
 
+/* qsv_latent_prep for up to 16 tokens (bfloat16) with q [n_tokens, N] = cq w_uq^T made in the same launch (w_uq [N, q_rank]); cq itself is not stored.  kept: w_uq is
+ * to stay in the caches.  qsv_latent_up_ok: the sizes it takes (addresses: w_uq on 16 bytes, the others on 8). */
+int qsv_latent_up_ok(int n_tokens, int q_off, int q_rank, int kv_off, int kv_rank, int rot_dim, int64_t down_stride, int N);
+int qsv_latent_up(void* q, const void* w_uq, int N, int kept, const void* down, int64_t down_stride, int q_off, int q_rank, const void* q_w,
+                  int kv_off, int kv_rank, const void* kv_w, int rot_dim, int rot_n, const float* rope,
+                  void* pool, const int64_t* slot, const int32_t* pos, float eps, int n_tokens, void* stream);
+
 /* qf[t, h] = scale * [ q_abs[h, t, 0 : rank] | rot(q[t, h, dim : dim + rot_dim]) ]  (float [T, H, rank + rot_dim]).
  * q: [T, H, dim + rot_dim], q_abs: [H, T, rank] (the query carried into the latent space), both in the storage type. */
 int qsv_latent_query(float* qf, const void* q, const void* q_abs, const float* rope, const int32_t* pos, float scale,

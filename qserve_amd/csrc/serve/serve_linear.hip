@@ -7,6 +7,7 @@
 // (Weights that pass once stream past the caches since: 32000 x 2048 of one or 16 rows 25 - 26 us, 4096 x 4096 8.9 -> 8.5.)
 #include "serve_common.h"
 #include "serve_expert_rows.h"
+#include "serve_latent_prep.h"
 #include "serve_stream.h"
 
 namespace {
@@ -226,6 +227,91 @@ int run_head_product(const HeadProductArgs& a, hipStream_t stream, const char* w
     else launch_head_product<4, QUERY>(a, steps, tail, stream);
     return qsv_launch_status(what);
 }
+// ---- a step's latent queries: out [T, N] = rms_norm(row's query latent) @ w [N, q_rank]^T, the rows' key-value halves beside it ------------
+// Up to 16 tokens.  The norm and the product were two launches, each a trip to memory behind the other.  Here a product's workgroup (16 weight rows) requests its
+// inputs' rows and then all of its weights, norms the rows into LDS while those are on their way (R rows a wave) and multiplies what it has in registers: one
+// trip.  Every workgroup norms every row, which is what bounds it; the first T workgroups write the cache rows.  The sums, roundings and the order of the
+// products are the two kernels': the same bits.
+// Measured, the two launches -> this one, weights from memory, 1 / 8 / 16 tokens, us: 768 to 3072 5.7 -> 3.4, 6.0 -> 3.6, 6.3 -> 4.6, to 2048 5.4 -> 3.3, 5.6 -> 3.6, 6.1 -> 4.4,
+// 512 to 3072 5.4 -> 3.0, 5.6 -> 3.3, 5.9 -> 3.9, 256 to 1536 4.5 -> 2.5, 4.7 -> 2.7, 4.8 -> 3.5.  The rows' norms grow with the tokens: 32 rows a workgroup lost at 48 and 64 tokens
+// (7.5 -> 9.0), and so do large products of more than 8 (1024 to 6144, 16 tokens 7.5 -> 7.5, left in the caches 6.9 -> 7.1; 768 to 6144 7.0 -> 6.4), which is latent_up_sizes' line;
+// beyond the sizes measured the two launches stay.
+template <int R, int S, bool ONCE>
+__device__ __forceinline__ void latent_up_product(const LatentPrep<bf16_t>& a, const bf16_t* W, bf16_t* out, int T, int N, int block, unsigned char* lds) {
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), K = a.q_rank;
+    const int r0 = 16 * block, stages = K / XK;
+    raw2u rx[R][S], rw[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        const int c = min(4 * (64 * s + lane), K - 4);
+        rw[s] = raw4(a.q_w, c);
+#pragma unroll
+        for (int r = 0; r < R; ++r) rx[r][s] = raw4(a.down + (size_t)min(w * R + r, T - 1) * a.down_stride + a.q_off, c);
+    }
+    v4u A[S][2];                                                     // stage w + 4 s: this wave's, as in stream_products
+    const bf16_t* wr = W + (size_t)min(r0 + (lane & 15), N - 1) * K + 8 * (lane >> 4);
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            const v4u* from = (const v4u*)(wr + min(w + STREAM_WAVES * s, stages - 1) * XK + 32 * ks);
+            A[s][ks] = ONCE ? __builtin_nontemporal_load(from) : *from;
+        }
+    requested();
+    float g[S][4];
+#pragma unroll
+    for (int s = 0; s < S; ++s) widen4(rw[s], g[s]);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int row = w * R + r;
+        float v[S][4], sum = 0.f;
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            widen4(rx[r][s], v[s]);
+            float q = 0.f;
+            const float s4 = square_sum4(v[s]);
+            if (4 * (64 * s + lane) < K) q += s4;
+            sum += wave_sum(q);
+        }
+        const float inv = 1.0f / sqrtf(sum / (float)K + a.eps);
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const int c = 4 * (64 * s + lane);
+            if (c >= K) continue;
+            *(uint2*)(lds + row * K * 2 + (c / XK) * 128 + ((((c & 63) >> 3) ^ (row & 7)) << 4) + (c & 4) * 2) =
+                make_uint2(pack_bf2(v[s][0] * inv * g[s][0], v[s][1] * inv * g[s][1]), pack_bf2(v[s][2] * inv * g[s][2], v[s][3] * inv * g[s][3]));
+        }
+    }
+    __syncthreads();
+    v4f acc = {0.f, 0.f, 0.f, 0.f};
+    const int in = min(lane & 15, 4 * R - 1);                        // (columns behind T are not stored)
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        const int stage = w + STREAM_WAVES * s;
+        if (stage >= stages) break;                                  // (wave-uniform)
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            const v4u B = *(const v4u*)(lds + in * K * 2 + stage * 128 + (((4 * ks + (lane >> 4)) ^ (in & 7)) << 4));
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, A[s][ks]), __builtin_bit_cast(bf8, B), acc, 0, 0, 0);
+        }
+    }
+    v4f* red = (v4f*)(lds + 4 * R * S * 512);                        // [wave][lane], behind the rows
+    red[w * 64 + lane] = acc;
+    __syncthreads();
+    const int c = lane & 15, n = r0 + 4 * (lane >> 4);
+    if (w || c >= T) return;
+    v4f v = red[lane];
+#pragma unroll
+    for (int o = 1; o < STREAM_WAVES; ++o) v += red[o * 64 + lane];
+    if (n < N) *(uint2*)(out + (size_t)c * N + n) = make_uint2(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]));   // (N is a multiple of four)
+}
+template <int R, int S, int P, bool ONCE>
+__global__ __launch_bounds__(64 * STREAM_WAVES, 2) void latent_up_kernel(LatentPrep<bf16_t> a, const bf16_t* W, bf16_t* out, int T, int N) {
+    __shared__ __attribute__((aligned(128))) unsigned char lds[4 * R * S * 512 + STREAM_WAVES * 1024];
+    const int b = (int)blockIdx.x - T;
+    if (b < 0) latent_prep_row<bf16_t, P, 64 * STREAM_WAVES, false>(a, blockIdx.x);
+    else latent_up_product<R, S, ONCE>(a, W, out, T, N, b, lds);
+}
 }  // namespace
 
 // out [T, H, N] = x[t, h] @ w[h], x rows x_tok / x_head elements apart, w [H, K, N]
@@ -335,4 +421,52 @@ extern "C" int qsv_decay_products(float* decay, const void* x, int64_t x_stride,
     if (n_rows <= 16) hipLaunchKernelGGL(decay_products_kernel<1>, dim3(blocks + more, 1), dim3(64 * STREAM_WAVES), 0, (hipStream_t)stream, a, g, blocks);
     else hipLaunchKernelGGL(decay_products_kernel<2>, dim3(blocks + more, (n_rows + 31) / 32), dim3(64 * STREAM_WAVES), 0, (hipStream_t)stream, a, g, blocks);
     return qsv_launch_status("qsv_decay_products");
+}
+
+// Whether qsv_latent_up takes a row's parts: the latents in groups of four columns, the query's in stages of the product
+static bool latent_up_sizes(int n, int q_off, int q_rank, int kv_off, int kv_rank, int rot_dim, int64_t down_stride, int N) {
+    return q_rank > 0 && n <= (N <= 4800000 / q_rank ? 16 : 8) && q_rank % XK == 0 && q_rank <= 1024 && kv_rank > 0 && kv_rank % 4 == 0 && rot_dim >= 0 && rot_dim % 4 == 0 && q_off % 4 == 0 && kv_off % 4 == 0 &&
+           down_stride % 4 == 0 && q_rank + kv_rank + rot_dim <= 4096 && N > 0 && N % 4 == 0 && N <= 6144;
+}
+extern "C" int qsv_latent_up_ok(int n, int q_off, int q_rank, int kv_off, int kv_rank, int rot_dim, int64_t down_stride, int N) {
+    return latent_up_sizes(n, q_off, q_rank, kv_off, kv_rank, rot_dim, down_stride, N);
+}
+// qsv_latent_prep of up to 16 tokens (bfloat16) with its query latents multiplied in the same launch: q [n, N] = cq @ w_uq [N, q_rank]^T
+extern "C" int qsv_latent_up(void* q, const void* w_uq, int N, int kept, const void* down, int64_t down_stride, int q_off, int q_rank, const void* q_w, int kv_off, int kv_rank,
+                             const void* kv_w, int rot_dim, int rot_n, const float* rope, void* pool, const int64_t* slot, const int32_t* pos, float eps, int n, void* stream) {
+    QSV_REQUIRE(q && w_uq && down && q_w && kv_w && pool && slot && pos && n >= 0, "qsv_latent_up: bad arguments");
+    QSV_REQUIRE(latent_up_sizes(n, q_off, q_rank, kv_off, kv_rank, rot_dim, down_stride, N) && rot_n >= 0 && rot_n <= rot_dim && rot_n % 2 == 0 && (rot_n == 0 || rope),
+                "qsv_latent_up: sizes it does not take");
+    QSV_REQUIRE(q_off >= 0 && kv_off >= 0 && q_off + q_rank <= down_stride && kv_off + kv_rank + rot_dim <= down_stride,
+                "qsv_latent_up: the slices do not fit a row of %lld elements", (long long)down_stride);
+    QSV_REQUIRE(((uintptr_t)w_uq % 16 | ((uintptr_t)q | (uintptr_t)down | (uintptr_t)q_w | (uintptr_t)kv_w | (uintptr_t)pool) % 8) == 0, "qsv_latent_up: addresses it does not take");
+    if (n == 0) return QSV_OK;
+    const LatentPrep<bf16_t> a = {(const bf16_t*)down, down_stride, q_off, q_rank, (const bf16_t*)q_w, nullptr, kv_off, kv_rank, (const bf16_t*)kv_w, rot_dim, rot_n,
+                                  rot_n ? rope : nullptr, (bf16_t*)pool, slot, pos, eps};
+    const int columns = (N + 15) / 16, width = q_rank + kv_rank + rot_dim;
+    const bool once = !kept && streams_once(w_uq, N, q_rank);
+    const dim3 grid(n + columns), block(64 * STREAM_WAVES);
+#define QSV_UP(R, S, P)                                                                                                                       \
+    do {                                                                                                                                      \
+        auto kernel = once ? latent_up_kernel<R, S, P, true> : latent_up_kernel<R, S, P, false>;                                              \
+        hipLaunchKernelGGL(kernel, grid, block, 0, (hipStream_t)stream, a, (const bf16_t*)w_uq, (bf16_t*)q, n, N);                            \
+    } while (0)
+#define QSV_UP_P(R, S)                                                                                                                        \
+    do {                                                                                                                                      \
+        if (width <= 2048) QSV_UP(R, S, 2);                                                                                                   \
+        else QSV_UP(R, S, 4);                                                                                                                 \
+    } while (0)
+#define QSV_UP_S(R)                                                                                                                           \
+    do {                                                                                                                                      \
+        if (q_rank <= 512) QSV_UP_P(R, 2);                                                                                                    \
+        else if (q_rank <= 768) QSV_UP_P(R, 3);                                                                                               \
+        else QSV_UP_P(R, 4);                                                                                                                  \
+    } while (0)
+    if (n <= 4) QSV_UP_S(1);
+    else if (n <= 8) QSV_UP_S(2);
+    else QSV_UP_S(4);
+#undef QSV_UP_S
+#undef QSV_UP_P
+#undef QSV_UP
+    return qsv_launch_status("qsv_latent_up");
 }

@@ -1,6 +1,7 @@
 // serve_rows.hip -- one-workgroup-per-token kernels of the serving engine: embedding, fused residual + layer norm, the
 // latent projections' norms + rotary + cache write, the latent query, the output gate.  Statistics and angles are float.
 #include "serve_common.h"
+#include "serve_latent_prep.h"
 #include "serve_route.h"
 
 #include <string.h>
@@ -337,83 +338,10 @@ __global__ __launch_bounds__(NT) void latent_prep_kernel(const T* __restrict__ d
         st(dst, kv_rank + i, v);
     }
 }
-// The same for sizes and addresses that are multiples of four: a thread owns groups of four columns of the row [query latent | key-value latent | rotated key],
-// all requested before the first sum; the two sums meet in one exchange.  Bound by the row's latency in a step, by memory in a prompt.
+// The same for sizes and addresses that are multiples of four (serve_latent_prep.h)
 template <typename T, int P>
-__global__ __launch_bounds__(NT) void latent_prep_vec_kernel(const T* __restrict__ down, int64_t down_stride, int q_off, int q_rank, const T* __restrict__ q_w,
-                                                             T* __restrict__ cq, int kv_off, int kv_rank, const T* __restrict__ kv_w, int rot_dim, int rot_n,
-                                                             const float* __restrict__ rope, T* __restrict__ pool, const int64_t* __restrict__ slot,
-                                                             const int32_t* __restrict__ pos, float eps) {
-    __shared__ float red[2][NT / 64];
-    const size_t t = blockIdx.x;
-    const T* row = down + t * down_stride;
-    const int width = q_rank + kv_rank + rot_dim, half = rot_n / 2;
-    typename Raw4<T>::type rx[P], rw[P];
-    float co[P][2], sn[P][2];
-    const float* cs = rope ? rope + (size_t)pos[t] * (size_t)rot_n : nullptr;
-    T* dst = pool + (size_t)slot[t] * (size_t)(kv_rank + rot_dim);
-#pragma unroll
-    for (int k = 0; k < P; ++k) {
-        const int c = min((k * NT + (int)threadIdx.x) * 4, width - 4);
-        rx[k] = raw4(row, c < q_rank ? q_off + c : kv_off + c - q_rank);
-        rw[k] = raw4(c < q_rank ? q_w : kv_w, c < q_rank ? c : min(c - q_rank, kv_rank - 4));     // (no weight on the rotated part)
-    }
-    if (rope) {
-#pragma unroll
-        for (int k = 0; k < P; ++k) {                               // (a group's first pair may be rotated and its second not)
-            const int d = (k * NT + (int)threadIdx.x) * 4 - q_rank - kv_rank, p = max(0, min(d, rot_n - 2)) / 2, q = max(0, min(d + 2, rot_n - 2)) / 2;
-            co[k][0] = cs[p];
-            sn[k][0] = cs[half + p];
-            co[k][1] = cs[q];
-            sn[k][1] = cs[half + q];
-        }
-    }
-    requested();
-    float v[P][4], sq = 0.f, sk = 0.f;
-#pragma unroll
-    for (int k = 0; k < P; ++k) {
-        const int c = (k * NT + (int)threadIdx.x) * 4;
-        widen4(rx[k], v[k]);
-        const float s = v[k][0] * v[k][0] + v[k][1] * v[k][1] + v[k][2] * v[k][2] + v[k][3] * v[k][3];
-        if (c < q_rank) sq += s;
-        else if (c < q_rank + kv_rank) sk += s;
-    }
-    sq = wave_sum(sq);
-    sk = wave_sum(sk);
-    if ((threadIdx.x & 63) == 0) {
-        red[0][threadIdx.x >> 6] = sq;
-        red[1][threadIdx.x >> 6] = sk;
-    }
-    __syncthreads();
-    sq = sk = 0.f;
-#pragma unroll
-    for (int i = 0; i < NT / 64; ++i) {
-        sq += red[0][i];
-        sk += red[1][i];
-    }
-    const float qinv = 1.0f / sqrtf(sq / (float)q_rank + eps), kinv = 1.0f / sqrtf(sk / (float)kv_rank + eps);
-#pragma unroll
-    for (int k = 0; k < P; ++k) {
-        const int c = (k * NT + (int)threadIdx.x) * 4, d = c - q_rank - kv_rank;
-        if (c >= width) continue;
-        float w[4];
-        widen4(rw[k], w);
-        if (d < 0) {
-            const float inv = c < q_rank ? qinv : kinv;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) v[k][j] = v[k][j] * inv * w[j];
-        } else {
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-                if (d + 2 * j < rot_n) {
-                    const float a = v[k][2 * j], b = v[k][2 * j + 1];
-                    v[k][2 * j] = a * co[k][j] - b * sn[k][j];
-                    v[k][2 * j + 1] = b * co[k][j] + a * sn[k][j];
-                }
-        }
-        if (c < q_rank) st4t(cq, t * q_rank + c, v[k]);
-        else st4t(dst, c - q_rank, v[k]);
-    }
+__global__ __launch_bounds__(NT) void latent_prep_vec_kernel(LatentPrep<T> a) {
+    latent_prep_row<T, P, NT, true>(a, blockIdx.x);
 }
 extern "C" int qsv_latent_prep(const void* down, int64_t down_stride, int q_off, int q_rank, const void* q_w, void* cq,
                                int kv_off, int kv_rank, const void* kv_w, int rot_dim, int rot_n, const float* rope,
@@ -430,8 +358,9 @@ extern "C" int qsv_latent_prep(const void* down, int64_t down_stride, int q_off,
         fits4(q_w, dtype) && fits4(cq, dtype) && fits4(kv_w, dtype) && fits4(pool, dtype)) {
 #define QSV_LPV(P)                                                                                                                            \
     QSV_DISPATCH(dtype, "qsv_latent_prep",                                                                                                    \
-                 hipLaunchKernelGGL((latent_prep_vec_kernel<T, P>), dim3(n), dim3(NT), 0, (hipStream_t)stream, (const T*)down, down_stride, q_off, q_rank, \
-                                    (const T*)q_w, (T*)cq, kv_off, kv_rank, (const T*)kv_w, rot_dim, rot_n, rot_n ? rope : nullptr, (T*)pool, slot, pos, eps))
+                 hipLaunchKernelGGL((latent_prep_vec_kernel<T, P>), dim3(n), dim3(NT), 0, (hipStream_t)stream,                                \
+                                    (LatentPrep<T>{(const T*)down, down_stride, q_off, q_rank, (const T*)q_w, (T*)cq, kv_off, kv_rank, (const T*)kv_w, rot_dim, rot_n, \
+                                                   rot_n ? rope : nullptr, (T*)pool, slot, pos, eps})))
         if (width <= NT * 4) QSV_LPV(1);
         else if (width <= NT * 8) QSV_LPV(2);
         else QSV_LPV(4);

@@ -49,9 +49,10 @@ class LatentAttention:
         ops, T, H = self.ops, h.size(0), self.H
         rope = self.rotary.reserve(batch.max_pos + 1) if self.rot_n else None
         down = self.ops.linear(h, self.w_down)
-        cq = ops.latent_prep(down, self.q_off, self.q_rank, self.dq_norm, self.kv_off, self.rank, self.dkv_norm, self.rot_dim,
-                             self.rot_n, rope, pool, batch.slot, batch.pos, self.eps)
-        q = self.ops.linear(cq, self.w_uq)                                                   # [T, H (dim + rot_dim)]
+        prep = (down, self.q_off, self.q_rank, self.dq_norm, self.kv_off, self.rank, self.dkv_norm, self.rot_dim, self.rot_n, rope, pool, batch.slot, batch.pos, self.eps)
+        q = ops.latent_up(*prep, self.w_uq)                                                  # [T, H (dim + rot_dim)]
+        if q is None:
+            q = self.ops.linear(ops.latent_prep(*prep), self.w_uq)
         gate = down[:, self.g_off:self.g_off + H * self.vdim] if self.gated else None
         plan = ops.latent_prompt_plan(batch, self.window, H, self.dim, self.rot_dim, self.vdim, self.rank, self.scale, pool, (self.w_uk, self.w_uv))
         if plan is not None:

@@ -327,6 +327,22 @@ class HipOps:
                    "latent_prep")
         return cq
 
+    def latent_up(self, down, q_off, q_rank, q_w, kv_off, kv_rank, kv_w, rot_dim, rot_n, rope, pool, slot, pos, eps, w_uq):
+        """linear(latent_prep(...), w_uq) [T, N] for a step's few rows in one launch; None where that takes two."""
+        T, N = down.size(0), w_uq.size(0)
+        if not (T > 0 and w_uq.size(1) == q_rank and _streams(down[:, q_off:q_off + q_rank], w_uq) and _called_plainly(q_w, kv_w)
+                and self.L.qsv_latent_up_ok(T, q_off, q_rank, kv_off, kv_rank, rot_dim, down.stride(0), N)
+                and (q_w.data_ptr() | kv_w.data_ptr() | pool.data_ptr()) % 8 == 0):
+            return None
+        self._need(down, q_w, kv_w, rope, pool, slot, pos, w_uq)
+        assert pool.size(-1) == kv_rank + rot_dim and slot.dtype == torch.int64 and pos.dtype == torch.int32
+        assert rope is None or (rope.dtype == torch.float32 and rope.size(-1) * 2 == rot_n)
+        q = torch.empty((T, N), dtype=self.dtype, device=down.device)
+        self.check(self.L.qsv_latent_up(q.data_ptr(), w_uq.data_ptr(), N, int(self._kept(T)), down.data_ptr(), down.stride(0), q_off, q_rank, q_w.data_ptr(), kv_off,
+                                        kv_rank, kv_w.data_ptr(), rot_dim, rot_n, 0 if rope is None else rope.data_ptr(), pool.data_ptr(), slot.data_ptr(), pos.data_ptr(),
+                                        eps, T, self._s()), "latent_up")
+        return q
+
     def latent_query(self, q, q_abs, rope, pos, scale, heads, dim, rot_dim, rot_n, rank):
         T = q.size(0)
         qf = torch.empty((T, heads, rank + rot_dim), dtype=torch.float32, device=q.device)
@@ -1441,6 +1457,9 @@ class TorchOps:
         kr = _rotate(down[:, kv_off + kv_rank:kv_off + kv_rank + rot_dim].float(), rope, pos, rot_n)
         pool[slot] = torch.cat([c, kr], dim=-1).to(self.dtype)
         return cq
+
+    def latent_up(self, *prep):
+        return None
 
     def latent_query(self, q, q_abs, rope, pos, scale, heads, dim, rot_dim, rot_n, rank):
         T = q.size(0)

@@ -77,7 +77,7 @@ def random_weights(cfg, dev, seed=0):
 
 class OpTimer:
     """HIP events around every call of the ops object's methods (one step at a time)."""
-    NAMES = ("embed", "add_layer_norm", "layer_norm_rows", "latent_prep", "latent_queries", "latent_prompt", "head_products", "latent_attention", "sigmoid_gate",
+    NAMES = ("embed", "add_layer_norm", "layer_norm_rows", "latent_prep", "latent_up", "latent_queries", "latent_prompt", "head_products", "latent_attention", "sigmoid_gate",
              "moe_route", "moe_experts", "moe_experts_shared", "embed_streams", "hc_read", "hc_write", "dyt_sum_rows", "rms_pair_mean", "glu",
              "attention_prep", "rotate_heads", "decay", "decay_products", "conv_silu_unit", "recurrent_scan", "head_rms_gate", "embed_sinusoid",
              "add_rms_norm", "rms_norm_rows", "normed_attention_prep", "max_gates", "add_normed_rms_norm", "qk_norm_rope_prep", "pool_blocks",

@@ -76,3 +76,32 @@ def test_mean_of_normed_rows_on_the_way_to_the_router(ops, T, S, D):
     ops.rms_pair_mean = None
     h, routed = ops.hc_write(other, pair, mix, w_out, then_read=then, route=route)
     assert torch.equal(h, ref) and torch.equal(x, other) and torch.equal(routed[0], idx) and torch.equal(routed[1], wt)
+
+
+# the smallest and largest latent, one to four stages a wave and waves without one, one to four rows a wave, part groups of weight rows
+@pytest.mark.parametrize("T", [1, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("q_rank, kv_rank, rot_dim, rot_n, N", [(64, 8, 0, 0, 1024), (768, 512, 64, 64, 3072), (768, 512, 0, 0, 2048), (320, 256, 64, 22, 1532), (1024, 2000, 64, 64, 1028),
+                                                                (512, 512, 64, 32, 3076)])
+def test_latents_normed_by_their_product(ops, T, q_rank, kv_rank, rot_dim, rot_n, N):
+    g = torch.Generator().manual_seed(T + q_rank)
+    R = kv_rank + rot_dim
+    down, qw, kw, w = _rand(g, T, q_rank + R + 16), _rand(g, q_rank), _rand(g, kv_rank), _rand(g, N, q_rank, scale=q_rank ** -0.5)
+    rope = torch.randn(T + 1, 2, rot_n // 2, generator=g).to(DEV) if rot_n else None
+    pos, slot = torch.arange(T, 0, -1, dtype=torch.int32, device=DEV), torch.randperm(2 * T, generator=g)[:T].to(DEV)
+    pools = [torch.zeros(2 * T, R, dtype=BF, device=DEV) for _ in range(2)]
+    args = [(down, 8, q_rank, qw, q_rank + 12, kv_rank, kw, rot_dim, rot_n, rope, p, slot, pos, 1e-5) for p in pools]
+    out = ops.latent_up(*args[0], w)
+    assert out is not None and torch.equal(out, ops.linear(ops.latent_prep(*args[1]), w)) and torch.equal(*pools)
+    kept = make_ops("hip", BF, DEV)
+    kept.kept_above = 0
+    assert torch.equal(out, kept.latent_up(*args[0], w))
+
+
+def test_latents_that_take_two_launches(ops):
+    g = torch.Generator().manual_seed(1)
+    pos, slot = torch.arange(64, dtype=torch.int32, device=DEV), torch.arange(65, device=DEV)
+    for T, q_rank, kv_rank, N, off in ((17, 768, 512, 2048, 0), (9, 1024, 512, 6144, 0), (4, 768, 512, 6160, 0), (4, 1088, 512, 2048, 0), (4, 96, 512, 2048, 0), (4, 768, 510, 2048, 0),
+                                       (4, 768, 512, 2048, 4)):
+        down, pool = _rand(g, T, q_rank + kv_rank + off)[:, off:].contiguous(), torch.zeros(65, kv_rank, dtype=BF, device=DEV)
+        qw = _rand(g, q_rank + 1)[1:] if off else _rand(g, q_rank)
+        assert ops.latent_up(down, 0, q_rank, qw, q_rank, kv_rank, _rand(g, kv_rank), 0, 0, None, pool, slot[:T], pos[:T], 1e-5, _rand(g, N, q_rank)) is None

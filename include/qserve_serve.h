@@ -280,6 +280,13 @@ int qsv_scaled_sum_rms_norms_route(float* x, void* h0, void* h1, const void* a, 
                                    const int32_t* tokens, const void* table, float eps, int n, int D, int32_t* idx, float* weight, const void* router,
                                    const void* bias, int renorm, int E, int top_k, int G, int keep, int score_fn, const float* correction, int group_top, float scale,
                                    void* stream);
+/* ... and out [n, N] = h0 w^T (w [N, D], N a multiple of four, D of 64 up to 2048, one or two rows) in the same launch; the sum goes to x_out, rows of its own.  kept: w is to
+ * stay in the caches. */
+int qsv_sum_norms_product(void* out, const void* w, int N, int kept, float* x_out, const float* x, void* h0, void* h1, const void* a, const void* sa, const float* ys,
+                          const int32_t* slot_idx, const float* slot_weight, int slot_top, int n_experts, const void* slot_scale, const void* c, const void* sc,
+                          const float* g0, const float* g1, const int32_t* tokens, const void* table, float eps, int n, int D, int32_t* idx, float* weight,
+                          const void* router, const void* bias, int renorm, int E, int top_k, int G, int keep, int score_fn, const float* correction, int group_top,
+                          float scale, void* stream);
 int qsv_hc_write_route(float* x, const void* y, const float* mix, const float* w_out, int n, int streams, int D, void* h_next, const float* w_in_next,
                        const void* norm_w, const void* norm_b, float alpha, int32_t* idx, float* weight, const void* router, const void* bias, int renorm, int E,
                        int top_k, int G, int keep, int score_fn, const float* correction, int group_top, float scale, void* stream);

@@ -157,8 +157,9 @@ struct SlotRows {
 };
 // a[p] = four columns of y[t] from c + p * step on, p < P (zeros behind D).  The rows of four slots are requested together, beside their weights and indices
 // where a slot's row is its number (a row without an expert holds anything: it is taken out by value).
-template <typename Y, int P, bool PLACED>
-__device__ __forceinline__ void slot_sum4_as(const SlotRows& s, size_t t, int D, int c, int step, float (&a)[P][4]) {
+// behind(): called once the first four are requested.
+template <typename Y, int P, bool PLACED, class Behind>
+__device__ __forceinline__ void slot_sum4_as(const SlotRows& s, size_t t, int D, int c, int step, float (&a)[P][4], Behind behind) {
     const float* weight = s.weight ? s.weight : (const float*)s.idx;           // (none: something that can be read)
     auto four = [&](int k0) __attribute__((always_inline)) {
         typename Raw4<Y>::type r[4][P];
@@ -173,6 +174,7 @@ __device__ __forceinline__ void slot_sum4_as(const SlotRows& s, size_t t, int D,
 #pragma unroll
             for (int p = 0; p < P; ++p) r[q][p] = raw4((const Y*)s.ys, row * D + min(c + p * step, D - 4));
         }
+        if (k0 == 0) behind();
         requested();
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -193,12 +195,16 @@ __device__ __forceinline__ void slot_sum4_as(const SlotRows& s, size_t t, int D,
     four(0);                                                                   // (outside the loop, whose head waits for what the caller has requested)
     for (int k0 = 4; k0 < s.top; k0 += 4) four(k0);
 }
-template <typename Y, int P>
-__device__ __forceinline__ void slot_sum4(const SlotRows& s, size_t t, int D, int c, int step, float (&a)[P][4]) {
+template <typename Y, int P, class Behind>
+__device__ __forceinline__ void slot_sum4(const SlotRows& s, size_t t, int D, int c, int step, float (&a)[P][4], Behind behind) {
 #pragma unroll
     for (int p = 0; p < P; ++p) a[p][0] = a[p][1] = a[p][2] = a[p][3] = 0.f;
-    if (s.place) slot_sum4_as<Y, P, true>(s, t, D, c, step, a);
-    else slot_sum4_as<Y, P, false>(s, t, D, c, step, a);
+    if (s.place) slot_sum4_as<Y, P, true>(s, t, D, c, step, a, behind);
+    else slot_sum4_as<Y, P, false>(s, t, D, c, step, a, behind);
+}
+template <typename Y, int P>
+__device__ __forceinline__ void slot_sum4(const SlotRows& s, size_t t, int D, int c, int step, float (&a)[P][4]) {
+    slot_sum4<Y>(s, t, D, c, step, a, [] __device__() {});
 }
 
 // A recurrence's decay from its gate z: sigmoid(z)^(1 / tau) = exp(-softplus(-z) / tau), or, with a log rate, exp(-exp(a) softplus(z))

@@ -9,6 +9,7 @@
 #include "serve_expert_rows.h"
 #include "serve_latent_prep.h"
 #include "serve_stream.h"
+#include "serve_sum_norms.h"
 
 namespace {
 // What becomes of a product x [T, K] @ w [N, K]^T: rounded to bfloat16 it is stored, stored as float (a caller that would widen it), or, as a decay's gate, turned
@@ -227,6 +228,49 @@ int run_head_product(const HeadProductArgs& a, hipStream_t stream, const char* w
     else launch_head_product<4, QUERY>(a, steps, tail, stream);
     return qsv_launch_status(what);
 }
+// ---- products of few rows that their workgroups make themselves: 16 weight rows a workgroup, its weights in registers ---------------------
+// The stages of a wave, w + 4 s as in stream_products (stages behind the row's end repeat the last)
+template <int S, bool ONCE>
+__device__ __forceinline__ void request_stages(const bf16_t* W, int N, int K, int block, v4u (&A)[S][2]) {
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), stages = K / XK;
+    const bf16_t* row = W + (size_t)min(16 * block + (lane & 15), N - 1) * K + 8 * (lane >> 4);
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            const v4u* from = (const v4u*)(row + min(w + STREAM_WAVES * s, stages - 1) * XK + 32 * ks);
+            A[s][ks] = ONCE ? __builtin_nontemporal_load(from) : *from;
+        }
+}
+// out [T, N] from them and `held` rows of K elements in LDS (of every 128 bytes piece p at p ^ (row & 7)), T <= held; red: 4 KiB of LDS.  The order of the sums is that
+// of skinny_product.  N a multiple of four.
+template <int S>
+__device__ __forceinline__ void register_product(const v4u (&A)[S][2], const unsigned char* rows, int held, int K, unsigned char* red_, bf16_t* out, int T, int N, int block) {
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), stages = K / XK;
+    __syncthreads();                                                 // the rows are there
+    v4f acc = {0.f, 0.f, 0.f, 0.f};
+    const int in = min(lane & 15, held - 1);                         // (columns behind T are not stored)
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        const int stage = w + STREAM_WAVES * s;
+        if (stage >= stages) break;                                  // (wave-uniform)
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            const v4u B = *(const v4u*)(rows + in * K * 2 + stage * 128 + (((4 * ks + (lane >> 4)) ^ (in & 7)) << 4));
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, A[s][ks]), __builtin_bit_cast(bf8, B), acc, 0, 0, 0);
+        }
+    }
+    v4f* red = (v4f*)red_;                                           // [wave][lane]
+    red[w * 64 + lane] = acc;
+    __syncthreads();
+    const int c = lane & 15, n = 16 * block + 4 * (lane >> 4);
+    if (w || c >= T) return;
+    v4f v = red[lane];
+#pragma unroll
+    for (int o = 1; o < STREAM_WAVES; ++o) v += red[o * 64 + lane];
+    if (n < N) *(uint2*)(out + (size_t)c * N + n) = make_uint2(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]));
+}
+
 // ---- a step's latent queries: out [T, N] = rms_norm(row's query latent) @ w [N, q_rank]^T, the rows' key-value halves beside it ------------
 // Up to 16 tokens.  The norm and the product were two launches, each a trip to memory behind the other.  Here a product's workgroup (16 weight rows) requests its
 // inputs' rows and then all of its weights, norms the rows into LDS while those are on their way (R rows a wave) and multiplies what it has in registers: one
@@ -239,7 +283,6 @@ int run_head_product(const HeadProductArgs& a, hipStream_t stream, const char* w
 template <int R, int S, bool ONCE>
 __device__ __forceinline__ void latent_up_product(const LatentPrep<bf16_t>& a, const bf16_t* W, bf16_t* out, int T, int N, int block, unsigned char* lds) {
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), K = a.q_rank;
-    const int r0 = 16 * block, stages = K / XK;
     raw2u rx[R][S], rw[S];
 #pragma unroll
     for (int s = 0; s < S; ++s) {
@@ -248,15 +291,8 @@ __device__ __forceinline__ void latent_up_product(const LatentPrep<bf16_t>& a, c
 #pragma unroll
         for (int r = 0; r < R; ++r) rx[r][s] = raw4(a.down + (size_t)min(w * R + r, T - 1) * a.down_stride + a.q_off, c);
     }
-    v4u A[S][2];                                                     // stage w + 4 s: this wave's, as in stream_products
-    const bf16_t* wr = W + (size_t)min(r0 + (lane & 15), N - 1) * K + 8 * (lane >> 4);
-#pragma unroll
-    for (int s = 0; s < S; ++s)
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const v4u* from = (const v4u*)(wr + min(w + STREAM_WAVES * s, stages - 1) * XK + 32 * ks);
-            A[s][ks] = ONCE ? __builtin_nontemporal_load(from) : *from;
-        }
+    v4u A[S][2];
+    request_stages<S, ONCE>(W, N, K, block, A);
     requested();
     float g[S][4];
 #pragma unroll
@@ -282,28 +318,7 @@ __device__ __forceinline__ void latent_up_product(const LatentPrep<bf16_t>& a, c
                 make_uint2(pack_bf2(v[s][0] * inv * g[s][0], v[s][1] * inv * g[s][1]), pack_bf2(v[s][2] * inv * g[s][2], v[s][3] * inv * g[s][3]));
         }
     }
-    __syncthreads();
-    v4f acc = {0.f, 0.f, 0.f, 0.f};
-    const int in = min(lane & 15, 4 * R - 1);                        // (columns behind T are not stored)
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-        const int stage = w + STREAM_WAVES * s;
-        if (stage >= stages) break;                                  // (wave-uniform)
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const v4u B = *(const v4u*)(lds + in * K * 2 + stage * 128 + (((4 * ks + (lane >> 4)) ^ (in & 7)) << 4));
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, A[s][ks]), __builtin_bit_cast(bf8, B), acc, 0, 0, 0);
-        }
-    }
-    v4f* red = (v4f*)(lds + 4 * R * S * 512);                        // [wave][lane], behind the rows
-    red[w * 64 + lane] = acc;
-    __syncthreads();
-    const int c = lane & 15, n = r0 + 4 * (lane >> 4);
-    if (w || c >= T) return;
-    v4f v = red[lane];
-#pragma unroll
-    for (int o = 1; o < STREAM_WAVES; ++o) v += red[o * 64 + lane];
-    if (n < N) *(uint2*)(out + (size_t)c * N + n) = make_uint2(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]));   // (N is a multiple of four)
+    register_product<S>(A, lds, 4 * R, K, lds + 4 * R * S * 512, out, T, N, block);
 }
 template <int R, int S, int P, bool ONCE>
 __global__ __launch_bounds__(64 * STREAM_WAVES, 2) void latent_up_kernel(LatentPrep<bf16_t> a, const bf16_t* W, bf16_t* out, int T, int N) {
@@ -311,6 +326,47 @@ __global__ __launch_bounds__(64 * STREAM_WAVES, 2) void latent_up_kernel(LatentP
     const int b = (int)blockIdx.x - T;
     if (b < 0) latent_prep_row<bf16_t, P, 64 * STREAM_WAVES, false>(a, blockIdx.x);
     else latent_up_product<R, S, ONCE>(a, W, out, T, N, b, lds);
+}
+
+// ---- a parallel layer's norms with the mixer's product of the first one: scaled_sum_row and out [T, N] = h0 @ w [N, D]^T --------------------
+// One or two tokens.  The norms' kernel is one workgroup a token, a chain from the parts' rows to the router's choice, and the product waited for it.  Here its
+// workgroups make the first norm's rows themselves, while their weights are on the way; the first T do the norms' kernel's work as before, the router's included, which
+// nothing waits for before the next launch.  x is read by every workgroup, so the sum goes to rows of its own (x_out).  The same bits.
+// Measured, the two launches -> this one, weights from memory, 4 of 16 experts' rows and a shared one's, rows of 2048, one / two tokens, us: to 2560 10.0 -> 6.5, 10.3 -> 8.2, 4096
+// 11.0 -> 8.6, 10.9 -> 9.9, 5120 12.0 -> 10.7, 11.8 -> 12.8, 8192 14.0 -> 14.0, 13.9 -> 15.4; of 1024 to 2560 8.4 -> 5.2, 8.6 -> 5.5, 512 to 1536 6.6 -> 4.1, 6.7 -> 5.1; 64 experts,
+// 4096 18.3 -> 16.3, 18.5 -> 16.3.  A workgroup reads as many bytes of parts as of weights, so wide products lose: the line is at 6144 for one token, 4096 for two.
+struct SumProduct {
+    float* x_out;
+    const float* x;
+    bf16_t *h0, *h1;
+    ScaledParts parts;
+    const float *g0, *g1;
+    const int32_t* tokens;
+    const bf16_t* table;
+    float eps;
+    int D;
+    SlotRows slots;
+    RouteArgs route;
+    bf16_t* out;
+    const bf16_t* W;
+    int T, N;
+};
+template <int VPT, int NP, typename Y, int EC, bool ONCE>
+__global__ __launch_bounds__(256, 2) void sum_norms_product_kernel(SumProduct a) {
+    __shared__ __attribute__((aligned(128))) unsigned char lds[2 * VPT * 2048 + STREAM_WAVES * 1024];
+    const int block = (int)blockIdx.x - a.T;
+    if (block < 0) {
+        scaled_sum_row<bf16_t, VPT, NP, Y, EC, 256, false>(blockIdx.x, a.x_out, a.x, a.h0, a.h1, a.parts, a.g0, a.g1, a.tokens, a.table, a.eps, a.D, a.slots, a.route, nullptr,
+                                                          NothingMore());
+        return;
+    }
+    constexpr int S = 4 * VPT;
+    v4u A[S][2];
+    scaled_sum_row<bf16_t, VPT, NP, Y, 0, 256, true>(0, nullptr, a.x, nullptr, nullptr, a.parts, a.g0, a.g1, a.tokens, a.table, a.eps, a.D, a.slots, a.route, lds,
+                                                     [&]() __attribute__((always_inline)) { request_stages<S, ONCE>(a.W, a.N, a.D, block, A); });
+    if (a.T > 1)
+        scaled_sum_row<bf16_t, VPT, NP, Y, 0, 256, true>(1, nullptr, a.x, nullptr, nullptr, a.parts, a.g0, a.g1, a.tokens, a.table, a.eps, a.D, a.slots, a.route, lds, NothingMore());
+    register_product<S>(A, lds, a.T, a.D, lds + 2 * VPT * 2048, a.out, a.T, a.N, block);
 }
 }  // namespace
 
@@ -469,4 +525,44 @@ extern "C" int qsv_latent_up(void* q, const void* w_uq, int N, int kept, const v
 #undef QSV_UP_P
 #undef QSV_UP
     return qsv_launch_status("qsv_latent_up");
+}
+
+extern "C" int qsv_sum_norms_product(void* out, const void* w, int N, int kept, float* x_out, const float* x, void* h0, void* h1, const void* a, const void* sa, const float* ys,
+                                     const int32_t* slot_idx, const float* slot_weight, int slot_top, int n_experts, const void* slot_scale, const void* c, const void* sc,
+                                     const float* g0, const float* g1, const int32_t* tokens, const void* table, float eps, int n, int D, int32_t* idx, float* weight,
+                                     const void* router, const void* bias, int renorm, int E, int top_k, int G, int keep, int score_fn, const float* correction, int group_top,
+                                     float scale, void* stream) {
+    QSV_REQUIRE(out && w && x_out && h0 && h1 && g0 && g1 && n >= 0 && n <= 2 && D > 0 && D % XK == 0 && D <= 2048 && N > 0 && N % 4 == 0 && N <= 1 << 24 &&
+                    (tokens ? table && !a && !ys && !c : x && x != x_out && a && ys && slot_idx && slot_top > 0 && n_experts > 0), "qsv_sum_norms_product: bad arguments");
+    const RouteArgs r = {idx, weight, router, bias, correction, renorm, E, top_k, G, keep, score_fn, group_top, scale};
+    QSV_REQUIRE(route_ok(r), "qsv_sum_norms_product: %d experts in %d groups, %d groups kept, top %d", E, G, keep, top_k);
+    QSV_REQUIRE(((uintptr_t)w % 16 | ((uintptr_t)x | (uintptr_t)x_out | (uintptr_t)ys | (uintptr_t)g0 | (uintptr_t)g1) % 16 |
+                 ((uintptr_t)out | (uintptr_t)h0 | (uintptr_t)h1 | (uintptr_t)a | (uintptr_t)sa | (uintptr_t)slot_scale | (uintptr_t)c | (uintptr_t)sc | (uintptr_t)table) % 8) == 0,
+                "qsv_sum_norms_product: addresses it does not take");
+    if (n == 0) return QSV_OK;
+    const SumProduct p = {x_out, x, (bf16_t*)h0, (bf16_t*)h1, {{a, c, nullptr}, {sa, sc, nullptr}, slot_scale}, g0, g1, tokens, (const bf16_t*)table, eps, D,
+                          {ys, nullptr, slot_weight, slot_idx, slot_top, n_experts}, r, (bf16_t*)out, (const bf16_t*)w, n, N};
+    const bool once = !kept && streams_once(w, N, D);
+#define QSV_SNP(V, NP, Y, EC)                                                                                                                 \
+    do {                                                                                                                                      \
+        auto kernel = once ? sum_norms_product_kernel<V, NP, Y, EC, true> : sum_norms_product_kernel<V, NP, Y, EC, false>;                    \
+        hipLaunchKernelGGL(kernel, dim3(n + (N + 15) / 16), dim3(256), 0, (hipStream_t)stream, p);                                            \
+    } while (0)
+#define QSV_SNP_V(NP, Y, EC)                   \
+    do {                                       \
+        if (D <= 1024) QSV_SNP(1, NP, Y, EC);  \
+        else QSV_SNP(2, NP, Y, EC);            \
+    } while (0)
+#define QSV_SNP_P(EC)                          \
+    do {                                       \
+        if (tokens) QSV_SNP_V(0, void, EC);    \
+        else if (c) QSV_SNP_V(2, float, EC);   \
+        else QSV_SNP_V(1, float, EC);          \
+    } while (0)
+    if (E <= 8) QSV_SNP_P(8);
+    else QSV_SNP_P(16);
+#undef QSV_SNP
+#undef QSV_SNP_V
+#undef QSV_SNP_P
+    return qsv_launch_status("qsv_sum_norms_product");
 }

@@ -3,6 +3,7 @@
 #include "serve_common.h"
 #include "serve_latent_prep.h"
 #include "serve_route.h"
+#include "serve_sum_norms.h"
 
 #include <string.h>
 
@@ -601,138 +602,12 @@ extern "C" int qsv_add_rms_norm(float* x, void* h, const void* a, const void* b,
 // ---- x += s0 a + s1 b + s2 c (element-wise scales); h0 = rms_norm(x) * g0, h1 = rms_norm(x) * g1 -------------------------------------------
 // The parallel layer with a norm of its own for each side: one statistic, two gains (float, one per coordinate).  tokens: x starts as the
 // embedding row.  a, b, c (storage type), their scales and h1 may be NULL; h0 == NULL: the sum only.
-struct ScaledParts {
-    const void *y[3], *s[3];
-    const void* slot_scale;
-};
-// One trip to memory: the NP parts (and, Y other than void, what a mixture of experts left per slot, summed and rounded here as a tensor would hold it,
-// scaled by slot_scale: added behind the first part) are requested before the first is used.  Rows of more than 4096 columns with two parts and more take two trips:
-// in one their registers leave two waves to a SIMD (three parts of 8192, 1024 / 2048 rows 29.1 / 53.6 -> 23.9 / 43.6 us).
-// THREADS: 64 or 128 for rows of up to 256 and 512 columns (idle waves repeat the row's last column: three parts of 256, 8192 rows 13.7 -> 7.4 us); VPT: groups
-// of four columns a thread, the least that holds the row (three parts of 2304, 2048 rows: three groups 15.3 us, four 18.1).
-// EC other than 0: the rows of the second norm go through a router on their way out (serve_route.h).
 template <typename T, int VPT, int NP, typename Y = void, int EC = 0, int THREADS = NT>
 __global__ __launch_bounds__(THREADS) void scaled_sum_rms_norms_vec_kernel(float* __restrict__ x, T* __restrict__ h0, T* __restrict__ h1, ScaledParts p,
                                                                       const float* __restrict__ g0, const float* __restrict__ g1,
                                                                       const int32_t* __restrict__ tokens, const T* __restrict__ table, float eps, int D, SlotRows slots,
                                                                       RouteArgs route) {
-    constexpr bool SLOTS = !std::is_void<Y>::value;
-    constexpr int CH = VPT > 4 && NP >= 2 ? VPT / 2 : VPT, PARTS = NP ? NP : 1;
-    static_assert(VPT % CH == 0 && (CH == VPT || (!SLOTS && EC == 0)) && (EC == 0 || THREADS == NT), "");
-    __shared__ float red[THREADS / 64 + 1];
-    __shared__ __attribute__((aligned(16))) RouteRoom<T, VPT, EC> room;
-    RouteHead<T, EC ? EC : 1> head;
-    const size_t t = blockIdx.x;
-    float v[VPT][4], ysum[CH][4], yf[CH][4];
-    raw4f rg0[VPT], rg1[VPT];
-    const bool norms = h0 != nullptr, two = norms && h1 != nullptr;
-    const T* sf[PARTS];
-#pragma unroll
-    for (int j = 0; j < NP; ++j) sf[j] = p.s[j] ? (const T*)p.s[j] : (const T*)p.y[j];      // (no scale: a row that there is)
-    const T* sy = SLOTS ? (p.slot_scale ? (const T*)p.slot_scale : (const T*)p.y[0]) : nullptr;
-    const float *first = norms ? g0 : x, *second = two ? g1 : first;
-    const size_t row = tokens ? (size_t)tokens[t] * D : 0;
-    float s = 0.f;
-#pragma unroll
-    for (int k0 = 0; k0 < VPT; k0 += CH) {
-        typename Raw4<T>::type rz[CH][PARTS], rf[CH][PARTS], ryf[CH], rt[CH];
-        raw4f rx[CH];
-        float z[CH][PARTS][4], f[CH][PARTS][4];
-        if (tokens) {
-#pragma unroll
-            for (int k = 0; k < CH; ++k) rt[k] = raw4(table, row + min(((int)threadIdx.x + (k0 + k) * THREADS) * 4, D - 4));
-        }
-#pragma unroll
-        for (int k = 0; k < CH; ++k) {
-            const int at = min(((int)threadIdx.x + (k0 + k) * THREADS) * 4, D - 4);
-            if (!tokens) rx[k] = raw4(x, t * D + at);
-#pragma unroll
-            for (int j = 0; j < NP; ++j) {
-                rz[k][j] = raw4((const T*)p.y[j], t * D + at);
-                rf[k][j] = raw4(sf[j], at);
-            }
-            if constexpr (SLOTS) ryf[k] = raw4(sy, at);
-        }
-        if constexpr (EC > 0) head.request(route, D);
-        if constexpr (SLOTS) {
-            slot_sum4<Y>(slots, t, D, threadIdx.x * 4, THREADS * 4, ysum);
-            round_stored<T>(ysum);
-        }
-        if constexpr (VPT <= 2) {                                    // (wider rows would hold too much)
-#pragma unroll
-            for (int k = 0; k < VPT; ++k) {
-                const int at = min(((int)threadIdx.x + k * THREADS) * 4, D - 4);
-                rg0[k] = raw4(first, at);
-                rg1[k] = raw4(second, at);
-            }
-        }
-        requested();
-#pragma unroll
-        for (int k = 0; k < CH; ++k) {
-            if (tokens) widen4(rt[k], v[k0 + k]);
-            else widen4(rx[k], v[k0 + k]);
-#pragma unroll
-            for (int j = 0; j < NP; ++j) {
-                widen4(rz[k][j], z[k][j]);
-                widen4(rf[k][j], f[k][j]);
-                if (!p.s[j]) f[k][j][0] = f[k][j][1] = f[k][j][2] = f[k][j][3] = 1.f;
-            }
-            if constexpr (SLOTS) {
-                widen4(ryf[k], yf[k]);
-                if (!p.slot_scale) yf[k][0] = yf[k][1] = yf[k][2] = yf[k][3] = 1.f;
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < CH; ++k) {
-            const int i = (threadIdx.x + (k0 + k) * THREADS) * 4;
-            if (i >= D) continue;
-            float(&u)[4] = v[k0 + k];
-            float y[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int j = 0; j < NP; ++j) {
-                if (SLOTS && j == 1)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) y[e] += yf[k][e] * ysum[k][e];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) y[e] += f[k][j][e] * z[k][j][e];
-            }
-            if (SLOTS && NP < 2)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) y[e] += yf[k][e] * ysum[k][e];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) u[e] += y[e];
-            st4t(x, t * D + i, u);
-            s += u[0] * u[0] + u[1] * u[1] + u[2] * u[2] + u[3] * u[3];
-        }
-    }
-    if (!h0) return;
-    const float inv = 1.0f / sqrtf(block_sum<THREADS>(s, red) / (float)D + eps);
-#pragma unroll
-    for (int k = 0; k < VPT; ++k) {
-        const int i = (threadIdx.x + k * THREADS) * 4;
-        if (i >= D) continue;
-        float a[4], n[4];
-        if constexpr (VPT <= 2) widen4(rg0[k], a);
-        else ld4t(g0, i, a);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            v[k][e] *= inv;
-            n[e] = v[k][e] * a[e];
-        }
-        st4t(h0, t * D + i, n);
-        if (h1) {
-            if constexpr (VPT <= 2) widen4(rg1[k], a);
-            else ld4t(g1, i, a);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) n[e] = v[k][e] * a[e];
-            st4t(h1, t * D + i, n);
-            if constexpr (EC > 0) st4t(room.row, i, n);
-        }
-    }
-    if constexpr (EC > 0) {
-        __syncthreads();
-        route_row<T, EC>(route, head, t, room.row, D, room.part, room.cs);
-    }
+    scaled_sum_row<T, VPT, NP, Y, EC, THREADS, false>(blockIdx.x, x, x, h0, h1, p, g0, g1, tokens, table, eps, D, slots, route, nullptr, NothingMore());
 }
 template <typename T>
 __global__ __launch_bounds__(NT) void scaled_sum_rms_norms_kernel(float* __restrict__ x, T* __restrict__ h0, T* __restrict__ h1, ScaledParts p,

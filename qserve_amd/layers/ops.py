@@ -85,6 +85,12 @@ def _called_plainly(*ts):
             and not (torch.is_grad_enabled() and any(t.requires_grad for t in ts)))
 
 
+def _weight_streams(w, T):
+    """Whether T rows times w^T go through that kernel by what w is."""
+    return (type(w) in (torch.Tensor, torch.nn.Parameter) and w.is_cuda and w.dim() == 2 and w.dtype == torch.bfloat16 and w.is_contiguous() and w.numel() and
+            w.data_ptr() % 16 == 0 and w.device.index == torch.cuda.current_device() and _skinny(T, w.size(0), w.size(1)))
+
+
 def _streams(x, w):
     """Whether x @ w^T goes through the kernel for the few rows of a decoding step."""
     return (type(x) is torch.Tensor and type(w) in (torch.Tensor, torch.nn.Parameter) and x.is_cuda and _called_plainly(x, w) and x.dim() == 2 and w.dim() == 2
@@ -684,6 +690,45 @@ class HipOps:
                                             dtype_code(w.dtype), float(eps), n, x.size(1), self.code, self._s()), "rms_norm_rows")
         return out
 
+    def _sum_routing(self, x, parts, gains, tokens, table, route):
+        """scaled_sum_rms_norms' rows through their router in the same launch: -> (*_routing, T, D), or None where moe_route is to be called."""
+        (a, sa), (e, se), (c, sc) = (list(parts) + [(None, None)] * 3)[:3]
+        T, D = (tokens.numel(), table.size(1)) if tokens is not None else x.shape
+        steps = (tokens is not None and not parts) or (tokens is None and isinstance(a, torch.Tensor) and isinstance(e, ExpertRows) and not isinstance(c, ExpertRows)
+                                                       and e.place is None and e.ys.dtype == torch.float32)
+        q = self._routing(route, T, D, x, a, sa, se, c, sc, table, *gains) if steps and len(gains) == 2 else None
+        return None if q is None else (*q, T, D)
+
+    def _sum_route_args(self, x, parts, gains, tokens, table, eps, q):
+        """-> (the two norms' rows, the arguments of the launch behind the stream's)."""
+        (a, sa), (e, se), (c, sc) = (list(parts) + [(None, None)] * 3)[:3]
+        T, D = q[3:]
+        hs = [torch.empty((T, D), dtype=self.dtype, device=gains[0].device) for _ in gains]
+        self._need(x, tokens, table, a, sa, se, c, sc, *gains, *((e.ys, e.idx, e.wt) if e is not None else ()))
+        assert (x is None or (x.dtype == torch.float32 and x.shape == (T, D))) and all(g.dtype == torch.float32 and g.numel() == D for g in gains)
+        assert all(y is None or (y.shape == (T, D) and (s is None or (s.dtype == self.dtype and s.numel() == D))) for y, s in ((a, sa), (e, se), (c, sc)))
+        at = lambda t: 0 if t is None else t.data_ptr()                              # noqa: E731
+        slots = (0, 0, 0, 0, 0) if e is None else (e.ys.data_ptr(), e.idx.data_ptr(), at(e.wt), e.idx.size(1), e.experts)
+        return hs, (hs[0].data_ptr(), hs[1].data_ptr(), at(a), at(sa), *slots, at(se), at(c), at(sc), gains[0].data_ptr(), gains[1].data_ptr(), at(tokens),
+                    at(table) if tokens is not None else 0, float(eps), T, D, *q[2])
+
+    def scaled_sum_rms_norms_product(self, x, parts, gains, eps, route, w, tokens=None, table=None):
+        """scaled_sum_rms_norms with its router and linear(its first norm's rows, w), in one launch for one or two tokens: -> (x, norms, (experts, weights), product), x
+        in a tensor of its own; None where that takes other launches (products wider than 6144 and 4096 too, sum_norms_product_kernel has the times)."""
+        T = tokens.numel() if tokens is not None else x.size(0)
+        if not (0 < T <= 2 and self.code == BF16 and _weight_streams(w, T) and _called_plainly(w) and w.size(0) % 4 == 0 and w.size(0) <= (6144 if T == 1 else 4096)
+                and w.size(1) % 64 == 0 and w.size(1) <= 2048):
+            return None
+        q = self._sum_routing(x, parts, gains, tokens, table, route)
+        if q is None or q[4] != w.size(1):
+            return None
+        hs, args = self._sum_route_args(x, parts, gains, tokens, table, eps, q)
+        new = torch.empty((T, q[4]), dtype=torch.float32, device=w.device)
+        out = torch.empty((T, w.size(0)), dtype=self.dtype, device=w.device)
+        self.check(self.L.qsv_sum_norms_product(out.data_ptr(), w.data_ptr(), w.size(0), int(self._kept(T)), new.data_ptr(), 0 if x is None else x.data_ptr(), *args),
+                   "sum_norms_product")
+        return new, hs, q[:2], out
+
     def scaled_sum_rms_norms(self, x, parts, gains, eps, tokens=None, table=None, route=None):
         """x += sum of scale * y over parts [(y, scale)] (up to three; y storage type, scale per coordinate in the storage type or None) in
         place, or, with tokens, x <- table[tokens] (+ the parts; x None: made here); -> (x, [rms_norm(x) * g in the storage type for the (up to
@@ -691,24 +736,13 @@ class HipOps:
         route: the arguments of moe_route behind the second norm's rows: -> (x, norms, their (experts, weights) or None where moe_route is to be called)."""
         assert len(parts) <= 3 and len(gains) <= 2
         if route is not None:
-            (a, sa), (e, se), (c, sc) = (list(parts) + [(None, None)] * 3)[:3]
-            T, D = (tokens.numel(), table.size(1)) if tokens is not None else x.shape
-            steps = (tokens is not None and not parts) or (tokens is None and isinstance(a, torch.Tensor) and isinstance(e, ExpertRows) and not isinstance(c, ExpertRows)
-                                                           and e.place is None and e.ys.dtype == torch.float32)
-            q = self._routing(route, T, D, x, a, sa, se, c, sc, table, *gains) if steps and len(gains) == 2 else None
+            q = self._sum_routing(x, parts, gains, tokens, table, route)
             if q is None:
                 return (*self.scaled_sum_rms_norms(x, parts, gains, eps, tokens, table), None)
             if x is None:
-                x = torch.empty((T, D), dtype=torch.float32, device=table.device)
-            hs = [torch.empty((T, D), dtype=self.dtype, device=x.device) for _ in gains]
-            self._need(x, tokens, table, a, sa, se, c, sc, *gains, *((e.ys, e.idx, e.wt) if e is not None else ()))
-            assert x.dtype == torch.float32 and x.shape == (T, D) and all(g.dtype == torch.float32 and g.numel() == D for g in gains)
-            assert all(y is None or (y.shape == x.shape and (s is None or (s.dtype == self.dtype and s.numel() == D))) for y, s in ((a, sa), (e, se), (c, sc)))
-            at = lambda t: 0 if t is None else t.data_ptr()                          # noqa: E731
-            slots = (0, 0, 0, 0, 0) if e is None else (e.ys.data_ptr(), e.idx.data_ptr(), at(e.wt), e.idx.size(1), e.experts)
-            self.check(self.L.qsv_scaled_sum_rms_norms_route(x.data_ptr(), hs[0].data_ptr(), hs[1].data_ptr(), at(a), at(sa), *slots, at(se), at(c), at(sc), gains[0].data_ptr(),
-                                                             gains[1].data_ptr(), at(tokens), at(table) if tokens is not None else 0, float(eps), T, D, *q[2]),
-                       "scaled_sum_rms_norms_route")
+                x = torch.empty((q[3], q[4]), dtype=torch.float32, device=table.device)
+            hs, args = self._sum_route_args(x, parts, gains, tokens, table, eps, q)
+            self.check(self.L.qsv_scaled_sum_rms_norms_route(x.data_ptr(), *args), "scaled_sum_rms_norms_route")
             return x, hs, q[:2]
         if any(isinstance(y, ExpertRows) for y, _ in parts):
             T, D = x.shape
@@ -1812,6 +1846,9 @@ class TorchOps:
 
     def rms_norm_rows(self, x, rows, w, eps):
         return self._rms(x if rows is None else x[rows.long()], w, eps).to(self.dtype)
+
+    def scaled_sum_rms_norms_product(self, *args, **kw):
+        return None
 
     def scaled_sum_rms_norms(self, x, parts, gains, eps, tokens=None, table=None, route=None):
         if route is not None:

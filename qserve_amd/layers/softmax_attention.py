@@ -305,9 +305,9 @@ class DifferentialAttention:
         self.cache_rows = [] if shared_kv else [(kv_heads, vdim + 2 * dim)]
         self.state_specs = [StateSpec((taps - 1, self.C), copies=2)] if taps > 1 else []
 
-    def __call__(self, h, batch, pools, states, beside=None):
+    def __call__(self, h, batch, pools, states, beside=None, proj=None):
         ops, H, d, dv, pool = self.ops, self.H, self.dim, self.vdim, pools[0]
-        proj = self.ops.linear(h, self.w_in)
+        proj = self.ops.linear(h, self.w_in) if proj is None else proj
         q = ops.conv_heads_cache(proj, self.conv, states[0] if self.taps > 1 else None, batch, 2 * H * d, 0 if self.shared_kv else self.G, 2 * d, dv,
                                  pool, self.scale, self.temperature)
         o = ops.diff_attention(q, pool, batch, H, d, dv, self.lam, self.out_scale, self.eps, proj[:, self.C:self.C + H * dv], self.page, beside=beside)
@@ -333,9 +333,9 @@ class TiedRotaryAttention:
         self.w_in, self.w_o = torch.cat([w["q"], w["k"]], dim=0).contiguous(), w["o"].contiguous()
         self.cache_rows, self.state_specs = [(kv_heads, 2 * dim)], []
 
-    def __call__(self, h, batch, pools, states, beside=None):
+    def __call__(self, h, batch, pools, states, beside=None, proj=None):
         ops, T, H, G, d, pool, rot = self.ops, h.size(0), self.H, self.G, self.dim, pools[0], self.rotary
-        proj = self.ops.linear(h, self.w_in)
+        proj = self.ops.linear(h, self.w_in) if proj is None else proj
         k = proj[:, H * d:]
         rope = rot.reserve(batch.max_pos + 1) if rot is not None else None
         plain = ops.maps_attention_ok(d, d, 1, self.page)        # queries in the storage type without the zeros in front

@@ -117,23 +117,25 @@ class Rivolix:
             L = self.layers[i]
             return [L["norm1"]] + ([L["norm2"]] if L["ff"] is not None else [])
 
-        def norms(x, parts, i, **start):                       # (a mixture's router runs in the kernel that makes its input)
+        def norms(x, parts, i, **start):                       # (a mixture's router runs in the kernel that makes its input, a short step's mixer's product too)
             ff = self.layers[i]["ff"] if i < n else None
             if type(ff) is SigmoidMoE:
-                return ops.scaled_sum_rms_norms(x, parts, gains(i), self.eps, route=ff.routing, **start)
-            return (*ops.scaled_sum_rms_norms(x, parts, gains(i), self.eps, **start), None)
+                mixer = self.layers[i]["mixer"]
+                made = ops.scaled_sum_rms_norms_product(x, parts, gains(i), self.eps, ff.routing, mixer.w_in, **start) if type(mixer) in (DifferentialAttention, TiedRotaryAttention) else None
+                return made or (*ops.scaled_sum_rms_norms(x, parts, gains(i), self.eps, route=ff.routing, **start), None)
+            return (*ops.scaled_sum_rms_norms(x, parts, gains(i), self.eps, **start), None, None)
 
-        x, hs, routed = norms(None, [], 0, tokens=batch.tokens, table=self.embed)
+        x, hs, routed, proj = norms(None, [], 0, tokens=batch.tokens, table=self.embed)
         for i, L in enumerate(self.layers):
             p0, p1, s0, s1 = self.slices[i]
             # neither side reads the other: a step's experts run in the launches of the mixer's attention and output product
             experts = L["ff"].pending(hs[1], routed) if routed is not None else None
-            parts = [(L["mixer"](hs[0], batch, pools[p0:p1], states[s0:s1], beside=experts), L["ls1"])]
+            parts = [(L["mixer"](hs[0], batch, pools[p0:p1], states[s0:s1], beside=experts, proj=proj), L["ls1"])]
             if L["ff"] is not None:
                 ys = L["ff"](hs[1], rows=True, routed=routed) if experts is None else experts.results()
                 parts += [(y, L["ls2"]) for y in ys]
             # the next layer's two inputs come out of the pass that adds this layer's outputs to the stream
-            _, hs, routed = norms(x, parts, i + 1)
+            x, hs, routed, proj = norms(x, parts, i + 1)
             if tap is not None:
                 tap(i, x)
         return x

@@ -82,7 +82,7 @@ class OpTimer:
              "attention_prep", "rotate_heads", "decay", "decay_products", "conv_silu_unit", "recurrent_scan", "head_rms_gate", "embed_sinusoid",
              "add_rms_norm", "rms_norm_rows", "normed_attention_prep", "max_gates", "add_normed_rms_norm", "qk_norm_rope_prep", "pool_blocks",
              "min_gru_scan", "relu_sq", "embed_rms_norm", "residual_conv", "scaled_add_rms_norm", "rotate_qk", "talking_attention",
-             "scaled_sum_rms_norms", "conv_heads_cache", "diff_attention", "single_map_attention", "linear", "float_linear")
+             "scaled_sum_rms_norms", "scaled_sum_rms_norms_product", "conv_heads_cache", "diff_attention", "single_map_attention", "linear", "float_linear")
     # another form of the same operation: its time is that operation's
     FORMS = {"latent_prompt": "latent_attention", "moe_experts_shared": "moe_experts", "float_linear": "linear"}
 
@@ -887,7 +887,7 @@ def bench_rivolix(name, s, dev, steps, warmup):
     g = torch.Generator().manual_seed(1)
     prompts = [torch.randint(0, VOCAB, (L,), generator=g).tolist() for _ in range(NB)]
     slots = [eng.open_sequence() for _ in range(NB)]
-    stateless = ("diff_attention", "single_map_attention", "scaled_sum_rms_norms", "conv_heads_cache", "qk_norm_rope_prep", "glu", "moe_route")
+    stateless = ("diff_attention", "single_map_attention", "scaled_sum_rms_norms", "scaled_sum_rms_norms_product", "conv_heads_cache", "qk_norm_rope_prep", "glu", "moe_route")
     pre_ms, ops_pre, rep_pre = [], None, {}
     for i in range(0, NB, BP):
         items = [(slots[j], prompts[j]) for j in range(i, i + BP)]

@@ -105,3 +105,29 @@ def test_latents_that_take_two_launches(ops):
         down, pool = _rand(g, T, q_rank + kv_rank + off)[:, off:].contiguous(), torch.zeros(65, kv_rank, dtype=BF, device=DEV)
         qw = _rand(g, q_rank + 1)[1:] if off else _rand(g, q_rank)
         assert ops.latent_up(down, 0, q_rank, qw, q_rank, kv_rank, _rand(g, kv_rank), 0, 0, None, pool, slot[:T], pos[:T], 1e-5, _rand(g, N, q_rank)) is None
+
+
+# one and two rows, one and several stages a wave (and waves without one), rows shorter than their threads, part groups of weight rows; each form of the sum, more experts than a trip takes
+@pytest.mark.parametrize("T", [1, 2])
+@pytest.mark.parametrize("D, N, E", [(64, 1024, 8), (576, 1028, 16), (1024, 4096, 5), (1088, 2560, 16), (2048, 5120, 16), (2048, 4096, 40), (1024, 6148, 16)])
+def test_norms_with_the_product_of_the_first(ops, T, D, N, E):
+    g = torch.Generator().manual_seed(T + D)
+    f32 = dict(dtype=torch.float32)
+    gains, w, table = [_rand(g, D, **f32) for _ in range(2)], _rand(g, N, D, scale=D ** -0.5), _rand(g, 11, D)
+    route = dict(router=_rand(g, E, D, scale=3.0 * D ** -0.5), top_k=2, groups=1, keep=1, score="sigmoid", scale=1.5)
+    tokens, x = torch.randint(0, 11, (T,), generator=g, dtype=torch.int32).to(DEV), _rand(g, T, D, **f32)
+    forms = [(None, [], dict(tokens=tokens, table=table))]
+    for top, weighted, parts in ((2, True, 2), (4, False, 3), (6, True, 3)):
+        idx = torch.randint(-1, E, (T, top), generator=g, dtype=torch.int32).to(DEV)
+        y = ExpertRows(ops, _rand(g, T * top, D, **f32), None, torch.rand(T, top, generator=g).to(DEV) if weighted else None, idx, _rand(g, T, D), E)
+        forms.append((x, [(_rand(g, T, D), _rand(g, D)), (y, _rand(g, D) if weighted else None), (_rand(g, T, D), _rand(g, D))][:parts], {}))
+    if N > (6144 if T == 1 else 4096):                                      # (two launches)
+        assert ops.scaled_sum_rms_norms_product(None, [], gains, 1e-5, route, w, tokens=tokens, table=table) is None
+        return
+    for at, parts, kw in forms:
+        x1, h1, r1, out = ops.scaled_sum_rms_norms_product(at, parts, gains, 1e-5, route, w, **kw)
+        x2, h2, r2 = ops.scaled_sum_rms_norms(None if at is None else at.clone(), parts, gains, 1e-5, route=route, **kw)
+        assert torch.equal(x1, x2) and all(torch.equal(a, b) for a, b in zip((*h1, *r1), (*h2, *r2))) and torch.equal(out, ops.linear(h2[0], w))
+        assert at is None or at is x and x1 is not x
+    assert ops.scaled_sum_rms_norms_product(None, [], gains, 1e-5, route, w, tokens=torch.zeros(3, dtype=torch.int32, device=DEV), table=table) is None
+    assert ops.scaled_sum_rms_norms_product(None, [], gains[:1], 1e-5, route, w, tokens=tokens, table=table) is None

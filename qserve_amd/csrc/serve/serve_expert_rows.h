@@ -131,13 +131,17 @@ __device__ __forceinline__ void expert_finish(const ExpertArgs& a, int r0, int c
 }
 
 // The work of workgroup (bx, by) of the launch's grid; lds: EXPERT_LDS bytes.
-template <int ACT, bool FOUT>
+// FORM: slots by the router's indices (SLOTS_EARLY, where early_experts says so: the indices and, behind them, the first weights are requested into LDS, where no load
+// into registers waits for them, and the slots are looked for while they are on their way) or sorted runs.  A form holds its own code only: a launch of a
+// step fetches its instructions anew, and what it jumps over costs it too (in one kernel with the others the early form gave steps of 64 sequences 0.7 % and took 0.5 from those of one; apart it gives 2.8 and takes nothing).
+enum { SLOTS, SLOTS_EARLY, SORTED_RUNS };
+template <int ACT, bool FOUT, int FORM = SLOTS>
 __device__ __forceinline__ void expert_rows_block(const ExpertArgs& a, const SharedArgs& sh, int bx, int by, unsigned char* lds) {
     unsigned char* rings = lds;
     unsigned short* list = (unsigned short*)(lds + STREAM_WAVES * XRING);
     int* listed = (int*)(list + XLIST);
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r0 = bx * XR;
-    if (sh.W && by == 0) {                                                 // (first: it has the most inputs)
+    if (FORM == SLOTS && sh.W && by == 0) {                                                 // (first: it has the most inputs)
         if (r0 >= sh.rows) return;
         const ExpertArgs b = {sh.out, sh.X, sh.W, nullptr, nullptr, nullptr, nullptr, sh.n, 1, sh.rows, sh.K, a.limit, sh.wide, true, false, 0};
         auto chunk = [&](int c0, auto once) __attribute__((always_inline)) {
@@ -161,39 +165,46 @@ __device__ __forceinline__ void expert_rows_block(const ExpertArgs& a, const Sha
         return;
     }
     if (r0 >= a.rows) return;
-    const int which = by - (sh.W ? 1 : 0), rows_here = min(XR, a.rows - r0);
+    const int which = by - (FORM == SLOTS && sh.W ? 1 : 0), rows_here = min(XR, a.rows - r0);
     int e = which;
-    if (a.by_slot) {                                                               // the expert of slot `which`, by its first slot
+    if (FORM == SLOTS && a.by_slot) {                                              // the expert of slot `which`, by its first slot
         e = a.idx[which];
         if ((unsigned)e >= (unsigned)a.by_slot) return;
     }
     const bf16_t* W0 = a.W + ((size_t)e * a.rows + r0) * (size_t)a.K;
     unsigned char* ring = rings + w * XRING;
-    // `count` inputs: X row by row_of(i), output row (and weight) by slot_of(i)
-    auto walk = [&](int count, auto row_of, auto slot_of) {
-        auto chunk = [&](int c0, auto once) __attribute__((always_inline)) {
-            constexpr bool ONCE = decltype(once)::value;
+    // `count` inputs: X row by row_of(i), output row (and weight) by slot_of(i); pre_: the first chunk's weights are on their way
+    auto walk = [&](int count, auto pre_, auto row_of, auto slot_of) __attribute__((always_inline)) {
+        auto chunk = [&](int c0, auto once, auto pre) __attribute__((always_inline)) {
+            constexpr bool ONCE = decltype(once)::value, PRE = decltype(pre)::value;
             const int c = min(32, count - c0);
             auto rows = [&](int i) { return a.X + (size_t)row_of(c0 + min(i, c - 1)) * (size_t)a.K; };
             auto slots = [&](int i, int64_t& slot, float& iw) { slot_of(c0 + i, slot, iw); };
             if (c <= 16) {
                 v4f acc[XR / 16][1];
-                stream_products<XR / 16, 1, ONCE>(W0, a.K, rows_here, ring, w, lane, rows, acc);
+                stream_products<XR / 16, 1, ONCE, PRE>(W0, a.K, rows_here, ring, w, lane, rows, acc);
                 expert_finish<ACT, FOUT, 1>(a, r0, c, rings, w, lane, slots, acc);
             } else {
                 v4f acc[XR / 16][2];
-                stream_products<XR / 16, 2, ONCE>(W0, a.K, rows_here, ring, w, lane, rows, acc);
+                stream_products<XR / 16, 2, ONCE, PRE>(W0, a.K, rows_here, ring, w, lane, rows, acc);
                 expert_finish<ACT, FOUT, 2>(a, r0, c, rings, w, lane, slots, acc);
             }
         };
-        if (count <= 0) return;
-        if (count <= 32 && a.once) chunk(0, std::true_type());
-        else
-            for (int c0 = 0; c0 < count; c0 += 32) chunk(c0, std::false_type());
+        if (count <= 0) {
+            if (decltype(pre_)::value) wait_vm<0>();                               // (the workgroup's LDS is another's once it ends)
+            return;
+        }
+        if (count <= 32 && a.once) return chunk(0, std::true_type(), pre_);
+        int c0 = 0;
+        if constexpr (decltype(pre_)::value) {
+            chunk(0, std::false_type(), pre_);
+            c0 = 32;
+        }
+        for (; c0 < count; c0 += 32) chunk(c0, std::false_type(), std::false_type());
     };
-    if (a.offsets) {
+    if constexpr (FORM == SORTED_RUNS) {
         const int64_t s0 = a.offsets[e];
-        walk((int)(a.offsets[e + 1] - s0),
+        walk((int)(a.offsets[e + 1] - s0), std::false_type(),
              [&](int i) {
                  const int64_t s = s0 + i;
                  return a.x_index ? a.x_index[s] / a.div : s;
@@ -204,19 +215,40 @@ __device__ __forceinline__ void expert_rows_block(const ExpertArgs& a, const Sha
              });
         return;
     }
-    for (int n0 = 0; n0 < a.n; n0 += XLIST) {
+    constexpr bool EARLY_W = FORM == SLOTS_EARLY;
+    constexpr int PIECES = XLIST / EXPERT_THREADS;
+    const int* held = (const int*)(ring + XRING - 2048);                           // (an input's place: not requested before the search is done)
+    if constexpr (EARLY_W) {
+        const int span = (a.n + EXPERT_THREADS - 1) / EXPERT_THREADS * 64;
+        const unsigned dst = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(lds_ptr)held);
+        wait_vm<0>();
+#pragma unroll
+        for (int q = 0; q < PIECES; ++q)
+            if (64 * q < span) lds_copy4(dst + 256 * q, a.idx + min(w * span + 64 * q + lane, a.n - 1));
+        if (a.once) request_early<XR / 16, true>(W0, a.K, rows_here, ring, w, lane);
+        else request_early<XR / 16, false>(W0, a.K, rows_here, ring, w, lane);
+        wait_vm<EARLY * 2 * (XR / 16)>();
+    }
+    for (int n0 = 0; n0 < a.n; n0 += XLIST) {                                      // (EARLY_W: once)
         // this expert's slots among the next XLIST, in order: wave w looks at a quarter of them
         const int len = min(XLIST, a.n - n0), span = (len + EXPERT_THREADS - 1) / EXPERT_THREADS * 64;
         int found = 0;
-        unsigned long long hit[XLIST / EXPERT_THREADS];
+        unsigned long long hit[PIECES];
+        if constexpr (EARLY_W) {
 #pragma unroll
-        for (int q = 0; q < XLIST / EXPERT_THREADS; ++q) {
-            const int i = w * span + 64 * q + lane;
-            hit[q] = __ballot(64 * q < span && i < len && a.idx[n0 + i] == e);
-            found += __popcll(hit[q]);
+            for (int q = 0; q < PIECES; ++q) hit[q] = __ballot(64 * q < span && w * span + 64 * q + lane < len && held[64 * q + lane] == e);
+        } else {
+#pragma unroll
+            for (int q = 0; q < PIECES; ++q) {
+                const int i = w * span + 64 * q + lane;
+                hit[q] = __ballot(64 * q < span && i < len && a.idx[n0 + i] == e);
+            }
         }
+#pragma unroll
+        for (int q = 0; q < PIECES; ++q) found += __popcll(hit[q]);
         if (lane == 0) listed[w] = found;
-        __syncthreads();
+        if constexpr (EARLY_W) barrier_in_flight();
+        else __syncthreads();
         int at = 0, count = 0;
 #pragma unroll
         for (int o = 0; o < STREAM_WAVES; ++o) {
@@ -224,21 +256,31 @@ __device__ __forceinline__ void expert_rows_block(const ExpertArgs& a, const Sha
             count += listed[o];
         }
 #pragma unroll
-        for (int q = 0; q < XLIST / EXPERT_THREADS; ++q) {
+        for (int q = 0; q < PIECES; ++q) {
             if (hit[q] >> lane & 1) list[at + __popcll(hit[q] & ((1ull << lane) - 1))] = (unsigned short)(w * span + 64 * q + lane);
             at += __popcll(hit[q]);
         }
-        __syncthreads();
-        if (a.by_slot && list[0] != which) return;                                 // (an earlier slot's workgroups do this expert)
-        walk(count, [&](int i) { return (int64_t)((n0 + list[i]) / a.div); },
-             [&](int i, int64_t& slot, float& iw) {
-                 slot = n0 + list[i];
-                 if (a.in_weight) iw = a.in_weight[slot];
-             });
+        if constexpr (EARLY_W) barrier_in_flight();
+        else __syncthreads();
+        if (FORM == SLOTS && a.by_slot && list[0] != which) return;                     // (an earlier slot's workgroups do this expert)
+        auto row_of = [&](int i) { return (int64_t)((n0 + list[i]) / a.div); };
+        auto slot_of = [&](int i, int64_t& slot, float& iw) {
+            slot = n0 + list[i];
+            if (a.in_weight) iw = a.in_weight[slot];
+        };
+        walk(count, std::integral_constant<bool, EARLY_W>(), row_of, slot_of);
+        if constexpr (EARLY_W) return;
         __syncthreads();
     }
 }
 
+// Whether the weights are requested before the slots are looked for, of a launch that plan_expert_rows has passed.  Measured, 16 experts, 16 / 24 slots each, out of memory, us: 1024 x
+// 2048 16.7 -> 15.7, 17.7 -> 16.8, 1408 x 2048 21.6 -> 21.0, 23.1 -> 21.9, 2048 x 1408 19.4 -> 18.8, 21.3 -> 20.5, 2816 x 2048 37.9 -> 36.3, 40.1 -> 38.7, 5632 x 2048 69.3 -> 68.4,
+// 73.8 -> 72.2.  The first requests of an expert that no slot has are for nothing (a quarter of its weights): steps of 4 tokens, top 4 of 16, took 4 % longer, so four
+// slots an expert on average, of which one expert in 50 has none.
+inline bool early_experts(const ExpertArgs& a, const SharedArgs& sh, int n_experts) {
+    return a.idx && !sh.W && !a.by_slot && a.n <= XLIST && a.n >= 4 * n_experts && a.K >= EARLY_MIN;
+}
 // Checks of a launch (a, sh as its caller filled them in), what it derives from them, and its grid; act: clamped units become ACT_GLU.
 inline int plan_expert_rows(const char* what, ExpertArgs& a, SharedArgs& sh, int n_experts, int& act, bool kept, dim3& grid) {
     QSV_REQUIRE(a.out && a.X && a.W && n_experts > 0 && a.rows > 0 && a.div > 0, "%s: bad arguments", what);

@@ -385,10 +385,10 @@ __global__ __launch_bounds__(NT) void moe_down_vec_kernel(T* __restrict__ y, con
 }
 
 // expert_rows_block (serve_expert_rows.h) as a launch of its own
-template <int ACT, bool FOUT>
+template <int ACT, bool FOUT, int FORM>
 __global__ __launch_bounds__(NT, 2) void expert_rows_kernel(ExpertArgs a, SharedArgs sh) {
     __shared__ __attribute__((aligned(128))) unsigned char lds[EXPERT_LDS];
-    expert_rows_block<ACT, FOUT>(a, sh, blockIdx.x, blockIdx.y, lds);
+    expert_rows_block<ACT, FOUT, FORM>(a, sh, blockIdx.x, blockIdx.y, lds);
 }
 
 // ---- expert-sorted form (many tokens): the products are the vendor's, per expert over contiguous runs of sorted slots; these
@@ -452,10 +452,18 @@ static int launch_expert_rows(const char* what, ExpertArgs a, int n_experts, int
     const int rc = plan_expert_rows(what, a, sh, n_experts, act, kept, grid);
     if (rc != QSV_OK) return rc;
     const dim3 block(NT);
-    if (float_out) hipLaunchKernelGGL((expert_rows_kernel<ACT_NONE, true>), grid, block, 0, (hipStream_t)stream, a, sh);
-    else if (act == ACT_RELU_SQ) hipLaunchKernelGGL((expert_rows_kernel<ACT_RELU_SQ, false>), grid, block, 0, (hipStream_t)stream, a, sh);
-    else if (act == ACT_GLU) hipLaunchKernelGGL((expert_rows_kernel<ACT_GLU, false>), grid, block, 0, (hipStream_t)stream, a, sh);
-    else hipLaunchKernelGGL((expert_rows_kernel<ACT_NONE, false>), grid, block, 0, (hipStream_t)stream, a, sh);
+    const bool early = early_experts(a, sh, n_experts);
+#define QSV_EXPERTS(ACT, FOUT)                                                                                                                          \
+    do {                                                                                                                                                \
+        auto kernel = a.offsets ? expert_rows_kernel<ACT, FOUT, SORTED_RUNS> : early ? expert_rows_kernel<ACT, FOUT, SLOTS_EARLY>                       \
+                                                                                     : expert_rows_kernel<ACT, FOUT, SLOTS>;                            \
+        hipLaunchKernelGGL(kernel, grid, block, 0, (hipStream_t)stream, a, sh);                                                                         \
+    } while (0)
+    if (float_out) QSV_EXPERTS(ACT_NONE, true);                                    // (sorted runs: never)
+    else if (act == ACT_RELU_SQ) QSV_EXPERTS(ACT_RELU_SQ, false);
+    else if (act == ACT_GLU) QSV_EXPERTS(ACT_GLU, false);
+    else QSV_EXPERTS(ACT_NONE, false);
+#undef QSV_EXPERTS
     return qsv_launch_status(what);
 }
 extern "C" int qsv_expert_rows(void* out, const void* X, const int64_t* x_index, int div, const void* W, const int64_t* offsets,

@@ -336,7 +336,7 @@ class HipOps:
     def latent_up(self, down, q_off, q_rank, q_w, kv_off, kv_rank, kv_w, rot_dim, rot_n, rope, pool, slot, pos, eps, w_uq):
         """linear(latent_prep(...), w_uq) [T, N] for a step's few rows in one launch; None where that takes two."""
         T, N = down.size(0), w_uq.size(0)
-        if not (T > 0 and w_uq.size(1) == q_rank and _streams(down[:, q_off:q_off + q_rank], w_uq) and _called_plainly(q_w, kv_w)
+        if not (0 < T <= 16 and w_uq.size(1) == q_rank and _streams(down[:, q_off:q_off + q_rank], w_uq) and _called_plainly(q_w, kv_w)
                 and self.L.qsv_latent_up_ok(T, q_off, q_rank, kv_off, kv_rank, rot_dim, down.stride(0), N)
                 and (q_w.data_ptr() | kv_w.data_ptr() | pool.data_ptr()) % 8 == 0):
             return None

@@ -131,3 +131,23 @@ def test_norms_with_the_product_of_the_first(ops, T, D, N, E):
         assert at is None or at is x and x1 is not x
     assert ops.scaled_sum_rms_norms_product(None, [], gains, 1e-5, route, w, tokens=torch.zeros(3, dtype=torch.int32, device=DEV), table=table) is None
     assert ops.scaled_sum_rms_norms_product(None, [], gains[:1], 1e-5, route, w, tokens=tokens, table=table) is None
+
+
+# three stages a wave and a row that ends inside one, rows that end inside a workgroup, all slots of a search, experts with none, up to 16, up to 32 and more slots; beside
+# experts that nobody chooses (so many that the slots are looked for first)
+@pytest.mark.parametrize("T, top, D, ff", [(16, 4, 768, 776), (64, 2, 776, 768), (64, 4, 2048, 1032), (256, 4, 1024, 840), (250, 4, 1304, 2048)])
+@pytest.mark.parametrize("act, weigh", [("relu_sq", "output"), ("swiglu", "input")])
+@pytest.mark.parametrize("kept", [None, 0])
+def test_expert_weights_requested_before_their_slots(ops, T, top, D, ff, act, weigh, kept):
+    g = torch.Generator().manual_seed(T + D)
+    E, more = 8, T * top // 4 + 1
+    rows = ff * (2 if act == "swiglu" else 1)
+    up, down, h = _rand(g, E, rows, D, scale=D ** -0.5), _rand(g, E, D, ff, scale=ff ** -0.5), _rand(g, T, D)
+    share = torch.tensor([0.0, 0.02, 0.05, 0.08, 0.1, 0.15, 0.2, 0.4])
+    idx = torch.multinomial(share, T * top, replacement=True, generator=g).int().view(T, top)
+    idx[0, 0] = -1
+    idx, wt = idx.to(DEV), torch.rand(T, top, generator=g).to(DEV)
+    ops.moe_expert_major_slots, ops.kept_above = 10 ** 9, kept
+    out = ops.moe_experts(h, up, down, idx, wt, act=act, weigh=weigh)
+    wide = [torch.cat([w, w.new_zeros(more - E, *w.shape[1:])]) for w in (up, down)]
+    assert torch.equal(out, ops.moe_experts(h, *wide, idx, wt, act=act, weigh=weigh))

@@ -799,7 +799,7 @@ __global__ __launch_bounds__(NT, (Shape<DT, CT, M>::STEP_OCC)) void maps_step_ke
 // 2048 x 1408 and a shared one): 1 token behind 64 / 333 / 4000 positions 30.0 -> 19.5, 35.6 -> 21.7, 47.6 -> 35.1; 16 behind 300 72.6 -> 56.4; 64 behind 100 /
 // 1000 / 3000 77 -> 70, 99 -> 83, 153 -> 129; 4 of 32 experts of 4096 x 2752, 1 / 16 / 64 behind 333 / 300 / 8000 83 -> 69, 370 -> 353, 582 -> 544.  Faster at every size tried, so
 // wherever the sizes fit (maps of 128 over values of 128 need more registers, 32 heads a pool over wide values more LDS: those run apart).
-template <int DT, int CT, int M>
+template <int DT, int CT, int M, int FORM>
 __global__ __launch_bounds__(NT, 2) void maps_beside_experts_kernel(MapsArgs a, ExpertArgs e, SharedArgs sh, int blocks, int ny, int tiles) {
     using S = Shape<DT, CT, M>;
     __shared__ __attribute__((aligned(128))) unsigned char lds[EXPERT_LDS];
@@ -809,7 +809,7 @@ __global__ __launch_bounds__(NT, 2) void maps_beside_experts_kernel(MapsArgs a, 
         return;
     }
     b -= blocks;
-    expert_rows_block<ACT_GLU, false>(e, sh, b % tiles, b / tiles, lds);
+    expert_rows_block<ACT_GLU, false, FORM>(e, sh, b % tiles, b / tiles, lds);
 }
 
 template <int VDIM, int M>
@@ -845,7 +845,9 @@ int launch_maps(MapsArgs a, const int32_t* prompt_tiles, int n_prompt, const int
                         "qsv_maps_attention_beside: not these experts or tiles");
             a.tiles = step_tiles;
             a.n_tiles = n_step;
-            hipLaunchKernelGGL((maps_beside_experts_kernel<DT, CT, M>), dim3((unsigned)all), dim3(NT), 0, st, a, e, sh, (int)blocks, gy, (int)grid.x);
+            // (workgroups by slot: the attention is the longer part, and beside the general form it takes 0.7 % of a step less; 3 and 4 tokens gain 2.5 % of a step by the small one)
+            auto kernel = few_slots(e, sh) && !e.by_slot ? maps_beside_experts_kernel<DT, CT, M, SLOTS_FEW> : maps_beside_experts_kernel<DT, CT, M, SLOTS>;
+            hipLaunchKernelGGL(kernel, dim3((unsigned)all), dim3(NT), 0, st, a, e, sh, (int)blocks, gy, (int)grid.x);
             rc = qsv_launch_status("qsv_maps_attention_beside");
             if (rc != QSV_OK) return rc;
             if (a.Z > 1) hipLaunchKernelGGL((maps_merge_kernel<S::VDIM, M>), dim3(n_step, gy), dim3(NT), 0, st, a);

@@ -132,16 +132,18 @@ __device__ __forceinline__ void expert_finish(const ExpertArgs& a, int r0, int c
 
 // The work of workgroup (bx, by) of the launch's grid; lds: EXPERT_LDS bytes.
 // FORM: slots by the router's indices (SLOTS_EARLY, where early_experts says so: the indices and, behind them, the first weights are requested into LDS, where no load
-// into registers waits for them, and the slots are looked for while they are on their way) or sorted runs.  A form holds its own code only: a launch of a
+// into registers waits for them, and the slots are looked for while they are on their way;
+// SLOTS_FEW, where few_slots says so: one group of inputs and one policy) or sorted runs.  A form holds its own code only: a launch of a
 // step fetches its instructions anew, and what it jumps over costs it too (in one kernel with the others the early form gave steps of 64 sequences 0.7 % and took 0.5 from those of one; apart it gives 2.8 and takes nothing).
-enum { SLOTS, SLOTS_EARLY, SORTED_RUNS };
+enum { SLOTS, SLOTS_EARLY, SORTED_RUNS, SLOTS_FEW };
 template <int ACT, bool FOUT, int FORM = SLOTS>
 __device__ __forceinline__ void expert_rows_block(const ExpertArgs& a, const SharedArgs& sh, int bx, int by, unsigned char* lds) {
     unsigned char* rings = lds;
     unsigned short* list = (unsigned short*)(lds + STREAM_WAVES * XRING);
     int* listed = (int*)(list + XLIST);
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r0 = bx * XR;
-    if (FORM == SLOTS && sh.W && by == 0) {                                                 // (first: it has the most inputs)
+    constexpr bool FEW = FORM == SLOTS_FEW, GENERAL = FORM == SLOTS || FEW;
+    if (GENERAL && sh.W && by == 0) {                                                 // (first: it has the most inputs)
         if (r0 >= sh.rows) return;
         const ExpertArgs b = {sh.out, sh.X, sh.W, nullptr, nullptr, nullptr, nullptr, sh.n, 1, sh.rows, sh.K, a.limit, sh.wide, true, false, 0};
         auto chunk = [&](int c0, auto once) __attribute__((always_inline)) {
@@ -149,7 +151,7 @@ __device__ __forceinline__ void expert_rows_block(const ExpertArgs& a, const Sha
             const int c = min(32, sh.n - c0);
             auto rows = [&](int i) { return sh.X + (size_t)(c0 + min(i, c - 1)) * (size_t)sh.K; };
             auto slots = [&](int i, int64_t& slot, float&) { slot = c0 + i; };
-            if (c <= 16) {
+            if (FEW || c <= 16) {
                 v4f acc[XR / 16][1];
                 stream_products<XR / 16, 1, ONCE>(sh.W + (size_t)r0 * sh.K, sh.K, min(XR, sh.rows - r0), rings + w * XRING, w, lane, rows, acc);
                 expert_finish<ACT, false, 1>(b, r0, c, rings, w, lane, slots, acc);
@@ -159,15 +161,14 @@ __device__ __forceinline__ void expert_rows_block(const ExpertArgs& a, const Sha
                 expert_finish<ACT, false, 2>(b, r0, c, rings, w, lane, slots, acc);
             }
         };
-        if (sh.n <= 32 && sh.once) chunk(0, std::true_type());
-        else
-            for (int c0 = 0; c0 < sh.n; c0 += 32) chunk(c0, std::false_type());
+        if (FEW || (sh.n <= 32 && sh.once)) return chunk(0, std::true_type());
+        for (int c0 = 0; c0 < sh.n; c0 += 32) chunk(c0, std::false_type());
         return;
     }
     if (r0 >= a.rows) return;
-    const int which = by - (FORM == SLOTS && sh.W ? 1 : 0), rows_here = min(XR, a.rows - r0);
+    const int which = by - (GENERAL && sh.W ? 1 : 0), rows_here = min(XR, a.rows - r0);
     int e = which;
-    if (FORM == SLOTS && a.by_slot) {                                              // the expert of slot `which`, by its first slot
+    if (GENERAL && a.by_slot) {                                              // the expert of slot `which`, by its first slot
         e = a.idx[which];
         if ((unsigned)e >= (unsigned)a.by_slot) return;
     }
@@ -180,7 +181,7 @@ __device__ __forceinline__ void expert_rows_block(const ExpertArgs& a, const Sha
             const int c = min(32, count - c0);
             auto rows = [&](int i) { return a.X + (size_t)row_of(c0 + min(i, c - 1)) * (size_t)a.K; };
             auto slots = [&](int i, int64_t& slot, float& iw) { slot_of(c0 + i, slot, iw); };
-            if (c <= 16) {
+            if (FEW || c <= 16) {
                 v4f acc[XR / 16][1];
                 stream_products<XR / 16, 1, ONCE, PRE>(W0, a.K, rows_here, ring, w, lane, rows, acc);
                 expert_finish<ACT, FOUT, 1>(a, r0, c, rings, w, lane, slots, acc);
@@ -194,7 +195,7 @@ __device__ __forceinline__ void expert_rows_block(const ExpertArgs& a, const Sha
             if (decltype(pre_)::value) wait_vm<0>();                               // (the workgroup's LDS is another's once it ends)
             return;
         }
-        if (count <= 32 && a.once) return chunk(0, std::true_type(), pre_);
+        if (FEW || (count <= 32 && a.once)) return chunk(0, std::true_type(), pre_);
         int c0 = 0;
         if constexpr (decltype(pre_)::value) {
             chunk(0, std::false_type(), pre_);
@@ -216,7 +217,7 @@ __device__ __forceinline__ void expert_rows_block(const ExpertArgs& a, const Sha
         return;
     }
     constexpr bool EARLY_W = FORM == SLOTS_EARLY;
-    constexpr int PIECES = XLIST / EXPERT_THREADS;
+    constexpr int PIECES = FEW ? 1 : XLIST / EXPERT_THREADS;
     const int* held = (const int*)(ring + XRING - 2048);                           // (an input's place: not requested before the search is done)
     if constexpr (EARLY_W) {
         const int span = (a.n + EXPERT_THREADS - 1) / EXPERT_THREADS * 64;
@@ -229,7 +230,7 @@ __device__ __forceinline__ void expert_rows_block(const ExpertArgs& a, const Sha
         else request_early<XR / 16, false>(W0, a.K, rows_here, ring, w, lane);
         wait_vm<EARLY * 2 * (XR / 16)>();
     }
-    for (int n0 = 0; n0 < a.n; n0 += XLIST) {                                      // (EARLY_W: once)
+    for (int n0 = 0; n0 < a.n; n0 += XLIST) {                                      // (EARLY_W, FEW: once)
         // this expert's slots among the next XLIST, in order: wave w looks at a quarter of them
         const int len = min(XLIST, a.n - n0), span = (len + EXPERT_THREADS - 1) / EXPERT_THREADS * 64;
         int found = 0;
@@ -262,14 +263,14 @@ __device__ __forceinline__ void expert_rows_block(const ExpertArgs& a, const Sha
         }
         if constexpr (EARLY_W) barrier_in_flight();
         else __syncthreads();
-        if (FORM == SLOTS && a.by_slot && list[0] != which) return;                     // (an earlier slot's workgroups do this expert)
+        if (GENERAL && a.by_slot && list[0] != which) return;                     // (an earlier slot's workgroups do this expert)
         auto row_of = [&](int i) { return (int64_t)((n0 + list[i]) / a.div); };
         auto slot_of = [&](int i, int64_t& slot, float& iw) {
             slot = n0 + list[i];
             if (a.in_weight) iw = a.in_weight[slot];
         };
         walk(count, std::integral_constant<bool, EARLY_W>(), row_of, slot_of);
-        if constexpr (EARLY_W) return;
+        if constexpr (EARLY_W || FEW) return;
         __syncthreads();
     }
 }
@@ -281,6 +282,9 @@ __device__ __forceinline__ void expert_rows_block(const ExpertArgs& a, const Sha
 inline bool early_experts(const ExpertArgs& a, const SharedArgs& sh, int n_experts) {
     return a.idx && !sh.W && !a.by_slot && a.n <= XLIST && a.n >= 4 * n_experts && a.K >= EARLY_MIN;
 }
+// Whether one group of inputs and the weights' one reading are all that a launch has: steps of 4 sequences 6600 -> 6440 us (Rivolix, 20 of them and their prompts), 8420 -> 8260
+// (Mumelix), 7270 -> 7100 (Vekalorn), of two 6460 -> 6350
+inline bool few_slots(const ExpertArgs& a, const SharedArgs& sh) { return a.idx && a.n <= 16 && a.once && (!sh.W || (sh.n <= 16 && sh.once)); }
 // Checks of a launch (a, sh as its caller filled them in), what it derives from them, and its grid; act: clamped units become ACT_GLU.
 inline int plan_expert_rows(const char* what, ExpertArgs& a, SharedArgs& sh, int n_experts, int& act, bool kept, dim3& grid) {
     QSV_REQUIRE(a.out && a.X && a.W && n_experts > 0 && a.rows > 0 && a.div > 0, "%s: bad arguments", what);

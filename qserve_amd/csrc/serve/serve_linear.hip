@@ -98,12 +98,12 @@ __global__ __launch_bounds__(64 * STREAM_WAVES, 2) void decay_products_kernel(Sk
 // A product (its first `blocks` workgroups, `columns` of them for the same inputs) beside the second products of a mixture's experts, which read nothing of it: a
 // launch and its start less (2048 x 2048 beside 4 of 16 experts of 2048 x 1408 and a shared one, 1 / 16 / 64 tokens 3.9 / 5.6 / 4.5 us; figures of a whole layer at
 // maps_beside_experts_kernel).
-template <int RB, int SG, bool ONCE>
+template <int RB, int SG, bool ONCE, int FORM>
 __global__ __launch_bounds__(64 * STREAM_WAVES, 2) void skinny_beside_experts_kernel(SkinnyJob a, ExpertArgs e, SharedArgs sh, int blocks, int columns, int tiles) {
     __shared__ __attribute__((aligned(128))) unsigned char lds[EXPERT_LDS];
     const int b = blockIdx.x;
     if (b < blocks) skinny_product<RB, SG, AS_IS, ONCE>(a, b % columns, b / columns, lds);
-    else expert_rows_block<ACT_NONE, true>(e, sh, (b - blocks) % tiles, (b - blocks) / tiles, lds);
+    else expert_rows_block<ACT_NONE, true, FORM>(e, sh, (b - blocks) % tiles, (b - blocks) / tiles, lds);
 }
 
 // ---- one product per head: y[t, h] = x[t, h] @ W[h], W [H, K, N] with N contiguous -------------------------------------------------------
@@ -429,7 +429,9 @@ static int launch_skinny(const char* what, void* out, const void* x, int64_t x_s
             if constexpr (HOW == AS_IS) {                                                                                                     \
                 const int64_t blocks = (int64_t)grid.x * grid.y, all = blocks + (int64_t)experts.x * experts.y;                               \
                 QSV_REQUIRE(all < (1ll << 31), "%s: too many workgroups", what);                                                              \
-                auto kernel = past ? skinny_beside_experts_kernel<RB, SG, true> : skinny_beside_experts_kernel<RB, SG, false>;                \
+                auto kernel = past ? skinny_beside_experts_kernel<RB, SG, true, SLOTS> : skinny_beside_experts_kernel<RB, SG, false, SLOTS>;  \
+                if (SG == 1 && few_slots(e, sh))                                                                                              \
+                    kernel = past ? skinny_beside_experts_kernel<RB, 1, true, SLOTS_FEW> : skinny_beside_experts_kernel<RB, 1, false, SLOTS_FEW>; \
                 hipLaunchKernelGGL(kernel, dim3((unsigned)all), block, 0, (hipStream_t)stream, a, e, sh, (int)blocks, (int)grid.x, (int)experts.x); \
             }                                                                                                                                 \
         } else if (past)                                                                                                                      \

@@ -456,7 +456,7 @@ static int launch_expert_rows(const char* what, ExpertArgs a, int n_experts, int
 #define QSV_EXPERTS(ACT, FOUT)                                                                                                                          \
     do {                                                                                                                                                \
         auto kernel = a.offsets ? expert_rows_kernel<ACT, FOUT, SORTED_RUNS> : early ? expert_rows_kernel<ACT, FOUT, SLOTS_EARLY>                       \
-                                                                                     : expert_rows_kernel<ACT, FOUT, SLOTS>;                            \
+                                             : few_slots(a, sh) ? expert_rows_kernel<ACT, FOUT, SLOTS_FEW> : expert_rows_kernel<ACT, FOUT, SLOTS>;      \
         hipLaunchKernelGGL(kernel, grid, block, 0, (hipStream_t)stream, a, sh);                                                                         \
     } while (0)
     if (float_out) QSV_EXPERTS(ACT_NONE, true);                                    // (sorted runs: never)

@@ -847,6 +847,7 @@ int launch_maps(MapsArgs a, const int32_t* prompt_tiles, int n_prompt, const int
             a.n_tiles = n_step;
             // (workgroups by slot: the attention is the longer part, and beside the general form it takes 0.7 % of a step less; 3 and 4 tokens gain 2.5 % of a step by the small one)
             auto kernel = few_slots(e, sh) && !e.by_slot ? maps_beside_experts_kernel<DT, CT, M, SLOTS_FEW> : maps_beside_experts_kernel<DT, CT, M, SLOTS>;
+            if (early_experts(e, beside->n_experts)) kernel = maps_beside_experts_kernel<DT, CT, M, SLOTS_EARLY>;
             hipLaunchKernelGGL(kernel, dim3((unsigned)all), dim3(NT), 0, st, a, e, sh, (int)blocks, gy, (int)grid.x);
             rc = qsv_launch_status("qsv_maps_attention_beside");
             if (rc != QSV_OK) return rc;

@@ -142,8 +142,8 @@ __device__ __forceinline__ void expert_rows_block(const ExpertArgs& a, const Sha
     unsigned short* list = (unsigned short*)(lds + STREAM_WAVES * XRING);
     int* listed = (int*)(list + XLIST);
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r0 = bx * XR;
-    constexpr bool FEW = FORM == SLOTS_FEW, GENERAL = FORM == SLOTS || FEW;
-    if (GENERAL && sh.W && by == 0) {                                                 // (first: it has the most inputs)
+    constexpr bool FEW = FORM == SLOTS_FEW, GENERAL = FORM == SLOTS || FEW, SHARED = FORM != SORTED_RUNS;
+    if (SHARED && sh.W && by == 0) {                                                 // (first: it has the most inputs)
         if (r0 >= sh.rows) return;
         const ExpertArgs b = {sh.out, sh.X, sh.W, nullptr, nullptr, nullptr, nullptr, sh.n, 1, sh.rows, sh.K, a.limit, sh.wide, true, false, 0};
         auto chunk = [&](int c0, auto once) __attribute__((always_inline)) {
@@ -166,7 +166,7 @@ __device__ __forceinline__ void expert_rows_block(const ExpertArgs& a, const Sha
         return;
     }
     if (r0 >= a.rows) return;
-    const int which = by - (GENERAL && sh.W ? 1 : 0), rows_here = min(XR, a.rows - r0);
+    const int which = by - (SHARED && sh.W ? 1 : 0), rows_here = min(XR, a.rows - r0);
     int e = which;
     if (GENERAL && a.by_slot) {                                              // the expert of slot `which`, by its first slot
         e = a.idx[which];
@@ -279,8 +279,8 @@ __device__ __forceinline__ void expert_rows_block(const ExpertArgs& a, const Sha
 // 2048 16.7 -> 15.7, 17.7 -> 16.8, 1408 x 2048 21.6 -> 21.0, 23.1 -> 21.9, 2048 x 1408 19.4 -> 18.8, 21.3 -> 20.5, 2816 x 2048 37.9 -> 36.3, 40.1 -> 38.7, 5632 x 2048 69.3 -> 68.4,
 // 73.8 -> 72.2.  The first requests of an expert that no slot has are for nothing (a quarter of its weights): steps of 4 tokens, top 4 of 16, took 4 % longer, so four
 // slots an expert on average, of which one expert in 50 has none.
-inline bool early_experts(const ExpertArgs& a, const SharedArgs& sh, int n_experts) {
-    return a.idx && !sh.W && !a.by_slot && a.n <= XLIST && a.n >= 4 * n_experts && a.K >= EARLY_MIN;
+inline bool early_experts(const ExpertArgs& a, int n_experts) {
+    return a.idx && !a.by_slot && a.n <= XLIST && a.n >= 4 * n_experts && a.K >= EARLY_MIN;
 }
 // Whether one group of inputs and the weights' one reading are all that a launch has: steps of 4 sequences 6600 -> 6440 us (Rivolix, 20 of them and their prompts), 8420 -> 8260
 // (Mumelix), 7270 -> 7100 (Vekalorn), of two 6460 -> 6350

@@ -430,7 +430,9 @@ static int launch_skinny(const char* what, void* out, const void* x, int64_t x_s
                 const int64_t blocks = (int64_t)grid.x * grid.y, all = blocks + (int64_t)experts.x * experts.y;                               \
                 QSV_REQUIRE(all < (1ll << 31), "%s: too many workgroups", what);                                                              \
                 auto kernel = past ? skinny_beside_experts_kernel<RB, SG, true, SLOTS> : skinny_beside_experts_kernel<RB, SG, false, SLOTS>;  \
-                if (SG == 1 && few_slots(e, sh))                                                                                              \
+                if (early_experts(e, beside->n_experts))                                                                                      \
+                    kernel = past ? skinny_beside_experts_kernel<RB, SG, true, SLOTS_EARLY> : skinny_beside_experts_kernel<RB, SG, false, SLOTS_EARLY>; \
+                else if (SG == 1 && few_slots(e, sh))                                                                                              \
                     kernel = past ? skinny_beside_experts_kernel<RB, 1, true, SLOTS_FEW> : skinny_beside_experts_kernel<RB, 1, false, SLOTS_FEW>; \
                 hipLaunchKernelGGL(kernel, dim3((unsigned)all), block, 0, (hipStream_t)stream, a, e, sh, (int)blocks, (int)grid.x, (int)experts.x); \
             }                                                                                                                                 \

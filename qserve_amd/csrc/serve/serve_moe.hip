@@ -452,7 +452,7 @@ static int launch_expert_rows(const char* what, ExpertArgs a, int n_experts, int
     const int rc = plan_expert_rows(what, a, sh, n_experts, act, kept, grid);
     if (rc != QSV_OK) return rc;
     const dim3 block(NT);
-    const bool early = early_experts(a, sh, n_experts);
+    const bool early = early_experts(a, n_experts);
 #define QSV_EXPERTS(ACT, FOUT)                                                                                                                          \
     do {                                                                                                                                                \
         auto kernel = a.offsets ? expert_rows_kernel<ACT, FOUT, SORTED_RUNS> : early ? expert_rows_kernel<ACT, FOUT, SLOTS_EARLY>                       \

@@ -276,9 +276,9 @@ __device__ __forceinline__ void expert_rows_block(const ExpertArgs& a, const Sha
 }
 
 // Whether the weights are requested before the slots are looked for, of a launch that plan_expert_rows has passed.  Measured, 16 experts, 16 / 24 slots each, out of memory, us: 1024 x
-// 2048 16.7 -> 15.7, 17.7 -> 16.8, 1408 x 2048 21.6 -> 21.0, 23.1 -> 21.9, 2048 x 1408 19.4 -> 18.8, 21.3 -> 20.5, 2816 x 2048 37.9 -> 36.3, 40.1 -> 38.7, 5632 x 2048 69.3 -> 68.4,
-// 73.8 -> 72.2.  The first requests of an expert that no slot has are for nothing (a quarter of its weights): steps of 4 tokens, top 4 of 16, took 4 % longer, so four
-// slots an expert on average, of which one expert in 50 has none.
+// 2048 16.7 -> 15.4, 17.7 -> 16.7, 1408 x 2048 21.6 -> 19.9, 23.1 -> 21.6, 2048 x 1408 19.4 -> 18.1, 21.3 -> 20.1, 2816 x 2048 37.9 -> 35.7, 40.1 -> 38.2, 5632 x 2048 69.3 -> 67.8,
+// 73.8 -> 72.7; steps of 32 and 64 sequences (Vekalorn, 20 and their prompts) 9202 -> 8924, 10741 -> 10446.  The first requests of an expert that no slot has are for nothing (a
+// quarter of its weights): steps of 4 tokens, top 4 of 16, took 4 % longer, so four slots an expert on average, of which one expert in 50 has none.
 inline bool early_experts(const ExpertArgs& a, int n_experts) {
     return a.idx && !a.by_slot && a.n <= XLIST && a.n >= 4 * n_experts && a.K >= EARLY_MIN;
 }

@@ -455,11 +455,11 @@ static int launch_expert_rows(const char* what, ExpertArgs a, int n_experts, int
     const bool early = early_experts(a, n_experts);
 #define QSV_EXPERTS(ACT, FOUT)                                                                                                                          \
     do {                                                                                                                                                \
-        auto kernel = a.offsets ? expert_rows_kernel<ACT, FOUT, SORTED_RUNS> : early ? expert_rows_kernel<ACT, FOUT, SLOTS_EARLY>                       \
-                                             : few_slots(a, sh) ? expert_rows_kernel<ACT, FOUT, SLOTS_FEW> : expert_rows_kernel<ACT, FOUT, SLOTS>;      \
+        auto kernel = early ? expert_rows_kernel<ACT, FOUT, SLOTS_EARLY> : few_slots(a, sh) ? expert_rows_kernel<ACT, FOUT, SLOTS_FEW> : expert_rows_kernel<ACT, FOUT, SLOTS>; \
+        if constexpr (!FOUT) kernel = a.offsets ? expert_rows_kernel<ACT, FOUT, SORTED_RUNS> : kernel;                                                  \
         hipLaunchKernelGGL(kernel, grid, block, 0, (hipStream_t)stream, a, sh);                                                                         \
     } while (0)
-    if (float_out) QSV_EXPERTS(ACT_NONE, true);                                    // (sorted runs: never)
+    if (float_out) QSV_EXPERTS(ACT_NONE, true);                                    // (never sorted runs)
     else if (act == ACT_RELU_SQ) QSV_EXPERTS(ACT_RELU_SQ, false);
     else if (act == ACT_GLU) QSV_EXPERTS(ACT_GLU, false);
     else QSV_EXPERTS(ACT_NONE, false);

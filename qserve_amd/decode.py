@@ -348,8 +348,9 @@ class DecodeEngine:
             tokens = torch.randint(0, cfg["vocab"], (T,), device=dev,
                                    generator=torch.Generator(device=dev).manual_seed(7))
         # the first norm's input straight from the table, the last one for the rows that are sampled from only
-        # (8 x 1024 x 4096 without the layers: 133 us as eleven launches of torch's and ours, 48 as three; other token tensors than a whole int64 one take torch's lookup)
-        ends = (fuse and dev.type == "cuda" and self.hid % 8 == 0 and self.hid <= 8192 and not (fuse_sum and _lib.qs_get_row_sum_order())
+        # (8 x 1024 x 4096 without the layers: 133 us as eleven launches of torch's and ours, 48 as three; other token tensors than a whole int64 one take torch's lookup,
+        # and so does an engine without layers: the first norm is its first layer's)
+        ends = (fuse and len(self.layers) > 0 and dev.type == "cuda" and self.hid % 8 == 0 and self.hid <= 8192 and not (fuse_sum and _lib.qs_get_row_sum_order())
                 and tokens.dtype == torch.int64 and tokens.device == self.embed.device and tokens.shape == (T,) and tokens.is_contiguous())
         h = torch.empty((T, self.hid), dtype=f16, device=dev) if ends else torch.index_select(self.embed, 0, tokens)
         qa = torch.empty((T, self.hid), dtype=i8, device=dev)

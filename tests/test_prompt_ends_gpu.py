@@ -80,3 +80,19 @@ def test_prompt_phase(group, int4_kv):
     ref.prefill(70, tokens.to(torch.int32))             # (torch's lookup: the general path)
     assert torch.equal(eng.hidden, ref.hidden) and torch.equal(eng.lengths, ref.lengths)
     assert ((eng.final.float() - ref.final.float()).abs() <= 2.0 ** -10 * ref.final.float().abs()).all()
+
+
+def test_an_engine_without_layers():
+    """Embedding, norm and head alone: no layer's norm reads the table on the way."""
+    from qserve_backend import layernorm_ops
+    g = _gen(7)
+    cfg = dict(D.LLAMA3_8B, layers=0, vocab=512)
+    eng = D.DecodeEngine(cfg, 3, 70, 4, seed=5)
+    tokens = torch.randint(0, 512, (3 * 70,), device="cuda", generator=g)
+    eng.prefill(70, tokens)
+    rows = eng.embed[tokens.view(3, 70)[:, -1]]
+    ref = torch.empty_like(rows)
+    layernorm_ops.rms_norm(ref, rows, eng.norm_w, cfg["eps"])
+    assert torch.equal(eng.hidden, rows) and torch.equal(eng.final, ref) and eng.lengths.tolist() == [71] * 3
+    logits = torch.matmul(ref, eng.lm_head.t())
+    assert torch.equal(logits.gather(1, eng.tokens[:, None])[:, 0], logits.amax(1))

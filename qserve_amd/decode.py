@@ -38,6 +38,11 @@ def residual_add_(a, b):
     """a += b (fp16), the residual add the reference does with a torch add (llama_w4a8_unpad.py:348,360)."""
     _check(_lib.qs_residual_add(a.data_ptr(), b.data_ptr(), a.numel(), stream()), "residual_add")
 
+def _start_on(n, *tensors):
+    """Whether every tensor that there is starts on n bytes: a view into a checkpoint's one buffer need not."""
+    return all(t is None or t.data_ptr() % n == 0 for t in tensors)
+
+
 def argmax_rows_(logits, out):
     """out[r] = argmax(logits[r]) (fp16 [rows, n] -> int64 [rows]); the greedy sampler of the benchmark step."""
     assert logits.dtype == torch.float16 and logits.dim() == 2 and logits.stride(1) == 1 and out.dtype == torch.int64
@@ -255,9 +260,11 @@ class DecodeEngine:
                 ks = {layer[name].planes_slices(B) for layer in self.layers}
                 if len(ks) == 1 and 0 not in ks:
                     self.planes[name] = torch.empty((ks.pop(), B, hid), dtype=torch.int32, device=self.dev)
-        # the norm behind the last layer from down's planes: the product's own epilogue, the add and the norm took three launches
-        self.last_planes = chosen and "down" in self.planes
-        self._choose_rows(chosen)
+        # the norm behind the last layer from down's planes: the product's own epilogue, the add and the norm took three launches (which take gains that start
+        # anywhere and scales on 4 bytes)
+        last = self.layers[-1]["down"] if self.layers else None
+        self.last_planes = chosen and "down" in self.planes and _start_on(16, self.norm_w, last.s1_scales, getattr(last, "s1_szeros", None))
+        self._choose_rows()
         self.lengths = torch.full((B,), prompt_len, dtype=torch.int32, device=self.dev)   # context incl. new token
         self.tokens = torch.randint(0, cfg["vocab"], (B,), device=self.dev, generator=gen)
         # Tensor parallel: the (un-quantised) lm_head is cut over the vocabulary - rank r multiplies rows [v0, v0 + V/N)
@@ -278,7 +285,7 @@ class DecodeEngine:
         self.graph = None
         self.pieces = None
 
-    def _choose_rows(self, chosen):
+    def _choose_rows(self):
         """Which products of a step of few sequences run through the launches that read their weights straight into registers (fused.rows_planes), with the row operation
         in front of them inside.  Both sides measured for every line, launches replaced / replacing, us (Llama-3-8B's and Llama-2-7B's products, per-channel):
         * `o` behind the attention, up to 4 rows, two slices: 4.7 / 3.5, 3.7, 4.3, 4.3 (groups of 128: 5.7 / 4.0, 4.4, 5.1, 5.0);
@@ -292,9 +299,15 @@ class DecodeEngine:
         B, hid, inter = self.B, self.hid, self.inter
         group = self.group_size != -1
         self.rows = set()
-        if not (chosen and B <= 4 and hid == 4096 and set(self.planes) == {"o", "down"} and len(self.layers)
-                and fusedmod.rows_ok(B, hid, self.H * 128, 2, group)):
+        # (without the last norm from planes the last product would look for rows and a stream that these launches keep elsewhere)
+        if not (self.last_planes and B <= 4 and hid == 4096 and set(self.planes) == {"o", "down"} and fusedmod.rows_ok(B, hid, self.H * 128, 2, group)):
             return
+        # (the launches replaced take gains that start anywhere)
+        for L in self.layers:
+            lins = [L[n] for n in ("qkv", "o", "gate_up", "down")]
+            if not (_start_on(16, L["ln1"], L["ln2"], *(x.qweight for x in lins), *(t for x in (L["o"], L["down"]) for t in (x.s1_scales, getattr(x, "s1_szeros", None))))
+                    and _start_on(4, *(getattr(x, n, None) for x in lins for n in ("s2_zeros", "s2_scales")))):
+                return
         self.rows.add("o")
         self.rows_planes = {"o": torch.empty((2, B, hid), dtype=torch.int32, device=self.dev)}      # (in their own numbers of slices)
         plain = all(L[n].bias is None for L in self.layers for n in ("qkv", "gate_up"))
@@ -349,9 +362,10 @@ class DecodeEngine:
                                    generator=torch.Generator(device=dev).manual_seed(7))
         # the first norm's input straight from the table, the last one for the rows that are sampled from only
         # (8 x 1024 x 4096 without the layers: 133 us as eleven launches of torch's and ours, 48 as three; other token tensors than a whole int64 one take torch's lookup,
-        # and so does an engine without layers: the first norm is its first layer's)
+        # and so do an engine without layers, whose first norm that is, tables with gaps between their rows, and tables and gains that do not start on 16 bytes)
         ends = (fuse and len(self.layers) > 0 and dev.type == "cuda" and self.hid % 8 == 0 and self.hid <= 8192 and not (fuse_sum and _lib.qs_get_row_sum_order())
-                and tokens.dtype == torch.int64 and tokens.device == self.embed.device and tokens.shape == (T,) and tokens.is_contiguous())
+                and tokens.dtype == torch.int64 and tokens.device == self.embed.device and tokens.shape == (T,) and tokens.is_contiguous()
+                and self.embed.is_contiguous() and _start_on(16, self.embed, self.layers[0]["ln1"], self.norm_w))
         h = torch.empty((T, self.hid), dtype=f16, device=dev) if ends else torch.index_select(self.embed, 0, tokens)
         qa = torch.empty((T, self.hid), dtype=i8, device=dev)
         qo = torch.empty((T, self.H * 128), dtype=i8, device=dev)

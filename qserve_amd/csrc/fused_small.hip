@@ -92,28 +92,33 @@ __global__ __launch_bounds__(TPB) void general_norm_quant_kernel(int8_t* __restr
 }
 
 // ---------------------------------------------------------------------------------------------------------
+// What every fp16 norm of this file does to eight values, written once so that each kernel gives the same bits: the product of two fp16 values is exact in float, so a
+// sum of squares is the same with its additions fused or not, and the scaled value is a float of its own before it is fp16 (in one operation it would be rounded once).
+__device__ __forceinline__ float add_squares8(const h8& v, float s) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) s = fmaf((float)v[j], (float)v[j], s);
+    return s;
+}
+__device__ __forceinline__ h8 rms_scaled8(const h8& v, const h8& g, float rstd) {
+    h8 o;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        float r = (float)v[j] * rstd;
+        asm("" : "+v"(r));
+        const _Float16 t = (_Float16)r;                                  // (scalar_t)(x * s_variance), :358
+        o[j] = (_Float16)((float)t * (float)g[j]);                       // half * half
+    }
+    return o;
+}
 __global__ __launch_bounds__(TPB) void rms_norm_kernel(_Float16* __restrict__ out, const _Float16* __restrict__ in,
                                                        const _Float16* __restrict__ w, float eps, int hidden) {
     __shared__ float sm[TPB / 64];
     const size_t base = (size_t)blockIdx.x * hidden;
     float vs = 0.f;
-    for (int i = threadIdx.x * 8; i < hidden; i += TPB * 8) {
-        h8 v = load8(in + base + i);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) vs += (float)v[j] * (float)v[j];
-    }
+    for (int i = threadIdx.x * 8; i < hidden; i += TPB * 8) vs = add_squares8(load8(in + base + i), vs);
     const float rstd = 1.0f / sqrtf(block_reduce_once(vs, sm, 0) / hidden + eps);   // :347
-    for (int i = threadIdx.x * 8; i < hidden; i += TPB * 8) {
-        h8 v = load8(in + base + i);
-        h8 g = load8(w + i);
-        h8 o;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            _Float16 t = (_Float16)((float)v[j] * rstd);                 // (scalar_t)(x * s_variance), :358
-            o[j] = (_Float16)((float)t * (float)g[j]);                   // half * half
-        }
-        *reinterpret_cast<h8*>(out + base + i) = o;
-    }
+    for (int i = threadIdx.x * 8; i < hidden; i += TPB * 8)
+        *reinterpret_cast<h8*>(out + base + i) = rms_scaled8(load8(in + base + i), load8(w + i), rstd);
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -207,22 +212,14 @@ __device__ __forceinline__ void add_rms_norm_row(_Float16* __restrict__ out, con
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
         v[c] = v[c] + __builtin_bit_cast(h8, dfn.finish(raw[c]));
-        if ((c * TPB + (int)threadIdx.x) * 8 >= width) continue;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) vs += (float)v[c][j] * (float)v[c][j];
+        if ((c * TPB + (int)threadIdx.x) * 8 < width) vs = add_squares8(v[c], vs);
     }
     const float rstd = 1.0f / sqrtf(block_reduce_once(vs, sm, 0) / width + eps);
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
         const int i = (c * TPB + (int)threadIdx.x) * 8;
         if (i >= width) continue;
-        h8 o;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const _Float16 t = (_Float16)((float)v[c][j] * rstd);
-            o[j] = (_Float16)((float)t * (float)g[c][j]);
-        }
-        *reinterpret_cast<h8*>(out + i) = o;
+        *reinterpret_cast<h8*>(out + i) = rms_scaled8(v[c], g[c], rstd);
         *reinterpret_cast<h8*>(hidden_out + i) = v[c];
     }
 }

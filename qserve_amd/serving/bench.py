@@ -78,32 +78,42 @@ def random_weights(cfg, dev, seed=0):
 class OpTimer:
     """HIP events around every call of the ops object's methods (one step at a time)."""
     NAMES = ("embed", "add_layer_norm", "layer_norm_rows", "latent_prep", "latent_up", "latent_queries", "latent_prompt", "head_products", "latent_attention", "sigmoid_gate",
-             "moe_route", "moe_experts", "moe_experts_shared", "embed_streams", "hc_read", "hc_write", "dyt_sum_rows", "rms_pair_mean", "glu",
-             "attention_prep", "rotate_heads", "decay", "decay_products", "conv_silu_unit", "recurrent_scan", "head_rms_gate", "embed_sinusoid",
+             "moe_route", "moe_experts", "moe_experts_shared", "embed_streams", "hc_read", "hc_write", "hc_write_read", "dyt_sum_rows", "rms_pair_mean", "glu",
+             "attention_prep", "rotate_heads", "decay", "decay_products", "conv_silu_unit", "recurrent_scan", "recurrent_gated", "head_rms_gate", "embed_sinusoid",
              "add_rms_norm", "rms_norm_rows", "normed_attention_prep", "max_gates", "add_normed_rms_norm", "qk_norm_rope_prep", "pool_blocks",
              "min_gru_scan", "relu_sq", "embed_rms_norm", "residual_conv", "scaled_add_rms_norm", "rotate_qk", "talking_attention",
              "scaled_sum_rms_norms", "scaled_sum_rms_norms_product", "conv_heads_cache", "diff_attention", "single_map_attention", "linear", "float_linear")
-    # another form of the same operation: its time is that operation's
-    FORMS = {"latent_prompt": "latent_attention", "moe_experts_shared": "moe_experts", "float_linear": "linear"}
+    # another form of the same operation: its time is that operation's (a step's recurrence with its read-out normed and gated is the recurrence's launch)
+    FORMS = {"latent_prompt": "latent_attention", "moe_experts_shared": "moe_experts", "float_linear": "linear", "recurrent_gated": "recurrent_scan"}
+    # operations that call others of NAMES, and launch nothing themselves, where their own launch does not take the call: the others count then
+    HAND_OVER = ("add_layer_norm", "hc_write", "hc_write_read", "scaled_sum_rms_norms", "recurrent_gated")
+    # methods that models call and that launch nothing of their own
+    HOST = ("latent_prompt_plan", "maps_attention_ok", "moe_experts_pending")
 
     def __init__(self, ops):
         self.ops, self.events, self.calls, self.on = ops, [], [], False
         for n in self.NAMES:
-            setattr(ops, n, self._wrap(self.FORMS.get(n, n), getattr(ops, n)))
+            setattr(ops, n, self._wrap(self.FORMS.get(n, n), getattr(ops, n), n in self.HAND_OVER))
+        # a step whose operations are timed makes each of them apart: experts that ride in other operations' launches would count as those
+        pending = ops.moe_experts_pending
+        ops.moe_experts_pending = lambda *a, **k: None if self.on else pending(*a, **k)
 
     @staticmethod
     def _linear_users():
         """Modules whose products are not the ops object's: none (layers and models call its `linear` and `float_linear`)."""
         return []
 
-    def _wrap(self, name, fn):
+    def _wrap(self, name, fn, hands_over=False):
         def timed(*a, **k):
             if not self.on:
                 return fn(*a, **k)
+            before = len(self.events)
             e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             e0.record()
             r = fn(*a, **k)
             e1.record()
+            if hands_over and len(self.events) > before:
+                return r
             self.events.append((name, e0, e1))
             self.calls.append((name, fn, a, k))
             return r
@@ -126,8 +136,13 @@ class OpTimer:
             total += e0.elapsed_time(e1) / reps
         return total
 
+    def replays(self, names, reps):
+        """{name: replay} of those that the last step() ran."""
+        ran = {n for n, *_ in self.calls}
+        return {n: self.replay(n, reps) for n in names if n in ran}
+
     def step(self, fn):
-        """Run fn() with timing on -> ({op: ms summed over its launches}, total ms between first and last event)."""
+        """Run fn() with timing on, every operation in launches of its own -> ({op: ms summed over its launches}, total ms between first and last event)."""
         self.events, self.calls, self.on = [], [], True
         t0, t1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
         t0.record()
@@ -139,6 +154,16 @@ class OpTimer:
         for n, e0, e1 in self.events:
             out[n] = out.get(n, 0.0) + e0.elapsed_time(e1)
         return out, t0.elapsed_time(t1)
+
+
+def _rate(work, per, times, *ops):
+    """work in units of `per` a second over these operations' times (ms); None where the step ran none of them."""
+    ms = sum(times.get(n, 0.0) for n in ops)
+    return work / (ms * 1e-3) / per if ms else None
+
+
+def _of(rate, peak):
+    return None if rate is None else rate / peak
 
 
 def timed(fn, steps, warmup):
@@ -219,7 +244,7 @@ def bench_vekalorn(name, s, dev, steps, warmup):
     by = sum(NB * (min(ctx, s["window"]) if k == "latent_attention" else ctx) * rows[k] * 2.0 for k in kinds)
     att_dec = by / (att_dec_ms * 1e-3) / 1e9
     moe_flops = LAYERS * T * s["top"] * 2 * 2.0 * s["ff"] * s["width"]
-    moe_pre = moe_flops / (ops_pre["moe_experts"] * 1e-3) / 1e12
+    moe_pre = _rate(moe_flops, 1e12, ops_pre, "moe_experts")
     moe_bytes = LAYERS * min(s["experts"], NB * s["top"]) * 2 * s["ff"] * s["width"] * 2.0
     moe_dec = moe_bytes / (moe_dec_ms * 1e-3) / 1e9
     out = dict(model=f"Vekalorn-{name}", prefill_tokens_per_s=T / pre * 1e3, prefill_ms=pre, decode_tokens_per_s=NB / dec * 1e3,
@@ -227,10 +252,10 @@ def bench_vekalorn(name, s, dev, steps, warmup):
                decode_ms_gpu_events=dec_events_ms, decode_experts_kernels_ms=moe_dec_ms, context=ctx,
                prefill_ops_ms=ops_pre, decode_ops_ms=ops_dec, prefill_attention_kernels_ms=att_pre_ms,
                decode_attention_kernels_ms=att_dec_ms,
-               roofline=dict(prefill_attention_tflops=att_pre, prefill_attention_frac_bf16_peak=att_pre / BF16_PEAK_TFLOPS,
-                             decode_attention_gbs=att_dec, decode_attention_frac_hbm=att_dec / HBM_PEAK_GBS,
-                             prefill_experts_tflops=moe_pre, prefill_experts_frac_bf16_peak=moe_pre / BF16_PEAK_TFLOPS,
-                             decode_experts_gbs=moe_dec, decode_experts_frac_hbm=moe_dec / HBM_PEAK_GBS))
+               roofline=dict(prefill_attention_tflops=att_pre, prefill_attention_frac_bf16_peak=_of(att_pre, BF16_PEAK_TFLOPS),
+                             decode_attention_gbs=att_dec, decode_attention_frac_hbm=_of(att_dec, HBM_PEAK_GBS),
+                             prefill_experts_tflops=moe_pre, prefill_experts_frac_bf16_peak=_of(moe_pre, BF16_PEAK_TFLOPS),
+                             decode_experts_gbs=moe_dec, decode_experts_frac_hbm=_of(moe_dec, HBM_PEAK_GBS)))
     for sl in slots:
         eng.close_sequence(sl)
     del eng
@@ -351,8 +376,7 @@ def bench_mumelix(name, s, dev, steps, warmup):
         want = [k * L + L - 1 for k in range(BP)]
         if i == BP:                                          # one step with events around every launch
             ops_pre, _ = timer.step(lambda: eng.execute(items, want))
-            rep_pre = {k: timer.replay(k, 3) for k in ("latent_attention", "hc_read", "hc_write", "attention_prep", "conv_silu_unit", "head_rms_gate",
-                                                      "rms_pair_mean")}
+            rep_pre = timer.replays(("latent_attention", "hc_read", "hc_write", "attention_prep", "conv_silu_unit", "head_rms_gate", "rms_pair_mean"), 3)
             continue
         torch.cuda.synchronize()
         t0 = time.perf_counter()
@@ -369,7 +393,7 @@ def bench_mumelix(name, s, dev, steps, warmup):
 
     dec_eager = timed(decode, steps, warmup)
     ops_dec, dec_events_ms = timer.step(decode)
-    rep_dec = {k: timer.replay(k, 20) for k in ("latent_attention", "moe_experts", "hc_read", "hc_write")}
+    rep_dec = timer.replays(("latent_attention", "moe_experts", "hc_read", "hc_write", "hc_write_read"), 20)
     eng.decode_graphs = True
     dec = timed(decode, steps, warmup)
     graph_ok = any(v is not False for v in eng._graphs.values()) and bool(eng._graphs)
@@ -380,30 +404,30 @@ def bench_mumelix(name, s, dev, steps, warmup):
     R = m["a_dim"] + m["a_vdim"]
     # attention: useful work = q.k over dim and p.v over vdim (the kernel also multiplies the query's zero half)
     att_flops = n_att * BP * sum(p + 1 for p in range(L)) * m["a_heads"] * (m["a_dim"] + m["a_vdim"]) * 2.0
-    att_pre = att_flops / (rep_pre["latent_attention"] * 1e-3) / 1e12
+    att_pre = _rate(att_flops, 1e12, rep_pre, "latent_attention")
     att_bytes = n_att * NB * ctx * m["a_kv"] * R * 2.0
-    att_dec = att_bytes / (rep_dec["latent_attention"] * 1e-3) / 1e9
+    att_dec = _rate(att_bytes, 1e9, rep_dec, "latent_attention")
     # recurrences: 5 (gated linear attention) / 7 (delta rule) float operations per state element and token; decoding moves the state twice
     el = n_gla * m["g_heads"] * m["g_dim"] * m["g_vdim"], n_att * m["d_heads"] * m["d_dim"] * m["d_vdim"]
-    scan_pre = T * (5.0 * el[0] + 7.0 * el[1]) / (ops_pre["recurrent_scan"] * 1e-3) / 1e12
-    scan_dec = NB * (el[0] + el[1]) * 4.0 * 2 / (ops_dec["recurrent_scan"] * 1e-3) / 1e9
+    scan_pre = _rate(T * (5.0 * el[0] + 7.0 * el[1]), 1e12, ops_pre, "recurrent_scan")
+    scan_dec = _rate(NB * (el[0] + el[1]) * 4.0 * 2, 1e9, ops_dec, "recurrent_scan")
     moe_flops = LAYERS * T * s["top"] * 3 * 2.0 * s["ff"] * D
-    moe_pre = moe_flops / (ops_pre["moe_experts"] * 1e-3) / 1e12
+    moe_pre = _rate(moe_flops, 1e12, ops_pre, "moe_experts")
     moe_bytes = LAYERS * min(s["experts"], NB * s["top"]) * 3 * s["ff"] * D * 2.0
-    moe_dec = moe_bytes / (rep_dec["moe_experts"] * 1e-3) / 1e9
+    moe_dec = _rate(moe_bytes, 1e9, rep_dec, "moe_experts")
     # stream kernels: read S streams per sublayer, rewrite S streams (read + write) per sublayer, float
     hc_bytes = LAYERS * 2 * (S * D * 4.0 + D * 2.0) + LAYERS * 2 * (2 * S * D * 4.0 + D * 2.0)
-    hc_pre = T * hc_bytes / ((rep_pre["hc_read"] + rep_pre["hc_write"]) * 1e-3) / 1e9
+    hc_pre = _rate(T * hc_bytes, 1e9, rep_pre, "hc_read", "hc_write")
     out = dict(model=f"Mumelix-{name}", sizes=m, prefill_tokens_per_s=T / pre * 1e3, prefill_ms=pre, decode_tokens_per_s=NB / dec * 1e3,
                decode_ms=dec, decode_from_hipgraph=graph_ok, decode_ms_eager=dec_eager, decode_ms_gpu_events=dec_events_ms, context=ctx,
                prefill_ops_ms=ops_pre, decode_ops_ms=ops_dec, prefill_kernels_ms=rep_pre, decode_kernels_ms=rep_dec,
-               roofline=dict(prefill_attention_tflops=att_pre, prefill_attention_frac_bf16_peak=att_pre / BF16_PEAK_TFLOPS,
-                             decode_attention_gbs=att_dec, decode_attention_frac_hbm=att_dec / HBM_PEAK_GBS,
-                             prefill_experts_tflops=moe_pre, prefill_experts_frac_bf16_peak=moe_pre / BF16_PEAK_TFLOPS,
-                             decode_experts_gbs=moe_dec, decode_experts_frac_hbm=moe_dec / HBM_PEAK_GBS,
-                             prefill_recurrence_tflops=scan_pre, prefill_recurrence_frac_fp32_valu_peak=scan_pre / FP32_VALU_PEAK_TFLOPS,
-                             decode_recurrence_gbs=scan_dec, decode_recurrence_frac_hbm=scan_dec / HBM_PEAK_GBS,
-                             prefill_stream_kernels_gbs=hc_pre, prefill_stream_kernels_frac_hbm=hc_pre / HBM_PEAK_GBS))
+               roofline=dict(prefill_attention_tflops=att_pre, prefill_attention_frac_bf16_peak=_of(att_pre, BF16_PEAK_TFLOPS),
+                             decode_attention_gbs=att_dec, decode_attention_frac_hbm=_of(att_dec, HBM_PEAK_GBS),
+                             prefill_experts_tflops=moe_pre, prefill_experts_frac_bf16_peak=_of(moe_pre, BF16_PEAK_TFLOPS),
+                             decode_experts_gbs=moe_dec, decode_experts_frac_hbm=_of(moe_dec, HBM_PEAK_GBS),
+                             prefill_recurrence_tflops=scan_pre, prefill_recurrence_frac_fp32_valu_peak=_of(scan_pre, FP32_VALU_PEAK_TFLOPS),
+                             decode_recurrence_gbs=scan_dec, decode_recurrence_frac_hbm=_of(scan_dec, HBM_PEAK_GBS),
+                             prefill_stream_kernels_gbs=hc_pre, prefill_stream_kernels_frac_hbm=_of(hc_pre, HBM_PEAK_GBS)))
     for sl in slots:
         eng.close_sequence(sl)
     del eng
@@ -481,7 +505,7 @@ def bench_vepolix(name, s, dev, steps, warmup):
         want = [k * L + L - 1 for k in range(BP)]
         if i == BP:                                          # one step with events around every launch
             ops_pre, _ = timer.step(lambda: eng.execute(items, want))
-            rep_pre = {k: timer.replay(k, 3) for k in small if k != "recurrent_scan" and k != "max_gates"}   # (these two advance state)
+            rep_pre = timer.replays([k for k in small if k != "recurrent_scan" and k != "max_gates"], 3)   # (these two advance state)
             continue
         torch.cuda.synchronize()
         t0 = time.perf_counter()
@@ -498,7 +522,7 @@ def bench_vepolix(name, s, dev, steps, warmup):
 
     dec_eager = timed(decode, steps, warmup)
     ops_dec, dec_events_ms = timer.step(decode)
-    rep_dec = {k: timer.replay(k, 20) for k in ("latent_attention", "moe_experts", "add_rms_norm", "normed_attention_prep", "head_rms_gate")}
+    rep_dec = timer.replays(("latent_attention", "moe_experts", "add_rms_norm", "normed_attention_prep", "head_rms_gate"), 20)
     eng.decode_graphs = True
     dec = timed(decode, steps, warmup)
     graph_ok = any(v is not False for v in eng._graphs.values()) and bool(eng._graphs)
@@ -508,35 +532,35 @@ def bench_vepolix(name, s, dev, steps, warmup):
     n_rec = LAYERS - n_att
     R = m["a_dim"] + m["a_vdim"]
     att_flops = n_att * BP * sum(p + 1 for p in range(L)) * m["a_heads"] * (m["a_dim"] + m["a_vdim"]) * 2.0
-    att_pre = att_flops / (rep_pre["latent_attention"] * 1e-3) / 1e12
+    att_pre = _rate(att_flops, 1e12, rep_pre, "latent_attention")
     att_bytes = n_att * NB * ctx * m["a_kv"] * R * 2.0
-    att_dec = att_bytes / (rep_dec["latent_attention"] * 1e-3) / 1e9
+    att_dec = _rate(att_bytes, 1e9, rep_dec, "latent_attention")
     # recurrence: 5 float operations per state element and token (decay, k v, add; q S, add); decoding moves the state twice
     el = n_rec * m["g_heads"] * m["g_dim"] * m["g_vdim"]
-    scan_pre = T * 5.0 * el / (ops_pre["recurrent_scan"] * 1e-3) / 1e12
-    scan_dec = NB * el * 4.0 * 2 / (ops_dec["recurrent_scan"] * 1e-3) / 1e9
+    scan_pre = _rate(T * 5.0 * el, 1e12, ops_pre, "recurrent_scan")
+    scan_dec = _rate(NB * el * 4.0 * 2, 1e9, ops_dec, "recurrent_scan")
     moe_flops = n_rec * T * s["top"] * 3 * 2.0 * s["ff"] * D
-    moe_pre = moe_flops / (ops_pre["moe_experts"] * 1e-3) / 1e12
+    moe_pre = _rate(moe_flops, 1e12, ops_pre, "moe_experts")
     moe_bytes = n_rec * min(s["experts"], NB * s["top"]) * 3 * s["ff"] * D * 2.0
-    moe_dec = moe_bytes / (rep_dec["moe_experts"] * 1e-3) / 1e9
+    moe_dec = _rate(moe_bytes, 1e9, rep_dec, "moe_experts")
     # residual kernel: reads and writes the float stream, reads the sublayers' outputs (2 on attention layers, 3 on the others),
     # writes the next input; the first call only norms, the last only adds
     res_bytes = T * (LAYERS * (8.0 * D + 2.0 * D) + (2 * n_att + 3 * n_rec) * 2.0 * D)
-    res_pre = res_bytes / (rep_pre["add_rms_norm"] * 1e-3) / 1e9
+    res_pre = _rate(res_bytes, 1e9, rep_pre, "add_rms_norm")
     # query / key preparation: the projections in, queries (storage type) and cache rows out
     prep_bytes = n_att * T * 2.0 * (2 * m["a_heads"] * m["a_dim"] + 2 * m["a_kv"] * R)
-    prep_pre = prep_bytes / (rep_pre["normed_attention_prep"] * 1e-3) / 1e9
+    prep_pre = _rate(prep_bytes, 1e9, rep_pre, "normed_attention_prep")
     out = dict(model=f"Vepolix-{name}", sizes=m, prefill_tokens_per_s=T / pre * 1e3, prefill_ms=pre, decode_tokens_per_s=NB / dec * 1e3,
                decode_ms=dec, decode_from_hipgraph=graph_ok, decode_ms_eager=dec_eager, decode_ms_gpu_events=dec_events_ms, context=ctx,
                prefill_ops_ms=ops_pre, decode_ops_ms=ops_dec, prefill_kernels_ms=rep_pre, decode_kernels_ms=rep_dec,
-               roofline=dict(prefill_attention_tflops=att_pre, prefill_attention_frac_bf16_peak=att_pre / BF16_PEAK_TFLOPS,
-                             decode_attention_gbs=att_dec, decode_attention_frac_hbm=att_dec / HBM_PEAK_GBS,
-                             prefill_experts_tflops=moe_pre, prefill_experts_frac_bf16_peak=moe_pre / BF16_PEAK_TFLOPS,
-                             decode_experts_gbs=moe_dec, decode_experts_frac_hbm=moe_dec / HBM_PEAK_GBS,
-                             prefill_recurrence_tflops=scan_pre, prefill_recurrence_frac_fp32_valu_peak=scan_pre / FP32_VALU_PEAK_TFLOPS,
-                             decode_recurrence_gbs=scan_dec, decode_recurrence_frac_hbm=scan_dec / HBM_PEAK_GBS,
-                             prefill_prep_gbs=prep_pre, prefill_prep_frac_hbm=prep_pre / HBM_PEAK_GBS,
-                             prefill_residual_kernel_gbs=res_pre, prefill_residual_kernel_frac_hbm=res_pre / HBM_PEAK_GBS))
+               roofline=dict(prefill_attention_tflops=att_pre, prefill_attention_frac_bf16_peak=_of(att_pre, BF16_PEAK_TFLOPS),
+                             decode_attention_gbs=att_dec, decode_attention_frac_hbm=_of(att_dec, HBM_PEAK_GBS),
+                             prefill_experts_tflops=moe_pre, prefill_experts_frac_bf16_peak=_of(moe_pre, BF16_PEAK_TFLOPS),
+                             decode_experts_gbs=moe_dec, decode_experts_frac_hbm=_of(moe_dec, HBM_PEAK_GBS),
+                             prefill_recurrence_tflops=scan_pre, prefill_recurrence_frac_fp32_valu_peak=_of(scan_pre, FP32_VALU_PEAK_TFLOPS),
+                             decode_recurrence_gbs=scan_dec, decode_recurrence_frac_hbm=_of(scan_dec, HBM_PEAK_GBS),
+                             prefill_prep_gbs=prep_pre, prefill_prep_frac_hbm=_of(prep_pre, HBM_PEAK_GBS),
+                             prefill_residual_kernel_gbs=res_pre, prefill_residual_kernel_frac_hbm=_of(res_pre, HBM_PEAK_GBS)))
     for sl in slots:
         eng.close_sequence(sl)
     del eng
@@ -626,7 +650,7 @@ def bench_pemolorn(name, s, dev, steps, warmup):
         want = [k * L + L - 1 for k in range(BP)]
         if i == BP:                                          # one step with events around every launch
             ops_pre, _ = timer.step(lambda: eng.execute(items, want))
-            rep_pre = {k: timer.replay(k, 3) for k in stateless}      # (the scan and the convolution advance state: timed in the step)
+            rep_pre = timer.replays(stateless, 3)      # (the scan and the convolution advance state: timed in the step)
             continue
         torch.cuda.synchronize()
         t0 = time.perf_counter()
@@ -643,7 +667,7 @@ def bench_pemolorn(name, s, dev, steps, warmup):
 
     dec_eager = timed(decode, steps, warmup)
     ops_dec, dec_events_ms = timer.step(decode)
-    rep_dec = {k: timer.replay(k, 20) for k in ("latent_attention", "moe_experts", "add_normed_rms_norm", "qk_norm_rope_prep")}
+    rep_dec = timer.replays(("latent_attention", "moe_experts", "add_normed_rms_norm", "qk_norm_rope_prep"), 20)
     eng.decode_graphs = True
     dec = timed(decode, steps, warmup)
     graph_ok = any(v is not False for v in eng._graphs.values()) and bool(eng._graphs)
@@ -660,31 +684,31 @@ def bench_pemolorn(name, s, dev, steps, warmup):
 
     # attention: useful work = q.k over dim and p.v over vdim for every visible key (the kernel also multiplies the query's zero half)
     att_flops = sum(BP * sum(seen(p, k) for p in range(L)) for k in kinds) * m["a_heads"] * R * 2.0
-    att_pre = att_flops / (rep_pre["latent_attention"] * 1e-3) / 1e12
+    att_pre = _rate(att_flops, 1e12, rep_pre, "latent_attention")
     att_bytes = sum(NB * seen(ctx - 1, k) for k in kinds) * m["a_kv"] * R * 2.0
-    att_dec = att_bytes / (rep_dec["latent_attention"] * 1e-3) / 1e9
+    att_dec = _rate(att_bytes, 1e9, rep_dec, "latent_attention")
     # the element-wise recurrence moves three pre-activations in and one value out per token and channel (bfloat16)
     scan_bytes = n_par * D * 4 * 2.0
-    scan_pre = T * scan_bytes / (ops_pre["min_gru_scan"] * 1e-3) / 1e9
-    scan_dec = NB * (scan_bytes + n_par * D * 8.0) / (ops_dec["min_gru_scan"] * 1e-3) / 1e9      # (+ the float state in and out)
+    scan_pre = _rate(T * scan_bytes, 1e9, ops_pre, "min_gru_scan")
+    scan_dec = _rate(NB * (scan_bytes + n_par * D * 8.0), 1e9, ops_dec, "min_gru_scan")      # (+ the float state in and out)
     active = s["top"] * s["experts"] / (s["experts"] + 4.0)  # chosen router outputs that are experts with weights, on average
     moe_flops = n_moe * T * active * 3 * 2.0 * s["ff"] * D
-    moe_pre = moe_flops / (ops_pre["moe_experts"] * 1e-3) / 1e12
+    moe_pre = _rate(moe_flops, 1e12, ops_pre, "moe_experts")
     moe_bytes = n_moe * min(s["experts"], NB * s["top"]) * 3 * s["ff"] * D * 2.0
-    moe_dec = moe_bytes / (rep_dec["moe_experts"] * 1e-3) / 1e9
+    moe_dec = _rate(moe_bytes, 1e9, rep_dec, "moe_experts")
     # residual kernel: per sublayer the float stream in and out, the sublayer's output in, the next input out; the first call only norms
     res_bytes = T * (2 * LAYERS * (8.0 * D + 4.0 * D) + 4.0 * D + 2.0 * D)
-    res_pre = res_bytes / (rep_pre["add_normed_rms_norm"] * 1e-3) / 1e9
+    res_pre = _rate(res_bytes, 1e9, rep_pre, "add_normed_rms_norm")
     out = dict(model=f"Pemolorn-{name}", sizes=m, prefill_tokens_per_s=T / pre * 1e3, prefill_ms=pre, decode_tokens_per_s=NB / dec * 1e3,
                decode_ms=dec, decode_from_hipgraph=graph_ok, decode_ms_eager=dec_eager, decode_ms_gpu_events=dec_events_ms, context=ctx,
                prefill_ops_ms=ops_pre, decode_ops_ms=ops_dec, prefill_kernels_ms=rep_pre, decode_kernels_ms=rep_dec,
-               roofline=dict(prefill_attention_tflops=att_pre, prefill_attention_frac_bf16_peak=att_pre / BF16_PEAK_TFLOPS,
-                             decode_attention_gbs=att_dec, decode_attention_frac_hbm=att_dec / HBM_PEAK_GBS,
-                             prefill_experts_tflops=moe_pre, prefill_experts_frac_bf16_peak=moe_pre / BF16_PEAK_TFLOPS,
-                             decode_experts_gbs=moe_dec, decode_experts_frac_hbm=moe_dec / HBM_PEAK_GBS,
-                             prefill_recurrence_gbs=scan_pre, prefill_recurrence_frac_hbm=scan_pre / HBM_PEAK_GBS,
-                             decode_recurrence_gbs=scan_dec, decode_recurrence_frac_hbm=scan_dec / HBM_PEAK_GBS,
-                             prefill_residual_kernel_gbs=res_pre, prefill_residual_kernel_frac_hbm=res_pre / HBM_PEAK_GBS))
+               roofline=dict(prefill_attention_tflops=att_pre, prefill_attention_frac_bf16_peak=_of(att_pre, BF16_PEAK_TFLOPS),
+                             decode_attention_gbs=att_dec, decode_attention_frac_hbm=_of(att_dec, HBM_PEAK_GBS),
+                             prefill_experts_tflops=moe_pre, prefill_experts_frac_bf16_peak=_of(moe_pre, BF16_PEAK_TFLOPS),
+                             decode_experts_gbs=moe_dec, decode_experts_frac_hbm=_of(moe_dec, HBM_PEAK_GBS),
+                             prefill_recurrence_gbs=scan_pre, prefill_recurrence_frac_hbm=_of(scan_pre, HBM_PEAK_GBS),
+                             decode_recurrence_gbs=scan_dec, decode_recurrence_frac_hbm=_of(scan_dec, HBM_PEAK_GBS),
+                             prefill_residual_kernel_gbs=res_pre, prefill_residual_kernel_frac_hbm=_of(res_pre, HBM_PEAK_GBS)))
     for sl in slots:
         eng.close_sequence(sl)
     del eng
@@ -769,7 +793,7 @@ def bench_sagupel(name, s, dev, steps, warmup):
         want = [k * L + L - 1 for k in range(BP)]
         if i == BP:                                          # one step with events around every launch
             ops_pre, _ = timer.step(lambda: eng.execute(items, want))
-            rep_pre = {k: timer.replay(k, 3) for k in stateless}
+            rep_pre = timer.replays(stateless, 3)
             continue
         torch.cuda.synchronize()
         t0 = time.perf_counter()
@@ -786,7 +810,7 @@ def bench_sagupel(name, s, dev, steps, warmup):
 
     dec_eager = timed(decode, steps, warmup)
     ops_dec, dec_events_ms = timer.step(decode)
-    rep_dec = {k: timer.replay(k, 20) for k in ("talking_attention", "latent_attention", "qk_norm_rope_prep", "glu", "head_rms_gate", "conv_silu_unit")}
+    rep_dec = timer.replays(("talking_attention", "latent_attention", "qk_norm_rope_prep", "glu", "head_rms_gate", "conv_silu_unit"), 20)
     eng.decode_graphs = True
     dec = timed(decode, steps, warmup)
     graph_ok = any(v is not False for v in eng._graphs.values()) and bool(eng._graphs)
@@ -798,31 +822,31 @@ def bench_sagupel(name, s, dev, steps, warmup):
     pairs = BP * sum(p + 1 for p in range(L))
     # useful work per visible pair: q.k and p.v of every head, and the mix of the heads' weights
     talk_flops = n_par * pairs * H * (R + H) * 2.0
-    talk_pre = talk_flops / (rep_pre["talking_attention"] * 1e-3) / 1e12
-    talk_dec = n_par * NB * ctx * m["a_kv"] * R * 2.0 / (rep_dec["talking_attention"] * 1e-3) / 1e9
+    talk_pre = _rate(talk_flops, 1e12, rep_pre, "talking_attention")
+    talk_dec = _rate(n_par * NB * ctx * m["a_kv"] * R * 2.0, 1e9, rep_dec, "talking_attention")
     att_flops = n_att * BP * sum(min(p + 1, W_) for p in range(L)) * H * R * 2.0
-    att_pre = att_flops / (rep_pre["latent_attention"] * 1e-3) / 1e12
-    att_dec = n_att * NB * min(ctx, W_) * m["a_kv"] * R * 2.0 / (rep_dec["latent_attention"] * 1e-3) / 1e9
+    att_pre = _rate(att_flops, 1e12, rep_pre, "latent_attention")
+    att_dec = _rate(n_att * NB * min(ctx, W_) * m["a_kv"] * R * 2.0, 1e9, rep_dec, "latent_attention")
     # recurrences: 5 (retention) / 7 (delta rule) float operations per state element and token; decoding moves the state twice
     el = n_ret * m["g_heads"] * m["g_dim"] * m["g_vdim"], n_par * m["d_heads"] * m["d_dim"] * m["d_vdim"]
-    scan_pre = T * (5.0 * el[0] + 7.0 * el[1]) / (ops_pre["recurrent_scan"] * 1e-3) / 1e12
-    scan_dec = NB * (el[0] + el[1]) * 4.0 * 2 / (ops_dec["recurrent_scan"] * 1e-3) / 1e9
+    scan_pre = _rate(T * (5.0 * el[0] + 7.0 * el[1]), 1e12, ops_pre, "recurrent_scan")
+    scan_dec = _rate(NB * (el[0] + el[1]) * 4.0 * 2, 1e9, ops_dec, "recurrent_scan")
     # residual kernel: per sublayer the float stream in and out, the sublayer's output in; one cast out per layer (the second norm's
     # reader is the convolution, which reads the float stream and writes one row)
     res_bytes = T * LAYERS * (2 * (8.0 * D + 2.0 * D) + 2.0 * D)
-    res_pre = res_bytes / (rep_pre["scaled_add_rms_norm"] * 1e-3) / 1e9
-    conv_pre = T * LAYERS * (4.0 * D + 2.0 * D) / (rep_pre["residual_conv"] * 1e-3) / 1e9
+    res_pre = _rate(res_bytes, 1e9, rep_pre, "scaled_add_rms_norm")
+    conv_pre = _rate(T * LAYERS * (4.0 * D + 2.0 * D), 1e9, rep_pre, "residual_conv")
     out = dict(model=f"Sagupel-{name}", sizes=m, prefill_tokens_per_s=T / pre * 1e3, prefill_ms=pre, decode_tokens_per_s=NB / dec * 1e3,
                decode_ms=dec, decode_from_hipgraph=graph_ok, decode_ms_eager=dec_eager, decode_ms_gpu_events=dec_events_ms, context=ctx,
                prefill_ops_ms=ops_pre, decode_ops_ms=ops_dec, prefill_kernels_ms=rep_pre, decode_kernels_ms=rep_dec,
-               roofline=dict(prefill_talking_attention_tflops=talk_pre, prefill_talking_attention_frac_bf16_peak=talk_pre / BF16_PEAK_TFLOPS,
-                             decode_talking_attention_gbs=talk_dec, decode_talking_attention_frac_hbm=talk_dec / HBM_PEAK_GBS,
-                             prefill_window_attention_tflops=att_pre, prefill_window_attention_frac_bf16_peak=att_pre / BF16_PEAK_TFLOPS,
-                             decode_window_attention_gbs=att_dec, decode_window_attention_frac_hbm=att_dec / HBM_PEAK_GBS,
-                             prefill_recurrence_tflops=scan_pre, prefill_recurrence_frac_fp32_valu_peak=scan_pre / FP32_VALU_PEAK_TFLOPS,
-                             decode_recurrence_gbs=scan_dec, decode_recurrence_frac_hbm=scan_dec / HBM_PEAK_GBS,
-                             prefill_residual_kernel_gbs=res_pre, prefill_residual_kernel_frac_hbm=res_pre / HBM_PEAK_GBS,
-                             prefill_input_conv_gbs=conv_pre, prefill_input_conv_frac_hbm=conv_pre / HBM_PEAK_GBS))
+               roofline=dict(prefill_talking_attention_tflops=talk_pre, prefill_talking_attention_frac_bf16_peak=_of(talk_pre, BF16_PEAK_TFLOPS),
+                             decode_talking_attention_gbs=talk_dec, decode_talking_attention_frac_hbm=_of(talk_dec, HBM_PEAK_GBS),
+                             prefill_window_attention_tflops=att_pre, prefill_window_attention_frac_bf16_peak=_of(att_pre, BF16_PEAK_TFLOPS),
+                             decode_window_attention_gbs=att_dec, decode_window_attention_frac_hbm=_of(att_dec, HBM_PEAK_GBS),
+                             prefill_recurrence_tflops=scan_pre, prefill_recurrence_frac_fp32_valu_peak=_of(scan_pre, FP32_VALU_PEAK_TFLOPS),
+                             decode_recurrence_gbs=scan_dec, decode_recurrence_frac_hbm=_of(scan_dec, HBM_PEAK_GBS),
+                             prefill_residual_kernel_gbs=res_pre, prefill_residual_kernel_frac_hbm=_of(res_pre, HBM_PEAK_GBS),
+                             prefill_input_conv_gbs=conv_pre, prefill_input_conv_frac_hbm=_of(conv_pre, HBM_PEAK_GBS)))
     for sl in slots:
         eng.close_sequence(sl)
     del eng
@@ -894,7 +918,7 @@ def bench_rivolix(name, s, dev, steps, warmup):
         want = [k * L + L - 1 for k in range(BP)]
         if i == BP:                                          # one step with events around every launch
             ops_pre, _ = timer.step(lambda: eng.execute(items, want))
-            rep_pre = {k: timer.replay(k, 3) for k in stateless}     # (the convolution writes the same history again)
+            rep_pre = timer.replays(stateless, 3)     # (the convolution writes the same history again)
             continue
         torch.cuda.synchronize()
         t0 = time.perf_counter()
@@ -911,7 +935,7 @@ def bench_rivolix(name, s, dev, steps, warmup):
 
     dec_eager = timed(decode, steps, warmup)
     ops_dec, dec_events_ms = timer.step(decode)
-    rep_dec = {k: timer.replay(k, 20) for k in stateless + ("moe_experts",)}
+    rep_dec = timer.replays(stateless + ("moe_experts",), 20)
     eng.decode_graphs = True
     dec = timed(decode, steps, warmup)
     graph_ok = any(v is not False for v in eng._graphs.values()) and bool(eng._graphs)
@@ -924,29 +948,29 @@ def bench_rivolix(name, s, dev, steps, warmup):
     R = d + dv                                               # (two maps of d / 2, or one of d)
     pairs = BP * sum(p + 1 for p in range(L))
     # useful work per visible pair: the two maps' q.k and p.v; one q.k and p.v
-    diff_pre = n_diff * pairs * H * (d + 2 * dv) * 2.0 / (rep_pre["diff_attention"] * 1e-3) / 1e12
-    tied_pre = n_tied * pairs * H * 2 * d * 2.0 / (rep_pre["single_map_attention"] * 1e-3) / 1e12
-    diff_dec = n_diff * NB * ctx * G * R * 2.0 / (rep_dec["diff_attention"] * 1e-3) / 1e9
-    tied_dec = n_tied * NB * ctx * G * 2 * d * 2.0 / (rep_dec["single_map_attention"] * 1e-3) / 1e9
-    moe_pre = LAYERS * T * s["top"] * 3 * 2.0 * s["ff"] * D / (ops_pre["moe_experts"] * 1e-3) / 1e12
-    moe_dec = LAYERS * min(s["experts"], NB * s["top"]) * 3 * s["ff"] * D * 2.0 / (rep_dec["moe_experts"] * 1e-3) / 1e9
+    diff_pre = _rate(n_diff * pairs * H * (d + 2 * dv) * 2.0, 1e12, rep_pre, "diff_attention")
+    tied_pre = _rate(n_tied * pairs * H * 2 * d * 2.0, 1e12, rep_pre, "single_map_attention")
+    diff_dec = _rate(n_diff * NB * ctx * G * R * 2.0, 1e9, rep_dec, "diff_attention")
+    tied_dec = _rate(n_tied * NB * ctx * G * 2 * d * 2.0, 1e9, rep_dec, "single_map_attention")
+    moe_pre = _rate(LAYERS * T * s["top"] * 3 * 2.0 * s["ff"] * D, 1e12, ops_pre, "moe_experts")
+    moe_dec = _rate(LAYERS * min(s["experts"], NB * s["top"]) * 3 * s["ff"] * D * 2.0, 1e9, rep_dec, "moe_experts")
     # residual kernel: the float stream in and out and two casts per layer; mixer, routed and shared outputs in; the first call gathers
-    res_pre = T * (LAYERS * (8.0 * D + 3 * 2.0 * D + 2 * 2.0 * D) + 6.0 * D) / (rep_pre["scaled_sum_rms_norms"] * 1e-3) / 1e9
+    res_pre = _rate(T * (LAYERS * (8.0 * D + 3 * 2.0 * D + 2 * 2.0 * D) + 6.0 * D), 1e9, rep_pre, "scaled_sum_rms_norms")
     # preparation: the projections in, queries and cache rows out
-    conv_pre = T * 2.0 * (n_diff * 2 * H * d + own * 2 * G * R) / (rep_pre["conv_heads_cache"] * 1e-3) / 1e9
-    prep_pre = n_tied * T * 2.0 * (2 * H * d + G * d + G * 2 * d) / (rep_pre["qk_norm_rope_prep"] * 1e-3) / 1e9
+    conv_pre = _rate(T * 2.0 * (n_diff * 2 * H * d + own * 2 * G * R), 1e9, rep_pre, "conv_heads_cache")
+    prep_pre = _rate(n_tied * T * 2.0 * (2 * H * d + G * d + G * 2 * d), 1e9, rep_pre, "qk_norm_rope_prep")
     out = dict(model=f"Rivolix-{name}", sizes=m, prefill_tokens_per_s=T / pre * 1e3, prefill_ms=pre, decode_tokens_per_s=NB / dec * 1e3,
                decode_ms=dec, decode_from_hipgraph=graph_ok, decode_ms_eager=dec_eager, decode_ms_gpu_events=dec_events_ms, context=ctx,
                prefill_ops_ms=ops_pre, decode_ops_ms=ops_dec, prefill_kernels_ms=rep_pre, decode_kernels_ms=rep_dec,
-               roofline=dict(prefill_diff_attention_tflops=diff_pre, prefill_diff_attention_frac_bf16_peak=diff_pre / BF16_PEAK_TFLOPS,
-                             decode_diff_attention_gbs=diff_dec, decode_diff_attention_frac_hbm=diff_dec / HBM_PEAK_GBS,
-                             prefill_tied_attention_tflops=tied_pre, prefill_tied_attention_frac_bf16_peak=tied_pre / BF16_PEAK_TFLOPS,
-                             decode_tied_attention_gbs=tied_dec, decode_tied_attention_frac_hbm=tied_dec / HBM_PEAK_GBS,
-                             prefill_experts_tflops=moe_pre, prefill_experts_frac_bf16_peak=moe_pre / BF16_PEAK_TFLOPS,
-                             decode_experts_gbs=moe_dec, decode_experts_frac_hbm=moe_dec / HBM_PEAK_GBS,
-                             prefill_residual_kernel_gbs=res_pre, prefill_residual_kernel_frac_hbm=res_pre / HBM_PEAK_GBS,
-                             prefill_conv_prep_gbs=conv_pre, prefill_conv_prep_frac_hbm=conv_pre / HBM_PEAK_GBS,
-                             prefill_tied_prep_gbs=prep_pre, prefill_tied_prep_frac_hbm=prep_pre / HBM_PEAK_GBS))
+               roofline=dict(prefill_diff_attention_tflops=diff_pre, prefill_diff_attention_frac_bf16_peak=_of(diff_pre, BF16_PEAK_TFLOPS),
+                             decode_diff_attention_gbs=diff_dec, decode_diff_attention_frac_hbm=_of(diff_dec, HBM_PEAK_GBS),
+                             prefill_tied_attention_tflops=tied_pre, prefill_tied_attention_frac_bf16_peak=_of(tied_pre, BF16_PEAK_TFLOPS),
+                             decode_tied_attention_gbs=tied_dec, decode_tied_attention_frac_hbm=_of(tied_dec, HBM_PEAK_GBS),
+                             prefill_experts_tflops=moe_pre, prefill_experts_frac_bf16_peak=_of(moe_pre, BF16_PEAK_TFLOPS),
+                             decode_experts_gbs=moe_dec, decode_experts_frac_hbm=_of(moe_dec, HBM_PEAK_GBS),
+                             prefill_residual_kernel_gbs=res_pre, prefill_residual_kernel_frac_hbm=_of(res_pre, HBM_PEAK_GBS),
+                             prefill_conv_prep_gbs=conv_pre, prefill_conv_prep_frac_hbm=_of(conv_pre, HBM_PEAK_GBS),
+                             prefill_tied_prep_gbs=prep_pre, prefill_tied_prep_frac_hbm=_of(prep_pre, HBM_PEAK_GBS)))
     for sl in slots:
         eng.close_sequence(sl)
     del eng

@@ -183,7 +183,8 @@ class NormedPair:
 class PendingExperts:
     """The two launches of a mixture's experts in a decoding step, not made yet: a kernel that reads nothing of them may take one along (`take`), and `results`
     makes those that nobody took.  The second product reads the first one's results, so taking it makes the first if need be.  Everything happens on the stream
-    that was current when the object was made; it keeps the inputs alive until then."""
+    that was current when the object was made: on another one nothing is taken and `results` raises, since its launches would run beside what they read.  The object
+    keeps the inputs alive until then."""
 
     def __init__(self, ops, jobs, keeps, results):
         self.ops, self.jobs, self.keeps, self._results, self.made, self.stream = ops, jobs, keeps, results, 0, ops._s()
@@ -202,6 +203,8 @@ class PendingExperts:
             self.made += 1
 
     def results(self):
+        if self.ops._s() != self.stream:
+            raise RuntimeError("a mixture's pending experts are asked for on another stream than the one they were made on")
         self._make(2)
         return list(self._results)
 

@@ -249,8 +249,13 @@ int qs_debug_gemm_clock_probe(void* buf, int workgroups);
  * in plan5 = {family, p0, p1, p2, p3}: family 1 = split-K kernel (m_tiles, waves, cross-block slices, xcd mapping),
  * 2 = LDS-pair kernel, 3 = ring kernel (m_tiles, units, token blocks, K slices), 4 = tiled kernel (8 = 256-token tile,
  * 4 = 128-token tile).  No reference counterpart: it makes the selection heuristics testable on a CPU-only machine
- * (tests/test_dispatch_plan.py).  per_group: 0 = per-channel, 1 = per-group-128.  Honours qs_set_gemm_variant. */
+ * (tests/test_dispatch_plan.py).  per_group: 0 = per-channel, 1 = per-group-128.  Honours qs_set_gemm_variant.
+ * The plan is that of ONE launch over all M tokens; a per-channel product of a prompt may run as two (next entry). */
 int qs_w4a8_gemm_plan(int per_group, int M, int N, int K, int* plan5);
+/* What qs_w4a8_per_chn_gemm (silu_mul: qs_w4a8_per_chn_gemm_silu_mul) does with these arguments: *first_tokens = the tokens of the first of two launches, the second
+ * one takes the others; 0: one launch.  Host only: the pointers are looked at for their alignment and not read. */
+int qs_w4a8_per_chn_gemm_rounds(const int8_t* in_feats, const int8_t* kernel, const void* wscales, const void* ascales, const void* w_szs, const void* a_ssums,
+                                const void* out, int silu_mul, int M, int N, int K, int* first_tokens);
 
 /* ------------------------------------------------------------------------------------------------------------
  * Decode attention over the paged, quantised KV cache.

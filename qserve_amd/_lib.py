@@ -33,6 +33,7 @@ SIGNATURES = {
     "qs_set_row_sum_order": (_i, [_i]),
     "qs_get_row_sum_order": (_i, []),
     "qs_w4a8_gemm_plan": (_i, [_i, _i, _i, _i, _vp]),
+    "qs_w4a8_per_chn_gemm_rounds": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp]),
     "qs_w4a8_gemm_planes_plan": (_i, [_i, _i, _i, _i, _vp]),
     "qs_w4a8_per_chn_gemm_planes": (_i, [_vp, _vp, _vp, _i, _i, _i, _vp]),
     "qs_w4a8_per_group_gemm_planes": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp]),

@@ -766,12 +766,15 @@ int whole_rounds(int M, int N, int K, bool act) {
     return family == 1 && p[2] == 1 && (others + 16 * p[0] - 1) / (16 * p[0]) * 4 * wide <= 256 ? first : 0;
 }
 // (pointers that the tiles alone take keep to them)
+int first_launch(const int8_t* A, const int8_t* W, const void* wscales, const void* wszs, const void* ascales, const void* assums, const void* out, int M, int N, int K, bool act) {
+    const auto at = [](const void* p) { return reinterpret_cast<uintptr_t>(p); };
+    const bool fit = A && W && wscales && wszs && ascales && assums && out && (at(A) | at(W) | at(out)) % 16 == 0 && (at(wscales) | at(wszs) | at(ascales) | at(assums)) % 4 == 0;
+    return fit ? whole_rounds(M, N, K, act) : 0;
+}
 template <class Launch>
 int in_rounds(const int8_t* A, const int8_t* W, const void* wscales, const void* wszs, const void* ascales, const void* assums, void* out, int out_width, int M, int N,
               int K, bool act, const Launch& launch) {
-    const auto at = [](const void* p) { return reinterpret_cast<uintptr_t>(p); };
-    const bool fit = A && W && wscales && wszs && ascales && assums && out && (at(A) | at(W) | at(out)) % 16 == 0 && (at(wscales) | at(wszs) | at(ascales) | at(assums)) % 4 == 0;
-    const int first = fit ? whole_rounds(M, N, K, act) : 0;
+    const int first = first_launch(A, W, wscales, wszs, ascales, assums, out, M, N, K, act);
     if (!first) return launch(A, ascales, assums, out, M, true);
     const int rc = launch(A, ascales, assums, out, first, true);
     if (rc != QS_OK) return rc;
@@ -779,6 +782,13 @@ int in_rounds(const int8_t* A, const int8_t* W, const void* wscales, const void*
     return launch(A + (size_t)first * K, half(ascales, first), half(assums, first), const_cast<_Float16*>(half(out, (size_t)first * out_width)), M - first, false);
 }
 }  // namespace
+
+extern "C" int qs_w4a8_per_chn_gemm_rounds(const int8_t* in_feats, const int8_t* kernel, const void* wscales, const void* ascales, const void* w_szs, const void* a_ssums,
+                                           const void* out, int silu_mul, int M, int N, int K, int* first_tokens) {
+    QS_REQUIRE(first_tokens, "w4a8_per_chn_gemm_rounds: null output");
+    *first_tokens = silu_mul && g_act_off ? 0 : first_launch(in_feats, kernel, wscales, w_szs, ascales, a_ssums, out, M, N, K, silu_mul != 0);
+    return QS_OK;
+}
 
 extern "C" int qs_w4a8_per_chn_gemm(const int8_t* in_feats, const int8_t* kernel, const void* wscales,
                                     const void* ascales, const void* w_szs, const void* a_ssums, void* out_feats,

@@ -14,7 +14,9 @@
 // row's chain of trips.  Measured for one token, launches replaced -> this, us: norm + qkv 6144 x 4096 9.9 -> 6.9, norm + gate_up 28672 x 4096 16.1 -> 14.5, o 4096 x
 // 4096 4.7 -> 3.5 (one slice 3.9, four 3.7), quantiser + down 4096 x 14336 10.2 -> 9.1, of 11008 9.6 -> 7.9; groups of 128 12.2 -> 8.6, 19.6 -> 19.2, 5.7 -> 4.0, 12.4 ->
 // 10.4; a step of four layers 216.9 -> 191.5.  Every workgroup does every row, so it loses from two rows on wherever there are many of them (gate_up 16.2 -> 19.4,
-// down 10.3 -> 12.7; three rows of qkv 10.0 -> 12.6); without a row operation (`o`) four rows take 4.7 -> 4.3.
+// down 10.3 -> 12.7; three rows of qkv 10.0 -> 12.6); without a row operation (`o`) four rows take 4.7 -> 4.3.  The entries take those too; the decode engine asks for the forms that
+// gain.  Registers: gate_up of one row with groups of 128 behind two planes holds 253 of 256, behind four (not asked for) 16 - 34 spill.  The norm is compiled for rows of 4096, the width
+// of everything measured.
 #include "common.h"
 #include "row_ops.h"
 

@@ -798,7 +798,8 @@ __global__ __launch_bounds__(NT, (Shape<DT, CT, M>::STEP_OCC)) void maps_step_ke
 // Attention, output product and experts apart -> both products' launches shared (MI355X, us, 16 heads on 4 pools, two maps of 64 over values of 128, 4 of 16 experts of
 // 2048 x 1408 and a shared one): 1 token behind 64 / 333 / 4000 positions 30.0 -> 19.5, 35.6 -> 21.7, 47.6 -> 35.1; 16 behind 300 72.6 -> 56.4; 64 behind 100 /
 // 1000 / 3000 77 -> 70, 99 -> 83, 153 -> 129; 4 of 32 experts of 4096 x 2752, 1 / 16 / 64 behind 333 / 300 / 8000 83 -> 69, 370 -> 353, 582 -> 544.  Faster at every size tried, so
-// wherever the sizes fit (maps of 128 over values of 128 need more registers, 32 heads a pool over wide values more LDS: those run apart).
+// wherever the sizes fit (maps of 128 over values of 128 need more registers, 32 heads a pool over wide values more LDS: those run apart).  At 256 registers two maps of 64 over values of 128
+// spill 6 - 8 and two of 96 over 96 spill 3; the figures above are with that.
 template <int DT, int CT, int M, int FORM>
 __global__ __launch_bounds__(NT, 2) void maps_beside_experts_kernel(MapsArgs a, ExpertArgs e, SharedArgs sh, int blocks, int ny, int tiles) {
     using S = Shape<DT, CT, M>;

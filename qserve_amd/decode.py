@@ -295,7 +295,8 @@ class DecodeEngine:
         * the quantiser of the attention's rows with o (in place of the attention's own, which its workgroups hand over to each other for), whole steps of four layers where
           the keys are not cut over workgroups: 1 row 183.1 / 176.9 (Llama-2-7B 185.6 / 178.8, groups 230.6 / 224.0), 2 rows 205.8 / 203.6, 3 rows 208.2 / 210.2; where they
           are, the merge quantises in its launch: 1 row of 1500 positions 189.7 / 194.4;
-        * the quantiser with down: 1 row 10.2 / 9.1 (11008 wide 9.6 / 7.9, groups 12.4 / 10.4), 2 rows 10.3 / 12.7."""
+        * the quantiser with down: 1 row 10.2 / 9.1 (11008 wide 9.6 / 7.9, groups 12.4 / 10.4), 2 rows 10.3 / 12.7.
+        Other hidden widths than 4096 were not measured and keep the launches that these replace."""
         B, hid, inter = self.B, self.hid, self.inter
         group = self.group_size != -1
         self.rows = set()
